@@ -64,7 +64,8 @@ bool logged(const LaunchRecord& r)
 {
     if (!t_launch_log)
         return false;
-    t_launch_log->records.push_back(r);
+    if (t_launch_log->keep)
+        t_launch_log->records.push_back(r);
     return true;
 }
 
@@ -2417,6 +2418,7 @@ int forward_local(int n, int c, size_t s, const HostTensor& tx, const HostTensor
     {
         // both launches are planned before the first is issued: a call that is rejected writes nothing
         LaunchLog plan;
+        plan.keep = false;
         ScopedLaunchLog scope(&plan);
         FusedStats<T> g = f;
         int err = sums_impl<T>(n, c, s, tx, x, nullptr, nullptr, ws, st, &g);
@@ -2465,6 +2467,7 @@ int backward_local(int n, int c, size_t s, const HostTensor& tx, const HostTenso
     {
         // both launches are planned before the first is issued: a call that is rejected writes nothing
         LaunchLog plan;
+        plan.keep = false;
         ScopedLaunchLog scope(&plan);
         FusedStats<T> g = f;
         int err = backprop1_impl<T>(n, c, s, tx, td, x, dy, mean, var, scale, nullptr, nullptr,

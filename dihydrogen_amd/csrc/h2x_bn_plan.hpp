@@ -67,6 +67,7 @@ struct LaunchRecord
 struct LaunchLog
 {
     std::vector<LaunchRecord> records;
+    bool keep = true; // false: nothing is issued and nothing recorded (validation of a call)
 };
 
 // While a log is installed on the calling thread, the entry points of

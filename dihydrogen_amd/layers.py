@@ -13,7 +13,7 @@ from typing import Callable, List, Optional, Sequence
 import torch
 
 from . import capi
-from .tensor import Tensor, _prod
+from .tensor import Layout, Tensor, _prod
 
 
 def _device_buffer(count: int, dtype, device="cuda", zero: bool = False) -> torch.Tensor:
@@ -26,76 +26,55 @@ def _device_buffer(count: int, dtype, device="cuda", zero: bool = False) -> torc
 _has_gpu: Optional[bool] = None
 
 
-def _stream_handle(stream: Optional[torch.cuda.Stream]) -> ctypes.c_void_p:
+def _stream_handle(stream: Optional[torch.cuda.Stream]) -> int:
+    """Handle of `stream`, or of the current stream of the current device (asked of torch's
+    bindings directly: torch.cuda.current_stream() makes an object first, 2.8 us against 0.2)."""
+    if stream is not None:
+        return stream.cuda_stream
     global _has_gpu
-    if stream is None:
-        if _has_gpu is None:
-            _has_gpu = torch.cuda.is_available()  # asked once: the answer does not change
-        if not _has_gpu:
-            # no GPU: the null stream; every launch then fails with HIP's own error.  (Launch
-            # audits, which play the kernels' indexing on the CPU, ignore the stream.)
-            return ctypes.c_void_p(0)
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+    if _has_gpu is None:
+        _has_gpu = torch.cuda.is_available()  # asked once: the answer does not change
+        if _has_gpu:
+            torch.cuda.init()
+    if not _has_gpu:
+        # no GPU: the null stream; every launch then fails with HIP's own error.  (Launch
+        # audits, which play the kernels' indexing on the CPU, ignore the stream.)
+        return 0
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
-def _ptr(t) -> ctypes.c_void_p:
-    if t is None:
-        return ctypes.c_void_p(0)
-    if isinstance(t, torch.Tensor):
-        return ctypes.c_void_p(t.data_ptr())
-    return ctypes.c_void_p(int(t))
-
-
-def _is_dense(t: Tensor) -> bool:
-    """No halo on the inner spatial dimensions: the layout the dense entry points
-    take (legacy/src/dnn_backend/batchnorm.cu:210-219)."""
-    nd = t.get_num_dims()
-    return all(t.overlap[d] == 0 for d in range(nd - 3))
-
-
-def _channel_geometry(t: Tensor):
-    """(num_samples, num_channels, spatial, spatial_real) of a dense local tensor."""
-    nd = t.get_num_dims()
-    if t.overlap[nd - 2] != 0 or t.overlap[nd - 1] != 0:
+def _dense_layout(t: Tensor) -> Layout:
+    """The layout of a tensor with no halo on its channel and sample dimensions."""
+    l = t.layout
+    if l.channel_halo:
         raise NotImplementedError("halo on the channel or sample dimension is not supported")
-    n, c = t.local_shape[nd - 1], t.local_shape[nd - 2]
-    return n, c, _prod(t.local_shape[: nd - 2]), _prod(t.local_real_shape[: nd - 2])
+    return l
 
 
-def _tensor_geometry(t: Tensor, num_samples: int) -> capi.TensorGeometry:
-    """h2x_tensor_geometry of a local tensor (local shape + get_strides())."""
-    nd = t.get_num_dims()
-    if t.overlap[nd - 2] != 0 or t.overlap[nd - 1] != 0:
-        raise NotImplementedError("halo on the channel or sample dimension is not supported")
-    g = capi.TensorGeometry()
-    g.num_dims = nd
-    strides = t.get_strides()
-    for i in range(nd):
-        g.local_shape[i] = t.local_shape[i]
-        g.strides[i] = strides[i]
-    g.local_shape[nd - 1] = num_samples
-    return g
+def _tensor_geometry(l: Layout, num_samples: int):
+    """h2x_tensor_geometry of a local tensor (local shape + get_strides()), as something the
+    native calls take for a pointer; keep it until the call has returned."""
+    if num_samples == l.samples:
+        return l.geometry_address
+    g = capi.TensorGeometry.from_buffer_copy(l.geometry)
+    g.local_shape[g.num_dims - 1] = num_samples
+    return _Struct(g)
 
 
-def _haloed_geometry(t: Tensor) -> capi.HaloedGeometry:
-    """h2x_haloed_geometry of a local tensor: local and real extents, halo widths."""
-    g = capi.HaloedGeometry()
-    g.num_dims = t.get_num_dims()
-    for i in range(g.num_dims):
-        g.local_shape[i] = t.local_shape[i]
-        g.real_shape[i] = t.local_real_shape[i]
-        g.lower_halo[i] = t.overlap[i]
-    return g
+class _Struct:
+    """A ctypes structure as a pointer argument of the native calls."""
+
+    def __init__(self, value):
+        self._value = value
+
+    def data_ptr(self) -> int:
+        return ctypes.addressof(self._value)
 
 
-def _share_a_haloed_geometry(*tensors: Tensor) -> bool:
+def _share_a_haloed_geometry(*layouts: Layout) -> bool:
     """Tensors with a halo on a spatial dimension whose local parts lie in memory alike."""
-    t0 = tensors[0]
-    nd = t0.get_num_dims()
-    return (any(t0.overlap[: nd - 2]) and t0.overlap[nd - 2] == 0 and t0.overlap[nd - 1] == 0
-            and all(t.local_shape == t0.local_shape and t.local_real_shape == t0.local_real_shape
-                    and t.overlap == t0.overlap and t.h2x_dtype == t0.h2x_dtype for t in tensors))
+    l0 = layouts[0]
+    return l0.haloed and not l0.channel_halo and all(l.alike == l0.alike for l in layouts)
 
 
 class BatchNormalization:
@@ -127,6 +106,7 @@ class BatchNormalization:
         self.clear_output_halo = clear_output_halo
         self.num_current_samples = 0
         self._lib = capi.load()
+        self._calls = capi.calls()
         self._workspace: Optional[torch.Tensor] = None
         self._workspace_channels = -1
 
@@ -144,29 +124,26 @@ class BatchNormalization:
     def _num_per_sum(self, t: Tensor) -> int:
         """Elements per channel of the global (global_stats) or local shape
         (batchnorm.hpp:232-236,414-418)."""
-        nd = t.get_num_dims()
-        shape = t.shape if self.global_stats else t.local_shape
-        return _prod(shape) // shape[nd - 2] if shape[nd - 2] else 0
+        l = t.layout
+        return l.per_channel_global if self.global_stats else l.per_channel_local
 
     # ---- forward -----------------------------------------------------------
     def forward_stage1(self, input: Tensor, mean: torch.Tensor, var: torch.Tensor,
                        is_training: bool = True) -> int:
-        self.set_num_samples(input.local_shape[-1])
+        lx = input.layout
+        self.num_current_samples = lx.samples
         if not is_training:
             return 0
-        n, c, s, sr = _channel_geometry(input)
-        active = input.is_split_root() and input.get_local_size() > 0
-        ns = self.num_current_samples if active else 0
-        if _is_dense(input):
-            capi.check(self._lib.h2x_bn_channel_sums_and_sqsums(
-                input.h2x_dtype, ns, c, s, sr, _ptr(input.get_base_ptr()), _ptr(mean), _ptr(var),
-                _ptr(self._ws(c)), _stream_handle(self.stream)), "channel_sums_and_sqsums")
+        _dense_layout(input)
+        ns = lx.samples if lx.active else 0
+        if lx.dense:
+            capi.check(self._calls.h2x_bn_channel_sums_and_sqsums(
+                lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, input.get_base_ptr(), mean, var,
+                self._ws(lx.channels), _stream_handle(self.stream)), "channel_sums_and_sqsums")
         else:  # halo on an inner spatial dimension: the generic path of batchnorm.cu:232-248
-            g = _tensor_geometry(input, ns)
-            capi.check(self._lib.h2x_bn_channel_sums_and_sqsums_strided(
-                input.h2x_dtype, ns, ctypes.byref(g), _ptr(input.get_base_ptr()), _ptr(mean),
-                _ptr(var), _ptr(self._ws(c)), _stream_handle(self.stream)),
-                "channel_sums_and_sqsums (strided)")
+            capi.check(self._calls.h2x_bn_channel_sums_and_sqsums_strided(
+                lx.dtype, ns, _tensor_geometry(lx, ns), input.get_base_ptr(), mean, var,
+                self._ws(lx.channels), _stream_handle(self.stream)), "channel_sums_and_sqsums (strided)")
         return 0
 
     def forward_allreduce(self, mean: torch.Tensor, var: torch.Tensor, is_training: bool = True) -> int:
@@ -177,32 +154,28 @@ class BatchNormalization:
     def sums_to_statistics(self, num_per_sum: int, mean, var, running_mean, running_var,
                            dtype: int = capi.F32) -> None:
         """batchnorm.hpp:494-503."""
-        capi.check(self._lib.h2x_bn_sums_to_statistics(
-            dtype, mean.numel(), num_per_sum, self.decay, _ptr(mean), _ptr(var), _ptr(running_mean),
-            _ptr(running_var), _stream_handle(self.stream)), "sums_to_statistics")
+        capi.check(self._calls.h2x_bn_sums_to_statistics(
+            dtype, mean.numel(), num_per_sum, self.decay, mean, var, running_mean, running_var,
+            _stream_handle(self.stream)), "sums_to_statistics")
 
     def batch_normalization(self, input: Tensor, mean, var, scale, bias, output: Tensor) -> None:
         """batchnorm.hpp:505-517."""
-        n, c, s, sr = _channel_geometry(input)
-        _, _, so, sro = _channel_geometry(output)
+        lx, ly = _dense_layout(input), _dense_layout(output)
         ns = self.num_current_samples
-        if self.clear_output_halo and ns == n and _share_a_haloed_geometry(input, output):
-            g = _haloed_geometry(output)
-            capi.check(self._lib.h2x_bn_batch_normalization_clearing(
-                input.h2x_dtype, ctypes.byref(g), _ptr(input.get_buffer()), _ptr(mean), _ptr(var), _ptr(scale),
-                _ptr(bias), _ptr(output.get_buffer()), self.epsilon, _stream_handle(self.stream)),
-                "batch_normalization (clearing)")
-        elif _is_dense(input) and _is_dense(output):
-            capi.check(self._lib.h2x_bn_batch_normalization(
-                input.h2x_dtype, ns, c, s, sr, sro, _ptr(input.get_base_ptr()), _ptr(mean), _ptr(var),
-                _ptr(scale), _ptr(bias), _ptr(output.get_base_ptr()), self.epsilon,
-                _stream_handle(self.stream)), "batch_normalization")
+        if self.clear_output_halo and ns == lx.samples and _share_a_haloed_geometry(lx, ly):
+            capi.check(self._calls.h2x_bn_batch_normalization_clearing(
+                lx.dtype, ly.haloed_geometry_address, input.get_buffer(), mean, var, scale, bias,
+                output.get_buffer(), self.epsilon, _stream_handle(self.stream)), "batch_normalization (clearing)")
+        elif lx.dense and ly.dense:
+            capi.check(self._calls.h2x_bn_batch_normalization(
+                lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ly.spatial_real, input.get_base_ptr(), mean,
+                var, scale, bias, output.get_base_ptr(), self.epsilon, _stream_handle(self.stream)),
+                "batch_normalization")
         else:
-            gx, gy = _tensor_geometry(input, ns), _tensor_geometry(output, ns)
-            capi.check(self._lib.h2x_bn_batch_normalization_strided(
-                input.h2x_dtype, ns, ctypes.byref(gx), ctypes.byref(gy), _ptr(input.get_base_ptr()),
-                _ptr(mean), _ptr(var), _ptr(scale), _ptr(bias), _ptr(output.get_base_ptr()),
-                self.epsilon, _stream_handle(self.stream)), "batch_normalization (strided)")
+            capi.check(self._calls.h2x_bn_batch_normalization_strided(
+                lx.dtype, ns, _tensor_geometry(lx, ns), _tensor_geometry(ly, ns), input.get_base_ptr(), mean, var,
+                scale, bias, output.get_base_ptr(), self.epsilon, _stream_handle(self.stream)),
+                "batch_normalization (strided)")
 
     def forward_stage2(self, input: Tensor, mean, var, running_mean, running_var, scale, bias,
                        output: Tensor, is_training: bool = True) -> int:
@@ -214,33 +187,30 @@ class BatchNormalization:
             self.batch_normalization(input, running_mean, running_var, scale, bias, output)  # :243-247
         return 0
 
-    def _runs_local(self, *tensors: Tensor) -> bool:
+    def _runs_local(self, l0: Layout, haloed: bool) -> bool:
         """No all-reduce between the stages, a rank that owns elements (and no halo to clear)."""
-        t0 = tensors[0]
-        return (self.fuse_local and not (self.global_stats and self.allreduce is not None)
-                and t0.is_split_root() and t0.get_local_size() > 0
-                and not (self.clear_output_halo and any(any(t.overlap) for t in tensors)))
+        return (self.fuse_local and l0.active and (self.allreduce is None or not self.global_stats)
+                and not (haloed and self.clear_output_halo))
 
     def forward(self, input, mean, var, running_mean, running_var, scale, bias, output,
                 is_training: bool = True) -> int:
-        if is_training and self._runs_local(input, output):
-            self.set_num_samples(input.local_shape[-1])
-            n, c, s, sr = _channel_geometry(input)
-            _, _, _, sro = _channel_geometry(output)
-            if _is_dense(input) and _is_dense(output):
-                capi.check(self._lib.h2x_bn_forward_local(
-                    input.h2x_dtype, self.num_current_samples, c, s, sr, sro, _ptr(input.get_base_ptr()),
-                    _ptr(scale), _ptr(bias), self._num_per_sum(input), self.decay, self.epsilon, _ptr(mean),
-                    _ptr(var), _ptr(running_mean), _ptr(running_var), _ptr(output.get_base_ptr()),
-                    _ptr(self._ws(c)), _stream_handle(self.stream)), "bn forward (local)")
+        lx, ly = input.layout, output.layout
+        if is_training and self._runs_local(lx, lx.haloed or ly.haloed):
+            _dense_layout(input), _dense_layout(output)
+            ns = self.num_current_samples = lx.samples
+            per_sum = lx.per_channel_global if self.global_stats else lx.per_channel_local
+            if lx.dense and ly.dense:
+                status = self._calls.h2x_bn_forward_local(
+                    lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ly.spatial_real, input.get_base_ptr(),
+                    scale, bias, per_sum, self.decay, self.epsilon, mean, var, running_mean, running_var,
+                    output.get_base_ptr(), self._ws(lx.channels), _stream_handle(self.stream))
             else:
-                ns = self.num_current_samples
-                gx, gy = _tensor_geometry(input, ns), _tensor_geometry(output, ns)
-                capi.check(self._lib.h2x_bn_forward_local_strided(
-                    input.h2x_dtype, ns, ctypes.byref(gx), ctypes.byref(gy), _ptr(input.get_base_ptr()),
-                    _ptr(scale), _ptr(bias), self._num_per_sum(input), self.decay, self.epsilon, _ptr(mean),
-                    _ptr(var), _ptr(running_mean), _ptr(running_var), _ptr(output.get_base_ptr()),
-                    _ptr(self._ws(c)), _stream_handle(self.stream)), "bn forward (local, strided)")
+                status = self._calls.h2x_bn_forward_local_strided(
+                    lx.dtype, ns, lx.geometry_address, _tensor_geometry(ly, ns), input.get_base_ptr(), scale, bias,
+                    per_sum, self.decay, self.epsilon, mean, var, running_mean, running_var, output.get_base_ptr(),
+                    self._ws(lx.channels), _stream_handle(self.stream))
+            if status:
+                capi.check(status, "bn forward (local)")
             return 0
         self.forward_stage1(input, mean, var, is_training)
         self.forward_allreduce(mean, var, is_training)
@@ -250,23 +220,19 @@ class BatchNormalization:
     # ---- backward ----------------------------------------------------------
     def backward_stage1(self, input: Tensor, d_output: Tensor, mean, var, scale, scale_gradient,
                         bias_gradient, mean_gradient, var_gradient) -> int:
-        self.set_num_samples(input.local_shape[-1])
-        n, c, s, sr = _channel_geometry(input)
-        _, _, _, sro = _channel_geometry(d_output)
-        active = input.is_split_root() and input.get_local_size() > 0
-        ns = self.num_current_samples if active else 0
-        tail = (_ptr(mean), _ptr(var), _ptr(scale), _ptr(scale_gradient), _ptr(bias_gradient),
-                _ptr(mean_gradient), _ptr(var_gradient), self.epsilon, _ptr(self._ws(c)),
-                _stream_handle(self.stream))
-        if _is_dense(input) and _is_dense(d_output):
-            capi.check(self._lib.h2x_bn_backprop1(
-                input.h2x_dtype, ns, c, s, sr, sro, _ptr(input.get_base_ptr()),
-                _ptr(d_output.get_base_ptr()), *tail), "backprop1")
+        lx, ld = _dense_layout(input), _dense_layout(d_output)
+        self.num_current_samples = lx.samples
+        ns = lx.samples if lx.active else 0
+        tail = (mean, var, scale, scale_gradient, bias_gradient, mean_gradient, var_gradient, self.epsilon,
+                self._ws(lx.channels), _stream_handle(self.stream))
+        if lx.dense and ld.dense:
+            capi.check(self._calls.h2x_bn_backprop1(
+                lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ld.spatial_real, input.get_base_ptr(),
+                d_output.get_base_ptr(), *tail), "backprop1")
         else:
-            gx, gd = _tensor_geometry(input, ns), _tensor_geometry(d_output, ns)
-            capi.check(self._lib.h2x_bn_backprop1_strided(
-                input.h2x_dtype, ns, ctypes.byref(gx), ctypes.byref(gd), _ptr(input.get_base_ptr()),
-                _ptr(d_output.get_base_ptr()), *tail), "backprop1 (strided)")
+            capi.check(self._calls.h2x_bn_backprop1_strided(
+                lx.dtype, ns, _tensor_geometry(lx, ns), _tensor_geometry(ld, ns), input.get_base_ptr(),
+                d_output.get_base_ptr(), *tail), "backprop1 (strided)")
         return 0
 
     def backward_allreduce(self, scale_gradient, bias_gradient, mean_gradient, var_gradient,
@@ -281,52 +247,47 @@ class BatchNormalization:
 
     def backward_stage2(self, input: Tensor, d_output: Tensor, mean, var, scale, mean_gradient,
                         var_gradient, d_input: Tensor) -> int:
-        n, c, s, sr = _channel_geometry(input)
-        _, _, _, sro = _channel_geometry(d_output)
-        _, _, _, sri = _channel_geometry(d_input)
+        lx, ld, li = _dense_layout(input), _dense_layout(d_output), _dense_layout(d_input)
         ns = self.num_current_samples
-        tail = (_ptr(input.get_base_ptr()), _ptr(d_output.get_base_ptr()), _ptr(mean), _ptr(var),
-                _ptr(scale), _ptr(mean_gradient), _ptr(var_gradient), _ptr(d_input.get_base_ptr()),
-                self.epsilon, _stream_handle(self.stream))
-        if self.clear_output_halo and ns == n and _share_a_haloed_geometry(input, d_output, d_input):
-            g = _haloed_geometry(d_input)
-            capi.check(self._lib.h2x_bn_backprop2_clearing(
-                input.h2x_dtype, self._num_per_sum(input), ctypes.byref(g), _ptr(input.get_buffer()),
-                _ptr(d_output.get_buffer()), _ptr(mean), _ptr(var), _ptr(scale), _ptr(mean_gradient),
-                _ptr(var_gradient), _ptr(d_input.get_buffer()), self.epsilon, _stream_handle(self.stream)),
-                "backprop2 (clearing)")
+        tail = (input.get_base_ptr(), d_output.get_base_ptr(), mean, var, scale, mean_gradient, var_gradient,
+                d_input.get_base_ptr(), self.epsilon, _stream_handle(self.stream))
+        if self.clear_output_halo and ns == lx.samples and _share_a_haloed_geometry(lx, ld, li):
+            capi.check(self._calls.h2x_bn_backprop2_clearing(
+                lx.dtype, self._num_per_sum(input), li.haloed_geometry_address, input.get_buffer(),
+                d_output.get_buffer(), mean, var, scale, mean_gradient, var_gradient, d_input.get_buffer(),
+                self.epsilon, _stream_handle(self.stream)), "backprop2 (clearing)")
         # the reference takes its fast path only for halo-free tensors (batchnorm.cu:1503-1506)
-        elif _is_dense(input) and _is_dense(d_output) and _is_dense(d_input):
-            capi.check(self._lib.h2x_bn_backprop2(
-                input.h2x_dtype, ns, c, s, sr, sro, sri, self._num_per_sum(input), *tail), "backprop2")
+        elif lx.dense and ld.dense and li.dense:
+            capi.check(self._calls.h2x_bn_backprop2(
+                lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ld.spatial_real, li.spatial_real,
+                self._num_per_sum(input), *tail), "backprop2")
         else:
-            gx, gd, gi = (_tensor_geometry(t, ns) for t in (input, d_output, d_input))
-            capi.check(self._lib.h2x_bn_backprop2_strided(
-                input.h2x_dtype, ns, self._num_per_sum(input), ctypes.byref(gx), ctypes.byref(gd),
-                ctypes.byref(gi), *tail), "backprop2 (strided)")
+            capi.check(self._calls.h2x_bn_backprop2_strided(
+                lx.dtype, ns, self._num_per_sum(input), _tensor_geometry(lx, ns), _tensor_geometry(ld, ns),
+                _tensor_geometry(li, ns), *tail), "backprop2 (strided)")
         return 0
 
     def backward(self, input, d_output, mean, var, scale, scale_gradient, bias_gradient,
                  mean_gradient, var_gradient, d_input) -> int:
-        if self._runs_local(input, d_output, d_input):
-            self.set_num_samples(input.local_shape[-1])
-            n, c, s, sr = _channel_geometry(input)
-            _, _, _, sro = _channel_geometry(d_output)
-            _, _, _, sri = _channel_geometry(d_input)
-            tail = (_ptr(input.get_base_ptr()), _ptr(d_output.get_base_ptr()), _ptr(mean), _ptr(var),
-                    _ptr(scale), _ptr(scale_gradient), _ptr(bias_gradient), _ptr(mean_gradient),
-                    _ptr(var_gradient), _ptr(d_input.get_base_ptr()), self.epsilon, _ptr(self._ws(c)),
-                    _stream_handle(self.stream))
-            if _is_dense(input) and _is_dense(d_output) and _is_dense(d_input):
-                capi.check(self._lib.h2x_bn_backward_local(
-                    input.h2x_dtype, self.num_current_samples, c, s, sr, sro, sri, self._num_per_sum(input),
-                    *tail), "bn backward (local)")
+        lx, ld, li = input.layout, d_output.layout, d_input.layout
+        if self._runs_local(lx, lx.haloed or ld.haloed or li.haloed):
+            _dense_layout(input), _dense_layout(d_output), _dense_layout(d_input)
+            ns = self.num_current_samples = lx.samples
+            per_sum = lx.per_channel_global if self.global_stats else lx.per_channel_local
+            if lx.dense and ld.dense and li.dense:
+                status = self._calls.h2x_bn_backward_local(
+                    lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ld.spatial_real, li.spatial_real,
+                    per_sum, input.get_base_ptr(), d_output.get_base_ptr(), mean, var, scale, scale_gradient,
+                    bias_gradient, mean_gradient, var_gradient, d_input.get_base_ptr(), self.epsilon,
+                    self._ws(lx.channels), _stream_handle(self.stream))
             else:
-                ns = self.num_current_samples
-                gx, gd, gi = (_tensor_geometry(t, ns) for t in (input, d_output, d_input))
-                capi.check(self._lib.h2x_bn_backward_local_strided(
-                    input.h2x_dtype, ns, self._num_per_sum(input), ctypes.byref(gx), ctypes.byref(gd),
-                    ctypes.byref(gi), *tail), "bn backward (local, strided)")
+                status = self._calls.h2x_bn_backward_local_strided(
+                    lx.dtype, ns, per_sum, lx.geometry_address, _tensor_geometry(ld, ns), _tensor_geometry(li, ns),
+                    input.get_base_ptr(), d_output.get_base_ptr(), mean, var, scale, scale_gradient, bias_gradient,
+                    mean_gradient, var_gradient, d_input.get_base_ptr(), self.epsilon, self._ws(lx.channels),
+                    _stream_handle(self.stream))
+            if status:
+                capi.check(status, "bn backward (local)")
             return 0
         self.backward_stage1(input, d_output, mean, var, scale, scale_gradient, bias_gradient,
                              mean_gradient, var_gradient)
@@ -361,11 +322,11 @@ def transform(op: int, tensors: Sequence[Tensor], params: Sequence[float] = (),
             raise ValueError("tensors of a transform must have the same local shape")  # :383-390
     if tensors[0].get_local_size() == 0:
         return
-    geoms = [_local_geometry(t) for t in tensors]
-    gp = (ctypes.POINTER(capi.TensorGeometry) * n)(*[ctypes.pointer(g) for g in geoms])
+    gp = (ctypes.c_void_p * n)(*[t.layout.geometry_address for t in tensors])
     tp = (ctypes.c_void_p * n)(*[t.get_base_ptr() for t in tensors])
     pp = (ctypes.c_double * 4)(*(list(params) + [0.0] * (4 - len(params))))
-    capi.check(capi.load().h2x_tensor_transform(op, tensors[0].h2x_dtype, n, gp, tp, pp, _stream_handle(stream)),
+    capi.check(capi.calls().h2x_tensor_transform(op, tensors[0].h2x_dtype, n, ctypes.addressof(gp),
+                                                 ctypes.addressof(tp), ctypes.addressof(pp), _stream_handle(stream)),
                "tensor transform")
 
 
@@ -381,13 +342,13 @@ def reduce_sum(src: Tensor, dst: Tensor, square: bool = False, region: Optional[
     lib = capi.load()
     gs, gd = _local_geometry(src, region), _local_geometry(dst)
     need = lib.h2x_tensor_reduce_sum_workspace_bytes(ctypes.byref(gs), ctypes.byref(gd))
-    key = torch.cuda.current_stream().cuda_stream if stream is None else stream.cuda_stream
+    key = _stream_handle(stream)
     ws = _reduce_workspaces.get(key)
     if ws is None or ws.numel() < need:
         ws = _reduce_workspaces[key] = _device_buffer(max(need, 256), torch.uint8)
-    capi.check(lib.h2x_tensor_reduce_sum(src.h2x_dtype, ctypes.byref(gs), ctypes.c_void_p(src.get_base_ptr()),
-                                         ctypes.byref(gd), ctypes.c_void_p(dst.get_base_ptr()), int(square),
-                                         ctypes.c_void_p(ws.data_ptr()), _stream_handle(stream)), "tensor reduce_sum")
+    capi.check(capi.calls().h2x_tensor_reduce_sum(src.h2x_dtype, ctypes.addressof(gs), src.get_base_ptr(),
+                                                  ctypes.addressof(gd), dst.get_base_ptr(), int(square), ws, key),
+               "tensor reduce_sum")
 
 
 class SoftmaxMode(Enum):
@@ -409,17 +370,19 @@ class Softmax:
         self.stream, self.allreduce = stream, allreduce
         self.mode = SoftmaxMode.CHANNEL
         self._lib = capi.load()
+        self._calls = capi.calls()
         self._ws: Optional[torch.Tensor] = None
+        self._scalars: Optional[torch.Tensor] = None
 
     def setup(self, input: Tensor, mode: SoftmaxMode) -> None:
         self.mode = mode
 
     @staticmethod
-    def _geometry(t: Tensor):
-        if any(t.overlap):
+    def _geometry(t: Tensor) -> Layout:
+        l = t.layout
+        if l.haloed:
             raise NotImplementedError("softmax assumes a dense local tensor")  # softmax.cu:562-563
-        nd = t.get_num_dims()
-        return t.local_shape[nd - 1], t.local_shape[nd - 2], _prod(t.local_shape[: nd - 2])
+        return l
 
     def _workspace(self, n: int) -> torch.Tensor:
         need = self._lib.h2x_softmax_instance_workspace_bytes(n)
@@ -427,60 +390,70 @@ class Softmax:
             self._ws = _device_buffer(need, torch.uint8)
         return self._ws
 
+    def _sample_scalars(self, t: Tensor, count: int) -> torch.Tensor:
+        """`count` scalars of t's type that nobody reads after the call: kept like the workspace."""
+        b = self._scalars
+        if b is None or b.dtype != t.dtype or b.numel() < count:
+            b = self._scalars = _device_buffer(count, t.dtype)
+        return b
+
     def forward(self, x: Tensor, y: Tensor) -> int:
-        n, c, s = self._geometry(x)
+        l = self._geometry(x)
+        n = l.samples
         if n == 0:
             return 0
         st = _stream_handle(self.stream)
         if self.mode == SoftmaxMode.CHANNEL:
-            capi.check(self._lib.h2x_softmax_channel_forward(
-                x.h2x_dtype, n, c, s, _ptr(x.get_base_ptr()), _ptr(y.get_base_ptr()), st), "softmax forward")
+            status = self._calls.h2x_softmax_channel_forward(
+                l.dtype, n, l.channels, l.spatial, x.get_base_ptr(), y.get_base_ptr(), st)
+            if status:
+                capi.check(status, "softmax forward")
             return 0
         # instance mode: softmax.cu:723-746
-        dt, size, ws = x.h2x_dtype, c * s, self._workspace(n)
-        smax = torch.empty(n, dtype=x.dtype, device=x.device)
-        sexp = torch.empty(n, dtype=x.dtype, device=x.device)
+        calls, dt, size, ws = self._calls, l.dtype, l.channels * l.spatial, self._workspace(n)
         if self.allreduce is None:
             # every sample is whole on this rank: the stages need not be separate calls
-            capi.check(self._lib.h2x_softmax_instance_forward_local(
-                dt, n, size, _ptr(x.get_base_ptr()), _ptr(y.get_base_ptr()), _ptr(smax), _ptr(sexp), _ptr(ws), st),
-                "softmax instance forward")
+            scalars = self._sample_scalars(x, 2 * n).data_ptr()
+            status = calls.h2x_softmax_instance_forward_local(
+                dt, n, size, x.get_base_ptr(), y.get_base_ptr(), scalars,
+                scalars + n * self._scalars.element_size(), ws, st)
+            if status:
+                capi.check(status, "softmax instance forward")
             return 0
-        capi.check(self._lib.h2x_softmax_instance_max(dt, n, size, _ptr(x.get_base_ptr()), _ptr(smax),
-                                                      _ptr(ws), st), "softmax instance max")
-        if self.allreduce:
-            self.allreduce(smax, True)
-        capi.check(self._lib.h2x_softmax_instance_exp(dt, n, size, _ptr(x.get_base_ptr()), _ptr(smax),
-                                                      _ptr(y.get_base_ptr()), _ptr(sexp), _ptr(ws), st),
-                   "softmax instance exp")
-        if self.allreduce:
-            self.allreduce(sexp, False)
-        capi.check(self._lib.h2x_softmax_instance_normalize(dt, n, size, _ptr(sexp), _ptr(y.get_base_ptr()), st),
+        smax = torch.empty(n, dtype=x.dtype, device=x.device)
+        sexp = torch.empty(n, dtype=x.dtype, device=x.device)
+        capi.check(calls.h2x_softmax_instance_max(dt, n, size, x.get_base_ptr(), smax, ws, st),
+                   "softmax instance max")
+        self.allreduce(smax, True)
+        capi.check(calls.h2x_softmax_instance_exp(dt, n, size, x.get_base_ptr(), smax, y.get_base_ptr(), sexp, ws,
+                                                  st), "softmax instance exp")
+        self.allreduce(sexp, False)
+        capi.check(calls.h2x_softmax_instance_normalize(dt, n, size, sexp, y.get_base_ptr(), st),
                    "softmax instance normalize")
         return 0
 
     def backward(self, y: Tensor, dy: Tensor, dx: Tensor) -> int:
-        n, c, s = self._geometry(dx)
+        l = self._geometry(dx)
+        n, dt = l.samples, y.layout.dtype
         if n == 0:
             return 0
         st = _stream_handle(self.stream)
         if self.mode == SoftmaxMode.CHANNEL:
-            capi.check(self._lib.h2x_softmax_channel_backward(
-                y.h2x_dtype, n, c, s, _ptr(y.get_base_ptr()), _ptr(dy.get_base_ptr()),
-                _ptr(dx.get_base_ptr()), st), "softmax backward")
+            status = self._calls.h2x_softmax_channel_backward(
+                dt, n, l.channels, l.spatial, y.get_base_ptr(), dy.get_base_ptr(), dx.get_base_ptr(), st)
+            if status:
+                capi.check(status, "softmax backward")
             return 0
         # instance mode: softmax.cu:770-783
-        dt, size, ws = y.h2x_dtype, c * s, self._workspace(n)
-        sdp = torch.empty(n, dtype=y.dtype, device=y.device)
-        capi.check(self._lib.h2x_softmax_instance_dot(dt, n, size, _ptr(y.get_base_ptr()),
-                                                      _ptr(dy.get_base_ptr()), _ptr(sdp), _ptr(ws), st),
+        calls, size, ws = self._calls, l.channels * l.spatial, self._workspace(n)
+        sdp = (self._sample_scalars(y, n) if self.allreduce is None
+               else torch.empty(n, dtype=y.dtype, device=y.device))
+        capi.check(calls.h2x_softmax_instance_dot(dt, n, size, y.get_base_ptr(), dy.get_base_ptr(), sdp, ws, st),
                    "softmax instance dot")
         if self.allreduce:
             self.allreduce(sdp, False)
-        capi.check(self._lib.h2x_softmax_instance_gradient(dt, n, size, _ptr(y.get_base_ptr()),
-                                                           _ptr(dy.get_base_ptr()), _ptr(sdp),
-                                                           _ptr(dx.get_base_ptr()), st),
-                   "softmax instance gradient")
+        capi.check(calls.h2x_softmax_instance_gradient(dt, n, size, y.get_base_ptr(), dy.get_base_ptr(), sdp,
+                                                       dx.get_base_ptr(), st), "softmax instance gradient")
         return 0
 
 
@@ -510,6 +483,7 @@ class HaloExchangeVirtual:
         self.tensors = list(tensors)
         self.periodic, self.stream = periodic, stream
         self._lib = capi.load()
+        self._calls = capi.calls()
         t0 = self.tensors[0]
         self.dist = t0.dist
         if len(self.tensors) != self.dist.num_ranks:
@@ -518,7 +492,7 @@ class HaloExchangeVirtual:
             raise NotImplementedError("shared (replicated) distributions are not exchanged")  # :30-31
         self.nd = t0.get_num_dims()
         self._recv = {}  # (rank, dim, side) -> torch buffer the rank unpacks from
-        self._faces = {}  # exchange arguments -> (pack faces, unpack faces)
+        self._faces = {}  # exchange arguments and addresses -> launches (label, entry point, descriptors)
         # optional callable(label, launch, num_faces): wraps every launch, for per-kernel timing
         self.launch_hook = None
 
@@ -564,7 +538,7 @@ class HaloExchangeVirtual:
     def _addresses(self):
         """Device addresses the cached face tables were built for; a tensor that
         was reallocated gets new tables."""
-        return tuple(t.get_buffer() if t.data is not None else 0 for t in self.tensors)
+        return tuple([t.data.data_ptr() if t.data is not None else 0 for t in self.tensors])
 
     def recv_buffer(self, rank: int, dim: int, side: int) -> torch.Tensor:
         """The buffer rank `rank` unpacks its (dim, side) halo from -- and its
@@ -598,101 +572,95 @@ class HaloExchangeVirtual:
         neighbour's LHS receive buffer and vice versa.  With ``fused`` the strips
         move straight from tensor to tensor in one launch per group of ranks;
         the result is the same."""
-        dtype = self.tensors[0].h2x_dtype
-        self._check_widths(dim, (width_rhs_send, width_rhs_recv, width_lhs_send, width_lhs_recv))
-        if fused:
-            if skip_unpack:
-                raise ValueError("a fused exchange has no separate unpack to skip")
-            self._exchange_dim_fused(dim, width_rhs_send, width_rhs_recv, width_lhs_send,
-                                     width_lhs_recv, is_reverse, op)
-            return
-        key = (dim, width_rhs_send, width_rhs_recv, width_lhs_send, width_lhs_recv, is_reverse,
-               skip_unpack, op, self._addresses())
-        cached = self._faces.get(key)
-        if cached is None:
-            widths = (width_rhs_send, width_rhs_recv, width_lhs_send, width_lhs_recv)
-            cached = []
-            for group in self._rank_groups(dim, max(widths)):
-                packs, unpacks = [], []
-                for r in group:
-                    if not self.is_exchange_required(r, dim, widths):
-                        continue
-                    for side in (capi.LHS, capi.RHS):
-                        peer = self.find_peer_rank(r, dim, side)
-                        if peer is None:
-                            continue
-                        w_send = width_rhs_send if side == capi.RHS else width_lhs_send
-                        w_recv = width_rhs_recv if side == capi.RHS else width_lhs_recv
-                        if w_send > 0:
-                            dst = self.recv_buffer(peer, dim, capi.LHS if side == capi.RHS else capi.RHS)
-                            packs.append(self.make_face(r, dim, side, w_send, dst, True, is_reverse, op))
-                        if w_recv > 0 and not skip_unpack:
-                            src = self.recv_buffer(r, dim, side)
-                            unpacks.append(self.make_face(r, dim, side, w_recv, src, False, is_reverse, op))
-                # the face tables depend only on the arguments and on the tensors'
-                # addresses (part of the key): build them once
-                cached.append(tuple((capi.HaloFace * len(f))(*f) if f else None for f in (packs, unpacks)))
-            self._faces[key] = cached
-        st = _stream_handle(self.stream)
-        for group in cached:
-            for what, arr in zip(("pack", "unpack"), group):
-                if arr is None:
-                    continue
-                launch = lambda arr=arr: capi.check(
-                    self._lib.h2x_halo_pack_or_unpack_batched(dtype, arr, len(arr), st), "halo pack/unpack")
-                if self.launch_hook is None:
-                    launch()
-                else:
-                    self.launch_hook(f"halo_dim{dim}_{what}", launch, len(arr))
+        self._issue(self._dim_launches(dim, width_rhs_send, width_rhs_recv, width_lhs_send, width_lhs_recv,
+                                       is_reverse, skip_unpack, op, fused))
 
-    def _exchange_dim_fused(self, dim, width_rhs_send, width_rhs_recv, width_lhs_send,
-                            width_lhs_recv, is_reverse, op) -> None:
-        dtype = self.tensors[0].h2x_dtype
-        widths = (width_rhs_send, width_rhs_recv, width_lhs_send, width_lhs_recv)
-        key = ("fused", dim) + widths + (is_reverse, op, self._addresses())
-        cached = self._faces.get(key)
-        if cached is None:
-            cached = []
-            # one launch for all ranks: nothing is read back between two launches
-            # here, so groups would only add launches (measured: 289 us against 301 us)
-            for group in [range(len(self.tensors))]:
-                moves = []
-                for r in group:  # r receives; both of its halos are neighbours in the table
-                    if not self.is_exchange_required(r, dim, widths):
-                        continue
-                    for side in (capi.LHS, capi.RHS):
-                        peer = self.find_peer_rank(r, dim, side)
-                        if peer is None:
-                            continue
-                        # what the peer sends towards r leaves the peer on the opposite side
-                        w_send = width_lhs_send if side == capi.RHS else width_rhs_send
-                        w_recv = width_rhs_recv if side == capi.RHS else width_lhs_recv
-                        if w_send != w_recv:
-                            raise ValueError("a fused exchange needs equal send and receive widths")
-                        if w_recv == 0:
-                            continue
-                        src, dst = self.tensors[peer], self.tensors[r]
-                        m = capi.HaloTransfer()
-                        m.src, m.dst = src.get_buffer(), dst.get_buffer()
-                        for i in range(self.nd):
-                            m.src_real_shape[i] = src.local_real_shape[i]
-                            m.dst_real_shape[i] = dst.local_real_shape[i]
-                        m.num_dims, m.dim, m.width = self.nd, dim, w_recv
-                        m.src_side = capi.LHS if side == capi.RHS else capi.RHS
-                        m.is_reverse, m.op = int(is_reverse), op.value
-                        moves.append(m)
-                cached.append((capi.HaloTransfer * len(moves))(*moves) if moves else None)
-            self._faces[key] = cached
-        st = _stream_handle(self.stream)
-        for arr in cached:
-            if arr is None:
-                continue
-            launch = lambda arr=arr: capi.check(
-                self._lib.h2x_halo_exchange_fused(dtype, arr, len(arr), st), "fused halo exchange")
+    def _issue(self, launches) -> None:
+        """Launches in order: (label, entry point, array of descriptors)."""
+        dtype, st = self.tensors[0].h2x_dtype, _stream_handle(self.stream)
+        for label, call, arr in launches:
             if self.launch_hook is None:
-                launch()
+                status = call(dtype, ctypes.addressof(arr), len(arr), st)
+                if status:
+                    capi.check(status, label)
             else:
-                self.launch_hook(f"halo_dim{dim}_fused", launch, len(arr))
+                self.launch_hook(label, lambda label=label, call=call, arr=arr: capi.check(
+                    call(dtype, ctypes.addressof(arr), len(arr), st), label), len(arr))
+
+    def _dim_launches(self, dim, width_rhs_send, width_rhs_recv, width_lhs_send, width_lhs_recv, is_reverse,
+                      skip_unpack, op, fused):
+        """The launches of one dimension's exchange.  They depend only on the arguments and on
+        the tensors' addresses: built once."""
+        widths = (width_rhs_send, width_rhs_recv, width_lhs_send, width_lhs_recv)
+        self._check_widths(dim, widths)
+        if fused and skip_unpack:
+            raise ValueError("a fused exchange has no separate unpack to skip")
+        key = (dim, widths, is_reverse, skip_unpack, op, fused, self._addresses())
+        launches = self._faces.get(key)
+        if launches is None:
+            build = self._fused_launches if fused else self._staged_launches
+            launches = self._faces[key] = build(dim, widths, is_reverse, skip_unpack, op)
+        return launches
+
+    def _staged_launches(self, dim, widths, is_reverse, skip_unpack, op):
+        width_rhs_send, width_rhs_recv, width_lhs_send, width_lhs_recv = widths
+        launches = []
+        for group in self._rank_groups(dim, max(widths)):
+            packs, unpacks = [], []
+            for r in group:
+                if not self.is_exchange_required(r, dim, widths):
+                    continue
+                for side in (capi.LHS, capi.RHS):
+                    peer = self.find_peer_rank(r, dim, side)
+                    if peer is None:
+                        continue
+                    w_send = width_rhs_send if side == capi.RHS else width_lhs_send
+                    w_recv = width_rhs_recv if side == capi.RHS else width_lhs_recv
+                    if w_send > 0:
+                        dst = self.recv_buffer(peer, dim, capi.LHS if side == capi.RHS else capi.RHS)
+                        packs.append(self.make_face(r, dim, side, w_send, dst, True, is_reverse, op))
+                    if w_recv > 0 and not skip_unpack:
+                        src = self.recv_buffer(r, dim, side)
+                        unpacks.append(self.make_face(r, dim, side, w_recv, src, False, is_reverse, op))
+            for what, faces in (("pack", packs), ("unpack", unpacks)):
+                if faces:
+                    launches.append((f"halo_dim{dim}_{what}", self._calls.h2x_halo_pack_or_unpack_batched,
+                                     (capi.HaloFace * len(faces))(*faces)))
+        return launches
+
+    def _fused_launches(self, dim, widths, is_reverse, skip_unpack, op):
+        # one launch for all ranks: nothing is read back between two launches
+        # here, so groups would only add launches (measured: 289 us against 301 us)
+        width_rhs_send, width_rhs_recv, width_lhs_send, width_lhs_recv = widths
+        moves = []
+        for r in range(len(self.tensors)):  # r receives; both of its halos are neighbours in the table
+            if not self.is_exchange_required(r, dim, widths):
+                continue
+            for side in (capi.LHS, capi.RHS):
+                peer = self.find_peer_rank(r, dim, side)
+                if peer is None:
+                    continue
+                # what the peer sends towards r leaves the peer on the opposite side
+                w_send = width_lhs_send if side == capi.RHS else width_rhs_send
+                w_recv = width_rhs_recv if side == capi.RHS else width_lhs_recv
+                if w_send != w_recv:
+                    raise ValueError("a fused exchange needs equal send and receive widths")
+                if w_recv == 0:
+                    continue
+                src, dst = self.tensors[peer], self.tensors[r]
+                m = capi.HaloTransfer()
+                m.src, m.dst = src.get_buffer(), dst.get_buffer()
+                for i in range(self.nd):
+                    m.src_real_shape[i] = src.local_real_shape[i]
+                    m.dst_real_shape[i] = dst.local_real_shape[i]
+                m.num_dims, m.dim, m.width = self.nd, dim, w_recv
+                m.src_side = capi.LHS if side == capi.RHS else capi.RHS
+                m.is_reverse, m.op = int(is_reverse), op.value
+                moves.append(m)
+        if not moves:
+            return []
+        return [(f"halo_dim{dim}_fused", self._calls.h2x_halo_exchange_fused,
+                 (capi.HaloTransfer * len(moves))(*moves))]
 
     # Faces of the innermost dimension touch one short run per row, and every
     # run costs a whole 128-byte line of memory traffic; the unpack writes into
@@ -735,12 +703,18 @@ class HaloExchangeVirtual:
         """All dimensions, innermost first, each seeing the halo cells the previous
         ones filled (halo_exchange_cuda.hpp:56-106)."""
         ov = self.tensors[0].overlap
-        wrs = ov if widths_rhs_send is None else widths_rhs_send
-        wrr = ov if widths_rhs_recv is None else widths_rhs_recv
-        wls = ov if widths_lhs_send is None else widths_lhs_send
-        wlr = ov if widths_lhs_recv is None else widths_lhs_recv
-        for d in range(self.nd):
-            self.exchange_dim(d, wrs[d], wrr[d], wls[d], wlr[d], is_reverse, skip_unpack, op, fused)
+        given = (widths_rhs_send, widths_rhs_recv, widths_lhs_send, widths_lhs_recv)
+        widths = tuple([ov if w is None else w for w in given])
+        if fused and skip_unpack:
+            raise ValueError("a fused exchange has no separate unpack to skip")
+        key = ("all", None if given == (None,) * 4 else tuple(map(tuple, widths)), is_reverse, skip_unpack, op, fused, self._addresses())
+        launches = self._faces.get(key)
+        if launches is None:
+            launches = []
+            for d in range(self.nd):
+                launches += self._dim_launches(d, *(w[d] for w in widths), is_reverse, skip_unpack, op, fused)
+            self._faces[key] = launches
+        self._issue(launches)
 
     def clear_halo(self, dim: int) -> None:
         """Tensor::clear_halo (legacy/src/tensor/tensor_mpi_cuda.cu:14-84) on every rank."""
@@ -748,10 +722,8 @@ class HaloExchangeVirtual:
             if t.overlap[dim] == 0 or t.get_local_size() == 0:
                 continue
             shape = capi.i64_array(t.local_real_shape)
-            capi.check(self._lib.h2x_halo_clear(t.h2x_dtype, _ptr(t.get_buffer()), self.nd, shape,
-                                                dim, t.overlap[dim], _stream_handle(self.stream)),
-                       "clear_halo")
-
+            capi.check(self._calls.h2x_halo_clear(t.h2x_dtype, t.get_buffer(), self.nd, ctypes.addressof(shape),
+                                                  dim, t.overlap[dim], _stream_handle(self.stream)), "clear_halo")
 
     def clear_halos(self, only_unfilled: bool = False) -> None:
         """clear_halo of every dimension that has a halo, on every rank, in batched
@@ -787,8 +759,8 @@ class HaloExchangeVirtual:
             self._faces[key] = (capi.HaloFace * len(faces))(*faces)
         arr = self._faces[key]
         if len(arr):
-            capi.check(self._lib.h2x_halo_clear_batched(self.tensors[0].h2x_dtype, arr, len(arr),
-                                                        _stream_handle(self.stream)), "clear_halos")
+            capi.check(self._calls.h2x_halo_clear_batched(self.tensors[0].h2x_dtype, ctypes.addressof(arr), len(arr),
+                                                          _stream_handle(self.stream)), "clear_halos")
 
 
 class TensorShufflerVirtual:
@@ -807,6 +779,8 @@ class TensorShufflerVirtual:
                  stream: Optional[torch.cuda.Stream] = None):
         self.src, self.dst, self.stream = list(src_tensors), list(dst_tensors), stream
         self._lib = capi.load()
+        self._calls = capi.calls()
+        self._arguments = {}  # addresses of a launch's tensors -> its argument arrays
         if len(self.src) != len(self.dst):
             raise ValueError("source and destination must have the same number of ranks")
         self.num_ranks = len(self.src)
@@ -896,26 +870,34 @@ class TensorShufflerVirtual:
         return plan
 
     def _launch(self, fn, plans, tensors: List[Tensor], arena: torch.Tensor) -> None:
-        live = [(p, t) for p, t in zip(plans, tensors) if p is not None]
+        live = [t for p, t in zip(plans, tensors) if p is not None]
         if not live:
             return
         n = len(live)
-        pa = (ctypes.c_void_p * n)(*[p for p, _ in live])
-        ta = (ctypes.c_void_p * n)(*[t.get_base_ptr() for _, t in live])
-        ba = (ctypes.c_void_p * n)(*[arena.data_ptr()] * n)
-        capi.check(fn(pa, ta, ba, n, _stream_handle(self.stream)), "shuffle")
+        # the argument arrays depend only on the tensors' addresses: kept until one is reallocated
+        addresses = [t.get_base_ptr() for t in live]
+        key = (id(fn), id(plans))
+        kept = self._arguments.get(key)
+        if kept is None or kept[0] != addresses:
+            pa = (ctypes.c_void_p * n)(*[p for p in plans if p is not None])
+            ta = (ctypes.c_void_p * n)(*addresses)
+            ba = (ctypes.c_void_p * n)(*[arena.data_ptr()] * n)
+            kept = self._arguments[key] = (addresses, pa, ta, ba)
+        _, pa, ta, ba = kept
+        capi.check(fn(ctypes.addressof(pa), ctypes.addressof(ta), ctypes.addressof(ba), n,
+                      _stream_handle(self.stream)), "shuffle")
 
     def shuffle_forward(self) -> None:
         """src tensors -> dst tensors (shuffle_mpi_cuda.cu:478-484)."""
         d = self._fwd
-        self._launch(self._lib.h2x_shuffle_pack_batched, d["pack"], self.src, d["arena"])
-        self._launch(self._lib.h2x_shuffle_unpack_batched, d["unpack"], self.dst, d["arena"])
+        self._launch(self._calls.h2x_shuffle_pack_batched, d["pack"], self.src, d["arena"])
+        self._launch(self._calls.h2x_shuffle_unpack_batched, d["unpack"], self.dst, d["arena"])
 
     def shuffle_backward(self) -> None:
         """dst tensors -> src tensors (shuffle_mpi_cuda.cu:485-490)."""
         d = self._bwd
-        self._launch(self._lib.h2x_shuffle_pack_batched, d["pack"], self.dst, d["arena"])
-        self._launch(self._lib.h2x_shuffle_unpack_batched, d["unpack"], self.src, d["arena"])
+        self._launch(self._calls.h2x_shuffle_pack_batched, d["pack"], self.dst, d["arena"])
+        self._launch(self._calls.h2x_shuffle_unpack_batched, d["unpack"], self.src, d["arena"])
 
     def __del__(self):
         try:

@@ -10,7 +10,9 @@ reversed (outermost first) order.
 """
 from __future__ import annotations
 
+import ctypes
 import math
+from functools import cached_property
 from typing import Iterable, List, Optional, Sequence
 
 import torch
@@ -118,6 +120,50 @@ def _block_start(extent: int, parts: int, index: int) -> int:
 _TORCH_DTYPES = {torch.float32: capi.F32, torch.float64: capi.F64}
 
 
+class Layout:
+    """What a layer call needs to know about a local tensor besides its address.  Shape,
+    distribution and type of a Tensor are fixed when it is made, so this is worked out once
+    (a layer call that launches a kernel of a few microseconds cannot afford it every time)."""
+
+    __slots__ = ("samples", "channels", "spatial", "spatial_real", "dense", "haloed", "channel_halo",
+                 "dtype", "active", "geometry", "geometry_address", "per_channel_local", "per_channel_global",
+                 "alike", "_haloed_geometry")
+
+    def __init__(self, t: "Tensor"):
+        nd = t.get_num_dims()
+        self.samples, self.channels = t.local_shape[nd - 1], t.local_shape[nd - 2]
+        self.spatial, self.spatial_real = _prod(t.local_shape[: nd - 2]), _prod(t.local_real_shape[: nd - 2])
+        # no halo on the inner spatial dimensions: the layout the dense entry points take
+        # (legacy/src/dnn_backend/batchnorm.cu:210-219)
+        self.dense = all(t.overlap[d] == 0 for d in range(nd - 3))
+        self.haloed = any(t.overlap)
+        self.channel_halo = t.overlap[nd - 2] != 0 or t.overlap[nd - 1] != 0
+        self.dtype = t.h2x_dtype
+        # a rank that owns elements
+        self.active = t.is_split_root() and t.get_local_size() > 0
+        g = self.geometry = capi.TensorGeometry()
+        g.num_dims = nd
+        for i, (extent, stride) in enumerate(zip(t.local_shape, t.get_strides())):
+            g.local_shape[i], g.strides[i] = extent, stride
+        self.geometry_address = ctypes.addressof(g)
+        # elements per channel of the local and of the global shape
+        self.per_channel_local, self.per_channel_global = (
+            _prod(s) // s[nd - 2] if s[nd - 2] else 0 for s in (t.local_shape, t.shape))
+        # tensors with equal keys lie in memory alike
+        self.alike = (tuple(t.local_shape), tuple(t.local_real_shape), tuple(t.overlap), self.dtype)
+        self._haloed_geometry = None
+
+    @property
+    def haloed_geometry_address(self) -> int:
+        """h2x_haloed_geometry: local and real extents, halo widths."""
+        if self._haloed_geometry is None:
+            g = self._haloed_geometry = capi.HaloedGeometry()
+            g.num_dims = self.geometry.num_dims
+            for i, (local, real, halo) in enumerate(zip(*self.alike[:3])):
+                g.local_shape[i], g.real_shape[i], g.lower_halo[i] = local, real, halo
+        return ctypes.addressof(self._haloed_geometry)
+
+
 class Tensor:
     """Tensor<DataType, LocaleVirtual, device allocator>: global shape plus
     distribution; `allocate()` creates the local real (haloed) buffer."""
@@ -180,6 +226,14 @@ class Tensor:
         si = rank_index // self.dist.get_num_ranks_per_split(dim)
         return _block_start(self.shape[dim], parts, si + 1) - _block_start(self.shape[dim], parts, si)
 
+    @cached_property
+    def layout(self) -> Layout:
+        return Layout(self)
+
+    @cached_property
+    def base_bytes(self) -> int:
+        return self.base_offset() * self.dtype.itemsize
+
     def base_offset(self) -> int:
         return sum(o * s for o, s in zip(self.overlap, self.get_strides()))
 
@@ -198,7 +252,7 @@ class Tensor:
 
     def get_base_ptr(self) -> int:
         """Device address of the first interior element (tensor.hpp:462-481)."""
-        return self.data.data_ptr() + self.base_offset() * self.data.element_size()
+        return self.data.data_ptr() + self.base_bytes
 
     def real_view(self) -> torch.Tensor:
         """The real local tensor as a torch view, outermost dimension first."""
