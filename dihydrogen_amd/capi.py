@@ -15,6 +15,7 @@ LIB_PATH = os.path.join(_HERE, "libh2x.so")
 H2X_MAX_DIMS = 6
 F32, F64 = 0, 1
 LHS, RHS = 0, 1
+HALO_GRID_MAX_RANKS = 16
 HALO_ID, HALO_SUM, HALO_MAX, HALO_MIN = 0, 1, 2, 3
 TRANSFORM_SCALE, TRANSFORM_COPY, TRANSFORM_SCALE_BIAS, TRANSFORM_SUMS_TO_STATISTICS = 0, 1, 2, 3
 
@@ -56,6 +57,18 @@ class HaloTransfer(ctypes.Structure):
         ("is_reverse", c_int32),
         ("op", c_int32),
     ]
+
+
+class HaloGridRank(ctypes.Structure):
+    """struct h2x_halo_grid_rank"""
+    _fields_ = [("tensor", c_void_p), ("local_shape", c_int64 * H2X_MAX_DIMS),
+                ("peer", c_int32 * 2 * H2X_MAX_DIMS)]
+
+
+class HaloGrid(ctypes.Structure):
+    """struct h2x_halo_grid"""
+    _fields_ = [("num_dims", c_int32), ("num_ranks", c_int32), ("overlap", c_int64 * H2X_MAX_DIMS),
+                ("ranks", POINTER(HaloGridRank))]
 
 
 class TensorGeometry(ctypes.Structure):
@@ -226,6 +239,9 @@ SIGNATURES = {
     "h2x_halo_clear": (c_int, [c_int, c_void_p, c_int, POINTER(c_int64), c_int, c_int, c_void_p]),
     "h2x_halo_clear_batched": (c_int, [c_int, POINTER(HaloFace), c_int, c_void_p]),
     "h2x_halo_exchange_fused": (c_int, [c_int, POINTER(HaloTransfer), c_int, c_void_p]),
+    "h2x_halo_grid_exchange": (c_int, [c_int, POINTER(HaloGrid), c_void_p]),
+    "h2x_halo_grid_fold": (c_int, [c_int, POINTER(HaloGrid), c_int, c_void_p]),
+    "h2x_halo_grid_clear": (c_int, [c_int, POINTER(HaloGrid), c_int, c_void_p]),
     "h2x_shuffle_plan_create": (c_int, [POINTER(ShuffleGeometry), POINTER(c_void_p)]),
     "h2x_shuffle_plan_destroy": (c_int, [c_void_p]),
     "h2x_shuffle_pack": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p]),

@@ -1,0 +1,651 @@
+// The forward halo exchange of a whole grid of ranks whose tensors share the
+// device, in one launch, and the clearing of their halos in one launch.
+//
+// The exchange proceeds dimension by dimension in the reference (legacy/include/
+// distconv/tensor/halo_exchange_cuda.hpp:56-106): the strip of a later dimension
+// carries the halo cells that an earlier one has filled.  Where every tensor is
+// addressable that order need not be played out: what ends up in a halo cell is
+// the cell of the rank that is reached by stepping to the neighbour along every
+// dimension in which the cell lies in the halo and a neighbour exists.  Along a
+// dimension without a neighbour the cell keeps its halo coordinate; no phase
+// writes such a cell of the source, so nothing that is read is written here and
+// the whole exchange has no order.  Strips go straight from tensor to tensor.
+//
+// The halo of a rank is cut into regions, one per combination of {interior,
+// lower, upper} of the outer two spatial dimensions, crossed with the two kinds
+// of work along the rows.  "Runs" are the interior of the row in 16-byte vectors
+// that may start on any element; the last vector of a row that is no whole number
+// of vectors starts early and moves a few elements twice.  "Ends" are the halo
+// cells at both ends of the row, for all ranks of a line along dimension 0 in the
+// same thread.  They are bound by whole lines of memory: a cell of 4 bytes costs
+// the read of a 128-byte line and its write-back.  The line of a row seam holds the
+// two halo cells that one rank receives and the two cells that its neighbours take;
+// serving the line of ranks together reads it once and writes it in the L2 that
+// has just read it.  Measured on four ranks of 64 x 256 x 128 x 32 cells with
+// halos of 3: 254 us, one rank per workgroup 300 us; eight ranks of 128^3 x 32
+// (periodic, all dimensions) 273 and 288 us, packing and unpacking 338 us.
+// Nontemporal loads lose the line before the store arrives (387 us).
+//
+// All regions of all ranks are one launch: an exchange of small shards is bound
+// by launches (4 ranks of 29 x 29 x 64 channels x 4 samples, clear and exchange: 14
+// launches 57 us, two 9.4 us).  Descriptors travel in the kernel arguments;
+// nothing is allocated or kept.
+#include "h2x_copy_kernel.hpp"
+
+#include <algorithm>
+
+namespace h2x
+{
+namespace grid
+{
+namespace
+{
+
+using copy::Audit;
+using copy::current_audit;
+using copy::DeviceMem;
+using copy::TraceMem;
+using copy::Words;
+
+constexpr int kMaxRanks = 16;
+constexpr int kMaxSpatial = 3;
+constexpr int kMaxRegions = 9 + 8;
+constexpr int kBlock = 256;
+// Ranks of a line whose ends a thread loads before it stores any (measured: 1, 2, 4; two hold
+// the fewest registers at the rate of four).
+constexpr int kRanksPerTurn = 2;
+
+// Whole words throughout: a byte cannot be read through the scalar cache, and a
+// workgroup spends most of its time before its first access on what it reads here.
+struct Rank
+{
+    char* tensor;                 // start of the real allocation
+    int32_t local[kMaxSpatial];   // interior extents
+    int32_t peer[kMaxSpatial][2]; // rank of the neighbour, or -1
+    FastDiv units;                // by vectors (or elements) of an interior row
+    FastDiv extent[2];            // by local[1], local[2]
+    uint32_t clear;               // bit 2 * d + side: this strip is cleared
+    uint32_t vectors;             // the interior row holds at least one vector
+};
+
+struct Args
+{
+    Rank rank[kMaxRanks];
+    uint32_t first[kMaxRegions]; // first workgroup of a region (beyond the last one: none)
+    uint32_t code[kMaxRegions];  // ends + 4 * digit of dimension 1 + 16 * digit of dimension 2;
+                                 // digits: 0 interior, 1 lower, 2 upper halo
+    FastDiv halo[kMaxSpatial];     // by the halo width (1 where there is none)
+    FastDiv both_ends;             // by twice the halo width of a row
+    FastDiv ranks;                 // by num_ranks
+    FastDiv lines;                 // by the number of lines
+    int32_t line;                  // ranks in a line
+    int32_t width[kMaxSpatial];
+    uint32_t outer; // channels x samples
+};
+
+// Cells of a rank in dimension d (1 or 2) of a region: extent, and the start in
+// the destination and - stepping to `src`, where there is a neighbour - in the
+// source.
+template <bool CLEAR>
+__host__ __device__ __forceinline__ void along(const Args& a, const Rank& me, int d, int digit, int* src, bool* moved,
+                                               FastDiv* div, uint32_t* to, uint32_t* from)
+{
+    const int w = a.width[d], local = me.local[d];
+    *div = digit == 0 ? me.extent[d - 1] : a.halo[d];
+    *to = digit == 0 ? w : digit == 1 ? 0 : w + local;
+    *from = *to;
+    if (digit == 0)
+        return;
+    if constexpr (CLEAR)
+    {
+        *moved = *moved || (me.clear >> (2 * d + digit - 1) & 1);
+    }
+    else
+    {
+        const int p = a.rank[*src].peer[d][digit - 1];
+        if (p >= 0)
+        {
+            *src = p;
+            *moved = true;
+            // the lower halo is the neighbour's last interior cells, the upper one its first
+            *from = digit == 1 ? a.rank[p].local[d] : w;
+        }
+    }
+}
+
+template <typename T, bool CLEAR, typename Mem>
+__host__ __device__ __forceinline__ void body(const Args& a, uint32_t block, uint32_t thread, const Mem& mem)
+{
+    constexpr int VEC = 16 / sizeof(T);
+    using W = typename Words<T, VEC>::unaligned_t;
+    uint32_t first = 0, code = a.code[0];
+#pragma unroll
+    for (int i = 1; i < kMaxRegions; ++i)
+        if (block >= a.first[i])
+        {
+            first = a.first[i];
+            code = a.code[i];
+        }
+    const bool ends = code & 1;
+    // Lines or ranks take turns workgroup by workgroup.
+    const FastDiv& turns = ends ? a.lines : a.ranks;
+    const uint32_t local_block = fastdiv(block - first, turns);
+    const int r = static_cast<int>((block - first - local_block * turns.divisor) * (ends ? a.line : 1));
+    const Rank& me = a.rank[r]; // ends: the first one of its line
+
+    int src = r;
+    bool moved = false; // some dimension has a neighbour to copy from (CLEAR: a strip to clear)
+    FastDiv div_y, div_z;
+    uint32_t y_to, z_to, y_from, z_from;
+    along<CLEAR>(a, me, 1, code >> 2 & 3, &src, &moved, &div_y, &y_to, &y_from);
+    along<CLEAR>(a, me, 2, code >> 4, &src, &moved, &div_z, &z_to, &z_from);
+    const FastDiv div_x = ends ? a.both_ends : me.units;
+    const uint32_t at = local_block * kBlock + thread;
+    if (at >= div_y.divisor * div_z.divisor * a.outer * div_x.divisor || (!ends && !moved))
+        return;
+    const uint32_t row = fastdiv(at, div_x);
+    uint32_t x = at - row * div_x.divisor;
+    const uint32_t yz = fastdiv(row, div_y);
+    const uint32_t y = row - yz * div_y.divisor;
+    const uint32_t o = fastdiv(yz, div_z);
+    const uint32_t z = yz - o * div_z.divisor;
+    // rows of the real tensors (whose elements are fewer than 2^31)
+    const uint32_t w = a.width[0];
+    auto real = [&](int q, int d) { return static_cast<uint32_t>(a.rank[q].local[d] + 2 * a.width[d]); };
+    const uint32_t row_to = (o * real(r, 2) + z_to + z) * real(r, 1) + y_to + y;
+    const uint32_t row_from = (o * real(src, 2) + z_from + z) * real(src, 1) + y_from + y;
+    if (!ends)
+    {
+        T* const to = reinterpret_cast<T*>(me.tensor) + row_to * real(r, 0) + w;
+        const T* const from = reinterpret_cast<const T*>(a.rank[src].tensor) + row_from * real(src, 0) + w;
+        if (me.vectors)
+        {
+            x *= VEC;
+            const uint32_t last = static_cast<uint32_t>(me.local[0]) - VEC;
+            x = x < last ? x : last;
+            W v;
+            if constexpr (CLEAR)
+                v = W(T(0));
+            else
+                v = mem.template load<VEC, false>(from + x);
+            mem.template store<VEC, false>(to + x, v);
+        }
+        else
+        {
+            mem.store1(to + x, CLEAR ? T(0) : mem.load1(from + x));
+        }
+        return;
+    }
+    // The ends of a row in every rank of the line: the lower end's cells, then the upper end's, then
+    // the next row's, so that what neighbouring lanes write at a row seam lies side by side.  `src` is
+    // the first rank of the line that the other dimensions step to.
+    const bool upper = x >= w;
+    const uint32_t j = upper ? x - w : x;
+#pragma unroll 1
+    for (int base = 0; base < a.line; base += kRanksPerTurn)
+    {
+        T v[kRanksPerTurn];
+        bool live[kRanksPerTurn];
+#pragma unroll
+        for (int i = 0; i < kRanksPerTurn; ++i)
+        {
+            live[i] = false;
+            if (base + i >= a.line)
+                continue;
+            if constexpr (CLEAR)
+            {
+                live[i] = moved || (a.rank[r + base + i].clear >> (upper ? 1 : 0) & 1);
+                v[i] = T(0);
+            }
+            else
+            {
+                // from the neighbour's other end of the row; without one from the same end, halo to halo
+                const Rank& same = a.rank[src + base + i];
+                const int lo = same.peer[0][0], hi = same.peer[0][1];
+                const Rank& below = a.rank[lo >= 0 ? lo : src + base + i];
+                const Rank& above = a.rank[hi >= 0 ? hi : src + base + i];
+                live[i] = moved || (upper ? hi : lo) >= 0;
+                const uint32_t at_lo = lo >= 0 ? below.local[0] : 0, at_hi = w + (hi >= 0 ? 0 : above.local[0]);
+                const uint32_t from = row_from * ((upper ? above.local[0] : below.local[0]) + 2 * w)
+                                      + (upper ? at_hi : at_lo) + j;
+                if (live[i])
+                    v[i] = mem.load1(reinterpret_cast<const T*>(upper ? above.tensor : below.tensor) + from);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < kRanksPerTurn; ++i)
+            if (live[i])
+            {
+                const Rank& q = a.rank[r + base + i];
+                mem.store1(reinterpret_cast<T*>(q.tensor)
+                               + (row_to * (q.local[0] + 2 * w) + (upper ? w + q.local[0] : 0) + j),
+                           v[i]);
+            }
+    }
+}
+
+// One dimension of the reverse exchange: the halo strips of `dim` are folded into
+// the boundary cells of the ranks they belong to.  A strip spans the real extents
+// of the other dimensions, so along memory it is runs of `width` times the real
+// extents below `dim`, one per index above it.  A thread serves the same vector of
+// the lower and of the upper strip: four loads in flight, and where `dim` is the
+// innermost dimension the ends of neighbouring rows, which share lines, in one
+// wave.  (Phases of different dimensions stay launches of their own: a later one
+// reads halo cells that an earlier one has added to.)
+template <typename T, typename Op, typename Mem>
+__host__ __device__ __forceinline__ void fold_body(const Args& a, uint32_t block, uint32_t thread, int dim, Op op,
+                                                   const Mem& mem)
+{
+    constexpr int VEC = 16 / sizeof(T);
+    using W = typename Words<T, VEC>::unaligned_t;
+    const uint32_t local_block = fastdiv(block, a.ranks);
+    const int r = static_cast<int>(block - local_block * a.ranks.divisor);
+    const Rank& me = a.rank[r];
+    const int lo = me.peer[dim][0], hi = me.peer[dim][1];
+    // real extents below, along and above the dimension
+    int64_t below = 1, above = a.outer;
+    for (int d = 0; d < kMaxSpatial; ++d)
+    {
+        const int64_t real = me.local[d] + 2 * a.width[d];
+        below *= d < dim ? real : 1;
+        above *= d > dim ? real : 1;
+    }
+    const int64_t w = a.width[dim];
+    const uint32_t run = static_cast<uint32_t>(w * below);
+    const uint32_t at = local_block * kBlock + thread;
+    const uint32_t row = fastdiv(at, me.units);
+    if (row >= above || (lo < 0 && hi < 0))
+        return;
+    auto pitch = [&](int q) { return (a.rank[q].local[dim] + 2 * w) * below; };
+    // the lower boundary cells take the lower neighbour's upper halo, and the other way round
+    T* const to_lo = reinterpret_cast<T*>(me.tensor) + (row * pitch(r) + w * below);
+    T* const to_hi = reinterpret_cast<T*>(me.tensor) + (row * pitch(r) + me.local[dim] * below);
+    const T *from_lo = nullptr, *from_hi = nullptr;
+    if (lo >= 0)
+        from_lo = reinterpret_cast<const T*>(a.rank[lo].tensor) + (row * pitch(lo) + (a.rank[lo].local[dim] + w) * below);
+    if (hi >= 0)
+        from_hi = reinterpret_cast<const T*>(a.rank[hi].tensor) + row * pitch(hi);
+    uint32_t x = at - row * me.units.divisor;
+    uint32_t n = 1;
+    if (me.vectors)
+    {
+        x *= VEC;
+        n = run - x < VEC ? run - x : VEC;
+    }
+    if (n == VEC)
+    {
+        W s0, s1, t0, t1;
+        if (lo >= 0)
+        {
+            s0 = mem.template load<VEC, false>(from_lo + x);
+            t0 = mem.template load<VEC, false>(to_lo + x);
+        }
+        if (hi >= 0)
+        {
+            s1 = mem.template load<VEC, false>(from_hi + x);
+            t1 = mem.template load<VEC, false>(to_hi + x);
+        }
+#pragma unroll
+        for (int j = 0; j < VEC; ++j)
+        {
+            t0[j] = op(t0[j], s0[j]);
+            t1[j] = op(t1[j], s1[j]);
+        }
+        if (lo >= 0)
+            mem.template store<VEC, false>(to_lo + x, t0);
+        if (hi >= 0)
+            mem.template store<VEC, false>(to_hi + x, t1);
+        return;
+    }
+    for (const uint32_t end = x + n; x < end; ++x)
+    {
+        T s0, s1, t0, t1;
+        if (lo >= 0)
+        {
+            s0 = mem.load1(from_lo + x);
+            t0 = mem.load1(to_lo + x);
+        }
+        if (hi >= 0)
+        {
+            s1 = mem.load1(from_hi + x);
+            t1 = mem.load1(to_hi + x);
+        }
+        if (lo >= 0)
+            mem.store1(to_lo + x, op(t0, s0));
+        if (hi >= 0)
+            mem.store1(to_hi + x, op(t1, s1));
+    }
+}
+
+template <typename T, typename Op>
+__global__ __launch_bounds__(kBlock, 8) void halo_fold_kernel(const Args a, int dim, Op op)
+{
+    fold_body<T, Op, DeviceMem>(a, blockIdx.x, threadIdx.x, dim, op, DeviceMem());
+}
+
+template <typename T, typename Op>
+int issue_fold(const Args& a, uint32_t blocks, int dim, hipStream_t stream)
+{
+    if (Audit* const audit = current_audit())
+    {
+        const TraceMem mem{audit};
+        for (uint32_t block = 0; block < blocks; ++block)
+            for (uint32_t thread = 0; thread < kBlock; ++thread)
+                fold_body<T, Op, TraceMem>(a, block, thread, dim, Op(), mem);
+        ++audit->launches;
+        audit->workgroups += blocks;
+        return H2X_SUCCESS;
+    }
+    halo_fold_kernel<T, Op><<<dim3(blocks), kBlock, 0, stream>>>(a, dim, Op());
+    return launch_status();
+}
+
+template <typename T>
+int issue_fold(int op, const Args& a, uint32_t blocks, int dim, hipStream_t stream)
+{
+    switch (op)
+    {
+    case H2X_HALO_ID: return issue_fold<T, copy::OpId>(a, blocks, dim, stream);
+    case H2X_HALO_SUM: return issue_fold<T, copy::OpSum>(a, blocks, dim, stream);
+    case H2X_HALO_MAX: return issue_fold<T, copy::OpMax>(a, blocks, dim, stream);
+    default: return issue_fold<T, copy::OpMin>(a, blocks, dim, stream);
+    }
+}
+
+template <typename T, bool CLEAR>
+__global__ __launch_bounds__(kBlock, 8) void halo_grid_kernel(const Args a)
+{
+    body<T, CLEAR, DeviceMem>(a, blockIdx.x, threadIdx.x, DeviceMem());
+}
+
+template <typename T, bool CLEAR>
+int issue(const Args& a, uint32_t blocks, hipStream_t stream)
+{
+    if (Audit* const audit = current_audit())
+    {
+        const TraceMem mem{audit};
+        for (uint32_t block = 0; block < blocks; ++block)
+            for (uint32_t thread = 0; thread < kBlock; ++thread)
+                body<T, CLEAR, TraceMem>(a, block, thread, mem);
+        ++audit->launches;
+        audit->workgroups += blocks;
+        return H2X_SUCCESS;
+    }
+    halo_grid_kernel<T, CLEAR><<<dim3(blocks), kBlock, 0, stream>>>(a);
+    return launch_status();
+}
+
+// Everything the kernel relies on: extents that fit, neighbours whose tensors
+// lie alike in the other dimensions and hold the strips that are read.
+// `cells`: halo widths of interior that a rank with a neighbour has to have.
+int make_args(const h2x_halo_grid& h, int cells, int only_unfilled, int elem_size, Args* a)
+{
+    const int nd = h.num_dims, ns = nd - 2;
+    if (nd < 3 || nd > kMaxSpatial + 2 || h.num_ranks < 1 || !h.ranks)
+        return H2X_ERR_INVALID_ARGUMENT;
+    if (h.num_ranks > kMaxRanks)
+        return H2X_ERR_UNSUPPORTED;
+    int64_t outer = 1;
+    for (int d = ns; d < nd; ++d)
+    {
+        if (h.overlap[d] != 0)
+            return H2X_ERR_UNSUPPORTED;
+        outer *= h.ranks[0].local_shape[d];
+    }
+    a->ranks = make_fastdiv(static_cast<uint32_t>(h.num_ranks));
+    for (int d = 0; d < kMaxSpatial; ++d)
+    {
+        const int64_t w = d < ns ? h.overlap[d] : 0;
+        if (w < 0 || w > (1 << 20))
+            return H2X_ERR_INVALID_ARGUMENT;
+        a->width[d] = static_cast<int32_t>(w);
+        a->halo[d] = make_fastdiv(static_cast<uint32_t>(std::max<int64_t>(w, 1)));
+    }
+    a->both_ends = make_fastdiv(static_cast<uint32_t>(std::max(2 * a->width[0], 1)));
+    const int64_t vec = 16 / elem_size;
+    for (int r = 0; r < h.num_ranks; ++r)
+    {
+        const h2x_halo_grid_rank& from = h.ranks[r];
+        Rank& k = a->rank[r];
+        if (!from.tensor)
+            return H2X_ERR_INVALID_ARGUMENT;
+        k.tensor = static_cast<char*>(from.tensor);
+        int64_t real = 1;
+        for (int d = 0; d < nd; ++d)
+        {
+            if (from.local_shape[d] < 1 || from.local_shape[d] >= (1ll << 31))
+                return H2X_ERR_INVALID_ARGUMENT;
+            if (d >= ns && from.local_shape[d] != h.ranks[0].local_shape[d])
+                return H2X_ERR_INVALID_ARGUMENT;
+            real *= from.local_shape[d] + 2 * (d < ns ? a->width[d] : 0);
+            if (real >= (1ll << 31))
+                return H2X_ERR_TOO_LARGE;
+        }
+        k.clear = 0;
+        for (int d = 0; d < kMaxSpatial; ++d)
+        {
+            k.local[d] = d < ns ? static_cast<int32_t>(from.local_shape[d]) : 1;
+            for (int side = 0; side < 2; ++side)
+            {
+                const int p = d < ns ? from.peer[d][side] : -1;
+                if (p >= h.num_ranks || p < -1)
+                    return H2X_ERR_INVALID_ARGUMENT;
+                k.peer[d][side] = p;
+                if (p >= 0)
+                {
+                    const h2x_halo_grid_rank& q = h.ranks[p];
+                    if (q.peer[d][1 - side] != r)
+                        return H2X_ERR_INVALID_ARGUMENT;
+                    for (int i = 0; i < nd; ++i)
+                        if (i != d && q.local_shape[i] != from.local_shape[i])
+                            return H2X_ERR_INVALID_ARGUMENT;
+                    if (cells > 0 && (q.local_shape[d] < cells * static_cast<int64_t>(a->width[d]) || a->width[d] == 0))
+                        return H2X_ERR_INVALID_ARGUMENT;
+                }
+                if (a->width[d] > 0 && (p < 0 || !only_unfilled))
+                    k.clear |= 1u << (2 * d + side);
+            }
+        }
+        k.vectors = k.local[0] >= vec;
+        k.units = make_fastdiv(static_cast<uint32_t>(k.vectors ? (k.local[0] + vec - 1) / vec : k.local[0]));
+        k.extent[0] = make_fastdiv(static_cast<uint32_t>(k.local[1]));
+        k.extent[1] = make_fastdiv(static_cast<uint32_t>(k.local[2]));
+    }
+    a->outer = static_cast<uint32_t>(outer);
+    return H2X_SUCCESS;
+}
+
+// Stepping along two dimensions leads to the same rank in either order, and neighbours along one
+// dimension have, or lack, neighbours along the others alike.
+bool is_grid(const Args& a, int num_ranks)
+{
+    for (int r = 0; r < num_ranks; ++r)
+        for (int d = 0; d < kMaxSpatial; ++d)
+            for (int side = 0; side < 2; ++side)
+            {
+                const int p = a.rank[r].peer[d][side];
+                if (p < 0)
+                    continue;
+                for (int e = 0; e < kMaxSpatial; ++e)
+                    for (int s = 0; e != d && s < 2; ++s)
+                    {
+                        const int q = a.rank[r].peer[e][s], pq = a.rank[p].peer[e][s];
+                        if ((q < 0) != (pq < 0) || (q >= 0 && a.rank[q].peer[d][side] != pq))
+                            return false;
+                    }
+            }
+    return true;
+}
+
+// Renumbers the ranks so that those in a line along dimension 0 follow one another, lower to
+// upper; all lines have to be of one length, and a step along another dimension to lead to the
+// same place in another line.
+bool order_into_lines(Args* a, int num_ranks)
+{
+    int order[kMaxRanks], place[kMaxRanks], n = 0;
+    bool taken[kMaxRanks] = {};
+    a->line = 0;
+    for (int closed = 0; closed < 2; ++closed) // open lines start where nothing is below, then rings
+        for (int r = 0; r < num_ranks; ++r)
+        {
+            if (taken[r] || (!closed && a->rank[r].peer[0][0] >= 0))
+                continue;
+            int length = 0;
+            for (int q = r; q >= 0 && !taken[q]; q = a->rank[q].peer[0][1], ++length)
+            {
+                taken[q] = true;
+                place[q] = n;
+                order[n++] = q;
+            }
+            if (a->line != 0 && a->line != length)
+                return false;
+            a->line = length;
+        }
+    Rank ranks[kMaxRanks];
+    for (int i = 0; i < num_ranks; ++i)
+    {
+        ranks[i] = a->rank[order[i]];
+        for (auto& sides : ranks[i].peer)
+            for (int32_t& p : sides)
+                p = p < 0 ? p : place[p];
+        for (int d = 1; d < kMaxSpatial; ++d)
+            for (const int32_t p : ranks[i].peer[d])
+                if (p >= 0 && p % a->line != i % a->line)
+                    return false;
+    }
+    std::copy(ranks, ranks + num_ranks, a->rank);
+    a->lines = make_fastdiv(static_cast<uint32_t>(num_ranks / a->line));
+    return true;
+}
+
+template <bool CLEAR>
+int run(h2x_dtype dtype, const h2x_halo_grid* h, int only_unfilled, h2x_stream_t stream)
+{
+    const int es = dtype == H2X_F32 ? 4 : dtype == H2X_F64 ? 8 : 0;
+    if (es == 0)
+        return H2X_ERR_UNSUPPORTED;
+    if (!h)
+        return H2X_ERR_INVALID_ARGUMENT;
+    Args a;
+    const int err = make_args(*h, CLEAR ? 0 : 1, only_unfilled, es, &a);
+    if (err != 0)
+        return err;
+    if (!is_grid(a, h->num_ranks))
+        return H2X_ERR_INVALID_ARGUMENT;
+    if (!order_into_lines(&a, h->num_ranks))
+        return H2X_ERR_UNSUPPORTED;
+    // Regions with the same work for every rank: blocks for the largest rank.
+    int num_regions = 0;
+    uint64_t blocks = 0;
+    std::fill(a.first, a.first + kMaxRegions, ~0u);
+    for (int ends = 1; ends >= 0; --ends)
+        for (int dz = 0; dz < 3; ++dz)
+            for (int dy = 0; dy < 3; ++dy)
+            {
+                if ((ends && a.width[0] == 0) || (dy && a.width[1] == 0) || (dz && a.width[2] == 0)
+                    || (!ends && !dy && !dz))
+                    continue;
+                uint64_t most = 0;
+                for (int r = 0; r < h->num_ranks; ++r)
+                {
+                    const Rank& k = a.rank[r];
+                    const int digit[2] = {dy, dz};
+                    bool any = false; // something to do for this rank
+                    for (int d = 1; d < 3; ++d)
+                        if (digit[d - 1])
+                            any = any || (CLEAR ? k.clear >> (2 * d + digit[d - 1] - 1) & 1
+                                                : k.peer[d][digit[d - 1] - 1] >= 0);
+                    if (ends)
+                        any = any || (CLEAR ? k.clear & 3 : k.peer[0][0] >= 0 || k.peer[0][1] >= 0);
+                    if (!any)
+                        continue;
+                    const uint64_t rows = static_cast<uint64_t>(dy ? a.width[1] : k.local[1])
+                                          * (dz ? a.width[2] : k.local[2]) * a.outer;
+                    most = std::max<uint64_t>(
+                        most, (rows * (ends ? 2 * a.width[0] : k.units.divisor) + kBlock - 1) / kBlock);
+                }
+                if (most == 0)
+                    continue;
+                const int g = num_regions++;
+                a.first[g] = static_cast<uint32_t>(blocks);
+                a.code[g] = static_cast<uint32_t>(ends + 4 * dy + 16 * dz);
+                blocks += most * (ends ? a.lines.divisor : a.ranks.divisor);
+                if (most >= 0x7fffff || blocks > 0x7fffffffull) // indexes of one rank stay below 2^31
+                    return H2X_ERR_TOO_LARGE;
+            }
+    if (blocks == 0)
+        return H2X_SUCCESS;
+    return es == 4 ? issue<uint32_t, CLEAR>(a, static_cast<uint32_t>(blocks), as_stream(stream))
+                   : issue<uint64_t, CLEAR>(a, static_cast<uint32_t>(blocks), as_stream(stream));
+}
+
+int run_fold(h2x_dtype dtype, const h2x_halo_grid* h, int op, h2x_stream_t stream)
+{
+    const int es = dtype == H2X_F32 ? 4 : dtype == H2X_F64 ? 8 : 0;
+    if (es == 0)
+        return H2X_ERR_UNSUPPORTED;
+    if (!h || op < H2X_HALO_ID || op > H2X_HALO_MIN)
+        return H2X_ERR_INVALID_ARGUMENT;
+    Args a;
+    int err = make_args(*h, 2, 0, es, &a);
+    if (err != 0)
+        return err;
+    const int64_t vec = 16 / es;
+    int64_t blocks[kMaxSpatial] = {};
+    FastDiv units[kMaxSpatial][kMaxRanks];
+    bool vectors[kMaxSpatial][kMaxRanks];
+    for (int dim = 0; dim < kMaxSpatial; ++dim)
+    {
+        bool any = false;
+        for (int r = 0; r < h->num_ranks; ++r)
+        {
+            const Rank& k = a.rank[r];
+            any = any || k.peer[dim][0] >= 0 || k.peer[dim][1] >= 0;
+            int64_t run = a.width[dim], above = a.outer;
+            for (int d = 0; d < kMaxSpatial; ++d)
+                (d < dim ? run : above) *= d == dim ? 1 : k.local[d] + 2 * a.width[d];
+            vectors[dim][r] = run >= vec;
+            const int64_t n = run >= vec ? (run + vec - 1) / vec : std::max<int64_t>(run, 1);
+            units[dim][r] = make_fastdiv(static_cast<uint32_t>(n));
+            blocks[dim] = std::max(blocks[dim], (n * above + kBlock - 1) / kBlock * h->num_ranks);
+        }
+        if (!any)
+            blocks[dim] = 0;
+        if (blocks[dim] > 0x7fffff) // the last index of a workgroup stays below 2^31
+            return H2X_ERR_TOO_LARGE;
+    }
+    for (int dim = 0; dim < kMaxSpatial && err == 0; ++dim)
+    {
+        if (blocks[dim] == 0)
+            continue;
+        for (int r = 0; r < h->num_ranks; ++r)
+        {
+            a.rank[r].units = units[dim][r];
+            a.rank[r].vectors = vectors[dim][r];
+        }
+        const uint32_t n = static_cast<uint32_t>(blocks[dim]);
+        err = es == 4 ? issue_fold<float>(op, a, n, dim, as_stream(stream))
+                      : issue_fold<double>(op, a, n, dim, as_stream(stream));
+    }
+    return err;
+}
+
+} // namespace
+} // namespace grid
+} // namespace h2x
+
+extern "C" int h2x_halo_grid_exchange(h2x_dtype dtype, const h2x_halo_grid* grid, h2x_stream_t stream)
+{
+    return h2x::grid::run<false>(dtype, grid, 0, stream);
+}
+
+extern "C" int h2x_halo_grid_clear(h2x_dtype dtype, const h2x_halo_grid* grid, int only_unfilled,
+                                   h2x_stream_t stream)
+{
+    return h2x::grid::run<true>(dtype, grid, only_unfilled, stream);
+}
+
+extern "C" int h2x_halo_grid_fold(h2x_dtype dtype, const h2x_halo_grid* grid, int op, h2x_stream_t stream)
+{
+    return h2x::grid::run_fold(dtype, grid, op, stream);
+}

@@ -22,6 +22,13 @@ def _device_buffer(count: int, dtype, device="cuda", zero: bool = False) -> torc
     return (torch.zeros if zero else torch.empty)(count, dtype=dtype, device=device)
 
 
+def _share_a_gpu(tensors: Sequence[Tensor]) -> bool:
+    """All tensors are allocated, on one GPU: what belongs to another rank can be read and written
+    where it lies.  (On the host, where launches can only be audited, strips are packed as they
+    would be for a transport.)"""
+    first = tensors[0].data
+    return all(t.data is not None and t.data.is_cuda and t.data.device == first.device for t in tensors)
+
 
 _has_gpu: Optional[bool] = None
 
@@ -465,6 +472,9 @@ class HaloExchangeAccumOp(Enum):
     MIN = capi.HALO_MIN
 
 
+_FULL_WIDTHS = (None, None, None, None)  # exchange(): every halo at its full width
+
+
 class HaloExchangeVirtual:
     """HaloExchange for all virtual ranks of one distributed tensor
     (legacy/include/distconv/tensor/halo_exchange_cuda.hpp:18-423).
@@ -494,7 +504,10 @@ class HaloExchangeVirtual:
         self._recv = {}  # (rank, dim, side) -> torch buffer the rank unpacks from
         self._faces = {}  # exchange arguments and addresses -> launches (label, entry point, descriptors)
         # optional callable(label, launch, num_faces): wraps every launch, for per-kernel timing
+        # (of the packing and unpacking launches: a hooked exchange runs dimension by dimension)
         self.launch_hook = None
+        self._buffers_wanted = False  # a receive buffer was handed out: exchanges fill them
+        self._grid_of = None  # (addresses, h2x_halo_grid or None, usable for exchanges)
 
     def get_halo_size(self, rank: int, dim: int, width: int) -> int:
         """halo_exchange_cuda.hpp:267-271."""
@@ -543,6 +556,10 @@ class HaloExchangeVirtual:
     def recv_buffer(self, rank: int, dim: int, side: int) -> torch.Tensor:
         """The buffer rank `rank` unpacks its (dim, side) halo from -- and its
         neighbour on that side packs into (get_recv_buffer, halo_exchange_cuda.hpp:277-283)."""
+        self._buffers_wanted = True
+        return self._receive_buffer(rank, dim, side)
+
+    def _receive_buffer(self, rank: int, dim: int, side: int) -> torch.Tensor:
         key = (rank, dim, side)
         if key not in self._recv:
             t = self.tensors[rank]
@@ -563,6 +580,42 @@ class HaloExchangeVirtual:
         f.inner = int((is_pack and not is_reverse) or ((not is_pack) and is_reverse))
         f.is_pack, f.op = int(is_pack), op.value
         return f
+
+    def _grid(self, cells: int) -> int:
+        """Address of the h2x_halo_grid of all ranks, or 0 where the launches that serve all of
+        them cannot: tensors that do not share a GPU (the packed strips are what could travel),
+        an empty rank, a halo on channels or samples, or next to a neighbour fewer than `cells`
+        halo widths of interior (an exchange needs one: its boundary strips are no halo; a
+        reverse one two: they do not overlap)."""
+        addresses = self._addresses()
+        kept = self._grid_of
+        if kept is None or kept[0] != addresses:
+            kept = self._grid_of = (addresses, *self._make_grid())
+        return kept[1] if kept[2] >= cells else 0
+
+    def _make_grid(self):
+        """(address of the h2x_halo_grid or 0, halo widths of interior that every rank has)"""
+        ts, ov = self.tensors, self.tensors[0].overlap
+        if (len(ts) > capi.HALO_GRID_MAX_RANKS or self.nd not in (4, 5) or not any(ov) or any(ov[self.nd - 2:])
+                or not _share_a_gpu(ts) or any(not 0 < t.get_local_size() <= t.get_local_real_size() < 2 ** 31 for t in ts)):
+            return 0, -1
+        ranks = (capi.HaloGridRank * len(ts))()
+        cells = 2
+        for r, (t, k) in enumerate(zip(ts, ranks)):
+            k.tensor = t.get_buffer()
+            for d in range(self.nd):
+                k.local_shape[d] = t.local_shape[d]
+                for side in (capi.LHS, capi.RHS):
+                    peer = self.find_peer_rank(r, d, side)
+                    k.peer[d][side] = -1 if peer is None else peer
+                    if peer is not None:
+                        cells = min(cells, t.local_shape[d] // ov[d])
+        g = capi.HaloGrid(self.nd, len(ts))
+        for d in range(self.nd):
+            g.overlap[d] = ov[d]
+        g.ranks = ranks
+        self._grid_memory = (g, ranks)
+        return ctypes.addressof(g), cells
 
     def exchange_dim(self, dim: int, width_rhs_send: int, width_rhs_recv: int, width_lhs_send: int,
                      width_lhs_recv: int, is_reverse: bool = False, skip_unpack: bool = False,
@@ -617,10 +670,10 @@ class HaloExchangeVirtual:
                     w_send = width_rhs_send if side == capi.RHS else width_lhs_send
                     w_recv = width_rhs_recv if side == capi.RHS else width_lhs_recv
                     if w_send > 0:
-                        dst = self.recv_buffer(peer, dim, capi.LHS if side == capi.RHS else capi.RHS)
+                        dst = self._receive_buffer(peer, dim, capi.LHS if side == capi.RHS else capi.RHS)
                         packs.append(self.make_face(r, dim, side, w_send, dst, True, is_reverse, op))
                     if w_recv > 0 and not skip_unpack:
-                        src = self.recv_buffer(r, dim, side)
+                        src = self._receive_buffer(r, dim, side)
                         unpacks.append(self.make_face(r, dim, side, w_recv, src, False, is_reverse, op))
             for what, faces in (("pack", packs), ("unpack", unpacks)):
                 if faces:
@@ -704,10 +757,23 @@ class HaloExchangeVirtual:
         ones filled (halo_exchange_cuda.hpp:56-106)."""
         ov = self.tensors[0].overlap
         given = (widths_rhs_send, widths_rhs_recv, widths_lhs_send, widths_lhs_recv)
-        widths = tuple([ov if w is None else w for w in given])
         if fused and skip_unpack:
             raise ValueError("a fused exchange has no separate unpack to skip")
-        key = ("all", None if given == (None,) * 4 else tuple(map(tuple, widths)), is_reverse, skip_unpack, op, fused, self._addresses())
+        if (given == _FULL_WIDTHS and (is_reverse or op is HaloExchangeAccumOp.ID) and self.launch_hook is None
+                and (fused or not (skip_unpack or self._buffers_wanted))):
+            # nobody looks at the receive buffers: straight from tensor to tensor
+            grid = self._grid(2 if is_reverse else 1)
+            if grid:
+                dtype, st = self.tensors[0].h2x_dtype, _stream_handle(self.stream)
+                if is_reverse:
+                    status = self._calls.h2x_halo_grid_fold(dtype, grid, op.value, st)
+                else:
+                    status = self._calls.h2x_halo_grid_exchange(dtype, grid, st)
+                if status:
+                    capi.check(status, "halo exchange (grid)")
+                return
+        widths = tuple([ov if w is None else w for w in given])
+        key = ("all", None if given == _FULL_WIDTHS else tuple(map(tuple, widths)), is_reverse, skip_unpack, op, fused, self._addresses())
         launches = self._faces.get(key)
         if launches is None:
             launches = []
@@ -738,6 +804,13 @@ class HaloExchangeVirtual:
         cleared cells, because neighbours along one dimension sit at the same
         position of every other dimension.  The tensors end up exactly as after
         clearing everything first."""
+        grid = self._grid(0)
+        if grid:
+            status = self._calls.h2x_halo_grid_clear(self.tensors[0].h2x_dtype, grid, int(only_unfilled),
+                                                     _stream_handle(self.stream))
+            if status:
+                capi.check(status, "clear_halos (grid)")
+            return
         key = ("clear", only_unfilled, self._addresses())
         if key not in self._faces:
             faces = []

@@ -886,6 +886,54 @@ int h2x_halo_exchange_fused(h2x_dtype dtype,
                             int num_transfers,
                             h2x_stream_t stream);
 
+/**
+ * One rank of a grid of ranks whose tensors share the device: the start of its
+ * real allocation, its interior extents (innermost first) and, per dimension
+ * and side (h2x_side), the index of the neighbour its halo is exchanged with, or
+ * -1.  Each rank is its neighbour's neighbour on the other side.
+ */
+typedef struct h2x_halo_grid_rank
+{
+    void* tensor;
+    int64_t local_shape[H2X_MAX_DIMS];
+    int32_t peer[H2X_MAX_DIMS][2];
+} h2x_halo_grid_rank;
+
+/** 3 to 5 dimensions, the last two (channels, samples) without halo; at most 16 ranks, none empty. */
+typedef struct h2x_halo_grid
+{
+    int32_t num_dims;
+    int32_t num_ranks;
+    int64_t overlap[H2X_MAX_DIMS]; /* halo width of every tensor */
+    const h2x_halo_grid_rank* ranks;
+} h2x_halo_grid;
+
+/**
+ * The forward exchange of full-width halos of all ranks and dimensions in one
+ * launch: leaves in every tensor what packing and unpacking dimension after
+ * dimension leaves there (legacy/include/distconv/tensor/
+ * halo_exchange_cuda.hpp:56-106), without buffers.  A rank with a neighbour
+ * needs at least the halo's width of interior cells along that dimension.
+ * `grid` is host memory, read before return.
+ */
+int h2x_halo_grid_exchange(h2x_dtype dtype, const h2x_halo_grid* grid, h2x_stream_t stream);
+
+/**
+ * The reverse exchange of full-width halos of all ranks, one launch a dimension:
+ * halo strips are combined with `op` (h2x_halo_op) into the boundary cells they
+ * belong to, innermost dimension first, as packing and unpacking them does.  A rank
+ * with a neighbour needs at least twice the halo's width of interior cells along
+ * that dimension (its two boundary strips must not share cells).
+ */
+int h2x_halo_grid_fold(h2x_dtype dtype, const h2x_halo_grid* grid, int op, h2x_stream_t stream);
+
+/**
+ * Zeroes the halos of all ranks in one launch: every side of every dimension,
+ * or with `only_unfilled` the sides without a neighbour (see
+ * h2x_halo_clear_batched).
+ */
+int h2x_halo_grid_clear(h2x_dtype dtype, const h2x_halo_grid* grid, int only_unfilled, h2x_stream_t stream);
+
 /* ------------------------------------------------------------------------ */
 /* Tensor shuffler pack / unpack                                             */
 /* ------------------------------------------------------------------------ */
