@@ -16,8 +16,11 @@ H2X_MAX_DIMS = 6
 F32, F64 = 0, 1
 LHS, RHS = 0, 1
 HALO_GRID_MAX_RANKS = 16
+SHUFFLE_DIRECT_MAX_RANKS = 64
 HALO_ID, HALO_SUM, HALO_MAX, HALO_MIN = 0, 1, 2, 3
 TRANSFORM_SCALE, TRANSFORM_COPY, TRANSFORM_SCALE_BIAS, TRANSFORM_SUMS_TO_STATISTICS = 0, 1, 2, 3
+
+ERR_UNSUPPORTED, ERR_TOO_LARGE = -2, -3
 
 ABI_VERSION = 1
 
@@ -133,6 +136,12 @@ class ShuffleGeometry(ctypes.Structure):
     ]
 
 
+class ShufflePart(ctypes.Structure):
+    """struct h2x_shuffle_part"""
+    _fields_ = [("origin", c_int64 * H2X_MAX_DIMS), ("extent", c_int64 * H2X_MAX_DIMS),
+                ("stride", c_int64 * H2X_MAX_DIMS), ("active", c_int32), ("reserved", c_int32)]
+
+
 class CopyAuditRegion(ctypes.Structure):
     """struct h2x_copy_audit_region"""
     _fields_ = [
@@ -244,6 +253,10 @@ SIGNATURES = {
     "h2x_halo_grid_clear": (c_int, [c_int, POINTER(HaloGrid), c_int, c_void_p]),
     "h2x_shuffle_plan_create": (c_int, [POINTER(ShuffleGeometry), POINTER(c_void_p)]),
     "h2x_shuffle_plan_destroy": (c_int, [c_void_p]),
+    "h2x_shuffle_direct_plan_create": (c_int, [c_int, c_int, c_int, POINTER(ShufflePart), POINTER(ShufflePart),
+                                               POINTER(c_void_p)]),
+    "h2x_shuffle_direct_plan_destroy": (c_int, [c_void_p]),
+    "h2x_shuffle_direct": (c_int, [c_void_p, POINTER(c_void_p), POINTER(c_void_p), c_int, c_void_p]),
     "h2x_shuffle_pack": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p]),
     "h2x_shuffle_unpack": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p]),
     "h2x_shuffle_pack_batched": (c_int, [POINTER(c_void_p), POINTER(c_void_p), POINTER(c_void_p),

@@ -126,6 +126,7 @@ PyMethodDef s_methods[] = {H2X_ENTRY(h2x_bn_channel_sums_and_sqsums),
                            H2X_ENTRY(h2x_halo_grid_exchange),
                            H2X_ENTRY(h2x_halo_grid_fold),
                            H2X_ENTRY(h2x_halo_grid_clear),
+                           H2X_ENTRY(h2x_shuffle_direct),
                            H2X_ENTRY(h2x_shuffle_pack_batched),
                            H2X_ENTRY(h2x_shuffle_unpack_batched),
                            {nullptr, nullptr, 0, nullptr}};

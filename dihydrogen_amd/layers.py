@@ -846,6 +846,10 @@ class TensorShufflerVirtual:
     one arena and every rank packs straight into its peers' chunks of it -- the
     all-to-all of the reference's ``transfer`` is therefore free -- and each
     direction is two launches: pack for all ranks, unpack for all ranks.
+
+    Tensors that all live on one GPU, no source in a destination's memory, need no
+    arena: each direction is one launch from tensor to tensor.  The arenas and the
+    packing plans are then never made.
     """
 
     def __init__(self, src_tensors: Sequence[Tensor], dst_tensors: Sequence[Tensor],
@@ -858,9 +862,11 @@ class TensorShufflerVirtual:
             raise ValueError("source and destination must have the same number of ranks")
         self.num_ranks = len(self.src)
         self.elem_size = torch.empty(0, dtype=self.src[0].dtype).element_size()
-        self._keep = []  # ctypes arrays referenced by geometries
-        self._fwd = self._direction(self.src, self.dst)
-        self._bwd = self._direction(self.dst, self.src)
+        self._directions = {}  # forward? -> plans and buffers of the packed path
+        self._direct = None  # (addresses, argument arrays or None): see _direct_arguments
+        self._direct_plan = self._make_direct_plan()
+        if self._direct_plan is None:
+            self._packed(True), self._packed(False)
 
     @staticmethod
     def get_buf_size(t: Tensor) -> int:
@@ -900,6 +906,63 @@ class TensorShufflerVirtual:
             ok = a.is_split_root() and b.dist.is_split_root_index(idx)
             counts.append(self._overlap_size(a, b, idx) if ok else 0)
         return counts
+
+    # -- tensor to tensor -----------------------------------------------------
+    def _make_direct_plan(self):
+        """Plan of the direct launches, or None where tensors do not share a GPU (packed strips
+        are what could travel) or the library cannot express the intersections."""
+        tensors, nd = self.src + self.dst, self.src[0].get_num_dims()
+        if self.num_ranks > capi.SHUFFLE_DIRECT_MAX_RANKS or not _share_a_gpu(tensors):
+            return None
+        parts = []
+        for ts in (self.src, self.dst):
+            arr = (capi.ShufflePart * self.num_ranks)()
+            for t, p in zip(ts, arr):
+                for d, stride in enumerate(t.get_strides()):
+                    p.origin[d], p.extent[d], p.stride[d] = t.global_index[d], t.local_shape[d], stride
+                p.active = int(t.is_split_root() and t.get_local_size() > 0)
+            parts.append(arr)
+        plan = ctypes.c_void_p()
+        status = self._lib.h2x_shuffle_direct_plan_create(nd, self.elem_size, self.num_ranks, *parts, ctypes.byref(plan))
+        if status in (capi.ERR_UNSUPPORTED, capi.ERR_TOO_LARGE):
+            return None
+        capi.check(status, "shuffle plan (direct)")
+        return plan
+
+    def _direct_arguments(self):
+        """Pointer arrays of the direct launches, or None where a source shares memory with a
+        destination.  They depend only on the tensors' addresses: kept until one is reallocated."""
+        addresses = [t.data.data_ptr() for t in self.src] + [t.data.data_ptr() for t in self.dst]
+        kept = self._direct
+        if kept is None or kept[0] != addresses:
+            ends = [a + t.data.numel() * self.elem_size for a, t in zip(addresses, self.src + self.dst)]
+            n = self.num_ranks
+            shared = any(addresses[i] < ends[j] and addresses[j] < ends[i] for i in range(n) for j in range(n, 2 * n))
+            arrays = None if shared else tuple(
+                (ctypes.c_void_p * n)(*[t.get_base_ptr() for t in ts]) for ts in (self.src, self.dst))
+            kept = self._direct = (addresses, arrays, arrays and tuple(ctypes.addressof(a) for a in arrays))
+        return kept[2]
+
+    def _shuffle(self, forward: bool) -> None:
+        if self._direct_plan is not None:
+            args = self._direct_arguments()
+            if args is not None:
+                status = self._calls.h2x_shuffle_direct(self._direct_plan.value, *args, int(not forward),
+                                                        _stream_handle(self.stream))
+                if status != capi.ERR_UNSUPPORTED:  # not the device the plan was made on: pack
+                    if status:
+                        capi.check(status, "shuffle (direct)")
+                    return
+        d, src, dst = self._packed(forward), *((self.src, self.dst) if forward else (self.dst, self.src))
+        self._launch(self._calls.h2x_shuffle_pack_batched, d["pack"], src, d["arena"])
+        self._launch(self._calls.h2x_shuffle_unpack_batched, d["unpack"], dst, d["arena"])
+
+    # -- through an arena -----------------------------------------------------
+    def _packed(self, forward: bool):
+        if forward not in self._directions:
+            self._directions[forward] = (self._direction(self.src, self.dst) if forward
+                                         else self._direction(self.dst, self.src))
+        return self._directions[forward]
 
     def _direction(self, src: List[Tensor], dst: List[Tensor]):
         """Plans and buffers for src -> dst."""
@@ -962,21 +1025,19 @@ class TensorShufflerVirtual:
 
     def shuffle_forward(self) -> None:
         """src tensors -> dst tensors (shuffle_mpi_cuda.cu:478-484)."""
-        d = self._fwd
-        self._launch(self._calls.h2x_shuffle_pack_batched, d["pack"], self.src, d["arena"])
-        self._launch(self._calls.h2x_shuffle_unpack_batched, d["unpack"], self.dst, d["arena"])
+        self._shuffle(True)
 
     def shuffle_backward(self) -> None:
         """dst tensors -> src tensors (shuffle_mpi_cuda.cu:485-490)."""
-        d = self._bwd
-        self._launch(self._calls.h2x_shuffle_pack_batched, d["pack"], self.dst, d["arena"])
-        self._launch(self._calls.h2x_shuffle_unpack_batched, d["unpack"], self.src, d["arena"])
+        self._shuffle(False)
 
     def __del__(self):
         try:
-            for d in (self._fwd, self._bwd):
+            for d in self._directions.values():
                 for p in d["pack"] + d["unpack"]:
                     if p is not None:
                         self._lib.h2x_shuffle_plan_destroy(p)
+            if self._direct_plan is not None:
+                self._lib.h2x_shuffle_direct_plan_destroy(self._direct_plan)
         except Exception:
             pass

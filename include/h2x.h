@@ -997,6 +997,43 @@ int h2x_shuffle_pack_batched(const h2x_shuffle_plan* const* plans, const void* c
 int h2x_shuffle_unpack_batched(const h2x_shuffle_plan* const* plans, void* const* tensors,
                                const void* const* buffers, int num_plans, h2x_stream_t stream);
 
+/**
+ * One rank's part of a distributed tensor: global index of its first element,
+ * interior extents, element strides of the real allocation, and whether the
+ * rank takes part (it owns elements and is a split root).
+ */
+typedef struct h2x_shuffle_part
+{
+    int64_t origin[H2X_MAX_DIMS];
+    int64_t extent[H2X_MAX_DIMS];
+    int64_t stride[H2X_MAX_DIMS];
+    int32_t active;
+    int32_t reserved;
+} h2x_shuffle_part;
+
+typedef struct h2x_shuffle_direct_plan h2x_shuffle_direct_plan;
+
+/**
+ * A shuffle between ranks whose tensors all share the device: every element
+ * goes straight from its source to its destination, without staging buffers,
+ * in one launch a direction; what packing all ranks and unpacking them leaves.
+ * `src` and `dst` describe the two distributions of one global tensor, num_ranks
+ * (at most 64) parts each; H2X_ERR_UNSUPPORTED where an intersection of two
+ * parts does not reduce to runs in three strided dimensions.  Allocates device
+ * memory and copies synchronously; call once per shuffler.
+ */
+int h2x_shuffle_direct_plan_create(int num_dims, int elem_size, int num_ranks, const h2x_shuffle_part* src,
+                                   const h2x_shuffle_part* dst, h2x_shuffle_direct_plan** plan);
+int h2x_shuffle_direct_plan_destroy(h2x_shuffle_direct_plan* plan);
+
+/**
+ * src -> dst, or with `backward` dst -> src.  Pointer arrays (num_ranks
+ * get_base_ptr() each) are host memory, read before return; no source tensor
+ * may share memory with a destination tensor.
+ */
+int h2x_shuffle_direct(const h2x_shuffle_direct_plan* plan, void* const* src, void* const* dst, int backward,
+                       h2x_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif
