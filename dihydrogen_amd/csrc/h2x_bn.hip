@@ -39,6 +39,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 // Partial sums of h2x_bn_channel_sums_and_sqsums_static, the entry point for
 // callers that can neither allocate nor bring a workspace.  Every device the
@@ -1341,6 +1342,9 @@ __global__ __launch_bounds__(kBlockSize) void bn_backprop2_short_kernel(
     }
 }
 
+// ---- whole channels in one workgroup: one launch ------------------------------
+#include "h2x_bn_once.hpp"
+
 // ---- host side ---------------------------------------------------------------
 
 template <typename T>
@@ -2495,6 +2499,30 @@ int backward_local(int n, int c, size_t s, const HostTensor& tx, const HostTenso
                                    nullptr, nullptr, dx, eps, st, &f);
 }
 
+// The tensors of a call given by local shapes and strides, which must be equal in shape.
+template <typename T>
+int two_tensors(int n, const h2x_tensor_geometry* gx, const h2x_tensor_geometry* gy, const void* x, const void* y,
+                HostTensor* tx, HostTensor* ty, int* c, size_t* s)
+{
+    int c2;
+    size_t s2;
+    int err = strided_tensor<T>(gx, x, n, tx, c, s);
+    if (!err)
+        err = strided_tensor<T>(gy, y, n, ty, &c2, &s2);
+    if (!err && (*c != c2 || *s != s2 || !same_local_shape(gx, gy)))
+        err = H2X_ERR_INVALID_ARGUMENT;
+    return err;
+}
+
+template <typename T>
+int three_tensors(int n, const h2x_tensor_geometry* gx, const h2x_tensor_geometry* gd, const h2x_tensor_geometry* go,
+                  const void* x, const void* dy, const void* dx, HostTensor* tx, HostTensor* td, HostTensor* to,
+                  int* c, size_t* s)
+{
+    int err = two_tensors<T>(n, gx, gd, x, dy, tx, td, c, s);
+    return err ? err : two_tensors<T>(n, gx, go, x, dx, tx, to, c, s);
+}
+
 template <typename T>
 int forward_local_strided(int n, const h2x_tensor_geometry* gx, const h2x_tensor_geometry* gy,
                           const void* x, const void* scale, const void* bias, size_t num_per_sum,
@@ -2502,13 +2530,9 @@ int forward_local_strided(int n, const h2x_tensor_geometry* gx, const h2x_tensor
                           void* running_var, void* y, void* ws, hipStream_t st)
 {
     HostTensor tx, ty;
-    int c, c2;
-    size_t s, s2;
-    int err = strided_tensor<T>(gx, x, n, &tx, &c, &s);
-    if (!err)
-        err = strided_tensor<T>(gy, y, n, &ty, &c2, &s2);
-    if (!err && (c != c2 || s != s2 || !same_local_shape(gx, gy)))
-        err = H2X_ERR_INVALID_ARGUMENT;
+    int c;
+    size_t s;
+    const int err = two_tensors<T>(n, gx, gy, x, y, &tx, &ty, &c, &s);
     return err ? err
                : forward_local<T>(n, c, s, tx, ty, x, scale, bias, num_per_sum, decay, eps, mean, var,
                                   running_mean, running_var, y, ws, st);
@@ -2522,20 +2546,165 @@ int backward_local_strided(int n, size_t num_per_sum, const h2x_tensor_geometry*
                            void* dx, double eps, void* ws, hipStream_t st)
 {
     HostTensor tx, td, to;
-    int c, c2, c3;
-    size_t s, s2, s3;
-    int err = strided_tensor<T>(gx, x, n, &tx, &c, &s);
-    if (!err)
-        err = strided_tensor<T>(gd, dy, n, &td, &c2, &s2);
-    if (!err)
-        err = strided_tensor<T>(go, dx, n, &to, &c3, &s3);
-    if (!err
-        && (c != c2 || s != s2 || c != c3 || s != s3 || !same_local_shape(gx, gd)
-            || !same_local_shape(gx, go)))
-        err = H2X_ERR_INVALID_ARGUMENT;
+    int c;
+    size_t s;
+    const int err = three_tensors<T>(n, gx, gd, go, x, dy, dx, &tx, &td, &to, &c, &s);
     return err ? err
                : backward_local<T>(n, c, s, tx, td, to, num_per_sum, x, dy, mean, var, scale, dscale,
                                    dbias, dmean, dvar, dx, eps, ws, st);
+}
+
+// ---- whole channels in one workgroup: which calls, which team -------------------
+// float only: the staged calls of double tensors are promised bit for bit, and here
+// the fp64 sums are added in another order.  All tensors of the call lie alike, a row
+// holds a vector, and offsets within a channel fit 30 bits.
+bool once_geometry(int num_samples, int num_channels, size_t spatial, std::initializer_list<const HostTensor*> ts,
+                   OnceGeometry* g)
+{
+    constexpr size_t vec = full_vec<float>();
+    const HostTensor& a = **ts.begin();
+    for (const HostTensor* t : ts)
+        if (t->strided != a.strided || t->map.stride_n != a.map.stride_n || t->map.stride_c != a.map.stride_c
+            || t->map.sy != a.map.sy || t->map.sz != a.map.sz || t->map.w.divisor != a.map.w.divisor
+            || t->map.h.divisor != a.map.h.divisor)
+            return false;
+    const size_t w = a.row, h = a.strided ? a.map.h.divisor : 1, d = a.strided ? spatial / (w * h) : 1;
+    if (w < vec || a.map.stride_n >= (1ll << 30))
+        return false;
+    const size_t spr = (w + vec - 1) / vec;
+    const size_t end = (num_samples - 1) * static_cast<size_t>(a.map.stride_n)
+                       + (d - 1) * static_cast<size_t>(a.map.sz) + (h - 1) * static_cast<size_t>(a.map.sy) + w;
+    const size_t vectors = num_samples * d * h * spr;
+    if (end >= (1ull << 30) || vectors >= (1ull << 30))
+        return false;
+    g->vectors = static_cast<uint32_t>(vectors);
+    g->width = static_cast<uint32_t>(w);
+    g->spr = make_fastdiv(static_cast<uint32_t>(spr));
+    g->h = make_fastdiv(static_cast<uint32_t>(h));
+    g->d = make_fastdiv(static_cast<uint32_t>(d));
+    g->sy = a.map.sy;
+    g->sz = a.map.sz;
+    g->stride_n = static_cast<uint32_t>(a.map.stride_n);
+    g->stride_c = a.map.stride_c;
+    g->num_channels = static_cast<uint32_t>(num_channels);
+    return true;
+}
+
+template <int TEAM>
+unsigned int once_grid(const OnceGeometry& g)
+{
+    constexpr unsigned int teams = once_block<TEAM>() / TEAM;
+    return ((g.num_channels + teams - 1) / teams + kNumXcd - 1) / kNumXcd * kNumXcd;
+}
+
+// Rows of at least this many bytes without halos between them are stored past the caches.
+constexpr size_t kStreamRow = 512;
+// Channels from which a variant that fills a CU with one channel pays: below, the two-launch
+// kernels spread a channel of this size over the idle CUs (N 4, C 64, 128 x 128 forward 11.7 us,
+// in one launch 12.3; C 64, 28^3 x 2 9.6 and 9.1).
+constexpr unsigned int kOnceManyChannels = 96;
+
+template <int TEAM, int K, bool STREAM>
+void issue_once(const OnceGeometry& g, const OnceForward<float>& a, hipStream_t st)
+{
+    bn_once_forward_kernel<float, TEAM, K, STREAM><<<once_grid<TEAM>(g), once_block<TEAM>(), 0, st>>>(g, a);
+}
+template <int TEAM, int K, bool STREAM>
+void issue_once(const OnceGeometry& g, const OnceBackward<float>& a, hipStream_t st)
+{
+    constexpr int kInLds = TEAM * K > 8192 ? 9 : 0; // 144 of the 160 KB
+    bn_once_backward_kernel<float, TEAM, K, STREAM, kInLds><<<once_grid<TEAM>(g), once_block<TEAM>(), 0, st>>>(g, a);
+}
+
+// The smallest team whose K vectors a thread hold the channel: four where that is enough
+// workgroups (more threads wait for memory together), more only beyond 1024 threads.
+// False: no variant holds it.
+template <bool STREAM, typename A>
+bool once_launch(const OnceGeometry& g, const A& a, hipStream_t st)
+{
+    constexpr bool kForward = std::is_same<A, OnceForward<float>>::value;
+    if (g.vectors <= 64 * 2)
+        issue_once<64, 2, STREAM>(g, a, st);
+    else if (g.vectors <= 256 * 4)
+        issue_once<256, 4, STREAM>(g, a, st);
+    else if (g.vectors <= 512 * 4)
+        issue_once<512, 4, STREAM>(g, a, st);
+    else if (g.vectors <= 1024 * 4)
+        issue_once<1024, 4, STREAM>(g, a, st);
+    else if (g.vectors <= 1024 * 8)
+        issue_once<1024, 8, STREAM>(g, a, st);
+    else if (g.num_channels >= kOnceManyChannels && g.vectors <= 1024 * 16)
+        issue_once<1024, 16, STREAM>(g, a, st);
+    else if (kForward && g.num_channels >= kOnceManyChannels && g.vectors <= 1024 * 20)
+        issue_once<1024, kForward ? 20 : 16, STREAM>(g, a, st);
+    else
+        return false;
+    return true;
+}
+
+template <typename A>
+bool once_launch(const OnceGeometry& g, const A& a, hipStream_t st)
+{
+    return g.h.divisor * g.d.divisor == 1 && g.width * sizeof(float) >= kStreamRow ? once_launch<true>(g, a, st)
+                                                                                  : once_launch<false>(g, a, st);
+}
+
+template <typename T>
+int forward_once(int n, const h2x_tensor_geometry* gx, const h2x_tensor_geometry* gy, const void* x,
+                 const void* scale, const void* bias, size_t num_per_sum, double decay, double eps, void* mean,
+                 void* var, void* running_mean, void* running_var, void* y, void* ws, hipStream_t st)
+{
+    HostTensor tx, ty;
+    int c;
+    size_t s;
+    const int err = two_tensors<T>(n, gx, gy, x, y, &tx, &ty, &c, &s);
+    if (err)
+        return err;
+    if constexpr (sizeof(T) == 4)
+    {
+        OnceGeometry g;
+        if (x && y && n > 0 && c > 0 && s > 0 && num_per_sum > 0 && once_geometry(n, c, s, {&tx, &ty}, &g))
+        {
+            const OnceForward<T> a{static_cast<const T*>(x), static_cast<const T*>(scale), static_cast<const T*>(bias),
+                                   static_cast<T*>(mean), static_cast<T*>(var), static_cast<T*>(running_mean),
+                                   static_cast<T*>(running_var), static_cast<T*>(y), static_cast<T>(num_per_sum),
+                                   static_cast<T>(decay), static_cast<T>(eps)};
+            if (once_launch(g, a, st))
+                return launch_status();
+        }
+    }
+    return forward_local<T>(n, c, s, tx, ty, x, scale, bias, num_per_sum, decay, eps, mean, var, running_mean,
+                            running_var, y, ws, st);
+}
+
+template <typename T>
+int backward_once(int n, size_t num_per_sum, const h2x_tensor_geometry* gx, const h2x_tensor_geometry* gd,
+                  const h2x_tensor_geometry* go, const void* x, const void* dy, const void* mean, const void* var,
+                  const void* scale, void* dscale, void* dbias, void* dmean, void* dvar, void* dx, double eps,
+                  void* ws, hipStream_t st)
+{
+    HostTensor tx, td, to;
+    int c;
+    size_t s;
+    const int err = three_tensors<T>(n, gx, gd, go, x, dy, dx, &tx, &td, &to, &c, &s);
+    if (err)
+        return err;
+    if constexpr (sizeof(T) == 4)
+    {
+        OnceGeometry g;
+        if (x && dy && dx && n > 0 && c > 0 && s > 0 && once_geometry(n, c, s, {&tx, &td, &to}, &g))
+        {
+            const OnceBackward<T> a{static_cast<const T*>(x), static_cast<const T*>(dy), static_cast<const T*>(mean),
+                                    static_cast<const T*>(var), static_cast<const T*>(scale), static_cast<T*>(dscale),
+                                    static_cast<T*>(dbias), static_cast<T*>(dmean), static_cast<T*>(dvar),
+                                    static_cast<T*>(dx), static_cast<T>(num_per_sum),
+                                    static_cast<T>(num_per_sum - 1), static_cast<T>(eps)};
+            if (once_launch(g, a, st))
+                return launch_status();
+        }
+    }
+    return backward_local<T>(n, c, s, tx, td, to, num_per_sum, x, dy, mean, var, scale, dscale, dbias, dmean, dvar,
+                             dx, eps, ws, st);
 }
 
 } // namespace
@@ -2908,6 +3077,48 @@ extern "C" int h2x_bn_backward_local_strided(h2x_dtype dtype, int num_samples, s
                                                dx_geometry, x, dy, mean, var, scale, dscale, dbias,
                                                dmean, dvar, dx, epsilon, workspace, as_stream(stream)),
                  backward_local_strided<double>(num_samples, num_per_sum, x_geometry, dy_geometry,
+                                                dx_geometry, x, dy, mean, var, scale, dscale, dbias,
+                                                dmean, dvar, dx, epsilon, workspace,
+                                                as_stream(stream)));
+}
+
+extern "C" int h2x_bn_forward_once(h2x_dtype dtype, int num_samples,
+                                            const h2x_tensor_geometry* x_geometry,
+                                            const h2x_tensor_geometry* y_geometry, const void* x,
+                                            const void* scale, const void* bias, size_t num_per_sum,
+                                            double decay, double epsilon, void* mean, void* var,
+                                            void* running_mean, void* running_var, void* y,
+                                            void* workspace, h2x_stream_t stream)
+{
+    if (num_samples < 0 || !x_geometry || !y_geometry || !scale || !bias || !mean || !var
+        || !running_mean || !running_var || !workspace)
+        return H2X_ERR_INVALID_ARGUMENT;
+    H2X_BY_DTYPE(dtype,
+                 forward_once<float>(num_samples, x_geometry, y_geometry, x, scale, bias,
+                                              num_per_sum, decay, epsilon, mean, var, running_mean,
+                                              running_var, y, workspace, as_stream(stream)),
+                 forward_once<double>(num_samples, x_geometry, y_geometry, x, scale, bias,
+                                               num_per_sum, decay, epsilon, mean, var, running_mean,
+                                               running_var, y, workspace, as_stream(stream)));
+}
+
+extern "C" int h2x_bn_backward_once(h2x_dtype dtype, int num_samples, size_t num_per_sum,
+                                             const h2x_tensor_geometry* x_geometry,
+                                             const h2x_tensor_geometry* dy_geometry,
+                                             const h2x_tensor_geometry* dx_geometry, const void* x,
+                                             const void* dy, const void* mean, const void* var,
+                                             const void* scale, void* dscale, void* dbias,
+                                             void* dmean, void* dvar, void* dx, double epsilon,
+                                             void* workspace, h2x_stream_t stream)
+{
+    if (num_samples < 0 || !x_geometry || !dy_geometry || !dx_geometry || !mean || !var || !scale
+        || !dscale || !dbias || !dmean || !dvar || !workspace)
+        return H2X_ERR_INVALID_ARGUMENT;
+    H2X_BY_DTYPE(dtype,
+                 backward_once<float>(num_samples, num_per_sum, x_geometry, dy_geometry,
+                                               dx_geometry, x, dy, mean, var, scale, dscale, dbias,
+                                               dmean, dvar, dx, epsilon, workspace, as_stream(stream)),
+                 backward_once<double>(num_samples, num_per_sum, x_geometry, dy_geometry,
                                                 dx_geometry, x, dy, mean, var, scale, dscale, dbias,
                                                 dmean, dvar, dx, epsilon, workspace,
                                                 as_stream(stream)));

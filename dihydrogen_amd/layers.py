@@ -102,7 +102,7 @@ class BatchNormalization:
         self.num_dims, self.decay, self.epsilon = num_dims, float(decay), float(epsilon)
         self.global_stats, self.allreduce, self.stream = global_stats, allreduce, stream
         # forward()/backward() of a rank that all-reduces nothing between its two
-        # stages run as two launches each (h2x_bn_forward_local / _backward_local);
+        # stages run as one or two launches each (h2x_bn_forward_once / _backward_once);
         # the staged methods always use the staged entry points
         self.fuse_local = fuse_local
         # Haloed tensors of one geometry: normalise and the input gradient also clear
@@ -206,16 +206,10 @@ class BatchNormalization:
             _dense_layout(input), _dense_layout(output)
             ns = self.num_current_samples = lx.samples
             per_sum = lx.per_channel_global if self.global_stats else lx.per_channel_local
-            if lx.dense and ly.dense:
-                status = self._calls.h2x_bn_forward_local(
-                    lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ly.spatial_real, input.get_base_ptr(),
-                    scale, bias, per_sum, self.decay, self.epsilon, mean, var, running_mean, running_var,
-                    output.get_base_ptr(), self._ws(lx.channels), _stream_handle(self.stream))
-            else:
-                status = self._calls.h2x_bn_forward_local_strided(
-                    lx.dtype, ns, lx.geometry_address, _tensor_geometry(ly, ns), input.get_base_ptr(), scale, bias,
-                    per_sum, self.decay, self.epsilon, mean, var, running_mean, running_var, output.get_base_ptr(),
-                    self._ws(lx.channels), _stream_handle(self.stream))
+            status = self._calls.h2x_bn_forward_once(
+                lx.dtype, ns, lx.geometry_address, _tensor_geometry(ly, ns), input.get_base_ptr(), scale, bias, per_sum,
+                self.decay, self.epsilon, mean, var, running_mean, running_var, output.get_base_ptr(),
+                self._ws(lx.channels), _stream_handle(self.stream))
             if status:
                 capi.check(status, "bn forward (local)")
             return 0
@@ -281,18 +275,11 @@ class BatchNormalization:
             _dense_layout(input), _dense_layout(d_output), _dense_layout(d_input)
             ns = self.num_current_samples = lx.samples
             per_sum = lx.per_channel_global if self.global_stats else lx.per_channel_local
-            if lx.dense and ld.dense and li.dense:
-                status = self._calls.h2x_bn_backward_local(
-                    lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ld.spatial_real, li.spatial_real,
-                    per_sum, input.get_base_ptr(), d_output.get_base_ptr(), mean, var, scale, scale_gradient,
-                    bias_gradient, mean_gradient, var_gradient, d_input.get_base_ptr(), self.epsilon,
-                    self._ws(lx.channels), _stream_handle(self.stream))
-            else:
-                status = self._calls.h2x_bn_backward_local_strided(
-                    lx.dtype, ns, per_sum, lx.geometry_address, _tensor_geometry(ld, ns), _tensor_geometry(li, ns),
-                    input.get_base_ptr(), d_output.get_base_ptr(), mean, var, scale, scale_gradient, bias_gradient,
-                    mean_gradient, var_gradient, d_input.get_base_ptr(), self.epsilon, self._ws(lx.channels),
-                    _stream_handle(self.stream))
+            status = self._calls.h2x_bn_backward_once(
+                lx.dtype, ns, per_sum, lx.geometry_address, _tensor_geometry(ld, ns), _tensor_geometry(li, ns),
+                input.get_base_ptr(), d_output.get_base_ptr(), mean, var, scale, scale_gradient, bias_gradient,
+                mean_gradient, var_gradient, d_input.get_base_ptr(), self.epsilon, self._ws(lx.channels),
+                _stream_handle(self.stream))
             if status:
                 capi.check(status, "bn backward (local)")
             return 0

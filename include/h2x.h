@@ -421,6 +421,50 @@ int h2x_bn_backward_local_strided(h2x_dtype dtype,
                                   h2x_stream_t stream);
 
 /**
+ * The same again, in one launch each way where a channel fits the registers of
+ * a workgroup (float tensors that lie alike, up to about 80000 elements a channel
+ * forward and 65000 backward); otherwise what h2x_bn_forward_local_strided and
+ * h2x_bn_backward_local_strided do.  The terms of the sums are the same and are
+ * added in fp64, in another order.
+ */
+int h2x_bn_forward_once(h2x_dtype dtype,
+                                 int num_samples,
+                                 const h2x_tensor_geometry* x_geometry,
+                                 const h2x_tensor_geometry* y_geometry,
+                                 const void* x,
+                                 const void* scale,
+                                 const void* bias,
+                                 size_t num_per_sum,
+                                 double decay,
+                                 double epsilon,
+                                 void* mean,
+                                 void* var,
+                                 void* running_mean,
+                                 void* running_var,
+                                 void* y,
+                                 void* workspace,
+                                 h2x_stream_t stream);
+int h2x_bn_backward_once(h2x_dtype dtype,
+                                  int num_samples,
+                                  size_t num_per_sum,
+                                  const h2x_tensor_geometry* x_geometry,
+                                  const h2x_tensor_geometry* dy_geometry,
+                                  const h2x_tensor_geometry* dx_geometry,
+                                  const void* x,
+                                  const void* dy,
+                                  const void* mean,
+                                  const void* var,
+                                  const void* scale,
+                                  void* dscale,
+                                  void* dbias,
+                                  void* dmean,
+                                  void* dvar,
+                                  void* dx,
+                                  double epsilon,
+                                  void* workspace,
+                                  h2x_stream_t stream);
+
+/**
  * The local part of a haloed tensor as it lies in memory: the real (allocated)
  * extents and where the interior starts in them.  Innermost first; the last
  * two dimensions are channel and sample and carry no halo; num_dims is 3, 4
