@@ -1344,6 +1344,8 @@ __global__ __launch_bounds__(kBlockSize) void bn_backprop2_short_kernel(
 
 // ---- whole channels in one workgroup: one launch ------------------------------
 #include "h2x_bn_once.hpp"
+// ---- whole channels in several workgroups: one launch behind a small fill -------
+#include "h2x_bn_team.hpp"
 
 // ---- host side ---------------------------------------------------------------
 
@@ -2556,8 +2558,9 @@ int backward_local_strided(int n, size_t num_per_sum, const h2x_tensor_geometry*
 
 // ---- whole channels in one workgroup: which calls, which team -------------------
 // float only: the staged calls of double tensors are promised bit for bit, and here
-// the fp64 sums are added in another order.  All tensors of the call lie alike, a row
-// holds a vector, and offsets within a channel fit 30 bits.
+// the fp64 sums are added in another order (N 8, C 32, 33^3, double, 36 + 62 us, by teams
+// 32 + 45).  All tensors of the call lie alike, a row holds a vector, and offsets within a
+// channel fit 30 bits.
 bool once_geometry(int num_samples, int num_channels, size_t spatial, std::initializer_list<const HostTensor*> ts,
                    OnceGeometry* g)
 {
@@ -2597,8 +2600,16 @@ unsigned int once_grid(const OnceGeometry& g)
     return ((g.num_channels + teams - 1) / teams + kNumXcd - 1) / kNumXcd * kNumXcd;
 }
 
-// Rows of at least this many bytes without halos between them are stored past the caches.
+// Dense rows of at least this many bytes are stored past the caches; shorter ones end in
+// partial lines, which the L2 merges with the neighbours' (N 1024, C 1024, 7 x 7, 206 MB: 324 us,
+// past the caches 406).
 constexpr size_t kStreamRow = 512;
+// Haloed rows, whose ends are partial lines as well, are stored normally up to this size of a
+// tensor; larger outputs push the inputs out of the memory-side cache.  Forward + backward going
+// round three sets of tensors, stored normally and past the caches: N 1, C 256, 28^3, 28 MB, 29 and
+// 37 us; N 4, C 64, 30^3, 34 MB, 46.8 and 44.9 (one set over and over 38.8 and 44.7); N 8, C 64, 30^3,
+// 67 MB, 91 and 80; N 2, C 512, 28^3, 111 MB, 158 and 147.
+constexpr size_t kHaloedNormalStores = size_t(48) << 20;
 // Channels from which a variant that fills a CU with one channel pays: below, the two-launch
 // kernels spread a channel of this size over the idle CUs (N 4, C 64, 128 x 128 forward 11.7 us,
 // in one launch 12.3; C 64, 28^3 x 2 9.6 and 9.1).
@@ -2642,17 +2653,134 @@ bool once_launch(const OnceGeometry& g, const A& a, hipStream_t st)
     return true;
 }
 
-template <typename A>
-bool once_launch(const OnceGeometry& g, const A& a, hipStream_t st)
+// Bytes from the first to behind the last element of a tensor of the call.
+size_t reach_bytes(const OnceGeometry& g, int n)
 {
-    return g.h.divisor * g.d.divisor == 1 && g.width * sizeof(float) >= kStreamRow ? once_launch<true>(g, a, st)
-                                                                                  : once_launch<false>(g, a, st);
+    const size_t last = static_cast<size_t>(g.num_channels - 1) * g.stride_c
+                        + static_cast<size_t>(n - 1) * g.stride_n + static_cast<size_t>(g.d.divisor - 1) * g.sz
+                        + static_cast<size_t>(g.h.divisor - 1) * g.sy + g.width;
+    return last * sizeof(float);
 }
 
+bool dense_rows(const OnceGeometry& g)
+{
+    return g.h.divisor * g.d.divisor == 1;
+}
+
+bool streamed(const OnceGeometry& g, int n)
+{
+    return dense_rows(g) ? g.width * sizeof(float) >= kStreamRow : reach_bytes(g, n) > kHaloedNormalStores;
+}
+
+template <typename A>
+bool once_launch(const OnceGeometry& g, const A& a, int n, hipStream_t st)
+{
+    return streamed(g, n) ? once_launch<true>(g, a, st) : once_launch<false>(g, a, st);
+}
+
+// ---- whole channels in several workgroups: which calls, which team ---------------
+bool apart(const void* a, const void* b, size_t bytes)
+{
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x + bytes <= y || y + bytes <= x;
+}
+
+template <typename T, int TEAM, int K, bool STREAM>
+void issue_team(const TeamGeometry& g, const OnceForward<T>& a, unsigned long long* slots, hipStream_t st)
+{
+    bn_team_forward_kernel<T, TEAM, K, STREAM><<<g.once.num_channels * g.members.divisor, TEAM, 0, st>>>(g, a, slots);
+}
+template <typename T, int TEAM, int K, bool STREAM>
+void issue_team(const TeamGeometry& g, const OnceBackward<T>& a, unsigned long long* slots, hipStream_t st)
+{
+    bn_team_backward_kernel<T, TEAM, K, STREAM><<<g.once.num_channels * g.members.divisor, TEAM, 0, st>>>(g, a, slots);
+}
+
+// Members of TEAM threads with K vectors each; false if that is fewer than `least` or
+// more than `most` members, or more slots than the workspace has.
+template <int TEAM, int K, template <typename> class A, typename T>
+bool team_launch(const OnceGeometry& once, const A<T>& a, bool stream, uint32_t least, uint32_t most,
+                 uint32_t max_polls, void* ws, hipStream_t st)
+{
+    constexpr int kSums = std::is_same<A<T>, OnceForward<T>>::value ? 2 : 4;
+    const uint32_t members = (once.vectors + TEAM * K - 1) / (TEAM * K);
+    const size_t blocks = static_cast<size_t>(members) * once.num_channels;
+    const size_t count = blocks * kSums;
+    if (members > most || blocks < least || count >= (1u << 30)
+        || count * sizeof(double) > partials_bytes(static_cast<int>(once.num_channels)))
+        return false;
+    TeamGeometry g;
+    g.once = once;
+    g.members = make_fastdiv(members);
+    g.span = ((once.vectors + members - 1) / members + TEAM - 1) / TEAM * TEAM;
+    g.max_polls = max_polls;
+    unsigned long long* const slots = static_cast<unsigned long long*>(ws);
+    bn_team_clear_kernel<<<static_cast<unsigned int>((count + kBlockSize - 1) / kBlockSize), kBlockSize, 0, st>>>(
+        slots, static_cast<uint32_t>(count));
+    if (stream)
+        issue_team<T, TEAM, K, true>(g, a, slots, st);
+    else
+        issue_team<T, TEAM, K, false>(g, a, slots, st);
+    return true;
+}
+
+// Looks of about a microsecond: a team that other streams keep off the chip for longer
+// works its sums out (2 ms against the tens of microseconds of a launch).
+constexpr uint32_t kTeamPolls = 2048;
+// Fewer workgroups leave the chip to the two-launch kernels, which cut a channel finer
+// (N 4, C 16, 40^3 in 256 workgroups 9.9 + 13.0 us, in two launches 10.3 + 16.3; half of
+// that, C 8, in 256 smaller ones 8.8 + 10.4 and 7.8 + 10.9).
+constexpr uint32_t kTeamLeastBlocks = 192;
+// Forward a member holds 128 KB, in smaller pieces where that is not enough workgroups
+// (N 2, C 32, 48^3: 12.0 us, whole ones 13.0); up to 128 members (N 16, C 16, 64^3 in 128
+// of them 98 us, in two launches 118).
+template <typename T>
+bool team_variant(const OnceGeometry& g, const OnceForward<T>& a, bool stream, uint32_t least, uint32_t most,
+                  uint32_t polls, void* ws, hipStream_t st)
+{
+    return team_launch<512, 16>(g, a, stream, 2 * least, most, polls, ws, st)
+           || team_launch<512, 8>(g, a, stream, least, most, polls, ws, st);
+}
+
+// Backward 64 KB of each tensor, 128 KB where a team would have more than 64 members
+// (N 8, C 64, 64^3: 355 us, in 128 members 379, in two launches 407), and no more than 64
+// of those (N 16, C 16, 64^3: 251 us, in two launches 195): a larger team waits longer for
+// its last member than it saves.
+template <typename T>
+bool team_variant(const OnceGeometry& g, const OnceBackward<T>& a, bool stream, uint32_t least, uint32_t most,
+                  uint32_t polls, void* ws, hipStream_t st)
+{
+    most /= 2;
+    return team_launch<512, 8>(g, a, stream, least, most, polls, ws, st)
+           || team_launch<1024, 8>(g, a, stream, least, most, polls, ws, st);
+}
+
+// False: the call is not for teams.
+template <typename T, template <typename> class A>
+bool launch_by_teams(const OnceGeometry& g, const A<T>& a, int n, std::initializer_list<const void*> inputs,
+                     const void* output, uint32_t least, uint32_t polls, void* ws, hipStream_t st)
+{
+    const size_t bytes = reach_bytes(g, n);
+    for (const void* p : inputs)
+        if (!apart(p, output, bytes))
+            return false;
+    int device = 0, cus = 0;
+    if (hipGetDevice(&device) != hipSuccess
+        || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
+        return false;
+    // short segments have kernels of their own (N 2048, C 256, 7 x 7: 141 us, by teams 172)
+    const bool stream = streamed(g, n);
+    if (dense_rows(g) && !stream)
+        return false;
+    return team_variant(g, a, stream, least, std::min<uint32_t>(cus / 2, kMaxMembers), polls, ws, st);
+}
+
+// team_polls: by teams or not at all, however few workgroups that is, with this many looks.
 template <typename T>
 int forward_once(int n, const h2x_tensor_geometry* gx, const h2x_tensor_geometry* gy, const void* x,
                  const void* scale, const void* bias, size_t num_per_sum, double decay, double eps, void* mean,
-                 void* var, void* running_mean, void* running_var, void* y, void* ws, hipStream_t st)
+                 void* var, void* running_mean, void* running_var, void* y, void* ws, hipStream_t st,
+                  const uint32_t* team_polls = nullptr)
 {
     HostTensor tx, ty;
     int c;
@@ -2660,7 +2788,7 @@ int forward_once(int n, const h2x_tensor_geometry* gx, const h2x_tensor_geometry
     const int err = two_tensors<T>(n, gx, gy, x, y, &tx, &ty, &c, &s);
     if (err)
         return err;
-    if constexpr (sizeof(T) == 4)
+    if constexpr (sizeof(T) == 4) // see once_geometry
     {
         OnceGeometry g;
         if (x && y && n > 0 && c > 0 && s > 0 && num_per_sum > 0 && once_geometry(n, c, s, {&tx, &ty}, &g))
@@ -2669,10 +2797,16 @@ int forward_once(int n, const h2x_tensor_geometry* gx, const h2x_tensor_geometry
                                    static_cast<T*>(mean), static_cast<T*>(var), static_cast<T*>(running_mean),
                                    static_cast<T*>(running_var), static_cast<T*>(y), static_cast<T>(num_per_sum),
                                    static_cast<T>(decay), static_cast<T>(eps)};
-            if (once_launch(g, a, st))
+            if (team_polls)
+                return launch_by_teams(g, a, n, {x}, y, 1, *team_polls, ws, st) ? launch_status()
+                                                                            : H2X_ERR_UNSUPPORTED;
+            if (once_launch(g, a, n, st)
+                || launch_by_teams(g, a, n, {x}, y, kTeamLeastBlocks, kTeamPolls, ws, st))
                 return launch_status();
         }
     }
+    if (team_polls)
+        return H2X_ERR_UNSUPPORTED;
     return forward_local<T>(n, c, s, tx, ty, x, scale, bias, num_per_sum, decay, eps, mean, var, running_mean,
                             running_var, y, ws, st);
 }
@@ -2681,7 +2815,8 @@ template <typename T>
 int backward_once(int n, size_t num_per_sum, const h2x_tensor_geometry* gx, const h2x_tensor_geometry* gd,
                   const h2x_tensor_geometry* go, const void* x, const void* dy, const void* mean, const void* var,
                   const void* scale, void* dscale, void* dbias, void* dmean, void* dvar, void* dx, double eps,
-                  void* ws, hipStream_t st)
+                  void* ws, hipStream_t st,
+                   const uint32_t* team_polls = nullptr)
 {
     HostTensor tx, td, to;
     int c;
@@ -2689,7 +2824,7 @@ int backward_once(int n, size_t num_per_sum, const h2x_tensor_geometry* gx, cons
     const int err = three_tensors<T>(n, gx, gd, go, x, dy, dx, &tx, &td, &to, &c, &s);
     if (err)
         return err;
-    if constexpr (sizeof(T) == 4)
+    if constexpr (sizeof(T) == 4) // see once_geometry
     {
         OnceGeometry g;
         if (x && dy && dx && n > 0 && c > 0 && s > 0 && once_geometry(n, c, s, {&tx, &td, &to}, &g))
@@ -2699,10 +2834,16 @@ int backward_once(int n, size_t num_per_sum, const h2x_tensor_geometry* gx, cons
                                     static_cast<T*>(dbias), static_cast<T*>(dmean), static_cast<T*>(dvar),
                                     static_cast<T*>(dx), static_cast<T>(num_per_sum),
                                     static_cast<T>(num_per_sum - 1), static_cast<T>(eps)};
-            if (once_launch(g, a, st))
+            if (team_polls)
+                return launch_by_teams(g, a, n, {x, dy}, dx, 1, *team_polls, ws, st) ? launch_status()
+                                                                            : H2X_ERR_UNSUPPORTED;
+            if (once_launch(g, a, n, st)
+                || launch_by_teams(g, a, n, {x, dy}, dx, kTeamLeastBlocks, kTeamPolls, ws, st))
                 return launch_status();
         }
     }
+    if (team_polls)
+        return H2X_ERR_UNSUPPORTED;
     return backward_local<T>(n, c, s, tx, td, to, num_per_sum, x, dy, mean, var, scale, dscale, dbias, dmean, dvar,
                              dx, eps, ws, st);
 }
@@ -3122,4 +3263,74 @@ extern "C" int h2x_bn_backward_once(h2x_dtype dtype, int num_samples, size_t num
                                                 dx_geometry, x, dy, mean, var, scale, dscale, dbias,
                                                 dmean, dvar, dx, epsilon, workspace,
                                                 as_stream(stream)));
+}
+
+extern "C" int h2x_bn_forward_team(h2x_dtype dtype, int num_samples, const h2x_tensor_geometry* x_geometry,
+                                   const h2x_tensor_geometry* y_geometry, const void* x, const void* scale,
+                                   const void* bias, size_t num_per_sum, double decay, double epsilon, void* mean,
+                                   void* var, void* running_mean, void* running_var, void* y, void* workspace,
+                                   unsigned int max_polls, h2x_stream_t stream)
+{
+    if (num_samples < 0 || !x_geometry || !y_geometry || !scale || !bias || !mean || !var || !running_mean
+        || !running_var || !workspace)
+        return H2X_ERR_INVALID_ARGUMENT;
+    H2X_BY_DTYPE(dtype,
+                 forward_once<float>(num_samples, x_geometry, y_geometry, x, scale, bias, num_per_sum, decay, epsilon,
+                                     mean, var, running_mean, running_var, y, workspace, as_stream(stream), &max_polls),
+                 forward_once<double>(num_samples, x_geometry, y_geometry, x, scale, bias, num_per_sum, decay, epsilon,
+                                      mean, var, running_mean, running_var, y, workspace, as_stream(stream),
+                                      &max_polls));
+}
+
+extern "C" int h2x_bn_backward_team(h2x_dtype dtype, int num_samples, size_t num_per_sum,
+                                    const h2x_tensor_geometry* x_geometry, const h2x_tensor_geometry* dy_geometry,
+                                    const h2x_tensor_geometry* dx_geometry, const void* x, const void* dy,
+                                    const void* mean, const void* var, const void* scale, void* dscale, void* dbias,
+                                    void* dmean, void* dvar, void* dx, double epsilon, void* workspace,
+                                    unsigned int max_polls, h2x_stream_t stream)
+{
+    if (num_samples < 0 || !x_geometry || !dy_geometry || !dx_geometry || !mean || !var || !scale || !dscale || !dbias
+        || !dmean || !dvar || !workspace)
+        return H2X_ERR_INVALID_ARGUMENT;
+    H2X_BY_DTYPE(dtype,
+                 backward_once<float>(num_samples, num_per_sum, x_geometry, dy_geometry, dx_geometry, x, dy, mean, var,
+                                      scale, dscale, dbias, dmean, dvar, dx, epsilon, workspace, as_stream(stream),
+                                      &max_polls),
+                 backward_once<double>(num_samples, num_per_sum, x_geometry, dy_geometry, dx_geometry, x, dy, mean, var,
+                                       scale, dscale, dbias, dmean, dvar, dx, epsilon, workspace, as_stream(stream),
+                                       &max_polls));
+}
+
+// Plays on the host which elements the workgroups that hold channels in registers touch.
+extern "C" int h2x_bn_audit_once(int num_samples, const h2x_tensor_geometry* geometry, unsigned int member_vectors,
+                                 unsigned char* counted, unsigned char* stored, size_t elements)
+{
+    if (!geometry || !counted || !stored)
+        return H2X_ERR_INVALID_ARGUMENT;
+    HostTensor t;
+    int c;
+    size_t s;
+    const int err = strided_tensor<float>(geometry, counted, num_samples, &t, &c, &s);
+    if (err)
+        return err;
+    OnceGeometry g;
+    if (num_samples <= 0 || c <= 0 || s == 0 || !once_geometry(num_samples, c, s, {&t}, &g))
+        return H2X_ERR_UNSUPPORTED;
+    constexpr int VEC = full_vec<float>();
+    const uint32_t span = member_vectors ? member_vectors : g.vectors;
+    for (uint32_t ch = 0; ch < g.num_channels; ++ch)
+        for (uint32_t first = 0; first < g.vectors; first += span)
+            for (uint32_t i = first; i < std::min(first + span, g.vectors); ++i)
+            {
+                const uint32_t at = once_place<VEC>(g, i);
+                const size_t e = static_cast<size_t>(ch * g.stride_c) + (at >> 2);
+                if (e + VEC > elements)
+                    return H2X_ERR_INVALID_ARGUMENT;
+                for (int j = 0; j < VEC; ++j)
+                {
+                    stored[e + j] = 1;
+                    counted[e + j] += j >= static_cast<int>(at & 3);
+                }
+            }
+    return H2X_SUCCESS;
 }

@@ -61,7 +61,8 @@ __host__ __device__ __forceinline__ uint32_t once_place(const OnceGeometry& g, u
 
 // STREAM: past the caches.  Rows of a few hundred bytes are stored normally: their
 // ends are partial lines, which the L2 merges with the neighbours' (N 128, C 1024,
-// 7 x 7 forward 10.3 us, streaming 17.1; N 4, C 512, 56 x 56 10.3 and 8.8).
+// 7 x 7 forward 10.3 us, streaming 17.1; N 4, C 512, 56 x 56 10.3 and 8.8), unless
+// the tensors are haloed and large.
 template <typename T, int VEC, bool STREAM>
 __device__ __forceinline__ void store_once(T* p, const T (&r)[VEC])
 {

@@ -1,0 +1,278 @@
+// Batch-norm of a rank that shares its statistics with no one, for channels that are
+// too large for one workgroup: the workgroups of a team hold a channel in their
+// registers together, exchange their partial sums through memory and write y (dx)
+// from the registers.  Included by h2x_bn.hip after h2x_bn_once.hpp, whose geometry,
+// terms and stores these kernels share.
+//
+// The two-launch kernels are bound by memory and read x (backward: x and dy) twice, at
+// 5 to 7 TB/s; here every element is read once.  Bound by memory and by the wait for the
+// last member of a team.  Forward, backward in us, two launches each way -> by teams:
+//   N 8, C 64, 30^3, halo of 1      38, 53 -> 35, 44     N 32, C 256, 56 x 56     48, 85 -> 36, 52
+//   N 4, C 64, 64^3                116, 190 -> 90, 182   N 64, C 128, 40 x 40     27, 46 -> 21, 31
+//   N 8, C 64, 64^3                256, 407 -> 210, 355  N 2, C 32, 48^3          16, 28 -> 12, 18
+//   N 1, C 64, 96^3                 99, 162 -> 75, 147   N 64, C 64, 57^2, halo   31, 51 -> 33, 39
+// A counter of arrivals a team instead of looking at the slots themselves was slower the
+// larger the team (64 members, N 4, C 64, 64^3: 119 us against 98): one address.
+//
+// What is exchanged validates itself: a slot holds kNoSum (a NaN that no sum can be)
+// until its member has stored a sum, in one 64-bit access of the whole device's scope,
+// so nothing else has to be ordered.  A fill kernel clears the slots before each call.
+//
+// Nobody waits for ever: after max_polls looks a member works out the sums it misses
+// from memory, with the additions of the member they belong to, and gets the same
+// bits.  That is why outputs may not overlap inputs here.  Members are neighbouring
+// workgroups, and workgroups start in order, so a team is on the chip together unless
+// other streams fill it; the launch rule keeps a team within half of it.
+#pragma once
+
+constexpr uint32_t kMaxMembers = kBlockSize; // a thread looks after one slot, no team has fewer threads
+constexpr unsigned long long kNoSum = 0x7ff8000000000001ull;
+
+struct TeamGeometry
+{
+    OnceGeometry once;
+    FastDiv members;   // of a team
+    uint32_t span;     // vectors of a member, a multiple of its threads
+    uint32_t max_polls;
+};
+
+__global__ __launch_bounds__(kBlockSize) void bn_team_clear_kernel(unsigned long long* slots, uint32_t count)
+{
+    const uint32_t i = blockIdx.x * kBlockSize + threadIdx.x;
+    if (i < count)
+        __hip_atomic_store(slots + i, kNoSum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The sums of all members in v[] of every thread, given this member's own in v[] of
+// thread 0.  recompute(member, sums) is called by the whole workgroup.
+template <int TEAM, int N, typename F>
+__device__ __forceinline__ void team_exchange(double (&v)[N], const TeamGeometry& g, uint32_t c, uint32_t member,
+                                              unsigned long long* slots, double* lds, uint32_t* missing,
+                                              const F& recompute)
+{
+    const uint32_t members = g.members.divisor, t = threadIdx.x;
+    unsigned long long* const team = slots + static_cast<size_t>(c) * members * N;
+    if (t == 0)
+    {
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+        {
+            unsigned long long bits = __double_as_longlong(v[k]);
+            if (v[k] != v[k])
+                bits = 0x7ff8000000000000ull; // any NaN but kNoSum
+            __hip_atomic_store(team + member * N + k, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        missing[kMaxMembers] = 0;
+    }
+    __syncthreads();
+    double s[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+        s[k] = 0.0;
+    if (t < members)
+    {
+        bool there = false;
+        for (uint32_t poll = 0; poll < g.max_polls && !there; ++poll)
+        {
+            if (poll > 0)
+                __builtin_amdgcn_s_sleep(4);
+            there = true;
+#pragma unroll
+            for (int k = 0; k < N; ++k)
+            {
+                const unsigned long long bits =
+                    __hip_atomic_load(team + t * N + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                s[k] = __longlong_as_double(bits);
+                there = there && bits != kNoSum;
+            }
+        }
+        missing[t] = !there;
+        if (!there)
+            missing[kMaxMembers] = 1; // every writer stores the same
+    }
+    __syncthreads();
+    if (missing[kMaxMembers])
+        for (uint32_t m = 0; m < members; ++m)
+            if (missing[m]) // uniform
+            {
+                double r[N];
+                recompute(m, r);
+                if (t == m)
+                {
+#pragma unroll
+                    for (int k = 0; k < N; ++k)
+                        s[k] = r[k];
+                }
+            }
+    team_sum<TEAM>(s, lds);
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+        v[k] = s[k];
+}
+
+// The terms of one vector; `skip` leading elements belong to the vector before it.
+template <typename T, int VEC>
+__device__ __forceinline__ void add_forward_terms(double (&s)[2], const T (&v)[VEC], uint32_t skip)
+{
+#pragma unroll
+    for (int j = 0; j < VEC; ++j)
+        if (j >= static_cast<int>(skip))
+        {
+            const double d = static_cast<double>(v[j]);
+            s[0] += d;
+            s[1] = __builtin_fma(d, d, s[1]);
+        }
+}
+
+template <typename T, int VEC>
+__device__ __forceinline__ void add_backward_terms(double (&s)[4], const T (&x)[VEC], const T (&d)[VEC], uint32_t skip,
+                                                   T m, T sc, T inv_stdev)
+{
+#pragma unroll
+    for (int j = 0; j < VEC; ++j)
+        if (j >= static_cast<int>(skip))
+        {
+            const T xm = x[j] - m;
+            const T dxhat = d[j] * sc;
+            const double dd = static_cast<double>(d[j]);
+            s[0] = __builtin_fma(dd, static_cast<double>(xm * inv_stdev), s[0]);
+            s[1] += dd;
+            s[2] += static_cast<double>(dxhat);
+            s[3] += static_cast<double>(dxhat * xm);
+        }
+}
+
+template <typename T, int TEAM, int K, bool STREAM>
+__global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometry g, const OnceForward<T> a,
+                                                                      unsigned long long* slots)
+{
+    constexpr int VEC = 16 / sizeof(T);
+    constexpr int kWaves = TEAM / kWaveSize;
+    __shared__ double lds[3][2 * kWaves];
+    __shared__ uint32_t missing[kMaxMembers + 1];
+    const uint32_t c = fastdiv(blockIdx.x, g.members);
+    const uint32_t member = blockIdx.x - c * g.members.divisor;
+    const T* const x = a.x + c * g.once.stride_c;
+    const uint32_t first = member * g.span;
+    const uint32_t end = first + g.span < g.once.vectors ? first + g.span : g.once.vectors;
+    T v[K][VEC];
+    uint32_t at[K];
+    const auto live = [&](int u) { return first + u * TEAM < end && first + u * TEAM + threadIdx.x < end; };
+#pragma unroll
+    for (int u = 0; u < K; ++u)
+        if (live(u))
+        {
+            at[u] = once_place<VEC>(g.once, first + u * TEAM + threadIdx.x);
+            load_vec<T, VEC, false>(x + (at[u] >> 2), v[u]);
+        }
+    double s[2] = {0.0, 0.0};
+#pragma unroll
+    for (int u = 0; u < K; ++u)
+        if (live(u))
+            add_forward_terms<T, VEC>(s, v[u], at[u] & 3);
+    team_sum<TEAM>(s, lds[0]);
+    team_exchange<TEAM, 2>(s, g, c, member, slots, lds[1], missing, [&](uint32_t other, double (&r)[2]) {
+        r[0] = r[1] = 0.0;
+        const uint32_t stop = (other + 1) * g.span < g.once.vectors ? (other + 1) * g.span : g.once.vectors;
+        for (uint32_t i = other * g.span + threadIdx.x; i < stop; i += TEAM)
+        {
+            const uint32_t p = once_place<VEC>(g.once, i);
+            T w[VEC];
+            load_vec<T, VEC, false>(x + (p >> 2), w);
+            add_forward_terms<T, VEC>(r, w, p & 3);
+        }
+        __syncthreads(); // lds[2] may still be read
+        team_sum<TEAM>(r, lds[2]);
+    });
+    T m, variance;
+    sums_to_mean_var(static_cast<T>(s[0]), static_cast<T>(s[1]), a.n, &m, &variance);
+    if (member == 0 && threadIdx.x == 0)
+    {
+        a.mean[c] = m;
+        a.var[c] = variance;
+        a.running_mean[c] = fma_t(a.decay, a.running_mean[c], (T(1) - a.decay) * m);
+        a.running_var[c] = fma_t(a.decay, a.running_var[c], (T(1) - a.decay) * variance);
+    }
+    const T inv_stdev = inv_sqrt_t(variance + a.epsilon);
+    const T sc = a.scale[c], bi = a.bias[c];
+    T* const y = a.y + c * g.once.stride_c;
+#pragma unroll
+    for (int u = 0; u < K; ++u)
+        if (live(u))
+        {
+#pragma unroll
+            for (int j = 0; j < VEC; ++j)
+                v[u][j] = fma_t((v[u][j] - m) * inv_stdev, sc, bi);
+            store_once<T, VEC, STREAM>(y + (at[u] >> 2), v[u]);
+        }
+}
+
+template <typename T, int TEAM, int K, bool STREAM>
+__global__ __launch_bounds__(TEAM) void bn_team_backward_kernel(const TeamGeometry g, const OnceBackward<T> a,
+                                                                       unsigned long long* slots)
+{
+    constexpr int VEC = 16 / sizeof(T);
+    constexpr int kWaves = TEAM / kWaveSize;
+    __shared__ double lds[3][4 * kWaves];
+    __shared__ uint32_t missing[kMaxMembers + 1];
+    const uint32_t c = fastdiv(blockIdx.x, g.members);
+    const uint32_t member = blockIdx.x - c * g.members.divisor;
+    const int64_t base = c * g.once.stride_c;
+    const uint32_t first = member * g.span;
+    const uint32_t end = first + g.span < g.once.vectors ? first + g.span : g.once.vectors;
+    T xv[K][VEC], dv[K][VEC];
+    uint32_t at[K];
+    const auto live = [&](int u) { return first + u * TEAM < end && first + u * TEAM + threadIdx.x < end; };
+#pragma unroll
+    for (int u = 0; u < K; ++u)
+        if (live(u))
+        {
+            at[u] = once_place<VEC>(g.once, first + u * TEAM + threadIdx.x);
+            load_vec<T, VEC, false>(a.x + base + (at[u] >> 2), xv[u]);
+            load_vec<T, VEC, false>(a.dy + base + (at[u] >> 2), dv[u]);
+        }
+    const T m = a.mean[c];
+    const T sc = a.scale[c];
+    const T inv_stdev = inv_sqrt_t(a.var[c] + a.epsilon);
+    const T dvar_factor = inv_stdev * inv_stdev * inv_stdev / T(2);
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int u = 0; u < K; ++u)
+        if (live(u))
+            add_backward_terms<T, VEC>(s, xv[u], dv[u], at[u] & 3, m, sc, inv_stdev);
+    team_sum<TEAM>(s, lds[0]);
+    team_exchange<TEAM, 4>(s, g, c, member, slots, lds[1], missing, [&](uint32_t other, double (&r)[4]) {
+        r[0] = r[1] = r[2] = r[3] = 0.0;
+        const uint32_t stop = (other + 1) * g.span < g.once.vectors ? (other + 1) * g.span : g.once.vectors;
+        for (uint32_t i = other * g.span + threadIdx.x; i < stop; i += TEAM)
+        {
+            const uint32_t p = once_place<VEC>(g.once, i);
+            T w[VEC], d[VEC];
+            load_vec<T, VEC, false>(a.x + base + (p >> 2), w);
+            load_vec<T, VEC, false>(a.dy + base + (p >> 2), d);
+            add_backward_terms<T, VEC>(r, w, d, p & 3, m, sc, inv_stdev);
+        }
+        __syncthreads(); // lds[2] may still be read
+        team_sum<TEAM>(r, lds[2]);
+    });
+    const T dmean = static_cast<T>(s[2] * -static_cast<double>(inv_stdev));
+    const T dvar = static_cast<T>(s[3] * -static_cast<double>(dvar_factor));
+    if (member == 0 && threadIdx.x == 0)
+    {
+        a.dscale[c] = static_cast<T>(s[0]);
+        a.dbias[c] = static_cast<T>(s[1]);
+        a.dmean[c] = dmean;
+        a.dvar[c] = dvar;
+    }
+    const T dmean_term = dmean / a.n;
+    const T dvar_term = dvar * T(2) / a.n_minus_1;
+#pragma unroll
+    for (int u = 0; u < K; ++u)
+        if (live(u))
+        {
+#pragma unroll
+            for (int j = 0; j < VEC; ++j)
+                xv[u][j] = fma_t(xv[u][j] - m, dvar_term, fma_t(dv[u][j] * sc, inv_stdev, dmean_term));
+            store_once<T, VEC, STREAM>(a.dx + base + (at[u] >> 2), xv[u]);
+        }
+}

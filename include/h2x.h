@@ -421,11 +421,13 @@ int h2x_bn_backward_local_strided(h2x_dtype dtype,
                                   h2x_stream_t stream);
 
 /**
- * The same again, in one launch each way where a channel fits the registers of
- * a workgroup (float tensors that lie alike, up to about 80000 elements a channel
- * forward and 65000 backward); otherwise what h2x_bn_forward_local_strided and
- * h2x_bn_backward_local_strided do.  The terms of the sums are the same and are
- * added in fp64, in another order.
+ * The same again for float tensors that lie alike, reading every element once where
+ * a channel is held in registers between the sums and the output: by one workgroup
+ * (up to about 80000 elements a channel forward and 65000 backward) or by a team of
+ * workgroups (larger channels, up to about 4 million elements forward and 2 million
+ * backward, outputs that do not overlap inputs); otherwise what
+ * h2x_bn_forward_local_strided and h2x_bn_backward_local_strided do.  The terms of
+ * the sums are the same and are added in fp64, in another order.
  */
 int h2x_bn_forward_once(h2x_dtype dtype,
                                  int num_samples,
@@ -463,6 +465,64 @@ int h2x_bn_backward_once(h2x_dtype dtype,
                                   double epsilon,
                                   void* workspace,
                                   h2x_stream_t stream);
+
+/**
+ * By a team of workgroups a channel, or H2X_ERR_UNSUPPORTED where the tensors are
+ * not fit for that.  A workgroup that has looked max_polls times without finding
+ * the sums of all others works the missing ones out itself, with the same result;
+ * 0 makes each do so at once.
+ */
+int h2x_bn_forward_team(h2x_dtype dtype,
+                        int num_samples,
+                        const h2x_tensor_geometry* x_geometry,
+                        const h2x_tensor_geometry* y_geometry,
+                        const void* x,
+                        const void* scale,
+                        const void* bias,
+                        size_t num_per_sum,
+                        double decay,
+                        double epsilon,
+                        void* mean,
+                        void* var,
+                        void* running_mean,
+                        void* running_var,
+                        void* y,
+                        void* workspace,
+                        unsigned int max_polls,
+                        h2x_stream_t stream);
+int h2x_bn_backward_team(h2x_dtype dtype,
+                         int num_samples,
+                         size_t num_per_sum,
+                         const h2x_tensor_geometry* x_geometry,
+                         const h2x_tensor_geometry* dy_geometry,
+                         const h2x_tensor_geometry* dx_geometry,
+                         const void* x,
+                         const void* dy,
+                         const void* mean,
+                         const void* var,
+                         const void* scale,
+                         void* dscale,
+                         void* dbias,
+                         void* dmean,
+                         void* dvar,
+                         void* dx,
+                         double epsilon,
+                         void* workspace,
+                         unsigned int max_polls,
+                         h2x_stream_t stream);
+
+/**
+ * Plays on the host which elements of a float tensor (offsets from its first interior
+ * element, below `elements`) the workgroups that hold channels in registers count
+ * into the sums (how often) and store, in pieces of member_vectors vectors (0:
+ * whole channels).  H2X_ERR_UNSUPPORTED: such tensors run in two launches.
+ */
+int h2x_bn_audit_once(int num_samples,
+                      const h2x_tensor_geometry* geometry,
+                      unsigned int member_vectors,
+                      unsigned char* counted,
+                      unsigned char* stored,
+                      size_t elements);
 
 /**
  * The local part of a haloed tensor as it lies in memory: the real (allocated)

@@ -1,0 +1,131 @@
+"""Batch-norm with channels held in registers, by one workgroup or by a team, against the two-launch
+calls, at the edges of the variants (vectors a channel: the tile sizes and one more)."""
+import ctypes
+
+import pytest
+
+from dihydrogen_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+
+class _Problem:
+    """One haloed (or dense) N, C, D, H, W tensor set and the three ways to run it."""
+
+    def __init__(self, n, c, d, h, w, halo=0):
+        import torch
+        self.torch, self.n, self.c = torch, n, c
+        hd = halo if d > 1 else 0
+        real = (n, c, d + 2 * hd, h + 2 * halo, w + 2 * halo)
+        g = torch.Generator(device="cuda").manual_seed(n + c + w)
+        self.x, self.dy = (torch.randn(real, device="cuda", generator=g) for _ in range(2))
+        self.x += 0.5
+        self.inner = (slice(None), slice(None), slice(hd, hd + d), slice(halo, halo + h), slice(halo, halo + w))
+        first = hd * self.x.stride(2) + halo * self.x.stride(3) + halo
+        self.offset = first * self.x.element_size()
+        self.geometry = capi.TensorGeometry()
+        self.geometry.num_dims = 5
+        for i, (e, s) in enumerate(zip((w, h, d, c, n), reversed(self.x.stride()))):
+            self.geometry.local_shape[i], self.geometry.strides[i] = e, s
+        self.per = n * d * h * w
+        self.scale = torch.empty(c, device="cuda").uniform_(0.5, 1.5, generator=g)
+        self.bias = torch.empty(c, device="cuda").normal_(0, 0.1, generator=g)
+        self.ws = torch.empty(capi.load().h2x_bn_workspace_bytes(c), dtype=torch.uint8, device="cuda")
+
+    def run(self, kind, *polls, in_place=False):
+        """(outputs, halo untouched?) of h2x_bn_{forward,backward}_<kind>."""
+        torch, lib = self.torch, capi.load()
+        gp = ctypes.byref(self.geometry)
+        vec = lambda v: torch.full_like(self.scale, v)
+        mean, var, rm, rv = vec(float("nan")), vec(float("nan")), vec(0.25), vec(0.75)
+        grads = [vec(float("nan")) for _ in range(4)]
+        x = self.x.clone()
+        y = x if in_place else torch.full_like(x, 7)
+        at = lambda t: t.data_ptr() + self.offset
+        p = lambda t: t.data_ptr()
+        st = torch.cuda.current_stream().cuda_stream
+        status = getattr(lib, "h2x_bn_forward_" + kind)(
+            capi.F32, self.n, gp, gp, at(x), p(self.scale), p(self.bias), self.per, 0.9, 1e-5, p(mean), p(var), p(rm),
+            p(rv), at(y), p(self.ws), *polls, st)
+        assert status == 0, status
+        if in_place:
+            x = self.x.clone()
+        dx = x if in_place else torch.full_like(x, 7)
+        status = getattr(lib, "h2x_bn_backward_" + kind)(
+            capi.F32, self.n, self.per, gp, gp, gp, at(x), at(self.dy), p(mean), p(var), p(self.scale),
+            *[p(t) for t in grads], at(dx), 1e-5, p(self.ws), *polls, st)
+        assert status == 0, status
+        torch.cuda.synchronize()
+        for out in (y, dx):
+            if not in_place:
+                rest = out.clone()
+                rest[self.inner] = 7
+                assert bool((rest == 7).all()), "stored outside the interior"
+        return [y[self.inner], dx[self.inner], mean, var, rm, rv] + grads
+
+
+def _close(got, want):
+    """The fp64 sums differ by their order only (2^-52 of the sum of the terms' magnitudes), so the statistics by at
+    most a rounding to float; a handful of operations follow: 16 units in the last place of the
+    largest value."""
+    for a, b in zip(got, want):
+        assert bool(((a - b).abs() <= 16 * 1.2e-7 * b.abs().max()).all())
+
+
+# vectors a channel of the variants' edges; 96 channels reach the largest ones
+ONCE = [(1, 5, 1, 16, 32), (1, 5, 1, 3, 172), (2, 3, 1, 32, 64), (3, 3, 1, 37, 37), (8, 3, 1, 32, 32),
+        (8, 3, 1, 32, 64), (5, 2, 1, 59, 111), (4, 97, 1, 128, 128), (4, 96, 1, 128, 129), (5, 96, 1, 128, 128),
+        (40, 1030, 1, 7, 7), (3, 7, 1, 2, 2)]
+
+
+@pytest.mark.parametrize("in_place", [False, True])
+@pytest.mark.parametrize("shape", ONCE)
+def test_channel_in_one_workgroup(shape, in_place):
+    p = _Problem(*shape)
+    _close(p.run("once", in_place=in_place), p.run("local_strided"))
+
+
+@pytest.mark.parametrize("shape", [(2, 5, 6, 9, 11), (4, 70, 4, 5, 30), (2, 96, 16, 32, 61)])
+def test_haloed_channel_in_one_workgroup(shape):
+    p = _Problem(*shape, halo=2)
+    _close(p.run("once"), p.run("local_strided"))
+
+
+# few members and many, a last member that is nearly empty, haloed rows; the last three
+# reach every variant and both kinds of stores by the dispatch's own rule
+TEAM = [(1, 3, 1, 64, 300, 0), (2, 2, 40, 32, 32, 0), (1, 2, 33, 35, 37, 1),
+        (3, 2, 1, 257, 129, 0), (2, 3, 17, 18, 19, 2), (31, 2, 64, 32, 32, 0),
+        (2, 32, 48, 48, 48, 0), (5, 24, 48, 48, 48, 0), (2, 64, 45, 62, 62, 1)]
+
+
+@pytest.mark.parametrize("shape", TEAM)
+def test_channel_in_a_team(shape):
+    """As the two-launch calls, and with the same bits when no member waits and each works out
+    the sums of all others."""
+    import torch
+    p = _Problem(*shape)
+    by_team = p.run("team", 2048)
+    _close(by_team, p.run("local_strided"))
+    small = p.x.numel() < 4_000_000  # every member reads its whole channel
+    if small:
+        for a, b in zip(by_team, p.run("team", 0)):
+            assert torch.equal(a, b)
+    _close(p.run("once"), by_team)
+
+
+def test_nan_reaches_the_whole_channel_of_a_team_only():
+    import torch
+    p = _Problem(2, 3, 40, 32, 32)
+    p.x[1, 1, 30, 2, 3] = float("nan")
+    out, ref = p.run("team", 2048), p.run("local_strided")
+    for a, b in zip(out, ref):
+        assert torch.equal(torch.isnan(a), torch.isnan(b))
+
+
+def test_overlapping_outputs_are_not_for_teams():
+    p = _Problem(2, 2, 40, 32, 32)
+    x, lib, gp = p.x.data_ptr(), capi.load(), ctypes.byref(p.geometry)
+    v = [p.scale.clone().data_ptr() for _ in range(4)]
+    assert lib.h2x_bn_forward_team(capi.F32, 2, gp, gp, x, p.scale.data_ptr(), p.bias.data_ptr(), p.per, 0.9, 1e-5, *v, x,
+                                   p.ws.data_ptr(), 2048, None) == -2  # unsupported
+    _close(p.run("once", in_place=True), p.run("local_strided"))
