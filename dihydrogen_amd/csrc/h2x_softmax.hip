@@ -8,7 +8,7 @@
 // 4*VEC-byte accesses and no LDS staging; the reference stages a
 // C x 256 tile in LDS and walks it three times
 // (legacy/src/dnn_backend/softmax.cu:538-593,621-669).  Above 32 channels the
-// four waves of a workgroup share the channels of 64 * VEC pixels, still in
+// waves of a workgroup share the channels of 64 * VEC pixels, still in
 // registers; channel counts beyond the largest such tile fall back to a kernel
 // that re-reads its inputs; tensors with one pixel per sample have kernels
 // that put the channels, which are contiguous then, on the lanes of a wave or,
@@ -379,15 +379,32 @@ __global__ __launch_bounds__(kBlockSize) void softmax_bwd_wide_kernel(
         }
 }
 
+// The waves' partial sums in place i, added pairwise: a chain of WAVES additions would give
+// back the accuracy that the waves' shorter chains gain.
+template <typename T, int WAVES, int N>
+__device__ __forceinline__ T sum_of_waves(const T (&lds)[WAVES][N], int i)
+{
+    T t[WAVES];
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+        t[w] = lds[w][i];
+#pragma unroll
+    for (int step = WAVES / 2; step >= 1; step /= 2)
+#pragma unroll
+        for (int w = 0; w < step; ++w)
+            t[w] += t[w + step];
+    return t[0];
+}
+
 // forward, up to WAVES * CPW channels, register-resident.  A workgroup serves
-// 64 * VEC neighbouring pixels; its WAVES (four, or eight above 512 channels)
-// waves share the channels (wave g takes c = g, g + WAVES, ...: CPW of them at
-// most) and keep their values in registers, so
-// x is read once; maxima and sums are combined through LDS in wave order.  The
-// arithmetic, partial sums included, is that of softmax_fwd_wide_kernel, which
-// re-reads its tile twice and whose tiles of 64 * C elements the L2 does not
-// hold once every CU runs eight of them (N 16, C 150, 128 x 128: 100 us there,
-// 60 us with the tile in registers).
+// 64 * VEC neighbouring pixels; its WAVES waves share the channels (wave g takes
+// c = g, g + WAVES, ...: CPW of them at most) and keep their values in registers,
+// so x is read once; maxima and sums are combined through LDS in a fixed order.
+// softmax_fwd_wide_kernel, with the same terms, re-reads its tile twice, and its
+// tiles of 64 * C elements the L2 does not hold once every CU runs eight of them
+// (N 16, C 150, 128 x 128: 100 us there, 63 us with the tile in registers).  Bound by
+// memory where there are several tiles a CU, else by a wave's chain of loads,
+// exponentials and sums.
 template <typename T, int VEC, int CPW, int WAVES>
 __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
     const T* __restrict__ x, T* __restrict__ y, int num_channels, size_t spatial, int flat_samples)
@@ -457,11 +474,7 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
 #pragma unroll
     for (int j = 0; j < VEC; ++j)
     {
-        T t = lds[0][lane * VEC + j];
-#pragma unroll
-        for (int w = 1; w < WAVES; ++w)
-            t += lds[w][lane * VEC + j];
-        inv[j] = T(1) / t;
+        inv[j] = T(1) / sum_of_waves<T, WAVES>(lds, lane * VEC + j);
     }
     if (active)
     {
@@ -480,7 +493,9 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
     }
 }
 
-// backward likewise: y and dy of up to WAVES * CPW channels in registers.
+// backward likewise: y and dy of up to WAVES * CPW channels in registers.  All of y is
+// asked for before any of dy: alternating, the wave waited more often (N 4, C 150,
+// 65 x 97 in four waves 15.9 us against 10.2).
 template <typename T, int VEC, int CPW, int WAVES>
 __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
     const T* __restrict__ y, const T* __restrict__ dy, T* __restrict__ dx, int num_channels,
@@ -509,10 +524,11 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
 #pragma unroll
         for (int k = 0; k < CPW; ++k)
             if (g + k * WAVES < num_channels)
-            {
                 yv[k] = P::load(yp + static_cast<size_t>(g + k * WAVES) * spatial);
+#pragma unroll
+        for (int k = 0; k < CPW; ++k)
+            if (g + k * WAVES < num_channels)
                 gv[k] = P::load(gp + static_cast<size_t>(g + k * WAVES) * spatial);
-            }
 #pragma unroll
         for (int k = 0; k < CPW; ++k)
             if (g + k * WAVES < num_channels)
@@ -527,11 +543,7 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
 #pragma unroll
     for (int j = 0; j < VEC; ++j)
     {
-        T t = lds[0][lane * VEC + j];
-#pragma unroll
-        for (int w = 1; w < WAVES; ++w)
-            t += lds[w][lane * VEC + j];
-        dp[j] = t;
+        dp[j] = sum_of_waves<T, WAVES>(lds, lane * VEC + j);
     }
     if (active)
     {
@@ -777,21 +789,16 @@ void launch_bwd(const T* y, const T* dy, T* dx, int n, int c, size_t s, hipStrea
         <<<pixel_grid_xcd(s, VEC, n, flat), kBlockSize, 0, st>>>(y, dy, dx, c, s, flat);
 }
 
-// Which kernel serves which channel count (float; measured on MI355X).  Up to
-// 32 channels a thread keeps all channels of its pixels (softmax_*_reg_kernel:
-// config 4, 21 channels, 28 / 40 us).  Beyond, the four waves of a workgroup
-// share the channels (softmax_*_split_kernel) with the smallest register tile
-// that holds them and two pixels a lane where the geometry allows: against one
-// thread per pixel with 64 or 128 channels in registers, N 4, C 100, 256 x 256
-// takes 34 instead of 68 us forward and 53 instead of 63 us backward; against
-// the re-reading kernel N 16, C 150, 128 x 128 takes 60 instead of 100 us and 89
-// instead of 150 us, N 8, C 256, 64 x 64 18 instead of 59 us and 19 instead of
-// 55 us.  Tiles wider than needed cost time (every lane walks the whole tile
-// under a predicate), hence the steps of 16.  More channels than the largest
-// tile holds (eight waves: 1024 forward, 768 backward; double: 256) take the
-// re-reading kernel.
-template <typename T, int VEC, int CPW, int WAVES = kWavesPerBlock>
-int launch_fwd_split(const T* x, T* y, int n, int c, size_t s, hipStream_t st)
+// Which kernel serves which channel count (measured on MI355X).  Up to 32 channels a
+// thread keeps all channels of its pixels (softmax_*_reg_kernel: 21 channels of
+// N 16, 256 x 256 in 28 / 40 us).  Beyond, the waves of a workgroup share the channels
+// (softmax_*_split_kernel) with the smallest register tile that holds them: tiles wider
+// than needed cost time, since every lane walks the whole tile under a predicate.  Eight
+// waves against four, N 4, C 150, 65 x 97: forward 10.2 and 11.7 us; N 1: 5.7 and 8.0; N 16:
+// 29.8 and 34.3.  More channels than the largest tile holds (1024 forward, 768 backward;
+// double: 512 and 256) take the re-reading kernel.
+template <int VEC, int CPW, int WAVES, typename T>
+int launch_split(const T* x, T* y, int n, int c, size_t s, hipStream_t st)
 {
     const int flat = VEC == 1 ? flat_samples(n, s) : 0;
     softmax_fwd_split_kernel<T, VEC, CPW, WAVES>
@@ -799,13 +806,72 @@ int launch_fwd_split(const T* x, T* y, int n, int c, size_t s, hipStream_t st)
     return launch_status();
 }
 
-template <typename T, int VEC, int CPW, int WAVES = kWavesPerBlock>
-int launch_bwd_split(const T* y, const T* dy, T* dx, int n, int c, size_t s, hipStream_t st)
+template <int VEC, int CPW, int WAVES, typename T>
+int launch_split(const T* y, const T* dy, T* dx, int n, int c, size_t s, hipStream_t st)
 {
     const int flat = VEC == 1 ? flat_samples(n, s) : 0;
     softmax_bwd_split_kernel<T, VEC, CPW, WAVES>
         <<<wide_grid(s, VEC, n, flat), WAVES * kWaveSize, 0, st>>>(y, dy, dx, c, s, flat);
     return launch_status();
+}
+
+constexpr int kNoSplit = -1000; // not the status of a launch
+
+// The split kernel for 33 channels and more, or kNoSplit.  Eight waves with up to 64
+// channels each; sixteen, whose chains of exponentials and sums are half as long, where
+// the tiles of 64 pixels are no more than the CUs (N 4, C 500, 21 x 21: forward 10.6 us, backward
+// 9.1, eight waves 12.4 and 11.3; N 8, C 400, 64 x 64: 32.3 and 36.8, eight waves 30.1 and 35.3),
+// and beyond what eight hold.  Two pixels a lane where that leaves two tiles a CU
+// forward, one backward (N 1, C 60, 384 x 384, 1152 tiles of two pixels a lane: 13.3 and 22.2 us,
+// one pixel 14.3 and 25.4; N 8, C 256, 64 x 64, 256 of them: 17.8 and 21.6, one pixel 16.5 and 23.7).
+template <typename T, typename... P>
+int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
+{
+    constexpr bool kForward = sizeof...(P) == 2;
+    constexpr bool kFloat = sizeof(T) == 4;
+    const int flat = flat_samples(n, s);
+    const size_t pixels = flat > 0 ? s * n : s, samples = flat > 0 ? 1 : n;
+    const size_t tiles = (pixels + kWaveSize - 1) / kWaveSize * samples;
+    if ((tiles <= 256 && c > 64) || c > (kFloat ? 512 : 256))
+    {
+        if (c <= 128) return launch_split<1, 8, 16>(p..., n, c, s, st);
+        if (c <= 192) return launch_split<1, 12, 16>(p..., n, c, s, st);
+        if (c <= 256) return launch_split<1, 16, 16>(p..., n, c, s, st);
+        if constexpr (kFloat || kForward)
+        {
+            if (c <= 384) return launch_split<1, 24, 16>(p..., n, c, s, st);
+            if (c <= 512) return launch_split<1, 32, 16>(p..., n, c, s, st);
+        }
+        if constexpr (kFloat)
+        {
+            if (c <= 768) return launch_split<1, 48, 16>(p..., n, c, s, st);
+        }
+        if constexpr (kFloat && kForward)
+        {
+            if (c <= 1024) return launch_split<1, 64, 16>(p..., n, c, s, st);
+        }
+        return kNoSplit;
+    }
+    if constexpr (kFloat)
+    {
+        if (v >= 2 && c <= 256 && (s + 2 * kWaveSize - 1) / (2 * kWaveSize) * n >= (kForward ? 512 : 256))
+        {
+            if (c <= 64) return launch_split<2, 8, 8>(p..., n, c, s, st);
+            if (c <= 128) return launch_split<2, 16, 8>(p..., n, c, s, st);
+            if (c <= 192) return launch_split<2, 24, 8>(p..., n, c, s, st);
+            return launch_split<2, 32, 8>(p..., n, c, s, st);
+        }
+    }
+    if (c <= 64) return launch_split<1, 8, 8>(p..., n, c, s, st);
+    if (c <= 128) return launch_split<1, 16, 8>(p..., n, c, s, st);
+    if (c <= 192) return launch_split<1, 24, 8>(p..., n, c, s, st);
+    if (c <= 256) return launch_split<1, 32, 8>(p..., n, c, s, st);
+    if constexpr (kFloat)
+    {
+        if (c <= 384) return launch_split<1, 48, 8>(p..., n, c, s, st);
+        if (c <= 512) return launch_split<1, 64, 8>(p..., n, c, s, st);
+    }
+    return kNoSplit;
 }
 
 template <typename T>
@@ -855,22 +921,10 @@ int forward_impl(int n, int c, size_t s, const void* xv, void* yv, hipStream_t s
             if (c <= 8) H2X_FWD(2, 8);
             if (c <= 16) H2X_FWD(2, 16);
             if (c <= 32) H2X_FWD(2, 32);
-            if (c <= 64) return launch_fwd_split<T, 2, 16>(x, y, n, c, s, st);
-            if (c <= 128) return launch_fwd_split<T, 2, 32>(x, y, n, c, s, st);
-            if (c <= 192) return launch_fwd_split<T, 2, 48>(x, y, n, c, s, st);
-            if (c <= 256) return launch_fwd_split<T, 2, 64>(x, y, n, c, s, st);
         }
         if (c <= 8) H2X_FWD(1, 8);
         if (c <= 16) H2X_FWD(1, 16);
         if (c <= 32) H2X_FWD(1, 32);
-        if (c <= 64) return launch_fwd_split<T, 1, 16>(x, y, n, c, s, st);
-        if (c <= 128) return launch_fwd_split<T, 1, 32>(x, y, n, c, s, st);
-        if (c <= 192) return launch_fwd_split<T, 1, 48>(x, y, n, c, s, st);
-        if (c <= 256) return launch_fwd_split<T, 1, 64>(x, y, n, c, s, st);
-        if (c <= 384) return launch_fwd_split<T, 1, 96>(x, y, n, c, s, st);
-        if (c <= 512) return launch_fwd_split<T, 1, 128>(x, y, n, c, s, st);
-        if (c <= 768) return launch_fwd_split<T, 1, 96, 8>(x, y, n, c, s, st);
-        if (c <= 1024) return launch_fwd_split<T, 1, 128, 8>(x, y, n, c, s, st);
     }
     else
     {
@@ -883,12 +937,11 @@ int forward_impl(int n, int c, size_t s, const void* xv, void* yv, hipStream_t s
         if (c <= 8) H2X_FWD(1, 8);
         if (c <= 16) H2X_FWD(1, 16);
         if (c <= 32) H2X_FWD(1, 32);
-        if (c <= 64) return launch_fwd_split<T, 1, 16>(x, y, n, c, s, st);
-        if (c <= 128) return launch_fwd_split<T, 1, 32>(x, y, n, c, s, st);
-        if (c <= 192) return launch_fwd_split<T, 1, 48>(x, y, n, c, s, st);
-        if (c <= 256) return launch_fwd_split<T, 1, 64>(x, y, n, c, s, st);
     }
 #undef H2X_FWD
+    const int status = launch_split_for<T>(v4, n, c, s, st, x, y);
+    if (status != kNoSplit)
+        return status;
     const int flat = flat_samples(n, s);
     softmax_fwd_wide_kernel<T><<<wide_grid(s, 1, n, flat), kBlockSize, 0, st>>>(x, y, c, s, flat);
     return launch_status();
@@ -940,21 +993,10 @@ int backward_impl(int n, int c, size_t s, const void* yv, const void* dyv, void*
             if (c <= 8) H2X_BWD(2, 8);
             if (c <= 16) H2X_BWD(2, 16);
             if (c <= 32) H2X_BWD(2, 32);
-            if (c <= 64) return launch_bwd_split<T, 2, 16>(y, dy, dx, n, c, s, st);
-            if (c <= 128) return launch_bwd_split<T, 2, 32>(y, dy, dx, n, c, s, st);
-            if (c <= 192) return launch_bwd_split<T, 2, 48>(y, dy, dx, n, c, s, st);
-            if (c <= 256) return launch_bwd_split<T, 2, 64>(y, dy, dx, n, c, s, st);
         }
         if (c <= 8) H2X_BWD(1, 8);
         if (c <= 16) H2X_BWD(1, 16);
         if (c <= 32) H2X_BWD(1, 32);
-        if (c <= 64) return launch_bwd_split<T, 1, 16>(y, dy, dx, n, c, s, st);
-        if (c <= 128) return launch_bwd_split<T, 1, 32>(y, dy, dx, n, c, s, st);
-        if (c <= 192) return launch_bwd_split<T, 1, 48>(y, dy, dx, n, c, s, st);
-        if (c <= 256) return launch_bwd_split<T, 1, 64>(y, dy, dx, n, c, s, st);
-        if (c <= 384) return launch_bwd_split<T, 1, 96>(y, dy, dx, n, c, s, st);
-        if (c <= 512) return launch_bwd_split<T, 1, 128>(y, dy, dx, n, c, s, st);
-        if (c <= 768) return launch_bwd_split<T, 1, 96, 8>(y, dy, dx, n, c, s, st);
     }
     else
     {
@@ -966,12 +1008,11 @@ int backward_impl(int n, int c, size_t s, const void* yv, const void* dyv, void*
         if (c <= 8) H2X_BWD(1, 8);
         if (c <= 16) H2X_BWD(1, 16);
         if (c <= 32) H2X_BWD(1, 32);
-        if (c <= 64) return launch_bwd_split<T, 1, 16>(y, dy, dx, n, c, s, st);
-        if (c <= 128) return launch_bwd_split<T, 1, 32>(y, dy, dx, n, c, s, st);
-        if (c <= 192) return launch_bwd_split<T, 1, 48>(y, dy, dx, n, c, s, st);
-        if (c <= 256) return launch_bwd_split<T, 1, 64>(y, dy, dx, n, c, s, st);
     }
 #undef H2X_BWD
+    const int status = launch_split_for<T>(v4, n, c, s, st, y, dy, dx);
+    if (status != kNoSplit)
+        return status;
     const int flat = flat_samples(n, s);
     softmax_bwd_wide_kernel<T><<<wide_grid(s, 1, n, flat), kBlockSize, 0, st>>>(y, dy, dx, c, s, flat);
     return launch_status();
