@@ -115,6 +115,7 @@ PyMethodDef s_methods[] = {H2X_ENTRY(h2x_bn_channel_sums_and_sqsums),
                            H2X_ENTRY(h2x_softmax_instance_exp),
                            H2X_ENTRY(h2x_softmax_instance_normalize),
                            H2X_ENTRY(h2x_softmax_instance_forward_local),
+                           H2X_ENTRY(h2x_softmax_instance_backward_local),
                            H2X_ENTRY(h2x_softmax_instance_dot),
                            H2X_ENTRY(h2x_softmax_instance_gradient),
                            H2X_ENTRY(h2x_halo_pack_or_unpack_batched),

@@ -17,6 +17,7 @@
 
 #include <cfloat>
 #include <cmath>
+#include <type_traits>
 
 namespace h2x
 {
@@ -574,13 +575,77 @@ __device__ __forceinline__ T wave_butterfly_sum(T v)
     return v;
 }
 
-template <typename T, int CPL>
-__global__ __launch_bounds__(kBlockSize) void softmax_fwd_row_kernel(
+// Maximum or sum over a workgroup: the lanes of a wave as a butterfly, the waves pairwise.
+template <int WAVES, typename T>
+__device__ __forceinline__ T block_combine(T v, bool is_max, T* lds)
+{
+    const auto both = [is_max](T p, T q) { return is_max ? (q > p ? q : p) : p + q; };
+#pragma unroll
+    for (int m = kWaveSize / 2; m >= 1; m >>= 1)
+        v = both(v, __shfl_xor(v, m, kWaveSize));
+    __syncthreads(); // lds may still be read from the previous call
+    if ((threadIdx.x & (kWaveSize - 1)) == 0)
+        lds[threadIdx.x / kWaveSize] = v;
+    __syncthreads();
+    T r[WAVES];
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+        r[w] = lds[w];
+#pragma unroll
+    for (int step = WAVES / 2; step >= 1; step /= 2)
+#pragma unroll
+        for (int w = 0; w < step; ++w)
+            r[w] = both(r[w], r[w + step]);
+    return r[0];
+}
+
+template <typename T>
+__device__ __forceinline__ T wave_max(T v)
+{
+#pragma unroll
+    for (int d = 1; d < kWaveSize; d *= 2)
+    {
+        const T o = __shfl_xor(v, d, kWaveSize);
+        v = o > v ? o : v;
+    }
+    return v;
+}
+
+// The same over the LANES threads that serve a sample: a wave, or a workgroup of that many threads.
+template <int LANES, typename T>
+__device__ __forceinline__ T lanes_max(T v, T* lds)
+{
+    if constexpr (LANES == kWaveSize)
+        return wave_max(v);
+    else
+        return block_combine<LANES / kWaveSize>(v, true, lds);
+}
+
+template <int LANES, typename T>
+__device__ __forceinline__ T lanes_sum(T v, T* lds)
+{
+    if constexpr (LANES == kWaveSize)
+        return wave_butterfly_sum(v);
+    else
+        return block_combine<LANES / kWaveSize>(v, false, lds);
+}
+
+template <int LANES>
+constexpr int lanes_block()
+{
+    return LANES < kBlockSize ? kBlockSize : LANES;
+}
+
+// LANES: a wave, or a workgroup where a wave would not hold the channels or samples are few
+// (N 16, C 4096: forward 9.0 us, backward 7.3 in a kernel that walked them three times).
+template <typename T, int CPL, int LANES>
+__global__ __launch_bounds__(lanes_block<LANES>()) void softmax_fwd_row_kernel(
     const T* __restrict__ x, T* __restrict__ y, int num_channels, int num_samples)
 {
-    const int lane = threadIdx.x % kWaveSize;
-    const int n = blockIdx.x * kWavesPerBlock + threadIdx.x / kWaveSize;
-    if (n >= num_samples)
+    __shared__ T lds[lanes_block<LANES>() / kWaveSize];
+    const int lane = threadIdx.x % LANES;
+    const int n = blockIdx.x * (lanes_block<LANES>() / LANES) + threadIdx.x / LANES;
+    if (n >= num_samples) // all lanes of a sample
         return;
     const T* xp = x + static_cast<size_t>(n) * num_channels;
     T* yp = y + static_cast<size_t>(n) * num_channels;
@@ -589,43 +654,39 @@ __global__ __launch_bounds__(kBlockSize) void softmax_fwd_row_kernel(
     T mx = kMin;
 #pragma unroll
     for (int k = 0; k < CPL; ++k)
-        if (lane + k * kWaveSize < num_channels)
-            v[k] = xp[lane + k * kWaveSize];
+        if (lane + k * LANES < num_channels)
+            v[k] = xp[lane + k * LANES];
 #pragma unroll
     for (int k = 0; k < CPL; ++k)
-        if (lane + k * kWaveSize < num_channels)
+        if (lane + k * LANES < num_channels)
             mx = v[k] > mx ? v[k] : mx;
-#pragma unroll
-    for (int m = kWaveSize / 2; m >= 1; m >>= 1)
-    {
-        const T o = __shfl_xor(mx, m, kWaveSize);
-        mx = o > mx ? o : mx;
-    }
+    mx = lanes_max<LANES>(mx, lds);
     T sum = T(0);
 #pragma unroll
     for (int k = 0; k < CPL; ++k)
-        if (lane + k * kWaveSize < num_channels)
+        if (lane + k * LANES < num_channels)
         {
             v[k] = exp_t(v[k] - mx);
             sum += v[k];
         }
-    const T inv = T(1) / wave_butterfly_sum(sum);
+    const T inv = T(1) / lanes_sum<LANES>(sum, lds);
 #pragma unroll
     for (int k = 0; k < CPL; ++k)
-        if (lane + k * kWaveSize < num_channels)
+        if (lane + k * LANES < num_channels)
         {
             const T r = v[k] * inv;
-            yp[lane + k * kWaveSize] = r > kMin ? r : kMin;
+            yp[lane + k * LANES] = r > kMin ? r : kMin;
         }
 }
 
-template <typename T, int CPL>
-__global__ __launch_bounds__(kBlockSize) void softmax_bwd_row_kernel(
+template <typename T, int CPL, int LANES>
+__global__ __launch_bounds__(lanes_block<LANES>()) void softmax_bwd_row_kernel(
     const T* __restrict__ y, const T* __restrict__ dy, T* __restrict__ dx, int num_channels,
     int num_samples)
 {
-    const int lane = threadIdx.x % kWaveSize;
-    const int n = blockIdx.x * kWavesPerBlock + threadIdx.x / kWaveSize;
+    __shared__ T lds[lanes_block<LANES>() / kWaveSize];
+    const int lane = threadIdx.x % LANES;
+    const int n = blockIdx.x * (lanes_block<LANES>() / LANES) + threadIdx.x / LANES;
     if (n >= num_samples)
         return;
     const size_t base = static_cast<size_t>(n) * num_channels;
@@ -634,47 +695,26 @@ __global__ __launch_bounds__(kBlockSize) void softmax_bwd_row_kernel(
     T dp = T(0);
 #pragma unroll
     for (int k = 0; k < CPL; ++k)
-        if (lane + k * kWaveSize < num_channels)
+        if (lane + k * LANES < num_channels)
         {
-            yv[k] = y[base + lane + k * kWaveSize];
-            gv[k] = dy[base + lane + k * kWaveSize];
+            yv[k] = y[base + lane + k * LANES];
+            gv[k] = dy[base + lane + k * LANES];
         }
 #pragma unroll
     for (int k = 0; k < CPL; ++k)
-        if (lane + k * kWaveSize < num_channels)
+        if (lane + k * LANES < num_channels)
             dp = fma_t(yv[k], gv[k], dp);
-    dp = wave_butterfly_sum(dp);
+    dp = lanes_sum<LANES>(dp, lds);
 #pragma unroll
     for (int k = 0; k < CPL; ++k)
-        if (lane + k * kWaveSize < num_channels)
-            dx[base + lane + k * kWaveSize] = yv[k] > kMin ? yv[k] * (gv[k] - dp) : T(0);
+        if (lane + k * LANES < num_channels)
+            dx[base + lane + k * LANES] = yv[k] > kMin ? yv[k] * (gv[k] - dp) : T(0);
 }
 
-// One pixel per sample and more channels than a wave holds in registers: a
+// One pixel per sample and more channels than a workgroup holds in registers: a
 // workgroup takes a sample and walks its channels (contiguous) three times
 // forward, twice backward; the re-reads come from the L2.  Thread t adds up the
-// channels t, t + 256, ...; the lanes of a wave are combined as a butterfly and
-// the waves through LDS in wave order.
-template <typename T>
-__device__ __forceinline__ T block_combine(T v, bool is_max, T* lds)
-{
-#pragma unroll
-    for (int m = kWaveSize / 2; m >= 1; m >>= 1)
-    {
-        const T o = __shfl_xor(v, m, kWaveSize);
-        v = is_max ? (o > v ? o : v) : v + o;
-    }
-    __syncthreads(); // lds may still be read from the previous call
-    if ((threadIdx.x & (kWaveSize - 1)) == 0)
-        lds[threadIdx.x / kWaveSize] = v;
-    __syncthreads();
-    T r = lds[0];
-#pragma unroll
-    for (int w = 1; w < kWavesPerBlock; ++w)
-        r = is_max ? (lds[w] > r ? lds[w] : r) : r + lds[w];
-    return r;
-}
-
+// channels t, t + 256, ....
 template <typename T>
 __global__ __launch_bounds__(kBlockSize) void softmax_fwd_long_row_kernel(
     const T* __restrict__ x, T* __restrict__ y, int num_channels)
@@ -686,11 +726,11 @@ __global__ __launch_bounds__(kBlockSize) void softmax_fwd_long_row_kernel(
     T mx = kMin;
     for (int c = threadIdx.x; c < num_channels; c += kBlockSize)
         mx = xp[c] > mx ? xp[c] : mx;
-    mx = block_combine(mx, true, lds);
+    mx = block_combine<kWavesPerBlock>(mx, true, lds);
     T sum = T(0);
     for (int c = threadIdx.x; c < num_channels; c += kBlockSize)
         sum += exp_t(xp[c] - mx);
-    const T inv = T(1) / block_combine(sum, false, lds);
+    const T inv = T(1) / block_combine<kWavesPerBlock>(sum, false, lds);
     for (int c = threadIdx.x; c < num_channels; c += kBlockSize)
     {
         const T r = exp_t(xp[c] - mx) * inv;
@@ -708,7 +748,7 @@ __global__ __launch_bounds__(kBlockSize) void softmax_bwd_long_row_kernel(
     T dp = T(0);
     for (int c = threadIdx.x; c < num_channels; c += kBlockSize)
         dp = fma_t(y[base + c], dy[base + c], dp);
-    dp = block_combine(dp, false, lds);
+    dp = block_combine<kWavesPerBlock>(dp, false, lds);
     for (int c = threadIdx.x; c < num_channels; c += kBlockSize)
     {
         const T yi = y[base + c];
@@ -788,6 +828,9 @@ void launch_bwd(const T* y, const T* dy, T* dx, int n, int c, size_t s, hipStrea
     softmax_bwd_reg_kernel<T, VEC, CMAX>
         <<<pixel_grid_xcd(s, VEC, n, flat), kBlockSize, 0, st>>>(y, dy, dx, c, s, flat);
 }
+
+// More samples than this fill the chip with a wave each.
+constexpr int kManySamples = 2048;
 
 // Which kernel serves which channel count (measured on MI355X).  Up to 32 channels a
 // thread keeps all channels of its pixels (softmax_*_reg_kernel: 21 channels of
@@ -874,28 +917,62 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
     return kNoSplit;
 }
 
+// Calls f(elements a lane, lanes) with constants for samples of `size` contiguous elements that
+// lanes hold in registers: a wave while samples are short, or many (it needs no barrier), else
+// a workgroup, of 1024 threads with up to MAX_LARGE elements each where 256 would have more than 16.
+// SPREAD: a workgroup from 257 elements (the sums are fp64; sums of the data's type keep the order that
+// a wave gives them: N 64, 600 channels 4.5 us, in a workgroup 4.1).
+template <bool SPREAD, int MAX_LARGE = 0, typename F>
+int with_lanes(int n, size_t size, const F& f)
+{
+#define H2X_LANES(CPL, LANES)                                                                      \
+    return f(std::integral_constant<int, CPL>(), std::integral_constant<int, LANES>())
+    if (size <= 1 * kWaveSize) H2X_LANES(1, kWaveSize);
+    if (size <= 2 * kWaveSize) H2X_LANES(2, kWaveSize);
+    if (size <= 4 * kWaveSize) H2X_LANES(4, kWaveSize);
+    if (!SPREAD || n > kManySamples)
+    {
+        if (size <= 8 * kWaveSize) H2X_LANES(8, kWaveSize);
+        if (size <= 16 * kWaveSize) H2X_LANES(16, kWaveSize);
+        if (size <= 32 * kWaveSize) H2X_LANES(32, kWaveSize);
+    }
+    if (size <= 4 * kBlockSize) H2X_LANES(4, kBlockSize);
+    if (size <= 8 * kBlockSize) H2X_LANES(8, kBlockSize);
+    if (size <= 16 * kBlockSize) H2X_LANES(16, kBlockSize);
+    if constexpr (MAX_LARGE == 0)
+    {
+        H2X_LANES(32, kBlockSize);
+    }
+    else
+    {
+        if (size <= 8 * 1024) H2X_LANES(8, 1024);
+        if (MAX_LARGE > 16 && size <= 16 * 1024) H2X_LANES(16, 1024);
+        H2X_LANES(MAX_LARGE, 1024);
+    }
+#undef H2X_LANES
+}
+
+template <int LANES>
+unsigned int lanes_grid(int n)
+{
+    constexpr unsigned int samples = lanes_block<LANES>() / LANES;
+    return (static_cast<unsigned int>(n) + samples - 1) / samples;
+}
+
 template <typename T>
 int forward_impl(int n, int c, size_t s, const void* xv, void* yv, hipStream_t st)
 {
     const T* x = static_cast<const T*>(xv);
     T* y = static_cast<T*>(yv);
     constexpr int kWords = sizeof(T) / 4;
+    if (s == 1 && c <= 32 * kBlockSize)
+        return with_lanes<false>(n, c, [&](auto cpl, auto lanes) {
+            constexpr int CPL = decltype(cpl)::value, LANES = decltype(lanes)::value;
+            softmax_fwd_row_kernel<T, CPL, LANES><<<lanes_grid<LANES>(n), lanes_block<LANES>(), 0, st>>>(x, y, c, n);
+            return launch_status();
+        });
     if (s == 1)
     {
-        const unsigned int blocks = (static_cast<unsigned int>(n) + kWavesPerBlock - 1) / kWavesPerBlock;
-#define H2X_FWD_ROW(CP)                                                                            \
-    do                                                                                             \
-    {                                                                                              \
-        softmax_fwd_row_kernel<T, CP><<<blocks, kBlockSize, 0, st>>>(x, y, c, n);                   \
-        return launch_status();                                                                    \
-    } while (0)
-        if (c <= 1 * kWaveSize) H2X_FWD_ROW(1);
-        if (c <= 2 * kWaveSize) H2X_FWD_ROW(2);
-        if (c <= 4 * kWaveSize) H2X_FWD_ROW(4);
-        if (c <= 8 * kWaveSize) H2X_FWD_ROW(8);
-        if (c <= 16 * kWaveSize) H2X_FWD_ROW(16);
-        if (c <= 32 * kWaveSize) H2X_FWD_ROW(32);
-#undef H2X_FWD_ROW
         softmax_fwd_long_row_kernel<T><<<n, kBlockSize, 0, st>>>(x, y, c);
         return launch_status();
     }
@@ -955,22 +1032,14 @@ int backward_impl(int n, int c, size_t s, const void* yv, const void* dyv, void*
     const T* dy = static_cast<const T*>(dyv);
     T* dx = static_cast<T*>(dxv);
     constexpr int kWords = sizeof(T) / 4;
+    if (s == 1 && c <= 32 * kBlockSize)
+        return with_lanes<false>(n, c, [&](auto cpl, auto lanes) {
+            constexpr int CPL = decltype(cpl)::value, LANES = decltype(lanes)::value;
+            softmax_bwd_row_kernel<T, CPL, LANES><<<lanes_grid<LANES>(n), lanes_block<LANES>(), 0, st>>>(y, dy, dx, c, n);
+            return launch_status();
+        });
     if (s == 1)
     {
-        const unsigned int blocks = (static_cast<unsigned int>(n) + kWavesPerBlock - 1) / kWavesPerBlock;
-#define H2X_BWD_ROW(CP)                                                                            \
-    do                                                                                             \
-    {                                                                                              \
-        softmax_bwd_row_kernel<T, CP><<<blocks, kBlockSize, 0, st>>>(y, dy, dx, c, n);              \
-        return launch_status();                                                                    \
-    } while (0)
-        if (c <= 1 * kWaveSize) H2X_BWD_ROW(1);
-        if (c <= 2 * kWaveSize) H2X_BWD_ROW(2);
-        if (c <= 4 * kWaveSize) H2X_BWD_ROW(4);
-        if (c <= 8 * kWaveSize) H2X_BWD_ROW(8);
-        if (c <= 16 * kWaveSize) H2X_BWD_ROW(16);
-        if (c <= 32 * kWaveSize) H2X_BWD_ROW(32);
-#undef H2X_BWD_ROW
         softmax_bwd_long_row_kernel<T><<<n, kBlockSize, 0, st>>>(y, dy, dx, c);
         return launch_status();
     }
@@ -1035,18 +1104,6 @@ int inst_groups_per_sample_max(int num_samples)
 {
     const int g = (kInstTargetGroups + num_samples - 1) / (num_samples > 0 ? num_samples : 1);
     return g < 8 ? 8 : (g > kInstMaxGroupsPerSample ? kInstMaxGroupsPerSample : g);
-}
-
-template <typename T>
-__device__ __forceinline__ T wave_max(T v)
-{
-#pragma unroll
-    for (int d = 1; d < kWaveSize; d *= 2)
-    {
-        const T o = __shfl_xor(v, d, kWaveSize);
-        v = o > v ? o : v;
-    }
-    return v;
 }
 
 enum InstReduce : int
@@ -1222,44 +1279,41 @@ __global__ __launch_bounds__(kBlockSize) void softmax_inst_map_kernel(
     P::store(out + off, v);
 }
 
-// Samples of at most 8192 elements (the softmax behind a classifier: 10 to
-// a few thousand classes): a wave -- beyond 2048 elements a workgroup -- takes a
-// sample, holds it in registers (CPL elements a lane) and combines its lanes with
-// shuffles (and its waves through LDS), so a reduction is one launch without
-// partials, and the whole forward pass of samples that are whole on this rank is
-// one launch too (N 4096, 10 elements a sample: 18 us in five launches before).
-// Sums are accumulated in fp64, lane by lane and then across the lanes as a
-// butterfly; the staged and the fused path add in the same order.
+// Samples that the lanes of a wave or a workgroup hold in registers (the softmax behind a
+// classifier: 10 to a few thousand classes; up to 32 K elements): a reduction is one launch
+// without partials, and a whole pass of samples that are whole on this rank is one
+// launch too.  Sums are accumulated in fp64, lane by lane and then across the lanes;
+// the staged and the fused path add in the same order.
 enum InstSmall : int
 {
     kSmallMax = 0,     // result[n] = max x
     kSmallExpSum = 1,  // out = exp(x - param[n]); result[n] = sum
     kSmallSumExp = 2,  // result[n] = sum exp(x - param[n])
     kSmallDot = 3,     // result[n] = sum a * b
-    kSmallForward = 4  // result[n] = max, result2[n] = sum, out = max(exp(x - max) / sum, min_output)
+    kSmallForward = 4, // result[n] = max, result2[n] = sum, out = max(exp(x - max) / sum, min_output)
+    kSmallBackward = 5 // result[n] = sum a * b, out = a > min_output ? a * (b - result[n]) : 0
 };
 
 template <typename T, int CPL, int MODE, int LANES>
-__global__ __launch_bounds__(kBlockSize) void softmax_inst_small_kernel(
+__global__ __launch_bounds__(lanes_block<LANES>()) void softmax_inst_small_kernel(
     const T* __restrict__ a, const T* __restrict__ b, T* __restrict__ out,
     const T* __restrict__ sample_param, T* __restrict__ result, T* __restrict__ result2,
     int sample_size, int num_samples, T min_output)
 {
-    // LANES lanes serve a sample: a wave, or the whole workgroup (whose waves are then
-    // combined through LDS in wave order; every thread of the workgroup has the same n)
-    __shared__ double lds[kWavesPerBlock];
+    constexpr bool kDot = MODE == kSmallDot || MODE == kSmallBackward;
+    __shared__ double lds[lanes_block<LANES>() / kWaveSize];
     const int lane = threadIdx.x % LANES;
-    const int n = (blockIdx.x * kBlockSize + threadIdx.x) / LANES;
-    if (n >= num_samples)
+    const int n = blockIdx.x * (lanes_block<LANES>() / LANES) + threadIdx.x / LANES;
+    if (n >= num_samples) // all lanes of a sample
         return;
     const size_t base = static_cast<size_t>(n) * sample_size;
-    T va[CPL], vb[CPL];
+    T va[CPL], vb[kDot ? CPL : 1];
 #pragma unroll
     for (int k = 0; k < CPL; ++k)
         if (lane + k * LANES < sample_size)
         {
             va[k] = a[base + lane + k * LANES];
-            if constexpr (MODE == kSmallDot)
+            if constexpr (kDot)
                 vb[k] = b[base + lane + k * LANES];
         }
     T shift = T(0);
@@ -1273,14 +1327,14 @@ __global__ __launch_bounds__(kBlockSize) void softmax_inst_small_kernel(
         if constexpr (LANES == kWaveSize)
             mx = wave_max(mx);
         else
-            mx = static_cast<T>(block_combine(static_cast<double>(mx), true, lds));
+            mx = static_cast<T>(block_combine<LANES / kWaveSize>(static_cast<double>(mx), true, lds));
         if (lane == 0)
             result[n] = mx;
         if constexpr (MODE == kSmallMax)
             return;
         shift = mx;
     }
-    else if constexpr (MODE != kSmallDot)
+    else if constexpr (!kDot)
     {
         shift = sample_param[n];
     }
@@ -1289,7 +1343,7 @@ __global__ __launch_bounds__(kBlockSize) void softmax_inst_small_kernel(
     for (int k = 0; k < CPL; ++k)
         if (lane + k * LANES < sample_size)
         {
-            if constexpr (MODE == kSmallDot)
+            if constexpr (kDot)
             {
                 acc = __builtin_fma(static_cast<double>(va[k]), static_cast<double>(vb[k]), acc);
             }
@@ -1299,14 +1353,10 @@ __global__ __launch_bounds__(kBlockSize) void softmax_inst_small_kernel(
                 acc += static_cast<double>(va[k]);
             }
         }
-    if constexpr (LANES == kWaveSize)
-        acc = wave_butterfly_sum(acc);
-    else
-        acc = block_combine(acc, false, lds);
-    const T total = static_cast<T>(acc);
+    const T total = static_cast<T>(lanes_sum<LANES>(acc, lds));
     if (lane == 0)
         (MODE == kSmallForward ? result2 : result)[n] = total;
-    if constexpr (MODE == kSmallExpSum || MODE == kSmallForward)
+    if constexpr (MODE == kSmallExpSum || MODE == kSmallForward || MODE == kSmallBackward)
     {
 #pragma unroll
         for (int k = 0; k < CPL; ++k)
@@ -1317,37 +1367,33 @@ __global__ __launch_bounds__(kBlockSize) void softmax_inst_small_kernel(
                     const T r = va[k] / total;
                     va[k] = r > min_output ? r : min_output;
                 }
+                else if constexpr (MODE == kSmallBackward)
+                {
+                    va[k] = va[k] > min_output ? va[k] * (vb[k] - total) : T(0);
+                }
                 out[base + lane + k * LANES] = va[k];
             }
     }
 }
 
-constexpr size_t kInstSmallSample = 32 * kBlockSize;
+// Elements a lane of 1024 holds.  Twice as many leave one CU too much to do
+// (30 samples of 57600: forward 22.0 us, in five launches 16.7).
+template <typename T>
+constexpr int kInstLargeLanes = 128 / sizeof(T);
+template <typename T>
+constexpr size_t kInstSmallSample = kInstLargeLanes<T> * size_t(1024);
 
 template <typename T, int MODE>
 int inst_small(int n, size_t sample_size, const void* a, const void* b, void* out,
                const void* param, void* result, void* result2, T min_output, hipStream_t st)
 {
-#define H2X_INST_SMALL(CP, LN)                                                                     \
-    do                                                                                             \
-    {                                                                                              \
-        const unsigned int teams = kBlockSize / LN;                                                \
-        softmax_inst_small_kernel<T, CP, MODE, LN>                                                 \
-            <<<(static_cast<unsigned int>(n) + teams - 1) / teams, kBlockSize, 0, st>>>(           \
-                static_cast<const T*>(a), static_cast<const T*>(b), static_cast<T*>(out),          \
-                static_cast<const T*>(param), static_cast<T*>(result), static_cast<T*>(result2),   \
-                static_cast<int>(sample_size), n, min_output);                                     \
-        return launch_status();                                                                    \
-    } while (0)
-    if (sample_size <= 1 * kWaveSize) H2X_INST_SMALL(1, kWaveSize);
-    if (sample_size <= 2 * kWaveSize) H2X_INST_SMALL(2, kWaveSize);
-    if (sample_size <= 4 * kWaveSize) H2X_INST_SMALL(4, kWaveSize);
-    if (sample_size <= 8 * kWaveSize) H2X_INST_SMALL(8, kWaveSize);
-    if (sample_size <= 16 * kWaveSize) H2X_INST_SMALL(16, kWaveSize);
-    if (sample_size <= 32 * kWaveSize) H2X_INST_SMALL(32, kWaveSize);
-    if (sample_size <= 16 * kBlockSize) H2X_INST_SMALL(16, kBlockSize);
-    H2X_INST_SMALL(32, kBlockSize);
-#undef H2X_INST_SMALL
+    return with_lanes<sizeof(T) == 4, kInstLargeLanes<T>>(n, sample_size, [&](auto cpl, auto lanes) {
+        constexpr int CPL = decltype(cpl)::value, LANES = decltype(lanes)::value;
+        softmax_inst_small_kernel<T, CPL, MODE, LANES><<<lanes_grid<LANES>(n), lanes_block<LANES>(), 0, st>>>(
+            static_cast<const T*>(a), static_cast<const T*>(b), static_cast<T*>(out), static_cast<const T*>(param),
+            static_cast<T*>(result), static_cast<T*>(result2), static_cast<int>(sample_size), n, min_output);
+        return launch_status();
+    });
 }
 
 template <typename T>
@@ -1378,7 +1424,7 @@ template <typename T, int MODE>
 int inst_reduce(int n, size_t sample_size, const void* a, const void* b, void* out,
                 const void* param, void* result, void* workspace, hipStream_t st)
 {
-    if (sample_size <= kInstSmallSample && n > 0)
+    if (sample_size <= kInstSmallSample<T> && n > 0)
     {
         constexpr int kSmallMode = MODE == kInstMax      ? kSmallMax
                                    : MODE == kInstExpSum ? kSmallExpSum
@@ -1429,7 +1475,7 @@ template <typename T>
 int inst_forward_local(int n, size_t sample_size, const void* x, void* y, void* sample_max,
                        void* sample_exp, void* workspace, hipStream_t st)
 {
-    if (sample_size <= kInstSmallSample && n > 0)
+    if (sample_size <= kInstSmallSample<T> && n > 0)
         return inst_small<T, kSmallForward>(n, sample_size, x, nullptr, y, nullptr, sample_max,
                                             sample_exp, inst_min_output<T>(), st);
     int err = inst_reduce<T, kInstMax>(n, sample_size, x, nullptr, nullptr, nullptr, sample_max,
@@ -1440,6 +1486,17 @@ int inst_forward_local(int n, size_t sample_size, const void* x, void* y, void* 
         err = inst_reduce<T, kInstSumExp>(n, sample_size, x, nullptr, y, sample_max, sample_exp,
                                           workspace, st);
     return err ? err : inst_map<T, kMapFromInput>(n, sample_size, x, nullptr, sample_exp, sample_max, y, st);
+}
+
+template <typename T>
+int inst_backward_local(int n, size_t sample_size, const void* y, const void* dy, void* dx, void* sample_dp,
+                        void* workspace, hipStream_t st)
+{
+    if (sample_size <= kInstSmallSample<T> && n > 0)
+        return inst_small<T, kSmallBackward>(n, sample_size, y, dy, dx, nullptr, sample_dp, nullptr,
+                                             inst_min_output<T>(), st);
+    const int err = inst_reduce<T, kInstDot>(n, sample_size, y, dy, nullptr, nullptr, sample_dp, workspace, st);
+    return err ? err : inst_map<T, kMapGradient>(n, sample_size, y, dy, sample_dp, nullptr, dx, st);
 }
 
 bool inst_bad(int num_samples, size_t sample_size)
@@ -1588,4 +1645,16 @@ extern "C" int h2x_softmax_instance_forward_local(h2x_dtype dtype, int num_sampl
                                               workspace, as_stream(stream))),
                    (inst_forward_local<double>(num_samples, sample_size, x, y, sample_max, sample_exp,
                                                workspace, as_stream(stream))));
+}
+
+extern "C" int h2x_softmax_instance_backward_local(h2x_dtype dtype, int num_samples, size_t sample_size,
+                                                   const void* y, const void* dy, void* dx, void* sample_dp,
+                                                   void* workspace, h2x_stream_t stream)
+{
+    if (!y || !dy || !dx || !sample_dp || !workspace)
+        return num_samples == 0 || sample_size == 0 ? H2X_SUCCESS : H2X_ERR_INVALID_ARGUMENT;
+    H2X_INST_ENTRY((inst_backward_local<float>(num_samples, sample_size, y, dy, dx, sample_dp, workspace,
+                                               as_stream(stream))),
+                   (inst_backward_local<double>(num_samples, sample_size, y, dy, dx, sample_dp, workspace,
+                                                as_stream(stream))));
 }

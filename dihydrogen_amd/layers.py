@@ -440,12 +440,16 @@ class Softmax:
             return 0
         # instance mode: softmax.cu:770-783
         calls, size, ws = self._calls, l.channels * l.spatial, self._workspace(n)
-        sdp = (self._sample_scalars(y, n) if self.allreduce is None
-               else torch.empty(n, dtype=y.dtype, device=y.device))
+        if self.allreduce is None:
+            status = calls.h2x_softmax_instance_backward_local(
+                dt, n, size, y.get_base_ptr(), dy.get_base_ptr(), dx.get_base_ptr(), self._sample_scalars(y, n), ws, st)
+            if status:
+                capi.check(status, "softmax instance backward")
+            return 0
+        sdp = torch.empty(n, dtype=y.dtype, device=y.device)
         capi.check(calls.h2x_softmax_instance_dot(dt, n, size, y.get_base_ptr(), dy.get_base_ptr(), sdp, ws, st),
                    "softmax instance dot")
-        if self.allreduce:
-            self.allreduce(sdp, False)
+        self.allreduce(sdp, False)
         capi.check(calls.h2x_softmax_instance_gradient(dt, n, size, y.get_base_ptr(), dy.get_base_ptr(), sdp,
                                                        dx.get_base_ptr(), st), "softmax instance gradient")
         return 0

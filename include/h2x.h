@@ -854,6 +854,14 @@ int h2x_softmax_instance_dot(h2x_dtype dtype, int num_samples, size_t sample_siz
 int h2x_softmax_instance_gradient(h2x_dtype dtype, int num_samples, size_t sample_size,
                                   const void* y, const void* dy, const void* sample_dp, void* dx,
                                   h2x_stream_t stream);
+/**
+ * What h2x_softmax_instance_dot and _gradient leave in sample_dp and dx, bit for
+ * bit, for samples that are whole on this rank; one launch where a workgroup holds
+ * a sample.
+ */
+int h2x_softmax_instance_backward_local(h2x_dtype dtype, int num_samples, size_t sample_size,
+                                        const void* y, const void* dy, void* dx, void* sample_dp,
+                                        void* workspace, h2x_stream_t stream);
 
 /* ------------------------------------------------------------------------ */
 /* Halo pack / unpack                                                        */
