@@ -305,17 +305,23 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+_calls = None
+
+
 def calls():
     """The native module whose functions call the library (csrc/h2x_python.cpp): the entry points
     the layers call once per step, under their own names, taking torch tensors, addresses or None
     for pointers and returning the status.  Raises if it is absent."""
-    load()
-    try:
-        from . import _h2xcall
-    except ImportError as e:
-        raise H2XError("_h2xcall.so is missing: build it with `make -C dihydrogen_amd/csrc` "
-                       "(or __graft_entry__.build()); there is no fallback path") from e
-    return _h2xcall
+    global _calls
+    if _calls is None:
+        load()
+        try:
+            from . import _h2xcall
+        except ImportError as e:
+            raise H2XError("_h2xcall.so is missing: build it with `make -C dihydrogen_amd/csrc` "
+                           "(or __graft_entry__.build()); there is no fallback path") from e
+        _calls = _h2xcall
+    return _calls
 
 
 def check(status: int, what: str = "") -> None:

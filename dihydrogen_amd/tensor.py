@@ -12,7 +12,6 @@ from __future__ import annotations
 
 import ctypes
 import math
-from functools import cached_property
 from typing import Iterable, List, Optional, Sequence
 
 import torch
@@ -120,48 +119,82 @@ def _block_start(extent: int, parts: int, index: int) -> int:
 _TORCH_DTYPES = {torch.float32: capi.F32, torch.float64: capi.F64}
 
 
+class _once:
+    """A property that is worked out at its first use and then an attribute of the instance
+    (functools.cached_property takes a lock to do so)."""
+
+    def __init__(self, compute):
+        self.compute, self.name = compute, compute.__name__
+        self.__doc__ = compute.__doc__
+
+    def __get__(self, instance, owner=None):
+        if instance is None:
+            return self
+        value = instance.__dict__[self.name] = self.compute(instance)
+        return value
+
+
 class Layout:
     """What a layer call needs to know about a local tensor besides its address.  Shape,
     distribution and type of a Tensor are fixed when it is made, so this is worked out once
-    (a layer call that launches a kernel of a few microseconds cannot afford it every time)."""
-
-    __slots__ = ("samples", "channels", "spatial", "spatial_real", "dense", "haloed", "channel_halo",
-                 "dtype", "active", "geometry", "geometry_address", "per_channel_local", "per_channel_global",
-                 "alike", "_haloed_geometry")
+    (a layer call that launches a kernel of a few microseconds cannot afford it every time), and
+    what only some calls need when one of them does: a tensor may be new at every call."""
 
     def __init__(self, t: "Tensor"):
-        nd = t.get_num_dims()
-        self.samples, self.channels = t.local_shape[nd - 1], t.local_shape[nd - 2]
-        self.spatial, self.spatial_real = _prod(t.local_shape[: nd - 2]), _prod(t.local_real_shape[: nd - 2])
+        local, real, overlap, shape, dist = t.local_shape, t.local_real_shape, t.overlap, t.shape, t.dist
+        self._local, self._real, self._overlap = local, real, overlap
+        ns = len(local) - 2
+        spatial = spatial_real = 1
+        for d in range(ns):
+            spatial *= local[d]
+            spatial_real *= real[d]
+        self.spatial, self.spatial_real = spatial, spatial_real
+        samples, channels = self.samples, self.channels = local[ns + 1], local[ns]
         # no halo on the inner spatial dimensions: the layout the dense entry points take
         # (legacy/src/dnn_backend/batchnorm.cu:210-219)
-        self.dense = all(t.overlap[d] == 0 for d in range(nd - 3))
-        self.haloed = any(t.overlap)
-        self.channel_halo = t.overlap[nd - 2] != 0 or t.overlap[nd - 1] != 0
-        self.dtype = t.h2x_dtype
+        self.dense = not any(overlap[:max(ns - 1, 0)])
+        self.haloed = any(overlap)
+        self.channel_halo = overlap[ns] != 0 or overlap[ns + 1] != 0
+        self.dtype = _TORCH_DTYPES[t.dtype]
         # a rank that owns elements
-        self.active = t.is_split_root() and t.get_local_size() > 0
-        g = self.geometry = capi.TensorGeometry()
-        g.num_dims = nd
-        for i, (extent, stride) in enumerate(zip(t.local_shape, t.get_strides())):
-            g.local_shape[i], g.strides[i] = extent, stride
-        self.geometry_address = ctypes.addressof(g)
+        self.active = spatial * samples * channels > 0 and (dist.locale_shape == dist.split_shape or t.is_split_root())
         # elements per channel of the local and of the global shape
-        self.per_channel_local, self.per_channel_global = (
-            _prod(s) // s[nd - 2] if s[nd - 2] else 0 for s in (t.local_shape, t.shape))
-        # tensors with equal keys lie in memory alike
-        self.alike = (tuple(t.local_shape), tuple(t.local_real_shape), tuple(t.overlap), self.dtype)
-        self._haloed_geometry = None
+        self.per_channel_local = spatial * samples if channels else 0
+        self.per_channel_global = math.prod(shape) // shape[ns] if shape[ns] else 0
 
-    @property
-    def haloed_geometry_address(self) -> int:
+    @_once
+    def alike(self):
+        """Tensors with equal keys lie in memory alike."""
+        return tuple(self._local), tuple(self._real), tuple(self._overlap), self.dtype
+
+    @_once
+    def geometry(self):
+        """h2x_tensor_geometry: local extents and the strides of the real allocation."""
+        g = capi.TensorGeometry()
+        nd = g.num_dims = len(self._local)
+        strides, stride = [], 1
+        for extent in self._real:
+            strides.append(stride)
+            stride *= extent
+        g.local_shape[:nd] = self._local
+        g.strides[:nd] = strides
+        return g
+
+    @_once
+    def geometry_address(self) -> int:
+        return ctypes.addressof(self.geometry)
+
+    @_once
+    def haloed_geometry(self):
         """h2x_haloed_geometry: local and real extents, halo widths."""
-        if self._haloed_geometry is None:
-            g = self._haloed_geometry = capi.HaloedGeometry()
-            g.num_dims = self.geometry.num_dims
-            for i, (local, real, halo) in enumerate(zip(*self.alike[:3])):
-                g.local_shape[i], g.real_shape[i], g.lower_halo[i] = local, real, halo
-        return ctypes.addressof(self._haloed_geometry)
+        g = capi.HaloedGeometry()
+        nd = g.num_dims = len(self._local)
+        g.local_shape[:nd], g.real_shape[:nd], g.lower_halo[:nd] = self._local, self._real, self._overlap
+        return g
+
+    @_once
+    def haloed_geometry_address(self) -> int:
+        return ctypes.addressof(self.haloed_geometry)
 
 
 class Tensor:
@@ -173,19 +206,16 @@ class Tensor:
         self.shape = [int(v) for v in shape]
         if len(self.shape) != dist.num_dims:
             raise ValueError("shape and distribution disagree on the number of dimensions")
-        if dist.num_ranks != locale.size:
+        if math.prod(dist.locale_shape) != locale.size:
             raise ValueError("distribution does not cover the locale")
         self.locale, self.dist, self.dtype, self.device = locale, dist, dtype, device
         self.proc_index = dist.rank_index(locale.rank)
-        self.split_index = [p // dist.get_num_ranks_per_split(d) for d, p in enumerate(self.proc_index)]
+        self.split_index = [p // (l // s) for p, l, s in zip(self.proc_index, dist.locale_shape, dist.split_shape)]
         self.global_index, self.local_shape = [], []
-        for d, extent in enumerate(self.shape):
-            parts = dist.split_shape[d]
+        for extent, parts, index in zip(self.shape, dist.split_shape, self.split_index):
+            lo, hi = 0, extent
             if parts > 1:
-                lo = _block_start(extent, parts, self.split_index[d])
-                hi = _block_start(extent, parts, self.split_index[d] + 1)
-            else:
-                lo, hi = 0, extent
+                lo, hi = _block_start(extent, parts, index), _block_start(extent, parts, index + 1)
             self.global_index.append(lo)
             self.local_shape.append(hi - lo)
         self.overlap = list(dist.overlap)
@@ -226,11 +256,11 @@ class Tensor:
         si = rank_index // self.dist.get_num_ranks_per_split(dim)
         return _block_start(self.shape[dim], parts, si + 1) - _block_start(self.shape[dim], parts, si)
 
-    @cached_property
+    @_once
     def layout(self) -> Layout:
         return Layout(self)
 
-    @cached_property
+    @_once
     def base_bytes(self) -> int:
         return self.base_offset() * self.dtype.itemsize
 
