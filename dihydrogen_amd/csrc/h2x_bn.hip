@@ -2205,13 +2205,8 @@ int backprop2_impl(int num_samples, int num_channels, size_t spatial, size_t num
     return issued();
 }
 
-// Normalise / input gradient over tensors of one haloed geometry, the halo of
-// the output cleared (bn_clearing_kernel).
-template <typename T>
-int clearing_impl(bool backward, size_t num_per_sum, const h2x_haloed_geometry* g, const void* x,
-                  const void* dy, const void* mean, const void* var, const void* scale,
-                  const void* bias, const void* dmean, const void* dvar, void* out, double epsilon,
-                  hipStream_t stream)
+// The allocation of a (sample, channel) segment: its interior, and its elements.
+int real_box(const h2x_haloed_geometry* g, RealBox* out, size_t* elements)
 {
     if (!g || g->num_dims < 3 || g->num_dims > 5)
         return H2X_ERR_INVALID_ARGUMENT;
@@ -2240,14 +2235,33 @@ int clearing_impl(bool backward, size_t num_per_sum, const h2x_haloed_geometry* 
         box.lo[d] = static_cast<uint32_t>(g->lower_halo[d]);
         box.hi[d] = static_cast<uint32_t>(g->lower_halo[d] + g->local_shape[d]);
     }
+    box.wr = make_fastdiv(static_cast<uint32_t>(extent[0]));
+    box.hr = make_fastdiv(static_cast<uint32_t>(extent[1]));
+    *out = box;
+    *elements = real;
+    return H2X_SUCCESS;
+}
+
+// Normalise / input gradient over tensors of one haloed geometry, the halo of
+// the output cleared (bn_clearing_kernel).
+template <typename T>
+int clearing_impl(bool backward, size_t num_per_sum, const h2x_haloed_geometry* g, const void* x,
+                  const void* dy, const void* mean, const void* var, const void* scale,
+                  const void* bias, const void* dmean, const void* dvar, void* out, double epsilon,
+                  hipStream_t stream)
+{
+    RealBox box;
+    size_t real;
+    const int err = real_box(g, &box, &real);
+    if (err)
+        return err;
+    const int nd = g->num_dims;
     const int num_channels = static_cast<int>(g->local_shape[nd - 2]);
     const size_t segments = static_cast<size_t>(g->local_shape[nd - 1]) * num_channels;
     if (segments == 0 || real == 0)
         return H2X_SUCCESS;
     if (!x || !out || (backward && !dy))
         return H2X_ERR_INVALID_ARGUMENT;
-    box.wr = make_fastdiv(static_cast<uint32_t>(extent[0]));
-    box.hr = make_fastdiv(static_cast<uint32_t>(extent[1]));
     const bool vectors = real % full_vec<T>() == 0 && aligned16(x) && aligned16(out)
                          && (!backward || aligned16(dy));
     const int vw = vectors ? full_vec<T>() : 1;
@@ -2593,8 +2607,8 @@ bool once_geometry(int num_samples, int num_channels, size_t spatial, std::initi
     return true;
 }
 
-template <int TEAM>
-unsigned int once_grid(const OnceGeometry& g)
+template <int TEAM, typename G>
+unsigned int once_grid(const G& g)
 {
     constexpr unsigned int teams = once_block<TEAM>() / TEAM;
     return ((g.num_channels + teams - 1) / teams + kNumXcd - 1) / kNumXcd * kNumXcd;
@@ -2615,13 +2629,13 @@ constexpr size_t kHaloedNormalStores = size_t(48) << 20;
 // in one launch 12.3; C 64, 28^3 x 2 9.6 and 9.1).
 constexpr unsigned int kOnceManyChannels = 96;
 
-template <int TEAM, int K, bool STREAM>
-void issue_once(const OnceGeometry& g, const OnceForward<float>& a, hipStream_t st)
+template <int TEAM, int K, bool STREAM, typename G>
+void issue_once(const G& g, const OnceForward<float>& a, hipStream_t st)
 {
     bn_once_forward_kernel<float, TEAM, K, STREAM><<<once_grid<TEAM>(g), once_block<TEAM>(), 0, st>>>(g, a);
 }
-template <int TEAM, int K, bool STREAM>
-void issue_once(const OnceGeometry& g, const OnceBackward<float>& a, hipStream_t st)
+template <int TEAM, int K, bool STREAM, typename G>
+void issue_once(const G& g, const OnceBackward<float>& a, hipStream_t st)
 {
     constexpr int kInLds = TEAM * K > 8192 ? 9 : 0; // 144 of the 160 KB
     bn_once_backward_kernel<float, TEAM, K, STREAM, kInLds><<<once_grid<TEAM>(g), once_block<TEAM>(), 0, st>>>(g, a);
@@ -2630,8 +2644,8 @@ void issue_once(const OnceGeometry& g, const OnceBackward<float>& a, hipStream_t
 // The smallest team whose K vectors a thread hold the channel: four where that is enough
 // workgroups (more threads wait for memory together), more only beyond 1024 threads.
 // False: no variant holds it.
-template <bool STREAM, typename A>
-bool once_launch(const OnceGeometry& g, const A& a, hipStream_t st)
+template <bool STREAM, typename G, typename A>
+bool once_launch(const G& g, const A& a, hipStream_t st)
 {
     constexpr bool kForward = std::is_same<A, OnceForward<float>>::value;
     if (g.vectors <= 64 * 2)
@@ -2685,21 +2699,21 @@ bool apart(const void* a, const void* b, size_t bytes)
     return x + bytes <= y || y + bytes <= x;
 }
 
-template <typename T, int TEAM, int K, bool STREAM>
-void issue_team(const TeamGeometry& g, const OnceForward<T>& a, unsigned long long* slots, hipStream_t st)
+template <typename T, int TEAM, int K, bool STREAM, typename G>
+void issue_team(const TeamGeometry<G>& g, const OnceForward<T>& a, unsigned long long* slots, hipStream_t st)
 {
     bn_team_forward_kernel<T, TEAM, K, STREAM><<<g.once.num_channels * g.members.divisor, TEAM, 0, st>>>(g, a, slots);
 }
-template <typename T, int TEAM, int K, bool STREAM>
-void issue_team(const TeamGeometry& g, const OnceBackward<T>& a, unsigned long long* slots, hipStream_t st)
+template <typename T, int TEAM, int K, bool STREAM, typename G>
+void issue_team(const TeamGeometry<G>& g, const OnceBackward<T>& a, unsigned long long* slots, hipStream_t st)
 {
     bn_team_backward_kernel<T, TEAM, K, STREAM><<<g.once.num_channels * g.members.divisor, TEAM, 0, st>>>(g, a, slots);
 }
 
 // Members of TEAM threads with K vectors each; false if that is fewer than `least` or
 // more than `most` members, or more slots than the workspace has.
-template <int TEAM, int K, template <typename> class A, typename T>
-bool team_launch(const OnceGeometry& once, const A<T>& a, bool stream, uint32_t least, uint32_t most,
+template <int TEAM, int K, typename G, template <typename> class A, typename T>
+bool team_launch(const G& once, const A<T>& a, bool stream, uint32_t least, uint32_t most,
                  uint32_t max_polls, void* ws, hipStream_t st)
 {
     constexpr int kSums = std::is_same<A<T>, OnceForward<T>>::value ? 2 : 4;
@@ -2709,7 +2723,7 @@ bool team_launch(const OnceGeometry& once, const A<T>& a, bool stream, uint32_t 
     if (members > most || blocks < least || count >= (1u << 30)
         || count * sizeof(double) > partials_bytes(static_cast<int>(once.num_channels)))
         return false;
-    TeamGeometry g;
+    TeamGeometry<G> g;
     g.once = once;
     g.members = make_fastdiv(members);
     g.span = ((once.vectors + members - 1) / members + TEAM - 1) / TEAM * TEAM;
@@ -2717,10 +2731,10 @@ bool team_launch(const OnceGeometry& once, const A<T>& a, bool stream, uint32_t 
     unsigned long long* const slots = static_cast<unsigned long long*>(ws);
     bn_team_clear_kernel<<<static_cast<unsigned int>((count + kBlockSize - 1) / kBlockSize), kBlockSize, 0, st>>>(
         slots, static_cast<uint32_t>(count));
-    if (stream)
+    if (stream || G::kClears)
         issue_team<T, TEAM, K, true>(g, a, slots, st);
     else
-        issue_team<T, TEAM, K, false>(g, a, slots, st);
+        issue_team<T, TEAM, K, G::kClears>(g, a, slots, st);
     return true;
 }
 
@@ -2734,8 +2748,8 @@ constexpr uint32_t kTeamLeastBlocks = 192;
 // Forward a member holds 128 KB, in smaller pieces where that is not enough workgroups
 // (N 2, C 32, 48^3: 12.0 us, whole ones 13.0); up to 128 members (N 16, C 16, 64^3 in 128
 // of them 98 us, in two launches 118).
-template <typename T>
-bool team_variant(const OnceGeometry& g, const OnceForward<T>& a, bool stream, uint32_t least, uint32_t most,
+template <typename G, typename T>
+bool team_variant(const G& g, const OnceForward<T>& a, bool stream, uint32_t least, uint32_t most,
                   uint32_t polls, void* ws, hipStream_t st)
 {
     return team_launch<512, 16>(g, a, stream, 2 * least, most, polls, ws, st)
@@ -2746,8 +2760,8 @@ bool team_variant(const OnceGeometry& g, const OnceForward<T>& a, bool stream, u
 // (N 8, C 64, 64^3: 355 us, in 128 members 379, in two launches 407), and no more than 64
 // of those (N 16, C 16, 64^3: 251 us, in two launches 195): a larger team waits longer for
 // its last member than it saves.
-template <typename T>
-bool team_variant(const OnceGeometry& g, const OnceBackward<T>& a, bool stream, uint32_t least, uint32_t most,
+template <typename G, typename T>
+bool team_variant(const G& g, const OnceBackward<T>& a, bool stream, uint32_t least, uint32_t most,
                   uint32_t polls, void* ws, hipStream_t st)
 {
     most /= 2;
@@ -2755,12 +2769,11 @@ bool team_variant(const OnceGeometry& g, const OnceBackward<T>& a, bool stream, 
            || team_launch<1024, 8>(g, a, stream, least, most, polls, ws, st);
 }
 
-// False: the call is not for teams.
-template <typename T, template <typename> class A>
-bool launch_by_teams(const OnceGeometry& g, const A<T>& a, int n, std::initializer_list<const void*> inputs,
+// False: the call is not for teams.  bytes: from the first to behind the last element of a tensor.
+template <typename G, typename A>
+bool launch_by_teams(const G& g, const A& a, size_t bytes, bool stream, std::initializer_list<const void*> inputs,
                      const void* output, uint32_t least, uint32_t polls, void* ws, hipStream_t st)
 {
-    const size_t bytes = reach_bytes(g, n);
     for (const void* p : inputs)
         if (!apart(p, output, bytes))
             return false;
@@ -2768,11 +2781,18 @@ bool launch_by_teams(const OnceGeometry& g, const A<T>& a, int n, std::initializ
     if (hipGetDevice(&device) != hipSuccess
         || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
         return false;
+    return team_variant(g, a, stream, least, std::min<uint32_t>(cus / 2, kMaxMembers), polls, ws, st);
+}
+
+template <typename A>
+bool launch_by_teams(const OnceGeometry& g, const A& a, int n, std::initializer_list<const void*> inputs,
+                     const void* output, uint32_t least, uint32_t polls, void* ws, hipStream_t st)
+{
     // short segments have kernels of their own (N 2048, C 256, 7 x 7: 141 us, by teams 172)
     const bool stream = streamed(g, n);
     if (dense_rows(g) && !stream)
         return false;
-    return team_variant(g, a, stream, least, std::min<uint32_t>(cus / 2, kMaxMembers), polls, ws, st);
+    return launch_by_teams(g, a, reach_bytes(g, n), stream, inputs, output, least, polls, ws, st);
 }
 
 // team_polls: by teams or not at all, however few workgroups that is, with this many looks.
@@ -2846,6 +2866,40 @@ int backward_once(int n, size_t num_per_sum, const h2x_tensor_geometry* gx, cons
         return H2X_ERR_UNSUPPORTED;
     return backward_local<T>(n, c, s, tx, td, to, num_per_sum, x, dy, mean, var, scale, dscale, dbias, dmean, dvar,
                              dx, eps, ws, st);
+}
+
+// The same for tensors of one haloed geometry whose outputs' halos are cleared, by one workgroup
+// or a team a channel; H2X_ERR_UNSUPPORTED: in the staged calls.
+template <typename A>
+int clearing_once(const h2x_haloed_geometry* h, const A& a, std::initializer_list<const void*> inputs, void* output,
+                  void* ws, hipStream_t st)
+{
+    ClearGeometry g;
+    size_t real;
+    const int err = real_box(h, &g.box, &real);
+    if (err)
+        return err;
+    constexpr size_t vec = full_vec<float>();
+    const int nd = h->num_dims;
+    const size_t n = h->local_shape[nd - 1], c = h->local_shape[nd - 2];
+    size_t interior = 1;
+    for (int d = 0; d < nd - 2; ++d)
+        interior *= h->local_shape[d];
+    bool fit = n > 0 && c > 0 && interior > 0 && real % vec == 0 && aligned16(output) && output;
+    for (const void* p : inputs)
+        fit = fit && p && aligned16(p);
+    if (!fit || n * c * real >= (1ull << 28) || c > 0x7fffffffull)
+        return H2X_ERR_UNSUPPORTED;
+    g.per_segment = make_fastdiv(static_cast<uint32_t>(real / vec));
+    g.vectors = static_cast<uint32_t>(n * (real / vec));
+    g.stride_n = static_cast<uint32_t>(c * real);
+    g.stride_c = static_cast<int64_t>(real);
+    g.num_channels = static_cast<uint32_t>(c);
+    if (once_launch<true>(g, a, st)
+        || launch_by_teams(g, a, n * c * real * sizeof(float), true, inputs, output, kTeamLeastBlocks, kTeamPolls, ws,
+                           st))
+        return launch_status();
+    return H2X_ERR_UNSUPPORTED;
 }
 
 } // namespace
@@ -3301,6 +3355,42 @@ extern "C" int h2x_bn_backward_team(h2x_dtype dtype, int num_samples, size_t num
                                        &max_polls));
 }
 
+extern "C" int h2x_bn_forward_clearing(h2x_dtype dtype, const h2x_haloed_geometry* geometry, const void* x_buffer,
+                                       const void* scale, const void* bias, size_t num_per_sum, double decay,
+                                       double epsilon, void* mean, void* var, void* running_mean, void* running_var,
+                                       void* y_buffer, void* workspace, h2x_stream_t stream)
+{
+    if (!geometry || !scale || !bias || !mean || !var || !running_mean || !running_var || !workspace)
+        return H2X_ERR_INVALID_ARGUMENT;
+    if (dtype != H2X_F32 || num_per_sum == 0)
+        return H2X_ERR_UNSUPPORTED;
+    typedef float T;
+    const OnceForward<T> a{static_cast<const T*>(x_buffer), static_cast<const T*>(scale), static_cast<const T*>(bias),
+                           static_cast<T*>(mean), static_cast<T*>(var), static_cast<T*>(running_mean),
+                           static_cast<T*>(running_var), static_cast<T*>(y_buffer), static_cast<T>(num_per_sum),
+                           static_cast<T>(decay), static_cast<T>(epsilon)};
+    return clearing_once(geometry, a, {x_buffer}, y_buffer, workspace, as_stream(stream));
+}
+
+extern "C" int h2x_bn_backward_clearing(h2x_dtype dtype, size_t num_per_sum, const h2x_haloed_geometry* geometry,
+                                        const void* x_buffer, const void* dy_buffer, const void* mean,
+                                        const void* var, const void* scale, void* dscale, void* dbias, void* dmean,
+                                        void* dvar, void* dx_buffer, double epsilon, void* workspace,
+                                        h2x_stream_t stream)
+{
+    if (!geometry || !mean || !var || !scale || !dscale || !dbias || !dmean || !dvar || !workspace)
+        return H2X_ERR_INVALID_ARGUMENT;
+    if (dtype != H2X_F32)
+        return H2X_ERR_UNSUPPORTED;
+    typedef float T;
+    const OnceBackward<T> a{static_cast<const T*>(x_buffer), static_cast<const T*>(dy_buffer),
+                            static_cast<const T*>(mean), static_cast<const T*>(var), static_cast<const T*>(scale),
+                            static_cast<T*>(dscale), static_cast<T*>(dbias), static_cast<T*>(dmean),
+                            static_cast<T*>(dvar), static_cast<T*>(dx_buffer), static_cast<T>(num_per_sum),
+                            static_cast<T>(num_per_sum - 1), static_cast<T>(epsilon)};
+    return clearing_once(geometry, a, {x_buffer, dy_buffer}, dx_buffer, workspace, as_stream(stream));
+}
+
 // Plays on the host which elements the workgroups that hold channels in registers touch.
 extern "C" int h2x_bn_audit_once(int num_samples, const h2x_tensor_geometry* geometry, unsigned int member_vectors,
                                  unsigned char* counted, unsigned char* stored, size_t elements)
@@ -3323,13 +3413,13 @@ extern "C" int h2x_bn_audit_once(int num_samples, const h2x_tensor_geometry* geo
             for (uint32_t i = first; i < std::min(first + span, g.vectors); ++i)
             {
                 const uint32_t at = once_place<VEC>(g, i);
-                const size_t e = static_cast<size_t>(ch * g.stride_c) + (at >> 2);
+                const size_t e = static_cast<size_t>(ch * g.stride_c) + OnceGeometry::offset(at);
                 if (e + VEC > elements)
                     return H2X_ERR_INVALID_ARGUMENT;
                 for (int j = 0; j < VEC; ++j)
                 {
                     stored[e + j] = 1;
-                    counted[e + j] += j >= static_cast<int>(at & 3);
+                    counted[e + j] += OnceGeometry::counts(at, j);
                 }
             }
     return H2X_SUCCESS;

@@ -28,8 +28,14 @@
 // serves the other half and merges the halves written.
 #pragma once
 
+// Tensors that lie alike: rows of interior elements.
 struct OnceGeometry
 {
+    static constexpr bool kClears = false;
+    // of a place: the element offset of a vector, and whether its element j counts
+    static __host__ __device__ __forceinline__ uint32_t offset(uint32_t at) { return at >> 2; }
+    static __host__ __device__ __forceinline__ bool counts(uint32_t at, int j) { return j >= static_cast<int>(at & 3); }
+
     uint32_t vectors;           // of one channel, all samples
     uint32_t width;             // elements of a row
     FastDiv spr;                // vectors a row is padded to
@@ -57,6 +63,40 @@ __host__ __device__ __forceinline__ uint32_t once_place(const OnceGeometry& g, u
         at += (r - q * g.h.divisor) * g.sy + (q - n * g.d.divisor) * g.sz;
     }
     return (at + n * g.stride_n) * 4 + (x - first);
+}
+
+// Tensors of one haloed geometry whose outputs' halos are cleared: the vectors of the
+// whole allocation; halo elements are read and not counted, and stored as zeros.  Their
+// stores leave no partial lines (forward + backward, N 8, C 64, 30^3 with a halo of 1, us
+// going round three sets of tensors: 87 in six launches, 72 here, 81 without clearing).
+struct ClearGeometry
+{
+    static constexpr bool kClears = true;
+    static __host__ __device__ __forceinline__ uint32_t offset(uint32_t at) { return at >> 4; }
+    static __host__ __device__ __forceinline__ bool counts(uint32_t at, int j) { return (at >> j) & 1; }
+
+    uint32_t vectors;     // of one channel, all samples
+    FastDiv per_segment;  // vectors of a segment
+    RealBox box;
+    uint32_t stride_n;    // the last element of a channel is less than 2^28 elements from its first
+    int64_t stride_c;
+    uint32_t num_channels;
+};
+
+// Element offset of vector i of a channel, times sixteen, plus a bit for each interior element.
+template <int VEC>
+__host__ __device__ __forceinline__ uint32_t once_place(const ClearGeometry& g, uint32_t i)
+{
+    static_assert(VEC <= 4, "four bits hold the interior elements");
+    const uint32_t n = fastdiv(i, g.per_segment);
+    const uint32_t e = (i - n * g.per_segment.divisor) * VEC;
+    bool inside[VEC];
+    interior_mask<VEC>(g.box, e, inside);
+    uint32_t mask = 0;
+#pragma unroll
+    for (int j = 0; j < VEC; ++j)
+        mask |= static_cast<uint32_t>(inside[j]) << j;
+    return (e + n * g.stride_n) * 16 + mask;
 }
 
 // STREAM: past the caches.  Rows of a few hundred bytes are stored normally: their
@@ -126,8 +166,8 @@ struct OnceForward
     T n, decay, epsilon;
 };
 
-template <typename T, int TEAM, int K, bool STREAM>
-__global__ __launch_bounds__(once_block<TEAM>()) void bn_once_forward_kernel(const OnceGeometry g,
+template <typename T, int TEAM, int K, bool STREAM, typename G>
+__global__ __launch_bounds__(once_block<TEAM>()) void bn_once_forward_kernel(const G g,
                                                                             const OnceForward<T> a)
 {
     static_assert(TEAM == kWaveSize || TEAM >= kBlockSize, "a wave or a workgroup");
@@ -145,7 +185,7 @@ __global__ __launch_bounds__(once_block<TEAM>()) void bn_once_forward_kernel(con
         if (u * TEAM < g.vectors && u * TEAM + t < g.vectors)
         {
             at[u] = once_place<VEC>(g, u * TEAM + t);
-            load_vec<T, VEC, false>(x + (at[u] >> 2), v[u]);
+            load_vec<T, VEC, false>(x + G::offset(at[u]), v[u]);
         }
     double s[2] = {0.0, 0.0};
 #pragma unroll
@@ -154,7 +194,7 @@ __global__ __launch_bounds__(once_block<TEAM>()) void bn_once_forward_kernel(con
         {
 #pragma unroll
             for (int j = 0; j < VEC; ++j)
-                if (j >= static_cast<int>(at[u] & 3))
+                if (G::counts(at[u], j))
                 {
                     const double d = static_cast<double>(v[u][j]);
                     s[0] += d;
@@ -180,8 +220,8 @@ __global__ __launch_bounds__(once_block<TEAM>()) void bn_once_forward_kernel(con
         {
 #pragma unroll
             for (int j = 0; j < VEC; ++j)
-                v[u][j] = fma_t((v[u][j] - m) * inv_stdev, sc, bi);
-            store_once<T, VEC, STREAM>(y + (at[u] >> 2), v[u]);
+                v[u][j] = G::kClears && !G::counts(at[u], j) ? T(0) : fma_t((v[u][j] - m) * inv_stdev, sc, bi);
+            store_once<T, VEC, STREAM>(y + G::offset(at[u]), v[u]);
         }
 }
 
@@ -195,8 +235,8 @@ struct OnceBackward
 
 // IN_LDS: that many of a thread's K vectors of dy stay in LDS, where the registers
 // of a CU do not hold both tensors (each thread reads what it has written).
-template <typename T, int TEAM, int K, bool STREAM, int IN_LDS = 0>
-__global__ __launch_bounds__(once_block<TEAM>()) void bn_once_backward_kernel(const OnceGeometry g,
+template <typename T, int TEAM, int K, bool STREAM, int IN_LDS, typename G>
+__global__ __launch_bounds__(once_block<TEAM>()) void bn_once_backward_kernel(const G g,
                                                                              const OnceBackward<T> a)
 {
     static_assert(TEAM == kWaveSize || TEAM >= kBlockSize, "a wave or a workgroup");
@@ -222,11 +262,11 @@ __global__ __launch_bounds__(once_block<TEAM>()) void bn_once_backward_kernel(co
         if (live(u))
         {
             at[u] = once_place<VEC>(g, u * TEAM + t);
-            load_vec<T, VEC, false>(a.x + base + (at[u] >> 2), xv[u]);
+            load_vec<T, VEC, false>(a.x + base + G::offset(at[u]), xv[u]);
             if (u < IN_LDS)
             {
                 T d[VEC];
-                load_vec<T, VEC, false>(a.dy + base + (at[u] >> 2), d);
+                load_vec<T, VEC, false>(a.dy + base + G::offset(at[u]), d);
                 V p;
 #pragma unroll
                 for (int j = 0; j < VEC; ++j)
@@ -235,7 +275,7 @@ __global__ __launch_bounds__(once_block<TEAM>()) void bn_once_backward_kernel(co
             }
             else
             {
-                load_vec<T, VEC, false>(a.dy + base + (at[u] >> 2), dv[u < IN_LDS ? 0 : u - IN_LDS]);
+                load_vec<T, VEC, false>(a.dy + base + G::offset(at[u]), dv[u < IN_LDS ? 0 : u - IN_LDS]);
             }
         }
     const T m = a.mean[c];
@@ -251,7 +291,7 @@ __global__ __launch_bounds__(once_block<TEAM>()) void bn_once_backward_kernel(co
             gradient(u, d);
 #pragma unroll
             for (int j = 0; j < VEC; ++j)
-                if (j >= static_cast<int>(at[u] & 3))
+                if (G::counts(at[u], j))
                 {
                     const T xm = xv[u][j] - m;
                     const T dxhat = d[j] * sc;
@@ -282,7 +322,9 @@ __global__ __launch_bounds__(once_block<TEAM>()) void bn_once_backward_kernel(co
             gradient(u, d);
 #pragma unroll
             for (int j = 0; j < VEC; ++j)
-                xv[u][j] = fma_t(xv[u][j] - m, dvar_term, fma_t(d[j] * sc, inv_stdev, dmean_term));
-            store_once<T, VEC, STREAM>(a.dx + base + (at[u] >> 2), xv[u]);
+                xv[u][j] = G::kClears && !G::counts(at[u], j)
+                               ? T(0)
+                               : fma_t(xv[u][j] - m, dvar_term, fma_t(d[j] * sc, inv_stdev, dmean_term));
+            store_once<T, VEC, STREAM>(a.dx + base + G::offset(at[u]), xv[u]);
         }
 }

@@ -28,9 +28,10 @@
 constexpr uint32_t kMaxMembers = kBlockSize; // a thread looks after one slot, no team has fewer threads
 constexpr unsigned long long kNoSum = 0x7ff8000000000001ull;
 
+template <typename G>
 struct TeamGeometry
 {
-    OnceGeometry once;
+    G once;
     FastDiv members;   // of a team
     uint32_t span;     // vectors of a member, a multiple of its threads
     uint32_t max_polls;
@@ -45,8 +46,8 @@ __global__ __launch_bounds__(kBlockSize) void bn_team_clear_kernel(unsigned long
 
 // The sums of all members in v[] of every thread, given this member's own in v[] of
 // thread 0.  recompute(member, sums) is called by the whole workgroup.
-template <int TEAM, int N, typename F>
-__device__ __forceinline__ void team_exchange(double (&v)[N], const TeamGeometry& g, uint32_t c, uint32_t member,
+template <int TEAM, int N, typename G, typename F>
+__device__ __forceinline__ void team_exchange(double (&v)[N], const TeamGeometry<G>& g, uint32_t c, uint32_t member,
                                               unsigned long long* slots, double* lds, uint32_t* missing,
                                               const F& recompute)
 {
@@ -110,13 +111,13 @@ __device__ __forceinline__ void team_exchange(double (&v)[N], const TeamGeometry
         v[k] = s[k];
 }
 
-// The terms of one vector; `skip` leading elements belong to the vector before it.
-template <typename T, int VEC>
-__device__ __forceinline__ void add_forward_terms(double (&s)[2], const T (&v)[VEC], uint32_t skip)
+// The terms of the vector at place `at`.
+template <typename G, typename T, int VEC>
+__device__ __forceinline__ void add_forward_terms(double (&s)[2], const T (&v)[VEC], uint32_t at)
 {
 #pragma unroll
     for (int j = 0; j < VEC; ++j)
-        if (j >= static_cast<int>(skip))
+        if (G::counts(at, j))
         {
             const double d = static_cast<double>(v[j]);
             s[0] += d;
@@ -124,13 +125,13 @@ __device__ __forceinline__ void add_forward_terms(double (&s)[2], const T (&v)[V
         }
 }
 
-template <typename T, int VEC>
-__device__ __forceinline__ void add_backward_terms(double (&s)[4], const T (&x)[VEC], const T (&d)[VEC], uint32_t skip,
+template <typename G, typename T, int VEC>
+__device__ __forceinline__ void add_backward_terms(double (&s)[4], const T (&x)[VEC], const T (&d)[VEC], uint32_t at,
                                                    T m, T sc, T inv_stdev)
 {
 #pragma unroll
     for (int j = 0; j < VEC; ++j)
-        if (j >= static_cast<int>(skip))
+        if (G::counts(at, j))
         {
             const T xm = x[j] - m;
             const T dxhat = d[j] * sc;
@@ -142,8 +143,8 @@ __device__ __forceinline__ void add_backward_terms(double (&s)[4], const T (&x)[
         }
 }
 
-template <typename T, int TEAM, int K, bool STREAM>
-__global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometry g, const OnceForward<T> a,
+template <typename T, int TEAM, int K, bool STREAM, typename G>
+__global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometry<G> g, const OnceForward<T> a,
                                                                       unsigned long long* slots)
 {
     constexpr int VEC = 16 / sizeof(T);
@@ -163,13 +164,13 @@ __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometr
         if (live(u))
         {
             at[u] = once_place<VEC>(g.once, first + u * TEAM + threadIdx.x);
-            load_vec<T, VEC, false>(x + (at[u] >> 2), v[u]);
+            load_vec<T, VEC, false>(x + G::offset(at[u]), v[u]);
         }
     double s[2] = {0.0, 0.0};
 #pragma unroll
     for (int u = 0; u < K; ++u)
         if (live(u))
-            add_forward_terms<T, VEC>(s, v[u], at[u] & 3);
+            add_forward_terms<G, T, VEC>(s, v[u], at[u]);
     team_sum<TEAM>(s, lds[0]);
     team_exchange<TEAM, 2>(s, g, c, member, slots, lds[1], missing, [&](uint32_t other, double (&r)[2]) {
         r[0] = r[1] = 0.0;
@@ -178,8 +179,8 @@ __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometr
         {
             const uint32_t p = once_place<VEC>(g.once, i);
             T w[VEC];
-            load_vec<T, VEC, false>(x + (p >> 2), w);
-            add_forward_terms<T, VEC>(r, w, p & 3);
+            load_vec<T, VEC, false>(x + G::offset(p), w);
+            add_forward_terms<G, T, VEC>(r, w, p);
         }
         __syncthreads(); // lds[2] may still be read
         team_sum<TEAM>(r, lds[2]);
@@ -202,13 +203,13 @@ __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometr
         {
 #pragma unroll
             for (int j = 0; j < VEC; ++j)
-                v[u][j] = fma_t((v[u][j] - m) * inv_stdev, sc, bi);
-            store_once<T, VEC, STREAM>(y + (at[u] >> 2), v[u]);
+                v[u][j] = G::kClears && !G::counts(at[u], j) ? T(0) : fma_t((v[u][j] - m) * inv_stdev, sc, bi);
+            store_once<T, VEC, STREAM>(y + G::offset(at[u]), v[u]);
         }
 }
 
-template <typename T, int TEAM, int K, bool STREAM>
-__global__ __launch_bounds__(TEAM) void bn_team_backward_kernel(const TeamGeometry g, const OnceBackward<T> a,
+template <typename T, int TEAM, int K, bool STREAM, typename G>
+__global__ __launch_bounds__(TEAM) void bn_team_backward_kernel(const TeamGeometry<G> g, const OnceBackward<T> a,
                                                                        unsigned long long* slots)
 {
     constexpr int VEC = 16 / sizeof(T);
@@ -228,8 +229,8 @@ __global__ __launch_bounds__(TEAM) void bn_team_backward_kernel(const TeamGeomet
         if (live(u))
         {
             at[u] = once_place<VEC>(g.once, first + u * TEAM + threadIdx.x);
-            load_vec<T, VEC, false>(a.x + base + (at[u] >> 2), xv[u]);
-            load_vec<T, VEC, false>(a.dy + base + (at[u] >> 2), dv[u]);
+            load_vec<T, VEC, false>(a.x + base + G::offset(at[u]), xv[u]);
+            load_vec<T, VEC, false>(a.dy + base + G::offset(at[u]), dv[u]);
         }
     const T m = a.mean[c];
     const T sc = a.scale[c];
@@ -239,7 +240,7 @@ __global__ __launch_bounds__(TEAM) void bn_team_backward_kernel(const TeamGeomet
 #pragma unroll
     for (int u = 0; u < K; ++u)
         if (live(u))
-            add_backward_terms<T, VEC>(s, xv[u], dv[u], at[u] & 3, m, sc, inv_stdev);
+            add_backward_terms<G, T, VEC>(s, xv[u], dv[u], at[u], m, sc, inv_stdev);
     team_sum<TEAM>(s, lds[0]);
     team_exchange<TEAM, 4>(s, g, c, member, slots, lds[1], missing, [&](uint32_t other, double (&r)[4]) {
         r[0] = r[1] = r[2] = r[3] = 0.0;
@@ -248,9 +249,9 @@ __global__ __launch_bounds__(TEAM) void bn_team_backward_kernel(const TeamGeomet
         {
             const uint32_t p = once_place<VEC>(g.once, i);
             T w[VEC], d[VEC];
-            load_vec<T, VEC, false>(a.x + base + (p >> 2), w);
-            load_vec<T, VEC, false>(a.dy + base + (p >> 2), d);
-            add_backward_terms<T, VEC>(r, w, d, p & 3, m, sc, inv_stdev);
+            load_vec<T, VEC, false>(a.x + base + G::offset(p), w);
+            load_vec<T, VEC, false>(a.dy + base + G::offset(p), d);
+            add_backward_terms<G, T, VEC>(r, w, d, p, m, sc, inv_stdev);
         }
         __syncthreads(); // lds[2] may still be read
         team_sum<TEAM>(r, lds[2]);
@@ -272,7 +273,9 @@ __global__ __launch_bounds__(TEAM) void bn_team_backward_kernel(const TeamGeomet
         {
 #pragma unroll
             for (int j = 0; j < VEC; ++j)
-                xv[u][j] = fma_t(xv[u][j] - m, dvar_term, fma_t(dv[u][j] * sc, inv_stdev, dmean_term));
-            store_once<T, VEC, STREAM>(a.dx + base + (at[u] >> 2), xv[u]);
+                xv[u][j] = G::kClears && !G::counts(at[u], j)
+                               ? T(0)
+                               : fma_t(xv[u][j] - m, dvar_term, fma_t(dv[u][j] * sc, inv_stdev, dmean_term));
+            store_once<T, VEC, STREAM>(a.dx + base + G::offset(at[u]), xv[u]);
         }
 }

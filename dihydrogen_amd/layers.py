@@ -131,8 +131,7 @@ class BatchNormalization:
     def _num_per_sum(self, t: Tensor) -> int:
         """Elements per channel of the global (global_stats) or local shape
         (batchnorm.hpp:232-236,414-418)."""
-        l = t.layout
-        return l.per_channel_global if self.global_stats else l.per_channel_local
+        return self._elements_per_sum(t.layout)
 
     # ---- forward -----------------------------------------------------------
     def forward_stage1(self, input: Tensor, mean: torch.Tensor, var: torch.Tensor,
@@ -194,18 +193,32 @@ class BatchNormalization:
             self.batch_normalization(input, running_mean, running_var, scale, bias, output)  # :243-247
         return 0
 
-    def _runs_local(self, l0: Layout, haloed: bool) -> bool:
-        """No all-reduce between the stages, a rank that owns elements (and no halo to clear)."""
-        return (self.fuse_local and l0.active and (self.allreduce is None or not self.global_stats)
-                and not (haloed and self.clear_output_halo))
+    def _runs_local(self, l0: Layout) -> bool:
+        """No all-reduce between the stages, a rank that owns elements."""
+        return self.fuse_local and l0.active and (self.allreduce is None or not self.global_stats)
+
+    def _elements_per_sum(self, l: Layout) -> int:
+        return l.per_channel_global if self.global_stats else l.per_channel_local
 
     def forward(self, input, mean, var, running_mean, running_var, scale, bias, output,
                 is_training: bool = True) -> int:
         lx, ly = input.layout, output.layout
-        if is_training and self._runs_local(lx, lx.haloed or ly.haloed):
+        local = is_training and self._runs_local(lx)
+        if local and self.clear_output_halo and (lx.haloed or ly.haloed):
+            local = False  # the stages, unless a whole pass clears the halo
+            if _share_a_haloed_geometry(lx, ly):
+                status = self._calls.h2x_bn_forward_clearing(
+                    lx.dtype, lx.haloed_geometry_address, input.get_buffer(), scale, bias, self._elements_per_sum(lx),
+                    self.decay, self.epsilon, mean, var, running_mean, running_var, output.get_buffer(),
+                    self._ws(lx.channels), _stream_handle(self.stream))
+                if status != capi.ERR_UNSUPPORTED:
+                    self.num_current_samples = lx.samples
+                    capi.check(status, "bn forward (clearing)")
+                    return 0
+        if local:
             _dense_layout(input), _dense_layout(output)
             ns = self.num_current_samples = lx.samples
-            per_sum = lx.per_channel_global if self.global_stats else lx.per_channel_local
+            per_sum = self._elements_per_sum(lx)
             status = self._calls.h2x_bn_forward_once(
                 lx.dtype, ns, lx.geometry_address, _tensor_geometry(ly, ns), input.get_base_ptr(), scale, bias, per_sum,
                 self.decay, self.epsilon, mean, var, running_mean, running_var, output.get_base_ptr(),
@@ -271,10 +284,23 @@ class BatchNormalization:
     def backward(self, input, d_output, mean, var, scale, scale_gradient, bias_gradient,
                  mean_gradient, var_gradient, d_input) -> int:
         lx, ld, li = input.layout, d_output.layout, d_input.layout
-        if self._runs_local(lx, lx.haloed or ld.haloed or li.haloed):
+        local = self._runs_local(lx)
+        if local and self.clear_output_halo and (lx.haloed or ld.haloed or li.haloed):
+            local = False
+            if _share_a_haloed_geometry(lx, ld, li):
+                status = self._calls.h2x_bn_backward_clearing(
+                    lx.dtype, self._elements_per_sum(lx), lx.haloed_geometry_address, input.get_buffer(),
+                    d_output.get_buffer(), mean, var, scale, scale_gradient, bias_gradient, mean_gradient,
+                    var_gradient, d_input.get_buffer(), self.epsilon, self._ws(lx.channels),
+                    _stream_handle(self.stream))
+                if status != capi.ERR_UNSUPPORTED:
+                    self.num_current_samples = lx.samples
+                    capi.check(status, "bn backward (clearing)")
+                    return 0
+        if local:
             _dense_layout(input), _dense_layout(d_output), _dense_layout(d_input)
             ns = self.num_current_samples = lx.samples
-            per_sum = lx.per_channel_global if self.global_stats else lx.per_channel_local
+            per_sum = self._elements_per_sum(lx)
             status = self._calls.h2x_bn_backward_once(
                 lx.dtype, ns, per_sum, lx.geometry_address, _tensor_geometry(ld, ns), _tensor_geometry(li, ns),
                 input.get_base_ptr(), d_output.get_base_ptr(), mean, var, scale, scale_gradient, bias_gradient,

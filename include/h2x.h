@@ -584,6 +584,44 @@ int h2x_bn_backprop2_clearing(h2x_dtype dtype,
                               h2x_stream_t stream);
 
 /**
+ * A whole forward or backward pass of a rank that shares its statistics with no one,
+ * the output's halo left cleared as by the two calls above: for float tensors whose
+ * channels one workgroup, or a team of them, holds in registers.
+ * H2X_ERR_UNSUPPORTED, with nothing launched, for others.
+ */
+int h2x_bn_forward_clearing(h2x_dtype dtype,
+                            const h2x_haloed_geometry* geometry,
+                            const void* x_buffer,
+                            const void* scale,
+                            const void* bias,
+                            size_t num_per_sum,
+                            double decay,
+                            double epsilon,
+                            void* mean,
+                            void* var,
+                            void* running_mean,
+                            void* running_var,
+                            void* y_buffer,
+                            void* workspace,
+                            h2x_stream_t stream);
+int h2x_bn_backward_clearing(h2x_dtype dtype,
+                             size_t num_per_sum,
+                             const h2x_haloed_geometry* geometry,
+                             const void* x_buffer,
+                             const void* dy_buffer,
+                             const void* mean,
+                             const void* var,
+                             const void* scale,
+                             void* dscale,
+                             void* dbias,
+                             void* dmean,
+                             void* dvar,
+                             void* dx_buffer,
+                             double epsilon,
+                             void* workspace,
+                             h2x_stream_t stream);
+
+/**
  * Launch audit, on the host: no GPU call is made and no pointer is followed.
  * No counterpart in the reference, whose kernels check nothing of the kind;
  * it exists so that the choice of kernels and their indexing can be verified

@@ -129,3 +129,44 @@ def test_overlapping_outputs_are_not_for_teams():
     assert lib.h2x_bn_forward_team(capi.F32, 2, gp, gp, x, p.scale.data_ptr(), p.bias.data_ptr(), p.per, 0.9, 1e-5, *v, x,
                                    p.ws.data_ptr(), 2048, None) == -2  # unsupported
     _close(p.run("once", in_place=True), p.run("local_strided"))
+
+
+@pytest.mark.parametrize("in_place", [False, True])
+@pytest.mark.parametrize("shape,halo", [((1, 2, 5, 6, 6), 1), ((3, 5, 10, 10, 10), 1), ((4, 3, 1, 30, 30), 1),
+                                        ((2, 4, 1, 58, 30), 3), ((2, 100, 30, 30, 30), 1), ((16, 64, 30, 30, 30), 1),
+                                        ((2, 64, 44, 62, 62), 1)])
+def test_whole_pass_that_clears_the_halo(shape, halo, in_place):
+    """As the two-launch calls on the interior, zeros in the halo, in one workgroup a channel and in teams
+    (which outputs that overlap inputs are not for: the call refuses or is done by one workgroup)."""
+    import torch
+    p = _Problem(*shape, halo=halo)
+    want = p.run("local_strided")
+    n, c, d, h, w = shape
+    hd = halo if d > 1 else 0
+    g = capi.HaloedGeometry()
+    g.num_dims = 5
+    for i, (e, o) in enumerate(zip((w, h, d, c, n), (halo, halo, hd, 0, 0))):
+        g.local_shape[i], g.real_shape[i], g.lower_halo[i] = e, e + 2 * o, o
+    lib, gp = capi.load(), ctypes.byref(g)
+    x, dy = (torch.full_like(t, float("nan")) for t in (p.x, p.dy))
+    x[p.inner], dy[p.inner] = p.x[p.inner], p.dy[p.inner]
+    vec = lambda v: torch.full_like(p.scale, v)
+    mean, var, rm, rv = vec(float("nan")), vec(float("nan")), vec(0.25), vec(0.75)
+    grads = [vec(float("nan")) for _ in range(4)]
+    a = lambda t: t.data_ptr()
+    y = x.clone() if in_place else torch.full_like(x, 7)
+    status = lib.h2x_bn_forward_clearing(capi.F32, gp, a(y if in_place else x), a(p.scale), a(p.bias), p.per, 0.9, 1e-5, a(mean),
+                                         a(var), a(rm), a(rv), a(y), a(p.ws), None)
+    if status == -2:
+        assert in_place and p.x[0, 0].numel() * n > 32768
+        return
+    assert status == 0
+    dx = x.clone() if in_place else torch.full_like(x, 7)
+    assert lib.h2x_bn_backward_clearing(capi.F32, p.per, gp, a(dx if in_place else x), a(dy), a(mean), a(var), a(p.scale),
+                                        *[a(t) for t in grads], a(dx), 1e-5, a(p.ws), None) == 0
+    torch.cuda.synchronize()
+    for out in (y, dx):
+        rest = out.clone()
+        rest[p.inner] = 0
+        assert bool((rest == 0).all())
+    _close([y[p.inner], dx[p.inner], mean, var, rm, rv] + grads, want)
