@@ -772,8 +772,8 @@ def main() -> int:
     nps = b._num_per_sum(bn3.x)
 
     def step():
-        """The timed step: the layer's own forward() and backward() (two launches each: the
-        second kernel of each finishes the first one's channel sums) and the exchange."""
+        """The timed step: the layer's own forward() and backward() (each a small fill and one kernel
+        that holds the channels in registers) and the exchange."""
         bn3.forward()
         bn3.backward()
         halo.run()
