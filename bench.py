@@ -772,7 +772,7 @@ def main() -> int:
     nps = b._num_per_sum(bn3.x)
 
     def step():
-        """The timed step: the layer's own forward() and backward() (each a small fill and one kernel
+        """The timed step: the layer's own forward() and backward() (each one kernel
         that holds the channels in registers) and the exchange."""
         bn3.forward()
         bn3.backward()

@@ -210,13 +210,14 @@ SIGNATURES = {
                                               POINTER(TensorGeometry), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                               c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_double, c_void_p,
                                               c_void_p]),
+    "h2x_bn_team_state_bytes": (c_size_t, [c_int]),
     "h2x_bn_forward_once": (c_int, [c_int, c_int, POINTER(TensorGeometry), POINTER(TensorGeometry), c_void_p,
-                                             c_void_p, c_void_p, c_size_t, c_double, c_double, c_void_p, c_void_p,
-                                             c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+                                    c_void_p, c_void_p, c_size_t, c_double, c_double, c_void_p, c_void_p,
+                                    c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "h2x_bn_backward_once": (c_int, [c_int, c_int, c_size_t, POINTER(TensorGeometry), POINTER(TensorGeometry),
-                                              POINTER(TensorGeometry), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
-                                              c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_double, c_void_p,
-                                              c_void_p]),
+                                     POINTER(TensorGeometry), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                                     c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_double, c_void_p,
+                                     c_void_p, c_void_p]),
     "h2x_bn_forward_team": (c_int, [c_int, c_int, POINTER(TensorGeometry), POINTER(TensorGeometry), c_void_p,
                                     c_void_p, c_void_p, c_size_t, c_double, c_double, c_void_p, c_void_p,
                                     c_void_p, c_void_p, c_void_p, c_void_p, c_uint32, c_void_p]),

@@ -1344,7 +1344,7 @@ __global__ __launch_bounds__(kBlockSize) void bn_backprop2_short_kernel(
 
 // ---- whole channels in one workgroup: one launch ------------------------------
 #include "h2x_bn_once.hpp"
-// ---- whole channels in several workgroups: one launch behind a small fill -------
+// ---- whole channels in several workgroups: one launch ---------------------------
 #include "h2x_bn_team.hpp"
 
 // ---- host side ---------------------------------------------------------------
@@ -2700,41 +2700,37 @@ bool apart(const void* a, const void* b, size_t bytes)
 }
 
 template <typename T, int TEAM, int K, bool STREAM, typename G>
-void issue_team(const TeamGeometry<G>& g, const OnceForward<T>& a, unsigned long long* slots, hipStream_t st)
+void issue_team(const TeamGeometry<G>& g, const OnceForward<T>& a, unsigned long long* states, hipStream_t st)
 {
-    bn_team_forward_kernel<T, TEAM, K, STREAM><<<g.once.num_channels * g.members.divisor, TEAM, 0, st>>>(g, a, slots);
+    bn_team_forward_kernel<T, TEAM, K, STREAM><<<g.once.num_channels * g.members.divisor, TEAM, 0, st>>>(g, a, states);
 }
 template <typename T, int TEAM, int K, bool STREAM, typename G>
-void issue_team(const TeamGeometry<G>& g, const OnceBackward<T>& a, unsigned long long* slots, hipStream_t st)
+void issue_team(const TeamGeometry<G>& g, const OnceBackward<T>& a, unsigned long long* states, hipStream_t st)
 {
-    bn_team_backward_kernel<T, TEAM, K, STREAM><<<g.once.num_channels * g.members.divisor, TEAM, 0, st>>>(g, a, slots);
+    bn_team_backward_kernel<T, TEAM, K, STREAM><<<g.once.num_channels * g.members.divisor, TEAM, 0, st>>>(g, a, states);
 }
 
-// Members of TEAM threads with K vectors each; false if that is fewer than `least` or
-// more than `most` members, or more slots than the workspace has.
+// Members of TEAM threads with K vectors each; false if that is fewer than `least` workgroups,
+// more than `most` members, or more sums than a channel's state has.
 template <int TEAM, int K, typename G, template <typename> class A, typename T>
 bool team_launch(const G& once, const A<T>& a, bool stream, uint32_t least, uint32_t most,
-                 uint32_t max_polls, void* ws, hipStream_t st)
+                 uint32_t max_polls, void* team_state, hipStream_t st)
 {
     constexpr int kSums = std::is_same<A<T>, OnceForward<T>>::value ? 2 : 4;
     const uint32_t members = (once.vectors + TEAM * K - 1) / (TEAM * K);
     const size_t blocks = static_cast<size_t>(members) * once.num_channels;
-    const size_t count = blocks * kSums;
-    if (members > most || blocks < least || count >= (1u << 30)
-        || count * sizeof(double) > partials_bytes(static_cast<int>(once.num_channels)))
+    if (members > most || members * kSums > kMaxTeamSums || blocks < least || blocks >= (1u << 30))
         return false;
     TeamGeometry<G> g;
     g.once = once;
     g.members = make_fastdiv(members);
     g.span = ((once.vectors + members - 1) / members + TEAM - 1) / TEAM * TEAM;
     g.max_polls = max_polls;
-    unsigned long long* const slots = static_cast<unsigned long long*>(ws);
-    bn_team_clear_kernel<<<static_cast<unsigned int>((count + kBlockSize - 1) / kBlockSize), kBlockSize, 0, st>>>(
-        slots, static_cast<uint32_t>(count));
+    unsigned long long* const states = static_cast<unsigned long long*>(team_state);
     if (stream || G::kClears)
-        issue_team<T, TEAM, K, true>(g, a, slots, st);
+        issue_team<T, TEAM, K, true>(g, a, states, st);
     else
-        issue_team<T, TEAM, K, G::kClears>(g, a, slots, st);
+        issue_team<T, TEAM, K, G::kClears>(g, a, states, st);
     return true;
 }
 
@@ -2750,10 +2746,10 @@ constexpr uint32_t kTeamLeastBlocks = 192;
 // of them 98 us, in two launches 118).
 template <typename G, typename T>
 bool team_variant(const G& g, const OnceForward<T>& a, bool stream, uint32_t least, uint32_t most,
-                  uint32_t polls, void* ws, hipStream_t st)
+                  uint32_t polls, void* team_state, hipStream_t st)
 {
-    return team_launch<512, 16>(g, a, stream, 2 * least, most, polls, ws, st)
-           || team_launch<512, 8>(g, a, stream, least, most, polls, ws, st);
+    return team_launch<512, 16>(g, a, stream, 2 * least, most, polls, team_state, st)
+           || team_launch<512, 8>(g, a, stream, least, most, polls, team_state, st);
 }
 
 // Backward 64 KB of each tensor, 128 KB where a team would have more than 64 members
@@ -2762,18 +2758,20 @@ bool team_variant(const G& g, const OnceForward<T>& a, bool stream, uint32_t lea
 // its last member than it saves.
 template <typename G, typename T>
 bool team_variant(const G& g, const OnceBackward<T>& a, bool stream, uint32_t least, uint32_t most,
-                  uint32_t polls, void* ws, hipStream_t st)
+                  uint32_t polls, void* team_state, hipStream_t st)
 {
     most /= 2;
-    return team_launch<512, 8>(g, a, stream, least, most, polls, ws, st)
-           || team_launch<1024, 8>(g, a, stream, least, most, polls, ws, st);
+    return team_launch<512, 8>(g, a, stream, least, most, polls, team_state, st)
+           || team_launch<1024, 8>(g, a, stream, least, most, polls, team_state, st);
 }
 
 // False: the call is not for teams.  bytes: from the first to behind the last element of a tensor.
 template <typename G, typename A>
 bool launch_by_teams(const G& g, const A& a, size_t bytes, bool stream, std::initializer_list<const void*> inputs,
-                     const void* output, uint32_t least, uint32_t polls, void* ws, hipStream_t st)
+                     const void* output, uint32_t least, uint32_t polls, void* team_state, hipStream_t st)
 {
+    if (!team_state)
+        return false;
     for (const void* p : inputs)
         if (!apart(p, output, bytes))
             return false;
@@ -2781,25 +2779,25 @@ bool launch_by_teams(const G& g, const A& a, size_t bytes, bool stream, std::ini
     if (hipGetDevice(&device) != hipSuccess
         || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
         return false;
-    return team_variant(g, a, stream, least, std::min<uint32_t>(cus / 2, kMaxMembers), polls, ws, st);
+    return team_variant(g, a, stream, least, std::min<uint32_t>(cus / 2, kMaxMembers), polls, team_state, st);
 }
 
 template <typename A>
 bool launch_by_teams(const OnceGeometry& g, const A& a, int n, std::initializer_list<const void*> inputs,
-                     const void* output, uint32_t least, uint32_t polls, void* ws, hipStream_t st)
+                     const void* output, uint32_t least, uint32_t polls, void* team_state, hipStream_t st)
 {
     // short segments have kernels of their own (N 2048, C 256, 7 x 7: 141 us, by teams 172)
     const bool stream = streamed(g, n);
     if (dense_rows(g) && !stream)
         return false;
-    return launch_by_teams(g, a, reach_bytes(g, n), stream, inputs, output, least, polls, ws, st);
+    return launch_by_teams(g, a, reach_bytes(g, n), stream, inputs, output, least, polls, team_state, st);
 }
 
 // team_polls: by teams or not at all, however few workgroups that is, with this many looks.
 template <typename T>
 int forward_once(int n, const h2x_tensor_geometry* gx, const h2x_tensor_geometry* gy, const void* x,
                  const void* scale, const void* bias, size_t num_per_sum, double decay, double eps, void* mean,
-                 void* var, void* running_mean, void* running_var, void* y, void* ws, hipStream_t st,
+                 void* var, void* running_mean, void* running_var, void* y, void* ws, void* team_state, hipStream_t st,
                   const uint32_t* team_polls = nullptr)
 {
     HostTensor tx, ty;
@@ -2818,10 +2816,10 @@ int forward_once(int n, const h2x_tensor_geometry* gx, const h2x_tensor_geometry
                                    static_cast<T*>(running_var), static_cast<T*>(y), static_cast<T>(num_per_sum),
                                    static_cast<T>(decay), static_cast<T>(eps)};
             if (team_polls)
-                return launch_by_teams(g, a, n, {x}, y, 1, *team_polls, ws, st) ? launch_status()
+                return launch_by_teams(g, a, n, {x}, y, 1, *team_polls, team_state, st) ? launch_status()
                                                                             : H2X_ERR_UNSUPPORTED;
             if (once_launch(g, a, n, st)
-                || launch_by_teams(g, a, n, {x}, y, kTeamLeastBlocks, kTeamPolls, ws, st))
+                || launch_by_teams(g, a, n, {x}, y, kTeamLeastBlocks, kTeamPolls, team_state, st))
                 return launch_status();
         }
     }
@@ -2835,7 +2833,7 @@ template <typename T>
 int backward_once(int n, size_t num_per_sum, const h2x_tensor_geometry* gx, const h2x_tensor_geometry* gd,
                   const h2x_tensor_geometry* go, const void* x, const void* dy, const void* mean, const void* var,
                   const void* scale, void* dscale, void* dbias, void* dmean, void* dvar, void* dx, double eps,
-                  void* ws, hipStream_t st,
+                  void* ws, void* team_state, hipStream_t st,
                    const uint32_t* team_polls = nullptr)
 {
     HostTensor tx, td, to;
@@ -2855,10 +2853,10 @@ int backward_once(int n, size_t num_per_sum, const h2x_tensor_geometry* gx, cons
                                     static_cast<T*>(dx), static_cast<T>(num_per_sum),
                                     static_cast<T>(num_per_sum - 1), static_cast<T>(eps)};
             if (team_polls)
-                return launch_by_teams(g, a, n, {x, dy}, dx, 1, *team_polls, ws, st) ? launch_status()
+                return launch_by_teams(g, a, n, {x, dy}, dx, 1, *team_polls, team_state, st) ? launch_status()
                                                                             : H2X_ERR_UNSUPPORTED;
             if (once_launch(g, a, n, st)
-                || launch_by_teams(g, a, n, {x, dy}, dx, kTeamLeastBlocks, kTeamPolls, ws, st))
+                || launch_by_teams(g, a, n, {x, dy}, dx, kTeamLeastBlocks, kTeamPolls, team_state, st))
                 return launch_status();
         }
     }
@@ -2872,7 +2870,7 @@ int backward_once(int n, size_t num_per_sum, const h2x_tensor_geometry* gx, cons
 // or a team a channel; H2X_ERR_UNSUPPORTED: in the staged calls.
 template <typename A>
 int clearing_once(const h2x_haloed_geometry* h, const A& a, std::initializer_list<const void*> inputs, void* output,
-                  void* ws, hipStream_t st)
+                  void* team_state, hipStream_t st)
 {
     ClearGeometry g;
     size_t real;
@@ -2896,8 +2894,8 @@ int clearing_once(const h2x_haloed_geometry* h, const A& a, std::initializer_lis
     g.stride_c = static_cast<int64_t>(real);
     g.num_channels = static_cast<uint32_t>(c);
     if (once_launch<true>(g, a, st)
-        || launch_by_teams(g, a, n * c * real * sizeof(float), true, inputs, output, kTeamLeastBlocks, kTeamPolls, ws,
-                           st))
+        || launch_by_teams(g, a, n * c * real * sizeof(float), true, inputs, output, kTeamLeastBlocks, kTeamPolls,
+                           team_state, st))
         return launch_status();
     return H2X_ERR_UNSUPPORTED;
 }
@@ -3277,13 +3275,18 @@ extern "C" int h2x_bn_backward_local_strided(h2x_dtype dtype, int num_samples, s
                                                 as_stream(stream)));
 }
 
+extern "C" size_t h2x_bn_team_state_bytes(int num_channels)
+{
+    return static_cast<size_t>(std::max(num_channels, 1)) * kStateWords * sizeof(unsigned long long);
+}
+
 extern "C" int h2x_bn_forward_once(h2x_dtype dtype, int num_samples,
                                             const h2x_tensor_geometry* x_geometry,
                                             const h2x_tensor_geometry* y_geometry, const void* x,
                                             const void* scale, const void* bias, size_t num_per_sum,
                                             double decay, double epsilon, void* mean, void* var,
                                             void* running_mean, void* running_var, void* y,
-                                            void* workspace, h2x_stream_t stream)
+                                            void* workspace, void* team_state, h2x_stream_t stream)
 {
     if (num_samples < 0 || !x_geometry || !y_geometry || !scale || !bias || !mean || !var
         || !running_mean || !running_var || !workspace)
@@ -3291,10 +3294,10 @@ extern "C" int h2x_bn_forward_once(h2x_dtype dtype, int num_samples,
     H2X_BY_DTYPE(dtype,
                  forward_once<float>(num_samples, x_geometry, y_geometry, x, scale, bias,
                                               num_per_sum, decay, epsilon, mean, var, running_mean,
-                                              running_var, y, workspace, as_stream(stream)),
+                                              running_var, y, workspace, team_state, as_stream(stream)),
                  forward_once<double>(num_samples, x_geometry, y_geometry, x, scale, bias,
                                                num_per_sum, decay, epsilon, mean, var, running_mean,
-                                               running_var, y, workspace, as_stream(stream)));
+                                               running_var, y, workspace, team_state, as_stream(stream)));
 }
 
 extern "C" int h2x_bn_backward_once(h2x_dtype dtype, int num_samples, size_t num_per_sum,
@@ -3304,7 +3307,7 @@ extern "C" int h2x_bn_backward_once(h2x_dtype dtype, int num_samples, size_t num
                                              const void* dy, const void* mean, const void* var,
                                              const void* scale, void* dscale, void* dbias,
                                              void* dmean, void* dvar, void* dx, double epsilon,
-                                             void* workspace, h2x_stream_t stream)
+                                             void* workspace, void* team_state, h2x_stream_t stream)
 {
     if (num_samples < 0 || !x_geometry || !dy_geometry || !dx_geometry || !mean || !var || !scale
         || !dscale || !dbias || !dmean || !dvar || !workspace)
@@ -3312,27 +3315,27 @@ extern "C" int h2x_bn_backward_once(h2x_dtype dtype, int num_samples, size_t num
     H2X_BY_DTYPE(dtype,
                  backward_once<float>(num_samples, num_per_sum, x_geometry, dy_geometry,
                                                dx_geometry, x, dy, mean, var, scale, dscale, dbias,
-                                               dmean, dvar, dx, epsilon, workspace, as_stream(stream)),
+                                               dmean, dvar, dx, epsilon, workspace, team_state, as_stream(stream)),
                  backward_once<double>(num_samples, num_per_sum, x_geometry, dy_geometry,
                                                 dx_geometry, x, dy, mean, var, scale, dscale, dbias,
-                                                dmean, dvar, dx, epsilon, workspace,
+                                                dmean, dvar, dx, epsilon, workspace, team_state,
                                                 as_stream(stream)));
 }
 
 extern "C" int h2x_bn_forward_team(h2x_dtype dtype, int num_samples, const h2x_tensor_geometry* x_geometry,
                                    const h2x_tensor_geometry* y_geometry, const void* x, const void* scale,
                                    const void* bias, size_t num_per_sum, double decay, double epsilon, void* mean,
-                                   void* var, void* running_mean, void* running_var, void* y, void* workspace,
+                                   void* var, void* running_mean, void* running_var, void* y, void* team_state,
                                    unsigned int max_polls, h2x_stream_t stream)
 {
     if (num_samples < 0 || !x_geometry || !y_geometry || !scale || !bias || !mean || !var || !running_mean
-        || !running_var || !workspace)
+        || !running_var || !team_state)
         return H2X_ERR_INVALID_ARGUMENT;
     H2X_BY_DTYPE(dtype,
                  forward_once<float>(num_samples, x_geometry, y_geometry, x, scale, bias, num_per_sum, decay, epsilon,
-                                     mean, var, running_mean, running_var, y, workspace, as_stream(stream), &max_polls),
+                                     mean, var, running_mean, running_var, y, nullptr, team_state, as_stream(stream), &max_polls),
                  forward_once<double>(num_samples, x_geometry, y_geometry, x, scale, bias, num_per_sum, decay, epsilon,
-                                      mean, var, running_mean, running_var, y, workspace, as_stream(stream),
+                                      mean, var, running_mean, running_var, y, nullptr, team_state, as_stream(stream),
                                       &max_polls));
 }
 
@@ -3340,27 +3343,27 @@ extern "C" int h2x_bn_backward_team(h2x_dtype dtype, int num_samples, size_t num
                                     const h2x_tensor_geometry* x_geometry, const h2x_tensor_geometry* dy_geometry,
                                     const h2x_tensor_geometry* dx_geometry, const void* x, const void* dy,
                                     const void* mean, const void* var, const void* scale, void* dscale, void* dbias,
-                                    void* dmean, void* dvar, void* dx, double epsilon, void* workspace,
+                                    void* dmean, void* dvar, void* dx, double epsilon, void* team_state,
                                     unsigned int max_polls, h2x_stream_t stream)
 {
     if (num_samples < 0 || !x_geometry || !dy_geometry || !dx_geometry || !mean || !var || !scale || !dscale || !dbias
-        || !dmean || !dvar || !workspace)
+        || !dmean || !dvar || !team_state)
         return H2X_ERR_INVALID_ARGUMENT;
     H2X_BY_DTYPE(dtype,
                  backward_once<float>(num_samples, num_per_sum, x_geometry, dy_geometry, dx_geometry, x, dy, mean, var,
-                                      scale, dscale, dbias, dmean, dvar, dx, epsilon, workspace, as_stream(stream),
+                                      scale, dscale, dbias, dmean, dvar, dx, epsilon, nullptr, team_state, as_stream(stream),
                                       &max_polls),
                  backward_once<double>(num_samples, num_per_sum, x_geometry, dy_geometry, dx_geometry, x, dy, mean, var,
-                                       scale, dscale, dbias, dmean, dvar, dx, epsilon, workspace, as_stream(stream),
+                                       scale, dscale, dbias, dmean, dvar, dx, epsilon, nullptr, team_state, as_stream(stream),
                                        &max_polls));
 }
 
 extern "C" int h2x_bn_forward_clearing(h2x_dtype dtype, const h2x_haloed_geometry* geometry, const void* x_buffer,
                                        const void* scale, const void* bias, size_t num_per_sum, double decay,
                                        double epsilon, void* mean, void* var, void* running_mean, void* running_var,
-                                       void* y_buffer, void* workspace, h2x_stream_t stream)
+                                       void* y_buffer, void* team_state, h2x_stream_t stream)
 {
-    if (!geometry || !scale || !bias || !mean || !var || !running_mean || !running_var || !workspace)
+    if (!geometry || !scale || !bias || !mean || !var || !running_mean || !running_var)
         return H2X_ERR_INVALID_ARGUMENT;
     if (dtype != H2X_F32 || num_per_sum == 0)
         return H2X_ERR_UNSUPPORTED;
@@ -3369,16 +3372,16 @@ extern "C" int h2x_bn_forward_clearing(h2x_dtype dtype, const h2x_haloed_geometr
                            static_cast<T*>(mean), static_cast<T*>(var), static_cast<T*>(running_mean),
                            static_cast<T*>(running_var), static_cast<T*>(y_buffer), static_cast<T>(num_per_sum),
                            static_cast<T>(decay), static_cast<T>(epsilon)};
-    return clearing_once(geometry, a, {x_buffer}, y_buffer, workspace, as_stream(stream));
+    return clearing_once(geometry, a, {x_buffer}, y_buffer, team_state, as_stream(stream));
 }
 
 extern "C" int h2x_bn_backward_clearing(h2x_dtype dtype, size_t num_per_sum, const h2x_haloed_geometry* geometry,
                                         const void* x_buffer, const void* dy_buffer, const void* mean,
                                         const void* var, const void* scale, void* dscale, void* dbias, void* dmean,
-                                        void* dvar, void* dx_buffer, double epsilon, void* workspace,
+                                        void* dvar, void* dx_buffer, double epsilon, void* team_state,
                                         h2x_stream_t stream)
 {
-    if (!geometry || !mean || !var || !scale || !dscale || !dbias || !dmean || !dvar || !workspace)
+    if (!geometry || !mean || !var || !scale || !dscale || !dbias || !dmean || !dvar)
         return H2X_ERR_INVALID_ARGUMENT;
     if (dtype != H2X_F32)
         return H2X_ERR_UNSUPPORTED;
@@ -3388,7 +3391,7 @@ extern "C" int h2x_bn_backward_clearing(h2x_dtype dtype, size_t num_per_sum, con
                             static_cast<T*>(dscale), static_cast<T*>(dbias), static_cast<T*>(dmean),
                             static_cast<T*>(dvar), static_cast<T*>(dx_buffer), static_cast<T>(num_per_sum),
                             static_cast<T>(num_per_sum - 1), static_cast<T>(epsilon)};
-    return clearing_once(geometry, a, {x_buffer, dy_buffer}, dx_buffer, workspace, as_stream(stream));
+    return clearing_once(geometry, a, {x_buffer, dy_buffer}, dx_buffer, team_state, as_stream(stream));
 }
 
 // Plays on the host which elements the workgroups that hold channels in registers touch.

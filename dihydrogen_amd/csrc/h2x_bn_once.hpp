@@ -68,7 +68,7 @@ __host__ __device__ __forceinline__ uint32_t once_place(const OnceGeometry& g, u
 // Tensors of one haloed geometry whose outputs' halos are cleared: the vectors of the
 // whole allocation; halo elements are read and not counted, and stored as zeros.  Their
 // stores leave no partial lines (forward + backward, N 8, C 64, 30^3 with a halo of 1, us
-// going round three sets of tensors: 87 in six launches, 72 here, 81 without clearing).
+// going round three sets of tensors: 87 in six launches, 68 here, 78 without clearing).
 struct ClearGeometry
 {
     static constexpr bool kClears = true;

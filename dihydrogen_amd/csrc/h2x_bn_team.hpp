@@ -7,16 +7,24 @@
 // The two-launch kernels are bound by memory and read x (backward: x and dy) twice, at
 // 5 to 7 TB/s; here every element is read once.  Bound by memory and by the wait for the
 // last member of a team.  Forward, backward in us, two launches each way -> by teams:
-//   N 8, C 64, 30^3, halo of 1      38, 53 -> 35, 44     N 32, C 256, 56 x 56     48, 85 -> 36, 52
+//   N 8, C 64, 30^3, halo of 1      38, 53 -> 35, 43     N 32, C 256, 56 x 56     48, 85 -> 36, 52
 //   N 4, C 64, 64^3                116, 190 -> 90, 182   N 64, C 128, 40 x 40     27, 46 -> 21, 31
 //   N 8, C 64, 64^3                256, 407 -> 210, 355  N 2, C 32, 48^3          16, 28 -> 12, 18
 //   N 1, C 64, 96^3                 99, 162 -> 75, 147   N 64, C 64, 57^2, halo   31, 51 -> 33, 39
-// A counter of arrivals a team instead of looking at the slots themselves was slower the
+// (With a fill launch before each kernel; without it forward + backward of N 2, C 16, 48^3 with a
+// halo take 23.4 us instead of 26, N 8, C 64, 30^3 77.6 instead of 79.8.)
+// Looking at a counter of arrivals instead of the sums themselves was slower the
 // larger the team (64 members, N 4, C 64, 64^3: 119 us against 98): one address.
 //
-// What is exchanged validates itself: a slot holds kNoSum (a NaN that no sum can be)
-// until its member has stored a sum, in one 64-bit access of the whole device's scope,
-// so nothing else has to be ordered.  A fill kernel clears the slots before each call.
+// What is exchanged validates itself: half a sum travels with the tag of the call in one
+// 64-bit access of the whole device's scope, so nothing has to be ordered and nothing
+// cleared (a fill launch before the kernel cost 4.7 us behind streaming stores).  The tag is
+// the channel's counter plus one: a member reads the counter before it stores a sum,
+// and adds one to it when it has all sums, so all members of a call find the same
+// value, and no later call of that channel finds it again.  (A member that gave up
+// waiting may add early; who then reads a larger counter is not believed, believes
+// no one, and works all sums out.  The next call's counter is larger still.  Tags come
+// round after 2^32 arrivals; a word would have to lie untouched for just that long.)
 //
 // Nobody waits for ever: after max_polls looks a member works out the sums it misses
 // from memory, with the additions of the member they belong to, and gets the same
@@ -25,8 +33,13 @@
 // other streams fill it; the launch rule keeps a team within half of it.
 #pragma once
 
-constexpr uint32_t kMaxMembers = kBlockSize; // a thread looks after one slot, no team has fewer threads
-constexpr unsigned long long kNoSum = 0x7ff8000000000001ull;
+constexpr uint32_t kMaxTeamSums = 256; // of a channel: members times sums of a member
+constexpr uint32_t kMaxMembers = 128;  // a thread looks after one, no team has fewer threads
+
+// State of a channel, zero before its first call: the counter on a line of its own, then
+// two words a sum.
+constexpr uint32_t kCounterWords = 16;
+constexpr uint32_t kStateWords = kCounterWords + 2 * kMaxTeamSums;
 
 template <typename G>
 struct TeamGeometry
@@ -37,54 +50,61 @@ struct TeamGeometry
     uint32_t max_polls;
 };
 
-__global__ __launch_bounds__(kBlockSize) void bn_team_clear_kernel(unsigned long long* slots, uint32_t count)
+__device__ __forceinline__ unsigned long long team_load(const unsigned long long* p)
 {
-    const uint32_t i = blockIdx.x * kBlockSize + threadIdx.x;
-    if (i < count)
-        __hip_atomic_store(slots + i, kNoSum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void team_store(unsigned long long* p, uint32_t tag, uint32_t half)
+{
+    __hip_atomic_store(p, static_cast<unsigned long long>(tag) << 32 | half, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // The sums of all members in v[] of every thread, given this member's own in v[] of
-// thread 0.  recompute(member, sums) is called by the whole workgroup.
+// thread 0 and the tag it made of the counter.  recompute(member, sums) is called by the
+// whole workgroup.
 template <int TEAM, int N, typename G, typename F>
-__device__ __forceinline__ void team_exchange(double (&v)[N], const TeamGeometry<G>& g, uint32_t c, uint32_t member,
-                                              unsigned long long* slots, double* lds, uint32_t* missing,
-                                              const F& recompute)
+__device__ __forceinline__ void team_exchange(double (&v)[N], const TeamGeometry<G>& g, uint32_t member,
+                                              unsigned long long* state, uint32_t tag, double* lds,
+                                              uint32_t* missing, const F& recompute)
 {
     const uint32_t members = g.members.divisor, t = threadIdx.x;
-    unsigned long long* const team = slots + static_cast<size_t>(c) * members * N;
+    unsigned long long* const sums = state + kCounterWords;
     if (t == 0)
     {
 #pragma unroll
         for (int k = 0; k < N; ++k)
         {
-            unsigned long long bits = __double_as_longlong(v[k]);
-            if (v[k] != v[k])
-                bits = 0x7ff8000000000000ull; // any NaN but kNoSum
-            __hip_atomic_store(team + member * N + k, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned long long bits = __double_as_longlong(v[k]);
+            team_store(sums + 2 * k * members + member, tag, static_cast<uint32_t>(bits));
+            team_store(sums + (2 * k + 1) * members + member, tag, static_cast<uint32_t>(bits >> 32));
         }
         missing[kMaxMembers] = 0;
+        missing[kMaxMembers + 1] = tag;
     }
     __syncthreads();
+    tag = missing[kMaxMembers + 1];
     double s[N];
 #pragma unroll
     for (int k = 0; k < N; ++k)
         s[k] = 0.0;
     if (t < members)
     {
+        const unsigned long long* const mine = sums + t; // the members' words side by side: a look reads few lines
         bool there = false;
         for (uint32_t poll = 0; poll < g.max_polls && !there; ++poll)
         {
             if (poll > 0)
                 __builtin_amdgcn_s_sleep(4);
+            if (team_load(mine + (2 * N - 1) * members) >> 32 != tag) // the word stored last
+                continue;
             there = true;
 #pragma unroll
             for (int k = 0; k < N; ++k)
             {
-                const unsigned long long bits =
-                    __hip_atomic_load(team + t * N + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                s[k] = __longlong_as_double(bits);
-                there = there && bits != kNoSum;
+                const unsigned long long lo = team_load(mine + 2 * k * members),
+                                         hi = team_load(mine + (2 * k + 1) * members);
+                s[k] = __longlong_as_double(hi << 32 | (lo & 0xffffffffull));
+                there = there && lo >> 32 == tag && hi >> 32 == tag;
             }
         }
         missing[t] = !there;
@@ -92,6 +112,8 @@ __device__ __forceinline__ void team_exchange(double (&v)[N], const TeamGeometry
             missing[kMaxMembers] = 1; // every writer stores the same
     }
     __syncthreads();
+    if (t == 0)
+        __hip_atomic_fetch_add(state, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (missing[kMaxMembers])
         for (uint32_t m = 0; m < members; ++m)
             if (missing[m]) // uniform
@@ -145,15 +167,17 @@ __device__ __forceinline__ void add_backward_terms(double (&s)[4], const T (&x)[
 
 template <typename T, int TEAM, int K, bool STREAM, typename G>
 __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometry<G> g, const OnceForward<T> a,
-                                                                      unsigned long long* slots)
+                                                                      unsigned long long* states)
 {
     constexpr int VEC = 16 / sizeof(T);
     constexpr int kWaves = TEAM / kWaveSize;
     __shared__ double lds[3][2 * kWaves];
-    __shared__ uint32_t missing[kMaxMembers + 1];
+    __shared__ uint32_t missing[kMaxMembers + 2];
     const uint32_t c = fastdiv(blockIdx.x, g.members);
     const uint32_t member = blockIdx.x - c * g.members.divisor;
     const T* const x = a.x + c * g.once.stride_c;
+    unsigned long long* const state = states + static_cast<size_t>(c) * kStateWords;
+    const uint32_t tag = threadIdx.x == 0 ? static_cast<uint32_t>(team_load(state)) + 1 : 0;
     const uint32_t first = member * g.span;
     const uint32_t end = first + g.span < g.once.vectors ? first + g.span : g.once.vectors;
     T v[K][VEC];
@@ -172,7 +196,7 @@ __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometr
         if (live(u))
             add_forward_terms<G, T, VEC>(s, v[u], at[u]);
     team_sum<TEAM>(s, lds[0]);
-    team_exchange<TEAM, 2>(s, g, c, member, slots, lds[1], missing, [&](uint32_t other, double (&r)[2]) {
+    team_exchange<TEAM, 2>(s, g, member, state, tag, lds[1], missing, [&](uint32_t other, double (&r)[2]) {
         r[0] = r[1] = 0.0;
         const uint32_t stop = (other + 1) * g.span < g.once.vectors ? (other + 1) * g.span : g.once.vectors;
         for (uint32_t i = other * g.span + threadIdx.x; i < stop; i += TEAM)
@@ -210,15 +234,17 @@ __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometr
 
 template <typename T, int TEAM, int K, bool STREAM, typename G>
 __global__ __launch_bounds__(TEAM) void bn_team_backward_kernel(const TeamGeometry<G> g, const OnceBackward<T> a,
-                                                                       unsigned long long* slots)
+                                                                       unsigned long long* states)
 {
     constexpr int VEC = 16 / sizeof(T);
     constexpr int kWaves = TEAM / kWaveSize;
     __shared__ double lds[3][4 * kWaves];
-    __shared__ uint32_t missing[kMaxMembers + 1];
+    __shared__ uint32_t missing[kMaxMembers + 2];
     const uint32_t c = fastdiv(blockIdx.x, g.members);
     const uint32_t member = blockIdx.x - c * g.members.divisor;
     const int64_t base = c * g.once.stride_c;
+    unsigned long long* const state = states + static_cast<size_t>(c) * kStateWords;
+    const uint32_t tag = threadIdx.x == 0 ? static_cast<uint32_t>(team_load(state)) + 1 : 0;
     const uint32_t first = member * g.span;
     const uint32_t end = first + g.span < g.once.vectors ? first + g.span : g.once.vectors;
     T xv[K][VEC], dv[K][VEC];
@@ -242,7 +268,7 @@ __global__ __launch_bounds__(TEAM) void bn_team_backward_kernel(const TeamGeomet
         if (live(u))
             add_backward_terms<G, T, VEC>(s, xv[u], dv[u], at[u], m, sc, inv_stdev);
     team_sum<TEAM>(s, lds[0]);
-    team_exchange<TEAM, 4>(s, g, c, member, slots, lds[1], missing, [&](uint32_t other, double (&r)[4]) {
+    team_exchange<TEAM, 4>(s, g, member, state, tag, lds[1], missing, [&](uint32_t other, double (&r)[4]) {
         r[0] = r[1] = r[2] = r[3] = 0.0;
         const uint32_t stop = (other + 1) * g.span < g.once.vectors ? (other + 1) * g.span : g.once.vectors;
         for (uint32_t i = other * g.span + threadIdx.x; i < stop; i += TEAM)

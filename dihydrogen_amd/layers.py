@@ -116,6 +116,8 @@ class BatchNormalization:
         self._calls = capi.calls()
         self._workspace: Optional[torch.Tensor] = None
         self._workspace_channels = -1
+        self._state: Optional[torch.Tensor] = None
+        self._state_channels = -1
 
     # batchnorm.hpp:467-475
     def set_num_samples(self, n: int) -> None:
@@ -127,6 +129,16 @@ class BatchNormalization:
             self._workspace = _device_buffer(nbytes, torch.uint8)
             self._workspace_channels = num_channels
         return self._workspace
+
+    def _team_state(self, l: Layout, segment: int) -> Optional[torch.Tensor]:
+        """Where the workgroups that share a channel exchange its sums; smaller channels than 32 K
+        elements need none."""
+        if l.samples * segment <= 32768 or l.dtype != capi.F32:
+            return None
+        if self._state is None or self._state_channels < l.channels:
+            self._state = _device_buffer(self._lib.h2x_bn_team_state_bytes(l.channels), torch.uint8, zero=True)
+            self._state_channels = l.channels
+        return self._state
 
     def _num_per_sum(self, t: Tensor) -> int:
         """Elements per channel of the global (global_stats) or local shape
@@ -210,7 +222,7 @@ class BatchNormalization:
                 status = self._calls.h2x_bn_forward_clearing(
                     lx.dtype, lx.haloed_geometry_address, input.get_buffer(), scale, bias, self._elements_per_sum(lx),
                     self.decay, self.epsilon, mean, var, running_mean, running_var, output.get_buffer(),
-                    self._ws(lx.channels), _stream_handle(self.stream))
+                    self._team_state(lx, lx.spatial_real), _stream_handle(self.stream))
                 if status != capi.ERR_UNSUPPORTED:
                     self.num_current_samples = lx.samples
                     capi.check(status, "bn forward (clearing)")
@@ -222,7 +234,7 @@ class BatchNormalization:
             status = self._calls.h2x_bn_forward_once(
                 lx.dtype, ns, lx.geometry_address, _tensor_geometry(ly, ns), input.get_base_ptr(), scale, bias, per_sum,
                 self.decay, self.epsilon, mean, var, running_mean, running_var, output.get_base_ptr(),
-                self._ws(lx.channels), _stream_handle(self.stream))
+                self._ws(lx.channels), self._team_state(lx, lx.spatial), _stream_handle(self.stream))
             if status:
                 capi.check(status, "bn forward (local)")
             return 0
@@ -291,7 +303,7 @@ class BatchNormalization:
                 status = self._calls.h2x_bn_backward_clearing(
                     lx.dtype, self._elements_per_sum(lx), lx.haloed_geometry_address, input.get_buffer(),
                     d_output.get_buffer(), mean, var, scale, scale_gradient, bias_gradient, mean_gradient,
-                    var_gradient, d_input.get_buffer(), self.epsilon, self._ws(lx.channels),
+                    var_gradient, d_input.get_buffer(), self.epsilon, self._team_state(lx, lx.spatial_real),
                     _stream_handle(self.stream))
                 if status != capi.ERR_UNSUPPORTED:
                     self.num_current_samples = lx.samples
@@ -305,7 +317,7 @@ class BatchNormalization:
                 lx.dtype, ns, per_sum, lx.geometry_address, _tensor_geometry(ld, ns), _tensor_geometry(li, ns),
                 input.get_base_ptr(), d_output.get_base_ptr(), mean, var, scale, scale_gradient, bias_gradient,
                 mean_gradient, var_gradient, d_input.get_base_ptr(), self.epsilon, self._ws(lx.channels),
-                _stream_handle(self.stream))
+                self._team_state(lx, lx.spatial), _stream_handle(self.stream))
             if status:
                 capi.check(status, "bn backward (local)")
             return 0

@@ -428,7 +428,12 @@ int h2x_bn_backward_local_strided(h2x_dtype dtype,
  * backward, outputs that do not overlap inputs); otherwise what
  * h2x_bn_forward_local_strided and h2x_bn_backward_local_strided do.  The terms of
  * the sums are the same and are added in fp64, in another order.
+ *
+ * team_state: h2x_bn_team_state_bytes() of the number of channels, or more, zeroed
+ * once before the first call and then left to these calls, one after another, in any
+ * order and of any sizes; null: no teams.
  */
+size_t h2x_bn_team_state_bytes(int num_channels);
 int h2x_bn_forward_once(h2x_dtype dtype,
                                  int num_samples,
                                  const h2x_tensor_geometry* x_geometry,
@@ -445,6 +450,7 @@ int h2x_bn_forward_once(h2x_dtype dtype,
                                  void* running_var,
                                  void* y,
                                  void* workspace,
+                                 void* team_state,
                                  h2x_stream_t stream);
 int h2x_bn_backward_once(h2x_dtype dtype,
                                   int num_samples,
@@ -464,6 +470,7 @@ int h2x_bn_backward_once(h2x_dtype dtype,
                                   void* dx,
                                   double epsilon,
                                   void* workspace,
+                                  void* team_state,
                                   h2x_stream_t stream);
 
 /**
@@ -487,7 +494,7 @@ int h2x_bn_forward_team(h2x_dtype dtype,
                         void* running_mean,
                         void* running_var,
                         void* y,
-                        void* workspace,
+                        void* team_state,
                         unsigned int max_polls,
                         h2x_stream_t stream);
 int h2x_bn_backward_team(h2x_dtype dtype,
@@ -507,7 +514,7 @@ int h2x_bn_backward_team(h2x_dtype dtype,
                          void* dvar,
                          void* dx,
                          double epsilon,
-                         void* workspace,
+                         void* team_state,
                          unsigned int max_polls,
                          h2x_stream_t stream);
 
@@ -602,7 +609,7 @@ int h2x_bn_forward_clearing(h2x_dtype dtype,
                             void* running_mean,
                             void* running_var,
                             void* y_buffer,
-                            void* workspace,
+                            void* team_state,
                             h2x_stream_t stream);
 int h2x_bn_backward_clearing(h2x_dtype dtype,
                              size_t num_per_sum,
@@ -618,7 +625,7 @@ int h2x_bn_backward_clearing(h2x_dtype dtype,
                              void* dvar,
                              void* dx_buffer,
                              double epsilon,
-                             void* workspace,
+                             void* team_state,
                              h2x_stream_t stream);
 
 /**

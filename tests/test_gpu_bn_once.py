@@ -31,6 +31,7 @@ class _Problem:
         self.scale = torch.empty(c, device="cuda").uniform_(0.5, 1.5, generator=g)
         self.bias = torch.empty(c, device="cuda").normal_(0, 0.1, generator=g)
         self.ws = torch.empty(capi.load().h2x_bn_workspace_bytes(c), dtype=torch.uint8, device="cuda")
+        self.state = torch.zeros(capi.load().h2x_bn_team_state_bytes(c), dtype=torch.uint8, device="cuda")
 
     def run(self, kind, *polls, in_place=False):
         """(outputs, halo untouched?) of h2x_bn_{forward,backward}_<kind>."""
@@ -44,16 +45,17 @@ class _Problem:
         at = lambda t: t.data_ptr() + self.offset
         p = lambda t: t.data_ptr()
         st = torch.cuda.current_stream().cuda_stream
+        scratch = {"once": [p(self.ws), p(self.state)], "team": [p(self.state)]}.get(kind, [p(self.ws)])
         status = getattr(lib, "h2x_bn_forward_" + kind)(
             capi.F32, self.n, gp, gp, at(x), p(self.scale), p(self.bias), self.per, 0.9, 1e-5, p(mean), p(var), p(rm),
-            p(rv), at(y), p(self.ws), *polls, st)
+            p(rv), at(y), *scratch, *polls, st)
         assert status == 0, status
         if in_place:
             x = self.x.clone()
         dx = x if in_place else torch.full_like(x, 7)
         status = getattr(lib, "h2x_bn_backward_" + kind)(
             capi.F32, self.n, self.per, gp, gp, gp, at(x), at(self.dy), p(mean), p(var), p(self.scale),
-            *[p(t) for t in grads], at(dx), 1e-5, p(self.ws), *polls, st)
+            *[p(t) for t in grads], at(dx), 1e-5, *scratch, *polls, st)
         assert status == 0, status
         torch.cuda.synchronize()
         for out in (y, dx):
@@ -107,10 +109,22 @@ def test_channel_in_a_team(shape):
     by_team = p.run("team", 2048)
     _close(by_team, p.run("local_strided"))
     small = p.x.numel() < 4_000_000  # every member reads its whole channel
-    if small:
-        for a, b in zip(by_team, p.run("team", 0)):
+    for polls in ([0, 2048] if small else [2048, 2048]):  # and again with the state that these calls leave
+        for a, b in zip(by_team, p.run("team", polls)):
             assert torch.equal(a, b)
     _close(p.run("once"), by_team)
+
+
+def test_one_state_for_calls_of_other_sizes():
+    """Teams of other sizes, forward and backward, leave sums of earlier calls in the state: none is taken for a new one."""
+    import torch
+    problems = [_Problem(*s) for s in [(2, 3, 40, 32, 32), (7, 3, 40, 32, 32), (1, 3, 1, 64, 300), (3, 2, 17, 18, 19, 2)]]
+    wants = [p.run("team", 2048) for p in problems]
+    state = problems[0].state
+    for i in (0, 1, 2, 1, 3, 0, 2, 3, 1):
+        problems[i].state = state
+        for a, b in zip(problems[i].run("team", 2048), wants[i]):
+            assert torch.equal(a, b)
 
 
 def test_nan_reaches_the_whole_channel_of_a_team_only():
@@ -127,7 +141,7 @@ def test_overlapping_outputs_are_not_for_teams():
     x, lib, gp = p.x.data_ptr(), capi.load(), ctypes.byref(p.geometry)
     v = [p.scale.clone().data_ptr() for _ in range(4)]
     assert lib.h2x_bn_forward_team(capi.F32, 2, gp, gp, x, p.scale.data_ptr(), p.bias.data_ptr(), p.per, 0.9, 1e-5, *v, x,
-                                   p.ws.data_ptr(), 2048, None) == -2  # unsupported
+                                   p.state.data_ptr(), 2048, None) == -2  # unsupported
     _close(p.run("once", in_place=True), p.run("local_strided"))
 
 
@@ -156,14 +170,14 @@ def test_whole_pass_that_clears_the_halo(shape, halo, in_place):
     a = lambda t: t.data_ptr()
     y = x.clone() if in_place else torch.full_like(x, 7)
     status = lib.h2x_bn_forward_clearing(capi.F32, gp, a(y if in_place else x), a(p.scale), a(p.bias), p.per, 0.9, 1e-5, a(mean),
-                                         a(var), a(rm), a(rv), a(y), a(p.ws), None)
+                                         a(var), a(rm), a(rv), a(y), a(p.state), None)
     if status == -2:
         assert in_place and p.x[0, 0].numel() * n > 32768
         return
     assert status == 0
     dx = x.clone() if in_place else torch.full_like(x, 7)
     assert lib.h2x_bn_backward_clearing(capi.F32, p.per, gp, a(dx if in_place else x), a(dy), a(mean), a(var), a(p.scale),
-                                        *[a(t) for t in grads], a(dx), 1e-5, a(p.ws), None) == 0
+                                        *[a(t) for t in grads], a(dx), 1e-5, a(p.state), None) == 0
     torch.cuda.synchronize()
     for out in (y, dx):
         rest = out.clone()
