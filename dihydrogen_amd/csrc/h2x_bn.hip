@@ -38,6 +38,7 @@
 #include "h2x_device.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <type_traits>
 
@@ -2737,60 +2738,85 @@ bool team_launch(const G& once, const A<T>& a, bool stream, uint32_t least, uint
 // Looks of about a microsecond: a team that other streams keep off the chip for longer
 // works its sums out (2 ms against the tens of microseconds of a launch).
 constexpr uint32_t kTeamPolls = 2048;
-// Fewer workgroups leave the chip to the two-launch kernels, which cut a channel finer
-// (N 4, C 16, 40^3 in 256 workgroups 9.9 + 13.0 us, in two launches 10.3 + 16.3; half of
-// that, C 8, in 256 smaller ones 8.8 + 10.4 and 7.8 + 10.9).
-constexpr uint32_t kTeamLeastBlocks = 192;
-// Forward a member holds 128 KB, in smaller pieces where that is not enough workgroups
-// (N 2, C 32, 48^3: 12.0 us, whole ones 13.0); up to 128 members (N 16, C 16, 64^3 in 128
-// of them 98 us, in two launches 118).
+// Workgroups from which a size of member is taken: smaller members where larger ones would be
+// fewer.  Below the last, channels are few and the two-launch kernels cut them finer (N 2, C 4, 40^3).
+constexpr uint32_t kLargeMembers = 384, kMediumMembers = 256, kSmallMembers = 128;
+
+// Forward a member holds 128, 64 or 32 KB (N 16, C 64, 112 x 112 in 448 workgroups of 128 KB 20.4 us, in
+// 832 of 64 KB 22.5; N 2, C 32, 48^3 in 448 of 64 KB 12.0, in 224 of 128 KB 13.0; N 2, C 32, 28^3 with a halo
+// in 224 of 32 KB 6.8 us, in two launches 9.8); up to 128 members (N 16, C 16, 64^3 in 128 of them 98 us, in
+// two launches 118).  `forced`: however few workgroups that is.
 template <typename G, typename T>
-bool team_variant(const G& g, const OnceForward<T>& a, bool stream, uint32_t least, uint32_t most,
-                  uint32_t polls, void* team_state, hipStream_t st)
+bool team_variant(const G& g, const OnceForward<T>& a, bool stream, bool forced, uint32_t most, uint32_t polls,
+                  void* team_state, hipStream_t st)
 {
-    return team_launch<512, 16>(g, a, stream, 2 * least, most, polls, team_state, st)
-           || team_launch<512, 8>(g, a, stream, least, most, polls, team_state, st);
+    return team_launch<512, 16>(g, a, stream, forced ? 1 : kLargeMembers, most, polls, team_state, st)
+           || team_launch<512, 8>(g, a, stream, forced ? 1 : kMediumMembers, most, polls, team_state, st)
+           || team_launch<512, 4>(g, a, stream, kSmallMembers, most, polls, team_state, st);
 }
 
 // Backward 64 KB of each tensor, 128 KB where a team would have more than 64 members
 // (N 8, C 64, 64^3: 355 us, in 128 members 379, in two launches 407), and no more than 64
 // of those (N 16, C 16, 64^3: 251 us, in two launches 195): a larger team waits longer for
-// its last member than it saves.
+// its last member than it saves.  32 KB where that is not enough workgroups
+// (N 2, C 32, 28^3 with a halo 8.0 us, in two launches 12.4).
 template <typename G, typename T>
-bool team_variant(const G& g, const OnceBackward<T>& a, bool stream, uint32_t least, uint32_t most,
-                  uint32_t polls, void* team_state, hipStream_t st)
+bool team_variant(const G& g, const OnceBackward<T>& a, bool stream, bool forced, uint32_t most, uint32_t polls,
+                  void* team_state, hipStream_t st)
 {
     most /= 2;
-    return team_launch<512, 8>(g, a, stream, least, most, polls, team_state, st)
-           || team_launch<1024, 8>(g, a, stream, least, most, polls, team_state, st);
+    return team_launch<512, 8>(g, a, stream, forced ? 1 : kMediumMembers, most, polls, team_state, st)
+           || team_launch<1024, 8>(g, a, stream, forced ? 1 : kMediumMembers, most, polls, team_state, st)
+           || team_launch<512, 4>(g, a, stream, kSmallMembers, most, polls, team_state, st);
+}
+
+// Channels that one workgroup of 1024 threads would hold, but few: the teams first
+// (forward + backward, N 8, C 64, 56 x 56 13.3 us, by workgroups 15.0; N 1, C 32, 32^3 13.1 and 16.8; N 1, C 96,
+// 32^3 15.3 and 17.5; but N 8, C 128, 56 x 56 16.6 and 15.6; half the size, N 4, C 64, 56 x 56, 13.0 and 11.0).
+template <typename G>
+bool teams_first(const G& g)
+{
+    return g.vectors > 4096 && g.num_channels <= kOnceManyChannels;
+}
+
+// CUs of the current device (0: there is none), asked for once: a device does not change, and
+// the question costs a small call most of a microsecond.
+uint32_t compute_units()
+{
+    static std::atomic<int> known[kMaxDevices];
+    int device = 0, cus = 0;
+    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMaxDevices)
+        return 0;
+    cus = known[device].load(std::memory_order_relaxed);
+    if (cus == 0
+        && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess)
+        known[device].store(cus, std::memory_order_relaxed);
+    return static_cast<uint32_t>(cus);
 }
 
 // False: the call is not for teams.  bytes: from the first to behind the last element of a tensor.
 template <typename G, typename A>
 bool launch_by_teams(const G& g, const A& a, size_t bytes, bool stream, std::initializer_list<const void*> inputs,
-                     const void* output, uint32_t least, uint32_t polls, void* team_state, hipStream_t st)
+                     const void* output, bool forced, uint32_t polls, void* team_state, hipStream_t st)
 {
     if (!team_state)
         return false;
     for (const void* p : inputs)
         if (!apart(p, output, bytes))
             return false;
-    int device = 0, cus = 0;
-    if (hipGetDevice(&device) != hipSuccess
-        || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
-        return false;
-    return team_variant(g, a, stream, least, std::min<uint32_t>(cus / 2, kMaxMembers), polls, team_state, st);
+    const uint32_t cus = compute_units();
+    return team_variant(g, a, stream, forced, std::min(cus / 2, kMaxMembers), polls, team_state, st);
 }
 
 template <typename A>
 bool launch_by_teams(const OnceGeometry& g, const A& a, int n, std::initializer_list<const void*> inputs,
-                     const void* output, uint32_t least, uint32_t polls, void* team_state, hipStream_t st)
+                     const void* output, bool forced, uint32_t polls, void* team_state, hipStream_t st)
 {
     // short segments have kernels of their own (N 2048, C 256, 7 x 7: 141 us, by teams 172)
     const bool stream = streamed(g, n);
     if (dense_rows(g) && !stream)
         return false;
-    return launch_by_teams(g, a, reach_bytes(g, n), stream, inputs, output, least, polls, team_state, st);
+    return launch_by_teams(g, a, reach_bytes(g, n), stream, inputs, output, forced, polls, team_state, st);
 }
 
 // team_polls: by teams or not at all, however few workgroups that is, with this many looks.
@@ -2816,10 +2842,11 @@ int forward_once(int n, const h2x_tensor_geometry* gx, const h2x_tensor_geometry
                                    static_cast<T*>(running_var), static_cast<T*>(y), static_cast<T>(num_per_sum),
                                    static_cast<T>(decay), static_cast<T>(eps)};
             if (team_polls)
-                return launch_by_teams(g, a, n, {x}, y, 1, *team_polls, team_state, st) ? launch_status()
+                return launch_by_teams(g, a, n, {x}, y, true, *team_polls, team_state, st) ? launch_status()
                                                                             : H2X_ERR_UNSUPPORTED;
-            if (once_launch(g, a, n, st)
-                || launch_by_teams(g, a, n, {x}, y, kTeamLeastBlocks, kTeamPolls, team_state, st))
+            const auto by_teams = [&] { return launch_by_teams(g, a, n, {x}, y, false, kTeamPolls, team_state, st); };
+            const bool teams = teams_first(g);
+            if ((teams && by_teams()) || once_launch(g, a, n, st) || (!teams && by_teams()))
                 return launch_status();
         }
     }
@@ -2853,10 +2880,11 @@ int backward_once(int n, size_t num_per_sum, const h2x_tensor_geometry* gx, cons
                                     static_cast<T*>(dx), static_cast<T>(num_per_sum),
                                     static_cast<T>(num_per_sum - 1), static_cast<T>(eps)};
             if (team_polls)
-                return launch_by_teams(g, a, n, {x, dy}, dx, 1, *team_polls, team_state, st) ? launch_status()
+                return launch_by_teams(g, a, n, {x, dy}, dx, true, *team_polls, team_state, st) ? launch_status()
                                                                             : H2X_ERR_UNSUPPORTED;
-            if (once_launch(g, a, n, st)
-                || launch_by_teams(g, a, n, {x, dy}, dx, kTeamLeastBlocks, kTeamPolls, team_state, st))
+            const auto by_teams = [&] { return launch_by_teams(g, a, n, {x, dy}, dx, false, kTeamPolls, team_state, st); };
+            const bool teams = teams_first(g);
+            if ((teams && by_teams()) || once_launch(g, a, n, st) || (!teams && by_teams()))
                 return launch_status();
         }
     }
@@ -2893,9 +2921,12 @@ int clearing_once(const h2x_haloed_geometry* h, const A& a, std::initializer_lis
     g.stride_n = static_cast<uint32_t>(c * real);
     g.stride_c = static_cast<int64_t>(real);
     g.num_channels = static_cast<uint32_t>(c);
-    if (once_launch<true>(g, a, st)
-        || launch_by_teams(g, a, n * c * real * sizeof(float), true, inputs, output, kTeamLeastBlocks, kTeamPolls,
-                           team_state, st))
+    const auto by_teams = [&] {
+        return launch_by_teams(g, a, n * c * real * sizeof(float), true, inputs, output, false, kTeamPolls, team_state,
+                               st);
+    };
+    const bool teams = teams_first(g);
+    if ((teams && by_teams()) || once_launch<true>(g, a, st) || (!teams && by_teams()))
         return launch_status();
     return H2X_ERR_UNSUPPORTED;
 }

@@ -131,9 +131,9 @@ class BatchNormalization:
         return self._workspace
 
     def _team_state(self, l: Layout, segment: int) -> Optional[torch.Tensor]:
-        """Where the workgroups that share a channel exchange its sums; smaller channels than 32 K
+        """Where the workgroups that share a channel exchange its sums; smaller channels than 16 K
         elements need none."""
-        if l.samples * segment <= 32768 or l.dtype != capi.F32:
+        if l.samples * segment <= 16384 or l.dtype != capi.F32:
             return None
         if self._state is None or self._state_channels < l.channels:
             self._state = _device_buffer(self._lib.h2x_bn_team_state_bytes(l.channels), torch.uint8, zero=True)

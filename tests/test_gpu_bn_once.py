@@ -77,7 +77,7 @@ def _close(got, want):
 # vectors a channel of the variants' edges; 96 channels reach the largest ones
 ONCE = [(1, 5, 1, 16, 32), (1, 5, 1, 3, 172), (2, 3, 1, 32, 64), (3, 3, 1, 37, 37), (8, 3, 1, 32, 32),
         (8, 3, 1, 32, 64), (5, 2, 1, 59, 111), (4, 97, 1, 128, 128), (4, 96, 1, 128, 129), (5, 96, 1, 128, 128),
-        (40, 1030, 1, 7, 7), (3, 7, 1, 2, 2)]
+        (40, 1030, 1, 7, 7), (3, 7, 1, 2, 2), (4, 96, 1, 64, 65), (4, 65, 1, 64, 64), (9, 43, 1, 43, 44)]
 
 
 @pytest.mark.parametrize("in_place", [False, True])
