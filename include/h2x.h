@@ -424,8 +424,8 @@ int h2x_bn_backward_local_strided(h2x_dtype dtype,
  * The same again for float tensors that lie alike, reading every element once where
  * a channel is held in registers between the sums and the output: by one workgroup
  * (up to about 80000 elements a channel forward and 65000 backward) or by a team of
- * workgroups (larger channels, up to about 4 million elements forward and 2 million
- * backward, outputs that do not overlap inputs); otherwise what
+ * workgroups (larger channels, or few, up to about 4 million elements forward and 2
+ * million backward, outputs that do not overlap inputs); otherwise what
  * h2x_bn_forward_local_strided and h2x_bn_backward_local_strided do.  The terms of
  * the sums are the same and are added in fp64, in another order.
  *
