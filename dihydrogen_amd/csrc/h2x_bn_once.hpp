@@ -11,9 +11,8 @@
 //   N 16, C 512, 7^3, halo of 1    54.9 -> 20.3         N 8, C 1024, 7 x 7     17.2 -> 9.5
 //
 // A channel is as large as the registers of one CU allow: 512 KB, of which the
-// largest variants hold 320 KB forward, 256 KB and 128 KB of LDS backward.  (One
-// workgroup per channel because teams of several workgroups would have to wait for
-// one another across XCDs.)
+// largest variants hold 320 KB forward, 256 KB and 128 KB of LDS backward.  Larger ones, and few, are for
+// teams of workgroups (h2x_bn_team.hpp).
 //
 // The elements are those of the other kernels: rows in vectors of 16 bytes that may
 // start on any element, the last vector of a row that is no whole number of vectors
