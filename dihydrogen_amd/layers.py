@@ -22,6 +22,14 @@ def _device_buffer(count: int, dtype, device="cuda", zero: bool = False) -> torc
     return (torch.zeros if zero else torch.empty)(count, dtype=dtype, device=device)
 
 
+def _buffer_of(stream: Optional[torch.cuda.Stream], *args, **kwargs) -> torch.Tensor:
+    """A _device_buffer for launches on `stream` (None: on the current one).  It is made on that
+    stream: what clears it comes before the launches that use it, and whoever gets its memory when
+    the layer gives it back comes after them.  On another stream neither would be ordered."""
+    with torch.cuda.stream(stream):
+        return _device_buffer(*args, **kwargs)
+
+
 def _share_a_gpu(tensors: Sequence[Tensor]) -> bool:
     """All tensors are allocated, on one GPU: what belongs to another rank can be read and written
     where it lies.  (On the host, where launches can only be audited, strips are packed as they
@@ -126,7 +134,7 @@ class BatchNormalization:
     def _ws(self, num_channels: int) -> torch.Tensor:
         if self._workspace is None or self._workspace_channels != num_channels:
             nbytes = self._lib.h2x_bn_workspace_bytes(num_channels)
-            self._workspace = _device_buffer(nbytes, torch.uint8)
+            self._workspace = _buffer_of(self.stream, nbytes, torch.uint8)
             self._workspace_channels = num_channels
         return self._workspace
 
@@ -136,7 +144,8 @@ class BatchNormalization:
         if l.samples * segment <= 16384 or l.dtype != capi.F32:
             return None
         if self._state is None or self._state_channels < l.channels:
-            self._state = _device_buffer(self._lib.h2x_bn_team_state_bytes(l.channels), torch.uint8, zero=True)
+            nbytes = self._lib.h2x_bn_team_state_bytes(l.channels)
+            self._state = _buffer_of(self.stream, nbytes, torch.uint8, zero=True)
             self._state_channels = l.channels
         return self._state
 
@@ -377,7 +386,7 @@ def reduce_sum(src: Tensor, dst: Tensor, square: bool = False, region: Optional[
     key = _stream_handle(stream)
     ws = _reduce_workspaces.get(key)
     if ws is None or ws.numel() < need:
-        ws = _reduce_workspaces[key] = _device_buffer(max(need, 256), torch.uint8)
+        ws = _reduce_workspaces[key] = _buffer_of(stream, max(need, 256), torch.uint8)
     capi.check(capi.calls().h2x_tensor_reduce_sum(src.h2x_dtype, ctypes.addressof(gs), src.get_base_ptr(),
                                                   ctypes.addressof(gd), dst.get_base_ptr(), int(square), ws, key),
                "tensor reduce_sum")
@@ -419,14 +428,14 @@ class Softmax:
     def _workspace(self, n: int) -> torch.Tensor:
         need = self._lib.h2x_softmax_instance_workspace_bytes(n)
         if self._ws is None or self._ws.numel() < need:
-            self._ws = _device_buffer(need, torch.uint8)
+            self._ws = _buffer_of(self.stream, need, torch.uint8)
         return self._ws
 
     def _sample_scalars(self, t: Tensor, count: int) -> torch.Tensor:
         """`count` scalars of t's type that nobody reads after the call: kept like the workspace."""
         b = self._scalars
         if b is None or b.dtype != t.dtype or b.numel() < count:
-            b = self._scalars = _device_buffer(count, t.dtype)
+            b = self._scalars = _buffer_of(self.stream, count, t.dtype)
         return b
 
     def forward(self, x: Tensor, y: Tensor) -> int:
@@ -452,8 +461,7 @@ class Softmax:
             if status:
                 capi.check(status, "softmax instance forward")
             return 0
-        smax = torch.empty(n, dtype=x.dtype, device=x.device)
-        sexp = torch.empty(n, dtype=x.dtype, device=x.device)
+        smax, sexp = (_buffer_of(self.stream, n, x.dtype, x.device) for _ in range(2))
         capi.check(calls.h2x_softmax_instance_max(dt, n, size, x.get_base_ptr(), smax, ws, st),
                    "softmax instance max")
         self.allreduce(smax, True)
@@ -484,7 +492,7 @@ class Softmax:
             if status:
                 capi.check(status, "softmax instance backward")
             return 0
-        sdp = torch.empty(n, dtype=y.dtype, device=y.device)
+        sdp = _buffer_of(self.stream, n, y.dtype, y.device)
         capi.check(calls.h2x_softmax_instance_dot(dt, n, size, y.get_base_ptr(), dy.get_base_ptr(), sdp, ws, st),
                    "softmax instance dot")
         self.allreduce(sdp, False)
@@ -586,14 +594,19 @@ class HaloExchangeVirtual:
         """The buffer rank `rank` unpacks its (dim, side) halo from -- and its
         neighbour on that side packs into (get_recv_buffer, halo_exchange_cuda.hpp:277-283)."""
         self._buffers_wanted = True
-        return self._receive_buffer(rank, dim, side)
+        made = (rank, dim, side) not in self._recv
+        buffer = self._receive_buffer(rank, dim, side)
+        if made and self.stream is not None and buffer.is_cuda:
+            # what the caller does with it on the current stream comes after it was cleared
+            torch.cuda.current_stream().wait_stream(self.stream)
+        return buffer
 
     def _receive_buffer(self, rank: int, dim: int, side: int) -> torch.Tensor:
         key = (rank, dim, side)
         if key not in self._recv:
             t = self.tensors[rank]
             n = self.get_halo_size(rank, dim, t.overlap[dim])  # sized for the full halo (:285-303)
-            self._recv[key] = _device_buffer(max(n, 1), t.dtype, t.device, zero=True)
+            self._recv[key] = _buffer_of(self.stream, max(n, 1), t.dtype, t.device, zero=True)
         return self._recv[key]
 
     def make_face(self, rank, dim, side, width, buf, is_pack, is_reverse, op) -> capi.HaloFace:
@@ -1004,7 +1017,7 @@ class TensorShufflerVirtual:
         recv_displs = [[sum(recv_counts[r][:p]) for p in range(n)] for r in range(n)]
         recv_sizes = [sum(recv_counts[r]) for r in range(n)]
         arena_offsets = [sum(recv_sizes[:r]) for r in range(n)]
-        arena = _device_buffer(max(sum(recv_sizes), 1), src[0].dtype, src[0].device, zero=True)
+        arena = _buffer_of(self.stream, max(sum(recv_sizes), 1), src[0].dtype, src[0].device, zero=True)
         if sum(recv_sizes) >= 2 ** 31:
             raise ValueError("arena exceeds the 32-bit displacements of the shuffler tables")
         pack_plans, unpack_plans = [], []

@@ -1,0 +1,47 @@
+"""A batch-norm layer that launches on its own stream while another stream, the current one, is busy: the state
+through which the workgroups of a channel exchange their sums is cleared before they use it."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("halo", [0, 1])
+def test_layer_on_its_own_stream_while_the_current_one_is_busy(halo):
+    import torch
+    from dihydrogen_amd.layers import BatchNormalization
+    from dihydrogen_amd.tensor import Distribution, LocaleVirtual, Tensor
+    dist = (Distribution.make_overlapped_distribution([2, 2, 2, 1, 1], [1, 1, 1, 0, 0]) if halo
+            else Distribution.make_localized_distribution(5))
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x, dy = (Tensor([48, 44, 40, 32, 2], LocaleVirtual(0, dist.num_ranks), dist).allocate() for _ in range(2))
+    for t in (x, dy):
+        t.data.normal_(0.5, 1, generator=g)
+    scale, bias = torch.full((32,), 1.25, device="cuda"), torch.full((32,), -0.5, device="cuda")
+
+    def outputs():
+        y, dx = (Tensor([48, 44, 40, 32, 2], LocaleVirtual(0, dist.num_ranks), dist).allocate() for _ in range(2))
+        return y, dx, [torch.full((32,), v, device="cuda") for v in (0, 0, 0, 1, 0, 0, 0, 0)]
+
+    def run(layer, y, dx, v):
+        layer.forward(x, *v[:4], scale, bias, y, True)
+        layer.backward(x, dy, *v[:2], scale, *v[4:], dx)
+
+    side = torch.cuda.Stream()
+    calls = 3
+    want, got = ([outputs() for _ in range(calls)] for _ in range(2))
+    layer = BatchNormalization(5, 0.9, 1e-5, clear_output_halo=bool(halo))
+    for out in want:
+        run(layer, *out)
+    busy = torch.empty(1 << 26, device="cuda")
+    torch.cuda.synchronize()
+    for _ in range(40):     # some milliseconds on the current stream, which `side` does not wait for
+        busy.normal_()
+    layer = BatchNormalization(5, 0.9, 1e-5, stream=side, clear_output_halo=bool(halo))
+    for out in got:
+        run(layer, *out)
+    assert layer._state is not None     # this size is for several workgroups a channel
+    del layer                           # its memory goes back while its launches are still queued
+    torch.cuda.synchronize()
+    for (ya, da, va), (yb, db, vb) in zip(want, got):
+        for a, b in zip([ya.data, da.data] + va, [yb.data, db.data] + vb):
+            assert torch.equal(a, b)

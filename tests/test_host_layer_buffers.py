@@ -1,0 +1,95 @@
+"""Buffers that a layer makes for its launches belong to the stream it launches on: cleared there before the
+launch, and on loan from that stream's memory.  On the CPU, with the library's calls stubbed out: nothing is
+launched and no address is followed."""
+import contextlib
+
+import pytest
+
+from dihydrogen_amd import capi, layers
+from dihydrogen_amd.layers import BatchNormalization, HaloExchangeVirtual, Softmax, SoftmaxMode, TensorShufflerVirtual
+from dihydrogen_amd.tensor import Distribution, LocaleVirtual, Tensor
+
+
+class _Stream:
+    cuda_stream = 77
+
+
+class _Calls:
+    """Entry points that launch nothing and say so."""
+
+    def __getattr__(self, name):
+        return lambda *args: 0
+
+
+@pytest.fixture
+def made(monkeypatch):
+    """(stream that was current when it was made, cleared) of every buffer."""
+    current, made = [None], []
+
+    @contextlib.contextmanager
+    def on(stream):
+        current.append(stream if stream is not None else current[-1])
+        yield
+        current.pop()
+
+    def device_buffer(count, dtype, device="cuda", zero=False):
+        import torch
+        made.append((current[-1], zero))
+        return torch.zeros(count, dtype=dtype)
+
+    monkeypatch.setattr(layers.torch.cuda, "stream", on)
+    monkeypatch.setattr(layers, "_device_buffer", device_buffer)
+    monkeypatch.setattr(capi, "calls", _Calls)
+    monkeypatch.setattr(TensorShufflerVirtual, "_plan", lambda *args: None)  # plans are made on a device
+    return made
+
+
+def _tensors(shape, dist, count):
+    return [Tensor(shape, LocaleVirtual(r % dist.num_ranks, dist.num_ranks), dist, device="cpu").allocate()
+            for r in range(count)]
+
+
+def _batch_norm(stream):
+    x, y, dy, dx = _tensors([32, 40, 40, 3, 2], Distribution.make_localized_distribution(5), 4)
+    bn = BatchNormalization(5, 0.9, 1e-5, stream=stream)
+    bn.forward(x, *[x.data] * 6, y)
+    bn.backward(x, dy, *[x.data] * 7, dx)
+
+
+def _softmax(stream):
+    x, y, dx = _tensors([8, 4, 5, 3], Distribution.make_localized_distribution(4), 3)
+    for allreduce in (None, lambda values, is_max: None):
+        sm = Softmax(stream, allreduce)
+        sm.setup(x, SoftmaxMode.INSTANCE)
+        sm.forward(x, y)
+        sm.backward(y, y, dx)
+
+
+def _halo(stream):
+    ranks = _tensors([8, 6, 2, 1], Distribution.make_overlapped_distribution([2, 1, 1, 1], [1, 0, 0, 0]), 2)
+    xch = HaloExchangeVirtual(ranks, stream=stream)
+    xch.exchange()
+    xch.recv_buffer(0, 0, capi.RHS)
+
+
+def _shuffle(stream):
+    src, dst = _tensors([8, 6, 2, 2], Distribution([1, 1, 1, 2]), 2), _tensors([8, 6, 2, 2], Distribution([2, 1, 1, 1]), 2)
+    TensorShufflerVirtual(src, dst, stream).shuffle_forward()
+
+
+def _reduce(stream):
+    dist = Distribution.make_localized_distribution(4)
+    layers._reduce_workspaces.clear()
+    layers.reduce_sum(_tensors([8, 6, 2, 2], dist, 1)[0], _tensors([1, 1, 2, 1], dist, 1)[0], stream=stream)
+    layers._reduce_workspaces.clear()
+
+
+@pytest.mark.parametrize("use", [_batch_norm, _softmax, _halo, _shuffle, _reduce])
+def test_buffers_are_made_on_the_stream_that_is_launched_on(use, made):
+    stream = _Stream()
+    use(stream)
+    assert made and all(s is stream for s, _ in made)
+    assert any(zero for _, zero in made) == (use in (_batch_norm, _halo, _shuffle))
+    made.clear()
+    use(None)
+    assert made and all(s is None for s, _ in made)
