@@ -626,9 +626,9 @@ class HaloExchangeVirtual:
     def _grid(self, cells: int) -> int:
         """Address of the h2x_halo_grid of all ranks, or 0 where the launches that serve all of
         them cannot: tensors that do not share a GPU (the packed strips are what could travel),
-        an empty rank, a halo on channels or samples, or next to a neighbour fewer than `cells`
-        halo widths of interior (an exchange needs one: its boundary strips are no halo; a
-        reverse one two: they do not overlap)."""
+        ranks that differ in their halo widths or type, an empty rank, a halo on channels or
+        samples, or next to a neighbour fewer than `cells` halo widths of interior (an exchange
+        needs one: its boundary strips are no halo; a reverse one two: they do not overlap)."""
         addresses = self._addresses()
         kept = self._grid_of
         if kept is None or kept[0] != addresses:
@@ -637,8 +637,9 @@ class HaloExchangeVirtual:
 
     def _make_grid(self):
         """(address of the h2x_halo_grid or 0, halo widths of interior that every rank has)"""
-        ts, ov = self.tensors, self.tensors[0].overlap
-        if (len(ts) > capi.HALO_GRID_MAX_RANKS or self.nd not in (4, 5) or not any(ov) or any(ov[self.nd - 2:])
+        ts, ov, dtype = self.tensors, self.tensors[0].overlap, self.tensors[0].dtype
+        if (any(t.overlap != ov or t.dtype != dtype for t in ts) or len(ts) > capi.HALO_GRID_MAX_RANKS
+                or self.nd not in (4, 5) or not any(ov) or any(ov[self.nd - 2:])
                 or not _share_a_gpu(ts) or any(not 0 < t.get_local_size() <= t.get_local_real_size() < 2 ** 31 for t in ts)):
             return 0, -1
         ranks = (capi.HaloGridRank * len(ts))()
