@@ -51,6 +51,8 @@ constexpr int kMaxRanks = 16;
 constexpr int kMaxSpatial = 3;
 constexpr int kMaxRegions = 9 + 8;
 constexpr int kBlock = 256;
+constexpr uint64_t kMaxRankBlocks = 0x7fffff;         // indexes of one rank stay below 2^31
+constexpr uint64_t kMaxBlocks = 0xffffffffu / kBlock; // a launch counts its threads in 32 bits
 // Ranks of a line whose ends a thread loads before it stores any (measured: 1, 2, 4; two hold
 // the fewest registers at the rate of four).
 constexpr int kRanksPerTurn = 2;
@@ -570,7 +572,7 @@ int run(h2x_dtype dtype, const h2x_halo_grid* h, int only_unfilled, h2x_stream_t
                 a.first[g] = static_cast<uint32_t>(blocks);
                 a.code[g] = static_cast<uint32_t>(ends + 4 * dy + 16 * dz);
                 blocks += most * (ends ? a.lines.divisor : a.ranks.divisor);
-                if (most >= 0x7fffff || blocks > 0x7fffffffull) // indexes of one rank stay below 2^31
+                if (most > kMaxRankBlocks || blocks > kMaxBlocks)
                     return H2X_ERR_TOO_LARGE;
             }
     if (blocks == 0)
@@ -591,12 +593,13 @@ int run_fold(h2x_dtype dtype, const h2x_halo_grid* h, int op, h2x_stream_t strea
     if (err != 0)
         return err;
     const int64_t vec = 16 / es;
-    int64_t blocks[kMaxSpatial] = {};
+    uint64_t blocks[kMaxSpatial] = {};
     FastDiv units[kMaxSpatial][kMaxRanks];
     bool vectors[kMaxSpatial][kMaxRanks];
     for (int dim = 0; dim < kMaxSpatial; ++dim)
     {
         bool any = false;
+        uint64_t most = 0; // workgroups of the largest rank
         for (int r = 0; r < h->num_ranks; ++r)
         {
             const Rank& k = a.rank[r];
@@ -607,11 +610,12 @@ int run_fold(h2x_dtype dtype, const h2x_halo_grid* h, int op, h2x_stream_t strea
             vectors[dim][r] = run >= vec;
             const int64_t n = run >= vec ? (run + vec - 1) / vec : std::max<int64_t>(run, 1);
             units[dim][r] = make_fastdiv(static_cast<uint32_t>(n));
-            blocks[dim] = std::max(blocks[dim], (n * above + kBlock - 1) / kBlock * h->num_ranks);
+            most = std::max<uint64_t>(most, (n * above + kBlock - 1) / kBlock);
         }
         if (!any)
-            blocks[dim] = 0;
-        if (blocks[dim] > 0x7fffff) // the last index of a workgroup stays below 2^31
+            continue;
+        blocks[dim] = most * h->num_ranks;
+        if (most > kMaxRankBlocks || blocks[dim] > kMaxBlocks)
             return H2X_ERR_TOO_LARGE;
     }
     for (int dim = 0; dim < kMaxSpatial && err == 0; ++dim)

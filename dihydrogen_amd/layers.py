@@ -509,6 +509,8 @@ class HaloExchangeAccumOp(Enum):
     MIN = capi.HALO_MIN
 
 
+# what the launches that serve a whole grid refuse (and then launch nothing) goes through buffers
+_NOT_FOR_THE_GRID = (capi.ERR_UNSUPPORTED, capi.ERR_TOO_LARGE)
 _FULL_WIDTHS = (None, None, None, None)  # exchange(): every halo at its full width
 
 
@@ -812,9 +814,10 @@ class HaloExchangeVirtual:
                     status = self._calls.h2x_halo_grid_fold(dtype, grid, op.value, st)
                 else:
                     status = self._calls.h2x_halo_grid_exchange(dtype, grid, st)
-                if status:
-                    capi.check(status, "halo exchange (grid)")
-                return
+                if status not in _NOT_FOR_THE_GRID:
+                    if status:
+                        capi.check(status, "halo exchange (grid)")
+                    return
         widths = tuple([ov if w is None else w for w in given])
         key = ("all", None if given == _FULL_WIDTHS else tuple(map(tuple, widths)), is_reverse, skip_unpack, op, fused, self._addresses())
         launches = self._faces.get(key)
@@ -851,9 +854,10 @@ class HaloExchangeVirtual:
         if grid:
             status = self._calls.h2x_halo_grid_clear(self.tensors[0].h2x_dtype, grid, int(only_unfilled),
                                                      _stream_handle(self.stream))
-            if status:
-                capi.check(status, "clear_halos (grid)")
-            return
+            if status not in _NOT_FOR_THE_GRID:
+                if status:
+                    capi.check(status, "clear_halos (grid)")
+                return
         key = ("clear", only_unfilled, self._addresses())
         if key not in self._faces:
             faces = []

@@ -39,3 +39,61 @@ def test_ranks_with_halos_of_unequal_widths(widths):
     for t in ts:
         assert np.array_equal(audit.counts(t.data)[1] > 0, packed._strip(t, 0, 0, t.overlap[0], inner=False).ravel()
                               | packed._strip(t, 0, 1, t.overlap[0], inner=False).ravel())
+
+
+@pytest.mark.parametrize("status", [-2, -3])
+@pytest.mark.parametrize("step", ["forward", "reverse", "clear"])
+def test_what_the_whole_grid_launches_refuse_goes_through_buffers(step, status, monkeypatch):
+    import torch
+    from dihydrogen_amd import layers
+    shape, locale, overlap = packed.HALO_CASES[1]
+    results = []
+    for refuse in (False, True):
+        with CopyAudit() as audit:
+            ts = packed._tensors(shape, locale, overlap, torch.float32, audit)
+            xch = layers.HaloExchangeVirtual(ts)
+            if refuse:
+                calls = xch._calls
+
+                class Refusing:
+                    def __getattr__(self, name):
+                        return (lambda *args: status) if name.startswith("h2x_halo_grid_") else getattr(calls, name)
+
+                xch._calls = Refusing()
+            if step == "clear":
+                xch.clear_halos()
+            else:
+                xch.exchange(is_reverse=step == "reverse")
+        packed._clean(audit.report)
+        assert bool(audit.buffers) == (refuse and step != "clear")
+        results.append([audit.counts(t.data)[1] > 0 for t in ts])
+    for a, b in zip(*results):
+        assert np.array_equal(a, b)
+
+
+def test_limits_of_a_reverse_exchange_are_those_of_one_rank_and_of_a_launch():
+    """Ranks of short rows, imaginary addresses: what is not refused fails for want of a GPU.  A launch
+    has up to 2^32 - 1 threads, one a row here, and one rank up to 2^31."""
+    import ctypes
+
+    import torch
+    from dihydrogen_amd import capi
+    if torch.cuda.is_available():
+        pytest.skip("a GPU is visible: these calls would launch on imaginary pointers")
+
+    def fold(num_ranks, rows):
+        ranks = (capi.HaloGridRank * num_ranks)()
+        for r, k in enumerate(ranks):
+            k.tensor = 1 << 20
+            k.local_shape[:4] = 2, rows, 1, 1
+            for d in range(4):
+                k.peer[d][:] = [(r - 1) % num_ranks, (r + 1) % num_ranks] if d == 0 else [-1, -1]
+        grid = capi.HaloGrid(4, num_ranks)
+        grid.overlap[0], grid.ranks = 1, ranks
+        return capi.load().h2x_halo_grid_fold(capi.F32, ctypes.byref(grid), capi.HALO_SUM, None)
+
+    assert fold(8, 1000) > 0
+    assert fold(8, 270_000_000) > 0                # 2.16 billion threads
+    assert fold(16, 256 * (0xffffff // 16)) > 0    # 4.29 billion
+    assert fold(16, 256 * (0xffffff // 16) + 1) == capi.ERR_TOO_LARGE
+    assert fold(2, 536_870_912) == capi.ERR_TOO_LARGE  # tensors of 2^31 elements
