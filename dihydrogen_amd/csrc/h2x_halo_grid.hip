@@ -418,7 +418,7 @@ int make_args(const h2x_halo_grid& h, int cells, int only_unfilled, int elem_siz
             if (from.local_shape[d] < 1 || from.local_shape[d] >= (1ll << 31))
                 return H2X_ERR_INVALID_ARGUMENT;
             if (d >= ns && from.local_shape[d] != h.ranks[0].local_shape[d])
-                return H2X_ERR_INVALID_ARGUMENT;
+                return H2X_ERR_UNSUPPORTED; // channels or samples spread unevenly: `outer` is one number
             real *= from.local_shape[d] + 2 * (d < ns ? a->width[d] : 0);
             if (real >= (1ll << 31))
                 return H2X_ERR_TOO_LARGE;

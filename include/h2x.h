@@ -1056,7 +1056,11 @@ typedef struct h2x_halo_grid_rank
     int32_t peer[H2X_MAX_DIMS][2];
 } h2x_halo_grid_rank;
 
-/** 3 to 5 dimensions, the last two (channels, samples) without halo; at most 16 ranks, none empty. */
+/**
+ * 3 to 5 dimensions, the last two (channels, samples) without halo and of one extent on all ranks;
+ * at most 16 ranks, none empty.  What these calls do not serve they refuse with
+ * H2X_ERR_UNSUPPORTED or H2X_ERR_TOO_LARGE and launch nothing.
+ */
 typedef struct h2x_halo_grid
 {
     int32_t num_dims;

@@ -97,3 +97,26 @@ def test_limits_of_a_reverse_exchange_are_those_of_one_rank_and_of_a_launch():
     assert fold(16, 256 * (0xffffff // 16)) > 0    # 4.29 billion
     assert fold(16, 256 * (0xffffff // 16) + 1) == capi.ERR_TOO_LARGE
     assert fold(2, 536_870_912) == capi.ERR_TOO_LARGE  # tensors of 2^31 elements
+
+
+@pytest.mark.parametrize("step", ["forward", "reverse", "clear"])
+def test_samples_spread_unevenly_over_the_ranks(step):
+    """Space and samples are both distributed: neighbours hold the same samples, other ranks fewer."""
+    import torch
+    from dihydrogen_amd import capi
+    from dihydrogen_amd.layers import HaloExchangeVirtual
+    with CopyAudit() as audit:
+        ts = packed._tensors((12, 10, 2, 3), (2, 2, 1, 2), (1, 1, 0, 0), torch.float32, audit)
+        assert len({t.local_shape[3] for t in ts}) == 2
+        xch = HaloExchangeVirtual(ts)
+        if step == "clear":
+            xch.clear_halos()
+        else:
+            xch.exchange(is_reverse=step == "reverse")
+    packed._clean(audit.report)
+    for r, t in enumerate(ts):
+        if step == "clear":
+            want = sum(packed._strip(t, d, side, 1, inner=False) for d in (0, 1) for side in (capi.LHS, capi.RHS)).ravel()
+        else:
+            want = packed._expected_exchange(xch, reverse=step == "reverse")[1][r] > 0
+        assert np.array_equal(audit.counts(t.data)[1] > 0, want)
