@@ -521,9 +521,12 @@ class HaloExchangeVirtual:
     The reference object belongs to one rank and hands packed strips to a
     transport.  Here the object holds every rank's local tensor; rank r's send
     buffer for (dim, side) *is* the receive buffer of its neighbour on that
-    side for the opposite side, so the transfer is free, and each dimension
-    phase is two launches (pack all ranks and sides, unpack all ranks and
-    sides).  ``periodic`` wraps neighbours at the grid edge; the reference
+    side for the opposite side, so the transfer is free.  A packed exchange is
+    two launches a dimension (pack all ranks and sides, unpack all ranks and
+    sides).  A full-width exchange of tensors that share a GPU goes straight
+    from tensor to tensor, in one launch (reverse: one a dimension), unless
+    a receive buffer was asked for, ``launch_hook`` is set or ``_grid`` names
+    another reason.  ``periodic`` wraps neighbours at the grid edge; the reference
     never does (MPI_PROC_NULL, halo_exchange_cuda.hpp:343-345).
     """
 
@@ -546,6 +549,9 @@ class HaloExchangeVirtual:
         # (of the packing and unpacking launches: a hooked exchange runs dimension by dimension)
         self.launch_hook = None
         self._buffers_wanted = False  # a receive buffer was handed out: exchanges fill them
+        # (addresses, is_reverse) of the last exchange that left no strips in the buffers, and the
+        # dimensions that were packed after it
+        self._direct, self._packed_since = None, ()
         self._grid_of = None  # (addresses, h2x_halo_grid or None, usable for exchanges)
 
     def get_halo_size(self, rank: int, dim: int, width: int) -> int:
@@ -594,14 +600,35 @@ class HaloExchangeVirtual:
 
     def recv_buffer(self, rank: int, dim: int, side: int) -> torch.Tensor:
         """The buffer rank `rank` unpacks its (dim, side) halo from -- and its
-        neighbour on that side packs into (get_recv_buffer, halo_exchange_cuda.hpp:277-283)."""
+        neighbour on that side packs into (get_recv_buffer, halo_exchange_cuda.hpp:277-283).
+
+        Once one has been asked for, every exchange that is not ``fused`` goes through the
+        buffers.  An exchange before that may have moved its strips straight from tensor to
+        tensor: they are packed now, from the tensors as they are.  That is what was received as
+        long as the tensors have not been written since; the cells of a strip that a later dimension's
+        phase writes, where strips of two dimensions cross, hold what that phase left."""
         self._buffers_wanted = True
+        self._pack_what_was_exchanged()
         made = (rank, dim, side) not in self._recv
         buffer = self._receive_buffer(rank, dim, side)
         if made and self.stream is not None and buffer.is_cuda:
             # what the caller does with it on the current stream comes after it was cleared
             torch.cuda.current_stream().wait_stream(self.stream)
         return buffer
+
+    def _pack_what_was_exchanged(self) -> None:
+        if self._direct is None:
+            return
+        addresses, is_reverse = self._direct
+        if addresses != self._addresses():
+            raise RuntimeError("the tensors were reallocated since the exchange: ask for a receive buffer before it")
+        dtype, st = self.tensors[0].h2x_dtype, _stream_handle(self.stream)
+        for dim, w in enumerate(self.tensors[0].overlap):
+            if dim in self._packed_since:
+                continue
+            for label, call, arr in self._dim_launches(dim, w, w, w, w, is_reverse, True, HaloExchangeAccumOp.ID, False):
+                capi.check(call(dtype, ctypes.addressof(arr), len(arr), st), label)
+        self._direct = None
 
     def _receive_buffer(self, rank: int, dim: int, side: int) -> torch.Tensor:
         key = (rank, dim, side)
@@ -670,6 +697,8 @@ class HaloExchangeVirtual:
         neighbour's LHS receive buffer and vice versa.  With ``fused`` the strips
         move straight from tensor to tensor in one launch per group of ranks;
         the result is the same."""
+        if not fused:
+            self._packed_since += (dim,)
         self._issue(self._dim_launches(dim, width_rhs_send, width_rhs_recv, width_lhs_send, width_lhs_recv,
                                        is_reverse, skip_unpack, op, fused))
 
@@ -817,6 +846,8 @@ class HaloExchangeVirtual:
                 if status not in _NOT_FOR_THE_GRID:
                     if status:
                         capi.check(status, "halo exchange (grid)")
+                    if not fused:
+                        self._direct, self._packed_since = (self._grid_of[0], is_reverse), ()
                     return
         widths = tuple([ov if w is None else w for w in given])
         key = ("all", None if given == _FULL_WIDTHS else tuple(map(tuple, widths)), is_reverse, skip_unpack, op, fused, self._addresses())
@@ -826,6 +857,8 @@ class HaloExchangeVirtual:
             for d in range(self.nd):
                 launches += self._dim_launches(d, *(w[d] for w in widths), is_reverse, skip_unpack, op, fused)
             self._faces[key] = launches
+        if not fused:
+            self._direct = None
         self._issue(launches)
 
     def clear_halo(self, dim: int) -> None:

@@ -121,3 +121,50 @@ def test_samples_spread_unevenly_over_the_ranks(step):
         else:
             want = packed._expected_exchange(xch, reverse=step == "reverse")[1][r] > 0
         assert np.array_equal(audit.counts(t.data)[1] > 0, want)
+
+
+@pytest.mark.parametrize("is_reverse", [False, True])
+def test_a_receive_buffer_asked_for_after_an_exchange_holds_its_strip(is_reverse):
+    """Exchanged straight from tensor to tensor, packed when a buffer is asked for, and by the next exchange itself."""
+    import torch
+    from dihydrogen_amd import capi
+    from dihydrogen_amd.layers import HaloExchangeVirtual
+    shape, locale, overlap = packed.HALO_CASES[4]
+    with CopyAudit() as audit:
+        ts = packed._tensors(shape, locale, overlap, torch.float32, audit)
+        xch = HaloExchangeVirtual(ts)
+        xch.exchange(is_reverse=is_reverse)
+        assert not audit.buffers
+        expected = [(r, d, s) for r in range(8) for d in range(3) for s in (capi.LHS, capi.RHS)
+                    if xch.find_peer_rank(r, d, s) is not None]
+        first = {key: xch.recv_buffer(*key) for key in expected}
+        written = {key: audit.counts(b) for key, b in first.items()}
+        for loads, stores in written.values():
+            assert (stores == 1).all() and not loads.any()
+        xch.exchange(is_reverse=is_reverse)
+        for key in expected:
+            assert xch.recv_buffer(*key).data_ptr() == first[key].data_ptr()
+            loads, stores = audit.counts(first[key])
+            assert (stores == 2).all() and (loads == 1).all()
+    packed._clean(audit.report)
+
+
+def test_strips_packed_since_an_exchange_are_not_packed_again():
+    import torch
+    from dihydrogen_amd import capi
+    from dihydrogen_amd.layers import HaloExchangeVirtual
+    shape, locale, overlap = packed.HALO_CASES[0]
+    with CopyAudit() as audit:
+        ts = packed._tensors(shape, locale, overlap, torch.float32, audit)
+        xch = HaloExchangeVirtual(ts)
+        xch.exchange()
+        xch.exchange_dim(0, 1, 1, 1, 1)
+        xch.exchange(fused=True)
+        for dim in (0, 1):
+            loads, stores = audit.counts(xch.recv_buffer(0, dim, capi.RHS))
+            assert (stores == 1).all() and (loads == (1 - dim)).all()
+        ts[0].data = ts[0].data.clone()
+        other = HaloExchangeVirtual(ts)
+        other._direct = ((0,) * 4, False)      # exchanged when the tensors lay elsewhere
+        with pytest.raises(RuntimeError, match="reallocated"):
+            other.recv_buffer(0, 0, capi.RHS)
