@@ -105,6 +105,8 @@ PyMethodDef s_methods[] = {H2X_ENTRY(h2x_bn_channel_sums_and_sqsums),
                            H2X_ENTRY(h2x_bn_backprop2),
                            H2X_ENTRY(h2x_bn_backprop2_strided),
                            H2X_ENTRY(h2x_bn_backprop2_clearing),
+                           H2X_ENTRY(h2x_bn_forward_local),
+                           H2X_ENTRY(h2x_bn_backward_local),
                            H2X_ENTRY(h2x_bn_forward_once),
                            H2X_ENTRY(h2x_bn_forward_clearing),
                            H2X_ENTRY(h2x_bn_backward_clearing),

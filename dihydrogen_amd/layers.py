@@ -92,6 +92,13 @@ def _share_a_haloed_geometry(*layouts: Layout) -> bool:
     return l0.haloed and not l0.channel_halo and all(l.alike == l0.alike for l in layouts)
 
 
+def _pair_in_order(l0: Layout, *layouts: Layout) -> bool:
+    """Dense tensors: the dense entry points pair the elements of a channel in order whatever the
+    extents (4-D and 5-D with one plane, H x W and W x H; the strided ones refuse them), provided
+    all have the memory for the samples of `l0`."""
+    return l0.dense and all(l.dense and l.samples * l.channels >= l0.samples * l0.channels for l in layouts)
+
+
 class BatchNormalization:
     """BatchNormalization<Backend, DataType>
     (legacy/include/distconv/dnn_backend/batchnorm.hpp:100-581).
@@ -240,6 +247,12 @@ class BatchNormalization:
             _dense_layout(input), _dense_layout(output)
             ns = self.num_current_samples = lx.samples
             per_sum = self._elements_per_sum(lx)
+            if lx.extents != ly.extents and _pair_in_order(lx, ly):
+                capi.check(self._calls.h2x_bn_forward_local(
+                    lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ly.spatial_real, input.get_base_ptr(),
+                    scale, bias, per_sum, self.decay, self.epsilon, mean, var, running_mean, running_var,
+                    output.get_base_ptr(), self._ws(lx.channels), _stream_handle(self.stream)), "bn forward (local)")
+                return 0
             status = self._calls.h2x_bn_forward_once(
                 lx.dtype, ns, lx.geometry_address, _tensor_geometry(ly, ns), input.get_base_ptr(), scale, bias, per_sum,
                 self.decay, self.epsilon, mean, var, running_mean, running_var, output.get_base_ptr(),
@@ -322,6 +335,13 @@ class BatchNormalization:
             _dense_layout(input), _dense_layout(d_output), _dense_layout(d_input)
             ns = self.num_current_samples = lx.samples
             per_sum = self._elements_per_sum(lx)
+            if (lx.extents != ld.extents or lx.extents != li.extents) and _pair_in_order(lx, ld, li):
+                capi.check(self._calls.h2x_bn_backward_local(
+                    lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ld.spatial_real, li.spatial_real, per_sum,
+                    input.get_base_ptr(), d_output.get_base_ptr(), mean, var, scale, scale_gradient, bias_gradient,
+                    mean_gradient, var_gradient, d_input.get_base_ptr(), self.epsilon, self._ws(lx.channels),
+                    _stream_handle(self.stream)), "bn backward (local)")
+                return 0
             status = self._calls.h2x_bn_backward_once(
                 lx.dtype, ns, per_sum, lx.geometry_address, _tensor_geometry(ld, ns), _tensor_geometry(li, ns),
                 input.get_base_ptr(), d_output.get_base_ptr(), mean, var, scale, scale_gradient, bias_gradient,

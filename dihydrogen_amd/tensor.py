@@ -150,6 +150,7 @@ class Layout:
             spatial_real *= real[d]
         self.spatial, self.spatial_real = spatial, spatial_real
         samples, channels = self.samples, self.channels = local[ns + 1], local[ns]
+        self.extents = tuple(local[:ns + 1])  # of one sample
         # no halo on the inner spatial dimensions: the layout the dense entry points take
         # (legacy/src/dnn_backend/batchnorm.cu:210-219)
         self.dense = not any(overlap[:max(ns - 1, 0)])

@@ -1,6 +1,6 @@
-"""Buffers that a layer makes for its launches belong to the stream it launches on: cleared there before the
-launch, and on loan from that stream's memory.  On the CPU, with the library's calls stubbed out: nothing is
-launched and no address is followed."""
+"""What the Python layers hand to the library.  Buffers that a layer makes for its launches belong to the stream it
+launches on: cleared there before the launch, and on loan from that stream's memory.  On the CPU, with the
+library's calls stubbed out: nothing is launched and no address is followed."""
 import contextlib
 
 import pytest
@@ -93,3 +93,23 @@ def test_buffers_are_made_on_the_stream_that_is_launched_on(use, made):
     made.clear()
     use(None)
     assert made and all(s is None for s, _ in made)
+
+
+def test_dense_tensors_of_other_extents_go_to_the_calls_that_take_them(made, monkeypatch):
+    called = []
+
+    class Recording:
+        def __getattr__(self, name):
+            return lambda *args: called.append(name) or 0
+
+    monkeypatch.setattr(capi, "calls", Recording)
+    dist = Distribution.make_localized_distribution
+    x = Tensor([8, 4, 6, 3], LocaleVirtual(0, 1), dist(4), device="cpu").allocate()
+    for shape, forward, backward in (([4, 8, 6, 3], "local", "local"), ([8, 4, 1, 6, 3], "local", "local"),
+                                     ([8, 4, 6, 3], "once", "once"), ([4, 8, 6, 2], "once", "once")):
+        y = Tensor(shape, LocaleVirtual(0, 1), dist(len(shape)), device="cpu").allocate()
+        bn = BatchNormalization(4, 0.9, 1e-5)
+        bn.forward(x, *[x.data] * 6, y)
+        bn.backward(x, y, *[x.data] * 7, x)
+        assert called == ["h2x_bn_forward_" + forward, "h2x_bn_backward_" + backward]
+        called.clear()
