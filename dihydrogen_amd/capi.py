@@ -211,6 +211,8 @@ SIGNATURES = {
                                               c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_double, c_void_p,
                                               c_void_p]),
     "h2x_bn_team_state_bytes": (c_size_t, [c_int]),
+    "h2x_bn_team_state_needed": (c_size_t, [c_int, c_int, POINTER(TensorGeometry)]),
+    "h2x_bn_team_state_needed_clearing": (c_size_t, [c_int, POINTER(HaloedGeometry)]),
     "h2x_bn_forward_once": (c_int, [c_int, c_int, POINTER(TensorGeometry), POINTER(TensorGeometry), c_void_p,
                                     c_void_p, c_void_p, c_size_t, c_double, c_double, c_void_p, c_void_p,
                                     c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),

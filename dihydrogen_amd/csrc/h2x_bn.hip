@@ -2642,6 +2642,14 @@ void issue_once(const G& g, const OnceBackward<float>& a, hipStream_t st)
     bn_once_backward_kernel<float, TEAM, K, STREAM, kInLds><<<once_grid<TEAM>(g), once_block<TEAM>(), 0, st>>>(g, a);
 }
 
+// A channel fits the registers of one workgroup, in a variant that pays.
+template <typename A, typename G>
+bool once_holds(const G& g)
+{
+    constexpr uint32_t kMost = 1024 * (std::is_same<A, OnceForward<float>>::value ? 20 : 16);
+    return g.vectors <= (g.num_channels >= kOnceManyChannels ? kMost : 1024 * 8);
+}
+
 // The smallest team whose K vectors a thread hold the channel: four where that is enough
 // workgroups (more threads wait for memory together), more only beyond 1024 threads.
 // False: no variant holds it.
@@ -2649,6 +2657,8 @@ template <bool STREAM, typename G, typename A>
 bool once_launch(const G& g, const A& a, hipStream_t st)
 {
     constexpr bool kForward = std::is_same<A, OnceForward<float>>::value;
+    if (!once_holds<A>(g))
+        return false;
     if (g.vectors <= 64 * 2)
         issue_once<64, 2, STREAM>(g, a, st);
     else if (g.vectors <= 256 * 4)
@@ -2659,12 +2669,10 @@ bool once_launch(const G& g, const A& a, hipStream_t st)
         issue_once<1024, 4, STREAM>(g, a, st);
     else if (g.vectors <= 1024 * 8)
         issue_once<1024, 8, STREAM>(g, a, st);
-    else if (g.num_channels >= kOnceManyChannels && g.vectors <= 1024 * 16)
+    else if (g.vectors <= 1024 * 16)
         issue_once<1024, 16, STREAM>(g, a, st);
-    else if (kForward && g.num_channels >= kOnceManyChannels && g.vectors <= 1024 * 20)
-        issue_once<1024, kForward ? 20 : 16, STREAM>(g, a, st);
     else
-        return false;
+        issue_once<1024, kForward ? 20 : 16, STREAM>(g, a, st);
     return true;
 }
 
@@ -2712,9 +2720,9 @@ void issue_team(const TeamGeometry<G>& g, const OnceBackward<T>& a, unsigned lon
 }
 
 // Members of TEAM threads with K vectors each; false if that is fewer than `least` workgroups,
-// more than `most` members, or more sums than a channel's state has.
+// more than `most` members, or more sums than a channel's state has.  Without a: whether.
 template <int TEAM, int K, typename G, template <typename> class A, typename T>
-bool team_launch(const G& once, const A<T>& a, bool stream, uint32_t least, uint32_t most,
+bool team_launch(const G& once, const A<T>* a, bool stream, uint32_t least, uint32_t most,
                  uint32_t max_polls, void* team_state, hipStream_t st)
 {
     constexpr int kSums = std::is_same<A<T>, OnceForward<T>>::value ? 2 : 4;
@@ -2722,6 +2730,8 @@ bool team_launch(const G& once, const A<T>& a, bool stream, uint32_t least, uint
     const size_t blocks = static_cast<size_t>(members) * once.num_channels;
     if (members > most || members * kSums > kMaxTeamSums || blocks < least || blocks >= (1u << 30))
         return false;
+    if (!a)
+        return true;
     TeamGeometry<G> g;
     g.once = once;
     g.members = make_fastdiv(members);
@@ -2729,9 +2739,9 @@ bool team_launch(const G& once, const A<T>& a, bool stream, uint32_t least, uint
     g.max_polls = max_polls;
     unsigned long long* const states = static_cast<unsigned long long*>(team_state);
     if (stream || G::kClears)
-        issue_team<T, TEAM, K, true>(g, a, states, st);
+        issue_team<T, TEAM, K, true>(g, *a, states, st);
     else
-        issue_team<T, TEAM, K, G::kClears>(g, a, states, st);
+        issue_team<T, TEAM, K, G::kClears>(g, *a, states, st);
     return true;
 }
 
@@ -2747,7 +2757,7 @@ constexpr uint32_t kLargeMembers = 384, kMediumMembers = 256, kSmallMembers = 12
 // in 224 of 32 KB 6.8 us, in two launches 9.8); up to 128 members (N 16, C 16, 64^3 in 128 of them 98 us, in
 // two launches 118).  `forced`: however few workgroups that is.
 template <typename G, typename T>
-bool team_variant(const G& g, const OnceForward<T>& a, bool stream, bool forced, uint32_t most, uint32_t polls,
+bool team_variant(const G& g, const OnceForward<T>* a, bool stream, bool forced, uint32_t most, uint32_t polls,
                   void* team_state, hipStream_t st)
 {
     return team_launch<512, 16>(g, a, stream, forced ? 1 : kLargeMembers, most, polls, team_state, st)
@@ -2761,7 +2771,7 @@ bool team_variant(const G& g, const OnceForward<T>& a, bool stream, bool forced,
 // its last member than it saves.  32 KB where that is not enough workgroups
 // (N 2, C 32, 28^3 with a halo 8.0 us, in two launches 12.4).
 template <typename G, typename T>
-bool team_variant(const G& g, const OnceBackward<T>& a, bool stream, bool forced, uint32_t most, uint32_t polls,
+bool team_variant(const G& g, const OnceBackward<T>* a, bool stream, bool forced, uint32_t most, uint32_t polls,
                   void* team_state, hipStream_t st)
 {
     most /= 2;
@@ -2794,6 +2804,33 @@ uint32_t compute_units()
     return static_cast<uint32_t>(cus);
 }
 
+// A team keeps within half of the chip.
+uint32_t most_members()
+{
+    const uint32_t cus = compute_units();
+    return cus ? std::min(cus / 2, kMaxMembers) : kMaxMembers;
+}
+
+// Bytes of the state for calls on tensors like this, apart from one another: 0 if none is for teams.
+template <typename G>
+size_t team_state_needed(const G& g)
+{
+    const uint32_t most = most_members();
+    const OnceForward<float>* const forward = nullptr;
+    const OnceBackward<float>* const backward = nullptr;
+    const bool teams = ((teams_first(g) || !once_holds<OnceForward<float>>(g))
+                        && team_variant(g, forward, true, false, most, 0, nullptr, nullptr))
+                       || ((teams_first(g) || !once_holds<OnceBackward<float>>(g))
+                           && team_variant(g, backward, true, false, most, 0, nullptr, nullptr));
+    return teams ? g.num_channels * kStateWords * sizeof(unsigned long long) : 0;
+}
+
+// Short segments have kernels of their own (N 2048, C 256, 7 x 7: 141 us, by teams 172).
+bool for_teams(const OnceGeometry& g, int n)
+{
+    return !dense_rows(g) || streamed(g, n);
+}
+
 // False: the call is not for teams.  bytes: from the first to behind the last element of a tensor.
 template <typename G, typename A>
 bool launch_by_teams(const G& g, const A& a, size_t bytes, bool stream, std::initializer_list<const void*> inputs,
@@ -2804,19 +2841,15 @@ bool launch_by_teams(const G& g, const A& a, size_t bytes, bool stream, std::ini
     for (const void* p : inputs)
         if (!apart(p, output, bytes))
             return false;
-    const uint32_t cus = compute_units();
-    return team_variant(g, a, stream, forced, std::min(cus / 2, kMaxMembers), polls, team_state, st);
+    return team_variant(g, &a, stream, forced, most_members(), polls, team_state, st);
 }
 
 template <typename A>
 bool launch_by_teams(const OnceGeometry& g, const A& a, int n, std::initializer_list<const void*> inputs,
                      const void* output, bool forced, uint32_t polls, void* team_state, hipStream_t st)
 {
-    // short segments have kernels of their own (N 2048, C 256, 7 x 7: 141 us, by teams 172)
-    const bool stream = streamed(g, n);
-    if (dense_rows(g) && !stream)
-        return false;
-    return launch_by_teams(g, a, reach_bytes(g, n), stream, inputs, output, forced, polls, team_state, st);
+    return for_teams(g, n)
+           && launch_by_teams(g, a, reach_bytes(g, n), streamed(g, n), inputs, output, forced, polls, team_state, st);
 }
 
 // team_polls: by teams or not at all, however few workgroups that is, with this many looks.
@@ -2894,15 +2927,12 @@ int backward_once(int n, size_t num_per_sum, const h2x_tensor_geometry* gx, cons
                              dx, eps, ws, st);
 }
 
-// The same for tensors of one haloed geometry whose outputs' halos are cleared, by one workgroup
-// or a team a channel; H2X_ERR_UNSUPPORTED: in the staged calls.
-template <typename A>
-int clearing_once(const h2x_haloed_geometry* h, const A& a, std::initializer_list<const void*> inputs, void* output,
-                  void* team_state, hipStream_t st)
+// Tensors of one haloed geometry whose outputs' halos are cleared, as whole allocations: up to 2^28
+// elements, vectors of 16 bytes within one segment.  bytes: of a tensor.
+int clear_geometry(const h2x_haloed_geometry* h, ClearGeometry* g, size_t* bytes)
 {
-    ClearGeometry g;
     size_t real;
-    const int err = real_box(h, &g.box, &real);
+    const int err = real_box(h, &g->box, &real);
     if (err)
         return err;
     constexpr size_t vec = full_vec<float>();
@@ -2911,19 +2941,35 @@ int clearing_once(const h2x_haloed_geometry* h, const A& a, std::initializer_lis
     size_t interior = 1;
     for (int d = 0; d < nd - 2; ++d)
         interior *= h->local_shape[d];
-    bool fit = n > 0 && c > 0 && interior > 0 && real % vec == 0 && aligned16(output) && output;
+    if (n == 0 || c == 0 || interior == 0 || real % vec != 0 || n * c * real >= (1ull << 28) || c > 0x7fffffffull)
+        return H2X_ERR_UNSUPPORTED;
+    g->per_segment = make_fastdiv(static_cast<uint32_t>(real / vec));
+    g->vectors = static_cast<uint32_t>(n * (real / vec));
+    g->stride_n = static_cast<uint32_t>(c * real);
+    g->stride_c = static_cast<int64_t>(real);
+    g->num_channels = static_cast<uint32_t>(c);
+    *bytes = n * c * real * sizeof(float);
+    return H2X_SUCCESS;
+}
+
+// The same for such tensors, by one workgroup or a team a channel; H2X_ERR_UNSUPPORTED: in the
+// staged calls.
+template <typename A>
+int clearing_once(const h2x_haloed_geometry* h, const A& a, std::initializer_list<const void*> inputs, void* output,
+                  void* team_state, hipStream_t st)
+{
+    ClearGeometry g;
+    size_t bytes;
+    const int err = clear_geometry(h, &g, &bytes);
+    if (err)
+        return err;
+    bool fit = aligned16(output) && output;
     for (const void* p : inputs)
         fit = fit && p && aligned16(p);
-    if (!fit || n * c * real >= (1ull << 28) || c > 0x7fffffffull)
+    if (!fit)
         return H2X_ERR_UNSUPPORTED;
-    g.per_segment = make_fastdiv(static_cast<uint32_t>(real / vec));
-    g.vectors = static_cast<uint32_t>(n * (real / vec));
-    g.stride_n = static_cast<uint32_t>(c * real);
-    g.stride_c = static_cast<int64_t>(real);
-    g.num_channels = static_cast<uint32_t>(c);
     const auto by_teams = [&] {
-        return launch_by_teams(g, a, n * c * real * sizeof(float), true, inputs, output, false, kTeamPolls, team_state,
-                               st);
+        return launch_by_teams(g, a, bytes, true, inputs, output, false, kTeamPolls, team_state, st);
     };
     const bool teams = teams_first(g);
     if ((teams && by_teams()) || once_launch<true>(g, a, st) || (!teams && by_teams()))
@@ -3309,6 +3355,29 @@ extern "C" int h2x_bn_backward_local_strided(h2x_dtype dtype, int num_samples, s
 extern "C" size_t h2x_bn_team_state_bytes(int num_channels)
 {
     return static_cast<size_t>(std::max(num_channels, 1)) * kStateWords * sizeof(unsigned long long);
+}
+
+extern "C" size_t h2x_bn_team_state_needed(h2x_dtype dtype, int num_samples, const h2x_tensor_geometry* geometry)
+{
+    HostTensor t;
+    OnceGeometry g;
+    int c;
+    size_t s;
+    // (an address: only its alignment is looked at, and that decides nothing here)
+    if (dtype != H2X_F32 || num_samples <= 0 || !geometry
+        || strided_tensor<float>(geometry, geometry, num_samples, &t, &c, &s) || c <= 0 || s == 0
+        || !once_geometry(num_samples, c, s, {&t}, &g) || !for_teams(g, num_samples))
+        return 0;
+    return team_state_needed(g);
+}
+
+extern "C" size_t h2x_bn_team_state_needed_clearing(h2x_dtype dtype, const h2x_haloed_geometry* geometry)
+{
+    ClearGeometry g;
+    size_t bytes;
+    if (dtype != H2X_F32 || !geometry || clear_geometry(geometry, &g, &bytes))
+        return 0;
+    return team_state_needed(g);
 }
 
 extern "C" int h2x_bn_forward_once(h2x_dtype dtype, int num_samples,

@@ -145,13 +145,15 @@ class BatchNormalization:
             self._workspace_channels = num_channels
         return self._workspace
 
-    def _team_state(self, l: Layout, segment: int) -> Optional[torch.Tensor]:
-        """Where the workgroups that share a channel exchange its sums; smaller channels than 16 K
-        elements need none."""
-        if l.samples * segment <= 16384 or l.dtype != capi.F32:
+    def _team_state(self, l: Layout, clearing: bool) -> Optional[torch.Tensor]:
+        """Where the workgroups that share a channel exchange its sums; None where no workgroups
+        do.  Smaller channels than 16 K elements need none."""
+        if l.samples * l.spatial_real <= 16384 or l.dtype != capi.F32:
             return None
         if self._state is None or self._state_channels < l.channels:
-            nbytes = self._lib.h2x_bn_team_state_bytes(l.channels)
+            nbytes = l.clearing_team_state_bytes if clearing else l.team_state_bytes
+            if nbytes == 0:
+                return None
             self._state = _buffer_of(self.stream, nbytes, torch.uint8, zero=True)
             self._state_channels = l.channels
         return self._state
@@ -238,7 +240,7 @@ class BatchNormalization:
                 status = self._calls.h2x_bn_forward_clearing(
                     lx.dtype, lx.haloed_geometry_address, input.get_buffer(), scale, bias, self._elements_per_sum(lx),
                     self.decay, self.epsilon, mean, var, running_mean, running_var, output.get_buffer(),
-                    self._team_state(lx, lx.spatial_real), _stream_handle(self.stream))
+                    self._team_state(lx, True), _stream_handle(self.stream))
                 if status != capi.ERR_UNSUPPORTED:
                     self.num_current_samples = lx.samples
                     capi.check(status, "bn forward (clearing)")
@@ -256,7 +258,7 @@ class BatchNormalization:
             status = self._calls.h2x_bn_forward_once(
                 lx.dtype, ns, lx.geometry_address, _tensor_geometry(ly, ns), input.get_base_ptr(), scale, bias, per_sum,
                 self.decay, self.epsilon, mean, var, running_mean, running_var, output.get_base_ptr(),
-                self._ws(lx.channels), self._team_state(lx, lx.spatial), _stream_handle(self.stream))
+                self._ws(lx.channels), self._team_state(lx, False), _stream_handle(self.stream))
             if status:
                 capi.check(status, "bn forward (local)")
             return 0
@@ -325,7 +327,7 @@ class BatchNormalization:
                 status = self._calls.h2x_bn_backward_clearing(
                     lx.dtype, self._elements_per_sum(lx), lx.haloed_geometry_address, input.get_buffer(),
                     d_output.get_buffer(), mean, var, scale, scale_gradient, bias_gradient, mean_gradient,
-                    var_gradient, d_input.get_buffer(), self.epsilon, self._team_state(lx, lx.spatial_real),
+                    var_gradient, d_input.get_buffer(), self.epsilon, self._team_state(lx, True),
                     _stream_handle(self.stream))
                 if status != capi.ERR_UNSUPPORTED:
                     self.num_current_samples = lx.samples
@@ -346,7 +348,7 @@ class BatchNormalization:
                 lx.dtype, ns, per_sum, lx.geometry_address, _tensor_geometry(ld, ns), _tensor_geometry(li, ns),
                 input.get_base_ptr(), d_output.get_base_ptr(), mean, var, scale, scale_gradient, bias_gradient,
                 mean_gradient, var_gradient, d_input.get_base_ptr(), self.epsilon, self._ws(lx.channels),
-                self._team_state(lx, lx.spatial), _stream_handle(self.stream))
+                self._team_state(lx, False), _stream_handle(self.stream))
             if status:
                 capi.check(status, "bn backward (local)")
             return 0

@@ -186,6 +186,16 @@ class Layout:
         return ctypes.addressof(self.geometry)
 
     @_once
+    def team_state_bytes(self) -> int:
+        """State for batch-norm calls on tensors like this (0: none is for teams of workgroups)."""
+        return capi.load().h2x_bn_team_state_needed(self.dtype, self.samples, self.geometry)
+
+    @_once
+    def clearing_team_state_bytes(self) -> int:
+        """The same for calls that clear their output's halo."""
+        return capi.load().h2x_bn_team_state_needed_clearing(self.dtype, self.haloed_geometry)
+
+    @_once
     def haloed_geometry(self):
         """h2x_haloed_geometry: local and real extents, halo widths."""
         g = capi.HaloedGeometry()

@@ -431,9 +431,11 @@ int h2x_bn_backward_local_strided(h2x_dtype dtype,
  *
  * team_state: h2x_bn_team_state_bytes() of the number of channels, or more, zeroed
  * once before the first call and then left to these calls, one after another, in any
- * order and of any sizes; null: no teams.
+ * order and of any sizes; null: no teams.  h2x_bn_team_state_needed() is that for calls
+ * on tensors like the one given, or 0 where they never use a state.
  */
 size_t h2x_bn_team_state_bytes(int num_channels);
+size_t h2x_bn_team_state_needed(h2x_dtype dtype, int num_samples, const h2x_tensor_geometry* geometry);
 int h2x_bn_forward_once(h2x_dtype dtype,
                                  int num_samples,
                                  const h2x_tensor_geometry* x_geometry,
@@ -594,8 +596,10 @@ int h2x_bn_backprop2_clearing(h2x_dtype dtype,
  * A whole forward or backward pass of a rank that shares its statistics with no one,
  * the output's halo left cleared as by the two calls above: for float tensors whose
  * channels one workgroup, or a team of them, holds in registers.
- * H2X_ERR_UNSUPPORTED, with nothing launched, for others.
+ * H2X_ERR_UNSUPPORTED, with nothing launched, for others.  team_state as above;
+ * h2x_bn_team_state_needed_clearing() is its size for these calls, or 0.
  */
+size_t h2x_bn_team_state_needed_clearing(h2x_dtype dtype, const h2x_haloed_geometry* geometry);
 int h2x_bn_forward_clearing(h2x_dtype dtype,
                             const h2x_haloed_geometry* geometry,
                             const void* x_buffer,

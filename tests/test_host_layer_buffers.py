@@ -50,7 +50,7 @@ def _tensors(shape, dist, count):
 
 
 def _batch_norm(stream):
-    x, y, dy, dx = _tensors([32, 40, 40, 3, 2], Distribution.make_localized_distribution(5), 4)
+    x, y, dy, dx = _tensors([40, 40, 32, 32, 2], Distribution.make_localized_distribution(5), 4)
     bn = BatchNormalization(5, 0.9, 1e-5, stream=stream)
     bn.forward(x, *[x.data] * 6, y)
     bn.backward(x, dy, *[x.data] * 7, dx)
