@@ -452,6 +452,14 @@ int halo_box(const h2x_halo_face& f, HostBox* out, bool origin_only = false)
     return H2X_SUCCESS;
 }
 
+// The two boundary strips of a tensor with less than two halo widths of interior share cells: what is
+// unpacked into the upper one goes into a later launch, so that no cell is combined with two strips at
+// a time.
+bool unpacked_later(const h2x_halo_face& f)
+{
+    return f.side == H2X_RHS && f.real_shape[f.dim] < 4 * static_cast<int64_t>(f.width);
+}
+
 } // namespace
 } // namespace h2x
 
@@ -496,20 +504,23 @@ extern "C" int h2x_halo_pack_or_unpack_batched(h2x_dtype dtype, const h2x_halo_f
     {
         if (!(ops_present & (1u << op)))
             continue;
-        Launcher l(as_stream(stream), es, dtype, op);
-        for (int i = 0; i < num_faces; ++i)
+        for (const bool later : {false, true})
         {
-            const int eff = faces[i].is_pack ? H2X_HALO_ID : faces[i].op;
-            if (eff != op)
-                continue;
-            const int err = l.add(boxes[i], faces[i].tensor, faces[i].buffer,
-                                  faces[i].is_pack ? kPack : kUnpack);
+            Launcher l(as_stream(stream), es, dtype, op);
+            for (int i = 0; i < num_faces; ++i)
+            {
+                const h2x_halo_face& f = faces[i];
+                const int eff = f.is_pack ? H2X_HALO_ID : f.op;
+                if (eff != op || (!f.is_pack && f.inner && unpacked_later(f)) != later)
+                    continue;
+                const int err = l.add(boxes[i], f.tensor, f.buffer, f.is_pack ? kPack : kUnpack);
+                if (err != 0)
+                    return err;
+            }
+            const int err = l.flush();
             if (err != 0)
                 return err;
         }
-        const int err = l.flush();
-        if (err != 0)
-            return err;
     }
     return H2X_SUCCESS;
 }
@@ -672,19 +683,29 @@ extern "C" int h2x_halo_exchange_fused(h2x_dtype dtype, const h2x_halo_transfer*
     {
         if (!(ops_present & (1u << op)))
             continue;
-        Launcher l(as_stream(stream), es, dtype, op);
-        for (int i = 0; i < num_transfers; ++i)
+        for (const bool later : {false, true})
         {
-            if (transfers[i].op != op)
-                continue;
-            const int err = l.add(boxes[i], transfers[i].dst, const_cast<void*>(transfers[i].src),
-                                  kTransfer);
+            Launcher l(as_stream(stream), es, dtype, op);
+            for (int i = 0; i < num_transfers; ++i)
+            {
+                const h2x_halo_transfer& t = transfers[i];
+                if (t.op != op)
+                    continue;
+                h2x_halo_face to;
+                to.dim = t.dim;
+                to.width = t.width;
+                to.side = t.src_side == H2X_LHS ? H2X_RHS : H2X_LHS;
+                to.real_shape[t.dim] = t.dst_real_shape[t.dim];
+                if ((t.is_reverse && unpacked_later(to)) != later)
+                    continue;
+                const int err = l.add(boxes[i], t.dst, const_cast<void*>(t.src), kTransfer);
+                if (err != 0)
+                    return err;
+            }
+            const int err = l.flush();
             if (err != 0)
                 return err;
         }
-        const int err = l.flush();
-        if (err != 0)
-            return err;
     }
     return H2X_SUCCESS;
 }

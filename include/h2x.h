@@ -971,7 +971,9 @@ int h2x_halo_pack_or_unpack(h2x_dtype dtype,
 /**
  * The same for `num_faces` independent strips in as few launches as possible
  * (both sides of a dimension, several tensors).  Faces of one call must not
- * overlap in what they write.  `faces` is host memory, read before return.
+ * overlap in what they write, except the two boundary strips of a tensor with
+ * less than two halo widths of interior: the upper one is unpacked after the
+ * lower one.  `faces` is host memory, read before return.
  */
 int h2x_halo_pack_or_unpack_batched(h2x_dtype dtype,
                                     const h2x_halo_face* faces,
@@ -1039,8 +1041,10 @@ typedef struct h2x_halo_transfer
 
 /**
  * `num_transfers` strips in as few launches as possible.  No transfer of a
- * call may write what another one reads or writes (true for all strips of one
- * dimension of an exchange).  `transfers` is host memory, read before return.
+ * call may write what another one reads or writes, except the two boundary strips
+ * of a tensor, which are combined one after the other where they share cells.  (True
+ * for all strips of one dimension of an exchange between ranks with at least a halo
+ * width of interior.)  `transfers` is host memory, read before return.
  */
 int h2x_halo_exchange_fused(h2x_dtype dtype,
                             const h2x_halo_transfer* transfers,
