@@ -486,6 +486,15 @@ public:
                         HaloExchangeAccumOp op)
     {
         const h2x_dtype dt = TensorType::h2x_type();
+        // strips of a rank with less than a halo width of interior reach into its halo,
+        // which the neighbours' strips are written to: all are read before any is written
+        for (auto& r : m_ranks)
+        {
+            const auto& t = r->get_tensor();
+            if (t.get_local_size() > 0
+                && static_cast<int64_t>(t.get_local_shape()[dim]) < std::max(width_rhs, width_lhs))
+                return exchange(dim, width_rhs, width_lhs, width_lhs, width_rhs, stream, is_reverse, false, op);
+        }
         // all ranks in one launch: nothing is read back between launches here,
         // so rank groups would only add launches
         {

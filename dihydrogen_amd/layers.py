@@ -717,8 +717,8 @@ class HaloExchangeVirtual:
         """One dimension for all ranks; the order pack -> (transfer) -> unpack of
         halo_exchange_cuda_mpi.hpp:25-100.  A rank's RHS strip goes to its RHS
         neighbour's LHS receive buffer and vice versa.  With ``fused`` the strips
-        move straight from tensor to tensor in one launch per group of ranks;
-        the result is the same."""
+        move straight from tensor to tensor in one launch (where every rank has at
+        least that much interior); the result is the same."""
         if not fused:
             self._packed_since += (dim,)
         self._issue(self._dim_launches(dim, width_rhs_send, width_rhs_recv, width_lhs_send, width_lhs_recv,
@@ -747,7 +747,10 @@ class HaloExchangeVirtual:
         key = (dim, widths, is_reverse, skip_unpack, op, fused, self._addresses())
         launches = self._faces.get(key)
         if launches is None:
-            build = self._fused_launches if fused else self._staged_launches
+            # strips of a rank with less than a halo width of interior reach into its halo, which the
+            # neighbours' strips are written to: all are read before any is written
+            direct = fused and all(t.local_shape[dim] >= max(widths) for t in self.tensors if t.get_local_size())
+            build = self._fused_launches if direct else self._staged_launches
             launches = self._faces[key] = build(dim, widths, is_reverse, skip_unpack, op)
         return launches
 

@@ -35,3 +35,20 @@ def test_both_strips_are_added(shape, locale, overlap, launches, fused, dtype):
     torch.cuda.synchronize()
     for t, b in zip(ts, want):
         assert torch.equal(t.real_view().cpu(), b)
+
+
+@pytest.mark.parametrize("is_reverse", [False, True])
+def test_ranks_narrower_than_a_halo(is_reverse):
+    import torch
+    from dihydrogen_amd.layers import HaloExchangeAccumOp, HaloExchangeVirtual
+    from test_gpu_direct import _tensors
+    results = []
+    for fused in (True, False):
+        ts = _tensors((5, 9, 30, 4), (3, 2, 1, 1), None, (2, 2, 0, 0), torch.float32, 2)
+        for t in ts:
+            t.data.mul_(1000).round_()      # whole numbers: sums are exact
+        HaloExchangeVirtual(ts, periodic=True).exchange(
+            is_reverse=is_reverse, op=HaloExchangeAccumOp.SUM if is_reverse else HaloExchangeAccumOp.ID, fused=fused)
+        results.append([t.data for t in ts])
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
