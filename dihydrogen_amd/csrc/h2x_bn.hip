@@ -15,6 +15,10 @@
 // accesses when the geometry allows, several loads in flight per lane,
 // per-channel parameters fetched once per workgroup.
 //
+// Float tensors that lie alike and whose channels fit the registers of one or
+// several workgroups are read once (h2x_bn_once.hpp, h2x_bn_team.hpp); what
+// follows is about the kernels that read them twice.
+//
 // Cache policy.  The layer reads x four times (sums, apply, backprop1,
 // backprop2) and dy twice, while y and dx are written once.  x of the headline
 // shapes is about the size of the 256 MB memory-side cache, so what must not
@@ -2574,7 +2578,8 @@ int backward_local_strided(int n, size_t num_per_sum, const h2x_tensor_geometry*
 // ---- whole channels in one workgroup: which calls, which team -------------------
 // float only: the staged calls of double tensors are promised bit for bit, and here
 // the fp64 sums are added in another order (N 8, C 32, 33^3, double, 36 + 62 us, by teams
-// 32 + 45).  All tensors of the call lie alike, a row holds a vector, and offsets within a
+// 32 + 45; members that add what the staged workgroups add, in their order, would keep the
+// bits: not built).  All tensors of the call lie alike, a row holds a vector, and offsets within a
 // channel fit 30 bits.
 bool once_geometry(int num_samples, int num_channels, size_t spatial, std::initializer_list<const HostTensor*> ts,
                    OnceGeometry* g)
@@ -2638,7 +2643,11 @@ void issue_once(const G& g, const OnceForward<float>& a, hipStream_t st)
 template <int TEAM, int K, bool STREAM, typename G>
 void issue_once(const G& g, const OnceBackward<float>& a, hipStream_t st)
 {
-    constexpr int kInLds = TEAM * K > 8192 ? 9 : 0; // 144 of the 160 KB
+    // 144 of the 160 KB.  With 16 vectors a thread and nine of dy parked there the kernel still spills
+    // 4 registers (5 words of scratch a lane), 16 (9 words) where it clears the halo; against the
+    // two launches it remains the faster one: N 4, C 256, 112 x 112 with a halo, cleared, backward 47.5 ->
+    // 38.7 us, N 2, C 512, 30^3 97 -> 90, N 16, C 1024, 54 x 54 154 -> 142 (going round three sets of tensors).
+    constexpr int kInLds = TEAM * K > 8192 ? 9 : 0;
     bn_once_backward_kernel<float, TEAM, K, STREAM, kInLds><<<once_grid<TEAM>(g), once_block<TEAM>(), 0, st>>>(g, a);
 }
 

@@ -5,10 +5,11 @@
 // The two-launch kernels read x (backward: x and dy) twice, and the second launch
 // waits for the first; up to tens of megabytes both cost more than what has to be
 // moved.  Forward + backward, fp32, two launches each way -> one:
-//   N 128, C 1024, 7 x 7           52.1 -> 31.2 us      N 16, C 512, 14 x 14   22.1 -> 10.4
-//   N 16, C 256, 28 x 28           26.1 -> 13.6         N 8, C 64, 56 x 56     19.5 -> 15.0
-//   N 64, C 1024, 14 x 14          78.5 -> 49.4         N 4, C 512, 56 x 56    43.8 -> 19.7
-//   N 16, C 512, 7^3, halo of 1    54.9 -> 20.3         N 8, C 1024, 7 x 7     17.2 -> 9.5
+//   N 128, C 1024, 7 x 7           51.8 -> 25.3 us      N 16, C 512, 14 x 14   21.0 -> 9.8
+//   N 16, C 256, 28 x 28           25.4 -> 12.5         N 4, C 64, 56 x 56     16.5 -> 11.0
+//   N 64, C 1024, 14 x 14          78.2 -> 43.7         N 4, C 512, 56 x 56    43.4 -> 19.8
+//   N 16, C 512, 7^3, halo of 1    54.7 -> 19.3         N 8, C 1024, 7 x 7     17.0 -> 7.7
+// (one set of tensors over and over: up to 256 MB of it stay in the memory-side cache)
 //
 // A channel is as large as the registers of one CU allow: 512 KB, of which the
 // largest variants hold 320 KB forward, 256 KB and 128 KB of LDS backward.  Larger ones, and few, are for
