@@ -719,7 +719,7 @@ class HaloExchangeVirtual:
         neighbour's LHS receive buffer and vice versa.  With ``fused`` the strips
         move straight from tensor to tensor in one launch (where every rank has at
         least that much interior); the result is the same."""
-        if not fused:
+        if not fused and self._direct is not None and dim not in self._packed_since:
             self._packed_since += (dim,)
         self._issue(self._dim_launches(dim, width_rhs_send, width_rhs_recv, width_lhs_send, width_lhs_recv,
                                        is_reverse, skip_unpack, op, fused))

@@ -158,11 +158,13 @@ def test_strips_packed_since_an_exchange_are_not_packed_again():
         ts = packed._tensors(shape, locale, overlap, torch.float32, audit)
         xch = HaloExchangeVirtual(ts)
         xch.exchange()
-        xch.exchange_dim(0, 1, 1, 1, 1)
+        for _ in range(3):
+            xch.exchange_dim(0, 1, 1, 1, 1)
+        assert xch._packed_since == (0,)        # noted once, however often it is packed
         xch.exchange(fused=True)
         for dim in (0, 1):
             loads, stores = audit.counts(xch.recv_buffer(0, dim, capi.RHS))
-            assert (stores == 1).all() and (loads == (1 - dim)).all()
+            assert (stores == (3, 1)[dim]).all() and (loads == (3, 0)[dim]).all()
         ts[0].data = ts[0].data.clone()
         other = HaloExchangeVirtual(ts)
         other._direct = ((0,) * 4, False)      # exchanged when the tensors lay elsewhere
