@@ -5,10 +5,16 @@ One "step" is one pass of the path BASELINE.json's metric is quoted on:
   * 3-D batch-norm forward + backward on NCDHW 4 x 64 x 64^3 fp32 (config 3),
   * one full halo exchange (pack + unpack, 3 dimension phases, width 1) of a
     periodic 2 x 2 x 2 grid of virtual ranks, each N1 C32 128^3 fp32 (config 2).
-`value` is the algorithmic bytes of a step divided by its wall time, inputs
-resident in HBM.  Every BASELINE config, the exchange's phases and the
-follow-on operators are timed separately under "breakdown" (GPU time through
-HIP-graph replay, and the eager Python figure beside it where it differs).
+`value` is the bytes that the launches of a step have to move divided by its wall
+time, inputs resident in HBM: the batch-norm reads x and writes y, then reads x and
+dy and writes dx (it holds the channels in registers between its sums and its
+output), and every strip of the exchange is packed and unpacked, read and written
+each time (the hook that times its launches asks for that; without it an exchange
+goes straight from tensor to tensor).  "by_reference_passes" prices the same step by
+the passes of the reference's kernels, which read x (backward: x and dy) twice.
+Every BASELINE config, the exchange's phases and the follow-on operators are timed
+separately under "breakdown" (GPU time through HIP-graph replay, and the eager Python
+figure beside it where it differs), each by the bytes that its own launches move.
 
 Prints ONE JSON line.  `--gpus N` with N > 1 exits: this build runs on one GPU.
 """
@@ -27,6 +33,9 @@ if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0  # MI355X published HBM3E bandwidth
+# Times a batch-norm moves the elements of a tensor, forward and backward: holding the channels in
+# registers (x -> y; x, dy -> dx), and in the staged and the two-launch calls, which read x (x, dy) twice.
+BN_ONCE, BN_STAGED = (2, 3), (3, 5)
 SEED = 1234
 
 
@@ -543,7 +552,8 @@ def cpu_baseline(repeats: int = 5):
     tr = med(rows)
     configs["C5_shuffle_row_copy"] = entry(n5 * per_rank, n5 * field.size, tr,
                                            "all 4 ranks, forward direction, OpenMP row-copy path")
-    # the step the headline value is quoted on: C3 in full + C2 scaled to its 2-rank sample
+    # the step the headline value is quoted on, by the oracle's passes (the reference's): C3 in full + C2
+    # scaled to its 2-rank sample
     step_bytes = 8 * 67108864 * 4 + halo_bytes
     return {
         "value": step_bytes / (t3 + t2) / 1e9,
@@ -585,6 +595,8 @@ PMC_SOURCES_SHA = "3bcdabae02179b5c"
 PMC_COMMIT = "3387492"
 
 KERNEL_OF = {
+    "bn_forward": "bn_team_forward_kernel<float,512,16>",
+    "bn_backward": "bn_team_backward_kernel<float,512,8>",
     "bn_sums": "bn_sums_kernel<float,4> (+bn_finish_kernel<float,2>)",
     "bn_statistics": "bn_statistics_kernel<float>",
     "bn_apply": "bn_apply_kernel<float,4>",
@@ -600,7 +612,7 @@ KERNEL_OF = {
 
 
 # the sources of the kernels of the step (batch-norm and box copy), whose traffic PMC_TRAFFIC holds
-STEP_KERNEL_SOURCES = ("h2x_bn.hip", "h2x_bn_maps.hpp", "h2x_copy.hip", "h2x_copy_acc.hip", "h2x_copy_kernel.hpp", "h2x_device.hpp")
+STEP_KERNEL_SOURCES = ("h2x_bn.hip", "h2x_bn_maps.hpp", "h2x_bn_once.hpp", "h2x_bn_team.hpp", "h2x_copy.hip", "h2x_copy_acc.hip", "h2x_copy_kernel.hpp", "h2x_device.hpp")
 
 
 def kernel_sources_sha() -> str:
@@ -740,11 +752,11 @@ def main() -> int:
     bn3 = BatchNormWorkload((4, 64, 64, 64, 64), SEED + 3)
     halo = HaloWorkload(128, 32, SEED + 2)
     S3 = bn3.elems
-    bn_bytes = 8 * S3 * 4
-    step_bytes = bn_bytes + halo.bytes
+    step_bytes = sum(BN_ONCE) * S3 * 4 + halo.bytes
+    reference_bytes = sum(BN_STAGED) * S3 * 4 + halo.bytes
     step_elems = S3 + halo.elems
     face_bytes = halo.bytes // (6 * 16)  # one face of one rank, read + write (16 faces per dimension)
-    algo_bytes = {"bn_sums": S3 * 4, "bn_statistics": 0, "bn_apply": 2 * S3 * 4, "bn_backprop1": 2 * S3 * 4,
+    algo_bytes = {"bn_forward": BN_ONCE[0] * S3 * 4, "bn_backward": BN_ONCE[1] * S3 * 4, "bn_sums": S3 * 4, "bn_statistics": 0, "bn_apply": 2 * S3 * 4, "bn_backprop1": 2 * S3 * 4,
                   "bn_backprop2": 3 * S3 * 4}
     faces_per_launch = {}  # halo label -> faces in one launch (the exchange may split a phase)
 
@@ -774,13 +786,13 @@ def main() -> int:
     def step():
         """The timed step: the layer's own forward() and backward() (each one kernel
         that holds the channels in registers) and the exchange."""
-        bn3.forward()
-        bn3.backward()
+        timed("bn_forward", bn3.forward)
+        timed("bn_backward", bn3.backward)
         halo.run()
 
     def step_staged():
         """The same work with the staged batch-norm entry points (what a rank that all-reduces
-        between the stages runs), every launch labelled: the per-launch table."""
+        between the stages runs), every launch labelled, for the per-launch table."""
         timed("bn_sums", lambda: b.forward_stage1(bn3.x, bn3.mean, bn3.var, True))
         timed("bn_statistics", lambda: b.sums_to_statistics(nps, bn3.mean, bn3.var, bn3.rm, bn3.rv))
         timed("bn_apply", lambda: b.batch_normalization(bn3.x, bn3.mean, bn3.var, bn3.scale, bn3.bias, bn3.y))
@@ -798,23 +810,20 @@ def main() -> int:
         return tot
 
     # warm-up, with every launch bracketed by events: finds the dominant kernel
+    step()  # first-use allocations
     recording[0] = True
     for _ in range(max(args.warmup, 3)):
-        step_staged()
+        step()
     torch.cuda.synchronize()
     share0 = kernel_share(events)
     dominant = max(share0, key=share0.get)
-    events.clear()
-    step()  # the fused entry points once, untimed (first-use allocations)
-    torch.cuda.synchronize()
     events.clear()
     # parity gate of the step's two configurations, before the timed region
     parity = {"C3_bn3d_fwd_bwd": gate_batchnorm(bn3), "C2_halo_8ranks": gate_halo(halo)}
     torch.cuda.synchronize()
 
     # timed region: only the dominant kernel's launches carry events, and only in every
-    # EVENT_EVERY-th step (a pair of timing events costs the stream 2-3 us: bracketing all four
-    # launches of every step would take 3 % off the figure the events are there to explain)
+    # EVENT_EVERY-th step (a pair of timing events costs the stream 2-3 us)
     only[0] = {l for l, k in KERNEL_OF.items() if k == dominant}
     t0 = time.perf_counter()
     for i in range(args.steps):
@@ -828,10 +837,11 @@ def main() -> int:
     dominant_events = dict(events)
     events.clear()
 
-    # a second, fully instrumented pass for the per-launch table
+    # a second, fully instrumented pass for the per-launch table, and the staged calls
     only[0] = None
-    for _ in range(args.steps):
-        step_staged()
+    for one in (step, step_staged):
+        for _ in range(args.steps):
+            one()
     torch.cuda.synchronize()
     recording[0] = False
     halo.xch.launch_hook = None
@@ -908,23 +918,25 @@ def main() -> int:
                     "timing": "HIP-graph replay of (512 MB read-only flush, call) pairs minus the replay of the "
                               "flushes alone (GPU time, caches cold)"}
 
-        breakdown["C3_bn3d_fwd"] = entry(3 * S3 * 4, S3, bn3.forward)
-        breakdown["C3_bn3d_bwd"] = entry(5 * S3 * 4, S3, bn3.backward)
-        breakdown["C3_bn3d_fwd_bwd"] = entry(8 * S3 * 4, S3, lambda: (bn3.forward(), bn3.backward()), inner=2)
-        breakdown["C3_bn3d_fwd_bwd_cold"] = cold_entry(8 * S3 * 4, S3, lambda: (bn3.forward(), bn3.backward()), inner=1)
+        breakdown["C3_bn3d_fwd"] = entry(BN_ONCE[0] * S3 * 4, S3, bn3.forward)
+        breakdown["C3_bn3d_bwd"] = entry(BN_ONCE[1] * S3 * 4, S3, bn3.backward)
+        breakdown["C3_bn3d_fwd_bwd"] = entry(sum(BN_ONCE) * S3 * 4, S3, lambda: (bn3.forward(), bn3.backward()), inner=2)
+        breakdown["C3_bn3d_fwd_bwd_cold"] = cold_entry(sum(BN_ONCE) * S3 * 4, S3,
+                                                       lambda: (bn3.forward(), bn3.backward()), inner=1)
         bn3.bn.fuse_local = False
         bn3.forward(), bn3.backward()
         parity["C3_bn3d_fwd_bwd_staged"] = gate_batchnorm(bn3)
-        breakdown["C3_bn3d_fwd_bwd_staged"] = entry(8 * S3 * 4, S3, lambda: (bn3.forward(), bn3.backward()), inner=2)
+        breakdown["C3_bn3d_fwd_bwd_staged"] = entry(sum(BN_STAGED) * S3 * 4, S3, lambda: (bn3.forward(), bn3.backward()), inner=2)
         bn3.bn.fuse_local = True
-        breakdown["C2_halo_8ranks"] = entry(halo.bytes, halo.elems, halo.run, inner=2)
+        # without a hook the exchange goes straight from tensor to tensor: every strip read and written once
+        breakdown["C2_halo_8ranks"] = entry(halo.bytes // 2, halo.elems // 2, halo.run, inner=2)
         for d, name in enumerate(("dim0_W", "dim1_H", "dim2_D")):
             ov = [1 if k == d else 0 for k in range(5)]
             fn = lambda ov=ov: halo.xch.exchange(ov, ov, ov, ov)
             breakdown[f"C2_halo_{name}"] = entry(halo.bytes // 3, halo.elems // 3, fn)
             breakdown[f"C2_halo_{name}_cold"] = cold_entry(halo.bytes // 3, halo.elems // 3, fn)
-        breakdown["C2_halo_8ranks_cold"] = cold_entry(halo.bytes, halo.elems, halo.run, inner=1)
-        # the same exchange as tensor-to-tensor transfers (no buffers): half the bytes per strip
+        breakdown["C2_halo_8ranks_cold"] = cold_entry(halo.bytes // 2, halo.elems // 2, halo.run, inner=1)
+        # the same exchange asked for as tensor-to-tensor transfers
         for t in halo.ranks:          # poison the halos: the fused exchange has to fill every cell again
             keep = t.interior_view().clone()
             t.real_view().fill_(float("nan"))
@@ -947,12 +959,12 @@ def main() -> int:
                 halo.xch.clear_halo(d)
 
         breakdown["C2_clear_halo_8ranks"] = entry(halo.bytes // 4, halo.elems // 2, clear_all, inner=2)
-        # the same strips cleared by one batched call (3 launches instead of 24)
+        # the same strips cleared by one call (one launch instead of 24)
         breakdown["C2_clear_halos_batched_8ranks"] = entry(halo.bytes // 4, halo.elems // 2, halo.xch.clear_halos,
                                                           inner=2)
-        # pack: read + write; accumulating unpack: read buffer, read + write tensor -> 5/4 of the forward bytes
+        # tensor to tensor as well: every strip read, the cells it is added to read and written
         breakdown["C2_halo_reverse_sum_8ranks"] = entry(
-            halo.bytes * 5 // 4, halo.elems,
+            halo.bytes * 3 // 4, halo.elems // 2,
             lambda: halo.xch.exchange(is_reverse=True, op=HaloExchangeAccumOp.SUM), inner=2)
         # tensor::Transform / ReduceSum at the config 3 shape: scale in place (read + write), copy into a
         # second tensor (read + write), per-channel sums and sums of squares (one read each)
@@ -970,31 +982,31 @@ def main() -> int:
         # what a convolution does before it runs (convolution.hpp:400-411): clear the halos, exchange.
         # Bytes: the exchange's; the clearing is overhead.  On the periodic grid every strip is overwritten
         # by the exchange, on the open one half of them.
-        breakdown["C2_clear_then_exchange"] = entry(halo.bytes, halo.elems,
+        breakdown["C2_clear_then_exchange"] = entry(halo.bytes // 2, halo.elems // 2,
                                                     lambda: (halo.xch.clear_halos(), halo.run()), inner=2)
         breakdown["C2_clear_unfilled_then_exchange"] = entry(
-            halo.bytes, halo.elems, lambda: (halo.xch.clear_halos(only_unfilled=True), halo.run()), inner=2)
+            halo.bytes // 2, halo.elems // 2, lambda: (halo.xch.clear_halos(only_unfilled=True), halo.run()), inner=2)
         yard_x, yard_y = bn3.x.data, bn3.y.data
         breakdown["yardstick_torch_copy_268MB"] = entry(2 * S3 * 4, S3, lambda: yard_y.copy_(yard_x), eager=False)
         del bn3, halo, b, yard_x, yard_y
         torch.cuda.empty_cache()
         # the same on an open (non-periodic) 2 x 2 x 2 grid: every rank has a neighbour on 3 of its 6 sides
         halo_open = HaloWorkload(128, 32, SEED + 2, periodic=False)
-        breakdown["C2open_clear_then_exchange"] = entry(halo_open.bytes // 2, halo_open.elems // 2,
+        breakdown["C2open_clear_then_exchange"] = entry(halo_open.bytes // 4, halo_open.elems // 4,
                                                         lambda: (halo_open.xch.clear_halos(), halo_open.run()), inner=2)
         breakdown["C2open_clear_unfilled_then_exchange"] = entry(
-            halo_open.bytes // 2, halo_open.elems // 2,
+            halo_open.bytes // 4, halo_open.elems // 4,
             lambda: (halo_open.xch.clear_halos(only_unfilled=True), halo_open.run()), inner=2)
         del halo_open
         torch.cuda.empty_cache()
-        # strided batch-norm: the config 3 shard with a halo of 1 on all three spatial dimensions
+        # batch-norm of a haloed tensor: the config 3 shard with a halo of 1 on all three spatial dimensions
         bn3h = BatchNormWorkload((4, 64, 64, 64, 64), SEED + 6, overlap=1)
         bn3h.forward(), bn3h.backward()
         parity["C3_bn3d_haloed_fwd_bwd"] = gate_batchnorm(bn3h)
-        breakdown["C3_bn3d_haloed_fwd_bwd"] = entry(8 * bn3h.elems * 4, bn3h.elems,
+        breakdown["C3_bn3d_haloed_fwd_bwd"] = entry(sum(BN_ONCE) * bn3h.elems * 4, bn3h.elems,
                                                     lambda: (bn3h.forward(), bn3h.backward()), inner=2)
-        # the same shard with clear_output_halo: normalise and the input gradient walk the whole real
-        # tensors in aligned vectors and leave the halos of y and dx cleared (what the convolution that
+        # the same shard with clear_output_halo: the passes walk the whole real tensors in aligned
+        # vectors and leave the halos of y and dx cleared (what the convolution that
         # follows would do with a separate clear_halo per dimension); the gate also looks at the halos
         bn3h.bn.clear_output_halo = True
         for t in (bn3h.y, bn3h.dx):
@@ -1006,16 +1018,16 @@ def main() -> int:
             nonzero_real, nonzero_interior = int((t.real_view() != 0).sum()), int((t.interior_view() != 0).sum())
             _gate(nonzero_real == nonzero_interior and not bool(torch.isnan(t.real_view()).any()),
                   f"clearing batch-norm: halo of {what} is not zero")
-        breakdown["C3_bn3d_haloed_clearing_fwd_bwd"] = entry(8 * bn3h.elems * 4, bn3h.elems,
+        breakdown["C3_bn3d_haloed_clearing_fwd_bwd"] = entry(sum(BN_ONCE) * bn3h.elems * 4, bn3h.elems,
                                                              lambda: (bn3h.forward(), bn3h.backward()), inner=2)
         del bn3h
         torch.cuda.empty_cache()
-        # short segments (the last stage of a ResNet): a workgroup serves a window of whole channels
+        # short segments (the last stage of a ResNet): a workgroup holds a channel in registers
         bn7 = BatchNormWorkload((256, 2048, 7, 7), SEED + 7)
         bn7.forward(), bn7.backward()
         parity["bn2d_7x7_N256_C2048"] = gate_batchnorm(bn7)
-        breakdown["bn2d_7x7_N256_C2048_fwd"] = entry(3 * bn7.elems * 4, bn7.elems, bn7.forward)
-        breakdown["bn2d_7x7_N256_C2048_bwd"] = entry(5 * bn7.elems * 4, bn7.elems, bn7.backward)
+        breakdown["bn2d_7x7_N256_C2048_fwd"] = entry(BN_ONCE[0] * bn7.elems * 4, bn7.elems, bn7.forward)
+        breakdown["bn2d_7x7_N256_C2048_bwd"] = entry(BN_ONCE[1] * bn7.elems * 4, bn7.elems, bn7.backward)
         del bn7
         torch.cuda.empty_cache()
         # configs 1 and 4 fit in the memory-side cache: warm = back to back, cold = after a 512 MB read
@@ -1023,16 +1035,17 @@ def main() -> int:
         bn1 = BatchNormWorkload((8, 64, 56, 56), SEED + 1)
         bn1.forward()
         parity["C1_bn2d_fwd"] = gate_batchnorm(bn1, backward=False)
-        breakdown["C1_bn2d_fwd"] = entry(3 * bn1.elems * 4, bn1.elems, bn1.forward)
+        breakdown["C1_bn2d_fwd"] = entry(BN_ONCE[0] * bn1.elems * 4, bn1.elems, bn1.forward)
         med, mn = _time_events_cold(bn1.forward, flush, it, wu)
         breakdown["C1_bn2d_fwd_cold"] = {
-            "bytes": 3 * bn1.elems * 4, "ms_median": med, "ms_min": mn, "GB/s": _gbs(3 * bn1.elems * 4, med),
-            "frac_of_peak": _gbs(3 * bn1.elems * 4, med) / HBM_PEAK_GBS,
-            "timing": "events around one eager call after a cache-evicting read (2 launches)"}
+            "bytes": BN_ONCE[0] * bn1.elems * 4, "ms_median": med, "ms_min": mn,
+            "GB/s": _gbs(BN_ONCE[0] * bn1.elems * 4, med),
+            "frac_of_peak": _gbs(BN_ONCE[0] * bn1.elems * 4, med) / HBM_PEAK_GBS,
+            "timing": "events around one eager call after a cache-evicting read"}
         bn1.bn.fuse_local = False
         bn1.forward()
         parity["C1_bn2d_fwd_staged"] = gate_batchnorm(bn1, backward=False)
-        breakdown["C1_bn2d_fwd_staged"] = entry(3 * bn1.elems * 4, bn1.elems, bn1.forward)
+        breakdown["C1_bn2d_fwd_staged"] = entry(BN_STAGED[0] * bn1.elems * 4, bn1.elems, bn1.forward)
         del bn1
         sm = SoftmaxWorkload((16, 21, 256, 256), SEED + 4)
         sm.forward(), sm.backward()
@@ -1058,28 +1071,29 @@ def main() -> int:
         torch.cuda.empty_cache()
         shf = ShuffleWorkload((128, 128, 64, 32), SEED + 5)
         parity["C5_shuffle"] = gate_shuffle(shf)
-        breakdown["C5_shuffle_fwd"] = entry(4 * shf.elems * 4, shf.elems, shf.forward)
-        breakdown["C5_shuffle_bwd"] = entry(4 * shf.elems * 4, shf.elems, shf.backward)
-        breakdown["C5_shuffle_round_trip"] = entry(8 * shf.elems * 4, 2 * shf.elems,
+        # straight from tensor to tensor: every element read and written once a direction
+        breakdown["C5_shuffle_fwd"] = entry(2 * shf.elems * 4, shf.elems, shf.forward)
+        breakdown["C5_shuffle_bwd"] = entry(2 * shf.elems * 4, shf.elems, shf.backward)
+        breakdown["C5_shuffle_round_trip"] = entry(4 * shf.elems * 4, 2 * shf.elems,
                                                    lambda: (shf.forward(), shf.backward()), inner=2)
-        breakdown["C5_shuffle_fwd_cold"] = cold_entry(4 * shf.elems * 4, shf.elems, shf.forward)
-        breakdown["C5_shuffle_bwd_cold"] = cold_entry(4 * shf.elems * 4, shf.elems, shf.backward)
-        breakdown["C5_shuffle_round_trip_cold"] = cold_entry(8 * shf.elems * 4, 2 * shf.elems,
+        breakdown["C5_shuffle_fwd_cold"] = cold_entry(2 * shf.elems * 4, shf.elems, shf.forward)
+        breakdown["C5_shuffle_bwd_cold"] = cold_entry(2 * shf.elems * 4, shf.elems, shf.backward)
+        breakdown["C5_shuffle_round_trip_cold"] = cold_entry(4 * shf.elems * 4, 2 * shf.elems,
                                                              lambda: (shf.forward(), shf.backward()), inner=1)
         del shf
         torch.cuda.empty_cache()
-        # the spatial side with a halo of 1 (what a convolution behind the shuffle needs): the unpack
-        # writes rows of 64 floats into rows of 66, the backward pack reads them
+        # the spatial side with a halo of 1 (what a convolution behind the shuffle needs): rows of 64
+        # floats go into rows of 66, and back
         shfh = ShuffleWorkload((128, 128, 64, 32), SEED + 5, dst_overlap=1)
         parity["C5_shuffle_haloed_dst"] = gate_shuffle(shfh)
-        breakdown["C5_shuffle_haloed_dst_round_trip"] = entry(8 * shfh.elems * 4, 2 * shfh.elems,
+        breakdown["C5_shuffle_haloed_dst_round_trip"] = entry(4 * shfh.elems * 4, 2 * shfh.elems,
                                                               lambda: (shfh.forward(), shfh.backward()), inner=2)
         del shfh
         torch.cuda.empty_cache()
-        # the same tensor between 16 ranks: 256 boxes a direction, one launch each for pack and unpack
+        # the same tensor between 16 ranks: 256 boxes a direction, in one launch
         shf16 = ShuffleWorkload((128, 128, 64, 32), SEED + 5, ranks=16, grid=(4, 4))
         parity["C5_shuffle_16ranks"] = gate_shuffle(shf16)
-        breakdown["C5_shuffle_16ranks_round_trip"] = entry(8 * shf16.elems * 4, 2 * shf16.elems,
+        breakdown["C5_shuffle_16ranks_round_trip"] = entry(4 * shf16.elems * 4, 2 * shf16.elems,
                                                            lambda: (shf16.forward(), shf16.backward()), inner=2)
         del shf16, evict, evict_t, evict_stat
         torch.cuda.empty_cache()
@@ -1105,6 +1119,7 @@ def main() -> int:
             "seed": SEED,
         },
         "frac_of_hbm_peak": value / HBM_PEAK_GBS,
+        "by_reference_passes": {"step_bytes": reference_bytes, "GB/s": _gbs(reference_bytes, ms_per_step)},
         "elements_per_s": step_elems / (ms_per_step * 1e-3),
         "kernel_sources": sources_sha,
         "parity_gate": "ok",
