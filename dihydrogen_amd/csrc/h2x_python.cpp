@@ -6,8 +6,8 @@
 // one METH_FASTCALL function whose argument conversions are generated from its
 // C signature: integers and floats as they are, and for a pointer None, an
 // address, or any object with a data_ptr() method (a torch tensor).  Every
-// function returns the status of the C function.  The GIL is released during
-// the call, as ctypes does.
+// function returns what the C function returns (a status or a size).  The GIL
+// is released during the call, as ctypes does.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -63,7 +63,7 @@ bool convert(PyObject* o, P* out)
 template <auto F>
 struct Entry;
 
-template <typename... P, int (*F)(P...)>
+template <typename R, typename... P, R (*F)(P...)>
 struct Entry<F>
 {
     template <size_t... I>
@@ -72,11 +72,14 @@ struct Entry<F>
         std::tuple<P...> v;
         if (!(convert(args[I], &std::get<I>(v)) && ...))
             return nullptr;
-        int status;
+        R result;
         Py_BEGIN_ALLOW_THREADS
-        status = F(std::get<I>(v)...);
+        result = F(std::get<I>(v)...);
         Py_END_ALLOW_THREADS
-        return PyLong_FromLong(status);
+        if constexpr (std::is_signed<R>::value)
+            return PyLong_FromLong(result);
+        else
+            return PyLong_FromSize_t(result);
     }
 
     static PyObject* fastcall(PyObject*, PyObject* const* args, Py_ssize_t nargs)
@@ -107,6 +110,8 @@ PyMethodDef s_methods[] = {H2X_ENTRY(h2x_bn_channel_sums_and_sqsums),
                            H2X_ENTRY(h2x_bn_backprop2_clearing),
                            H2X_ENTRY(h2x_bn_forward_local),
                            H2X_ENTRY(h2x_bn_backward_local),
+                           H2X_ENTRY(h2x_bn_team_state_needed),
+                           H2X_ENTRY(h2x_bn_team_state_needed_clearing),
                            H2X_ENTRY(h2x_bn_forward_once),
                            H2X_ENTRY(h2x_bn_forward_clearing),
                            H2X_ENTRY(h2x_bn_backward_clearing),

@@ -26,6 +26,8 @@ def _buffer_of(stream: Optional[torch.cuda.Stream], *args, **kwargs) -> torch.Te
     """A _device_buffer for launches on `stream` (None: on the current one).  It is made on that
     stream: what clears it comes before the launches that use it, and whoever gets its memory when
     the layer gives it back comes after them.  On another stream neither would be ordered."""
+    if stream is None:
+        return _device_buffer(*args, **kwargs)
     with torch.cuda.stream(stream):
         return _device_buffer(*args, **kwargs)
 

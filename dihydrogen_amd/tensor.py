@@ -188,12 +188,12 @@ class Layout:
     @_once
     def team_state_bytes(self) -> int:
         """State for batch-norm calls on tensors like this (0: none is for teams of workgroups)."""
-        return capi.load().h2x_bn_team_state_needed(self.dtype, self.samples, self.geometry)
+        return capi.calls().h2x_bn_team_state_needed(self.dtype, self.samples, self.geometry_address)
 
     @_once
     def clearing_team_state_bytes(self) -> int:
         """The same for calls that clear their output's halo."""
-        return capi.load().h2x_bn_team_state_needed_clearing(self.dtype, self.haloed_geometry)
+        return capi.calls().h2x_bn_team_state_needed_clearing(self.dtype, self.haloed_geometry_address)
 
     @_once
     def haloed_geometry(self):

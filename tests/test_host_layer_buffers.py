@@ -17,8 +17,10 @@ class _Stream:
 class _Calls:
     """Entry points that launch nothing and say so."""
 
+    native = capi.calls()
+
     def __getattr__(self, name):
-        return lambda *args: 0
+        return getattr(self.native, name) if "_needed" in name else lambda *args: 0
 
 
 @pytest.fixture
