@@ -632,11 +632,11 @@ class HaloExchangeVirtual:
         long as the tensors have not been written since; the cells of a strip that a later dimension's
         phase writes, where strips of two dimensions cross, hold what that phase left."""
         self._buffers_wanted = True
+        written = self._direct is not None or (rank, dim, side) not in self._recv
         self._pack_what_was_exchanged()
-        made = (rank, dim, side) not in self._recv
         buffer = self._receive_buffer(rank, dim, side)
-        if made and self.stream is not None and buffer.is_cuda:
-            # what the caller does with it on the current stream comes after it was cleared
+        if written and self.stream is not None and buffer.is_cuda:
+            # what the caller does with it on the current stream comes after it was cleared or packed
             torch.cuda.current_stream().wait_stream(self.stream)
         return buffer
 

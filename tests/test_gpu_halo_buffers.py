@@ -39,3 +39,22 @@ def test_buffers_after_an_exchange(case, is_reverse):
                 same.narrow(axis, n - first - w, w).fill_(False)
         same = same.ravel()
         assert torch.equal(got[same], want[same]), (r, dim, side)
+
+
+def test_buffers_packed_on_a_stream_of_the_exchange_are_there_for_the_current_one():
+    """Asked for after the exchange's own stream has been waited for: what is packed then is waited for as well."""
+    import torch
+    from dihydrogen_amd import capi
+    from dihydrogen_amd.layers import HaloExchangeVirtual
+    side = torch.cuda.Stream()
+    ts = _tensors((512, 300, 32, 2), (2, 1, 1, 1), None, (1, 0, 0, 0), torch.float32, 3)
+    want = ts[0].interior_view()[..., -1].flatten().clone()
+    torch.cuda.synchronize()
+    xch = HaloExchangeVirtual(ts, stream=side)
+    xch.exchange()
+    side.synchronize()
+    busy = torch.empty(1 << 26, device="cuda")
+    with torch.cuda.stream(side):
+        for _ in range(20):     # the packing waits behind some milliseconds
+            busy.normal_()
+    assert torch.equal(xch.recv_buffer(1, 0, capi.LHS), want)

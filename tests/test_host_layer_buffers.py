@@ -115,3 +115,29 @@ def test_dense_tensors_of_other_extents_go_to_the_calls_that_take_them(made, mon
         bn.backward(x, y, *[x.data] * 7, x)
         assert called == ["h2x_bn_forward_" + forward, "h2x_bn_backward_" + backward]
         called.clear()
+
+
+def test_what_is_packed_on_a_stream_of_its_own_is_waited_for(made, monkeypatch):
+    """recv_buffer() after an exchange straight from tensor to tensor: its caller's stream waits for the packing."""
+    import torch
+    waited = []
+
+    class Current:
+        def wait_stream(self, stream):
+            waited.append(stream)
+
+    monkeypatch.setattr(layers.torch.cuda, "current_stream", Current)
+    monkeypatch.setattr(layers, "_share_a_gpu", lambda tensors: True)
+
+    class OnGpu(torch.Tensor):
+        is_cuda = True
+
+    monkeypatch.setattr(layers, "_device_buffer", lambda count, dtype, *args, **kwargs: torch.zeros(count, dtype=dtype).as_subclass(OnGpu))
+    ranks = _tensors([8, 6, 2, 1], Distribution.make_overlapped_distribution([2, 1, 1, 1], [1, 0, 0, 0]), 2)
+    stream = _Stream()
+    xch = HaloExchangeVirtual(ranks, stream=stream)
+    xch.exchange()
+    xch.recv_buffer(0, 0, capi.RHS)
+    assert waited == [stream]
+    xch.recv_buffer(1, 0, capi.LHS)     # packed with the first
+    assert waited == [stream]
