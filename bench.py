@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the MI355X DistConv hot path (one GPU).
 
-One "step" is one pass of the path BASELINE.json's metric is quoted on:
+One "step" is one pass of the path that the metric is quoted on:
   * 3-D batch-norm forward + backward on NCDHW 4 x 64 x 64^3 fp32 (config 3),
   * one full halo exchange (pack + unpack, 3 dimension phases, width 1) of a
     periodic 2 x 2 x 2 grid of virtual ranks, each N1 C32 128^3 fp32 (config 2).
@@ -12,7 +12,7 @@ output), and every strip of the exchange is packed and unpacked, read and writte
 each time (the hook that times its launches asks for that; without it an exchange
 goes straight from tensor to tensor).  "by_reference_passes" prices the same step by
 the passes of the reference's kernels, which read x (backward: x and dy) twice.
-Every BASELINE config, the exchange's phases and the follow-on operators are timed
+Every configuration (C1 to C5), the exchange's phases and the follow-on operators are timed
 separately under "breakdown" (GPU time through HIP-graph replay, and the eager Python
 figure beside it where it differs), each by the bytes that its own launches move.
 
@@ -445,7 +445,7 @@ def cpu_baseline(repeats: int = 5):
     """The CPU oracle (this repository's restatement of the reference kernels:
     the reference has no CPU implementation of batch-norm, softmax or halo
     packing, and its CPU shuffler is restated too) timed on the host cores, per
-    BASELINE config, on bounded samples that are stated with each figure."""
+    configuration, on bounded samples that are stated with each figure."""
     import numpy as np
     import oracle
     from oracle import geometry as G
@@ -1083,6 +1083,8 @@ def main() -> int:
         breakdown["C5_shuffle_bwd_cold"] = cold_entry(2 * shf.elems * 4, shf.elems, shf.backward)
         breakdown["C5_shuffle_round_trip_cold"] = cold_entry(4 * shf.elems * 4, 2 * shf.elems,
                                                              lambda: (shf.forward(), shf.backward()), inner=1)
+        breakdown["C5_shuffle_round_trip_cold"]["note"] = (
+            "the second half finds part of what the first has written in the memory-side cache: not a rate of HBM")
         del shf
         torch.cuda.empty_cache()
         # the spatial side with a halo of 1 (what a convolution behind the shuffle needs): rows of 64

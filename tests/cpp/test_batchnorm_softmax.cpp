@@ -323,7 +323,7 @@ int main()
         DISTCONV_CHECK_HIP(hipStreamDestroy(a));
         DISTCONV_CHECK_HIP(hipStreamDestroy(b));
     }
-    errors += test_bn(Shape({56, 56, 64, 8}));
+    errors += test_bn(Shape({56, 56, 64, 8}));   // 2-D batch-norm of a small batch
     errors += test_bn(Shape({5, 7, 3, 2}));
     errors += test_bn(Shape({16, 16, 16, 8, 4})); // 5-D
     errors += test_softmax(Shape({64, 64, 21, 4}));

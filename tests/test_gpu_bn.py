@@ -16,7 +16,7 @@ TOL = 1e-5
 
 CASES = [
     # (N, C, spatial dims...) numpy order
-    (8, 64, 56, 56),
+    (8, 64, 56, 56),        # 2-D activations of a small batch
     (2, 3, 4, 5),           # tiny, spatial % 4 == 0
     (2, 3, 5, 7),           # scalar path (spatial % 4 != 0)
     (3, 5, 3, 4, 5),        # 5-D

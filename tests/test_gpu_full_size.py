@@ -1,4 +1,4 @@
-"""GPU parity at the full sizes of BASELINE.json's configurations.
+"""GPU parity at the full sizes of the benchmark's configurations.
 
 Batch-norm (configs 1 and 3) and softmax (config 4) are compared with the
 oracle in full (it finishes in seconds); halo (config 2) and shuffle (config 5)

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-5
 
 CASES = [
-    (16, 21, 64, 64),     # BASELINE config 4 at reduced spatial size (full size in test_gpu_full_size.py)
+    (16, 21, 64, 64),     # a segmentation head at reduced spatial size (full size in test_gpu_full_size.py)
     (2, 21, 7, 9),        # scalar path
     (3, 4, 8, 8),
     (2, 1, 4, 4),         # one channel
