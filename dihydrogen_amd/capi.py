@@ -212,6 +212,7 @@ SIGNATURES = {
                                               c_void_p]),
     "h2x_bn_team_state_bytes": (c_size_t, [c_int]),
     "h2x_bn_team_state_needed": (c_size_t, [c_int, c_int, POINTER(TensorGeometry)]),
+    "h2x_bn_ordered_state_needed": (c_size_t, [c_int, POINTER(TensorGeometry)]),
     "h2x_bn_team_state_needed_clearing": (c_size_t, [c_int, POINTER(HaloedGeometry)]),
     "h2x_bn_forward_once": (c_int, [c_int, c_int, POINTER(TensorGeometry), POINTER(TensorGeometry), c_void_p,
                                     c_void_p, c_void_p, c_size_t, c_double, c_double, c_void_p, c_void_p,
@@ -228,6 +229,8 @@ SIGNATURES = {
                                      c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_double, c_void_p, c_uint32,
                                      c_void_p]),
     "h2x_bn_audit_once": (c_int, [c_int, POINTER(TensorGeometry), c_uint32, c_void_p, c_void_p, c_size_t]),
+    "h2x_bn_audit_ordered": (c_int, [c_int, POINTER(TensorGeometry), c_int, c_uint32, c_void_p, c_void_p, c_void_p,
+                                     c_size_t]),
     "h2x_bn_batch_normalization_clearing": (c_int, [c_int, POINTER(HaloedGeometry), c_void_p, c_void_p, c_void_p,
                                                     c_void_p, c_void_p, c_void_p, c_double, c_void_p]),
     "h2x_bn_backprop2_clearing": (c_int, [c_int, c_size_t, POINTER(HaloedGeometry), c_void_p, c_void_p, c_void_p,

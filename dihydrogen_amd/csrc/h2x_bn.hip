@@ -1352,6 +1352,8 @@ __global__ __launch_bounds__(kBlockSize) void bn_backprop2_short_kernel(
 // ---- whole channels in several workgroups: one launch ---------------------------
 #include "h2x_bn_team.hpp"
 
+#include "h2x_bn_ordered.hpp"
+
 // ---- host side ---------------------------------------------------------------
 
 template <typename T>
@@ -1466,8 +1468,8 @@ int strided_tensor(const h2x_tensor_geometry* g, const void* p, int num_samples,
 // the one before it (N 16, C 64, 57 x 57: forward 23 -> 15 us against element by element).
 constexpr size_t kMinUnalignedSegment = 256;
 
-template <typename T>
-int common_vector(std::initializer_list<const HostTensor*> ts, bool* strided)
+template <typename T, typename H> // H: HostTensor or const HostTensor
+int common_vector(std::initializer_list<H*> ts, bool* strided)
 {
     const int full = full_vec<T>();
     *strided = false;
@@ -1826,6 +1828,49 @@ int zero_outputs(std::initializer_list<void*> outs, int num_channels, hipStream_
     return issued();
 }
 
+// How a long-segment reduction over tensors `ts` (which it sets up for the launch) is cut: into
+// units of whole tiles, which `groups` workgroups a channel take in turn.
+struct ReductionPlan
+{
+    bool folded, strided;
+    int vw;
+    int num_samples;
+    size_t spatial;
+    Chunking ch;
+    size_t units, groups;
+    int groups_max;
+};
+
+// unroll: vectors of a tile a thread.  Units of doubles are tiles of kUnroll vectors in both directions, which
+// the kernels that read once keep in registers (h2x_bn_ordered.hpp).
+template <typename T>
+int plan_reduction(int num_samples, int num_channels, size_t spatial, std::initializer_list<HostTensor*> ts, int unroll,
+                   ReductionPlan* p)
+{
+    p->folded = fold_samples(&num_samples, &spatial, ts);
+    bool any = false;
+    for (const HostTensor* t : ts)
+        any = any || t->strided;
+    if (spatial >= (1ull << 31) && any)
+        return H2X_ERR_TOO_LARGE;
+    p->vw = common_vector<T>(ts, &p->strided);
+    if (p->strided && p->vw > 1)
+        spatial = pad_rows<T>(ts, spatial);
+    if (spatial >= (1ull << 31) && p->strided)
+        return H2X_ERR_TOO_LARGE;
+    p->num_samples = num_samples;
+    p->spatial = spatial;
+    p->groups_max = max_groups_per_channel(num_channels);
+    const int budget = reduction_groups_per_channel(num_channels, p->strided);
+    const size_t tile = static_cast<size_t>(kBlockSize) * p->vw * (sizeof(T) == 8 ? kUnroll : unroll);
+    p->ch = make_chunking(spatial, num_samples, budget, tile, tile);
+    p->units = static_cast<size_t>(p->ch.chunks_per_seg) * num_samples;
+    if (p->units > 0xffffffffull || num_channels > 65535)
+        return H2X_ERR_TOO_LARGE;
+    p->groups = std::min<size_t>(p->units, budget);
+    return H2X_SUCCESS;
+}
+
 // `fused_out` non-null: the caller finishes the reduction itself (a fused
 // consumer kernel): every workgroup stores partials, no finishing launch.
 template <typename T>
@@ -1868,28 +1913,21 @@ int sums_impl(int num_samples, int num_channels, size_t spatial, const HostTenso
         return issued();
     }
     HostTensor tx = tx_in;
-    const bool folded = fold_samples(&num_samples, &spatial, {&tx});
-    if (spatial >= (1ull << 31) && tx.strided)
-        return H2X_ERR_TOO_LARGE;
-    bool strided;
-    const int vw = common_vector<T>({&tx}, &strided);
-    if (strided && vw > 1)
-        spatial = pad_rows<T>({&tx}, spatial);
-    if (spatial >= (1ull << 31) && strided)
-        return H2X_ERR_TOO_LARGE;
-    const int gmax = max_groups_per_channel(num_channels);
-    const int budget = reduction_groups_per_channel(num_channels, strided);
-    const size_t tile = static_cast<size_t>(kBlockSize) * vw * kUnroll;
-    const Chunking ch = make_chunking(spatial, num_samples, budget, tile, tile);
-    const size_t units = static_cast<size_t>(ch.chunks_per_seg) * num_samples;
-    if (units > 0xffffffffull || num_channels > 65535)
-        return H2X_ERR_TOO_LARGE;
-    const size_t groups = std::min<size_t>(units, budget);
+    ReductionPlan plan;
+    const int err = plan_reduction<T>(num_samples, num_channels, spatial, {&tx}, kUnroll, &plan);
+    if (err)
+        return err;
+    const bool strided = plan.strided;
+    const int vw = plan.vw, gmax = plan.groups_max;
+    const size_t units = plan.units, groups = plan.groups;
+    const Chunking& ch = plan.ch;
+    num_samples = plan.num_samples;
+    spatial = plan.spatial;
     double* partials = static_cast<double*>(workspace);
     const dim3 grid(static_cast<unsigned int>(groups), num_channels);
     LaunchRecord rec = long_record(kKernelSums, strided, vw, grid, num_samples, num_channels,
                                    spatial, ch, {&tx}, false);
-    rec.folded = folded;
+    rec.folded = plan.folded;
     rec.num_units = static_cast<unsigned int>(units);
     rec.num_sums = 2;
     rec.groups_max = gmax;
@@ -2067,28 +2105,21 @@ int backprop1_impl(int num_samples, int num_channels, size_t spatial, const Host
         return issued();
     }
     HostTensor tx = tx_in, td = td_in;
-    const bool folded = fold_samples(&num_samples, &spatial, {&tx, &td});
-    if (spatial >= (1ull << 31) && (tx.strided || td.strided))
-        return H2X_ERR_TOO_LARGE;
-    bool strided;
-    const int vw = common_vector<T>({&tx, &td}, &strided);
-    if (strided && vw > 1)
-        spatial = pad_rows<T>({&tx, &td}, spatial);
-    if (spatial >= (1ull << 31) && strided)
-        return H2X_ERR_TOO_LARGE;
-    const int gmax = max_groups_per_channel(num_channels);
-    const int budget = reduction_groups_per_channel(num_channels, strided);
-    const size_t tile = static_cast<size_t>(kBlockSize) * vw * (kUnroll / 2);
-    const Chunking ch = make_chunking(spatial, num_samples, budget, tile, tile);
-    const size_t units = static_cast<size_t>(ch.chunks_per_seg) * num_samples;
-    if (units > 0xffffffffull || num_channels > 65535)
-        return H2X_ERR_TOO_LARGE;
-    const size_t groups = std::min<size_t>(units, budget);
+    ReductionPlan plan;
+    const int err = plan_reduction<T>(num_samples, num_channels, spatial, {&tx, &td}, kUnroll / 2, &plan);
+    if (err)
+        return err;
+    const bool strided = plan.strided;
+    const int vw = plan.vw, gmax = plan.groups_max;
+    const size_t units = plan.units, groups = plan.groups;
+    const Chunking& ch = plan.ch;
+    num_samples = plan.num_samples;
+    spatial = plan.spatial;
     double* partials = static_cast<double*>(workspace);
     const dim3 grid(static_cast<unsigned int>(groups), num_channels);
     LaunchRecord rec = long_record(kKernelBackprop1, strided, vw, grid, num_samples, num_channels,
                                    spatial, ch, {&tx, &td}, false);
-    rec.folded = folded;
+    rec.folded = plan.folded;
     rec.num_units = static_cast<unsigned int>(units);
     rec.num_sums = 4;
     rec.groups_max = gmax;
@@ -2577,20 +2608,26 @@ int backward_local_strided(int n, size_t num_per_sum, const h2x_tensor_geometry*
 
 // ---- whole channels in one workgroup: which calls, which team -------------------
 // float only: the staged calls of double tensors are promised bit for bit, and here
-// the fp64 sums are added in another order (N 8, C 32, 33^3, double, 36 + 62 us, by teams
-// 32 + 45; members that add what the staged workgroups add, in their order, would keep the
-// bits: not built).  All tensors of the call lie alike, a row holds a vector, and offsets within a
-// channel fit 30 bits.
-bool once_geometry(int num_samples, int num_channels, size_t spatial, std::initializer_list<const HostTensor*> ts,
-                   OnceGeometry* g)
+// the fp64 sums are added in another order (ordered_geometry below keeps it).  All tensors of the call lie
+// alike, a row holds a vector, and offsets within a channel fit 30 bits.
+bool lie_alike(std::initializer_list<const HostTensor*> ts)
 {
-    constexpr size_t vec = full_vec<float>();
     const HostTensor& a = **ts.begin();
     for (const HostTensor* t : ts)
         if (t->strided != a.strided || t->map.stride_n != a.map.stride_n || t->map.stride_c != a.map.stride_c
             || t->map.sy != a.map.sy || t->map.sz != a.map.sz || t->map.w.divisor != a.map.w.divisor
             || t->map.h.divisor != a.map.h.divisor)
             return false;
+    return true;
+}
+
+bool once_geometry(int num_samples, int num_channels, size_t spatial, std::initializer_list<const HostTensor*> ts,
+                   OnceGeometry* g)
+{
+    constexpr size_t vec = full_vec<float>();
+    const HostTensor& a = **ts.begin();
+    if (!lie_alike(ts))
+        return false;
     const size_t w = a.row, h = a.strided ? a.map.h.divisor : 1, d = a.strided ? spatial / (w * h) : 1;
     if (w < vec || a.map.stride_n >= (1ll << 30))
         return false;
@@ -2761,6 +2798,21 @@ constexpr uint32_t kTeamPolls = 2048;
 // fewer.  Below the last, channels are few and the two-launch kernels cut them finer (N 2, C 4, 40^3).
 constexpr uint32_t kLargeMembers = 384, kMediumMembers = 256, kSmallMembers = 128;
 
+// CUs of the current device (0: there is none), asked for once: a device does not change, and
+// the question costs a small call most of a microsecond.
+uint32_t compute_units()
+{
+    static std::atomic<int> known[kMaxDevices];
+    int device = 0, cus = 0;
+    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMaxDevices)
+        return 0;
+    cus = known[device].load(std::memory_order_relaxed);
+    if (cus == 0
+        && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess)
+        known[device].store(cus, std::memory_order_relaxed);
+    return static_cast<uint32_t>(cus);
+}
+
 // Forward a member holds 128, 64 or 32 KB (N 16, C 64, 112 x 112 in 448 workgroups of 128 KB 20.4 us, in
 // 832 of 64 KB 22.5; N 2, C 32, 48^3 in 448 of 64 KB 12.0, in 224 of 128 KB 13.0; N 2, C 32, 28^3 with a halo
 // in 224 of 32 KB 6.8 us, in two launches 9.8); up to 128 members (N 16, C 16, 64^3 in 128 of them 98 us, in
@@ -2796,21 +2848,6 @@ template <typename G>
 bool teams_first(const G& g)
 {
     return g.vectors > 4096 && g.num_channels <= kOnceManyChannels;
-}
-
-// CUs of the current device (0: there is none), asked for once: a device does not change, and
-// the question costs a small call most of a microsecond.
-uint32_t compute_units()
-{
-    static std::atomic<int> known[kMaxDevices];
-    int device = 0, cus = 0;
-    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMaxDevices)
-        return 0;
-    cus = known[device].load(std::memory_order_relaxed);
-    if (cus == 0
-        && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess)
-        known[device].store(cus, std::memory_order_relaxed);
-    return static_cast<uint32_t>(cus);
 }
 
 // A team keeps within half of the chip.
@@ -2861,6 +2898,171 @@ bool launch_by_teams(const OnceGeometry& g, const A& a, int n, std::initializer_
            && launch_by_teams(g, a, reach_bytes(g, n), streamed(g, n), inputs, output, forced, polls, team_state, st);
 }
 
+// ---- whole channels of doubles, in the order of the staged calls ------------------
+// Tensors that lie alike (`ts`: the inputs, x first), whose staged reduction is one of the long-segment kernels in
+// vectors, with no more groups a channel than the staged kernels add in one go.
+bool ordered_geometry(int num_samples, int num_channels, size_t spatial, std::initializer_list<const HostTensor*> ts,
+                      const HostTensor& output, OrderedGeometry* g, bool* rows)
+{
+    HostTensor t[2];
+    size_t inputs = 0;
+    for (const HostTensor* i : ts)
+    {
+        if (!lie_alike({i, &output}))
+            return false;
+        t[inputs++] = *i;
+    }
+    ShortGeometry sg;
+    const bool one = inputs == 1;
+    if (one ? short_segments<double>(num_samples, num_channels, spatial, {&t[0]}, &sg)
+            : short_segments<double>(num_samples, num_channels, spatial, {&t[0], &t[1]}, &sg))
+        return false;
+    const size_t last = (num_samples - 1) * static_cast<size_t>(t[0].map.stride_n) + short_span(t[0], spatial);
+    ReductionPlan plan;
+    if (last >= (1ull << 30) || t[0].map.stride_n >= (1ll << 30)
+        || (one ? plan_reduction<double>(num_samples, num_channels, spatial, {&t[0]}, kUnroll, &plan)
+                : plan_reduction<double>(num_samples, num_channels, spatial, {&t[0], &t[1]}, kUnroll / 2, &plan)))
+        return false;
+    // (outputs are stored in the same vectors, so they have to be aligned where those are)
+    if (plan.vw != full_vec<double>() || (!plan.strided && !output.aligned) || plan.groups > kBlockSize
+        || plan.spatial >= (1ull << 31) || plan.units >= (1ull << 31))
+        return false;
+    const uint32_t batches = static_cast<uint32_t>(plan.ch.chunk / (kBlockSize * 2 * kOrderedBatch));
+    const uint32_t rounds = static_cast<uint32_t>((plan.units + plan.groups - 1) / plan.groups);
+    *rows = plan.strided;
+    g->map = t[0].map;
+    g->spatial = static_cast<uint32_t>(plan.spatial);
+    g->chunk = static_cast<uint32_t>(plan.ch.chunk);
+    g->per_segment = make_fastdiv(static_cast<uint32_t>(plan.ch.chunks_per_seg));
+    g->unit_batches = make_fastdiv(batches);
+    g->group_batches = make_fastdiv(batches * rounds);
+    g->units = static_cast<uint32_t>(plan.units);
+    g->groups = static_cast<uint32_t>(plan.groups);
+    g->num_channels = static_cast<uint32_t>(num_channels);
+    g->max_polls = kTeamPolls;
+    return true;
+}
+
+template <int TEAM, int K, bool TEAMS, bool ROWS, bool STREAM>
+void issue_ordered(const OrderedGeometry& g, const OnceForward<double>& a, unsigned long long* states, uint32_t blocks,
+                   hipStream_t st)
+{
+    bn_ordered_forward_kernel<TEAM, K, TEAMS, ROWS, STREAM><<<blocks, TEAM, 0, st>>>(g, a, states);
+}
+template <int TEAM, int K, bool TEAMS, bool ROWS, bool STREAM>
+void issue_ordered(const OrderedGeometry& g, const OnceBackward<double>& a, unsigned long long* states, uint32_t blocks,
+                   hipStream_t st)
+{
+    bn_ordered_backward_kernel<TEAM, K, TEAMS, ROWS, STREAM><<<blocks, TEAM, 0, st>>>(g, a, states);
+}
+
+// Groups that a workgroup of TEAM threads with K vectors each holds.
+template <int TEAM, int K>
+uint32_t ordered_holds(const OrderedGeometry& g)
+{
+    return TEAM / kBlockSize * (K / kOrderedBatch / g.group_batches.divisor);
+}
+
+template <int TEAM, int K, bool TEAMS, typename A>
+void ordered_issue(const OrderedGeometry& g, const A& a, bool rows, bool stream, void* state, hipStream_t st)
+{
+    unsigned long long* const states = static_cast<unsigned long long*>(state);
+    const uint32_t blocks = TEAMS ? g.num_channels * g.members.divisor : (g.num_channels + kNumXcd - 1) / kNumXcd * kNumXcd;
+    if (!rows)
+        issue_ordered<TEAM, K, TEAMS, false, true>(g, a, states, blocks, st);
+    else if (stream)
+        issue_ordered<TEAM, K, TEAMS, true, true>(g, a, states, blocks, st);
+    else
+        issue_ordered<TEAM, K, TEAMS, true, false>(g, a, states, blocks, st);
+}
+
+// One workgroup a channel.  Without a: whether.
+template <int TEAM, int K, typename A>
+bool ordered_once(OrderedGeometry g, const A* a, bool rows, bool stream, hipStream_t st)
+{
+    if (g.groups > ordered_holds<TEAM, K>(g))
+        return false;
+    g.passes = K / kOrderedBatch / g.group_batches.divisor;
+    g.members = make_fastdiv(1);
+    if (a)
+        ordered_issue<TEAM, K, false>(g, *a, rows, stream, nullptr, st);
+    return true;
+}
+
+// A team a channel, of at least `least` workgroups over all channels.
+template <int TEAM, int K, typename A>
+bool ordered_team(OrderedGeometry g, const A* a, bool rows, bool stream, uint32_t least, uint32_t most, void* state,
+                  hipStream_t st)
+{
+    constexpr uint32_t kSums = std::is_same<A, OnceForward<double>>::value ? 2 : 4;
+    const uint32_t own = ordered_holds<TEAM, K>(g);
+    if (own < 2)
+        return false;
+    const uint32_t width = own % 4 == 0 ? 4 : 2, members = (g.groups + own - 1) / own;
+    const size_t blocks = static_cast<size_t>(members) * g.num_channels;
+    if (members > most || (g.groups + width - 1) / width * kSums > kMaxTeamSums || blocks < least || blocks >= (1u << 30))
+        return false;
+    g.passes = K / kOrderedBatch / g.group_batches.divisor;
+    g.members = make_fastdiv(members);
+    if (a)
+        ordered_issue<TEAM, K, true>(g, *a, rows, stream, state, st);
+    return true;
+}
+
+// Which of them, as for floats (once_launch, team_variant).  most_members 0: no teams, where the outputs
+// overlap the inputs or there is no state.  *team: whether it is one.
+template <typename A>
+bool ordered_variant(const OrderedGeometry& g, const A* a, bool rows, bool stream, uint32_t most, bool forced, void* state,
+                     hipStream_t st, bool* team)
+{
+    constexpr bool kForward = std::is_same<A, OnceForward<double>>::value;
+    const size_t vectors = static_cast<size_t>(g.groups) * g.group_batches.divisor * kOrderedBatch * kBlockSize;
+    const bool few = g.num_channels <= kOnceManyChannels;
+    const auto by_teams = [&] {
+        *team = true;
+        if constexpr (kForward)
+            return ordered_team<512, 16>(g, a, rows, stream, forced ? 1 : kLargeMembers, most, state, st)
+                   || ordered_team<512, 8>(g, a, rows, stream, forced ? 1 : kMediumMembers, most, state, st)
+                   || ordered_team<512, 4>(g, a, rows, stream, forced ? 1 : kSmallMembers, most, state, st);
+        else
+            return ordered_team<512, 8>(g, a, rows, stream, forced ? 1 : kMediumMembers, most / 2, state, st)
+                   || ordered_team<512, 4>(g, a, rows, stream, forced ? 1 : kSmallMembers, most / 2, state, st);
+    };
+    if ((forced || (few && vectors > 4096)) && by_teams())
+        return true;
+    *team = false;
+    if (forced)
+        return false;
+    if (ordered_once<256, 4>(g, a, rows, stream, st) || ordered_once<512, 4>(g, a, rows, stream, st)
+        || ordered_once<1024, 4>(g, a, rows, stream, st) || ordered_once<1024, 8>(g, a, rows, stream, st))
+        return true;
+    if constexpr (kForward)
+        if (!few && ordered_once<1024, 16>(g, a, rows, stream, st))
+            return true;
+    return by_teams();
+}
+
+// False: the staged kernels, in two launches.
+template <typename A>
+bool ordered_launch(int n, int c, size_t s, std::initializer_list<const HostTensor*> ts, const HostTensor& output,
+                    std::initializer_list<const void*> inputs, const void* out, const A& a, void* state,
+                    const uint32_t* team_polls, hipStream_t st)
+{
+    OrderedGeometry g;
+    bool rows, team;
+    if (!ordered_geometry(n, c, s, ts, output, &g, &rows))
+        return false;
+    const size_t bytes = (static_cast<size_t>(c - 1) * output.map.stride_c + static_cast<size_t>(n - 1) * output.map.stride_n
+                          + short_span(output, s)) * sizeof(double);
+    bool teams = state != nullptr;
+    for (const void* p : inputs)
+        teams = teams && apart(p, out, bytes);
+    if (team_polls)
+        g.max_polls = *team_polls;
+    return ordered_variant(g, &a, rows, !output.strided || bytes > kHaloedNormalStores, teams ? most_members() : 0,
+                           team_polls != nullptr, state, st, &team);
+}
+
 // team_polls: by teams or not at all, however few workgroups that is, with this many looks.
 template <typename T>
 int forward_once(int n, const h2x_tensor_geometry* gx, const h2x_tensor_geometry* gy, const void* x,
@@ -2891,6 +3093,15 @@ int forward_once(int n, const h2x_tensor_geometry* gx, const h2x_tensor_geometry
             if ((teams && by_teams()) || once_launch(g, a, n, st) || (!teams && by_teams()))
                 return launch_status();
         }
+    }
+    else if (x && y && n > 0 && c > 0 && s > 0 && num_per_sum > 0)
+    {
+        const OnceForward<T> a{static_cast<const T*>(x), static_cast<const T*>(scale), static_cast<const T*>(bias),
+                               static_cast<T*>(mean), static_cast<T*>(var), static_cast<T*>(running_mean),
+                               static_cast<T*>(running_var), static_cast<T*>(y), static_cast<T>(num_per_sum),
+                               static_cast<T>(decay), static_cast<T>(eps)};
+        if (ordered_launch(n, c, s, {&tx}, ty, {x}, y, a, team_state, team_polls, st))
+            return launch_status();
     }
     if (team_polls)
         return H2X_ERR_UNSUPPORTED;
@@ -2929,6 +3140,16 @@ int backward_once(int n, size_t num_per_sum, const h2x_tensor_geometry* gx, cons
             if ((teams && by_teams()) || once_launch(g, a, n, st) || (!teams && by_teams()))
                 return launch_status();
         }
+    }
+    else if (x && dy && dx && n > 0 && c > 0 && s > 0)
+    {
+        const OnceBackward<T> a{static_cast<const T*>(x), static_cast<const T*>(dy), static_cast<const T*>(mean),
+                                static_cast<const T*>(var), static_cast<const T*>(scale), static_cast<T*>(dscale),
+                                static_cast<T*>(dbias), static_cast<T*>(dmean), static_cast<T*>(dvar),
+                                static_cast<T*>(dx), static_cast<T>(num_per_sum),
+                                static_cast<T>(num_per_sum - 1), static_cast<T>(eps)};
+        if (ordered_launch(n, c, s, {&tx, &td}, to, {x, dy}, dx, a, team_state, team_polls, st))
+            return launch_status();
     }
     if (team_polls)
         return H2X_ERR_UNSUPPORTED;
@@ -3380,6 +3601,27 @@ extern "C" size_t h2x_bn_team_state_needed(h2x_dtype dtype, int num_samples, con
     return team_state_needed(g);
 }
 
+extern "C" size_t h2x_bn_ordered_state_needed(int num_samples, const h2x_tensor_geometry* geometry)
+{
+    HostTensor t;
+    OrderedGeometry g;
+    int c;
+    size_t s;
+    bool rows, forward = false, backward = false;
+    // the address counts by its alignment: as of tensors made by an allocator
+    const void* const aligned = reinterpret_cast<const void*>(uintptr_t(256));
+    if (num_samples <= 0 || !geometry || strided_tensor<double>(geometry, aligned, num_samples, &t, &c, &s) || c <= 0 || s == 0)
+        return 0;
+    const OnceForward<double>* const f = nullptr;
+    const OnceBackward<double>* const b = nullptr;
+    const uint32_t most = most_members();
+    forward = ordered_geometry(num_samples, c, s, {&t}, t, &g, &rows)
+              && ordered_variant(g, f, rows, true, most, false, nullptr, nullptr, &forward) && forward;
+    backward = ordered_geometry(num_samples, c, s, {&t, &t}, t, &g, &rows)
+               && ordered_variant(g, b, rows, true, most, false, nullptr, nullptr, &backward) && backward;
+    return forward || backward ? h2x_bn_team_state_bytes(c) : 0;
+}
+
 extern "C" size_t h2x_bn_team_state_needed_clearing(h2x_dtype dtype, const h2x_haloed_geometry* geometry)
 {
     ClearGeometry g;
@@ -3534,5 +3776,54 @@ extern "C" int h2x_bn_audit_once(int num_samples, const h2x_tensor_geometry* geo
                     counted[e + j] += OnceGeometry::counts(at, j);
                 }
             }
+    return H2X_SUCCESS;
+}
+
+// Plays on the host which elements the workgroups that keep the staged order touch.
+extern "C" int h2x_bn_audit_ordered(int num_samples, const h2x_tensor_geometry* geometry, int backward,
+                                    unsigned int passes, unsigned char* counted, unsigned char* stored,
+                                    unsigned short* group, size_t elements)
+{
+    if (!geometry || !counted || !stored || !group || passes == 0)
+        return H2X_ERR_INVALID_ARGUMENT;
+    HostTensor t;
+    OrderedGeometry g;
+    int c;
+    size_t s;
+    bool rows;
+    // (as of tensors made by an allocator)
+    const int err = strided_tensor<double>(geometry, reinterpret_cast<const void*>(uintptr_t(256)), num_samples, &t, &c, &s);
+    if (err)
+        return err;
+    if (num_samples <= 0 || c <= 0 || s == 0
+        || !(backward ? ordered_geometry(num_samples, c, s, {&t, &t}, t, &g, &rows)
+                      : ordered_geometry(num_samples, c, s, {&t}, t, &g, &rows)))
+        return H2X_ERR_UNSUPPORTED;
+    constexpr int kTeam = 2 * kBlockSize;
+    g.passes = passes;
+    const uint32_t members = (g.groups + 2 * passes - 1) / (2 * passes);
+    for (uint32_t ch = 0; ch < g.num_channels; ++ch)
+        for (uint32_t i = 0; i < members; ++i)
+            for (uint32_t p = 0; p < passes; ++p)
+                for (uint32_t thread = 0; thread < kTeam; ++thread)
+                    for (uint32_t u = 0; u < g.group_batches.divisor * kOrderedBatch; ++u)
+                    {
+                        const uint32_t k = ordered_group<kTeam>(g, team_member(i, members), p, thread / kBlockSize);
+                        const uint32_t b = u / kOrderedBatch, j = u % kOrderedBatch, th = thread % kBlockSize;
+                        const uint32_t at = rows ? ordered_place<true>(g, k, b, j, th) : ordered_place<false>(g, k, b, j, th);
+                        if (at == kNowhere)
+                            continue;
+                        const size_t e = static_cast<size_t>(ch * g.map.stride_c) + (at >> 1);
+                        if (e + 2 > elements)
+                            return H2X_ERR_INVALID_ARGUMENT;
+                        for (uint32_t v = 0; v < 2; ++v)
+                        {
+                            stored[e + v] = 1;
+                            if (v < (at & 1))
+                                continue;
+                            ++counted[e + v];
+                            group[e + v] = static_cast<unsigned short>(k + 1);
+                        }
+                    }
     return H2X_SUCCESS;
 }

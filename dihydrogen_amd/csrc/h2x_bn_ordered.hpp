@@ -1,0 +1,441 @@
+// Batch-norm of double tensors of a rank that shares its statistics with no one, every
+// element read once, with the bits of the staged calls.  Included by h2x_bn.hip after
+// h2x_bn_team.hpp.
+//
+// The staged calls of double tensors are promised bit for bit, so the sums have to be
+// added in their order: bn_sums_kernel and bn_backprop1_kernel give each group of 256
+// threads some units (chunks of a segment) and leave one partial sum a group, and
+// channel_totals adds those, thread t starting with partial t.  Here a workgroup, or a
+// team of workgroups where a channel is larger or channels are few, holds the vectors
+// of several such groups in its registers: 256 neighbouring threads play one group, one
+// after another its passes; the sums of a group are those of the staged workgroup, and the
+// partial sums are added along the staged tree.  What the members of a team exchange
+// are sums of two or four neighbouring partials, the first steps of that tree.
+//
+// Bound by memory, and by the wait for the last member of a team.  Two launches each way ->
+// this, forward + backward, us going round three sets of tensors:
+//   N 8, C 32, 33^3              97 -> 88       N 4, C 64, 56 x 56            20 -> 14
+//   N 64, C 512, 20 x 20        136 -> 110      N 8, C 100, 64 x 64           39 -> 30
+//   N 16, C 32, 112 x 112        69 -> 55       N 12, C 9, 113 x 123, halo    28 -> 23
+//   N 4, C 213, 17 x 20 x 23, halo of 1  85 -> 76
+// (33^3 is 18 units a segment, the last of them half empty: 144 groups, 36 members.)
+#pragma once
+
+struct OrderedGeometry
+{
+    TensorMap map;         // of every tensor of the call
+    uint32_t spatial;      // elements of a (padded) segment
+    uint32_t chunk;        // elements of a unit, a multiple of four vectors a thread
+    FastDiv per_segment;   // units of a segment
+    FastDiv unit_batches;  // batches of four vectors a thread of a unit
+    FastDiv group_batches; // of all units of a group
+    uint32_t units;        // of a channel; group k takes units k, k + groups, ...
+    uint32_t groups;       // of a channel, at most kBlockSize
+    uint32_t passes;       // groups that 256 threads of a workgroup play one after another
+    uint32_t num_channels;
+    FastDiv members;       // of a team
+    uint32_t max_polls;
+};
+
+constexpr int kOrderedBatch = 4; // vectors a thread: kUnroll of the staged kernels
+constexpr uint32_t kNowhere = ~0u;
+
+// Vector j of batch `batch` of a group, of its thread t: element offset from the start of the
+// channel, times two, plus the element it skips; kNowhere: there is none.  (Offsets below 2^30.)
+template <bool ROWS>
+__host__ __device__ __forceinline__ uint32_t ordered_place(const OrderedGeometry& g, uint32_t group, uint32_t batch,
+                                                           uint32_t j, uint32_t t)
+{
+    const uint32_t round = fastdiv(batch, g.unit_batches);
+    const uint32_t unit = group + round * g.groups;
+    if (group >= g.groups || unit >= g.units)
+        return kNowhere;
+    const uint32_t n = fastdiv(unit, g.per_segment);
+    const uint32_t begin = (unit - n * g.per_segment.divisor) * g.chunk;
+    const uint32_t end = begin + g.chunk < g.spatial ? begin + g.chunk : g.spatial;
+    const uint32_t slot = (batch - round * g.unit_batches.divisor) * kOrderedBatch + j;
+    const uint32_t i = begin + (slot * kBlockSize + t) * 2;
+    if (i + 2 > end)
+        return kNowhere;
+    const uint32_t start = n * static_cast<uint32_t>(g.map.stride_n);
+    if constexpr (!ROWS)
+        return (start + i) * 2;
+    Place pl{0, 0, 0, 0};
+    place_vector<2>(g.map, row_split<2>(g.map, i, &pl), &pl);
+    return (start + static_cast<uint32_t>(row_offset(g.map, pl)) + static_cast<uint32_t>(pl.first)) * 2 + pl.skip;
+}
+
+// The group that a thread plays in its pass p, as member `member` of its team.
+template <int TEAM>
+__host__ __device__ __forceinline__ uint32_t ordered_group(const OrderedGeometry& g, uint32_t member, uint32_t p,
+                                                           uint32_t quarter)
+{
+    return (member * g.passes + p) * (TEAM / kBlockSize) + quarter;
+}
+
+// Steps of wave_sum from those that add lanes `first` apart (1, 2 or 4).  Lanes that are no multiple of
+// `first` hold nothing and get nothing.
+__device__ __forceinline__ double wave_sum_from(double v, uint32_t first)
+{
+    if (first < 2)
+        v += dpp_move<kDppQuadSwap1>(v);
+    if (first < 4)
+        v += dpp_move<kDppQuadSwap2>(v);
+    v += dpp_move<kDppRowRor4>(v);
+    v += dpp_move<kDppRowRor8>(v);
+    v += __shfl_xor(v, 16, kWaveSize);
+    v += __shfl_xor(v, 32, kWaveSize);
+    return v;
+}
+
+// The partial sums of the groups that a member plays, in lds as the sums of their four waves:
+// sums[group of the member][wave][k].  add(u, s): the terms of a thread's vector u.
+template <int TEAM, int K, int N, typename F>
+__device__ __forceinline__ void ordered_partials(const OrderedGeometry& g, double* sums, const F& add)
+{
+    constexpr int kQuarters = TEAM / kBlockSize;
+    const uint32_t wave = threadIdx.x / kWaveSize;
+    double s[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+        s[k] = 0.0;
+#pragma unroll
+    for (int b = 0; b < K / kOrderedBatch; ++b)
+    {
+        const uint32_t p = fastdiv(b, g.group_batches);
+        if (p >= g.passes) // uniform
+            continue;
+#pragma unroll
+        for (int j = 0; j < kOrderedBatch; ++j)
+            add(b * kOrderedBatch + j, s);
+        if (b - p * g.group_batches.divisor + 1 < g.group_batches.divisor)
+            continue;
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+        {
+            const double t = wave_sum(s[k]);
+            if (threadIdx.x % kWaveSize == 0)
+                sums[((p * kQuarters + wave / kWavesPerBlock) * kWavesPerBlock + wave % kWavesPerBlock) * N + k] = t;
+            s[k] = 0.0;
+        }
+    }
+}
+
+// Partial sum k of a group of the member, as block_sum adds its waves; nothing beyond the last group.
+template <int N>
+__device__ __forceinline__ double ordered_partial(const double* sums, uint32_t local, bool there, int k)
+{
+    if (!there)
+        return 0.0;
+    const double* const w = sums + local * kWavesPerBlock * N + k;
+    double t = w[0];
+#pragma unroll
+    for (int i = 1; i < kWavesPerBlock; ++i)
+        t += w[i * N];
+    return 0.0 + t; // as channel_totals starts
+}
+
+// channel_totals over what the first 256 threads hold: lanes `first` apart.  lds: N times four doubles.
+template <int N>
+__device__ __forceinline__ void ordered_totals(double (&v)[N], uint32_t first, double* lds)
+{
+    if (threadIdx.x < kBlockSize)
+    {
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+        {
+            const double t = wave_sum_from(v[k], first);
+            if (threadIdx.x % kWaveSize == 0)
+                lds[k * kWavesPerBlock + threadIdx.x / kWaveSize] = t;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+    {
+        double t = lds[k * kWavesPerBlock];
+#pragma unroll
+        for (int w = 1; w < kWavesPerBlock; ++w)
+            t += lds[k * kWavesPerBlock + w];
+        v[k] = t;
+    }
+}
+
+// The sums of the channel in v[] of every thread, from the partial sums in `sums`.  Teams: as
+// team_exchange, tags and all; recompute(m) leaves the partial sums of member m in `sums`.
+template <int TEAM, int K, int N, bool TEAMS, typename F>
+__device__ __forceinline__ void ordered_exchange(double (&v)[N], const OrderedGeometry& g, uint32_t member,
+                                                 unsigned long long* state, uint32_t tag, double* sums, double* lds,
+                                                 uint32_t* missing, const F& recompute)
+{
+    constexpr uint32_t kQuarters = TEAM / kBlockSize;
+    const uint32_t t = threadIdx.x, own = g.passes * kQuarters; // groups of a member
+    if constexpr (!TEAMS)
+    {
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+            v[k] = t < own ? ordered_partial<N>(sums, t, t < g.groups, k) : 0.0;
+        ordered_totals<N>(v, 1, lds);
+    }
+    else
+    {
+        // an item: what the tree makes of two or four neighbouring partial sums
+        const uint32_t width = own % 4 == 0 ? 4 : 2, per_member = own / width;
+        const uint32_t items = (g.groups + width - 1) / width, item = t / width;
+        const auto item_of = [&](uint32_t m, uint32_t i, int k) {
+            const auto at = [&](uint32_t j) {
+                return ordered_partial<N>(sums, i * width + j, m * own + i * width + j < g.groups, k);
+            };
+            const double low = at(0) + at(1);
+            return width == 2 ? low : low + (at(2) + at(3));
+        };
+        unsigned long long* const words = state + kCounterWords;
+        if (t < kMaxMembers)
+            missing[t] = 0;
+        if (t == 0)
+        {
+            missing[kMaxMembers] = 0;
+            missing[kMaxMembers + 1] = tag;
+        }
+        __syncthreads();
+        tag = missing[kMaxMembers + 1];
+        if (t < per_member && member * per_member + t < items)
+        {
+#pragma unroll
+            for (int k = 0; k < N; ++k)
+            {
+                const unsigned long long bits = __double_as_longlong(item_of(member, t, k));
+                team_store(words + 2 * k * items + member * per_member + t, tag, static_cast<uint32_t>(bits));
+                team_store(words + (2 * k + 1) * items + member * per_member + t, tag, static_cast<uint32_t>(bits >> 32));
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+            v[k] = 0.0;
+        const bool reads = t % width == 0 && t < kBlockSize && item < items;
+        if (reads)
+        {
+            const unsigned long long* const mine = words + item;
+            bool there = false;
+            for (uint32_t poll = 0; poll < g.max_polls && !there; ++poll)
+            {
+                if (poll > 0)
+                    __builtin_amdgcn_s_sleep(4);
+                if (team_load(mine + (2 * N - 1) * items) >> 32 != tag) // the word stored last
+                    continue;
+                there = true;
+#pragma unroll
+                for (int k = 0; k < N; ++k)
+                {
+                    const unsigned long long lo = team_load(mine + 2 * k * items),
+                                             hi = team_load(mine + (2 * k + 1) * items);
+                    v[k] = __longlong_as_double(hi << 32 | (lo & 0xffffffffull));
+                    there = there && lo >> 32 == tag && hi >> 32 == tag;
+                }
+            }
+            if (!there) // every writer stores the same
+                missing[item / per_member] = missing[kMaxMembers] = 1;
+        }
+        __syncthreads();
+        if (t == 0)
+            __hip_atomic_fetch_add(state, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (missing[kMaxMembers])
+            for (uint32_t m = 0; m < g.members.divisor; ++m)
+                if (missing[m]) // uniform
+                {
+                    __syncthreads(); // the sums may still be read
+                    recompute(m);
+                    __syncthreads();
+                    if (reads && item / per_member == m)
+                    {
+#pragma unroll
+                        for (int k = 0; k < N; ++k)
+                            v[k] = item_of(m, item - m * per_member, k);
+                    }
+                }
+        ordered_totals<N>(v, width, lds);
+    }
+}
+
+// Channel and member of a workgroup.
+template <bool TEAMS>
+__device__ __forceinline__ uint32_t ordered_channel(const OrderedGeometry& g, uint32_t* member)
+{
+    if constexpr (!TEAMS)
+    {
+        *member = 0;
+        return xcd_contiguous(blockIdx.x, gridDim.x);
+    }
+    const uint32_t c = fastdiv(blockIdx.x, g.members);
+    *member = team_member(blockIdx.x - c * g.members.divisor, g.members.divisor);
+    return c;
+}
+
+template <int TEAM, int K, bool TEAMS, bool ROWS, bool STREAM>
+__global__ __launch_bounds__(TEAM, TEAMS ? 4 : 1) void bn_ordered_forward_kernel(const OrderedGeometry g, const OnceForward<double> a,
+                                                                  unsigned long long* states)
+{
+    typedef double T;
+    constexpr int VEC = 2, kQuarters = TEAM / kBlockSize;
+    __shared__ double sums[kQuarters * (K / kOrderedBatch) * kWavesPerBlock * 2], lds[2 * kWavesPerBlock];
+    __shared__ uint32_t missing[TEAMS ? kMaxMembers + 2 : 1];
+    uint32_t member;
+    const uint32_t c = ordered_channel<TEAMS>(g, &member);
+    if (c >= g.num_channels)
+        return;
+    unsigned long long* const state = TEAMS ? states + static_cast<size_t>(c) * kStateWords : nullptr;
+    const uint32_t tag = TEAMS && threadIdx.x == 0 ? static_cast<uint32_t>(team_load(state)) + 1 : 0;
+    const uint32_t quarter = __builtin_amdgcn_readfirstlane(threadIdx.x / kBlockSize), t = threadIdx.x % kBlockSize;
+    const T* const x = a.x + c * g.map.stride_c;
+    const auto place = [&](uint32_t m, int u) {
+        const uint32_t p = fastdiv(u / kOrderedBatch, g.group_batches);
+        return p >= g.passes ? kNowhere
+                             : ordered_place<ROWS>(g, ordered_group<TEAM>(g, m, p, quarter),
+                                                   u / kOrderedBatch - p * g.group_batches.divisor, u % kOrderedBatch, t);
+    };
+    const auto terms = [](double (&s)[2], const T (&v)[VEC], uint32_t at) {
+#pragma unroll
+        for (int j = 0; j < VEC; ++j)
+            if (!ROWS || j >= static_cast<int>(at & 1))
+            {
+                s[0] += v[j];
+                s[1] += v[j] * v[j];
+            }
+    };
+    T v[K][VEC];
+    uint32_t at[K];
+#pragma unroll
+    for (int u = 0; u < K; ++u)
+    {
+        at[u] = place(member, u);
+        if (at[u] != kNowhere)
+            load_vec<T, VEC, !ROWS>(x + (at[u] >> 1), v[u]);
+    }
+    ordered_partials<TEAM, K, 2>(g, sums, [&](int u, double (&s)[2]) {
+        if (at[u] != kNowhere)
+            terms(s, v[u], at[u]);
+    });
+    double s[2];
+    ordered_exchange<TEAM, K, 2, TEAMS>(s, g, member, state, tag, sums, lds, missing, [&](uint32_t other) {
+        ordered_partials<TEAM, K, 2>(g, sums, [&](int u, double (&r)[2]) {
+            const uint32_t p = place(other, u);
+            if (p == kNowhere)
+                return;
+            T w[VEC];
+            load_vec<T, VEC, !ROWS>(x + (p >> 1), w);
+            terms(r, w, p);
+        });
+    });
+    T m, variance;
+    sums_to_mean_var(s[0], s[1], a.n, &m, &variance);
+    if (member == 0 && threadIdx.x == 0)
+    {
+        a.mean[c] = m;
+        a.var[c] = variance;
+        a.running_mean[c] = fma_t(a.decay, a.running_mean[c], (T(1) - a.decay) * m);
+        a.running_var[c] = fma_t(a.decay, a.running_var[c], (T(1) - a.decay) * variance);
+    }
+    const T inv_stdev = inv_sqrt_t(variance + a.epsilon);
+    const T sc = a.scale[c], bi = a.bias[c];
+    T* const y = a.y + c * g.map.stride_c;
+#pragma unroll
+    for (int u = 0; u < K; ++u)
+        if (at[u] != kNowhere)
+        {
+#pragma unroll
+            for (int j = 0; j < VEC; ++j)
+                v[u][j] = fma_t((v[u][j] - m) * inv_stdev, sc, bi);
+            store_once<T, VEC, STREAM>(y + (at[u] >> 1), v[u]);
+        }
+}
+
+template <int TEAM, int K, bool TEAMS, bool ROWS, bool STREAM>
+__global__ __launch_bounds__(TEAM, TEAMS ? 4 : 1) void bn_ordered_backward_kernel(const OrderedGeometry g,
+                                                                   const OnceBackward<double> a,
+                                                                   unsigned long long* states)
+{
+    typedef double T;
+    constexpr int VEC = 2, kQuarters = TEAM / kBlockSize;
+    __shared__ double sums[kQuarters * (K / kOrderedBatch) * kWavesPerBlock * 4], lds[4 * kWavesPerBlock];
+    __shared__ uint32_t missing[TEAMS ? kMaxMembers + 2 : 1];
+    uint32_t member;
+    const uint32_t c = ordered_channel<TEAMS>(g, &member);
+    if (c >= g.num_channels)
+        return;
+    unsigned long long* const state = TEAMS ? states + static_cast<size_t>(c) * kStateWords : nullptr;
+    const uint32_t tag = TEAMS && threadIdx.x == 0 ? static_cast<uint32_t>(team_load(state)) + 1 : 0;
+    const uint32_t quarter = __builtin_amdgcn_readfirstlane(threadIdx.x / kBlockSize), t = threadIdx.x % kBlockSize;
+    const int64_t base = c * g.map.stride_c;
+    const auto place = [&](uint32_t m, int u) {
+        const uint32_t p = fastdiv(u / kOrderedBatch, g.group_batches);
+        return p >= g.passes ? kNowhere
+                             : ordered_place<ROWS>(g, ordered_group<TEAM>(g, m, p, quarter),
+                                                   u / kOrderedBatch - p * g.group_batches.divisor, u % kOrderedBatch, t);
+    };
+    T xv[K][VEC], dv[K][VEC];
+    uint32_t at[K];
+#pragma unroll
+    for (int u = 0; u < K; ++u)
+    {
+        at[u] = place(member, u);
+        if (at[u] != kNowhere)
+        {
+            load_vec<T, VEC, !ROWS>(a.x + base + (at[u] >> 1), xv[u]);
+            load_vec<T, VEC, !ROWS, kStreamGradient<K>>(a.dy + base + (at[u] >> 1), dv[u]);
+        }
+    }
+    const T m = a.mean[c];
+    const T sc = a.scale[c];
+    const T inv_stdev = inv_sqrt_t(a.var[c] + a.epsilon);
+    const T dvar_factor = inv_stdev * inv_stdev * inv_stdev / T(2);
+    const double neg_inv = -inv_stdev, neg_fac = -dvar_factor;
+    // as in bn_backprop1_kernel
+    const auto terms = [&](double (&s)[4], const T (&x)[VEC], const T (&d)[VEC], uint32_t p) {
+#pragma unroll
+        for (int j = 0; j < VEC; ++j)
+            if (!ROWS || j >= static_cast<int>(p & 1))
+            {
+                const T xm = x[j] - m;
+                const T dxhat = d[j] * sc;
+                s[0] = __builtin_fma(d[j], xm * inv_stdev, s[0]);
+                s[1] += d[j];
+                s[2] = __builtin_fma(dxhat, neg_inv, s[2]);
+                s[3] = __builtin_fma(dxhat * xm, neg_fac, s[3]);
+            }
+    };
+    ordered_partials<TEAM, K, 4>(g, sums, [&](int u, double (&s)[4]) {
+        if (at[u] != kNowhere)
+            terms(s, xv[u], dv[u], at[u]);
+    });
+    double s[4];
+    ordered_exchange<TEAM, K, 4, TEAMS>(s, g, member, state, tag, sums, lds, missing, [&](uint32_t other) {
+        ordered_partials<TEAM, K, 4>(g, sums, [&](int u, double (&r)[4]) {
+            const uint32_t p = place(other, u);
+            if (p == kNowhere)
+                return;
+            T w[VEC], d[VEC];
+            load_vec<T, VEC, !ROWS>(a.x + base + (p >> 1), w);
+            load_vec<T, VEC, !ROWS>(a.dy + base + (p >> 1), d);
+            terms(r, w, d, p);
+        });
+    });
+    if (member == 0 && threadIdx.x == 0)
+    {
+        a.dscale[c] = s[0];
+        a.dbias[c] = s[1];
+        a.dmean[c] = s[2];
+        a.dvar[c] = s[3];
+    }
+    const T dmean_term = s[2] / a.n;
+    const T dvar_term = s[3] * T(2) / a.n_minus_1;
+#pragma unroll
+    for (int u = 0; u < K; ++u)
+        if (at[u] != kNowhere)
+        {
+#pragma unroll
+            for (int j = 0; j < VEC; ++j)
+                xv[u][j] = fma_t(xv[u][j] - m, dvar_term, fma_t(dv[u][j] * sc, inv_stdev, dmean_term));
+            store_once<T, VEC, STREAM>(a.dx + base + (at[u] >> 1), xv[u]);
+        }
+}

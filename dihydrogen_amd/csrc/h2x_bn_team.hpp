@@ -55,7 +55,7 @@ struct TeamGeometry
 // memory behind them is reached unevenly.  Forward, backward in us, piece i -> this (going round three sets of
 // tensors): N 4, C 64, 64^3 108, 175 -> 103, 166; N 8, C 32, 64^3 113, 193 -> 107, 185; copies in these orders 114 -> 98.
 // (Whole teams on one XCD would wait for the slots of that XCD.)
-__device__ __forceinline__ uint32_t team_member(uint32_t i, uint32_t members)
+__host__ __device__ __forceinline__ uint32_t team_member(uint32_t i, uint32_t members)
 {
     const uint32_t xcd = i % kNumXcd, left = members % kNumXcd;
     return xcd * (members / kNumXcd) + (xcd < left ? xcd : left) + i / kNumXcd;

@@ -111,6 +111,7 @@ PyMethodDef s_methods[] = {H2X_ENTRY(h2x_bn_channel_sums_and_sqsums),
                            H2X_ENTRY(h2x_bn_forward_local),
                            H2X_ENTRY(h2x_bn_backward_local),
                            H2X_ENTRY(h2x_bn_team_state_needed),
+                           H2X_ENTRY(h2x_bn_ordered_state_needed),
                            H2X_ENTRY(h2x_bn_team_state_needed_clearing),
                            H2X_ENTRY(h2x_bn_forward_once),
                            H2X_ENTRY(h2x_bn_forward_clearing),

@@ -149,11 +149,13 @@ class BatchNormalization:
 
     def _team_state(self, l: Layout, clearing: bool) -> Optional[torch.Tensor]:
         """Where the workgroups that share a channel exchange its sums; None where no workgroups
-        do.  Smaller channels than 16 K elements need none."""
-        if l.samples * l.spatial_real <= 16384 or l.dtype != capi.F32:
+        do.  Smaller channels than 16 K floats or 4 K doubles need none."""
+        double = l.dtype == capi.F64
+        if l.samples * l.spatial_real <= (4096 if double else 16384) or double and clearing:
             return None
         if self._state is None or self._state_channels < l.channels:
-            nbytes = l.clearing_team_state_bytes if clearing else l.team_state_bytes
+            nbytes = (l.ordered_state_bytes if double else
+                      l.clearing_team_state_bytes if clearing else l.team_state_bytes)
             if nbytes == 0:
                 return None
             self._state = _buffer_of(self.stream, nbytes, torch.uint8, zero=True)

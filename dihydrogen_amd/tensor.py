@@ -191,6 +191,11 @@ class Layout:
         return capi.calls().h2x_bn_team_state_needed(self.dtype, self.samples, self.geometry_address)
 
     @_once
+    def ordered_state_bytes(self) -> int:
+        """The same for calls on double tensors, whose teams add in the order of the staged calls."""
+        return capi.calls().h2x_bn_ordered_state_needed(self.samples, self.geometry_address)
+
+    @_once
     def clearing_team_state_bytes(self) -> int:
         """The same for calls that clear their output's halo."""
         return capi.calls().h2x_bn_team_state_needed_clearing(self.dtype, self.haloed_geometry_address)

@@ -421,21 +421,24 @@ int h2x_bn_backward_local_strided(h2x_dtype dtype,
                                   h2x_stream_t stream);
 
 /**
- * The same again for float tensors that lie alike, reading every element once where
+ * The same again for tensors that lie alike, reading every element once where
  * a channel is held in registers between the sums and the output: by one workgroup
- * (up to about 80000 elements a channel forward and 65000 backward) or by a team of
- * workgroups (larger channels, or few, up to about 4 million elements forward and 2
+ * (up to about 80000 floats a channel forward and 65000 backward) or by a team of
+ * workgroups (larger channels, or few, up to about 4 million floats forward and 2
  * million backward, outputs that do not overlap inputs); otherwise what
  * h2x_bn_forward_local_strided and h2x_bn_backward_local_strided do.  The terms of
- * the sums are the same and are added in fp64, in another order.
+ * the sums are the same and are added in fp64: of floats in another order, of doubles in
+ * the same one (channels of up to half a million doubles, segments beyond 256 elements).
  *
  * team_state: h2x_bn_team_state_bytes() of the number of channels, or more, zeroed
  * once before the first call and then left to these calls, one after another, in any
  * order and of any sizes; null: no teams.  h2x_bn_team_state_needed() is that for calls
- * on tensors like the one given, or 0 where they never use a state.
+ * on float tensors like the one given, or 0 where they never use a state, and
+ * h2x_bn_ordered_state_needed() the same for double tensors.
  */
 size_t h2x_bn_team_state_bytes(int num_channels);
 size_t h2x_bn_team_state_needed(h2x_dtype dtype, int num_samples, const h2x_tensor_geometry* geometry);
+size_t h2x_bn_ordered_state_needed(int num_samples, const h2x_tensor_geometry* geometry);
 int h2x_bn_forward_once(h2x_dtype dtype,
                                  int num_samples,
                                  const h2x_tensor_geometry* x_geometry,
@@ -532,6 +535,20 @@ int h2x_bn_audit_once(int num_samples,
                       unsigned char* counted,
                       unsigned char* stored,
                       size_t elements);
+
+/**
+ * The same for double tensors: of the forward pass (`backward` 0) or the backward pass, by
+ * members of two groups of 256 threads that play `passes` of the staged workgroups each.
+ * `group`, as large: one more than the staged workgroup whose sum an element is added to.
+ */
+int h2x_bn_audit_ordered(int num_samples,
+                         const h2x_tensor_geometry* geometry,
+                         int backward,
+                         unsigned int passes,
+                         unsigned char* counted,
+                         unsigned char* stored,
+                         unsigned short* group,
+                         size_t elements);
 
 /**
  * The local part of a haloed tensor as it lies in memory: the real (allocated)

@@ -1,0 +1,78 @@
+"""The elements that the workgroups which read double tensors once touch (h2x_bn_audit_ordered plays the
+kernels' own indexing): every interior element counts once, in the sum of the staged workgroup that
+adds it in the two-launch calls, and nothing outside the interior is stored."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from dihydrogen_amd import capi
+
+# local shape (innermost first), strides: C, N last
+CASES = [
+    ((56, 56, 3, 5), (1, 56, 3136, 9408)),                        # aligned whole vectors
+    ((33, 33, 33, 2, 3), (1, 33, 1089, 35937, 71874)),            # segments of an odd length: one row each
+    ((17, 17, 2, 9), (1, 17, 289, 578)),                          # segments of 257 to 1023: samples are folded
+    ((300, 3, 7), (1, 300, 900)),
+    ((30, 30, 30, 2, 2), (1, 32, 1024, 32768, 65536)),            # haloed rows, planes and segments
+    ((33, 35, 2, 2, 2), (1, 37, 1443, 5772, 11544)),
+    ((128, 20, 3, 2), (1, 128, 16000, 3000)),                     # samples inside channels
+    ((2, 700, 2, 3), (1, 5, 3600, 7300)),                         # rows of one vector
+    ((2049, 2, 3), (1, 2049, 4098)),                              # one element beyond a tile
+    ((256, 16, 1, 70), (1, 256, 4096, 4096)),                     # more units than groups of a budget
+]
+
+
+def _geometry(shape, strides):
+    g = capi.TensorGeometry()
+    g.num_dims = len(shape)
+    for i, (e, s) in enumerate(zip(shape, strides)):
+        g.local_shape[i], g.strides[i] = e, s
+    return g
+
+
+def _play(shape, strides, backward, passes):
+    size = sum((e - 1) * s for e, s in zip(shape, strides)) + 1
+    counted, stored, group = np.zeros(size, np.uint8), np.zeros(size, np.uint8), np.zeros(size, np.uint16)
+    g = _geometry(shape, strides)
+    status = capi.load().h2x_bn_audit_ordered(shape[-1], ctypes.byref(g), backward, passes, counted.ctypes.data,
+                                              stored.ctypes.data, group.ctypes.data, size)
+    return status, counted, stored, group
+
+
+@pytest.mark.parametrize("passes", [1, 2, 4])
+@pytest.mark.parametrize("backward", [0, 1])
+@pytest.mark.parametrize("shape,strides", CASES)
+def test_every_element_counts_once_in_the_staged_order(shape, strides, backward, passes):
+    status, counted, stored, group = _play(shape, strides, backward, passes)
+    assert status == 0
+    at = sum(np.arange(e).reshape([-1] + [1] * i) * s for i, (e, s) in enumerate(zip(shape, strides)))
+    interior = np.zeros(counted.size, np.uint8)
+    interior[at.ravel()] = 1
+    assert np.array_equal(counted, interior) and np.array_equal(stored, interior)
+    assert np.array_equal(group > 0, interior > 0)
+    # however many groups a member plays, an element belongs to the same one
+    assert np.array_equal(group, _play(shape, strides, backward, 1)[3])
+
+
+@pytest.mark.parametrize("shape,strides", [((16, 16, 5, 4), (1, 16, 256, 1280)),     # short segments
+                                           ((1, 900, 2, 2), (1, 3, 2700, 5400)),     # rows below a vector
+                                           ((64, 64, 64, 4, 64), (1, 64, 4096, 262144, 1048576))])  # too many groups or offsets
+def test_what_runs_in_two_launches(shape, strides):
+    for backward in (0, 1):
+        b = (ctypes.c_ubyte * 16)()
+        status = capi.load().h2x_bn_audit_ordered(shape[-1], ctypes.byref(_geometry(shape, strides)), backward, 1, b, b, b, 16)
+        assert status in (-1, -2)
+
+
+@pytest.mark.parametrize("case,needed", [((8, 32, 33, 33, 33), True), ((8, 64, 1, 56, 56), True), ((1, 200, 1, 40, 40), False),
+                                         ((64, 512, 1, 14, 14), False), ((100, 64, 64, 64, 64), False)])
+def test_state_of_double_tensors(case, needed):
+    n, c, d, h, w = case
+    shape, strides, at = (w, h, d, c, n), [], 1
+    for e in shape:
+        strides.append(at)
+        at *= e
+    lib = capi.load()
+    got = lib.h2x_bn_ordered_state_needed(n, ctypes.byref(_geometry(shape, strides)))
+    assert got == (lib.h2x_bn_team_state_bytes(c) if needed else 0)
