@@ -2795,8 +2795,10 @@ bool team_launch(const G& once, const A<T>* a, bool stream, uint32_t least, uint
 // works its sums out (2 ms against the tens of microseconds of a launch).
 constexpr uint32_t kTeamPolls = 2048;
 // Workgroups from which a size of member is taken: smaller members where larger ones would be
-// fewer.  Below the last, channels are few and the two-launch kernels cut them finer (N 2, C 4, 40^3).
-constexpr uint32_t kLargeMembers = 384, kMediumMembers = 256, kSmallMembers = 128;
+// fewer.  The smallest ones beat the two launches however few they are (forward + backward, N 2, C 4, 40^3, 64
+// workgroups, 18.5 -> 13.3 us; N 10, C 13, 73 x 78, 91 of them, 19.1 -> 13.7; N 1, C 1, 64^3, 32 of them, 17.0 -> 13.2); a
+// handful is left to them.
+constexpr uint32_t kLargeMembers = 384, kMediumMembers = 256, kSmallMembers = 16;
 
 // CUs of the current device (0: there is none), asked for once: a device does not change, and
 // the question costs a small call most of a microsecond.
@@ -2813,6 +2815,17 @@ uint32_t compute_units()
     return static_cast<uint32_t>(cus);
 }
 
+// Members of 16 vectors a thread fit a CU twice (112 registers): a little more than that on every CU would be a second
+// round that is nearly empty, which smaller members fill (forward, N 1, C 72, 64^3, 576 of them, 30.5 us, by 1152 of half the
+// size 27.2; doubles, N 8, C 32, 33^3, 38.9 and 34.2; 448 of them beat 832, see below).
+template <typename G>
+bool fills_rounds(uint32_t vectors, const G& g)
+{
+    constexpr uint32_t kMember = 512 * 16;
+    const size_t blocks = static_cast<size_t>((vectors + kMember - 1) / kMember) * g.num_channels, slots = 2 * compute_units();
+    return blocks <= slots || blocks >= 2 * slots;
+}
+
 // Forward a member holds 128, 64 or 32 KB (N 16, C 64, 112 x 112 in 448 workgroups of 128 KB 20.4 us, in
 // 832 of 64 KB 22.5; N 2, C 32, 48^3 in 448 of 64 KB 12.0, in 224 of 128 KB 13.0; N 2, C 32, 28^3 with a halo
 // in 224 of 32 KB 6.8 us, in two launches 9.8); up to 128 members (N 16, C 16, 64^3 in 128 of them 98 us, in
@@ -2821,8 +2834,10 @@ template <typename G, typename T>
 bool team_variant(const G& g, const OnceForward<T>* a, bool stream, bool forced, uint32_t most, uint32_t polls,
                   void* team_state, hipStream_t st)
 {
-    return team_launch<512, 16>(g, a, stream, forced ? 1 : kLargeMembers, most, polls, team_state, st)
+    return (fills_rounds(g.vectors, g)
+            && team_launch<512, 16>(g, a, stream, forced ? 1 : kLargeMembers, most, polls, team_state, st))
            || team_launch<512, 8>(g, a, stream, forced ? 1 : kMediumMembers, most, polls, team_state, st)
+           || team_launch<512, 16>(g, a, stream, kLargeMembers, most, polls, team_state, st)
            || team_launch<512, 4>(g, a, stream, kSmallMembers, most, polls, team_state, st);
 }
 
@@ -3021,8 +3036,10 @@ bool ordered_variant(const OrderedGeometry& g, const A* a, bool rows, bool strea
     const auto by_teams = [&] {
         *team = true;
         if constexpr (kForward)
-            return ordered_team<512, 16>(g, a, rows, stream, forced ? 1 : kLargeMembers, most, state, st)
+            return (fills_rounds(static_cast<uint32_t>(vectors), g)
+                    && ordered_team<512, 16>(g, a, rows, stream, forced ? 1 : kLargeMembers, most, state, st))
                    || ordered_team<512, 8>(g, a, rows, stream, forced ? 1 : kMediumMembers, most, state, st)
+                   || ordered_team<512, 16>(g, a, rows, stream, kLargeMembers, most, state, st)
                    || ordered_team<512, 4>(g, a, rows, stream, forced ? 1 : kSmallMembers, most, state, st);
         else
             return ordered_team<512, 8>(g, a, rows, stream, forced ? 1 : kMediumMembers, most / 2, state, st)
