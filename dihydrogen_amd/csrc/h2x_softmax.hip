@@ -62,28 +62,35 @@ struct Pack
     __device__ __forceinline__ T& operator[](int j) { return e[j]; }
     __device__ __forceinline__ const T& operator[](int j) const { return e[j]; }
 
+    // STREAM: past the caches
+    template <bool STREAM = false>
     static __device__ __forceinline__ Pack load(const T* p)
     {
         Pack r;
         if constexpr (VEC == 1)
         {
-            r.e[0] = *p;
+            r.e[0] = STREAM ? __builtin_nontemporal_load(p) : *p;
         }
         else
         {
             typedef T V __attribute__((ext_vector_type(VEC)));
-            const V t = *reinterpret_cast<const V*>(p);
+            const V* const q = reinterpret_cast<const V*>(p);
+            const V t = STREAM ? __builtin_nontemporal_load(q) : *q;
 #pragma unroll
             for (int j = 0; j < VEC; ++j)
                 r.e[j] = t[j];
         }
         return r;
     }
+    template <bool STREAM = false>
     static __device__ __forceinline__ void store(T* p, const Pack& r)
     {
         if constexpr (VEC == 1)
         {
-            *p = r.e[0];
+            if constexpr (STREAM)
+                __builtin_nontemporal_store(r.e[0], p);
+            else
+                *p = r.e[0];
         }
         else
         {
@@ -92,7 +99,10 @@ struct Pack
 #pragma unroll
             for (int j = 0; j < VEC; ++j)
                 t[j] = r.e[j];
-            *reinterpret_cast<V*>(p) = t;
+            if constexpr (STREAM)
+                __builtin_nontemporal_store(t, reinterpret_cast<V*>(p));
+            else
+                *reinterpret_cast<V*>(p) = t;
         }
     }
 };
@@ -119,10 +129,27 @@ __device__ __forceinline__ bool lane_pixels(size_t index, int num_channels, size
     return exists;
 }
 
+// Cache policy.  The backward pass reads the y that the forward pass has written; x and dy are read
+// and dx is written once.  Tensors of which a call's set does not fit the 256 MB memory-side cache
+// are streamed (STREAM): x and dy are loaded and dx is stored past the caches, y alone stays.
+// Forward + backward, us going round three sets of tensors, before -> streamed: N 16, C 21, 256 x 256, 88 MB,
+// 74.6 -> 69.8; N 8, C 32, 256 x 256, 67 MB, 60.3 -> 53.5; N 16, C 500, 48 x 48, 74 MB, 90.5 -> 82.5; N 6, C 19,
+// 256 x 256, 30 MB, 29.8 -> 28.2; N 4, C 100, 128 x 128, 26 MB, 27.3 -> 25.6; below, the caches hold what is read: N 4, C 19,
+// 256 x 256, 20 MB, 20.8 and 21.3, N 2, C 16, 384 x 384, 19 MB, 24.1 and 26.8.  Rows that are no whole
+// vectors share their lines with the tile next door and are not streamed (N 30, C 179, 43 x 43, 40 MB,
+// 49.3 and 52.2; N 16, C 21, 255 x 257 78.5 both ways).  With y past the caches too the first takes 76.9.
+constexpr size_t kStreamBytes = size_t(24) << 20;
+
+template <typename T>
+bool streamed(int vector, int n, int c, size_t s)
+{
+    return vector == static_cast<int>(16 / sizeof(T)) && static_cast<size_t>(n) * c * s * sizeof(T) >= kStreamBytes;
+}
+
 // forward, register-resident.  Replaces fp_channel_kernel, softmax.cu:538-593:
 // running maximum starts at min_normal (positive), the sum is taken in channel
 // order, y = max(e * (1 / sum), min_normal).
-template <typename T, int VEC, int CMAX>
+template <typename T, int VEC, int CMAX, bool STREAM>
 __global__ __launch_bounds__(kBlockSize) void softmax_fwd_reg_kernel(
     const T* __restrict__ x, T* __restrict__ y, int num_channels, size_t spatial, int flat_samples)
 {
@@ -140,7 +167,7 @@ __global__ __launch_bounds__(kBlockSize) void softmax_fwd_reg_kernel(
 #pragma unroll
     for (int c = 0; c < CMAX; ++c)
         if (c < num_channels)
-            v[c] = P::load(xp + static_cast<size_t>(c) * spatial);
+            v[c] = P::template load<STREAM>(xp + static_cast<size_t>(c) * spatial);
 
     T mx[VEC], sum[VEC];
 #pragma unroll
@@ -272,7 +299,7 @@ __global__ __launch_bounds__(kBlockSize) void softmax_fwd_wide_kernel(
 
 // backward, register-resident.  Replaces bp_channel_kernel, softmax.cu:621-669:
 // dp accumulates y*dy in channel order with fused multiply-adds.
-template <typename T, int VEC, int CMAX>
+template <typename T, int VEC, int CMAX, bool STREAM>
 __global__ __launch_bounds__(kBlockSize) void softmax_bwd_reg_kernel(
     const T* __restrict__ y, const T* __restrict__ dy, T* __restrict__ dx, int num_channels,
     size_t spatial, int flat_samples)
@@ -294,7 +321,7 @@ __global__ __launch_bounds__(kBlockSize) void softmax_bwd_reg_kernel(
         if (c < num_channels)
         {
             yv[c] = P::load(yp + static_cast<size_t>(c) * spatial);
-            gv[c] = P::load(gp + static_cast<size_t>(c) * spatial);
+            gv[c] = P::template load<STREAM>(gp + static_cast<size_t>(c) * spatial);
         }
     T dp[VEC];
 #pragma unroll
@@ -313,7 +340,7 @@ __global__ __launch_bounds__(kBlockSize) void softmax_bwd_reg_kernel(
 #pragma unroll
             for (int j = 0; j < VEC; ++j)
                 yv[c][j] = yv[c][j] > kMin ? yv[c][j] * (gv[c][j] - dp[j]) : T(0);
-            P::store(op + static_cast<size_t>(c) * spatial, yv[c]);
+            P::template store<STREAM>(op + static_cast<size_t>(c) * spatial, yv[c]);
         }
 }
 
@@ -406,7 +433,7 @@ __device__ __forceinline__ T sum_of_waves(const T (&lds)[WAVES][N], int i)
 // (N 16, C 150, 128 x 128: 100 us there, 63 us with the tile in registers).  Bound by
 // memory where there are several tiles a CU, else by a wave's chain of loads,
 // exponentials and sums.
-template <typename T, int VEC, int CPW, int WAVES>
+template <typename T, int VEC, int CPW, int WAVES, bool STREAM>
 __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
     const T* __restrict__ x, T* __restrict__ y, int num_channels, size_t spatial, int flat_samples)
 {
@@ -435,7 +462,7 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
 #pragma unroll
         for (int k = 0; k < CPW; ++k)
             if (g + k * WAVES < num_channels)
-                v[k] = P::load(xp + static_cast<size_t>(g + k * WAVES) * spatial);
+                v[k] = P::template load<STREAM>(xp + static_cast<size_t>(g + k * WAVES) * spatial);
 #pragma unroll
         for (int k = 0; k < CPW; ++k)
             if (g + k * WAVES < num_channels)
@@ -497,7 +524,7 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
 // backward likewise: y and dy of up to WAVES * CPW channels in registers.  All of y is
 // asked for before any of dy: alternating, the wave waited more often (N 4, C 150,
 // 65 x 97 in four waves 15.9 us against 10.2).
-template <typename T, int VEC, int CPW, int WAVES>
+template <typename T, int VEC, int CPW, int WAVES, bool STREAM>
 __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
     const T* __restrict__ y, const T* __restrict__ dy, T* __restrict__ dx, int num_channels,
     size_t spatial, int flat_samples)
@@ -529,7 +556,7 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
 #pragma unroll
         for (int k = 0; k < CPW; ++k)
             if (g + k * WAVES < num_channels)
-                gv[k] = P::load(gp + static_cast<size_t>(g + k * WAVES) * spatial);
+                gv[k] = P::template load<STREAM>(gp + static_cast<size_t>(g + k * WAVES) * spatial);
 #pragma unroll
         for (int k = 0; k < CPW; ++k)
             if (g + k * WAVES < num_channels)
@@ -555,7 +582,7 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
 #pragma unroll
                 for (int j = 0; j < VEC; ++j)
                     yv[k][j] = yv[k][j] > kMin ? yv[k][j] * (gv[k][j] - dp[j]) : T(0);
-                P::store(op + static_cast<size_t>(g + k * WAVES) * spatial, yv[k]);
+                P::template store<STREAM>(op + static_cast<size_t>(g + k * WAVES) * spatial, yv[k]);
             }
     }
 }
@@ -814,19 +841,25 @@ dim3 wide_grid(size_t spatial, int vec, int num_samples, int flat)
 }
 
 template <typename T, int VEC, int CMAX>
-void launch_fwd(const T* x, T* y, int n, int c, size_t s, hipStream_t st)
+void launch_fwd(const T* x, T* y, int n, int c, size_t s, bool stream, hipStream_t st)
 {
     const int flat = VEC == 1 ? flat_samples(n, s) : 0;
-    softmax_fwd_reg_kernel<T, VEC, CMAX>
-        <<<pixel_grid_xcd(s, VEC, n, flat), kBlockSize, 0, st>>>(x, y, c, s, flat);
+    const dim3 grid = pixel_grid_xcd(s, VEC, n, flat);
+    if (stream)
+        softmax_fwd_reg_kernel<T, VEC, CMAX, true><<<grid, kBlockSize, 0, st>>>(x, y, c, s, flat);
+    else
+        softmax_fwd_reg_kernel<T, VEC, CMAX, false><<<grid, kBlockSize, 0, st>>>(x, y, c, s, flat);
 }
 
 template <typename T, int VEC, int CMAX>
-void launch_bwd(const T* y, const T* dy, T* dx, int n, int c, size_t s, hipStream_t st)
+void launch_bwd(const T* y, const T* dy, T* dx, int n, int c, size_t s, bool stream, hipStream_t st)
 {
     const int flat = VEC == 1 ? flat_samples(n, s) : 0;
-    softmax_bwd_reg_kernel<T, VEC, CMAX>
-        <<<pixel_grid_xcd(s, VEC, n, flat), kBlockSize, 0, st>>>(y, dy, dx, c, s, flat);
+    const dim3 grid = pixel_grid_xcd(s, VEC, n, flat);
+    if (stream)
+        softmax_bwd_reg_kernel<T, VEC, CMAX, true><<<grid, kBlockSize, 0, st>>>(y, dy, dx, c, s, flat);
+    else
+        softmax_bwd_reg_kernel<T, VEC, CMAX, false><<<grid, kBlockSize, 0, st>>>(y, dy, dx, c, s, flat);
 }
 
 // More samples than this fill the chip with a wave each.
@@ -841,20 +874,26 @@ constexpr int kManySamples = 2048;
 // 29.8 and 34.3.  More channels than the largest tile holds (1024 forward, 768 backward;
 // double: 512 and 256) take the re-reading kernel.
 template <int VEC, int CPW, int WAVES, typename T>
-int launch_split(const T* x, T* y, int n, int c, size_t s, hipStream_t st)
+int launch_split(const T* x, T* y, int n, int c, size_t s, bool stream, hipStream_t st)
 {
     const int flat = VEC == 1 ? flat_samples(n, s) : 0;
-    softmax_fwd_split_kernel<T, VEC, CPW, WAVES>
-        <<<wide_grid(s, VEC, n, flat), WAVES * kWaveSize, 0, st>>>(x, y, c, s, flat);
+    const dim3 grid = wide_grid(s, VEC, n, flat);
+    if (stream)
+        softmax_fwd_split_kernel<T, VEC, CPW, WAVES, true><<<grid, WAVES * kWaveSize, 0, st>>>(x, y, c, s, flat);
+    else
+        softmax_fwd_split_kernel<T, VEC, CPW, WAVES, false><<<grid, WAVES * kWaveSize, 0, st>>>(x, y, c, s, flat);
     return launch_status();
 }
 
 template <int VEC, int CPW, int WAVES, typename T>
-int launch_split(const T* y, const T* dy, T* dx, int n, int c, size_t s, hipStream_t st)
+int launch_split(const T* y, const T* dy, T* dx, int n, int c, size_t s, bool stream, hipStream_t st)
 {
     const int flat = VEC == 1 ? flat_samples(n, s) : 0;
-    softmax_bwd_split_kernel<T, VEC, CPW, WAVES>
-        <<<wide_grid(s, VEC, n, flat), WAVES * kWaveSize, 0, st>>>(y, dy, dx, c, s, flat);
+    const dim3 grid = wide_grid(s, VEC, n, flat);
+    if (stream)
+        softmax_bwd_split_kernel<T, VEC, CPW, WAVES, true><<<grid, WAVES * kWaveSize, 0, st>>>(y, dy, dx, c, s, flat);
+    else
+        softmax_bwd_split_kernel<T, VEC, CPW, WAVES, false><<<grid, WAVES * kWaveSize, 0, st>>>(y, dy, dx, c, s, flat);
     return launch_status();
 }
 
@@ -872,26 +911,27 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
 {
     constexpr bool kForward = sizeof...(P) == 2;
     constexpr bool kFloat = sizeof(T) == 4;
+    const bool stream = streamed<T>(v, n, c, s);
     const int flat = flat_samples(n, s);
     const size_t pixels = flat > 0 ? s * n : s, samples = flat > 0 ? 1 : n;
     const size_t tiles = (pixels + kWaveSize - 1) / kWaveSize * samples;
     if ((tiles <= 256 && c > 64) || c > (kFloat ? 512 : 256))
     {
-        if (c <= 128) return launch_split<1, 8, 16>(p..., n, c, s, st);
-        if (c <= 192) return launch_split<1, 12, 16>(p..., n, c, s, st);
-        if (c <= 256) return launch_split<1, 16, 16>(p..., n, c, s, st);
+        if (c <= 128) return launch_split<1, 8, 16>(p..., n, c, s, stream, st);
+        if (c <= 192) return launch_split<1, 12, 16>(p..., n, c, s, stream, st);
+        if (c <= 256) return launch_split<1, 16, 16>(p..., n, c, s, stream, st);
         if constexpr (kFloat || kForward)
         {
-            if (c <= 384) return launch_split<1, 24, 16>(p..., n, c, s, st);
-            if (c <= 512) return launch_split<1, 32, 16>(p..., n, c, s, st);
+            if (c <= 384) return launch_split<1, 24, 16>(p..., n, c, s, stream, st);
+            if (c <= 512) return launch_split<1, 32, 16>(p..., n, c, s, stream, st);
         }
         if constexpr (kFloat)
         {
-            if (c <= 768) return launch_split<1, 48, 16>(p..., n, c, s, st);
+            if (c <= 768) return launch_split<1, 48, 16>(p..., n, c, s, stream, st);
         }
         if constexpr (kFloat && kForward)
         {
-            if (c <= 1024) return launch_split<1, 64, 16>(p..., n, c, s, st);
+            if (c <= 1024) return launch_split<1, 64, 16>(p..., n, c, s, stream, st);
         }
         return kNoSplit;
     }
@@ -899,20 +939,20 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
     {
         if (v >= 2 && c <= 256 && (s + 2 * kWaveSize - 1) / (2 * kWaveSize) * n >= (kForward ? 512 : 256))
         {
-            if (c <= 64) return launch_split<2, 8, 8>(p..., n, c, s, st);
-            if (c <= 128) return launch_split<2, 16, 8>(p..., n, c, s, st);
-            if (c <= 192) return launch_split<2, 24, 8>(p..., n, c, s, st);
-            return launch_split<2, 32, 8>(p..., n, c, s, st);
+            if (c <= 64) return launch_split<2, 8, 8>(p..., n, c, s, stream, st);
+            if (c <= 128) return launch_split<2, 16, 8>(p..., n, c, s, stream, st);
+            if (c <= 192) return launch_split<2, 24, 8>(p..., n, c, s, stream, st);
+            return launch_split<2, 32, 8>(p..., n, c, s, stream, st);
         }
     }
-    if (c <= 64) return launch_split<1, 8, 8>(p..., n, c, s, st);
-    if (c <= 128) return launch_split<1, 16, 8>(p..., n, c, s, st);
-    if (c <= 192) return launch_split<1, 24, 8>(p..., n, c, s, st);
-    if (c <= 256) return launch_split<1, 32, 8>(p..., n, c, s, st);
+    if (c <= 64) return launch_split<1, 8, 8>(p..., n, c, s, stream, st);
+    if (c <= 128) return launch_split<1, 16, 8>(p..., n, c, s, stream, st);
+    if (c <= 192) return launch_split<1, 24, 8>(p..., n, c, s, stream, st);
+    if (c <= 256) return launch_split<1, 32, 8>(p..., n, c, s, stream, st);
     if constexpr (kFloat)
     {
-        if (c <= 384) return launch_split<1, 48, 8>(p..., n, c, s, st);
-        if (c <= 512) return launch_split<1, 64, 8>(p..., n, c, s, st);
+        if (c <= 384) return launch_split<1, 48, 8>(p..., n, c, s, stream, st);
+        if (c <= 512) return launch_split<1, 64, 8>(p..., n, c, s, stream, st);
     }
     return kNoSplit;
 }
@@ -977,10 +1017,11 @@ int forward_impl(int n, int c, size_t s, const void* xv, void* yv, hipStream_t s
         return launch_status();
     }
     const int v4 = s < kFlatBelow ? 1 : vector_width<T>(s, 4 / kWords, {xv, yv});
+    const bool stream = streamed<T>(v4, n, c, s);
 #define H2X_FWD(V, CM)                                                                             \
     do                                                                                             \
     {                                                                                              \
-        launch_fwd<T, V, CM>(x, y, n, c, s, st);                                                   \
+        launch_fwd<T, V, CM>(x, y, n, c, s, stream, st);                                                \
         return launch_status();                                                                    \
     } while (0)
     if constexpr (sizeof(T) == 4)
@@ -1044,10 +1085,11 @@ int backward_impl(int n, int c, size_t s, const void* yv, const void* dyv, void*
         return launch_status();
     }
     const int v4 = s < kFlatBelow ? 1 : vector_width<T>(s, 4 / kWords, {yv, dyv, dxv});
+    const bool stream = streamed<T>(v4, n, c, s);
 #define H2X_BWD(V, CM)                                                                             \
     do                                                                                             \
     {                                                                                              \
-        launch_bwd<T, V, CM>(y, dy, dx, n, c, s, st);                                              \
+        launch_bwd<T, V, CM>(y, dy, dx, n, c, s, stream, st);                                           \
         return launch_status();                                                                    \
     } while (0)
     if constexpr (sizeof(T) == 4)
