@@ -107,6 +107,15 @@ struct Pack
     }
 };
 
+// The wave of a thread, as the scalar that it is: which channels a wave takes, and where they
+// lie, is then worked out once a wave and not in every lane (1000 vector instructions a wave of
+// softmax_fwd_split_kernel with 24 channels, 560 with it; forward + backward, us: N 16, C 500, 48 x 48 83.0 -> 73.0, N 2,
+// C 900, 30 x 30 72 -> 64, N 30, C 179, 43 x 43 50.0 -> 47.4, N 4, C 150, 65 x 97 19.4 -> 18.6).
+__device__ __forceinline__ int wave_index()
+{
+    return __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+}
+
 // Where the VEC pixels of a lane start (offset of their first channel) and
 // whether they exist; `index` counts the lanes of the grid's x dimension in tile
 // order.  Tensors with few pixels per sample (flat_samples > 0; one pixel a lane)
@@ -223,7 +232,7 @@ __global__ __launch_bounds__(kBlockSize) void softmax_fwd_wide_kernel(
 {
     __shared__ T lds[kWavesPerBlock][kWaveSize];
     const int lane = threadIdx.x % kWaveSize;
-    const int g = threadIdx.x / kWaveSize;
+    const int g = wave_index();
     size_t base;
     const bool active =
         lane_pixels<1>(static_cast<size_t>(xcd_contiguous(blockIdx.x, gridDim.x)) * kWaveSize + lane,
@@ -353,7 +362,7 @@ __global__ __launch_bounds__(kBlockSize) void softmax_bwd_wide_kernel(
 {
     __shared__ T lds[kWavesPerBlock][kWaveSize];
     const int lane = threadIdx.x % kWaveSize;
-    const int g = threadIdx.x / kWaveSize;
+    const int g = wave_index();
     size_t base;
     const bool active =
         lane_pixels<1>(static_cast<size_t>(xcd_contiguous(blockIdx.x, gridDim.x)) * kWaveSize + lane,
@@ -440,7 +449,7 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
     using P = Pack<T, VEC>;
     __shared__ T lds[WAVES][kWaveSize * VEC];
     const int lane = threadIdx.x % kWaveSize;
-    const int g = threadIdx.x / kWaveSize;
+    const int g = wave_index();
     size_t base;
     const bool active = lane_pixels<VEC>(
         static_cast<size_t>(xcd_contiguous(blockIdx.x, gridDim.x)) * kWaveSize + lane, num_channels,
@@ -532,7 +541,7 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
     using P = Pack<T, VEC>;
     __shared__ T lds[WAVES][kWaveSize * VEC];
     const int lane = threadIdx.x % kWaveSize;
-    const int g = threadIdx.x / kWaveSize;
+    const int g = wave_index();
     size_t base;
     const bool active = lane_pixels<VEC>(
         static_cast<size_t>(xcd_contiguous(blockIdx.x, gridDim.x)) * kWaveSize + lane, num_channels,
