@@ -1708,25 +1708,22 @@ int short_elementwise_groups(ShortGeometry* g, int unroll, int budget, size_t pr
     do                                                                                             \
     {                                                                                              \
         if (sg.row % full_vec<T>() == 0)                                                           \
-            KERNEL<T, full_vec<T>(), kTailNone><<<GRID, kBlockSize, 0, stream>>>(__VA_ARGS__);     \
+            launch(KERNEL<T, full_vec<T>(), kTailNone>, GRID, kBlockSize, stream, __VA_ARGS__);    \
         else if (sg.row > full_vec<T>())                                                           \
-            KERNEL<T, full_vec<T>(), kTailOverlap><<<GRID, kBlockSize, 0, stream>>>(__VA_ARGS__);  \
+            launch(KERNEL<T, full_vec<T>(), kTailOverlap>, GRID, kBlockSize, stream, __VA_ARGS__); \
         else                                                                                       \
-            KERNEL<T, full_vec<T>(), kTailScalar><<<GRID, kBlockSize, 0, stream>>>(__VA_ARGS__);   \
+            launch(KERNEL<T, full_vec<T>(), kTailScalar>, GRID, kBlockSize, stream, __VA_ARGS__);  \
     } while (0)
 
 #define H2X_DISPATCH_SHORT_FUSED(KERNEL, FUSED, GRID, ...)                                         \
     do                                                                                             \
     {                                                                                              \
         if (sg.row % full_vec<T>() == 0)                                                           \
-            KERNEL<T, full_vec<T>(), kTailNone, FUSED>                                             \
-                <<<GRID, kBlockSize, 0, stream>>>(__VA_ARGS__);                                    \
+            launch(KERNEL<T, full_vec<T>(), kTailNone, FUSED>, GRID, kBlockSize, stream, __VA_ARGS__);\
         else if (sg.row > full_vec<T>())                                                           \
-            KERNEL<T, full_vec<T>(), kTailOverlap, FUSED>                                          \
-                <<<GRID, kBlockSize, 0, stream>>>(__VA_ARGS__);                                    \
+            launch(KERNEL<T, full_vec<T>(), kTailOverlap, FUSED>, GRID, kBlockSize, stream, __VA_ARGS__);\
         else                                                                                       \
-            KERNEL<T, full_vec<T>(), kTailScalar, FUSED>                                           \
-                <<<GRID, kBlockSize, 0, stream>>>(__VA_ARGS__);                                    \
+            launch(KERNEL<T, full_vec<T>(), kTailScalar, FUSED>, GRID, kBlockSize, stream, __VA_ARGS__);\
     } while (0)
 
 // Launches kernel<T, V, STRIDED> for the width and layout chosen at run time.
@@ -1736,16 +1733,16 @@ int short_elementwise_groups(ShortGeometry* g, int unroll, int budget, size_t pr
         if (strided)                                                                               \
         {                                                                                          \
             if (vw > 1)                                                                            \
-                KERNEL<T, full_vec<T>(), true><<<GRID, kBlockSize, 0, stream>>>(__VA_ARGS__);      \
+                launch(KERNEL<T, full_vec<T>(), true>, GRID, kBlockSize, stream, __VA_ARGS__);     \
             else                                                                                   \
-                KERNEL<T, 1, true><<<GRID, kBlockSize, 0, stream>>>(__VA_ARGS__);                  \
+                launch(KERNEL<T, 1, true>, GRID, kBlockSize, stream, __VA_ARGS__);                 \
         }                                                                                          \
         else                                                                                       \
         {                                                                                          \
             if (vw > 1)                                                                            \
-                KERNEL<T, full_vec<T>(), false><<<GRID, kBlockSize, 0, stream>>>(__VA_ARGS__);     \
+                launch(KERNEL<T, full_vec<T>(), false>, GRID, kBlockSize, stream, __VA_ARGS__);    \
             else                                                                                   \
-                KERNEL<T, 1, false><<<GRID, kBlockSize, 0, stream>>>(__VA_ARGS__);                 \
+                launch(KERNEL<T, 1, false>, GRID, kBlockSize, stream, __VA_ARGS__);                \
         }                                                                                          \
     } while (0)
 
@@ -1754,15 +1751,13 @@ int short_elementwise_groups(ShortGeometry* g, int unroll, int budget, size_t pr
     do                                                                                             \
     {                                                                                              \
         if (vw > 1 && strided)                                                                     \
-            KERNEL<T, full_vec<T>(), kLayoutRows, FUSED>                                           \
-                <<<GRID, kBlockSize, 0, stream>>>(__VA_ARGS__);                                    \
+            launch(KERNEL<T, full_vec<T>(), kLayoutRows, FUSED>, GRID, kBlockSize, stream, __VA_ARGS__);\
         else if (vw > 1)                                                                           \
-            KERNEL<T, full_vec<T>(), kLayoutDense, FUSED>                                          \
-                <<<GRID, kBlockSize, 0, stream>>>(__VA_ARGS__);                                    \
+            launch(KERNEL<T, full_vec<T>(), kLayoutDense, FUSED>, GRID, kBlockSize, stream, __VA_ARGS__);\
         else if (strided)                                                                          \
-            KERNEL<T, 1, kLayoutRows, FUSED><<<GRID, kBlockSize, 0, stream>>>(__VA_ARGS__);        \
+            launch(KERNEL<T, 1, kLayoutRows, FUSED>, GRID, kBlockSize, stream, __VA_ARGS__);       \
         else                                                                                       \
-            KERNEL<T, 1, kLayoutDense, FUSED><<<GRID, kBlockSize, 0, stream>>>(__VA_ARGS__);       \
+            launch(KERNEL<T, 1, kLayoutDense, FUSED>, GRID, kBlockSize, stream, __VA_ARGS__);      \
     } while (0)
 
 // ---- what a launch looks like to the log ----------------------------------------
@@ -1824,7 +1819,7 @@ int zero_outputs(std::initializer_list<void*> outs, int num_channels, hipStream_
     const int blocks = (num_channels + kBlockSize - 1) / kBlockSize;
     for (void* p : outs)
         if (!logged(small_record(kKernelFill, blocks, num_channels)))
-            fill_kernel<T><<<blocks, kBlockSize, 0, stream>>>(static_cast<T*>(p), num_channels, T(0));
+            launch(fill_kernel<T>, blocks, kBlockSize, stream, static_cast<T*>(p), num_channels, T(0));
     return issued();
 }
 
@@ -1907,9 +1902,8 @@ int sums_impl(int num_samples, int num_channels, size_t spatial, const HostTenso
         }
         const unsigned int blocks = (num_channels + kBlockSize - 1) / kBlockSize;
         if (groups > 1 && !logged(small_record(kKernelFinish, blocks, num_channels, 2)))
-            bn_finish_short_kernel<T, 2><<<blocks, kBlockSize, 0, stream>>>(
-                partials, groups, num_channels, static_cast<T*>(sums), static_cast<T*>(sqsums),
-                nullptr, nullptr);
+            launch(bn_finish_short_kernel<T, 2>, blocks, kBlockSize, stream, partials, groups, num_channels,
+                   static_cast<T*>(sums), static_cast<T*>(sqsums), nullptr, nullptr);
         return issued();
     }
     HostTensor tx = tx_in;
@@ -1943,9 +1937,8 @@ int sums_impl(int num_samples, int num_channels, size_t spatial, const HostTenso
         return issued();
     }
     if (groups > 1 && !logged(small_record(kKernelFinish, num_channels, num_channels, 2)))
-        bn_finish_kernel<T, 2><<<num_channels, kBlockSize, 0, stream>>>(
-            partials, static_cast<int>(groups), gmax, static_cast<T*>(sums),
-            static_cast<T*>(sqsums), nullptr, nullptr);
+        launch(bn_finish_kernel<T, 2>, num_channels, kBlockSize, stream, partials, static_cast<int>(groups), gmax,
+               static_cast<T*>(sums), static_cast<T*>(sqsums), nullptr, nullptr);
     return issued();
 }
 
@@ -1957,9 +1950,9 @@ int statistics_impl(int num_channels, size_t num_per_sum, double decay, void* me
         return H2X_SUCCESS;
     const int blocks = std::min((num_channels + kBlockSize - 1) / kBlockSize, 1024);
     if (!logged(small_record(kKernelStatistics, blocks, num_channels)))
-        bn_statistics_kernel<T><<<blocks, kBlockSize, 0, stream>>>(
-            num_channels, num_per_sum, static_cast<T>(decay), static_cast<T*>(mean),
-            static_cast<T*>(var), static_cast<T*>(running_mean), static_cast<T*>(running_var));
+        launch(bn_statistics_kernel<T>, blocks, kBlockSize, stream, num_channels, num_per_sum,
+               static_cast<T>(decay), static_cast<T*>(mean), static_cast<T*>(var), static_cast<T*>(running_mean),
+               static_cast<T*>(running_var));
     return issued();
 }
 
@@ -2054,7 +2047,7 @@ int apply_impl(int num_samples, int num_channels, size_t spatial, const HostTens
                                  static_cast<const T*>(mean), static_cast<const T*>(var),
                                  static_cast<const T*>(scale), static_cast<const T*>(bias),
                                  static_cast<T*>(y), static_cast<T>(epsilon), num_channels, spatial,
-                                 tx.map, ty.map, ch.chunk, ch.chunks_per_seg);
+                                 tx.map, ty.map, ch.chunk, ch.chunks_per_seg, FusedStats<T>());
     return issued();
 }
 
@@ -2099,9 +2092,8 @@ int backprop1_impl(int num_samples, int num_channels, size_t spatial, const Host
         }
         const unsigned int blocks = (num_channels + kBlockSize - 1) / kBlockSize;
         if (groups > 1 && !logged(small_record(kKernelFinish, blocks, num_channels, 4)))
-            bn_finish_short_kernel<T, 4><<<blocks, kBlockSize, 0, stream>>>(
-                partials, groups, num_channels, static_cast<T*>(dscale), static_cast<T*>(dbias),
-                static_cast<T*>(dmean), static_cast<T*>(dvar));
+            launch(bn_finish_short_kernel<T, 4>, blocks, kBlockSize, stream, partials, groups, num_channels,
+                   static_cast<T*>(dscale), static_cast<T*>(dbias), static_cast<T*>(dmean), static_cast<T*>(dvar));
         return issued();
     }
     HostTensor tx = tx_in, td = td_in;
@@ -2138,9 +2130,8 @@ int backprop1_impl(int num_samples, int num_channels, size_t spatial, const Host
         return issued();
     }
     if (groups > 1 && !logged(small_record(kKernelFinish, num_channels, num_channels, 4)))
-        bn_finish_kernel<T, 4><<<num_channels, kBlockSize, 0, stream>>>(
-            partials, static_cast<int>(groups), gmax, static_cast<T*>(dscale),
-            static_cast<T*>(dbias), static_cast<T*>(dmean), static_cast<T*>(dvar));
+        launch(bn_finish_kernel<T, 4>, num_channels, kBlockSize, stream, partials, static_cast<int>(groups), gmax,
+               static_cast<T*>(dscale), static_cast<T*>(dbias), static_cast<T*>(dmean), static_cast<T*>(dvar));
     return issued();
 }
 
@@ -2237,7 +2228,7 @@ int backprop2_impl(int num_samples, int num_channels, size_t spatial, size_t num
                                  static_cast<const T*>(dmean), static_cast<const T*>(dvar),
                                  static_cast<T*>(dx), static_cast<T>(epsilon), num_per_sum,
                                  num_channels, spatial, tx.map, td.map, to.map, ch.chunk,
-                                 ch.chunks_per_seg, disjoint);
+                                 ch.chunks_per_seg, disjoint, FusedStats<T>());
     return issued();
 }
 
@@ -2325,7 +2316,7 @@ int clearing_impl(bool backward, size_t num_per_sum, const h2x_haloed_geometry* 
             return H2X_SUCCESS;
     }
 #define H2X_LAUNCH_CLEARING(VEC, BACKWARD)                                                         \
-    bn_clearing_kernel<T, VEC, BACKWARD><<<grid, kBlockSize, 0, stream>>>(                         \
+    launch(bn_clearing_kernel<T, VEC, BACKWARD>, grid, kBlockSize, stream,                         \
         static_cast<const T*>(x), static_cast<const T*>(dy), static_cast<const T*>(mean),          \
         static_cast<const T*>(var), static_cast<const T*>(scale), static_cast<const T*>(bias),     \
         static_cast<const T*>(dmean), static_cast<const T*>(dvar), static_cast<T*>(out),           \
@@ -2675,7 +2666,7 @@ constexpr unsigned int kOnceManyChannels = 96;
 template <int TEAM, int K, bool STREAM, typename G>
 void issue_once(const G& g, const OnceForward<float>& a, hipStream_t st)
 {
-    bn_once_forward_kernel<float, TEAM, K, STREAM><<<once_grid<TEAM>(g), once_block<TEAM>(), 0, st>>>(g, a);
+    launch(bn_once_forward_kernel<float, TEAM, K, STREAM, G>, once_grid<TEAM>(g), once_block<TEAM>(), st, g, a);
 }
 template <int TEAM, int K, bool STREAM, typename G>
 void issue_once(const G& g, const OnceBackward<float>& a, hipStream_t st)
@@ -2685,7 +2676,8 @@ void issue_once(const G& g, const OnceBackward<float>& a, hipStream_t st)
     // two launches it remains the faster one: N 4, C 256, 112 x 112 with a halo, cleared, backward 47.5 ->
     // 38.7 us, N 2, C 512, 30^3 97 -> 90, N 16, C 1024, 54 x 54 154 -> 142 (going round three sets of tensors).
     constexpr int kInLds = TEAM * K > 8192 ? 9 : 0;
-    bn_once_backward_kernel<float, TEAM, K, STREAM, kInLds><<<once_grid<TEAM>(g), once_block<TEAM>(), 0, st>>>(g, a);
+    launch(bn_once_backward_kernel<float, TEAM, K, STREAM, kInLds, G>, once_grid<TEAM>(g), once_block<TEAM>(), st,
+           g, a);
 }
 
 // A channel fits the registers of one workgroup, in a variant that pays.
@@ -2757,12 +2749,14 @@ bool apart(const void* a, const void* b, size_t bytes)
 template <typename T, int TEAM, int K, bool STREAM, typename G>
 void issue_team(const TeamGeometry<G>& g, const OnceForward<T>& a, unsigned long long* states, hipStream_t st)
 {
-    bn_team_forward_kernel<T, TEAM, K, STREAM><<<g.once.num_channels * g.members.divisor, TEAM, 0, st>>>(g, a, states);
+    launch(bn_team_forward_kernel<T, TEAM, K, STREAM, G>, g.once.num_channels * g.members.divisor, TEAM, st, g, a,
+           states);
 }
 template <typename T, int TEAM, int K, bool STREAM, typename G>
 void issue_team(const TeamGeometry<G>& g, const OnceBackward<T>& a, unsigned long long* states, hipStream_t st)
 {
-    bn_team_backward_kernel<T, TEAM, K, STREAM><<<g.once.num_channels * g.members.divisor, TEAM, 0, st>>>(g, a, states);
+    launch(bn_team_backward_kernel<T, TEAM, K, STREAM, G>, g.once.num_channels * g.members.divisor, TEAM, st, g, a,
+           states);
 }
 
 // Members of TEAM threads with K vectors each; false if that is fewer than `least` workgroups,
@@ -2962,13 +2956,13 @@ template <int TEAM, int K, bool TEAMS, bool ROWS, bool STREAM>
 void issue_ordered(const OrderedGeometry& g, const OnceForward<double>& a, unsigned long long* states, uint32_t blocks,
                    hipStream_t st)
 {
-    bn_ordered_forward_kernel<TEAM, K, TEAMS, ROWS, STREAM><<<blocks, TEAM, 0, st>>>(g, a, states);
+    launch(bn_ordered_forward_kernel<TEAM, K, TEAMS, ROWS, STREAM>, blocks, TEAM, st, g, a, states);
 }
 template <int TEAM, int K, bool TEAMS, bool ROWS, bool STREAM>
 void issue_ordered(const OrderedGeometry& g, const OnceBackward<double>& a, unsigned long long* states, uint32_t blocks,
                    hipStream_t st)
 {
-    bn_ordered_backward_kernel<TEAM, K, TEAMS, ROWS, STREAM><<<blocks, TEAM, 0, st>>>(g, a, states);
+    launch(bn_ordered_backward_kernel<TEAM, K, TEAMS, ROWS, STREAM>, blocks, TEAM, st, g, a, states);
 }
 
 // Groups that a workgroup of TEAM threads with K vectors each holds.

@@ -1118,7 +1118,7 @@ int run_direct(const DirectArgs& a, uint32_t grid, hipStream_t stream)
         audit->workgroups += grid;
         return H2X_SUCCESS;
     }
-    shuffle_direct_kernel<T, FROM><<<dim3(grid), kCopyBlock, 0, stream>>>(a);
+    launch(shuffle_direct_kernel<T, FROM>, dim3(grid), kCopyBlock, stream, a);
     return launch_status();
 }
 

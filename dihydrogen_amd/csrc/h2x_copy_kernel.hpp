@@ -733,7 +733,7 @@ int run_box_copy(uint32_t grid, hipStream_t stream,
         audit->workgroups += grid;
         return H2X_SUCCESS;
     }
-    box_copy_kernel<T, VEC, Op, SPARSE, MODE, TABLE><<<dim3(grid), kCopyBlock, 0, stream>>>(batch, op);
+    launch(box_copy_kernel<T, VEC, Op, SPARSE, MODE, TABLE>, dim3(grid), kCopyBlock, stream, batch, op);
     return launch_status();
 }
 

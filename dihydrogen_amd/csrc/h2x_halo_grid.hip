@@ -338,7 +338,7 @@ int issue_fold(const Args& a, uint32_t blocks, int dim, hipStream_t stream)
         audit->workgroups += blocks;
         return H2X_SUCCESS;
     }
-    halo_fold_kernel<T, Op><<<dim3(blocks), kBlock, 0, stream>>>(a, dim, Op());
+    launch(halo_fold_kernel<T, Op>, dim3(blocks), kBlock, stream, a, dim, Op());
     return launch_status();
 }
 
@@ -373,7 +373,7 @@ int issue(const Args& a, uint32_t blocks, hipStream_t stream)
         audit->workgroups += blocks;
         return H2X_SUCCESS;
     }
-    halo_grid_kernel<T, CLEAR><<<dim3(blocks), kBlock, 0, stream>>>(a);
+    launch(halo_grid_kernel<T, CLEAR>, dim3(blocks), kBlock, stream, a);
     return launch_status();
 }
 

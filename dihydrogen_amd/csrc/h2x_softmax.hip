@@ -855,9 +855,9 @@ void launch_fwd(const T* x, T* y, int n, int c, size_t s, bool stream, hipStream
     const int flat = VEC == 1 ? flat_samples(n, s) : 0;
     const dim3 grid = pixel_grid_xcd(s, VEC, n, flat);
     if (stream)
-        softmax_fwd_reg_kernel<T, VEC, CMAX, true><<<grid, kBlockSize, 0, st>>>(x, y, c, s, flat);
+        launch(softmax_fwd_reg_kernel<T, VEC, CMAX, true>, grid, kBlockSize, st, x, y, c, s, flat);
     else
-        softmax_fwd_reg_kernel<T, VEC, CMAX, false><<<grid, kBlockSize, 0, st>>>(x, y, c, s, flat);
+        launch(softmax_fwd_reg_kernel<T, VEC, CMAX, false>, grid, kBlockSize, st, x, y, c, s, flat);
 }
 
 template <typename T, int VEC, int CMAX>
@@ -866,9 +866,9 @@ void launch_bwd(const T* y, const T* dy, T* dx, int n, int c, size_t s, bool str
     const int flat = VEC == 1 ? flat_samples(n, s) : 0;
     const dim3 grid = pixel_grid_xcd(s, VEC, n, flat);
     if (stream)
-        softmax_bwd_reg_kernel<T, VEC, CMAX, true><<<grid, kBlockSize, 0, st>>>(y, dy, dx, c, s, flat);
+        launch(softmax_bwd_reg_kernel<T, VEC, CMAX, true>, grid, kBlockSize, st, y, dy, dx, c, s, flat);
     else
-        softmax_bwd_reg_kernel<T, VEC, CMAX, false><<<grid, kBlockSize, 0, st>>>(y, dy, dx, c, s, flat);
+        launch(softmax_bwd_reg_kernel<T, VEC, CMAX, false>, grid, kBlockSize, st, y, dy, dx, c, s, flat);
 }
 
 // More samples than this fill the chip with a wave each.
@@ -888,9 +888,9 @@ int launch_split(const T* x, T* y, int n, int c, size_t s, bool stream, hipStrea
     const int flat = VEC == 1 ? flat_samples(n, s) : 0;
     const dim3 grid = wide_grid(s, VEC, n, flat);
     if (stream)
-        softmax_fwd_split_kernel<T, VEC, CPW, WAVES, true><<<grid, WAVES * kWaveSize, 0, st>>>(x, y, c, s, flat);
+        launch(softmax_fwd_split_kernel<T, VEC, CPW, WAVES, true>, grid, WAVES * kWaveSize, st, x, y, c, s, flat);
     else
-        softmax_fwd_split_kernel<T, VEC, CPW, WAVES, false><<<grid, WAVES * kWaveSize, 0, st>>>(x, y, c, s, flat);
+        launch(softmax_fwd_split_kernel<T, VEC, CPW, WAVES, false>, grid, WAVES * kWaveSize, st, x, y, c, s, flat);
     return launch_status();
 }
 
@@ -900,9 +900,11 @@ int launch_split(const T* y, const T* dy, T* dx, int n, int c, size_t s, bool st
     const int flat = VEC == 1 ? flat_samples(n, s) : 0;
     const dim3 grid = wide_grid(s, VEC, n, flat);
     if (stream)
-        softmax_bwd_split_kernel<T, VEC, CPW, WAVES, true><<<grid, WAVES * kWaveSize, 0, st>>>(y, dy, dx, c, s, flat);
+        launch(softmax_bwd_split_kernel<T, VEC, CPW, WAVES, true>, grid, WAVES * kWaveSize, st, y, dy, dx, c, s,
+               flat);
     else
-        softmax_bwd_split_kernel<T, VEC, CPW, WAVES, false><<<grid, WAVES * kWaveSize, 0, st>>>(y, dy, dx, c, s, flat);
+        launch(softmax_bwd_split_kernel<T, VEC, CPW, WAVES, false>, grid, WAVES * kWaveSize, st, y, dy, dx, c, s,
+               flat);
     return launch_status();
 }
 
@@ -1017,12 +1019,12 @@ int forward_impl(int n, int c, size_t s, const void* xv, void* yv, hipStream_t s
     if (s == 1 && c <= 32 * kBlockSize)
         return with_lanes<false>(n, c, [&](auto cpl, auto lanes) {
             constexpr int CPL = decltype(cpl)::value, LANES = decltype(lanes)::value;
-            softmax_fwd_row_kernel<T, CPL, LANES><<<lanes_grid<LANES>(n), lanes_block<LANES>(), 0, st>>>(x, y, c, n);
+            launch(softmax_fwd_row_kernel<T, CPL, LANES>, lanes_grid<LANES>(n), lanes_block<LANES>(), st, x, y, c, n);
             return launch_status();
         });
     if (s == 1)
     {
-        softmax_fwd_long_row_kernel<T><<<n, kBlockSize, 0, st>>>(x, y, c);
+        launch(softmax_fwd_long_row_kernel<T>, n, kBlockSize, st, x, y, c);
         return launch_status();
     }
     const int v4 = s < kFlatBelow ? 1 : vector_width<T>(s, 4 / kWords, {xv, yv});
@@ -1070,7 +1072,7 @@ int forward_impl(int n, int c, size_t s, const void* xv, void* yv, hipStream_t s
     if (status != kNoSplit)
         return status;
     const int flat = flat_samples(n, s);
-    softmax_fwd_wide_kernel<T><<<wide_grid(s, 1, n, flat), kBlockSize, 0, st>>>(x, y, c, s, flat);
+    launch(softmax_fwd_wide_kernel<T>, wide_grid(s, 1, n, flat), kBlockSize, st, x, y, c, s, flat);
     return launch_status();
 }
 
@@ -1085,12 +1087,13 @@ int backward_impl(int n, int c, size_t s, const void* yv, const void* dyv, void*
     if (s == 1 && c <= 32 * kBlockSize)
         return with_lanes<false>(n, c, [&](auto cpl, auto lanes) {
             constexpr int CPL = decltype(cpl)::value, LANES = decltype(lanes)::value;
-            softmax_bwd_row_kernel<T, CPL, LANES><<<lanes_grid<LANES>(n), lanes_block<LANES>(), 0, st>>>(y, dy, dx, c, n);
+            launch(softmax_bwd_row_kernel<T, CPL, LANES>, lanes_grid<LANES>(n), lanes_block<LANES>(), st, y, dy,
+                   dx, c, n);
             return launch_status();
         });
     if (s == 1)
     {
-        softmax_bwd_long_row_kernel<T><<<n, kBlockSize, 0, st>>>(y, dy, dx, c);
+        launch(softmax_bwd_long_row_kernel<T>, n, kBlockSize, st, y, dy, dx, c);
         return launch_status();
     }
     const int v4 = s < kFlatBelow ? 1 : vector_width<T>(s, 4 / kWords, {yv, dyv, dxv});
@@ -1134,7 +1137,7 @@ int backward_impl(int n, int c, size_t s, const void* yv, const void* dyv, void*
     if (status != kNoSplit)
         return status;
     const int flat = flat_samples(n, s);
-    softmax_bwd_wide_kernel<T><<<wide_grid(s, 1, n, flat), kBlockSize, 0, st>>>(y, dy, dx, c, s, flat);
+    launch(softmax_bwd_wide_kernel<T>, wide_grid(s, 1, n, flat), kBlockSize, st, y, dy, dx, c, s, flat);
     return launch_status();
 }
 
@@ -1479,9 +1482,10 @@ int inst_small(int n, size_t sample_size, const void* a, const void* b, void* ou
 {
     return with_lanes<sizeof(T) == 4, kInstLargeLanes<T>>(n, sample_size, [&](auto cpl, auto lanes) {
         constexpr int CPL = decltype(cpl)::value, LANES = decltype(lanes)::value;
-        softmax_inst_small_kernel<T, CPL, MODE, LANES><<<lanes_grid<LANES>(n), lanes_block<LANES>(), 0, st>>>(
-            static_cast<const T*>(a), static_cast<const T*>(b), static_cast<T*>(out), static_cast<const T*>(param),
-            static_cast<T*>(result), static_cast<T*>(result2), static_cast<int>(sample_size), n, min_output);
+        launch(softmax_inst_small_kernel<T, CPL, MODE, LANES>, lanes_grid<LANES>(n), lanes_block<LANES>(), st,
+               static_cast<const T*>(a), static_cast<const T*>(b), static_cast<T*>(out),
+               static_cast<const T*>(param), static_cast<T*>(result), static_cast<T*>(result2),
+               static_cast<int>(sample_size), n, min_output);
         return launch_status();
     });
 }
@@ -1531,13 +1535,13 @@ void inst_partials(int n, size_t sample_size, const void* a, const void* b, void
     const int gmax = inst_groups_per_sample_max(n);
     const dim3 grid(ch.groups, n);
     if (v == kFull)
-        softmax_inst_reduce_kernel<T, kFull, MODE, COMBINE><<<grid, kBlockSize, 0, st>>>(
-            static_cast<const T*>(a), static_cast<const T*>(b), static_cast<T*>(out),
-            static_cast<const T*>(param), partials, sample_size, ch.chunk, gmax, max_partials);
+        launch(softmax_inst_reduce_kernel<T, kFull, MODE, COMBINE>, grid, kBlockSize, st, static_cast<const T*>(a),
+               static_cast<const T*>(b), static_cast<T*>(out), static_cast<const T*>(param), partials, sample_size,
+               ch.chunk, gmax, max_partials);
     else
-        softmax_inst_reduce_kernel<T, 1, MODE, COMBINE><<<grid, kBlockSize, 0, st>>>(
-            static_cast<const T*>(a), static_cast<const T*>(b), static_cast<T*>(out),
-            static_cast<const T*>(param), partials, sample_size, ch.chunk, gmax, max_partials);
+        launch(softmax_inst_reduce_kernel<T, 1, MODE, COMBINE>, grid, kBlockSize, st, static_cast<const T*>(a),
+               static_cast<const T*>(b), static_cast<T*>(out), static_cast<const T*>(param), partials, sample_size,
+               ch.chunk, gmax, max_partials);
 }
 
 template <typename T, int MODE>
@@ -1555,8 +1559,9 @@ int inst_reduce(int n, size_t sample_size, const void* a, const void* b, void* o
     int v;
     double* partials = static_cast<double*>(workspace);
     inst_partials<T, MODE>(n, sample_size, a, b, out, param, partials, st);
-    softmax_inst_finish_kernel<T, MODE == kInstMax><<<n, kBlockSize, 0, st>>>(
-        partials, inst_plan<T>(n, sample_size, a, b, out, &v).groups, inst_groups_per_sample_max(n), static_cast<T*>(result));
+    launch(softmax_inst_finish_kernel<T, MODE == kInstMax>, n, kBlockSize, st, partials,
+           inst_plan<T>(n, sample_size, a, b, out, &v).groups, inst_groups_per_sample_max(n),
+           static_cast<T*>(result));
     return launch_status();
 }
 
@@ -1570,13 +1575,13 @@ int inst_map(int n, size_t sample_size, const void* y, const void* dy, const voi
     const int gmax = inst_groups_per_sample_max(n);
     const T min_output = inst_min_output<T>();
     if (v == kFull)
-        softmax_inst_map_kernel<T, kFull, KIND, COMBINE><<<pixel_grid(sample_size, kFull, n), kBlockSize, 0, st>>>(
-            static_cast<const T*>(y), static_cast<const T*>(dy), static_cast<const T*>(param),
-            static_cast<const T*>(shift), static_cast<T*>(out), sample_size, min_output, sum_partials, gmax);
+        launch(softmax_inst_map_kernel<T, kFull, KIND, COMBINE>, pixel_grid(sample_size, kFull, n), kBlockSize, st,
+               static_cast<const T*>(y), static_cast<const T*>(dy), static_cast<const T*>(param),
+               static_cast<const T*>(shift), static_cast<T*>(out), sample_size, min_output, sum_partials, gmax);
     else
-        softmax_inst_map_kernel<T, 1, KIND, COMBINE><<<pixel_grid(sample_size, 1, n), kBlockSize, 0, st>>>(
-            static_cast<const T*>(y), static_cast<const T*>(dy), static_cast<const T*>(param),
-            static_cast<const T*>(shift), static_cast<T*>(out), sample_size, min_output, sum_partials, gmax);
+        launch(softmax_inst_map_kernel<T, 1, KIND, COMBINE>, pixel_grid(sample_size, 1, n), kBlockSize, st,
+               static_cast<const T*>(y), static_cast<const T*>(dy), static_cast<const T*>(param),
+               static_cast<const T*>(shift), static_cast<T*>(out), sample_size, min_output, sum_partials, gmax);
     return launch_status();
 }
 

@@ -41,6 +41,7 @@ def _share_a_gpu(tensors: Sequence[Tensor]) -> bool:
 
 
 _has_gpu: Optional[bool] = None
+_current_device = _current_stream = None  # torch's bindings, once there is a GPU
 
 
 def _stream_handle(stream: Optional[torch.cuda.Stream]) -> int:
@@ -48,7 +49,13 @@ def _stream_handle(stream: Optional[torch.cuda.Stream]) -> int:
     bindings directly: torch.cuda.current_stream() makes an object first, 2.8 us against 0.2)."""
     if stream is not None:
         return stream.cuda_stream
-    global _has_gpu
+    if _current_stream is not None:
+        return _current_stream(_current_device())
+    return _first_stream_handle()
+
+
+def _first_stream_handle() -> int:
+    global _has_gpu, _current_device, _current_stream
     if _has_gpu is None:
         _has_gpu = torch.cuda.is_available()  # asked once: the answer does not change
         if _has_gpu:
@@ -57,7 +64,8 @@ def _stream_handle(stream: Optional[torch.cuda.Stream]) -> int:
         # no GPU: the null stream; every launch then fails with HIP's own error.  (Launch
         # audits, which play the kernels' indexing on the CPU, ignore the stream.)
         return 0
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    _current_device, _current_stream = torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream
+    return _current_stream(_current_device())
 
 
 def _dense_layout(t: Tensor) -> Layout:
@@ -200,17 +208,20 @@ class BatchNormalization:
 
     def batch_normalization(self, input: Tensor, mean, var, scale, bias, output: Tensor) -> None:
         """batchnorm.hpp:505-517."""
-        lx, ly = _dense_layout(input), _dense_layout(output)
+        lx, ly = input.layout, output.layout
+        if lx.channel_halo or ly.channel_halo:
+            _dense_layout(input), _dense_layout(output)  # raises
         ns = self.num_current_samples
         if self.clear_output_halo and ns == lx.samples and _share_a_haloed_geometry(lx, ly):
             capi.check(self._calls.h2x_bn_batch_normalization_clearing(
                 lx.dtype, ly.haloed_geometry_address, input.get_buffer(), mean, var, scale, bias,
                 output.get_buffer(), self.epsilon, _stream_handle(self.stream)), "batch_normalization (clearing)")
         elif lx.dense and ly.dense:
-            capi.check(self._calls.h2x_bn_batch_normalization(
+            status = self._calls.h2x_bn_batch_normalization(
                 lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ly.spatial_real, input.get_base_ptr(), mean,
-                var, scale, bias, output.get_base_ptr(), self.epsilon, _stream_handle(self.stream)),
-                "batch_normalization")
+                var, scale, bias, output.get_base_ptr(), self.epsilon, _stream_handle(self.stream))
+            if status:
+                capi.check(status, "batch_normalization")
         else:
             capi.check(self._calls.h2x_bn_batch_normalization_strided(
                 lx.dtype, ns, _tensor_geometry(lx, ns), _tensor_geometry(ly, ns), input.get_base_ptr(), mean, var,
@@ -237,7 +248,12 @@ class BatchNormalization:
     def forward(self, input, mean, var, running_mean, running_var, scale, bias, output,
                 is_training: bool = True) -> int:
         lx, ly = input.layout, output.layout
-        local = is_training and self._runs_local(lx)
+        if not is_training:
+            # the stages would do nothing but this: no sums, no all-reduce
+            self.num_current_samples = lx.samples
+            self.batch_normalization(input, running_mean, running_var, scale, bias, output)
+            return 0
+        local = self._runs_local(lx)
         if local and self.clear_output_halo and (lx.haloed or ly.haloed):
             local = False  # the stages, unless a whole pass clears the halo
             if _share_a_haloed_geometry(lx, ly):
@@ -537,7 +553,6 @@ class HaloExchangeAccumOp(Enum):
 
 # what the launches that serve a whole grid refuse (and then launch nothing) goes through buffers
 _NOT_FOR_THE_GRID = (capi.ERR_UNSUPPORTED, capi.ERR_TOO_LARGE)
-_FULL_WIDTHS = (None, None, None, None)  # exchange(): every halo at its full width
 
 
 class HaloExchangeVirtual:
@@ -858,11 +873,10 @@ class HaloExchangeVirtual:
                  op: HaloExchangeAccumOp = HaloExchangeAccumOp.ID, fused: bool = False) -> None:
         """All dimensions, innermost first, each seeing the halo cells the previous
         ones filled (halo_exchange_cuda.hpp:56-106)."""
-        ov = self.tensors[0].overlap
-        given = (widths_rhs_send, widths_rhs_recv, widths_lhs_send, widths_lhs_recv)
         if fused and skip_unpack:
             raise ValueError("a fused exchange has no separate unpack to skip")
-        if (given == _FULL_WIDTHS and (is_reverse or op is HaloExchangeAccumOp.ID) and self.launch_hook is None
+        full = widths_rhs_send is widths_rhs_recv is widths_lhs_send is widths_lhs_recv is None
+        if (full and (is_reverse or op is HaloExchangeAccumOp.ID) and self.launch_hook is None
                 and (fused or not (skip_unpack or self._buffers_wanted))):
             # nobody looks at the receive buffers: straight from tensor to tensor
             grid = self._grid(2 if is_reverse else 1)
@@ -878,8 +892,10 @@ class HaloExchangeVirtual:
                     if not fused:
                         self._direct, self._packed_since = (self._grid_of[0], is_reverse), ()
                     return
-        widths = tuple([ov if w is None else w for w in given])
-        key = ("all", None if given == _FULL_WIDTHS else tuple(map(tuple, widths)), is_reverse, skip_unpack, op, fused, self._addresses())
+        ov = self.tensors[0].overlap
+        widths = tuple([ov if w is None else w
+                        for w in (widths_rhs_send, widths_rhs_recv, widths_lhs_send, widths_lhs_recv)])
+        key = ("all", None if full else tuple(map(tuple, widths)), is_reverse, skip_unpack, op, fused, self._addresses())
         launches = self._faces.get(key)
         if launches is None:
             launches = []
