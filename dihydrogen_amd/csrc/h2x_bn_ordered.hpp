@@ -83,9 +83,9 @@ __device__ __forceinline__ double wave_sum_from(double v, uint32_t first)
         v += dpp_move<kDppQuadSwap2>(v);
     v += dpp_move<kDppRowRor4>(v);
     v += dpp_move<kDppRowRor8>(v);
-    v += __shfl_xor(v, 16, kWaveSize);
-    v += __shfl_xor(v, 32, kWaveSize);
-    return v;
+    const auto add = [](double a, double b) { return a + b; };
+    v = combine_apart<16>(v, add);
+    return combine_apart<32>(v, add);
 }
 
 // The partial sums of the groups that a member plays, in lds as the sums of their four waves:

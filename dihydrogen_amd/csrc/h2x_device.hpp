@@ -94,6 +94,11 @@ constexpr int kDppRowRor4 = 0x124;
 constexpr int kDppRowRor8 = 0x128;
 
 template <int Ctrl>
+__device__ __forceinline__ float dpp_move(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), Ctrl, 0xf, 0xf, false));
+}
+template <int Ctrl>
 __device__ __forceinline__ double dpp_move(double v)
 {
     const long long bits = __double_as_longlong(v);
@@ -105,18 +110,71 @@ __device__ __forceinline__ double dpp_move(double v)
                                 | static_cast<unsigned int>(lo));
 }
 
+// What the two lanes that are D (16 or 32) apart hold, in both of them: the one in the even row
+// (lower half) first.  Swapped in the vector unit; a shuffle goes through LDS, and a reduction is a
+// chain of them that a workgroup waits for (batch-norm forward + backward with shuffles -> with swaps: doubles, N 8,
+// C 32, 33^3, 88.3 -> 86.8 us; N 8, C 64, 56 x 56 14.5 -> 14.3; N 8, C 64, 30^3 with a halo 77.1 -> 76.6).
+template <int D>
+__device__ __forceinline__ void lanes_apart(uint32_t v, uint32_t* even, uint32_t* odd)
+{
+    static_assert(D == 16 || D == 32, "rows of 16 lanes, or halves of the wave");
+    const auto p = D == 16 ? __builtin_amdgcn_permlane16_swap(v, v, false, false)
+                           : __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    *even = p[0];
+    *odd = p[1];
+}
+template <int D>
+__device__ __forceinline__ void lanes_apart(float v, float* even, float* odd)
+{
+    uint32_t e, o;
+    lanes_apart<D>(__float_as_uint(v), &e, &o);
+    *even = __uint_as_float(e);
+    *odd = __uint_as_float(o);
+}
+template <int D>
+__device__ __forceinline__ void lanes_apart(double v, double* even, double* odd)
+{
+    const unsigned long long bits = __double_as_longlong(v);
+    uint32_t el, ol, eh, oh;
+    lanes_apart<D>(static_cast<uint32_t>(bits), &el, &ol);
+    lanes_apart<D>(static_cast<uint32_t>(bits >> 32), &eh, &oh);
+    *even = __longlong_as_double(static_cast<long long>(static_cast<unsigned long long>(eh) << 32 | el));
+    *odd = __longlong_as_double(static_cast<long long>(static_cast<unsigned long long>(oh) << 32 | ol));
+}
+
+// v combined with what the lane D apart holds; f is commutative.
+template <int D, typename T, typename F>
+__device__ __forceinline__ T combine_apart(T v, const F& f)
+{
+    T even, odd;
+    lanes_apart<D>(v, &even, &odd);
+    return f(even, odd);
+}
+
 // Sum over the 64 lanes of a wave; every lane returns the total.  The
 // combination order is fixed (distance 1, 2, 4, 8 inside a row, then rows 16
 // and 32 apart), so the result does not depend on scheduling.
 __device__ __forceinline__ double wave_sum(double v)
 {
+    const auto add = [](double a, double b) { return a + b; };
     v += dpp_move<kDppQuadSwap1>(v);
     v += dpp_move<kDppQuadSwap2>(v);
     v += dpp_move<kDppRowRor4>(v);
     v += dpp_move<kDppRowRor8>(v);
-    v += __shfl_xor(v, 16, kWaveSize);
-    v += __shfl_xor(v, 32, kWaveSize);
-    return v;
+    v = combine_apart<16>(v, add);
+    return combine_apart<32>(v, add);
+}
+
+// Butterfly over the 64 lanes of a wave, 32 apart first: f is commutative, and every lane returns the same.
+template <typename T, typename F>
+__device__ __forceinline__ T wave_combine(T v, const F& f)
+{
+    v = combine_apart<32>(v, f);
+    v = combine_apart<16>(v, f);
+    v = f(v, dpp_move<kDppRowRor8>(v));
+    v = f(v, dpp_move<kDppRowRor4>(v)); // lanes 8 apart hold the same: 4 to the right is as good as 4 apart
+    v = f(v, dpp_move<kDppQuadSwap2>(v));
+    return f(v, dpp_move<kDppQuadSwap1>(v));
 }
 
 // Sum of K values per thread over a 256-thread workgroup.  `lds` must hold

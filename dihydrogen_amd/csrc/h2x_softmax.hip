@@ -599,16 +599,13 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
 // One pixel per sample (the output of a fully connected layer): the channels of
 // a sample are contiguous, so a wave takes a sample, lane l the channels l,
 // l + 64, ... (CPL of them at most), and maxima, sums and dot products are
-// combined across the lanes with a butterfly of shuffles.  The kernels above
+// combined across the lanes with a butterfly of permutes.  The kernels above
 // would put one sample on each lane and read with a stride of C elements
 // (N 256, C 1000: 176 us).
 template <typename T>
 __device__ __forceinline__ T wave_butterfly_sum(T v)
 {
-#pragma unroll
-    for (int m = kWaveSize / 2; m >= 1; m >>= 1)
-        v += __shfl_xor(v, m, kWaveSize);
-    return v;
+    return wave_combine(v, [](T p, T q) { return p + q; });
 }
 
 // Maximum or sum over a workgroup: the lanes of a wave as a butterfly, the waves pairwise.
@@ -616,9 +613,7 @@ template <int WAVES, typename T>
 __device__ __forceinline__ T block_combine(T v, bool is_max, T* lds)
 {
     const auto both = [is_max](T p, T q) { return is_max ? (q > p ? q : p) : p + q; };
-#pragma unroll
-    for (int m = kWaveSize / 2; m >= 1; m >>= 1)
-        v = both(v, __shfl_xor(v, m, kWaveSize));
+    v = wave_combine(v, both);
     __syncthreads(); // lds may still be read from the previous call
     if ((threadIdx.x & (kWaveSize - 1)) == 0)
         lds[threadIdx.x / kWaveSize] = v;
@@ -638,13 +633,7 @@ __device__ __forceinline__ T block_combine(T v, bool is_max, T* lds)
 template <typename T>
 __device__ __forceinline__ T wave_max(T v)
 {
-#pragma unroll
-    for (int d = 1; d < kWaveSize; d *= 2)
-    {
-        const T o = __shfl_xor(v, d, kWaveSize);
-        v = o > v ? o : v;
-    }
-    return v;
+    return wave_combine(v, [](T p, T q) { return q > p ? q : p; });
 }
 
 // The same over the LANES threads that serve a sample: a wave, or a workgroup of that many threads.
