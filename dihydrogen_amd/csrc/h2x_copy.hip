@@ -28,6 +28,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <new>
 #include <vector>
 
@@ -1021,6 +1022,22 @@ namespace
 // runs; the last vector of a run that is no whole number of vectors starts early
 // and moves a few elements twice (the source is not written meanwhile, so both
 // stores agree), runs shorter than a vector move element by element.
+//
+// Lines.  Where one side holds whole rows and the other parts of them, the boxes of
+// the parts (a "line") share the whole rows' lines of memory: served by different
+// XCDs, each fetches such a line for itself, or writes its part of it back to memory.
+// The workgroups of a line's boxes for the same rows therefore follow one another on
+// one XCD, and each moves whole rows, so that the boxes of a line stay abreast.  There
+// and back, N x C x H x W fp32, one line a box and then this: 64 x 225 x 20 x 26 on
+// 16 ranks of 4 x 4 57.8 -> 25.3 us, 97 x 30 x 69 x 66 on 4 x 4 66 -> 47,
+// 32 x 32 x 96 x 96 on 4 x 2 31 -> 26, 32 x 64 x 130 x 120 on 2 x 2 112 -> 89.
+// Not where the parts are whole lines of memory, and nothing is shared (32 x 32 x 128
+// x 128 on 2 x 2 41.4 and 41.8, all loads as below), nor for runs of kilobytes.
+//
+// Loads stream past the caches in shuffles of 64 MiB and more: a smaller tensor's
+// lines are served by the memory-side cache the next time (there and back, streamed
+// and not: 14 x 14 x 217 x 121 21.2 and 17.3 us, 97 x 30 x 69 x 66 52.7 and 47.8,
+// 32 x 32 x 128 x 128 41.8 and 50.4, 32 x 48 x 130 x 130 71.8 and 79.6).
 
 struct DirectBox
 {
@@ -1030,50 +1047,66 @@ struct DirectBox
     FastDiv extent[2];
     uint32_t run;
     uint32_t count;       // vectors (or elements)
-    uint32_t first_block;
+    uint32_t per_block;   // of a workgroup
+    uint32_t first_turn;  // of the box's line
     int32_t rank[2];
-    uint32_t reserved;
 };
 
 constexpr int kMaxDirectRanks = 64;
+constexpr uint32_t kXcds = 8;
+constexpr int64_t kLineBytes = 128; // of memory
+constexpr size_t kMaxLineMembers = 16;
+constexpr uint32_t kMaxLineUnits = 64; // four rows of a box in a workgroup
+constexpr int64_t kStreamedBytes = 64ll << 20;
 
 struct DirectArgs
 {
     const DirectBox* table;
-    FastDiv boxes;       // by the number of boxes
-    uint32_t take_turns; // workgroup by workgroup; otherwise one box follows another
+    FastDiv lines;       // by the number of lines
+    FastDiv all_members; // by the boxes of a line times the number of XCDs
+    uint32_t members;    // boxes of a line; they follow one another in the table
+    uint32_t take_turns; // line by line; otherwise one line follows another
     char* tensor[2][kMaxDirectRanks];
 };
 
-// FROM: 0 source to destination, 1 back.
-template <typename T, int FROM, typename Mem>
+// FROM: 0 source to destination, 1 back.  GROUPED: lines of several boxes.
+template <typename T, int FROM, bool GROUPED, bool STREAM, typename Mem>
 __host__ __device__ __forceinline__ void direct_body(const DirectArgs& a, uint32_t block, uint32_t thread,
                                                      const Mem& mem)
 {
     constexpr int VEC = 16 / sizeof(T);
-    uint32_t b, local_block;
-    if (a.take_turns) // with 8 or 16 boxes each is served by one XCD
+    uint32_t turn = block, member = 0;
+    if constexpr (GROUPED) // workgroups go to the XCDs round-robin: those of one turn are kXcds apart
     {
-        local_block = fastdiv(block, a.boxes);
-        b = block - local_block * a.boxes.divisor;
+        const uint32_t all = fastdiv(block, a.all_members);
+        const uint32_t in = block - all * a.all_members.divisor;
+        member = in / kXcds;
+        turn = all * kXcds + in % kXcds;
+    }
+    uint32_t line, local_turn;
+    if (a.take_turns) // with 8 or 16 lines each is served by one XCD
+    {
+        local_turn = fastdiv(turn, a.lines);
+        line = turn - local_turn * a.lines.divisor;
     }
     else
     {
-        uint32_t end = a.boxes.divisor;
-        b = 0;
-        while (end - b > 1)
+        uint32_t end = a.lines.divisor;
+        line = 0;
+        while (end - line > 1)
         {
-            const uint32_t mid = (b + end) / 2;
-            if (block >= a.table[mid].first_block)
-                b = mid;
+            const uint32_t mid = (line + end) / 2;
+            if (turn >= a.table[mid * a.members].first_turn)
+                line = mid;
             else
                 end = mid;
         }
-        local_block = block - a.table[b].first_block;
+        local_turn = turn - a.table[line * a.members].first_turn;
     }
-    const DirectBox box = a.table[b];
-    const uint32_t at = local_block * kCopyBlock + thread;
-    if (at >= box.count)
+    const DirectBox box = a.table[GROUPED ? line * a.members + member : line];
+    const uint32_t per_block = GROUPED ? box.per_block : kCopyBlock;
+    const uint32_t at = local_turn * per_block + thread;
+    if (thread >= per_block || at >= box.count)
         return;
     const uint32_t row = fastdiv(at, box.units);
     uint32_t x = at - row * box.units.divisor;
@@ -1091,7 +1124,10 @@ __host__ __device__ __forceinline__ void direct_body(const DirectArgs& a, uint32
     {
         x *= VEC;
         x = x < box.run - VEC ? x : box.run - VEC;
-        mem.template store<VEC, false>(to + x, mem.template load_last_use<VEC, false>(from + x));
+        if constexpr (!STREAM)
+            mem.template store<VEC, false>(to + x, mem.template load<VEC, false>(from + x));
+        else
+            mem.template store<VEC, false>(to + x, mem.template load_last_use<VEC, false>(from + x));
     }
     else
     {
@@ -1099,13 +1135,13 @@ __host__ __device__ __forceinline__ void direct_body(const DirectArgs& a, uint32
     }
 }
 
-template <typename T, int FROM>
+template <typename T, int FROM, bool GROUPED, bool STREAM>
 __global__ __launch_bounds__(kCopyBlock, 8) void shuffle_direct_kernel(const DirectArgs a)
 {
-    direct_body<T, FROM, DeviceMem>(a, blockIdx.x, threadIdx.x, DeviceMem());
+    direct_body<T, FROM, GROUPED, STREAM, DeviceMem>(a, blockIdx.x, threadIdx.x, DeviceMem());
 }
 
-template <typename T, int FROM>
+template <typename T, int FROM, bool GROUPED, bool STREAM>
 int run_direct(const DirectArgs& a, uint32_t grid, hipStream_t stream)
 {
     if (Audit* const audit = current_audit())
@@ -1113,12 +1149,12 @@ int run_direct(const DirectArgs& a, uint32_t grid, hipStream_t stream)
         const TraceMem mem{audit};
         for (uint32_t block = 0; block < grid; ++block)
             for (uint32_t thread = 0; thread < kCopyBlock; ++thread)
-                direct_body<T, FROM, TraceMem>(a, block, thread, mem);
+                direct_body<T, FROM, GROUPED, STREAM, TraceMem>(a, block, thread, mem);
         ++audit->launches;
         audit->workgroups += grid;
         return H2X_SUCCESS;
     }
-    launch(shuffle_direct_kernel<T, FROM>, dim3(grid), kCopyBlock, stream, a);
+    launch(shuffle_direct_kernel<T, FROM, GROUPED, STREAM>, dim3(grid), kCopyBlock, stream, a);
     return launch_status();
 }
 
@@ -1132,9 +1168,94 @@ struct h2x_shuffle_direct_plan
     std::vector<DirectBox> boxes; // host copy (a plan made while a launch audit is open has no other)
     DirectBox* table = nullptr;   // device copy
     int device = -1;
-    uint32_t grid = 0;
-    bool take_turns = false;
+    uint64_t grid = 0;
+    uint32_t members = 1, lines = 0;
+    bool take_turns = false, grouped = false, stream = false;
 };
+
+namespace h2x
+{
+namespace
+{
+
+// A box and, by side, the line it lies in: the rank and the box beyond the runs.
+struct FoundBox
+{
+    DirectBox box;
+    std::vector<int64_t> line[2];
+};
+
+// Puts the boxes of a line one after another, and says how many workgroups that takes.
+void order_boxes(const std::vector<FoundBox>& found, h2x_shuffle_direct_plan* p)
+{
+    std::map<std::vector<int64_t>, std::vector<const FoundBox*>> lines[2];
+    size_t most[2] = {1, 1};
+    uint32_t longest = 0;
+    for (const FoundBox& f : found)
+    {
+        longest = std::max(longest, f.box.units.divisor);
+        for (int side = 0; side < 2; ++side)
+        {
+            std::vector<const FoundBox*>& l = lines[side][f.line[side]];
+            l.push_back(&f);
+            most[side] = std::max(most[side], l.size());
+        }
+    }
+    const int side = most[1] > most[0];
+    bool parts = false; // lines of memory that boxes share
+    for (const FoundBox& f : found)
+    {
+        int64_t whole = f.box.run | f.box.at[side];
+        for (const int64_t stride : f.box.stride[side])
+            whole |= stride;
+        parts = parts || whole * p->elem_size % kLineBytes != 0;
+    }
+    const bool grouped = parts && most[side] > 1 && most[side] <= kMaxLineMembers && longest <= kMaxLineUnits
+                         && most[side] * lines[side].size() <= 2 * found.size();
+    const size_t members = grouped ? most[side] : 1;
+    std::vector<std::vector<const FoundBox*>> order;
+    if (grouped)
+        for (const auto& l : lines[side])
+            order.push_back(l.second);
+    else
+        for (const FoundBox& f : found)
+            order.push_back({&f});
+    uint64_t total = 0, largest = 0;
+    for (const std::vector<const FoundBox*>& l : order)
+    {
+        uint32_t units = 1;
+        uint64_t turns = 0;
+        for (const FoundBox* f : l)
+            units = std::max(units, f->box.units.divisor);
+        for (size_t m = 0; m < members; ++m)
+        {
+            DirectBox b = {};
+            if (m < l.size())
+            {
+                b = l[m]->box;
+                b.per_block = grouped ? kCopyBlock / units * b.units.divisor : kCopyBlock;
+                turns = std::max<uint64_t>(turns, (static_cast<uint64_t>(b.count) + b.per_block - 1) / b.per_block);
+            }
+            b.first_turn = static_cast<uint32_t>(total);
+            p->boxes.push_back(b);
+        }
+        total += turns;
+        largest = std::max(largest, turns);
+    }
+    // taking turns gives every line as many workgroups as the largest: not with a quarter of them idle
+    const uint64_t turns = largest * order.size();
+    p->take_turns = turns <= total + total / 4;
+    uint64_t grid = p->take_turns ? turns : total;
+    if (grouped)
+        grid = (grid + kXcds - 1) / kXcds * kXcds * members;
+    p->lines = static_cast<uint32_t>(order.size());
+    p->members = static_cast<uint32_t>(members);
+    p->grouped = grouped;
+    p->grid = grid;
+}
+
+} // namespace
+} // namespace h2x
 
 extern "C" int h2x_shuffle_direct_plan_create(int num_dims, int elem_size, int num_ranks,
                                               const h2x_shuffle_part* src, const h2x_shuffle_part* dst,
@@ -1157,66 +1278,84 @@ extern "C" int h2x_shuffle_direct_plan_create(int num_dims, int elem_size, int n
         return static_cast<int>(hipErrorOutOfMemory);
     p->elem_size = elem_size;
     p->num_ranks = num_ranks;
-    for (std::vector<char>& u : p->used)
-        u.assign(num_ranks, 0);
     const uint32_t vec = 16 / elem_size;
-    uint64_t total = 0, most = 0;
+    int64_t elements = 0;
     int err = H2X_SUCCESS;
-    for (int s = 0; s < num_ranks && err == 0; ++s)
-        for (int d = 0; d < num_ranks && err == 0; ++d)
-        {
-            if (!src[s].active || !dst[d].active)
-                continue;
-            int64_t extent[kMaxBoxDims], from = 0, to = 0;
-            bool empty = false;
-            for (int i = 0; i < num_dims; ++i)
+    try
+    {
+        for (std::vector<char>& u : p->used)
+            u.assign(num_ranks, 0);
+        std::vector<FoundBox> found;
+        for (int s = 0; s < num_ranks && err == 0; ++s)
+            for (int d = 0; d < num_ranks && err == 0; ++d)
             {
-                const int64_t lo = std::max(src[s].origin[i], dst[d].origin[i]);
-                const int64_t hi = std::min(src[s].origin[i] + src[s].extent[i], dst[d].origin[i] + dst[d].extent[i]);
-                extent[i] = hi - lo;
-                empty = empty || extent[i] <= 0;
-                from += (lo - src[s].origin[i]) * src[s].stride[i];
-                to += (lo - dst[d].origin[i]) * dst[d].stride[i];
+                if (!src[s].active || !dst[d].active)
+                    continue;
+                int64_t extent[kMaxBoxDims], from = 0, to = 0;
+                bool empty = false;
+                for (int i = 0; i < num_dims; ++i)
+                {
+                    const int64_t lo = std::max(src[s].origin[i], dst[d].origin[i]);
+                    const int64_t hi = std::min(src[s].origin[i] + src[s].extent[i], dst[d].origin[i] + dst[d].extent[i]);
+                    extent[i] = hi - lo;
+                    empty = empty || extent[i] <= 0;
+                    from += (lo - src[s].origin[i]) * src[s].stride[i];
+                    to += (lo - dst[d].origin[i]) * dst[d].stride[i];
+                }
+                if (empty)
+                    continue;
+                const HostBox h = reduce_box(num_dims, extent, dst[d].stride, to, from, src[s].stride);
+                const int runs = h.stride[0] == 1 && h.stride_src[0] == 1; // otherwise single elements
+                if (h.nd - runs > 3)
+                    err = H2X_ERR_UNSUPPORTED;
+                if (h.count >= (1ll << 31))
+                    err = H2X_ERR_TOO_LARGE;
+                if (err != 0)
+                    break;
+                DirectBox b = {};
+                b.at[0] = from;
+                b.at[1] = to;
+                for (int i = 0; i < 3; ++i)
+                {
+                    b.stride[0][i] = i + runs < h.nd ? h.stride_src[i + runs] : 0;
+                    b.stride[1][i] = i + runs < h.nd ? h.stride[i + runs] : 0;
+                }
+                for (int i = 0; i < 2; ++i)
+                    b.extent[i] = make_fastdiv(i + runs < h.nd ? static_cast<uint32_t>(h.extent[i + runs]) : 1u);
+                b.run = runs ? static_cast<uint32_t>(h.extent[0]) : 1u;
+                const uint32_t units = b.run >= vec ? (b.run + vec - 1) / vec : b.run;
+                b.units = make_fastdiv(units);
+                b.count = static_cast<uint32_t>(h.count / b.run) * units;
+                b.rank[0] = s;
+                b.rank[1] = d;
+                p->used[0][s] = p->used[1][d] = 1;
+                elements += h.count;
+                FoundBox f;
+                f.box = b;
+                int beyond = 0;
+                for (int64_t e = 1; beyond < num_dims && e * extent[beyond] <= b.run; ++beyond)
+                    e *= extent[beyond];
+                for (int side = 0; side < 2; ++side)
+                {
+                    f.line[side].push_back(side ? d : s);
+                    for (int i = beyond; i < num_dims; ++i)
+                    {
+                        f.line[side].push_back(std::max(src[s].origin[i], dst[d].origin[i]));
+                        f.line[side].push_back(extent[i]);
+                    }
+                }
+                found.push_back(f);
             }
-            if (empty)
-                continue;
-            const HostBox h = reduce_box(num_dims, extent, dst[d].stride, to, from, src[s].stride);
-            const int runs = h.stride[0] == 1 && h.stride_src[0] == 1; // otherwise single elements
-            if (h.nd - runs > 3)
-                err = H2X_ERR_UNSUPPORTED;
-            if (h.count >= (1ll << 31))
-                err = H2X_ERR_TOO_LARGE;
-            if (err != 0)
-                break;
-            DirectBox b = {};
-            b.at[0] = from;
-            b.at[1] = to;
-            for (int i = 0; i < 3; ++i)
-            {
-                b.stride[0][i] = i + runs < h.nd ? h.stride_src[i + runs] : 0;
-                b.stride[1][i] = i + runs < h.nd ? h.stride[i + runs] : 0;
-            }
-            for (int i = 0; i < 2; ++i)
-                b.extent[i] = make_fastdiv(i + runs < h.nd ? static_cast<uint32_t>(h.extent[i + runs]) : 1u);
-            b.run = runs ? static_cast<uint32_t>(h.extent[0]) : 1u;
-            const uint32_t units = b.run >= vec ? (b.run + vec - 1) / vec : b.run;
-            b.units = make_fastdiv(units);
-            b.count = static_cast<uint32_t>(h.count / b.run) * units;
-            b.rank[0] = s;
-            b.rank[1] = d;
-            p->used[0][s] = p->used[1][d] = 1;
-            b.first_block = static_cast<uint32_t>(total);
-            const uint64_t blocks = (static_cast<uint64_t>(b.count) + kCopyBlock - 1) / kCopyBlock;
-            total += blocks;
-            most = std::max(most, blocks);
-            if (total > 0x7fffffffull)
-                err = H2X_ERR_TOO_LARGE;
-            p->boxes.push_back(b);
-        }
-    // taking turns gives every box as many workgroups as the largest: not with a quarter of them idle
-    const uint64_t turns = most * p->boxes.size();
-    p->take_turns = turns <= total + total / 4 && turns <= 0x7fffffffull;
-    p->grid = static_cast<uint32_t>(p->take_turns ? turns : total);
+        if (err == 0)
+            order_boxes(found, p);
+    }
+    catch (const std::bad_alloc&)
+    {
+        err = static_cast<int>(hipErrorOutOfMemory);
+    }
+    if (err == 0 && p->grid > 0x7fffffffull)
+        err = H2X_ERR_TOO_LARGE;
+    p->stream = elements * elem_size >= kStreamedBytes;
     if (err == 0 && !p->boxes.empty() && !current_audit())
     {
         const size_t bytes = sizeof(DirectBox) * p->boxes.size();
@@ -1271,12 +1410,22 @@ extern "C" int h2x_shuffle_direct(const h2x_shuffle_direct_plan* plan, void* con
     a.table = current_audit() ? plan->boxes.data() : plan->table;
     if (!a.table)
         return H2X_ERR_INVALID_ARGUMENT; // made for an audit
-    a.boxes = make_fastdiv(static_cast<uint32_t>(plan->boxes.size()));
+    a.lines = make_fastdiv(plan->lines);
+    a.members = plan->members;
+    a.all_members = make_fastdiv(plan->members * kXcds);
     a.take_turns = plan->take_turns;
     const auto run = [&](auto element) {
         using T = decltype(element);
-        return backward ? run_direct<T, 1>(a, plan->grid, as_stream(stream))
-                        : run_direct<T, 0>(a, plan->grid, as_stream(stream));
+        const auto way = [&](auto grouped, auto streams) {
+            constexpr bool kGrouped = decltype(grouped)::value, kStream = decltype(streams)::value;
+            const uint32_t grid = static_cast<uint32_t>(plan->grid);
+            return backward ? run_direct<T, 1, kGrouped, kStream>(a, grid, as_stream(stream))
+                            : run_direct<T, 0, kGrouped, kStream>(a, grid, as_stream(stream));
+        };
+        const std::true_type yes;
+        const std::false_type no;
+        return plan->grouped ? plan->stream ? way(yes, yes) : way(yes, no)
+                             : plan->stream ? way(no, yes) : way(no, no);
     };
     switch (plan->elem_size)
     {
