@@ -56,6 +56,10 @@ constexpr uint64_t kMaxBlocks = 0xffffffffu / kBlock; // a launch counts its thr
 // Ranks of a line whose ends a thread loads before it stores any (measured: 1, 2, 4; two hold
 // the fewest registers at the rate of four).
 constexpr int kRanksPerTurn = 2;
+// Rows of a rank from which on the reverse exchange goes line by line: fewer take as long as one thread does
+// (5 x 2 x 14 x 6 x 47 of doubles on 2 x 1 x 4, 660 rows: line by line 8.4 us, rank by rank 7.9; 9 x 8 x 287 x 109
+// on 4 x 2, 5,500 rows: 9.4 and 11.1).
+constexpr int64_t kLineRows = 4096;
 
 // Whole words throughout: a byte cannot be read through the scalar cache, and a
 // workgroup spends most of its time before its first access on what it reads here.
@@ -325,6 +329,86 @@ __global__ __launch_bounds__(kBlock, 8) void halo_fold_kernel(const Args a, int 
     fold_body<T, Op, DeviceMem>(a, blockIdx.x, threadIdx.x, dim, op, DeviceMem());
 }
 
+// Dimension 0 for all ranks of a line in the same thread: the two lines of memory at a
+// seam of two ranks hold what both give and take, and a workgroup per rank reads them
+// twice and writes them back from two XCDs.  RINGS (every rank has both neighbours): a
+// thread serves one end of a row in every rank, so that the upper ends and the next
+// row's lower ends are neighbouring lanes' work; open lines: both sides of every seam,
+// so that no lane is idle.  Reverse exchanges, rank by rank and so (us; N x C x extents
+// on a grid, halo 1 unless noted): 1 x 32 x 128^3 on 2^3, periodic 96.7 -> 87.8 (seam by
+// seam 98.4), 4 x 32 x 64^3 on 1 x 2 x 4 110 -> 97, 8 x 16 x 64^3 of doubles on 2^3,
+// halo 3 173 -> 135, 15 x 8 x 33 x 57 x 45 of doubles on 2^3 43.0 -> 39.5 (end by end
+// 43.3), 8 x 64 x 112^2 on 2 x 2, periodic 15.8 -> 11.7.
+template <typename T, typename Op, bool RINGS, typename Mem>
+__host__ __device__ __forceinline__ void fold_ends_body(const Args& a, uint32_t block, uint32_t thread, Op op,
+                                                        const Mem& mem)
+{
+    constexpr int kCells = RINGS ? 1 : 2;
+    const uint32_t local_block = fastdiv(block, a.lines);
+    const int r = static_cast<int>((block - local_block * a.lines.divisor) * a.line);
+    const uint32_t w = a.width[0];
+    const uint32_t rows = static_cast<uint32_t>(a.rank[r].local[1] + 2 * a.width[1])
+                          * static_cast<uint32_t>(a.rank[r].local[2] + 2 * a.width[2]) * a.outer;
+    const uint32_t at = local_block * kBlock + thread;
+    const uint32_t row = fastdiv(at, RINGS ? a.both_ends : a.halo[0]);
+    if (row >= rows)
+        return;
+    const uint32_t x = at - row * (RINGS ? 2 * w : w);
+    const uint32_t j = x < w ? x : x - w;
+#pragma unroll 1
+    for (int base = 0; base < a.line; base += kRanksPerTurn)
+    {
+        T s[kRanksPerTurn][kCells], t[kRanksPerTurn][kCells];
+        T* to[kRanksPerTurn][kCells];
+        // a boundary cell of k takes a halo cell of its neighbour: the upper one from the lower halo, and so on
+        auto load = [&](int i, int c, const Rank& k, bool upper, const char* neighbour, uint32_t local) {
+            to[i][c] = reinterpret_cast<T*>(k.tensor) + (row * (k.local[0] + 2 * w) + (upper ? k.local[0] : w) + j);
+            s[i][c] = mem.load1(reinterpret_cast<const T*>(neighbour)
+                                + (row * (local + 2 * w) + (upper ? 0 : local + w) + j));
+            t[i][c] = mem.load1(to[i][c]);
+        };
+#pragma unroll
+        for (int i = 0; i < kRanksPerTurn; ++i)
+        {
+            to[i][0] = nullptr;
+            if (base + i >= a.line)
+                continue;
+            const Rank& k = a.rank[r + base + i];
+            if (k.peer[0][1] < 0)
+                continue;
+            const Rank& above = a.rank[k.peer[0][1]];
+            if constexpr (RINGS)
+            {
+                const Rank& below = a.rank[k.peer[0][0]];
+                const bool upper = x >= w;
+                load(i, 0, k, upper, upper ? above.tensor : below.tensor, upper ? above.local[0] : below.local[0]);
+            }
+            else
+            {
+                load(i, 0, k, true, above.tensor, above.local[0]);
+                load(i, 1, above, false, k.tensor, k.local[0]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < kRanksPerTurn; ++i)
+            if (to[i][0])
+            {
+#pragma unroll
+                for (int c = 0; c < kCells; ++c)
+                    mem.store1(to[i][c], op(t[i][c], s[i][c]));
+            }
+    }
+}
+
+template <typename T, typename Op, bool RINGS>
+__global__ __launch_bounds__(kBlock, 8) void halo_fold_ends_kernel(const Args a, Op op)
+{
+    fold_ends_body<T, Op, RINGS, DeviceMem>(a, blockIdx.x, threadIdx.x, op, DeviceMem());
+}
+
+// In place of the dimension: the ends of the rows, line by line.
+constexpr int kRings = -1, kOpenLines = -2;
+
 template <typename T, typename Op>
 int issue_fold(const Args& a, uint32_t blocks, int dim, hipStream_t stream)
 {
@@ -333,12 +417,22 @@ int issue_fold(const Args& a, uint32_t blocks, int dim, hipStream_t stream)
         const TraceMem mem{audit};
         for (uint32_t block = 0; block < blocks; ++block)
             for (uint32_t thread = 0; thread < kBlock; ++thread)
-                fold_body<T, Op, TraceMem>(a, block, thread, dim, Op(), mem);
+                if (dim == kRings)
+                    fold_ends_body<T, Op, true, TraceMem>(a, block, thread, Op(), mem);
+                else if (dim == kOpenLines)
+                    fold_ends_body<T, Op, false, TraceMem>(a, block, thread, Op(), mem);
+                else
+                    fold_body<T, Op, TraceMem>(a, block, thread, dim, Op(), mem);
         ++audit->launches;
         audit->workgroups += blocks;
         return H2X_SUCCESS;
     }
-    launch(halo_fold_kernel<T, Op>, dim3(blocks), kBlock, stream, a, dim, Op());
+    if (dim == kRings)
+        launch(halo_fold_ends_kernel<T, Op, true>, dim3(blocks), kBlock, stream, a, Op());
+    else if (dim == kOpenLines)
+        launch(halo_fold_ends_kernel<T, Op, false>, dim3(blocks), kBlock, stream, a, Op());
+    else
+        launch(halo_fold_kernel<T, Op>, dim3(blocks), kBlock, stream, a, dim, Op());
     return launch_status();
 }
 
@@ -592,6 +686,10 @@ int run_fold(h2x_dtype dtype, const h2x_halo_grid* h, int op, h2x_stream_t strea
     int err = make_args(*h, 2, 0, es, &a);
     if (err != 0)
         return err;
+    const int64_t rows = static_cast<int64_t>(a.rank[0].local[1] + 2 * a.width[1])
+                         * (a.rank[0].local[2] + 2 * a.width[2]) * a.outer;
+    const bool lines = rows >= kLineRows && a.width[0] > 0 && order_into_lines(&a, h->num_ranks);
+    const bool rings = lines && a.rank[0].peer[0][0] >= 0;
     const int64_t vec = 16 / es;
     uint64_t blocks[kMaxSpatial] = {};
     FastDiv units[kMaxSpatial][kMaxRanks];
@@ -610,11 +708,12 @@ int run_fold(h2x_dtype dtype, const h2x_halo_grid* h, int op, h2x_stream_t strea
             vectors[dim][r] = run >= vec;
             const int64_t n = run >= vec ? (run + vec - 1) / vec : std::max<int64_t>(run, 1);
             units[dim][r] = make_fastdiv(static_cast<uint32_t>(n));
-            most = std::max<uint64_t>(most, (n * above + kBlock - 1) / kBlock);
+            const int64_t threads = (dim == 0 && lines ? (rings ? 2 : 1) * run : n) * above;
+            most = std::max<uint64_t>(most, (threads + kBlock - 1) / kBlock);
         }
         if (!any)
             continue;
-        blocks[dim] = most * h->num_ranks;
+        blocks[dim] = most * (dim == 0 && lines ? a.lines.divisor : h->num_ranks);
         if (most > kMaxRankBlocks || blocks[dim] > kMaxBlocks)
             return H2X_ERR_TOO_LARGE;
     }
@@ -628,8 +727,9 @@ int run_fold(h2x_dtype dtype, const h2x_halo_grid* h, int op, h2x_stream_t strea
             a.rank[r].vectors = vectors[dim][r];
         }
         const uint32_t n = static_cast<uint32_t>(blocks[dim]);
-        err = es == 4 ? issue_fold<float>(op, a, n, dim, as_stream(stream))
-                      : issue_fold<double>(op, a, n, dim, as_stream(stream));
+        const int by = dim > 0 || !lines ? dim : rings ? kRings : kOpenLines;
+        err = es == 4 ? issue_fold<float>(op, a, n, by, as_stream(stream))
+                      : issue_fold<double>(op, a, n, by, as_stream(stream));
     }
     return err;
 }
