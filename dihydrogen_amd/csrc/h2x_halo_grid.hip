@@ -688,10 +688,10 @@ int run_fold(h2x_dtype dtype, const h2x_halo_grid* h, int op, h2x_stream_t strea
         return err;
     const int64_t rows = static_cast<int64_t>(a.rank[0].local[1] + 2 * a.width[1])
                          * (a.rank[0].local[2] + 2 * a.width[2]) * a.outer;
-    const bool lines = rows >= kLineRows && a.width[0] > 0 && order_into_lines(&a, h->num_ranks);
+    bool lines = rows >= kLineRows && a.width[0] > 0 && order_into_lines(&a, h->num_ranks);
     const bool rings = lines && a.rank[0].peer[0][0] >= 0;
     const int64_t vec = 16 / es;
-    uint64_t blocks[kMaxSpatial] = {};
+    uint64_t blocks[kMaxSpatial] = {}, longest = 0; // workgroups of the largest line
     FastDiv units[kMaxSpatial][kMaxRanks];
     bool vectors[kMaxSpatial][kMaxRanks];
     for (int dim = 0; dim < kMaxSpatial; ++dim)
@@ -708,14 +708,21 @@ int run_fold(h2x_dtype dtype, const h2x_halo_grid* h, int op, h2x_stream_t strea
             vectors[dim][r] = run >= vec;
             const int64_t n = run >= vec ? (run + vec - 1) / vec : std::max<int64_t>(run, 1);
             units[dim][r] = make_fastdiv(static_cast<uint32_t>(n));
-            const int64_t threads = (dim == 0 && lines ? (rings ? 2 : 1) * run : n) * above;
-            most = std::max<uint64_t>(most, (threads + kBlock - 1) / kBlock);
+            most = std::max<uint64_t>(most, (n * above + kBlock - 1) / kBlock);
+            if (dim == 0)
+                longest = std::max<uint64_t>(longest, ((rings ? 2 : 1) * run * above + kBlock - 1) / kBlock);
         }
         if (!any)
             continue;
-        blocks[dim] = most * (dim == 0 && lines ? a.lines.divisor : h->num_ranks);
+        blocks[dim] = most * h->num_ranks;
         if (most > kMaxRankBlocks || blocks[dim] > kMaxBlocks)
             return H2X_ERR_TOO_LARGE;
+    }
+    // (what can be launched is a matter of the ranks alone)
+    if (lines && blocks[0] > 0)
+    {
+        lines = longest <= kMaxRankBlocks && longest * a.lines.divisor <= kMaxBlocks;
+        blocks[0] = lines ? longest * a.lines.divisor : blocks[0];
     }
     for (int dim = 0; dim < kMaxSpatial && err == 0; ++dim)
     {
