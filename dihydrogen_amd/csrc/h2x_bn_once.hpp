@@ -77,6 +77,7 @@ struct ClearGeometry
 
     uint32_t vectors;     // of one channel, all samples
     FastDiv per_segment;  // vectors of a segment
+    uint32_t last;        // of these: the elements before it
     RealBox box;
     uint32_t stride_n;    // the last element of a channel is less than 2^28 elements from its first
     int64_t stride_c;
@@ -89,7 +90,9 @@ __host__ __device__ __forceinline__ uint32_t once_place(const ClearGeometry& g, 
 {
     static_assert(VEC <= 4, "four bits hold the interior elements");
     const uint32_t n = fastdiv(i, g.per_segment);
-    const uint32_t e = (i - n * g.per_segment.divisor) * VEC;
+    // (a last vector that starts early shares only halo cells with the one before it, which stores the same zeros)
+    const uint32_t first = (i - n * g.per_segment.divisor) * VEC;
+    const uint32_t e = first < g.last ? first : g.last;
     bool inside[VEC];
     interior_mask<VEC>(g.box, e, inside);
     uint32_t mask = 0;
