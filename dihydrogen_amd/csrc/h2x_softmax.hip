@@ -120,10 +120,10 @@ __device__ __forceinline__ int wave_index()
 // whether they exist; `index` counts the lanes of the grid's x dimension in tile
 // order.  Tensors with few pixels per sample (flat_samples > 0; one pixel a lane)
 // count their pixels through all samples, so that a tile of 64 or 256 pixels is
-// full whatever the size of a sample; otherwise blockIdx.y is the sample.
+// full whatever the size of a sample.
 template <int VEC>
 __device__ __forceinline__ bool lane_pixels(size_t index, int num_channels, size_t spatial,
-                                            int flat_samples, size_t* base)
+                                            int flat_samples, size_t* base, unsigned int sample)
 {
     const size_t p = index * VEC;
     if (flat_samples > 0)
@@ -134,8 +134,28 @@ __device__ __forceinline__ bool lane_pixels(size_t index, int num_channels, size
         return exists;
     }
     const bool exists = p < spatial;
-    *base = static_cast<size_t>(blockIdx.y) * num_channels * spatial + (exists ? p : 0);
+    *base = static_cast<size_t>(sample) * num_channels * spatial + (exists ? p : 0);
     return exists;
+}
+
+// The tiles of 64 lanes that a launch consists of: blockIdx.y counts the samples, or (one
+// row of workgroups) per_sample tiles of one sample are followed by those of the next.
+struct WideTiles
+{
+    FastDiv per_sample;
+    unsigned int samples;
+};
+
+template <int VEC>
+__device__ __forceinline__ bool tile_pixels(const WideTiles& t, int num_channels, size_t spatial, int flat_samples,
+                                            size_t* base)
+{
+    const unsigned int tile = xcd_contiguous(blockIdx.x, gridDim.x);
+    const unsigned int n = fastdiv(tile, t.per_sample);
+    const unsigned int sample = blockIdx.y + n;
+    const size_t first = static_cast<size_t>(tile - n * t.per_sample.divisor) * kWaveSize;
+    return lane_pixels<VEC>(first + threadIdx.x % kWaveSize, num_channels, spatial, flat_samples, base, sample)
+           && sample < t.samples;
 }
 
 // Cache policy.  The backward pass reads the y that the forward pass has written; x and dy are read
@@ -166,7 +186,7 @@ __global__ __launch_bounds__(kBlockSize) void softmax_fwd_reg_kernel(
     size_t base;
     if (!lane_pixels<VEC>(static_cast<size_t>(xcd_contiguous(blockIdx.x, gridDim.x)) * kBlockSize
                               + threadIdx.x,
-                          num_channels, spatial, flat_samples, &base))
+                          num_channels, spatial, flat_samples, &base, blockIdx.y))
         return;
     const T* xp = x + base;
     T* yp = y + base;
@@ -228,15 +248,14 @@ constexpr int kWideBatch = 8;
 // running sum over all channels (softmax.cu:565-580).
 template <typename T>
 __global__ __launch_bounds__(kBlockSize) void softmax_fwd_wide_kernel(
-    const T* __restrict__ x, T* __restrict__ y, int num_channels, size_t spatial, int flat_samples)
+    const T* __restrict__ x, T* __restrict__ y, int num_channels, size_t spatial, int flat_samples,
+    const WideTiles tiles)
 {
     __shared__ T lds[kWavesPerBlock][kWaveSize];
     const int lane = threadIdx.x % kWaveSize;
     const int g = wave_index();
     size_t base;
-    const bool active =
-        lane_pixels<1>(static_cast<size_t>(xcd_contiguous(blockIdx.x, gridDim.x)) * kWaveSize + lane,
-                       num_channels, spatial, flat_samples, &base);
+    const bool active = tile_pixels<1>(tiles, num_channels, spatial, flat_samples, &base);
     const T* xp = x + base;
     T* yp = y + base;
     constexpr T kMin = Limits<T>::min_normal;
@@ -317,7 +336,7 @@ __global__ __launch_bounds__(kBlockSize) void softmax_bwd_reg_kernel(
     size_t base;
     if (!lane_pixels<VEC>(static_cast<size_t>(xcd_contiguous(blockIdx.x, gridDim.x)) * kBlockSize
                               + threadIdx.x,
-                          num_channels, spatial, flat_samples, &base))
+                          num_channels, spatial, flat_samples, &base, blockIdx.y))
         return;
     const T* yp = y + base;
     const T* gp = dy + base;
@@ -358,15 +377,14 @@ __global__ __launch_bounds__(kBlockSize) void softmax_bwd_reg_kernel(
 template <typename T>
 __global__ __launch_bounds__(kBlockSize) void softmax_bwd_wide_kernel(
     const T* __restrict__ y, const T* __restrict__ dy, T* __restrict__ dx, int num_channels,
-    size_t spatial, int flat_samples)
+    size_t spatial, int flat_samples,
+    const WideTiles tiles)
 {
     __shared__ T lds[kWavesPerBlock][kWaveSize];
     const int lane = threadIdx.x % kWaveSize;
     const int g = wave_index();
     size_t base;
-    const bool active =
-        lane_pixels<1>(static_cast<size_t>(xcd_contiguous(blockIdx.x, gridDim.x)) * kWaveSize + lane,
-                       num_channels, spatial, flat_samples, &base);
+    const bool active = tile_pixels<1>(tiles, num_channels, spatial, flat_samples, &base);
     const T* yp = y + base;
     const T* gp = dy + base;
     T* op = dx + base;
@@ -444,16 +462,15 @@ __device__ __forceinline__ T sum_of_waves(const T (&lds)[WAVES][N], int i)
 // exponentials and sums.
 template <typename T, int VEC, int CPW, int WAVES, bool STREAM>
 __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
-    const T* __restrict__ x, T* __restrict__ y, int num_channels, size_t spatial, int flat_samples)
+    const T* __restrict__ x, T* __restrict__ y, int num_channels, size_t spatial, int flat_samples,
+    const WideTiles tiles)
 {
     using P = Pack<T, VEC>;
     __shared__ T lds[WAVES][kWaveSize * VEC];
     const int lane = threadIdx.x % kWaveSize;
     const int g = wave_index();
     size_t base;
-    const bool active = lane_pixels<VEC>(
-        static_cast<size_t>(xcd_contiguous(blockIdx.x, gridDim.x)) * kWaveSize + lane, num_channels,
-        spatial, flat_samples, &base);
+    const bool active = tile_pixels<VEC>(tiles, num_channels, spatial, flat_samples, &base);
     const T* xp = x + base;
     T* yp = y + base;
     constexpr T kMin = Limits<T>::min_normal;
@@ -536,16 +553,15 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
 template <typename T, int VEC, int CPW, int WAVES, bool STREAM>
 __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
     const T* __restrict__ y, const T* __restrict__ dy, T* __restrict__ dx, int num_channels,
-    size_t spatial, int flat_samples)
+    size_t spatial, int flat_samples,
+    const WideTiles tiles)
 {
     using P = Pack<T, VEC>;
     __shared__ T lds[WAVES][kWaveSize * VEC];
     const int lane = threadIdx.x % kWaveSize;
     const int g = wave_index();
     size_t base;
-    const bool active = lane_pixels<VEC>(
-        static_cast<size_t>(xcd_contiguous(blockIdx.x, gridDim.x)) * kWaveSize + lane, num_channels,
-        spatial, flat_samples, &base);
+    const bool active = tile_pixels<VEC>(tiles, num_channels, spatial, flat_samples, &base);
     const T* yp = y + base;
     const T* gp = dy + base;
     T* op = dx + base;
@@ -832,10 +848,23 @@ dim3 pixel_grid_xcd(size_t spatial, int vec, int num_samples, int flat)
     return tile_grid(spatial, kBlockSize, vec, num_samples, flat);
 }
 
-// 64 * vec pixels per workgroup.
-dim3 wide_grid(size_t spatial, int vec, int num_samples, int flat)
+// 64 * vec pixels per workgroup.  Tiles are counted through all samples where filling up each
+// sample's to a multiple of the XCDs would leave more than one of nine idle, on the same
+// XCDs for every sample (forward + backward, us, filled up and counted through: N 32, C 300, 14 x 14, 4 tiles
+// a sample, 23.3 and 18.0; N 25, C 120, 24 x 24, 9 tiles, 14.9 and 10.9; N 29, C 338, 24 x 37, 14 tiles,
+// 43.6 and 41.4; but N 30, C 179, 43 x 43, 29 tiles, 47.3 and 48.0, N 8, C 40, 128 x 128, 128 tiles,
+// 20.1 and 21.4: samples one after another reach the memory more evenly).
+dim3 wide_grid(size_t spatial, int vec, int num_samples, int flat, WideTiles* t)
 {
-    return tile_grid(spatial, kWaveSize, vec, num_samples, flat);
+    const dim3 by_sample = tile_grid(spatial, kWaveSize, vec, num_samples, flat);
+    const size_t per_block = static_cast<size_t>(kWaveSize) * vec;
+    const size_t tiles = (spatial + per_block - 1) / per_block;
+    t->samples = flat > 0 ? 1 : num_samples;
+    const bool through = flat == 0 && by_sample.x * static_cast<size_t>(8) > tiles * 9;
+    t->per_sample = make_fastdiv(through ? static_cast<uint32_t>(tiles) : by_sample.x);
+    if (!through)
+        return by_sample;
+    return dim3((static_cast<unsigned int>(tiles) * num_samples + kNumXcd - 1) / kNumXcd * kNumXcd);
 }
 
 template <typename T, int VEC, int CMAX>
@@ -875,11 +904,14 @@ template <int VEC, int CPW, int WAVES, typename T>
 int launch_split(const T* x, T* y, int n, int c, size_t s, bool stream, hipStream_t st)
 {
     const int flat = VEC == 1 ? flat_samples(n, s) : 0;
-    const dim3 grid = wide_grid(s, VEC, n, flat);
+    WideTiles tiles;
+    const dim3 grid = wide_grid(s, VEC, n, flat, &tiles);
     if (stream)
-        launch(softmax_fwd_split_kernel<T, VEC, CPW, WAVES, true>, grid, WAVES * kWaveSize, st, x, y, c, s, flat);
+        launch(softmax_fwd_split_kernel<T, VEC, CPW, WAVES, true>, grid, WAVES * kWaveSize, st, x, y, c, s, flat,
+               tiles);
     else
-        launch(softmax_fwd_split_kernel<T, VEC, CPW, WAVES, false>, grid, WAVES * kWaveSize, st, x, y, c, s, flat);
+        launch(softmax_fwd_split_kernel<T, VEC, CPW, WAVES, false>, grid, WAVES * kWaveSize, st, x, y, c, s, flat,
+               tiles);
     return launch_status();
 }
 
@@ -887,13 +919,14 @@ template <int VEC, int CPW, int WAVES, typename T>
 int launch_split(const T* y, const T* dy, T* dx, int n, int c, size_t s, bool stream, hipStream_t st)
 {
     const int flat = VEC == 1 ? flat_samples(n, s) : 0;
-    const dim3 grid = wide_grid(s, VEC, n, flat);
+    WideTiles tiles;
+    const dim3 grid = wide_grid(s, VEC, n, flat, &tiles);
     if (stream)
         launch(softmax_bwd_split_kernel<T, VEC, CPW, WAVES, true>, grid, WAVES * kWaveSize, st, y, dy, dx, c, s,
-               flat);
+               flat, tiles);
     else
         launch(softmax_bwd_split_kernel<T, VEC, CPW, WAVES, false>, grid, WAVES * kWaveSize, st, y, dy, dx, c, s,
-               flat);
+               flat, tiles);
     return launch_status();
 }
 
@@ -1061,7 +1094,9 @@ int forward_impl(int n, int c, size_t s, const void* xv, void* yv, hipStream_t s
     if (status != kNoSplit)
         return status;
     const int flat = flat_samples(n, s);
-    launch(softmax_fwd_wide_kernel<T>, wide_grid(s, 1, n, flat), kBlockSize, st, x, y, c, s, flat);
+    WideTiles tiles;
+    const dim3 grid = wide_grid(s, 1, n, flat, &tiles);
+    launch(softmax_fwd_wide_kernel<T>, grid, kBlockSize, st, x, y, c, s, flat, tiles);
     return launch_status();
 }
 
@@ -1126,7 +1161,9 @@ int backward_impl(int n, int c, size_t s, const void* yv, const void* dyv, void*
     if (status != kNoSplit)
         return status;
     const int flat = flat_samples(n, s);
-    launch(softmax_bwd_wide_kernel<T>, wide_grid(s, 1, n, flat), kBlockSize, st, y, dy, dx, c, s, flat);
+    WideTiles tiles;
+    const dim3 grid = wide_grid(s, 1, n, flat, &tiles);
+    launch(softmax_bwd_wide_kernel<T>, grid, kBlockSize, st, y, dy, dx, c, s, flat, tiles);
     return launch_status();
 }
 
