@@ -899,7 +899,8 @@ constexpr int kManySamples = 2048;
 // than needed cost time, since every lane walks the whole tile under a predicate.  Eight
 // waves against four, N 4, C 150, 65 x 97: forward 10.2 and 11.7 us; N 1: 5.7 and 8.0; N 16:
 // 29.8 and 34.3.  More channels than the largest tile holds (1024 forward, 768 backward;
-// double: 512 and 256) take the re-reading kernel.
+// double: 512 and 384, with five words of scratch a lane; N 18, C 270, 27 x 40 backward, re-reading 40.3 us, in
+// registers 27.9) take the re-reading kernel.
 template <int VEC, int CPW, int WAVES, typename T>
 int launch_split(const T* x, T* y, int n, int c, size_t s, bool stream, hipStream_t st)
 {
@@ -953,9 +954,9 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
         if (c <= 128) return launch_split<1, 8, 16>(p..., n, c, s, stream, st);
         if (c <= 192) return launch_split<1, 12, 16>(p..., n, c, s, stream, st);
         if (c <= 256) return launch_split<1, 16, 16>(p..., n, c, s, stream, st);
+        if (c <= 384) return launch_split<1, 24, 16>(p..., n, c, s, stream, st);
         if constexpr (kFloat || kForward)
         {
-            if (c <= 384) return launch_split<1, 24, 16>(p..., n, c, s, stream, st);
             if (c <= 512) return launch_split<1, 32, 16>(p..., n, c, s, stream, st);
         }
         if constexpr (kFloat)
