@@ -270,6 +270,11 @@ SIGNATURES = {
                                               c_void_p, c_void_p]),
     "h2x_softmax_instance_backward_local": (c_int, [c_int, c_int, c_size_t, c_void_p, c_void_p, c_void_p, c_void_p,
                                                     c_void_p, c_void_p]),
+    "h2x_softmax_instance_state_needed": (c_size_t, [c_int, c_int, c_size_t]),
+    "h2x_softmax_instance_forward_once": (c_int, [c_int, c_int, c_size_t, c_void_p, c_void_p, c_void_p, c_void_p,
+                                                  c_void_p, c_void_p, c_int, c_void_p]),
+    "h2x_softmax_instance_backward_once": (c_int, [c_int, c_int, c_size_t, c_void_p, c_void_p, c_void_p, c_void_p,
+                                                   c_void_p, c_void_p, c_int, c_void_p]),
     "h2x_halo_size": (c_size_t, [c_int, POINTER(c_int64), c_int, c_int]),
     "h2x_halo_pack_or_unpack": (c_int, [c_int, c_void_p, c_int, POINTER(c_int64), c_int, c_int,
                                         c_int, c_void_p, c_int, c_int, c_int, c_void_p]),

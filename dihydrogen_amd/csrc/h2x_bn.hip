@@ -93,7 +93,6 @@ struct ScopedLaunchLog
 };
 
 // Device address of `scratch` on the current device, looked up once per device.
-constexpr int kMaxDevices = 64;
 std::mutex static_scratch_mutex;
 void* static_scratch_address[kMaxDevices] = {};
 
@@ -2793,21 +2792,6 @@ constexpr uint32_t kTeamPolls = 2048;
 // workgroups, 18.5 -> 13.3 us; N 10, C 13, 73 x 78, 91 of them, 19.1 -> 13.7; N 1, C 1, 64^3, 32 of them, 17.0 -> 13.2); a
 // handful is left to them.
 constexpr uint32_t kLargeMembers = 384, kMediumMembers = 256, kSmallMembers = 16;
-
-// CUs of the current device (0: there is none), asked for once: a device does not change, and
-// the question costs a small call most of a microsecond.
-uint32_t compute_units()
-{
-    static std::atomic<int> known[kMaxDevices];
-    int device = 0, cus = 0;
-    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMaxDevices)
-        return 0;
-    cus = known[device].load(std::memory_order_relaxed);
-    if (cus == 0
-        && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess)
-        known[device].store(cus, std::memory_order_relaxed);
-    return static_cast<uint32_t>(cus);
-}
 
 // Members of 16 vectors a thread fit a CU twice (112 registers): a little more than that on every CU would be a second
 // round that is nearly empty, which smaller members fill (forward, N 1, C 72, 64^3, 576 of them, 30.5 us, by 1152 of half the

@@ -73,21 +73,6 @@ __host__ __device__ __forceinline__ uint32_t ordered_group(const OrderedGeometry
     return (member * g.passes + p) * (TEAM / kBlockSize) + quarter;
 }
 
-// Steps of wave_sum from those that add lanes `first` apart (1, 2 or 4).  Lanes that are no multiple of
-// `first` hold nothing and get nothing.
-__device__ __forceinline__ double wave_sum_from(double v, uint32_t first)
-{
-    if (first < 2)
-        v += dpp_move<kDppQuadSwap1>(v);
-    if (first < 4)
-        v += dpp_move<kDppQuadSwap2>(v);
-    v += dpp_move<kDppRowRor4>(v);
-    v += dpp_move<kDppRowRor8>(v);
-    const auto add = [](double a, double b) { return a + b; };
-    v = combine_apart<16>(v, add);
-    return combine_apart<32>(v, add);
-}
-
 // The partial sums of the groups that a member plays, in lds as the sums of their four waves:
 // sums[group of the member][wave][k].  add(u, s): the terms of a thread's vector u.
 template <int TEAM, int K, int N, typename F>

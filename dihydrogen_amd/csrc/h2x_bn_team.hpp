@@ -61,15 +61,6 @@ __host__ __device__ __forceinline__ uint32_t team_member(uint32_t i, uint32_t me
     return xcd * (members / kNumXcd) + (xcd < left ? xcd : left) + i / kNumXcd;
 }
 
-__device__ __forceinline__ unsigned long long team_load(const unsigned long long* p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void team_store(unsigned long long* p, uint32_t tag, uint32_t half)
-{
-    __hip_atomic_store(p, static_cast<unsigned long long>(tag) << 32 | half, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // The sums of all members in v[] of every thread, given this member's own in v[] of
 // thread 0 and the tag it made of the counter.  recompute(member, sums) is called by the
 // whole workgroup.

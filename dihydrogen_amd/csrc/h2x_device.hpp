@@ -5,6 +5,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+
 #include <cstdint>
 #include <tuple>
 
@@ -177,6 +179,21 @@ __device__ __forceinline__ T wave_combine(T v, const F& f)
     return f(v, dpp_move<kDppQuadSwap1>(v));
 }
 
+// Steps of wave_sum from those that add lanes `first` apart (1, 2 or 4).  Lanes that are no multiple of
+// `first` hold nothing and get nothing.
+__device__ __forceinline__ double wave_sum_from(double v, uint32_t first)
+{
+    if (first < 2)
+        v += dpp_move<kDppQuadSwap1>(v);
+    if (first < 4)
+        v += dpp_move<kDppQuadSwap2>(v);
+    v += dpp_move<kDppRowRor4>(v);
+    v += dpp_move<kDppRowRor8>(v);
+    const auto add = [](double a, double b) { return a + b; };
+    v = combine_apart<16>(v, add);
+    return combine_apart<32>(v, add);
+}
+
 // Sum of K values per thread over a 256-thread workgroup.  `lds` must hold
 // K * kWavesPerBlock doubles.  Every thread returns the totals in v[].
 template <int K>
@@ -204,6 +221,34 @@ __device__ __forceinline__ void block_sum(double (&v)[K], double* lds)
             t += lds[k * kWavesPerBlock + w];
         v[k] = t;
     }
+}
+
+// ---- teams of workgroups ---------------------------------------------------------
+// What the workgroups of a team exchange: 32 bits with the tag of their call.
+__device__ __forceinline__ unsigned long long team_load(const unsigned long long* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void team_store(unsigned long long* p, uint32_t tag, uint32_t half)
+{
+    __hip_atomic_store(p, static_cast<unsigned long long>(tag) << 32 | half, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+constexpr int kMaxDevices = 64;
+
+// CUs of the current device (0: there is none), asked for once: a device does not change, and
+// the question costs a small call most of a microsecond.
+inline uint32_t compute_units()
+{
+    static std::atomic<int> known[kMaxDevices];
+    int device = 0, cus = 0;
+    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMaxDevices)
+        return 0;
+    cus = known[device].load(std::memory_order_relaxed);
+    if (cus == 0
+        && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess)
+        known[device].store(cus, std::memory_order_relaxed);
+    return static_cast<uint32_t>(cus);
 }
 
 // ---- workgroup order ---------------------------------------------------------

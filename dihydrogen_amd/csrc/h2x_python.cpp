@@ -126,6 +126,10 @@ PyMethodDef s_methods[] = {H2X_ENTRY(h2x_bn_channel_sums_and_sqsums),
                            H2X_ENTRY(h2x_softmax_instance_normalize),
                            H2X_ENTRY(h2x_softmax_instance_forward_local),
                            H2X_ENTRY(h2x_softmax_instance_backward_local),
+                           H2X_ENTRY(h2x_softmax_instance_workspace_bytes),
+                           H2X_ENTRY(h2x_softmax_instance_state_needed),
+                           H2X_ENTRY(h2x_softmax_instance_forward_once),
+                           H2X_ENTRY(h2x_softmax_instance_backward_once),
                            H2X_ENTRY(h2x_softmax_instance_dot),
                            H2X_ENTRY(h2x_softmax_instance_gradient),
                            H2X_ENTRY(h2x_halo_pack_or_unpack_batched),

@@ -1206,13 +1206,9 @@ struct InstPartials
     T* result;
 };
 
-// The maximum of a sample from its partials, in every thread.
-template <typename T>
-__device__ __forceinline__ T inst_combine_max(const double* mine, int groups, double* lds)
+// The maximum over a workgroup, in every thread.
+__device__ __forceinline__ double inst_block_max(double m, double* lds)
 {
-    double m = static_cast<double>(Limits<T>::min_normal);
-    for (int g = threadIdx.x; g < groups; g += kBlockSize)
-        m = mine[g] > m ? mine[g] : m;
     m = wave_max(m);
     if ((threadIdx.x & (kWaveSize - 1)) == 0)
         lds[threadIdx.x / kWaveSize] = m;
@@ -1221,7 +1217,17 @@ __device__ __forceinline__ T inst_combine_max(const double* mine, int groups, do
 #pragma unroll
     for (int w = 1; w < kWavesPerBlock; ++w)
         r = lds[w] > r ? lds[w] : r;
-    return static_cast<T>(r);
+    return r;
+}
+
+// The maximum of a sample from its partials, in every thread.
+template <typename T>
+__device__ __forceinline__ T inst_combine_max(const double* mine, int groups, double* lds)
+{
+    double m = static_cast<double>(Limits<T>::min_normal);
+    for (int g = threadIdx.x; g < groups; g += kBlockSize)
+        m = mine[g] > m ? mine[g] : m;
+    return static_cast<T>(inst_block_max(m, lds));
 }
 
 // The sum likewise, in index order.
@@ -1529,11 +1535,25 @@ struct InstChunking
     int groups;
 };
 
-InstChunking inst_chunking(size_t sample_size, int num_samples, int vec)
+// Partials of a sample that a workgroup combines for itself: one a thread.  Samples of more are large enough
+// for the finishing launch not to count.
+constexpr int kInstCombine = kBlockSize;
+
+// Bytes of a chunk up to which a sample is cut into no more chunks than a workgroup combines, or a team
+// holds: 16, 32 or 64 KB for one, two or more samples, which leaves a reduction its workgroups (N 1, 3,000,001
+// floats: max and sum of exponentials 5.8 and 8.0 us, in chunks of 48 KB 6.4 and 10.1; N 2, 2,097,152 4.6 and 8.1 us, in
+// chunks of 32 KB 4.7 and 7.8).
+size_t inst_chunk_bytes(int num_samples)
+{
+    return size_t(kBlockSize) * 16 * (num_samples <= 1 ? 4 : num_samples == 2 ? 8 : 16);
+}
+
+InstChunking inst_chunking(size_t sample_size, int num_samples, int vec, size_t elem_bytes)
 {
     const int gmax = inst_groups_per_sample_max(num_samples);
     const size_t tile = static_cast<size_t>(kBlockSize) * vec * kInstUnroll;
-    size_t chunk = (sample_size + gmax - 1) / gmax;
+    size_t chunk = std::max((sample_size + gmax - 1) / gmax, std::min((sample_size + kInstCombine - 1) / kInstCombine,
+                                                                      inst_chunk_bytes(num_samples) / elem_bytes));
     chunk = (chunk + tile - 1) / tile * tile;
     InstChunking c;
     c.chunk = chunk;
@@ -1547,7 +1567,7 @@ InstChunking inst_plan(int n, size_t sample_size, const void* a, const void* b, 
 {
     constexpr int kFull = 16 / sizeof(T);
     *v = vector_width<T>(sample_size, kFull, {a, b ? b : a, out ? out : a});
-    return inst_chunking(sample_size, n, *v);
+    return inst_chunking(sample_size, n, *v, sizeof(T));
 }
 
 // The partial sums of a reduction at `partials` (groups_max of them a sample); no finishing launch.
@@ -1612,9 +1632,68 @@ int inst_map(int n, size_t sample_size, const void* y, const void* dy, const voi
     return launch_status();
 }
 
-// Partials of a sample that a workgroup combines for itself: one load a thread.  Samples of more are large enough
-// for the finishing launch not to count.
-constexpr int kInstCombine = kBlockSize;
+#include "h2x_softmax_team.hpp"
+
+// Vectors of 16 bytes a thread that members of four chunks hold at most: beyond, 1024 threads lack the registers.
+constexpr int kInstMostForward = 16, kInstMostBackward = 8;
+
+// A team for samples cut as the staged sums are, or false: of up to 64 members of one chunk, or of four (see
+// h2x_softmax_team.hpp).  Members fit a CU once at least, so a team is within a quarter of the chip.
+template <typename T>
+bool inst_team(int n, size_t sample_size, const void* a, const void* b, const void* out, int most, int* v, InstTeam* g)
+{
+    if (sample_size <= kInstSmallSample<T> || n <= 0)
+        return false;
+    const InstChunking ch = inst_plan<T>(n, sample_size, a, b, out, v);
+    const int each = static_cast<int>(ch.chunk / kBlockSize / (16 / sizeof(T))); // vectors of 16 bytes
+    const int chunks = ch.groups <= 64 ? 1 : 4;
+    const int members = (ch.groups + chunks - 1) / chunks;
+    if (ch.groups > kInstCombine || each > (chunks == 1 ? 16 : most) || 4 * members > static_cast<int>(compute_units()))
+        return false;
+    g->members = make_fastdiv(static_cast<uint32_t>(members));
+    g->chunks = static_cast<uint32_t>(chunks);
+    g->sample_size = static_cast<uint32_t>(sample_size); // up to 256 chunks of 64 KB
+    g->chunk = static_cast<uint32_t>(ch.chunk);
+    return true;
+}
+
+// Calls f(threads, elements a vector, vectors a thread) with constants.
+template <typename T, int MOST, typename F>
+void inst_team_variant(const InstTeam& g, int v, const F& f)
+{
+    using std::integral_constant;
+    constexpr int kFull = 16 / sizeof(T);
+    const size_t each = g.chunk / kBlockSize; // elements of a thread
+    const auto with = [&](auto team, auto vec) {
+        constexpr int kMost = kFull * 16 / decltype(vec)::value;
+        constexpr bool kAll = decltype(team)::value == kBlockSize;
+        if (each <= kFull * 4)
+            f(team, vec, integral_constant<int, kMost / 4>());
+        else if (kAll || MOST >= 8)
+        {
+            if (each <= kFull * 8)
+                f(team, vec, integral_constant<int, kAll || MOST >= 8 ? kMost / 2 : kMost / 4>());
+            else if (kAll || MOST >= 16)
+                f(team, vec, integral_constant<int, kAll || MOST >= 16 ? kMost : kMost / 4>());
+        }
+    };
+    const auto wide = [&](auto vec) {
+        if (g.chunks == 1)
+            with(integral_constant<int, kBlockSize>(), vec);
+        else
+            with(integral_constant<int, 4 * kBlockSize>(), vec);
+    };
+    if (v == kFull)
+        wide(integral_constant<int, kFull>());
+    else
+        wide(integral_constant<int, 1>());
+}
+
+bool inst_apart(const void* a, const void* b, size_t bytes)
+{
+    const uintptr_t p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
+    return p + bytes <= q || q + bytes <= p;
+}
 
 // Forward pass of samples that are whole on this rank: maximum, sum of the
 // exponentials (y is not written), y from x: 4 tensor passes instead of 5, and three
@@ -1668,6 +1747,48 @@ int inst_backward_local(int n, size_t sample_size, const void* y, const void* dy
     }
     const int err = inst_reduce<T, kInstDot>(n, sample_size, y, dy, nullptr, nullptr, sample_dp, workspace, st);
     return err ? err : inst_map<T, kMapGradient>(n, sample_size, y, dy, sample_dp, nullptr, dx, st);
+}
+
+// By teams, or false.  polls: looks at what the others have stored, of about a microsecond.
+template <typename T>
+bool inst_forward_team(int n, size_t sample_size, const void* x, void* y, void* sample_max, void* sample_exp,
+                       void* state, uint32_t polls, hipStream_t st)
+{
+    InstTeam g;
+    int v;
+    if (!state || !inst_team<T>(n, sample_size, x, nullptr, y, kInstMostForward, &v, &g)
+        || !inst_apart(x, y, n * sample_size * sizeof(T)))
+        return false;
+    g.max_polls = polls;
+    g.states = static_cast<unsigned long long*>(state);
+    inst_team_variant<T, kInstMostForward>(g, v, [&](auto team, auto vec, auto vectors) {
+        constexpr int TEAM = decltype(team)::value, VEC = decltype(vec)::value, V = decltype(vectors)::value;
+        launch(softmax_inst_team_forward_kernel<T, TEAM, VEC, V>, g.members.divisor * n, TEAM, st,
+               static_cast<const T*>(x), static_cast<T*>(y), static_cast<T*>(sample_max), static_cast<T*>(sample_exp),
+               g, inst_min_output<T>());
+    });
+    return true;
+}
+
+template <typename T>
+bool inst_backward_team(int n, size_t sample_size, const void* y, const void* dy, void* dx, void* sample_dp,
+                        void* state, uint32_t polls, hipStream_t st)
+{
+    InstTeam g;
+    int v;
+    const size_t bytes = n * sample_size * sizeof(T);
+    if (!state || !inst_team<T>(n, sample_size, y, dy, nullptr, kInstMostBackward, &v, &g) || !inst_apart(y, dx, bytes)
+        || !inst_apart(dy, dx, bytes) || vector_width<T>(sample_size, v, {dx}) != v) // the outputs take no part in the cut
+        return false;
+    g.max_polls = polls;
+    g.states = static_cast<unsigned long long*>(state);
+    inst_team_variant<T, kInstMostBackward>(g, v, [&](auto team, auto vec, auto vectors) {
+        constexpr int TEAM = decltype(team)::value, VEC = decltype(vec)::value, V = decltype(vectors)::value;
+        launch(softmax_inst_team_backward_kernel<T, TEAM, VEC, V>, g.members.divisor * n, TEAM, st,
+               static_cast<const T*>(y), static_cast<const T*>(dy), static_cast<T*>(dx), static_cast<T*>(sample_dp), g,
+               inst_min_output<T>());
+    });
+    return true;
 }
 
 bool inst_bad(int num_samples, size_t sample_size)
@@ -1828,4 +1949,55 @@ extern "C" int h2x_softmax_instance_backward_local(h2x_dtype dtype, int num_samp
                                                as_stream(stream))),
                    (inst_backward_local<double>(num_samples, sample_size, y, dy, dx, sample_dp, workspace,
                                                 as_stream(stream))));
+}
+
+// Looks from which a member works out what it misses (2 ms against the microseconds of a launch).
+constexpr int kInstPolls = 2048;
+
+extern "C" size_t h2x_softmax_instance_state_needed(h2x_dtype dtype, int num_samples, size_t sample_size)
+{
+    if ((dtype != H2X_F32 && dtype != H2X_F64) || num_samples <= 0 || inst_bad(num_samples, sample_size))
+        return 0;
+    const auto team = [&](auto zero) {
+        InstTeam g;
+        int v;
+        return inst_team<decltype(zero)>(num_samples, sample_size, nullptr, nullptr, nullptr, kInstMostForward, &v, &g);
+    };
+    return (dtype == H2X_F32 ? team(0.0f) : team(0.0)) ? num_samples * kInstStateWords * sizeof(unsigned long long) : 0;
+}
+
+extern "C" int h2x_softmax_instance_forward_once(h2x_dtype dtype, int num_samples, size_t sample_size, const void* x,
+                                                 void* y, void* sample_max, void* sample_exp, void* workspace,
+                                                 void* state, int max_polls, h2x_stream_t stream)
+{
+    if (!x || !y || !sample_max || !sample_exp || !workspace)
+        return num_samples == 0 || sample_size == 0 ? H2X_SUCCESS : H2X_ERR_INVALID_ARGUMENT;
+    const uint32_t polls = max_polls < 0 ? kInstPolls : max_polls;
+    if (!inst_bad(num_samples, sample_size)
+        && (dtype == H2X_F32   ? inst_forward_team<float>(num_samples, sample_size, x, y, sample_max, sample_exp, state,
+                                                          polls, as_stream(stream))
+            : dtype == H2X_F64 ? inst_forward_team<double>(num_samples, sample_size, x, y, sample_max, sample_exp,
+                                                           state, polls, as_stream(stream))
+                               : false))
+        return launch_status();
+    return h2x_softmax_instance_forward_local(dtype, num_samples, sample_size, x, y, sample_max, sample_exp, workspace,
+                                              stream);
+}
+
+extern "C" int h2x_softmax_instance_backward_once(h2x_dtype dtype, int num_samples, size_t sample_size, const void* y,
+                                                  const void* dy, void* dx, void* sample_dp, void* workspace,
+                                                  void* state, int max_polls, h2x_stream_t stream)
+{
+    if (!y || !dy || !dx || !sample_dp || !workspace)
+        return num_samples == 0 || sample_size == 0 ? H2X_SUCCESS : H2X_ERR_INVALID_ARGUMENT;
+    const uint32_t polls = max_polls < 0 ? kInstPolls : max_polls;
+    if (!inst_bad(num_samples, sample_size)
+        && (dtype == H2X_F32   ? inst_backward_team<float>(num_samples, sample_size, y, dy, dx, sample_dp, state, polls,
+                                                           as_stream(stream))
+            : dtype == H2X_F64 ? inst_backward_team<double>(num_samples, sample_size, y, dy, dx, sample_dp, state,
+                                                            polls, as_stream(stream))
+                               : false))
+        return launch_status();
+    return h2x_softmax_instance_backward_local(dtype, num_samples, sample_size, y, dy, dx, sample_dp, workspace,
+                                               stream);
 }

@@ -456,6 +456,7 @@ class Softmax:
         self._calls = capi.calls()
         self._ws: Optional[torch.Tensor] = None
         self._scalars: Optional[torch.Tensor] = None
+        self._state: Optional[torch.Tensor] = None
 
     def setup(self, input: Tensor, mode: SoftmaxMode) -> None:
         self.mode = mode
@@ -468,10 +469,17 @@ class Softmax:
         return l
 
     def _workspace(self, n: int) -> torch.Tensor:
-        need = self._lib.h2x_softmax_instance_workspace_bytes(n)
+        need = self._calls.h2x_softmax_instance_workspace_bytes(n)
         if self._ws is None or self._ws.numel() < need:
             self._ws = _buffer_of(self.stream, need, torch.uint8)
         return self._ws
+
+    def _team_state(self, l: Layout) -> Optional[torch.Tensor]:
+        """Where the workgroups that share a sample exchange its partial results; None where no workgroups do."""
+        need = l.instance_state_bytes
+        if need and (self._state is None or self._state.numel() < need):
+            self._state = _buffer_of(self.stream, need, torch.uint8, zero=True)
+        return self._state if need else None
 
     def _sample_scalars(self, t: Tensor, count: int) -> torch.Tensor:
         """`count` scalars of t's type that nobody reads after the call: kept like the workspace."""
@@ -497,9 +505,9 @@ class Softmax:
         if self.allreduce is None:
             # every sample is whole on this rank: the stages need not be separate calls
             scalars = self._sample_scalars(x, 2 * n).data_ptr()
-            status = calls.h2x_softmax_instance_forward_local(
+            status = calls.h2x_softmax_instance_forward_once(
                 dt, n, size, x.get_base_ptr(), y.get_base_ptr(), scalars,
-                scalars + n * self._scalars.element_size(), ws, st)
+                scalars + n * self._scalars.element_size(), ws, self._team_state(l), -1, st)
             if status:
                 capi.check(status, "softmax instance forward")
             return 0
@@ -529,8 +537,9 @@ class Softmax:
         # instance mode: softmax.cu:770-783
         calls, size, ws = self._calls, l.channels * l.spatial, self._workspace(n)
         if self.allreduce is None:
-            status = calls.h2x_softmax_instance_backward_local(
-                dt, n, size, y.get_base_ptr(), dy.get_base_ptr(), dx.get_base_ptr(), self._sample_scalars(y, n), ws, st)
+            status = calls.h2x_softmax_instance_backward_once(
+                dt, n, size, y.get_base_ptr(), dy.get_base_ptr(), dx.get_base_ptr(), self._sample_scalars(y, n), ws,
+                self._team_state(l), -1, st)
             if status:
                 capi.check(status, "softmax instance backward")
             return 0

@@ -196,6 +196,11 @@ class Layout:
         return capi.calls().h2x_bn_ordered_state_needed(self.samples, self.geometry_address)
 
     @_once
+    def instance_state_bytes(self) -> int:
+        """State for instance softmax of tensors like this (0: no workgroups share a sample)."""
+        return capi.calls().h2x_softmax_instance_state_needed(self.dtype, self.samples, self.channels * self.spatial)
+
+    @_once
     def clearing_team_state_bytes(self) -> int:
         """The same for calls that clear their output's halo."""
         return capi.calls().h2x_bn_team_state_needed_clearing(self.dtype, self.haloed_geometry_address)

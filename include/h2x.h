@@ -929,6 +929,27 @@ int h2x_softmax_instance_backward_local(h2x_dtype dtype, int num_samples, size_t
                                         const void* y, const void* dy, void* dx, void* sample_dp,
                                         void* workspace, h2x_stream_t stream);
 
+/**
+ * State (bytes) for h2x_softmax_instance_forward_once and _backward_once on samples like these;
+ * 0: several workgroups never share one.  Zero before its first call; one for calls
+ * that may run at the same time is one too few.
+ */
+size_t h2x_softmax_instance_state_needed(h2x_dtype dtype, int num_samples, size_t sample_size);
+
+/**
+ * h2x_softmax_instance_forward_local and _backward_local, bit for bit, in one launch where the
+ * workgroups of a team hold a sample together and exchange its partial results through
+ * `state` (NULL, or outputs that overlap inputs: by the calls named).  A workgroup that has
+ * looked max_polls times (negative: the library's choice, some 2 ms) for what others have
+ * to store works it out itself.
+ */
+int h2x_softmax_instance_forward_once(h2x_dtype dtype, int num_samples, size_t sample_size,
+                                      const void* x, void* y, void* sample_max, void* sample_exp,
+                                      void* workspace, void* state, int max_polls, h2x_stream_t stream);
+int h2x_softmax_instance_backward_once(h2x_dtype dtype, int num_samples, size_t sample_size,
+                                       const void* y, const void* dy, void* dx, void* sample_dp,
+                                       void* workspace, void* state, int max_polls, h2x_stream_t stream);
+
 /* ------------------------------------------------------------------------ */
 /* Halo pack / unpack                                                        */
 /* ------------------------------------------------------------------------ */

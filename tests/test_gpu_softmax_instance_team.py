@@ -1,0 +1,114 @@
+"""Instance softmax by teams of workgroups: the bits of the staged calls, also of members that work out what they
+miss, call after call on one state, and by the separate launches where a team is not for it."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# samples, elements of a sample: one more than a workgroup holds; whole and single-element vectors; 64 and 65 chunks
+# (members of one and of four), chunks of 4, 8 and 16 vectors a thread at their limits, and beyond (no team)
+CASES = [(1, 32769), (3, 32772), (2, 64 * 4096), (2, 64 * 4096 + 4), (1, 256 * 4096), (1, 256 * 4096 + 4), (2, 256 * 8192 - 4),
+         (2, 256 * 8192 + 8), (3, 256 * 8192), (3, 256 * 16384), (3, 256 * 16384 + 4), (5, 256 * 1024 - 1), (4, 256 * 2048 + 1),
+         (1, 773145), (3, 1048577 * 3), (40, 51 * 4096), (70, 64 * 4096 - 4), (9, 40001)]
+
+
+@pytest.mark.parametrize("polls", [-1, 0])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n,size", CASES)
+def test_teams_equal_the_staged_calls(n, size, dtype, polls):
+    import torch
+    from dihydrogen_amd import capi
+    lib = capi.load()
+    tdt, dt = (torch.float32, capi.F32) if dtype == np.float32 else (torch.float64, capi.F64)
+    g = torch.Generator(device="cuda").manual_seed(size)
+    need = lib.h2x_softmax_instance_state_needed(dt, n, size)
+    assert (need > 0) == (size * np.dtype(dtype).itemsize <= 256 * 16384 * {1: 1, 2: 2}.get(n, 4))
+    state = torch.zeros(max(need, 8), dtype=torch.uint8, device="cuda")
+    ws = torch.empty(lib.h2x_softmax_instance_workspace_bytes(n), dtype=torch.uint8, device="cuda")
+    p = lambda t: t.data_ptr()
+    per_sample = lambda: torch.full((n,), float("nan"), device="cuda", dtype=tdt)
+    for call in range(3):
+        x = torch.randn(n, size, device="cuda", dtype=tdt, generator=g) * 2
+        dy = torch.randn(n, size, device="cuda", dtype=tdt, generator=g)
+        if call == 1:
+            x[0, 5], x[-1, -1] = (float("inf") if n > 1 else 90.0), float("nan")
+        outs = []
+        for team in (True, False):
+            mx, ex, dp = per_sample(), per_sample(), per_sample()
+            y, dx = torch.full_like(x, 7), torch.full_like(x, 7)
+            if team:
+                in_place = call == 2
+                a, d = (x.clone(), dy.clone()) if in_place else (x, dy)
+                y, dx = (a, d) if in_place else (y, dx)
+                capi.check(lib.h2x_softmax_instance_forward_once(dt, n, size, p(a), p(y), p(mx), p(ex), p(ws), p(state), polls, None))
+                capi.check(lib.h2x_softmax_instance_backward_once(dt, n, size, p(y), p(d), p(dx), p(dp), p(ws), p(state), polls,
+                                                                  None))
+            else:
+                capi.check(lib.h2x_softmax_instance_max(dt, n, size, p(x), p(mx), p(ws), None))
+                capi.check(lib.h2x_softmax_instance_exp(dt, n, size, p(x), p(mx), p(y), p(ex), p(ws), None))
+                capi.check(lib.h2x_softmax_instance_normalize(dt, n, size, p(ex), p(y), None))
+                capi.check(lib.h2x_softmax_instance_dot(dt, n, size, p(y), p(dy), p(dp), p(ws), None))
+                capi.check(lib.h2x_softmax_instance_gradient(dt, n, size, p(y), p(dy), p(dp), p(dx), None))
+            torch.cuda.synchronize()
+            outs.append((mx, ex, y, dp, dx))
+        for name, a, b in zip(("max", "sum", "y", "dot", "dx"), *outs):
+            same = (a == b) | (torch.isnan(a) & torch.isnan(b))
+            assert bool(same.all()), (name, call)
+    if need:
+        # one arrival a member and direction: in place there is no team
+        members = state.view(torch.int64)[: need // 8].reshape(n, -1)[:, 0] // 4
+        assert bool((members > 1).all()) and bool((members <= 256).all())
+
+
+def test_layer_calls_on_growing_batches():
+    """One layer, tensors of different batch and sample sizes: against softmax in float64."""
+    import torch
+    from dihydrogen_amd.layers import Softmax, SoftmaxMode
+    from dihydrogen_amd.tensor import Distribution, LocaleVirtual, Tensor
+    sm = Softmax()
+    for n, c, h, w in ((2, 9, 70, 71), (5, 16, 64, 64), (1, 81, 115, 83), (5, 16, 64, 64)):
+        make = lambda: Tensor([w, h, c, n], LocaleVirtual(0, 1), Distribution.make_localized_distribution(4),
+                              torch.float32).allocate()
+        x, y, dy, dx = (make() for _ in range(4))
+        x.real_view().normal_(0, 2), dy.real_view().normal_(0, 1)
+        sm.setup(x, SoftmaxMode.INSTANCE)
+        assert sm.forward(x, y) == 0 and sm.backward(y, dy, dx) == 0
+        torch.cuda.synchronize()
+        flat = lambda t: t.real_view().reshape(n, -1).double()
+        want, got, d = torch.softmax(flat(x), 1), flat(y), flat(dy)
+        eps = torch.finfo(torch.float32).eps
+        assert bool(((got - want).abs() <= 16 * eps * want).all())
+        dot = (got * d).sum(1, keepdim=True)
+        # three roundings and that of the dot product, whose terms are added in float64
+        assert bool(((flat(dx) - got * (d - dot)).abs() <= 4 * eps * got * (d.abs() + dot.abs())).all())
+
+
+@pytest.mark.parametrize("before", [False, True])
+def test_replayed_calls(before):
+    """Calls in a captured graph, the state made before or during the capture, with calls on it in between."""
+    import torch
+    from dihydrogen_amd.layers import Softmax, SoftmaxMode
+    from dihydrogen_amd.tensor import Distribution, LocaleVirtual, Tensor
+    make = lambda: Tensor([64, 64, 30, 2], LocaleVirtual(0, 1), Distribution.make_localized_distribution(4),
+                          torch.float32).allocate()
+    x, y, dy, dx = (make() for _ in range(4))
+    layers = [Softmax() for _ in range(2)]
+    for sm in layers:
+        sm.setup(x, SoftmaxMode.INSTANCE)
+    run = lambda sm: (sm.forward(x, y), sm.backward(y, dy, dx))
+    run(layers[1])
+    if before:
+        run(layers[0])
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run(layers[0])
+    for replay in range(4):
+        x.data.normal_(0, 2), dy.data.normal_(0, 1)
+        run(layers[replay % 2])
+        torch.cuda.synchronize()
+        want = y.data.clone(), dx.data.clone()
+        y.data.fill_(7), dx.data.fill_(7)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y.data, want[0]) and torch.equal(dx.data, want[1])
