@@ -1835,8 +1835,12 @@ struct ReductionPlan
     int groups_max;
 };
 
+// Doubles of a channel that a team holds backward: 64 members of 512 threads with eight vectors.
+constexpr size_t kMostOrdered = 64 * 512 * 8 * 2;
+
 // unroll: vectors of a tile a thread.  Units of doubles are tiles of kUnroll vectors in both directions, which
-// the kernels that read once keep in registers (h2x_bn_ordered.hpp).
+// the kernels that read once keep in registers (h2x_bn_ordered.hpp); not those of channels beyond the largest team,
+// where shorter units fill the chip better (backward, N 8, C 2, 64 x 64 x 32 18.8 and 19.8 us).
 template <typename T>
 int plan_reduction(int num_samples, int num_channels, size_t spatial, std::initializer_list<HostTensor*> ts, int unroll,
                    ReductionPlan* p)
@@ -1856,7 +1860,8 @@ int plan_reduction(int num_samples, int num_channels, size_t spatial, std::initi
     p->spatial = spatial;
     p->groups_max = max_groups_per_channel(num_channels);
     const int budget = reduction_groups_per_channel(num_channels, p->strided);
-    const size_t tile = static_cast<size_t>(kBlockSize) * p->vw * (sizeof(T) == 8 ? kUnroll : unroll);
+    const bool held = sizeof(T) == 8 && num_samples * spatial <= kMostOrdered;
+    const size_t tile = static_cast<size_t>(kBlockSize) * p->vw * (held ? kUnroll : unroll);
     p->ch = make_chunking(spatial, num_samples, budget, tile, tile);
     p->units = static_cast<size_t>(p->ch.chunks_per_seg) * num_samples;
     if (p->units > 0xffffffffull || num_channels > 65535)
@@ -2792,6 +2797,12 @@ constexpr uint32_t kTeamPolls = 2048;
 // workgroups, 18.5 -> 13.3 us; N 10, C 13, 73 x 78, 91 of them, 19.1 -> 13.7; N 1, C 1, 64^3, 32 of them, 17.0 -> 13.2); a
 // handful is left to them.
 constexpr uint32_t kLargeMembers = 384, kMediumMembers = 256, kSmallMembers = 16;
+// Few channels of megabytes, of which a team of the smaller members would be too large: larger ones, so many workgroups
+// and more (forward, backward; N 2, C 4, 96 x 58 x 88 11.1, 18.1 -> 10.1, 13.6 us, in 240 of 64 KB, forward instead of
+// 120 members of 32 KB, backward of two launches; N 20, C 4, 200 x 200 9.6, 16.8 -> 9.1, 12.4; N 3, C 4, 96 x 96 x 90 forward
+// 23.0 -> 19.0 in 304 of 128 KB; but N 3, C 3, 64^3 forward 7.9 in 288 of 32 KB, 8.1 in 144 of 64 KB, and N 2, C 1, 96^3
+// backward 11.6 in two launches, 14.6 in 54 of 128 KB).
+constexpr uint32_t kFewMembers = 96, kFewLargerMembers = 160;
 
 // Members of 16 vectors a thread fit a CU twice (112 registers): a little more than that on every CU would be a second
 // round that is nearly empty, which smaller members fill (forward, N 1, C 72, 64^3, 576 of them, 30.5 us, by 1152 of half the
@@ -2816,7 +2827,11 @@ bool team_variant(const G& g, const OnceForward<T>* a, bool stream, bool forced,
             && team_launch<512, 16>(g, a, stream, forced ? 1 : kLargeMembers, most, polls, team_state, st))
            || team_launch<512, 8>(g, a, stream, forced ? 1 : kMediumMembers, most, polls, team_state, st)
            || team_launch<512, 16>(g, a, stream, kLargeMembers, most, polls, team_state, st)
-           || team_launch<512, 4>(g, a, stream, kSmallMembers, most, polls, team_state, st);
+           || team_launch<512, 4>(g, a, stream, kSmallMembers, most / 2, polls, team_state, st)
+           || team_launch<512, 8>(g, a, stream, kFewLargerMembers, most, polls, team_state, st)
+           || team_launch<512, 4>(g, a, stream, kSmallMembers, most, polls, team_state, st)
+           || team_launch<512, 8>(g, a, stream, kFewMembers, most, polls, team_state, st)
+           || team_launch<512, 16>(g, a, stream, kFewMembers, most, polls, team_state, st);
 }
 
 // Backward 64 KB of each tensor, 128 KB where a team would have more than 64 members
@@ -2831,7 +2846,9 @@ bool team_variant(const G& g, const OnceBackward<T>* a, bool stream, bool forced
     most /= 2;
     return team_launch<512, 8>(g, a, stream, forced ? 1 : kMediumMembers, most, polls, team_state, st)
            || team_launch<1024, 8>(g, a, stream, forced ? 1 : kMediumMembers, most, polls, team_state, st)
-           || team_launch<512, 4>(g, a, stream, kSmallMembers, most, polls, team_state, st);
+           || team_launch<512, 4>(g, a, stream, kSmallMembers, most, polls, team_state, st)
+           || team_launch<512, 8>(g, a, stream, kFewMembers, most, polls, team_state, st)
+           || team_launch<1024, 8>(g, a, stream, kFewMembers, most, polls, team_state, st);
 }
 
 // Channels that one workgroup of 1024 threads would hold, but few: the teams first
@@ -2920,7 +2937,10 @@ bool ordered_geometry(int num_samples, int num_channels, size_t spatial, std::in
     if (plan.vw != full_vec<double>() || (!plan.strided && !output.aligned) || plan.groups > kBlockSize
         || plan.spatial >= (1ull << 31) || plan.units >= (1ull << 31))
         return false;
-    const uint32_t batches = static_cast<uint32_t>(plan.ch.chunk / (kBlockSize * 2 * kOrderedBatch));
+    constexpr size_t kBatch = kBlockSize * 2 * kOrderedBatch; // elements
+    if (plan.ch.chunk % kBatch != 0)
+        return false;
+    const uint32_t batches = static_cast<uint32_t>(plan.ch.chunk / kBatch);
     const uint32_t rounds = static_cast<uint32_t>((plan.units + plan.groups - 1) / plan.groups);
     *rows = plan.strided;
     g->map = t[0].map;
@@ -3002,6 +3022,11 @@ bool ordered_team(OrderedGeometry g, const A* a, bool rows, bool stream, uint32_
     return true;
 }
 
+// Few channels of megabytes, as for floats: forward, backward in us, N 2, C 4, 96 x 58 x 44 11.8, 17.7 -> 10.9, 14.4; N 20,
+// C 4, 140 x 140 10.9, 16.3 -> 9.7, 13.2; but N 2, C 3, 50 x 52 x 55 with a halo backward 13.2 in two launches, 13.6 by 105
+// members; and N 2, C 1, 64^3 forward 6.8 in two launches, 8.5 by 128 members of 32 KB.
+constexpr uint32_t kFewDoubles = 128;
+
 // Which of them, as for floats (once_launch, team_variant).  most_members 0: no teams, where the outputs
 // overlap the inputs or there is no state.  *team: whether it is one.
 template <typename A>
@@ -3018,10 +3043,14 @@ bool ordered_variant(const OrderedGeometry& g, const A* a, bool rows, bool strea
                     && ordered_team<512, 16>(g, a, rows, stream, forced ? 1 : kLargeMembers, most, state, st))
                    || ordered_team<512, 8>(g, a, rows, stream, forced ? 1 : kMediumMembers, most, state, st)
                    || ordered_team<512, 16>(g, a, rows, stream, kLargeMembers, most, state, st)
-                   || ordered_team<512, 4>(g, a, rows, stream, forced ? 1 : kSmallMembers, most, state, st);
+                   || ordered_team<512, 4>(g, a, rows, stream, forced ? 1 : kSmallMembers, most / 2, state, st)
+                   || ordered_team<512, 8>(g, a, rows, stream, kFewLargerMembers, most, state, st)
+                   || ordered_team<512, 4>(g, a, rows, stream, forced ? 1 : kMediumMembers, most, state, st)
+                   || ordered_team<512, 16>(g, a, rows, stream, kFewLargerMembers, most, state, st);
         else
             return ordered_team<512, 8>(g, a, rows, stream, forced ? 1 : kMediumMembers, most / 2, state, st)
-                   || ordered_team<512, 4>(g, a, rows, stream, forced ? 1 : kSmallMembers, most / 2, state, st);
+                   || ordered_team<512, 4>(g, a, rows, stream, forced ? 1 : kSmallMembers, most / 2, state, st)
+                   || ordered_team<512, 8>(g, a, rows, stream, kFewDoubles, most / 2, state, st);
     };
     if ((forced || (few && vectors > 4096)) && by_teams())
         return true;
