@@ -2836,8 +2836,8 @@ bool team_variant(const G& g, const OnceForward<T>* a, bool stream, bool forced,
 
 // Backward 64 KB of each tensor, 128 KB where a team would have more than 64 members
 // (N 8, C 64, 64^3: 355 us, in 128 members 379, in two launches 407), and no more than 64
-// of those (N 16, C 16, 64^3: 251 us, in two launches 195): a larger team waits longer for
-// its last member than it saves.  32 KB where that is not enough workgroups
+// of those: in 128, which would take a state of twice the size, N 16, C 16, 64^3 231 us, in two
+// launches 202, N 16, C 10, 64^3 118 and 131.  32 KB where that is not enough workgroups
 // (N 2, C 32, 28^3 with a halo 8.0 us, in two launches 12.4).
 template <typename G, typename T>
 bool team_variant(const G& g, const OnceBackward<T>* a, bool stream, bool forced, uint32_t most, uint32_t polls,

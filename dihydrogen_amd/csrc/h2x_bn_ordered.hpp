@@ -14,9 +14,9 @@
 //
 // Bound by memory, and by the wait for the last member of a team.  Two launches each way ->
 // this, forward + backward, us going round three sets of tensors:
-//   N 8, C 32, 33^3              97 -> 88       N 4, C 64, 56 x 56            20 -> 14
-//   N 64, C 512, 20 x 20        136 -> 110      N 8, C 100, 64 x 64           39 -> 30
-//   N 16, C 32, 112 x 112        69 -> 55       N 12, C 9, 113 x 123, halo    28 -> 23
+//   N 8, C 32, 33^3              98 -> 87       N 4, C 64, 56 x 56            19 -> 14
+//   N 64, C 512, 20 x 20        137 -> 109      N 8, C 100, 64 x 64           40 -> 29
+//   N 16, C 32, 112 x 112        70 -> 55       N 12, C 9, 113 x 123, halo    27 -> 22
 //   N 4, C 213, 17 x 20 x 23, halo of 1  85 -> 76
 // (33^3 is 18 units a segment, the last of them half empty: 144 groups, 36 members.)
 #pragma once
