@@ -1062,14 +1062,13 @@ def main() -> int:
                 "frac_of_peak": _gbs(nb * sm.elems * 4, med) / HBM_PEAK_GBS,
                 "timing": "events around one eager call after a cache-evicting read"}
         del sm
-        # instance-mode softmax at the same shape, every sample whole on this rank: forward reads x three
-        # times and writes y once (max, sum of exponentials, y from x), backward reads y and dy twice
-        # and writes dx
+        # instance-mode softmax at the same shape, every sample whole on this rank: teams of workgroups read
+        # x, or y and dy, once and write once
         smi = SoftmaxWorkload((16, 21, 256, 256), SEED + 4, instance=True)
         smi.forward(), smi.backward()
         parity["C4_softmax_instance"] = gate_softmax(smi, instance=True)
-        breakdown["C4_softmax_instance_fwd"] = entry(4 * smi.elems * 4, smi.elems, smi.forward)
-        breakdown["C4_softmax_instance_bwd"] = entry(5 * smi.elems * 4, smi.elems, smi.backward)
+        breakdown["C4_softmax_instance_fwd"] = entry(2 * smi.elems * 4, smi.elems, smi.forward)
+        breakdown["C4_softmax_instance_bwd"] = entry(3 * smi.elems * 4, smi.elems, smi.backward)
         del smi
         torch.cuda.empty_cache()
         shf = ShuffleWorkload((128, 128, 64, 32), SEED + 5)
