@@ -1033,6 +1033,29 @@ unsigned int lanes_grid(int n)
     return (static_cast<unsigned int>(n) + samples - 1) / samples;
 }
 
+// Pixels a lane up to 32 channels, of those that alignment and registers allow.  A lane runs a chain of loads,
+// exponentials and stores as long as the channels times its pixels: with fewer than 2^18 pixels one, which
+// leaves more wavefronts, to 2^20 two; two also where tensors are large enough to come from memory.  Forward + backward,
+// us, 4, 2 and 1 a lane, going round three sets of tensors: N 1, C 16, 128 x 128 11.5, 7.9, 6.9; N 2, C 12,
+// 256 x 256 12.9, 10.3, 9.3; N 4, C 16, 256 x 256 21.2, 17.7, 17.7; N 8, C 16, 256 x 256 32.8, 29.7, 33.1; N 16, C 16,
+// 256 x 256 52.8 and 55.0; N 32, C 16, 256 x 256 108 and 104; N 1, C 32, 256 x 256, by 2 and 1, 15.7 and 12.4.
+int pixels_a_lane(int widest, size_t pixels, size_t bytes)
+{
+    constexpr size_t kOnePixel = size_t(1) << 18, kTwoPixels = size_t(1) << 20, kFromMemory = size_t(68) << 20;
+    return pixels < kOnePixel ? 1 : pixels < kTwoPixels || bytes >= kFromMemory ? std::min(widest, 2) : widest;
+}
+
+// Forward, few pixels and 17 channels and more, or 12 of doubles: the waves of a workgroup share the channels of 64
+// pixels (us, a lane with one pixel and so: N 1, C 32, 128 x 128 4.9 and 3.4; N 1, C 21, 128 x 128 4.4 and 3.4, C 16
+// 3.6 and 3.4; N 1, C 32, 256 x 256 5.8 and 6.0; doubles, N 1, C 32, 64 x 64 8.4 and 4.0; N 1, C 25, 256 x 256 10.0 and
+// 7.5; N 1, C 12, 256 x 256 5.4 and 5.8).  Backward a lane adds its products in channel order, up to 32 channels.
+template <typename T>
+bool few_pixels(int c, size_t pixels)
+{
+    constexpr bool kFloat = sizeof(T) == 4;
+    return c <= 32 && c >= (kFloat ? 17 : 12) && pixels <= (kFloat ? 768 : 1024) * size_t(kWaveSize);
+}
+
 template <typename T>
 int forward_impl(int n, int c, size_t s, const void* xv, void* yv, hipStream_t st)
 {
@@ -1050,8 +1073,11 @@ int forward_impl(int n, int c, size_t s, const void* xv, void* yv, hipStream_t s
         launch(softmax_fwd_long_row_kernel<T>, n, kBlockSize, st, x, y, c);
         return launch_status();
     }
-    const int v4 = s < kFlatBelow ? 1 : vector_width<T>(s, 4 / kWords, {xv, yv});
-    const bool stream = streamed<T>(v4, n, c, s);
+    const int widest = s < kFlatBelow ? 1 : vector_width<T>(s, 4 / kWords, {xv, yv});
+    const bool stream = streamed<T>(widest, n, c, s);
+    if (few_pixels<T>(c, n * s))
+        return launch_split_for<T>(1, n, c, s, st, x, y);
+    const int v4 = pixels_a_lane(widest, n * s, n * s * c * sizeof(T));
 #define H2X_FWD(V, CM)                                                                             \
     do                                                                                             \
     {                                                                                              \
@@ -1091,7 +1117,7 @@ int forward_impl(int n, int c, size_t s, const void* xv, void* yv, hipStream_t s
         if (c <= 32) H2X_FWD(1, 32);
     }
 #undef H2X_FWD
-    const int status = launch_split_for<T>(v4, n, c, s, st, x, y);
+    const int status = launch_split_for<T>(widest, n, c, s, st, x, y);
     if (status != kNoSplit)
         return status;
     const int flat = flat_samples(n, s);
@@ -1121,8 +1147,9 @@ int backward_impl(int n, int c, size_t s, const void* yv, const void* dyv, void*
         launch(softmax_bwd_long_row_kernel<T>, n, kBlockSize, st, y, dy, dx, c);
         return launch_status();
     }
-    const int v4 = s < kFlatBelow ? 1 : vector_width<T>(s, 4 / kWords, {yv, dyv, dxv});
-    const bool stream = streamed<T>(v4, n, c, s);
+    const int widest = s < kFlatBelow ? 1 : vector_width<T>(s, 4 / kWords, {yv, dyv, dxv});
+    const bool stream = streamed<T>(widest, n, c, s);
+    const int v4 = pixels_a_lane(widest, n * s, n * s * c * sizeof(T));
 #define H2X_BWD(V, CM)                                                                             \
     do                                                                                             \
     {                                                                                              \
@@ -1158,7 +1185,7 @@ int backward_impl(int n, int c, size_t s, const void* yv, const void* dyv, void*
         if (c <= 32) H2X_BWD(1, 32);
     }
 #undef H2X_BWD
-    const int status = launch_split_for<T>(v4, n, c, s, st, y, dy, dx);
+    const int status = launch_split_for<T>(widest, n, c, s, st, y, dy, dx);
     if (status != kNoSplit)
         return status;
     const int flat = flat_samples(n, s);
