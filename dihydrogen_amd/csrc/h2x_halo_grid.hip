@@ -85,6 +85,8 @@ struct Args
     FastDiv ranks;                 // by num_ranks
     FastDiv lines;                 // by the number of lines
     int32_t line;                  // ranks in a line
+    FastDiv seams;                 // by the number of seams in the dimension of a reverse exchange
+    int32_t seam[kMaxRanks];       // the lower rank of each
     int32_t width[kMaxSpatial];
     uint32_t outer; // channels x samples
 };
@@ -234,20 +236,24 @@ __host__ __device__ __forceinline__ void body(const Args& a, uint32_t block, uin
 // the boundary cells of the ranks they belong to.  A strip spans the real extents
 // of the other dimensions, so along memory it is runs of `width` times the real
 // extents below `dim`, one per index above it.  A thread serves the same vector of
-// the lower and of the upper strip: four loads in flight, and where `dim` is the
-// innermost dimension the ends of neighbouring rows, which share lines, in one
-// wave.  (Phases of different dimensions stay launches of their own: a later one
-// reads halo cells that an earlier one has added to.)
+// both strips of a seam, what each rank gives and takes there: four loads in
+// flight, and what a rank gives lies beside what it takes, in a line of memory that
+// they often share (both strips of a rank and, so, both of a seam, us, N x C x extents on
+// a grid: 13 x 47 x 27 x 42 x 15 on 1 x 2 x 1, periodic, halo of 1 10.9 and 9.3; 2 x 12 x 116 x
+// 316 x 84 on 2 x 4 x 1, periodic 15.0 and 13.8; 4 x 85 x 27 x 38 x 14 on 2 x 2 x 1, halos of 3
+// 12.6 and 11.8; counting ranks without a seam too, whose XCDs then idle, 14.8).  Phases of
+// different dimensions stay launches of their own: a later one reads halo cells that
+// an earlier one has added to.
 template <typename T, typename Op, typename Mem>
 __host__ __device__ __forceinline__ void fold_body(const Args& a, uint32_t block, uint32_t thread, int dim, Op op,
                                                    const Mem& mem)
 {
     constexpr int VEC = 16 / sizeof(T);
     using W = typename Words<T, VEC>::unaligned_t;
-    const uint32_t local_block = fastdiv(block, a.ranks);
-    const int r = static_cast<int>(block - local_block * a.ranks.divisor);
+    const uint32_t local_block = fastdiv(block, a.seams);
+    const int r = a.seam[block - local_block * a.seams.divisor];
     const Rank& me = a.rank[r];
-    const int lo = me.peer[dim][0], hi = me.peer[dim][1];
+    const int hi = me.peer[dim][1];
     // real extents below, along and above the dimension
     int64_t below = 1, above = a.outer;
     for (int d = 0; d < kMaxSpatial; ++d)
@@ -260,17 +266,14 @@ __host__ __device__ __forceinline__ void fold_body(const Args& a, uint32_t block
     const uint32_t run = static_cast<uint32_t>(w * below);
     const uint32_t at = local_block * kBlock + thread;
     const uint32_t row = fastdiv(at, me.units);
-    if (row >= above || (lo < 0 && hi < 0))
+    if (row >= above)
         return;
     auto pitch = [&](int q) { return (a.rank[q].local[dim] + 2 * w) * below; };
-    // the lower boundary cells take the lower neighbour's upper halo, and the other way round
-    T* const to_lo = reinterpret_cast<T*>(me.tensor) + (row * pitch(r) + w * below);
-    T* const to_hi = reinterpret_cast<T*>(me.tensor) + (row * pitch(r) + me.local[dim] * below);
-    const T *from_lo = nullptr, *from_hi = nullptr;
-    if (lo >= 0)
-        from_lo = reinterpret_cast<const T*>(a.rank[lo].tensor) + (row * pitch(lo) + (a.rank[lo].local[dim] + w) * below);
-    if (hi >= 0)
-        from_hi = reinterpret_cast<const T*>(a.rank[hi].tensor) + row * pitch(hi);
+    // this rank's upper boundary cells take the upper neighbour's lower halo, and the other way round
+    T* const mine = reinterpret_cast<T*>(me.tensor) + (row * pitch(r) + me.local[dim] * below);
+    T* const theirs = reinterpret_cast<T*>(a.rank[hi].tensor) + row * pitch(hi);
+    T* const to[2] = {mine, theirs + w * below};
+    const T* const from[2] = {theirs, mine + w * below};
     uint32_t x = at - row * me.units.divisor;
     uint32_t n = 1;
     if (me.vectors)
@@ -280,46 +283,29 @@ __host__ __device__ __forceinline__ void fold_body(const Args& a, uint32_t block
     }
     if (n == VEC)
     {
-        W s0, s1, t0, t1;
-        if (lo >= 0)
+        W s[2], t[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
         {
-            s0 = mem.template load<VEC, false>(from_lo + x);
-            t0 = mem.template load<VEC, false>(to_lo + x);
-        }
-        if (hi >= 0)
-        {
-            s1 = mem.template load<VEC, false>(from_hi + x);
-            t1 = mem.template load<VEC, false>(to_hi + x);
+            s[i] = mem.template load<VEC, false>(from[i] + x);
+            t[i] = mem.template load<VEC, false>(to[i] + x);
         }
 #pragma unroll
-        for (int j = 0; j < VEC; ++j)
+        for (int i = 0; i < 2; ++i)
         {
-            t0[j] = op(t0[j], s0[j]);
-            t1[j] = op(t1[j], s1[j]);
+#pragma unroll
+            for (int j = 0; j < VEC; ++j)
+                t[i][j] = op(t[i][j], s[i][j]);
+            mem.template store<VEC, false>(to[i] + x, t[i]);
         }
-        if (lo >= 0)
-            mem.template store<VEC, false>(to_lo + x, t0);
-        if (hi >= 0)
-            mem.template store<VEC, false>(to_hi + x, t1);
         return;
     }
     for (const uint32_t end = x + n; x < end; ++x)
     {
-        T s0, s1, t0, t1;
-        if (lo >= 0)
-        {
-            s0 = mem.load1(from_lo + x);
-            t0 = mem.load1(to_lo + x);
-        }
-        if (hi >= 0)
-        {
-            s1 = mem.load1(from_hi + x);
-            t1 = mem.load1(to_hi + x);
-        }
-        if (lo >= 0)
-            mem.store1(to_lo + x, op(t0, s0));
-        if (hi >= 0)
-            mem.store1(to_hi + x, op(t1, s1));
+        const T s0 = mem.load1(from[0] + x), t0 = mem.load1(to[0] + x);
+        const T s1 = mem.load1(from[1] + x), t1 = mem.load1(to[1] + x);
+        mem.store1(to[0] + x, op(t0, s0));
+        mem.store1(to[1] + x, op(t1, s1));
     }
 }
 
@@ -728,12 +714,18 @@ int run_fold(h2x_dtype dtype, const h2x_halo_grid* h, int op, h2x_stream_t strea
     {
         if (blocks[dim] == 0)
             continue;
+        uint32_t seams = 0;
         for (int r = 0; r < h->num_ranks; ++r)
         {
             a.rank[r].units = units[dim][r];
             a.rank[r].vectors = vectors[dim][r];
+            if (a.rank[r].peer[dim][1] >= 0)
+                a.seam[seams++] = r;
         }
-        const uint32_t n = static_cast<uint32_t>(blocks[dim]);
+        a.seams = make_fastdiv(seams);
+        uint32_t n = static_cast<uint32_t>(blocks[dim]);
+        if (dim > 0 || !lines)
+            n = n / h->num_ranks * seams;
         const int by = dim > 0 || !lines ? dim : rings ? kRings : kOpenLines;
         err = es == 4 ? issue_fold<float>(op, a, n, by, as_stream(stream))
                       : issue_fold<double>(op, a, n, by, as_stream(stream));
