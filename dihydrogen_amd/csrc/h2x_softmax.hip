@@ -1039,21 +1039,12 @@ unsigned int lanes_grid(int n)
 // us, 4, 2 and 1 a lane, going round three sets of tensors: N 1, C 16, 128 x 128 11.5, 7.9, 6.9; N 2, C 12,
 // 256 x 256 12.9, 10.3, 9.3; N 4, C 16, 256 x 256 21.2, 17.7, 17.7; N 8, C 16, 256 x 256 32.8, 29.7, 33.1; N 16, C 16,
 // 256 x 256 52.8 and 55.0; N 32, C 16, 256 x 256 108 and 104; N 1, C 32, 256 x 256, by 2 and 1, 15.7 and 12.4.
+// (Shared by the waves of a workgroup, as more channels are, C 32 of 128 x 128 pixels take 6.8 us instead of 8.9, but
+// their sums would not be added in channel order.)
 int pixels_a_lane(int widest, size_t pixels, size_t bytes)
 {
     constexpr size_t kOnePixel = size_t(1) << 18, kTwoPixels = size_t(1) << 20, kFromMemory = size_t(68) << 20;
     return pixels < kOnePixel ? 1 : pixels < kTwoPixels || bytes >= kFromMemory ? std::min(widest, 2) : widest;
-}
-
-// Forward, few pixels and 17 channels and more, or 12 of doubles: the waves of a workgroup share the channels of 64
-// pixels (us, a lane with one pixel and so: N 1, C 32, 128 x 128 4.9 and 3.4; N 1, C 21, 128 x 128 4.4 and 3.4, C 16
-// 3.6 and 3.4; N 1, C 32, 256 x 256 5.8 and 6.0; doubles, N 1, C 32, 64 x 64 8.4 and 4.0; N 1, C 25, 256 x 256 10.0 and
-// 7.5; N 1, C 12, 256 x 256 5.4 and 5.8).  Backward a lane adds its products in channel order, up to 32 channels.
-template <typename T>
-bool few_pixels(int c, size_t pixels)
-{
-    constexpr bool kFloat = sizeof(T) == 4;
-    return c <= 32 && c >= (kFloat ? 17 : 12) && pixels <= (kFloat ? 768 : 1024) * size_t(kWaveSize);
 }
 
 template <typename T>
@@ -1075,8 +1066,6 @@ int forward_impl(int n, int c, size_t s, const void* xv, void* yv, hipStream_t s
     }
     const int widest = s < kFlatBelow ? 1 : vector_width<T>(s, 4 / kWords, {xv, yv});
     const bool stream = streamed<T>(widest, n, c, s);
-    if (few_pixels<T>(c, n * s))
-        return launch_split_for<T>(1, n, c, s, st, x, y);
     const int v4 = pixels_a_lane(widest, n * s, n * s * c * sizeof(T));
 #define H2X_FWD(V, CM)                                                                             \
     do                                                                                             \

@@ -1,6 +1,5 @@
-"""Channel softmax up to 32 channels around the numbers of pixels and bytes where the pixels a lane serves change, or
-the waves of a workgroup share the channels: against softmax in float64 (the bounds are those of the streamed
-tensors)."""
+"""Channel softmax up to 32 channels around the numbers of pixels and bytes where the pixels a lane serves change:
+against softmax in float64 (the bounds are those of the streamed tensors)."""
 import pytest
 
 import test_gpu_softmax_streamed as streamed
