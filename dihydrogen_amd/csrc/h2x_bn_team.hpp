@@ -33,7 +33,7 @@
 // other streams fill it; the launch rule keeps a team within half of it.
 #pragma once
 
-constexpr uint32_t kMaxTeamSums = 256; // of a channel: members times sums of a member
+constexpr uint32_t kMaxTeamSums = 512; // of a channel: members times sums of a member
 constexpr uint32_t kMaxMembers = 128;  // a thread looks after one, no team has fewer threads
 
 // State of a channel, zero before its first call: the counter on a line of its own, then
