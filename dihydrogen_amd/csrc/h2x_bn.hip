@@ -2750,6 +2750,29 @@ bool apart(const void* a, const void* b, size_t bytes)
     return x + bytes <= y || y + bytes <= x;
 }
 
+// Whether a backward pass reads dy, for the last time, past the caches, so that x, which the forward pass has left in
+// the memory-side cache, stays there.  In dense tensors of `vectors` of 16 bytes a channel: from 48 MiB.  Smaller ones
+// the cache holds all together.  Backward in us, dy by the caches, past them (going round three sets of tensors): N 4,
+// C 40, 40^3, 41 MB, 26.0, 27.5; N 96, C 60, 38 x 38, 33 MB, 23.6, 27.2; N 134, C 60, 38 x 38, 46 MB, 29.6, 29.7; N 64, C 64,
+// 56 x 56, 51 MB, 34.0, 32.9; N 32, C 256, 56 x 56, 103 MB, 68, 63; doubles, N 4, C 32, 33^3, 37 MB, 28.9, 31.5; N 32, C 64,
+// 56 x 56, 51 MB, 32.8, 31.7; N 8, C 32, 33^3, 74 MB, 58, 53.  Forward + backward N 4, C 64, 64^3 269, 257, with x past
+// the caches too 10 more.  With halos at all sizes: N 4, C 64, 30^3, halo of 1, forward + backward 45, 39.
+constexpr size_t kStreamedGradient = size_t(48) << 20;
+
+bool streams_gradient(size_t vectors, uint32_t num_channels)
+{
+    return vectors * num_channels * 16 >= kStreamedGradient;
+}
+
+template <typename G>
+bool streams_gradient(const G& g)
+{
+    if constexpr (G::kClears)
+        return true;
+    else
+        return !dense_rows(g) || streams_gradient(g.vectors, g.num_channels);
+}
+
 template <typename T, int TEAM, int K, bool STREAM, typename G>
 void issue_team(const TeamGeometry<G>& g, const OnceForward<T>& a, unsigned long long* states, hipStream_t st)
 {
@@ -2759,8 +2782,14 @@ void issue_team(const TeamGeometry<G>& g, const OnceForward<T>& a, unsigned long
 template <typename T, int TEAM, int K, bool STREAM, typename G>
 void issue_team(const TeamGeometry<G>& g, const OnceBackward<T>& a, unsigned long long* states, hipStream_t st)
 {
-    launch(bn_team_backward_kernel<T, TEAM, K, STREAM, G>, g.once.num_channels * g.members.divisor, TEAM, st, g, a,
-           states);
+    const uint32_t blocks = g.once.num_channels * g.members.divisor;
+    if constexpr (K >= 8) // the smallest members are those of small tensors
+        if (streams_gradient(g.once))
+        {
+            launch(bn_team_backward_kernel<T, TEAM, K, STREAM, true, G>, blocks, TEAM, st, g, a, states);
+            return;
+        }
+    launch(bn_team_backward_kernel<T, TEAM, K, STREAM, false, G>, blocks, TEAM, st, g, a, states);
 }
 
 // Members of TEAM threads with K vectors each; false if that is fewer than `least` workgroups,
@@ -2969,7 +2998,13 @@ template <int TEAM, int K, bool TEAMS, bool ROWS, bool STREAM>
 void issue_ordered(const OrderedGeometry& g, const OnceBackward<double>& a, unsigned long long* states, uint32_t blocks,
                    hipStream_t st)
 {
-    launch(bn_ordered_backward_kernel<TEAM, K, TEAMS, ROWS, STREAM>, blocks, TEAM, st, g, a, states);
+    if constexpr (K >= 8)
+        if (g.streams_gradient)
+        {
+            launch(bn_ordered_backward_kernel<TEAM, K, TEAMS, ROWS, STREAM, true>, blocks, TEAM, st, g, a, states);
+            return;
+        }
+    launch(bn_ordered_backward_kernel<TEAM, K, TEAMS, ROWS, STREAM, false>, blocks, TEAM, st, g, a, states);
 }
 
 // Groups that a workgroup of TEAM threads with K vectors each holds.
@@ -3086,6 +3121,7 @@ bool ordered_launch(int n, int c, size_t s, std::initializer_list<const HostTens
         teams = teams && apart(p, out, bytes);
     if (team_polls)
         g.max_polls = *team_polls;
+    g.streams_gradient = output.strided || streams_gradient(n * s / 2, c);
     return ordered_variant(g, &a, rows, !output.strided || bytes > kHaloedNormalStores, teams ? most_members() : 0,
                            team_polls != nullptr, state, st, &team);
 }

@@ -35,6 +35,7 @@ struct OrderedGeometry
     uint32_t num_channels;
     FastDiv members;       // of a team
     uint32_t max_polls;
+    bool streams_gradient; // backward: dy past the caches
 };
 
 constexpr int kOrderedBatch = 4; // vectors a thread: kUnroll of the staged kernels
@@ -335,7 +336,7 @@ __global__ __launch_bounds__(TEAM, TEAMS ? 4 : 1) void bn_ordered_forward_kernel
         }
 }
 
-template <int TEAM, int K, bool TEAMS, bool ROWS, bool STREAM>
+template <int TEAM, int K, bool TEAMS, bool ROWS, bool STREAM, bool GRADIENT>
 __global__ __launch_bounds__(TEAM, TEAMS ? 4 : 1) void bn_ordered_backward_kernel(const OrderedGeometry g,
                                                                    const OnceBackward<double> a,
                                                                    unsigned long long* states)
@@ -367,7 +368,7 @@ __global__ __launch_bounds__(TEAM, TEAMS ? 4 : 1) void bn_ordered_backward_kerne
         if (at[u] != kNowhere)
         {
             load_vec<T, VEC, !ROWS>(a.x + base + (at[u] >> 1), xv[u]);
-            load_vec<T, VEC, !ROWS, kStreamGradient<K>>(a.dy + base + (at[u] >> 1), dv[u]);
+            load_vec<T, VEC, !ROWS, GRADIENT>(a.dy + base + (at[u] >> 1), dv[u]);
         }
     }
     const T m = a.mean[c];

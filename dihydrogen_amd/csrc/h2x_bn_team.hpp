@@ -235,14 +235,8 @@ __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometr
         }
 }
 
-// dy is read for the last time: past the caches where tensors are large, so that x, which the
-// forward pass has left in the memory-side cache, stays there (N 4, C 64, 64^3 forward + backward 288 -> 271 us; with x past
-// the caches too 281; tensors of a few MB, which have the smallest members, are all in the cache: N 8, C 64,
-// 56 x 56 14.1, past the caches 14.6).
-template <int K>
-constexpr bool kStreamGradient = K >= 8;
-
-template <typename T, int TEAM, int K, bool STREAM, typename G>
+// GRADIENT: dy, read for the last time, past the caches (see streams_gradient, where it is launched).
+template <typename T, int TEAM, int K, bool STREAM, bool GRADIENT, typename G>
 __global__ __launch_bounds__(TEAM) void bn_team_backward_kernel(const TeamGeometry<G> g, const OnceBackward<T> a,
                                                                        unsigned long long* states)
 {
@@ -266,7 +260,7 @@ __global__ __launch_bounds__(TEAM) void bn_team_backward_kernel(const TeamGeomet
         {
             at[u] = once_place<VEC>(g.once, first + u * TEAM + threadIdx.x);
             load_vec<T, VEC, false>(a.x + base + G::offset(at[u]), xv[u]);
-            load_vec<T, VEC, false, kStreamGradient<K>>(a.dy + base + G::offset(at[u]), dv[u]);
+            load_vec<T, VEC, false, GRADIENT>(a.dy + base + G::offset(at[u]), dv[u]);
         }
     const T m = a.mean[c];
     const T sc = a.scale[c];
