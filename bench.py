@@ -576,26 +576,26 @@ def cpu_baseline(repeats: int = 5):
 # TCC_EA0_WRREQ_64B), request counts summed over the L2 channels, per dispatch.
 # label -> (bytes read, bytes written) per launch
 PMC_TRAFFIC = {
-    "bn_forward": (270065984, 268831328),
-    "bn_backward": (541605952, 269626432),
+    "bn_forward": (270147456, 268852736),
+    "bn_backward": (541897088, 269621824),
     "bn_sums": (268455424, 131072),
-    "bn_apply": (268466176, 268454656),
-    "bn_backprop1": (536909952, 131104),
-    "bn_backprop2": (536906240, 268435456),
-    "halo_dim0_pack": (147806016, 8652800),    # 4 faces (2 ranks) a launch, four launches a step
-    "halo_dim0_unpack": (9219456, 43264000),
+    "bn_apply": (268466176, 268474496),
+    "bn_backprop1": (536909824, 131072),
+    "bn_backprop2": (536907264, 268435456),
+    "halo_dim0_pack": (147893888, 8652800),    # 4 faces (2 ranks) a launch, four launches a step
+    "halo_dim0_unpack": (9221184, 43264000),
     "halo_dim1_pack": (42624768, 34611200),
-    "halo_dim1_unpack": (34632448, 36217280),
+    "halo_dim1_unpack": (34632448, 36216416),
     "halo_dim2_pack": (34694400, 34611200),
-    "halo_dim2_unpack": (34632448, 34619648),
+    "halo_dim2_unpack": (34632448, 34619392),
 }
 # steps of the timed region whose dominant-kernel launches are bracketed by events: every EVENT_EVERY-th
 EVENT_EVERY = 4
 
 # sha256 (first 16 hex digits) of the kernel sources the table was measured with, see
 # kernel_sources_sha(); with other sources the traffic fields are omitted
-PMC_SOURCES_SHA = "3b6d5a7278fd1c8e"
-PMC_COMMIT = "80a40fd"
+PMC_SOURCES_SHA = "8aead0fd548e93b6"
+PMC_COMMIT = "b6c4b54"
 
 KERNEL_OF = {
     "bn_forward": "bn_team_forward_kernel<float,512,16>",
