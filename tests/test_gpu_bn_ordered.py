@@ -130,3 +130,12 @@ def test_a_state_is_used_where_it_is_needed(case, team):
     p.run("once")
     assert bool(p.state.any()) == team
     assert capi.load().h2x_bn_ordered_state_needed(case[0], ctypes.byref(p.geometry)) == (p.state.numel() if team else 0)
+
+
+# units that do not go evenly into the groups of a channel: one more than there are, one more than twice as many; of two
+# batches; teams, and workgroups that hold a channel; rows
+@pytest.mark.parametrize("shape", [(9, 600, 1, 40, 30, 0), (17, 600, 1, 40, 30, 0), (70, 60, 1, 38, 38, 0), (6, 700, 1, 62, 70, 0),
+                                   (35, 520, 1, 24, 23, 1), (260, 64, 1, 17, 20, 1)])
+def test_units_that_do_not_go_into_the_groups(shape):
+    p = _Problem(*shape)
+    _same(p.run("once"), p.run("local_strided"))

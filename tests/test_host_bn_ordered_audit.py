@@ -76,3 +76,20 @@ def test_state_of_double_tensors(case, needed):
     lib = capi.load()
     got = lib.h2x_bn_ordered_state_needed(n, ctypes.byref(_geometry(shape, strides)))
     assert got == (lib.h2x_bn_team_state_bytes(c) if needed else 0)
+
+
+@pytest.mark.parametrize("backward", [0, 1])
+@pytest.mark.parametrize("n,units", [(9, 1), (8, 1), (17, 1), (5, 3), (12, 2)])
+def test_no_more_groups_than_the_units_of_the_busiest_need(n, units, backward):
+    """A place of a team that a group leaves empty is an idle one: of 600 channels, which are cut into 8 groups at most."""
+    c, h, w = 600, 40, 30 + 52 * (units - 1)
+    status, counted, _, group = _play((w, h, c, n), (1, w, w * h, w * h * c), backward, 1)
+    assert status == 0
+    first = group.reshape(n, c, h * w)[:, 0]                     # of the first channel
+    played = np.zeros(int(first.max()) + 1, np.int64)
+    for sample in first:
+        for u in range(units):
+            played[sample[u * 2048]] += 1
+    assert played.sum() == n * units and played[0] == 0
+    busiest, groups = played.max(), len(played) - 1
+    assert groups <= 8 and groups * busiest - n * units < busiest
