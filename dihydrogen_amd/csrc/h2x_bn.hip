@@ -2843,7 +2843,22 @@ constexpr uint32_t kLargeMembers = 384, kMediumMembers = 256, kSmallMembers = 16
 // 23.0 -> 19.0 in 304 of 128 KB; but N 3, C 3, 64^3 forward 7.9 in 288 of 32 KB, 8.1 in 144 of 64 KB, and N 2, C 1, 96^3
 // backward 11.6 in two launches, 14.6 in 54 of 128 KB).
 constexpr uint32_t kFewMembers = 96, kFewLargerMembers = 160;
-constexpr size_t kHeldTensor = size_t(240) << 20;
+// Backward, teams of 65 to 128 members of 128 KB only in tensors that the memory-side cache nearly holds.  Dense ones below
+// 240 MiB: 7 % less than two launches on average (N 16, C 10, 64^3, 168 MB, 117 us and 131; N 2, C 6, 110 x 120 x 130 55 and
+// 69; N 8, C 13, 73 x 85 x 84, 217 MB, 162 and 170; 17 % more at worst; N 16, C 16, 64^3, 268 MB, 231 and 202).  With a halo below
+// 104 MiB, where x, dy and dx take half of it: 7 % less (N 100, C 8, 200 x 160, 102 MB, 87 and 101), beyond 9 % more (N 158, C
+// 13, 25 x 23 x 21 128 and 112; N 14, C 11, 65 x 66 x 48, halo of 2, 150 and 133); where the halo is cleared never
+// (4 % more; N 50, C 16, 33 x 36 x 45 with a halo of 2 206 and 171).
+constexpr size_t kHeldTensor = size_t(240) << 20, kHeldRows = size_t(104) << 20;
+
+bool for_large_teams(const OnceGeometry& g)
+{
+    return static_cast<size_t>(g.vectors) * g.num_channels * 16 < (dense_rows(g) ? kHeldTensor : kHeldRows);
+}
+bool for_large_teams(const ClearGeometry&)
+{
+    return false;
+}
 
 // Members of 16 vectors a thread fit a CU twice (112 registers): a little more than that on every CU would be a second
 // round that is nearly empty, which smaller members fill (forward, N 1, C 72, 64^3, 576 of them, 30.5 us, by 1152 of half the
@@ -2876,22 +2891,18 @@ bool team_variant(const G& g, const OnceForward<T>* a, bool stream, bool forced,
 }
 
 // Backward 64 KB of each tensor, 128 KB where a team would have more than 64 members
-// (N 8, C 64, 64^3: 355 us, in 128 members 379, in two launches 407), and 128 of those only
-// in tensors that the memory-side cache nearly holds (N 16, C 10, 64^3, 168 MB, 117 us, in two launches 131; N 2, C 6,
-// 110 x 120 x 130 55 and 69; N 100, C 8, 200 x 160 with a halo 87 and 101; N 8, C 13, 73 x 85 x 84, 217 MB, 162 and
-// 170; but N 16, C 16, 64^3, 268 MB, 231 and 202).  32 KB where that is not enough workgroups
+// (N 8, C 64, 64^3: 355 us, in 128 members 379, in two launches 407).  32 KB where that is not enough workgroups
 // (N 2, C 32, 28^3 with a halo 8.0 us, in two launches 12.4).
 template <typename G, typename T>
 bool team_variant(const G& g, const OnceBackward<T>* a, bool stream, bool forced, uint32_t most, uint32_t polls,
                   void* team_state, hipStream_t st)
 {
     most /= 2;
-    const bool held = static_cast<size_t>(g.vectors) * g.num_channels * 16 < kHeldTensor;
     return team_launch<512, 8>(g, a, stream, forced ? 1 : kMediumMembers, most, polls, team_state, st)
            || team_launch<1024, 8>(g, a, stream, forced ? 1 : kMediumMembers, most, polls, team_state, st)
            || team_launch<512, 4>(g, a, stream, kSmallMembers, most, polls, team_state, st)
            || team_launch<512, 8>(g, a, stream, kFewMembers, most, polls, team_state, st)
-           || team_launch<1024, 8>(g, a, stream, kFewMembers, held ? 2 * most : most, polls, team_state, st);
+           || team_launch<1024, 8>(g, a, stream, kFewMembers, for_large_teams(g) ? 2 * most : most, polls, team_state, st);
 }
 
 // Channels that one workgroup of 1024 threads would hold, but few: the teams first
