@@ -43,6 +43,8 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
+#include <limits>
 #include <mutex>
 #include <type_traits>
 
@@ -2803,19 +2805,10 @@ void issue_team(const TeamGeometry<G>& g, const OnceBackward<T>& a, unsigned lon
     launch(bn_team_backward_kernel<T, TEAM, K, STREAM, false, G>, blocks, TEAM, st, g, a, states);
 }
 
-// Members of TEAM threads with K vectors each; false if that is fewer than `least` workgroups,
-// more than `most` members, or more sums than a channel's state has.  Without a: whether.
 template <int TEAM, int K, typename G, template <typename> class A, typename T>
-bool team_launch(const G& once, const A<T>* a, bool stream, uint32_t least, uint32_t most,
-                 uint32_t max_polls, void* team_state, hipStream_t st)
+void team_launch(const G& once, const A<T>& a, bool stream, uint32_t members, uint32_t max_polls, void* team_state,
+                 hipStream_t st)
 {
-    constexpr int kSums = std::is_same<A<T>, OnceForward<T>>::value ? 2 : 4;
-    const uint32_t members = (once.vectors + TEAM * K - 1) / (TEAM * K);
-    const size_t blocks = static_cast<size_t>(members) * once.num_channels;
-    if (members > most || members * kSums > kMaxTeamSums || blocks < least || blocks >= (1u << 30))
-        return false;
-    if (!a)
-        return true;
     TeamGeometry<G> g;
     g.once = once;
     g.members = make_fastdiv(members);
@@ -2823,26 +2816,107 @@ bool team_launch(const G& once, const A<T>* a, bool stream, uint32_t least, uint
     g.max_polls = max_polls;
     unsigned long long* const states = static_cast<unsigned long long*>(team_state);
     if (stream || G::kClears)
-        issue_team<T, TEAM, K, true>(g, *a, states, st);
+        issue_team<T, TEAM, K, true>(g, a, states, st);
     else
-        issue_team<T, TEAM, K, G::kClears>(g, *a, states, st);
-    return true;
+        issue_team<T, TEAM, K, G::kClears>(g, a, states, st);
 }
 
 // Looks of about a microsecond: a team that other streams keep off the chip for longer
 // works its sums out (2 ms against the tens of microseconds of a launch).
 constexpr uint32_t kTeamPolls = 2048;
-// Workgroups from which a size of member is taken: smaller members where larger ones would be
-// fewer.  The smallest ones beat the two launches however few they are (forward + backward, N 2, C 4, 40^3, 64
-// workgroups, 18.5 -> 13.3 us; N 10, C 13, 73 x 78, 91 of them, 19.1 -> 13.7; N 1, C 1, 64^3, 32 of them, 17.0 -> 13.2); a
-// handful is left to them.
-constexpr uint32_t kLargeMembers = 384, kMediumMembers = 256, kSmallMembers = 16;
-// Few channels of megabytes, of which a team of the smaller members would be too large: larger ones, so many workgroups
-// and more (forward, backward; N 2, C 4, 96 x 58 x 88 11.1, 18.1 -> 10.1, 13.6 us, in 240 of 64 KB, forward instead of
-// 120 members of 32 KB, backward of two launches; N 20, C 4, 200 x 200 9.6, 16.8 -> 9.1, 12.4; N 3, C 4, 96 x 96 x 90 forward
-// 23.0 -> 19.0 in 304 of 128 KB; but N 3, C 3, 64^3 forward 7.9 in 288 of 32 KB, 8.1 in 144 of 64 KB, and N 2, C 1, 96^3
-// backward 11.6 in two launches, 14.6 in 54 of 128 KB).
-constexpr uint32_t kFewMembers = 96, kFewLargerMembers = 160;
+// Workgroups from which teams are taken, of the smallest members and of larger ones (forward + backward, N 1, C 1, 64^3, 32
+// workgroups of 32 KB, 17.0 us in two launches, 13.2 by them; backward N 2, C 1, 96^3 11.6 in two launches, 14.6 in 54 of 128 KB;
+// doubles, forward + backward, N 2, C 3, 50 x 52 x 55 with a halo of 1 21.8 in two launches, 24.2 in 108 of 64 KB).
+constexpr uint32_t kFewestMembers = 16, kFewestLarger = 128;
+
+// What a pass takes beyond what all ways to run it share, in us: the bytes it moves, at the rate that members of
+// its size reach, and for every round of workgroups that the chip holds at once what a member needs between its first
+// load and its last store, the longer the larger its team.  Members that are mostly padding cost what full ones do;
+// beyond the first round one that is not full costs half of what it lacks.  In two launches x (backward: x and dy)
+// is read twice.  Fitted to some 12000 calls of 4 to 300 MB a tensor, floats and doubles, each timed in all the ways that hold
+// it, going round three sets of tensors: the way these name takes 0.3 % longer than the fastest one on average, with halos
+// 0.7 (backward) and 1.8 %.  Rules on the number of workgroups alone took 0.6 to 3.5 % longer, and more where the last round
+// is nearly empty or members are mostly padding (forward, N 4, C 16, 96 x 63 x 84, 2000 members of 64 KB, 66 us, as now 53;
+// doubles, forward, backward, N 184, C 91, 23 x 26 with a halo of 1 64, 105 and 57, 85; N 160, C 133, 23 x 19 with a halo of 1 67, 112
+// and 58, 81).  Where two ways are close they may miss: forward, N 32, C 256, 56 x 56, 1792 members of 64 KB 42.0, 1024 of 128 KB 40.4.
+struct PassCost
+{
+    float wait; // of a round, for a team of 64
+    struct
+    {
+        float per_mb, per_round;
+    } members[3]; // of 512 threads with 4 and 8 vectors; then 512 with 16 (forward), 1024 with 8 (backward)
+    float launches, launches_per_mb;
+};
+// dense (or whole) tensors, and rows with a halo between them
+constexpr PassCost kForwardCost[2] = {{2.2f, {{0.31f, 2.5f}, {0.30f, 3.9f}, {0.28f, 6.8f}}, 4.2f, 0.57f},
+                                      {2.0f, {{0.31f, 3.1f}, {0.29f, 4.9f}, {0.30f, 6.8f}}, 5.3f, 0.49f}};
+constexpr PassCost kBackwardCost[2] = {{1.7f, {{0.49f, 2.8f}, {0.38f, 5.4f}, {0.41f, 9.2f}}, 9.3f, 0.78f},
+                                       {1.7f, {{0.47f, 2.9f}, {0.38f, 5.5f}, {0.36f, 10.0f}}, 4.7f, 0.76f}};
+// Workgroups of each size of member that a CU holds (measured: the time of a call steps up where there is one more).
+constexpr uint32_t kForwardOnCu[3] = {3, 3, 2}, kBackwardOnCu[3] = {3, 2, 1}, kBackwardDoublesOnCu[3] = {2, 2, 1};
+
+struct PassShape
+{
+    size_t bytes;        // of a tensor, and of the lines at the ends of haloed rows
+    uint32_t channels;
+    bool rows;           // haloed
+};
+
+// Rows that do not follow one another bring up to a line of what is between them along.
+size_t moved_bytes(size_t rows, size_t width, size_t pitch, size_t item)
+{
+    return rows * item * (width + std::min(pitch - width, size_t(128) / item));
+}
+
+// The cheapest of three sizes of members, teams of members[i] each (0: none), or -1: two launches.
+template <typename T, bool FORWARD>
+int cheapest_pass(const PassShape& p, const uint32_t (&members)[3], bool forced)
+{
+    const PassCost& cost = (FORWARD ? kForwardCost : kBackwardCost)[p.rows];
+    const auto& on_cu = FORWARD ? kForwardOnCu : sizeof(T) == 4 ? kBackwardOnCu : kBackwardDoublesOnCu;
+    const uint32_t cus = compute_units();
+    const float mb = p.bytes * 1e-6f;
+    float least = forced ? std::numeric_limits<float>::max() : cost.launches + cost.launches_per_mb * mb;
+    int best = -1;
+    for (int i = 0; i < 3; ++i)
+    {
+        if (members[i] == 0)
+            continue;
+        const float full = static_cast<float>(static_cast<uint64_t>(members[i]) * p.channels) / ((cus ? cus : 256) * on_cu[i]);
+        const float rounds = full <= 1 ? 1 : (full + std::ceil(full)) / 2;
+        const float us = cost.members[i].per_mb * mb + rounds * (cost.members[i].per_round + cost.wait * members[i] / 64);
+        if (us < least)
+        {
+            least = us;
+            best = i;
+        }
+    }
+    return best;
+}
+
+// `members`, or 0 where they are more than `most`, exchange more sums than a channel's state has, or are fewer than `least`
+// workgroups.
+uint32_t fit_team(size_t members, uint32_t channels, size_t sums, uint32_t most, uint32_t least)
+{
+    const size_t blocks = members * channels;
+    return members > most || sums > kMaxTeamSums || blocks < least || blocks >= (1u << 30)
+               ? 0
+               : static_cast<uint32_t>(members);
+}
+
+PassShape pass_shape(const OnceGeometry& g)
+{
+    const size_t rows = g.vectors / g.spr.divisor;
+    const size_t pitch = g.h.divisor > 1 ? g.sy : g.d.divisor > 1 ? g.sz : g.width;
+    return {moved_bytes(rows * g.num_channels, g.width, std::max<size_t>(pitch, g.width), sizeof(float)), g.num_channels,
+            !dense_rows(g)};
+}
+PassShape pass_shape(const ClearGeometry& g)
+{
+    return {static_cast<size_t>(g.vectors) * g.num_channels * 16, g.num_channels, false};
+}
+
 // Backward, teams of 65 to 128 members of 128 KB only in tensors that the memory-side cache nearly holds.  Dense ones below
 // 240 MiB: 7 % less than two launches on average (N 16, C 10, 64^3, 168 MB, 117 us and 131; N 2, C 6, 110 x 120 x 130 55 and
 // 69; N 8, C 13, 73 x 85 x 84, 217 MB, 162 and 170; 17 % more at worst; N 16, C 16, 64^3, 268 MB, 231 and 202).  With a halo below
@@ -2860,49 +2934,48 @@ bool for_large_teams(const ClearGeometry&)
     return false;
 }
 
-// Members of 16 vectors a thread fit a CU twice (112 registers): a little more than that on every CU would be a second
-// round that is nearly empty, which smaller members fill (forward, N 1, C 72, 64^3, 576 of them, 30.5 us, by 1152 of half the
-// size 27.2; doubles, N 8, C 32, 33^3, 38.9 and 34.2; 448 of them beat 832, see below).
-template <typename G>
-bool fills_rounds(uint32_t vectors, const G& g)
-{
-    constexpr uint32_t kMember = 512 * 16;
-    const size_t blocks = static_cast<size_t>((vectors + kMember - 1) / kMember) * g.num_channels, slots = 2 * compute_units();
-    return blocks <= slots || blocks >= 2 * slots;
-}
-
-// Forward a member holds 128, 64 or 32 KB (N 16, C 64, 112 x 112 in 448 workgroups of 128 KB 20.4 us, in
-// 832 of 64 KB 22.5; N 2, C 32, 48^3 in 448 of 64 KB 12.0, in 224 of 128 KB 13.0; N 2, C 32, 28^3 with a halo
-// in 224 of 32 KB 6.8 us, in two launches 9.8); up to 128 members (N 16, C 16, 64^3 in 128 of them 98 us, in
-// two launches 118).  `forced`: however few workgroups that is.
+// By teams, or false.  Without a: whether.  `forced`: however few workgroups that is, and however long it takes.
 template <typename G, typename T>
 bool team_variant(const G& g, const OnceForward<T>* a, bool stream, bool forced, uint32_t most, uint32_t polls,
                   void* team_state, hipStream_t st)
 {
-    return (fills_rounds(g.vectors, g)
-            && team_launch<512, 16>(g, a, stream, forced ? 1 : kLargeMembers, most, polls, team_state, st))
-           || team_launch<512, 8>(g, a, stream, forced ? 1 : kMediumMembers, most, polls, team_state, st)
-           || team_launch<512, 16>(g, a, stream, kLargeMembers, most, polls, team_state, st)
-           || team_launch<512, 4>(g, a, stream, kSmallMembers, most / 2, polls, team_state, st)
-           || team_launch<512, 8>(g, a, stream, kFewLargerMembers, most, polls, team_state, st)
-           || team_launch<512, 4>(g, a, stream, kSmallMembers, most, polls, team_state, st)
-           || team_launch<512, 8>(g, a, stream, kFewMembers, most, polls, team_state, st)
-           || team_launch<512, 16>(g, a, stream, kFewMembers, most, polls, team_state, st);
+    const auto fit = [&](uint32_t held, uint32_t least) {
+        const size_t m = (g.vectors + held - 1) / held;
+        return fit_team(m, g.num_channels, 2 * m, most, forced ? 1 : least);
+    };
+    const uint32_t members[3] = {fit(512 * 4, kFewestMembers), fit(512 * 8, kFewestLarger), fit(512 * 16, kFewestLarger)};
+    const int best = cheapest_pass<T, true>(pass_shape(g), members, forced);
+    if (best < 0 || !a)
+        return best >= 0;
+    if (best == 0)
+        team_launch<512, 4>(g, *a, stream, members[0], polls, team_state, st);
+    else if (best == 1)
+        team_launch<512, 8>(g, *a, stream, members[1], polls, team_state, st);
+    else
+        team_launch<512, 16>(g, *a, stream, members[2], polls, team_state, st);
+    return true;
 }
 
-// Backward 64 KB of each tensor, 128 KB where a team would have more than 64 members
-// (N 8, C 64, 64^3: 355 us, in 128 members 379, in two launches 407).  32 KB where that is not enough workgroups
-// (N 2, C 32, 28^3 with a halo 8.0 us, in two launches 12.4).
 template <typename G, typename T>
 bool team_variant(const G& g, const OnceBackward<T>* a, bool stream, bool forced, uint32_t most, uint32_t polls,
                   void* team_state, hipStream_t st)
 {
-    most /= 2;
-    return team_launch<512, 8>(g, a, stream, forced ? 1 : kMediumMembers, most, polls, team_state, st)
-           || team_launch<1024, 8>(g, a, stream, forced ? 1 : kMediumMembers, most, polls, team_state, st)
-           || team_launch<512, 4>(g, a, stream, kSmallMembers, most, polls, team_state, st)
-           || team_launch<512, 8>(g, a, stream, kFewMembers, most, polls, team_state, st)
-           || team_launch<1024, 8>(g, a, stream, kFewMembers, for_large_teams(g) ? 2 * most : most, polls, team_state, st);
+    const auto fit = [&](uint32_t held, uint32_t least, uint32_t at_most) {
+        const size_t m = (g.vectors + held - 1) / held;
+        return fit_team(m, g.num_channels, 4 * m, at_most, forced ? 1 : least);
+    };
+    const uint32_t members[3] = {fit(512 * 4, kFewestMembers, most / 2), fit(512 * 8, kFewestLarger, most / 2),
+                                 fit(1024 * 8, kFewestLarger, for_large_teams(g) ? most : most / 2)};
+    const int best = cheapest_pass<T, false>(pass_shape(g), members, forced);
+    if (best < 0 || !a)
+        return best >= 0;
+    if (best == 0)
+        team_launch<512, 4>(g, *a, stream, members[0], polls, team_state, st);
+    else if (best == 1)
+        team_launch<512, 8>(g, *a, stream, members[1], polls, team_state, st);
+    else
+        team_launch<1024, 8>(g, *a, stream, members[2], polls, team_state, st);
+    return true;
 }
 
 // Channels that one workgroup of 1024 threads would hold, but few: the teams first
@@ -3062,55 +3135,61 @@ bool ordered_once(OrderedGeometry g, const A* a, bool rows, bool stream, hipStre
     return true;
 }
 
-// A team a channel, of at least `least` workgroups over all channels.
-template <int TEAM, int K, typename A>
-bool ordered_team(OrderedGeometry g, const A* a, bool rows, bool stream, uint32_t least, uint32_t most, void* state,
-                  hipStream_t st)
+// Members of a team of workgroups of TEAM threads with K vectors each, or 0.
+template <int TEAM, int K, int SUMS>
+uint32_t ordered_members(const OrderedGeometry& g, uint32_t most, uint32_t least)
 {
-    constexpr uint32_t kSums = std::is_same<A, OnceForward<double>>::value ? 2 : 4;
     const uint32_t own = ordered_holds<TEAM, K>(g);
     if (own < 2)
-        return false;
-    const uint32_t width = own % 4 == 0 ? 4 : 2, members = (g.groups + own - 1) / own;
-    const size_t blocks = static_cast<size_t>(members) * g.num_channels;
-    if (members > most || (g.groups + width - 1) / width * kSums > kMaxTeamSums || blocks < least || blocks >= (1u << 30))
-        return false;
+        return 0;
+    const uint32_t width = own % 4 == 0 ? 4 : 2;
+    return fit_team((g.groups + own - 1) / own, g.num_channels, (g.groups + width - 1) / width * SUMS, most, least);
+}
+
+template <int TEAM, int K, typename A>
+void ordered_team(OrderedGeometry g, const A& a, bool rows, bool stream, uint32_t members, void* state, hipStream_t st)
+{
     g.passes = K / kOrderedBatch / g.group_batches.divisor;
     g.members = make_fastdiv(members);
-    if (a)
-        ordered_issue<TEAM, K, true>(g, *a, rows, stream, state, st);
+    ordered_issue<TEAM, K, true>(g, a, rows, stream, state, st);
+}
+
+// By teams, as for floats (team_variant).
+template <typename A>
+bool ordered_by_teams(const OrderedGeometry& g, const A* a, size_t bytes, bool rows, bool stream, uint32_t most, bool forced,
+                      void* state, hipStream_t st)
+{
+    constexpr bool kForward = std::is_same<A, OnceForward<double>>::value;
+    constexpr int kSums = kForward ? 2 : 4;
+    const uint32_t larger = forced ? 1 : kFewestLarger;
+    uint32_t members[3] = {ordered_members<512, 4, kSums>(g, most / 2, forced ? 1 : kFewestMembers),
+                           ordered_members<512, 8, kSums>(g, kForward ? most : most / 2, larger), 0};
+    if constexpr (kForward)
+        members[2] = ordered_members<512, 16, kSums>(g, most, larger);
+    const int best = cheapest_pass<double, kForward>({bytes, g.num_channels, rows}, members, forced);
+    if (best < 0 || !a)
+        return best >= 0;
+    if (best == 0)
+        ordered_team<512, 4>(g, *a, rows, stream, members[0], state, st);
+    else if (best == 1)
+        ordered_team<512, 8>(g, *a, rows, stream, members[1], state, st);
+    else if constexpr (kForward)
+        ordered_team<512, 16>(g, *a, rows, stream, members[2], state, st);
     return true;
 }
 
-// Few channels of megabytes, as for floats: forward, backward in us, N 2, C 4, 96 x 58 x 44 11.8, 17.7 -> 10.9, 14.4; N 20,
-// C 4, 140 x 140 10.9, 16.3 -> 9.7, 13.2; but N 2, C 3, 50 x 52 x 55 with a halo backward 13.2 in two launches, 13.6 by 105
-// members; and N 2, C 1, 64^3 forward 6.8 in two launches, 8.5 by 128 members of 32 KB.
-constexpr uint32_t kFewDoubles = 128;
-
 // Which of them, as for floats (once_launch, team_variant).  most_members 0: no teams, where the outputs
-// overlap the inputs or there is no state.  *team: whether it is one.
+// overlap the inputs or there is no state.  bytes: see PassShape.  *team: whether it is one.
 template <typename A>
-bool ordered_variant(const OrderedGeometry& g, const A* a, bool rows, bool stream, uint32_t most, bool forced, void* state,
-                     hipStream_t st, bool* team)
+bool ordered_variant(const OrderedGeometry& g, const A* a, size_t bytes, bool rows, bool stream, uint32_t most, bool forced,
+                     void* state, hipStream_t st, bool* team)
 {
     constexpr bool kForward = std::is_same<A, OnceForward<double>>::value;
     const size_t vectors = static_cast<size_t>(g.groups) * g.group_batches.divisor * kOrderedBatch * kBlockSize;
     const bool few = g.num_channels <= kOnceManyChannels;
     const auto by_teams = [&] {
         *team = true;
-        if constexpr (kForward)
-            return (fills_rounds(static_cast<uint32_t>(vectors), g)
-                    && ordered_team<512, 16>(g, a, rows, stream, forced ? 1 : kLargeMembers, most, state, st))
-                   || ordered_team<512, 8>(g, a, rows, stream, forced ? 1 : kMediumMembers, most, state, st)
-                   || ordered_team<512, 16>(g, a, rows, stream, kLargeMembers, most, state, st)
-                   || ordered_team<512, 4>(g, a, rows, stream, forced ? 1 : kSmallMembers, most / 2, state, st)
-                   || ordered_team<512, 8>(g, a, rows, stream, kFewLargerMembers, most, state, st)
-                   || ordered_team<512, 4>(g, a, rows, stream, forced ? 1 : kMediumMembers, most, state, st)
-                   || ordered_team<512, 16>(g, a, rows, stream, kFewLargerMembers, most, state, st);
-        else
-            return ordered_team<512, 8>(g, a, rows, stream, forced ? 1 : kMediumMembers, most / 2, state, st)
-                   || ordered_team<512, 4>(g, a, rows, stream, forced ? 1 : kSmallMembers, most / 2, state, st)
-                   || ordered_team<512, 8>(g, a, rows, stream, kFewDoubles, most / 2, state, st);
+        return ordered_by_teams(g, a, bytes, rows, stream, most, forced, state, st);
     };
     if ((forced || (few && vectors > 4096)) && by_teams())
         return true;
@@ -3124,6 +3203,15 @@ bool ordered_variant(const OrderedGeometry& g, const A* a, bool rows, bool strea
         if (!few && ordered_once<1024, 16>(g, a, rows, stream, st))
             return true;
     return by_teams();
+}
+
+size_t moved_bytes(const HostTensor& t, int n, int c, size_t s)
+{
+    const size_t all = static_cast<size_t>(n) * c * s;
+    if (!t.strided)
+        return all * sizeof(double);
+    const size_t w = t.row, h = t.map.h.divisor, pitch = h > 1 ? t.map.sy : s > w * h ? t.map.sz : w;
+    return moved_bytes(all / w, w, std::max(pitch, w), sizeof(double));
 }
 
 // False: the staged kernels, in two launches.
@@ -3144,7 +3232,8 @@ bool ordered_launch(int n, int c, size_t s, std::initializer_list<const HostTens
     if (team_polls)
         g.max_polls = *team_polls;
     g.streams_gradient = output.strided || streams_gradient(n * s / 2, c);
-    return ordered_variant(g, &a, rows, !output.strided || bytes > kHaloedNormalStores, teams ? most_members() : 0,
+    return ordered_variant(g, &a, moved_bytes(output, n, c, s), rows, !output.strided || bytes > kHaloedNormalStores,
+                           teams ? most_members() : 0,
                            team_polls != nullptr, state, st, &team);
 }
 
@@ -3706,13 +3795,14 @@ extern "C" size_t h2x_bn_ordered_state_needed(int num_samples, const h2x_tensor_
     const void* const aligned = reinterpret_cast<const void*>(uintptr_t(256));
     if (num_samples <= 0 || !geometry || strided_tensor<double>(geometry, aligned, num_samples, &t, &c, &s) || c <= 0 || s == 0)
         return 0;
+    const size_t moved = moved_bytes(t, num_samples, c, s);
     const OnceForward<double>* const f = nullptr;
     const OnceBackward<double>* const b = nullptr;
     const uint32_t most = most_members();
     forward = ordered_geometry(num_samples, c, s, {&t}, t, &g, &rows)
-              && ordered_variant(g, f, rows, true, most, false, nullptr, nullptr, &forward) && forward;
+              && ordered_variant(g, f, moved, rows, true, most, false, nullptr, nullptr, &forward) && forward;
     backward = ordered_geometry(num_samples, c, s, {&t, &t}, t, &g, &rows)
-               && ordered_variant(g, b, rows, true, most, false, nullptr, nullptr, &backward) && backward;
+               && ordered_variant(g, b, moved, rows, true, most, false, nullptr, nullptr, &backward) && backward;
     return forward || backward ? h2x_bn_team_state_bytes(c) : 0;
 }
 

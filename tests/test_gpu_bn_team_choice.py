@@ -10,6 +10,20 @@ from dihydrogen_amd import capi
 pytestmark = pytest.mark.gpu
 
 
+def _forward_members(p):
+    """Of a forward pass of the float problem p."""
+    lib, torch, t = capi.load(), p.torch, lambda v: v.data_ptr()
+    gp, at = ctypes.byref(p.geometry), lambda v: v.data_ptr() + p.offset
+    vec = [torch.ones_like(p.scale) for _ in range(4)]
+    y = torch.empty_like(p.x)
+    p.state.zero_()
+    status = lib.h2x_bn_forward_once(capi.F32, p.n, gp, gp, at(p.x), t(p.scale), t(p.bias), p.per, 0.9, 1e-5, *[t(v) for v in vec],
+                                     at(y), t(p.ws), t(p.state), torch.cuda.current_stream().cuda_stream)
+    assert status == 0
+    torch.cuda.synchronize()
+    return int(p.state.view(torch.int64)[0])
+
+
 def _backward_members(p):
     """Of a backward pass of the float problem p."""
     lib, torch, t = capi.load(), p.torch, lambda v: v.data_ptr()
@@ -30,3 +44,11 @@ def _backward_members(p):
                                            ((158, 13, 25, 23, 21, 1), 0), ((14, 11, 65, 66, 48, 2), 0)])
 def test_large_teams_backward(shape, members):
     assert _backward_members(once._Problem(*shape)) == members
+
+
+# 2000 members of 64 KB would be 2.6 rounds of the chip; 64 members a channel are one; a handful is left to two launches; one
+# workgroup holds the last
+@pytest.mark.parametrize("shape,members", [((4, 16, 96, 63, 84, 0), 63), ((4, 64, 64, 64, 64, 0), 32), ((8, 64, 1, 56, 56, 0), 4),
+                                           ((2, 2, 40, 20, 20, 0), 0), ((32, 512, 1, 28, 28, 0), 0)])
+def test_forward(shape, members):
+    assert _forward_members(once._Problem(*shape)) == members

@@ -93,3 +93,11 @@ def test_no_more_groups_than_the_units_of_the_busiest_need(n, units, backward):
     assert played.sum() == n * units and played[0] == 0
     busiest, groups = played.max(), len(played) - 1
     assert groups <= 8 and groups * busiest - n * units < busiest
+
+
+@pytest.mark.parametrize("n,c,h,w,halo", [(160, 133, 23, 19, 1), (184, 91, 23, 26, 1), (231, 51, 48, 12, 1)])
+def test_two_launches_where_members_are_mostly_padding(n, c, h, w, halo):
+    """Units of 2048 elements of which a segment's rows fill a third: teams of them take 1.1 to 1.5 times as long."""
+    lib, pitch = capi.load(), w + 2 * halo
+    plane = pitch * (h + 2 * halo)
+    assert lib.h2x_bn_ordered_state_needed(n, ctypes.byref(_geometry((w, h, c, n), (1, pitch, plane, plane * c)))) == 0
