@@ -2764,12 +2764,14 @@ bool apart(const void* a, const void* b, size_t bytes)
 }
 
 // Whether a backward pass reads dy, for the last time, past the caches, so that x, which the forward pass has left in
-// the memory-side cache, stays there.  In dense tensors of `vectors` of 16 bytes a channel: from 48 MiB.  Smaller ones
-// the cache holds all together.  Backward in us, dy by the caches, past them (going round three sets of tensors): N 4,
+// the memory-side cache, stays there.  In dense tensors, and whole allocations where the halo is cleared, of `vectors` of 16
+// bytes a channel: from 48 MiB.  Smaller ones the cache holds all together.  Backward in us, dy by the caches, past them (going round three sets of tensors): N 4,
 // C 40, 40^3, 41 MB, 26.0, 27.5; N 96, C 60, 38 x 38, 33 MB, 23.6, 27.2; N 134, C 60, 38 x 38, 46 MB, 29.6, 29.7; N 64, C 64,
 // 56 x 56, 51 MB, 34.0, 32.9; N 32, C 256, 56 x 56, 103 MB, 68, 63; doubles, N 4, C 32, 33^3, 37 MB, 28.9, 31.5; N 32, C 64,
 // 56 x 56, 51 MB, 32.8, 31.7; N 8, C 32, 33^3, 74 MB, 58, 53.  Forward + backward N 4, C 64, 64^3 269, 257, with x past
-// the caches too 10 more.  With halos at all sizes: N 4, C 64, 30^3, halo of 1, forward + backward 45, 39.
+// the caches too 10 more.  Cleared: of 28 to 44 MB 4 % more past the caches, of 60 to 95 MB 6 % less (235 calls).  Rows with a
+// halo between them at all sizes: below 28 MB equal, beyond 2 to 8 % less (664 calls; N 4, C 64, 30^3, halo of 1, forward +
+// backward 45, 39).
 constexpr size_t kStreamedGradient = size_t(48) << 20;
 
 bool streams_gradient(size_t vectors, uint32_t num_channels)
@@ -2780,10 +2782,10 @@ bool streams_gradient(size_t vectors, uint32_t num_channels)
 template <typename G>
 bool streams_gradient(const G& g)
 {
-    if constexpr (G::kClears)
-        return true;
-    else
-        return !dense_rows(g) || streams_gradient(g.vectors, g.num_channels);
+    if constexpr (!G::kClears)
+        if (!dense_rows(g))
+            return true;
+    return streams_gradient(g.vectors, g.num_channels);
 }
 
 template <typename T, int TEAM, int K, bool STREAM, typename G>

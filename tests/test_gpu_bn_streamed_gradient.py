@@ -22,3 +22,9 @@ def test_floats(shape):
 def test_doubles(shape):
     p = doubles._Problem(*shape)
     doubles._same(p.run("once"), p.run("local_strided"))
+
+
+# a halo that is cleared: whole allocations of 48 MiB and a little less
+@pytest.mark.parametrize("shape,halo", [((4, 48, 1, 254, 254), 1), ((4, 47, 1, 254, 254), 1)])
+def test_cleared_halo(shape, halo):
+    floats.test_whole_pass_that_clears_the_halo(shape, halo, False)
