@@ -2688,10 +2688,12 @@ void issue_once(const G& g, const OnceForward<float>& a, hipStream_t st)
 template <int TEAM, int K, bool STREAM, typename G>
 void issue_once(const G& g, const OnceBackward<float>& a, hipStream_t st)
 {
-    // 144 of the 160 KB.  With 16 vectors a thread and nine of dy parked there the kernel still spills
-    // 4 registers (5 words of scratch a lane), 16 (9 words) where it clears the halo; against the
-    // two launches it remains the faster one: N 4, C 256, 112 x 112 with a halo, cleared, backward 47.5 ->
-    // 38.7 us, N 2, C 512, 30^3 97 -> 90, N 16, C 1024, 54 x 54 154 -> 142 (going round three sets of tensors).
+    // 144 of the 160 KB.  With 16 vectors a thread and nine of dy parked there the kernel has registers for the rest only if
+    // it works the places of the vectors out again in each step (kept, 16 registers and a 16-byte spill that waits for the first
+    // load: backward, N 40, C 128, 38 x 38 22.3 -> 20.9 us, N 1, C 361, 35 x 46 x 38 69 -> 61, N 2, C 512, 30^3 with a halo 100
+    // -> 90).  Where the halo is cleared a place is long to work out (N 32, C 116, 13 x 9 x 9 25.2 -> 31.6): it is kept, 16 registers are
+    // spilled (9 words of scratch a lane), and the kernel remains faster than two launches: N 4, C 256, 112 x 112 47.5 ->
+    // 38.7, N 2, C 512, 30^3 97 -> 90, N 16, C 1024, 54 x 54 154 -> 142 (going round three sets of tensors).
     constexpr int kInLds = TEAM * K > 8192 ? 9 : 0;
     launch(bn_once_backward_kernel<float, TEAM, K, STREAM, kInLds, G>, once_grid<TEAM>(g), once_block<TEAM>(), st,
            g, a);
