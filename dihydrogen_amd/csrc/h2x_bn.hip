@@ -2904,7 +2904,7 @@ int cheapest_pass(const PassShape& p, const uint32_t (&members)[3], bool forced)
 uint32_t fit_team(size_t members, uint32_t channels, size_t sums, uint32_t most, uint32_t least)
 {
     const size_t blocks = members * channels;
-    return members > most || sums > kMaxTeamSums || blocks < least || blocks >= (1u << 30)
+    return members > most || sums > most_team_sums(channels) || blocks < least || blocks >= (1u << 30)
                ? 0
                : static_cast<uint32_t>(members);
 }
@@ -3009,7 +3009,7 @@ size_t team_state_needed(const G& g)
                         && team_variant(g, forward, true, false, most, 0, nullptr, nullptr))
                        || ((teams_first(g) || !once_holds<OnceBackward<float>>(g))
                            && team_variant(g, backward, true, false, most, 0, nullptr, nullptr));
-    return teams ? g.num_channels * kStateWords * sizeof(unsigned long long) : 0;
+    return teams ? team_state_at(g.num_channels) * sizeof(unsigned long long) : 0;
 }
 
 // Short segments have kernels of their own (N 2048, C 256, 7 x 7: 141 us, by teams 172).
@@ -3771,7 +3771,7 @@ extern "C" int h2x_bn_backward_local_strided(h2x_dtype dtype, int num_samples, s
 
 extern "C" size_t h2x_bn_team_state_bytes(int num_channels)
 {
-    return static_cast<size_t>(std::max(num_channels, 1)) * kStateWords * sizeof(unsigned long long);
+    return team_state_at(std::max(num_channels, 1)) * sizeof(unsigned long long);
 }
 
 extern "C" size_t h2x_bn_team_state_needed(h2x_dtype dtype, int num_samples, const h2x_tensor_geometry* geometry)

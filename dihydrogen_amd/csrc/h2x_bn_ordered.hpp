@@ -270,7 +270,7 @@ __global__ __launch_bounds__(TEAM, TEAMS ? 4 : 1) void bn_ordered_forward_kernel
     const uint32_t c = ordered_channel<TEAMS>(g, &member);
     if (c >= g.num_channels)
         return;
-    unsigned long long* const state = TEAMS ? states + static_cast<size_t>(c) * kStateWords : nullptr;
+    unsigned long long* const state = TEAMS ? states + team_state_at(c) : nullptr;
     const uint32_t tag = TEAMS && threadIdx.x == 0 ? static_cast<uint32_t>(team_load(state)) + 1 : 0;
     const uint32_t quarter = __builtin_amdgcn_readfirstlane(threadIdx.x / kBlockSize), t = threadIdx.x % kBlockSize;
     const T* const x = a.x + c * g.map.stride_c;
@@ -349,7 +349,7 @@ __global__ __launch_bounds__(TEAM, TEAMS ? 4 : 1) void bn_ordered_backward_kerne
     const uint32_t c = ordered_channel<TEAMS>(g, &member);
     if (c >= g.num_channels)
         return;
-    unsigned long long* const state = TEAMS ? states + static_cast<size_t>(c) * kStateWords : nullptr;
+    unsigned long long* const state = TEAMS ? states + team_state_at(c) : nullptr;
     const uint32_t tag = TEAMS && threadIdx.x == 0 ? static_cast<uint32_t>(team_load(state)) + 1 : 0;
     const uint32_t quarter = __builtin_amdgcn_readfirstlane(threadIdx.x / kBlockSize), t = threadIdx.x % kBlockSize;
     const int64_t base = c * g.map.stride_c;

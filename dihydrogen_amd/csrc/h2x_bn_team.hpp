@@ -33,13 +33,23 @@
 // other streams fill it; the launch rule keeps a team within half of it.
 #pragma once
 
-constexpr uint32_t kMaxTeamSums = 512; // of a channel: members times sums of a member
 constexpr uint32_t kMaxMembers = 128;  // a thread looks after one, no team has fewer threads
 
 // State of a channel, zero before its first call: the counter on a line of its own, then
-// two words a sum.
-constexpr uint32_t kCounterWords = 16;
-constexpr uint32_t kStateWords = kCounterWords + 2 * kMaxTeamSums;
+// two words a sum.  A channel has room for 256 sums, members times sums of a member: 128 forward, 64 backward.  Larger teams are
+// for channels of more than 8 MB, of which a tensor has few: the first 32 channels have room for twice that.
+// (Where a channel's state lies is the same for all calls on one state, whatever their sizes.)
+constexpr uint32_t kCounterWords = 16, kTeamSums = 256, kWideChannels = 32;
+
+__host__ __device__ __forceinline__ uint32_t most_team_sums(uint32_t channels)
+{
+    return channels <= kWideChannels ? 2 * kTeamSums : kTeamSums;
+}
+// Words before channel c.
+__host__ __device__ __forceinline__ size_t team_state_at(uint32_t c)
+{
+    return static_cast<size_t>(c) * (kCounterWords + 2 * kTeamSums) + (c < kWideChannels ? c : kWideChannels) * 2 * kTeamSums;
+}
 
 template <typename G>
 struct TeamGeometry
@@ -179,7 +189,7 @@ __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometr
     const uint32_t c = fastdiv(blockIdx.x, g.members);
     const uint32_t member = team_member(blockIdx.x - c * g.members.divisor, g.members.divisor);
     const T* const x = a.x + c * g.once.stride_c;
-    unsigned long long* const state = states + static_cast<size_t>(c) * kStateWords;
+    unsigned long long* const state = states + team_state_at(c);
     const uint32_t tag = threadIdx.x == 0 ? static_cast<uint32_t>(team_load(state)) + 1 : 0;
     const uint32_t first = member * g.span;
     const uint32_t end = first + g.span < g.once.vectors ? first + g.span : g.once.vectors;
@@ -247,7 +257,7 @@ __global__ __launch_bounds__(TEAM) void bn_team_backward_kernel(const TeamGeomet
     const uint32_t c = fastdiv(blockIdx.x, g.members);
     const uint32_t member = team_member(blockIdx.x - c * g.members.divisor, g.members.divisor);
     const int64_t base = c * g.once.stride_c;
-    unsigned long long* const state = states + static_cast<size_t>(c) * kStateWords;
+    unsigned long long* const state = states + team_state_at(c);
     const uint32_t tag = threadIdx.x == 0 ? static_cast<uint32_t>(team_load(state)) + 1 : 0;
     const uint32_t first = member * g.span;
     const uint32_t end = first + g.span < g.once.vectors ? first + g.span : g.once.vectors;

@@ -1662,8 +1662,9 @@ bool inst_team(int n, size_t sample_size, const void* a, const void* b, const vo
         return false;
     const InstChunking ch = inst_plan<T>(n, sample_size, a, b, out, v);
     const int each = static_cast<int>(ch.chunk / kBlockSize / (16 / sizeof(T))); // vectors of 16 bytes
-    const int chunks = ch.groups <= 64 ? 1 : 4;
+    const int chunks = ch.groups <= static_cast<int>(kInstMembers) ? 1 : 4;
     const int members = (ch.groups + chunks - 1) / chunks;
+    static_assert(4 * kInstMembers >= kInstCombine, "members of four hold all chunks");
     if (ch.groups > kInstCombine || each > (chunks == 1 ? 16 : most) || 4 * members > static_cast<int>(compute_units()))
         return false;
     g->members = make_fastdiv(static_cast<uint32_t>(members));

@@ -28,8 +28,9 @@
 
 // State of a sample, zero before its first call: the counter on a line of its own, then two
 // words a member for each of the two exchanges.
-constexpr uint32_t kInstCounterWords = 16;
-constexpr uint32_t kInstStateWords = kInstCounterWords + 2 * 2 * kInstCombine;
+// (256 chunks in members of four, or 64 in members of one.)
+constexpr uint32_t kInstMembers = 64, kInstCounterWords = 16;
+constexpr uint32_t kInstStateWords = kInstCounterWords + 2 * 2 * kInstMembers;
 
 struct InstTeam
 {
@@ -41,7 +42,7 @@ struct InstTeam
 };
 
 // What member m exchanges in thread TEAM / kBlockSize * m, given this member's own in thread 0.
-// recompute(member) is called by the whole workgroup.  shared: kInstCombine + 2 words.
+// recompute(member) is called by the whole workgroup.  shared: kInstMembers + 2 words.
 template <int TEAM, int WHICH, typename F>
 __device__ __forceinline__ double inst_exchange(double part, const InstTeam& g, uint32_t member,
                                                 unsigned long long* state, uint32_t* tag, uint32_t* shared,
@@ -49,18 +50,18 @@ __device__ __forceinline__ double inst_exchange(double part, const InstTeam& g, 
 {
     constexpr uint32_t kChunks = TEAM / kBlockSize;
     const uint32_t members = g.members.divisor, t = threadIdx.x;
-    unsigned long long* const low = state + kInstCounterWords + WHICH * 2 * kInstCombine;
-    unsigned long long* const high = low + kInstCombine;
+    unsigned long long* const low = state + kInstCounterWords + WHICH * 2 * kInstMembers;
+    unsigned long long* const high = low + kInstMembers;
     if (t == 0)
     {
         const unsigned long long bits = __double_as_longlong(part);
         team_store(low + member, *tag, static_cast<uint32_t>(bits));
         team_store(high + member, *tag, static_cast<uint32_t>(bits >> 32));
-        shared[kInstCombine] = 0;
-        shared[kInstCombine + 1] = *tag;
+        shared[kInstMembers] = 0;
+        shared[kInstMembers + 1] = *tag;
     }
     __syncthreads();
-    *tag = shared[kInstCombine + 1];
+    *tag = shared[kInstMembers + 1];
     double s = 0.0;
     const uint32_t mine = t / kChunks;
     if (t % kChunks == 0 && mine < members)
@@ -76,10 +77,10 @@ __device__ __forceinline__ double inst_exchange(double part, const InstTeam& g, 
         }
         shared[mine] = !there;
         if (!there)
-            shared[kInstCombine] = 1; // every writer stores the same
+            shared[kInstMembers] = 1; // every writer stores the same
     }
     __syncthreads();
-    if (shared[kInstCombine])
+    if (shared[kInstMembers])
         for (uint32_t m = 0; m < members; ++m)
             if (shared[m]) // uniform
             {
@@ -211,7 +212,7 @@ __global__ __launch_bounds__(TEAM, TEAM == kBlockSize ? 2 : 4) void softmax_inst
 {
     using P = Pack<T, VEC>;
     __shared__ double lds[TEAM / kWaveSize];
-    __shared__ uint32_t shared[kInstCombine + 2];
+    __shared__ uint32_t shared[kInstMembers + 2];
     const uint32_t n = fastdiv(blockIdx.x, g.members);
     const uint32_t member = blockIdx.x - n * g.members.divisor;
     unsigned long long* const state = g.states + static_cast<size_t>(n) * kInstStateWords;
@@ -269,7 +270,7 @@ __global__ __launch_bounds__(TEAM, TEAM == kBlockSize ? 2 : 4) void softmax_inst
 {
     using P = Pack<T, VEC>;
     __shared__ double lds[TEAM / kWaveSize];
-    __shared__ uint32_t shared[kInstCombine + 2];
+    __shared__ uint32_t shared[kInstMembers + 2];
     const uint32_t n = fastdiv(blockIdx.x, g.members);
     const uint32_t member = blockIdx.x - n * g.members.divisor;
     unsigned long long* const state = g.states + static_cast<size_t>(n) * kInstStateWords;

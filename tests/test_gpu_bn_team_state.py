@@ -22,3 +22,14 @@ def test_a_state_is_used_where_it_is_needed(shape):
     needed = capi.load().h2x_bn_team_state_needed(capi.F32, shape[0], ctypes.byref(p.geometry))
     assert bool(p.state.any()) == (needed > 0)
     assert needed in (0, p.state.numel())
+
+
+def test_one_state_for_the_largest_teams_and_more_channels():
+    """Channels beyond the 32nd have room for half as many sums as those before them; where a channel's lie is one place for
+    all calls."""
+    shapes = [(17, 3, 1, 368, 368), (8, 40, 1, 56, 56), (4, 33, 1, 66, 68), (17, 3, 1, 368, 368), (8, 64, 1, 56, 56)]
+    problems = [once._Problem(*s) for s in shapes]
+    wants = [p.run("local_strided") for p in problems]
+    for k in (0, 1, 2, 3, 4, 0, 4, 1):
+        problems[k].state = problems[4].state
+        once._close(problems[k].run("once"), wants[k])

@@ -112,3 +112,12 @@ def test_replayed_calls(before):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y.data, want[0]) and torch.equal(dx.data, want[1])
+
+
+def test_size_of_the_state():
+    """Two partials of up to 64 members a sample, and a line."""
+    from dihydrogen_amd import capi
+    need = capi.load().h2x_softmax_instance_state_needed
+    for dtype in (capi.F32, capi.F64):
+        for n, size in ((1, 40001), (3, 64 * 4096), (2, 256 * 2048), (40, 51 * 4096)):
+            assert need(dtype, n, size) == n * (128 + 2 * 64 * 2 * 8)

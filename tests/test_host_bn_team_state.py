@@ -61,3 +61,13 @@ def test_layers_make_a_state_where_it_is_used(case, needed, monkeypatch):
         bn.forward(x, *[x.data] * 6, x)
         bn.backward(x, x, *[x.data] * 7, x)
         assert (bn._state is not None) == needed
+
+
+def test_size_of_a_state():
+    """Room for 256 sums a channel, 512 for the first 32: of more channels no call has larger teams."""
+    lib = capi.load()
+    size = lib.h2x_bn_team_state_bytes
+    assert size(2048) <= 2048 * (128 + 256 * 16) + 32 * 256 * 16 + 256
+    assert [size(c + 1) - size(c) for c in (1, 31, 32, 2047)] == [8320, 8320, 4224, 4224]
+    # 71 members of 128 KB a channel backward: such channels are more than 8 MB, and a tensor of them that takes teams has few
+    assert _tensor(17, 27, 1, 368, 368, 0).layout.team_state_bytes == size(27)
