@@ -2759,12 +2759,6 @@ bool once_launch(const OnceGeometry& g, const A& a, int n, hipStream_t st)
 }
 
 // ---- whole channels in several workgroups: which calls, which team ---------------
-bool apart(const void* a, const void* b, size_t bytes)
-{
-    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
-    return x + bytes <= y || y + bytes <= x;
-}
-
 // Whether a backward pass reads dy, for the last time, past the caches, so that x, which the forward pass has left in
 // the memory-side cache, stays there.  In dense tensors, and whole allocations where the halo is cleared, of `vectors` of 16
 // bytes a channel: from 48 MiB.  Smaller ones the cache holds all together.  Backward in us, dy by the caches, past them (going round three sets of tensors): N 4,

@@ -188,44 +188,21 @@ __device__ __forceinline__ void ordered_exchange(double (&v)[N], const OrderedGe
         tag = missing[kMaxMembers + 1];
         if (t < per_member && member * per_member + t < items)
         {
+            double own_items[N];
 #pragma unroll
             for (int k = 0; k < N; ++k)
-            {
-                const unsigned long long bits = __double_as_longlong(item_of(member, t, k));
-                team_store(words + 2 * k * items + member * per_member + t, tag, static_cast<uint32_t>(bits));
-                team_store(words + (2 * k + 1) * items + member * per_member + t, tag, static_cast<uint32_t>(bits >> 32));
-            }
+                own_items[k] = item_of(member, t, k);
+            team_put<N>(words, items, member * per_member + t, tag, own_items);
         }
 #pragma unroll
         for (int k = 0; k < N; ++k)
             v[k] = 0.0;
         const bool reads = t % width == 0 && t < kBlockSize && item < items;
-        if (reads)
-        {
-            const unsigned long long* const mine = words + item;
-            bool there = false;
-            for (uint32_t poll = 0; poll < g.max_polls && !there; ++poll)
-            {
-                if (poll > 0)
-                    __builtin_amdgcn_s_sleep(4);
-                if (team_load(mine + (2 * N - 1) * items) >> 32 != tag) // the word stored last
-                    continue;
-                there = true;
-#pragma unroll
-                for (int k = 0; k < N; ++k)
-                {
-                    const unsigned long long lo = team_load(mine + 2 * k * items),
-                                             hi = team_load(mine + (2 * k + 1) * items);
-                    v[k] = __longlong_as_double(hi << 32 | (lo & 0xffffffffull));
-                    there = there && lo >> 32 == tag && hi >> 32 == tag;
-                }
-            }
-            if (!there) // every writer stores the same
-                missing[item / per_member] = missing[kMaxMembers] = 1;
-        }
+        if (reads && !team_get<N>(words, items, item, tag, g.max_polls, v)) // every writer stores the same
+            missing[item / per_member] = missing[kMaxMembers] = 1;
         __syncthreads();
         if (t == 0)
-            __hip_atomic_fetch_add(state, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            team_leave(state);
         if (missing[kMaxMembers])
             for (uint32_t m = 0; m < g.members.divisor; ++m)
                 if (missing[m]) // uniform
@@ -271,7 +248,7 @@ __global__ __launch_bounds__(TEAM, TEAMS ? 4 : 1) void bn_ordered_forward_kernel
     if (c >= g.num_channels)
         return;
     unsigned long long* const state = TEAMS ? states + team_state_at(c) : nullptr;
-    const uint32_t tag = TEAMS && threadIdx.x == 0 ? static_cast<uint32_t>(team_load(state)) + 1 : 0;
+    const uint32_t tag = TEAMS && threadIdx.x == 0 ? team_tag(state) : 0;
     const uint32_t quarter = __builtin_amdgcn_readfirstlane(threadIdx.x / kBlockSize), t = threadIdx.x % kBlockSize;
     const T* const x = a.x + c * g.map.stride_c;
     const auto place = [&](uint32_t m, int u) {
@@ -350,7 +327,7 @@ __global__ __launch_bounds__(TEAM, TEAMS ? 4 : 1) void bn_ordered_backward_kerne
     if (c >= g.num_channels)
         return;
     unsigned long long* const state = TEAMS ? states + team_state_at(c) : nullptr;
-    const uint32_t tag = TEAMS && threadIdx.x == 0 ? static_cast<uint32_t>(team_load(state)) + 1 : 0;
+    const uint32_t tag = TEAMS && threadIdx.x == 0 ? team_tag(state) : 0;
     const uint32_t quarter = __builtin_amdgcn_readfirstlane(threadIdx.x / kBlockSize), t = threadIdx.x % kBlockSize;
     const int64_t base = c * g.map.stride_c;
     const auto place = [&](uint32_t m, int u) {

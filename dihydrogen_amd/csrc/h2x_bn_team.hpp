@@ -16,19 +16,9 @@
 // Looking at a counter of arrivals instead of the sums themselves was slower the
 // larger the team (64 members, N 4, C 64, 64^3: 119 us against 98): one address.
 //
-// What is exchanged validates itself: half a sum travels with the tag of the call in one
-// 64-bit access of the whole device's scope, so nothing has to be ordered and nothing
-// cleared (a fill launch before the kernel cost 4.7 us behind streaming stores).  The tag is
-// the channel's counter plus one: a member reads the counter before it stores a sum,
-// and adds one to it when it has all sums, so all members of a call find the same
-// value, and no later call of that channel finds it again.  (A member that gave up
-// waiting may add early; who then reads a larger counter is not believed, believes
-// no one, and works all sums out.  The next call's counter is larger still.  Tags come
-// round after 2^32 arrivals; a word would have to lie untouched for just that long.)
-//
-// Nobody waits for ever: after max_polls looks a member works out the sums it misses
-// from memory, with the additions of the member they belong to, and gets the same
-// bits.  That is why outputs may not overlap inputs here.  Members are neighbouring
+// The exchange is that of h2x_device.hpp, with a counter a channel (a fill launch before the kernel instead of
+// tags cost 4.7 us behind streaming stores).  A member works out the sums it misses with the additions of the
+// member they belong to, and gets the same bits.  Members are neighbouring
 // workgroups, and workgroups start in order, so a team is on the chip together unless
 // other streams fill it; the launch rule keeps a team within half of it.
 #pragma once
@@ -39,7 +29,7 @@ constexpr uint32_t kMaxMembers = 128;  // a thread looks after one, no team has 
 // two words a sum.  A channel has room for 256 sums, members times sums of a member: 128 forward, 64 backward.  Larger teams are
 // for channels of more than 8 MB, of which a tensor has few: the first 32 channels have room for twice that.
 // (Where a channel's state lies is the same for all calls on one state, whatever their sizes.)
-constexpr uint32_t kCounterWords = 16, kTeamSums = 256, kWideChannels = 32;
+constexpr uint32_t kTeamSums = 256, kWideChannels = 32;
 
 __host__ __device__ __forceinline__ uint32_t most_team_sums(uint32_t channels)
 {
@@ -84,13 +74,7 @@ __device__ __forceinline__ void team_exchange(double (&v)[N], const TeamGeometry
     unsigned long long* const sums = state + kCounterWords;
     if (t == 0)
     {
-#pragma unroll
-        for (int k = 0; k < N; ++k)
-        {
-            const unsigned long long bits = __double_as_longlong(v[k]);
-            team_store(sums + 2 * k * members + member, tag, static_cast<uint32_t>(bits));
-            team_store(sums + (2 * k + 1) * members + member, tag, static_cast<uint32_t>(bits >> 32));
-        }
+        team_put<N>(sums, members, member, tag, v);
         missing[kMaxMembers] = 0;
         missing[kMaxMembers + 1] = tag;
     }
@@ -102,31 +86,14 @@ __device__ __forceinline__ void team_exchange(double (&v)[N], const TeamGeometry
         s[k] = 0.0;
     if (t < members)
     {
-        const unsigned long long* const mine = sums + t; // the members' words side by side: a look reads few lines
-        bool there = false;
-        for (uint32_t poll = 0; poll < g.max_polls && !there; ++poll)
-        {
-            if (poll > 0)
-                __builtin_amdgcn_s_sleep(4);
-            if (team_load(mine + (2 * N - 1) * members) >> 32 != tag) // the word stored last
-                continue;
-            there = true;
-#pragma unroll
-            for (int k = 0; k < N; ++k)
-            {
-                const unsigned long long lo = team_load(mine + 2 * k * members),
-                                         hi = team_load(mine + (2 * k + 1) * members);
-                s[k] = __longlong_as_double(hi << 32 | (lo & 0xffffffffull));
-                there = there && lo >> 32 == tag && hi >> 32 == tag;
-            }
-        }
+        const bool there = team_get<N>(sums, members, t, tag, g.max_polls, s);
         missing[t] = !there;
         if (!there)
             missing[kMaxMembers] = 1; // every writer stores the same
     }
     __syncthreads();
     if (t == 0)
-        __hip_atomic_fetch_add(state, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        team_leave(state);
     if (missing[kMaxMembers])
         for (uint32_t m = 0; m < members; ++m)
             if (missing[m]) // uniform
@@ -190,7 +157,7 @@ __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometr
     const uint32_t member = team_member(blockIdx.x - c * g.members.divisor, g.members.divisor);
     const T* const x = a.x + c * g.once.stride_c;
     unsigned long long* const state = states + team_state_at(c);
-    const uint32_t tag = threadIdx.x == 0 ? static_cast<uint32_t>(team_load(state)) + 1 : 0;
+    const uint32_t tag = threadIdx.x == 0 ? team_tag(state) : 0;
     const uint32_t first = member * g.span;
     const uint32_t end = first + g.span < g.once.vectors ? first + g.span : g.once.vectors;
     T v[K][VEC];
@@ -258,7 +225,7 @@ __global__ __launch_bounds__(TEAM) void bn_team_backward_kernel(const TeamGeomet
     const uint32_t member = team_member(blockIdx.x - c * g.members.divisor, g.members.divisor);
     const int64_t base = c * g.once.stride_c;
     unsigned long long* const state = states + team_state_at(c);
-    const uint32_t tag = threadIdx.x == 0 ? static_cast<uint32_t>(team_load(state)) + 1 : 0;
+    const uint32_t tag = threadIdx.x == 0 ? team_tag(state) : 0;
     const uint32_t first = member * g.span;
     const uint32_t end = first + g.span < g.once.vectors ? first + g.span : g.once.vectors;
     T xv[K][VEC], dv[K][VEC];

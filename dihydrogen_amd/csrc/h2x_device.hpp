@@ -224,7 +224,18 @@ __device__ __forceinline__ void block_sum(double (&v)[K], double* lds)
 }
 
 // ---- teams of workgroups ---------------------------------------------------------
-// What the workgroups of a team exchange: 32 bits with the tag of their call.
+// How the workgroups of a team exchange doubles through memory.  What is exchanged validates itself: half a double travels with
+// the tag of the call in one 64-bit access of the whole device's scope, so nothing has to be ordered and nothing
+// cleared.  The tag is the team's counter plus one: a member reads the counter before it stores anything, and
+// adds one to it when it has all that it needs, so all members of a call find the same value, and no later call
+// finds it again.  (A member that gave up waiting may add early; who then reads a larger counter is not
+// believed, believes no one, and works all out.  The next call's counter is larger still.  Tags come round after 2^32
+// arrivals; a word would have to lie untouched for just that long.)  Nobody waits for ever: after max_polls looks a
+// member works out what it misses from memory, which is why outputs may not overlap inputs.
+//
+// A team's state: the counter, on a line of its own, then the words, zero before the first call.
+constexpr uint32_t kCounterWords = 16;
+
 __device__ __forceinline__ unsigned long long team_load(const unsigned long long* p)
 {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -232,6 +243,62 @@ __device__ __forceinline__ unsigned long long team_load(const unsigned long long
 __device__ __forceinline__ void team_store(unsigned long long* p, uint32_t tag, uint32_t half)
 {
     __hip_atomic_store(p, static_cast<unsigned long long>(tag) << 32 | half, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The tag of a call.
+__device__ __forceinline__ uint32_t team_tag(const unsigned long long* state)
+{
+    return static_cast<uint32_t>(team_load(state)) + 1;
+}
+// One to the counter, by one thread of a member that has all it needs.
+__device__ __forceinline__ void team_leave(unsigned long long* state)
+{
+    __hip_atomic_fetch_add(state, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Stores v at place `at` of `places`; the same word of all places lies side by side, so that a look reads few lines.
+template <int N>
+__device__ __forceinline__ void team_put(unsigned long long* words, uint32_t places, uint32_t at, uint32_t tag,
+                                         const double (&v)[N])
+{
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+    {
+        const unsigned long long bits = __double_as_longlong(v[k]);
+        team_store(words + 2 * k * places + at, tag, static_cast<uint32_t>(bits));
+        team_store(words + (2 * k + 1) * places + at, tag, static_cast<uint32_t>(bits >> 32));
+    }
+}
+// What place `at` holds, once it holds it; false after max_polls looks.
+template <int N>
+__device__ __forceinline__ bool team_get(const unsigned long long* words, uint32_t places, uint32_t at, uint32_t tag,
+                                         uint32_t max_polls, double (&v)[N])
+{
+    const unsigned long long* const mine = words + at;
+    bool there = false;
+    for (uint32_t poll = 0; poll < max_polls && !there; ++poll)
+    {
+        if (poll > 0)
+            __builtin_amdgcn_s_sleep(4);
+        if constexpr (N > 1)
+            if (team_load(mine + (2 * N - 1) * places) >> 32 != tag) // the word stored last
+                continue;
+        there = true;
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+        {
+            const unsigned long long lo = team_load(mine + 2 * k * places), hi = team_load(mine + (2 * k + 1) * places);
+            v[k] = __longlong_as_double(hi << 32 | (lo & 0xffffffffull));
+            there = there && lo >> 32 == tag && hi >> 32 == tag;
+        }
+    }
+    return there;
+}
+
+// Whether two tensors of so many bytes do not overlap.
+inline bool apart(const void* a, const void* b, size_t bytes)
+{
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x + bytes <= y || y + bytes <= x;
 }
 
 constexpr int kMaxDevices = 64;

@@ -1706,12 +1706,6 @@ void inst_team_variant(const InstTeam& g, int v, const F& f)
         wide(integral_constant<int, 1>());
 }
 
-bool inst_apart(const void* a, const void* b, size_t bytes)
-{
-    const uintptr_t p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
-    return p + bytes <= q || q + bytes <= p;
-}
-
 // Forward pass of samples that are whole on this rank: maximum, sum of the
 // exponentials (y is not written), y from x: 4 tensor passes instead of 5, and three
 // launches instead of five where a sample has few partials (N 1, 158 652 elements 15.1 -> 9.8 us, backward, which saves
@@ -1774,7 +1768,7 @@ bool inst_forward_team(int n, size_t sample_size, const void* x, void* y, void* 
     InstTeam g;
     int v;
     if (!state || !inst_team<T>(n, sample_size, x, nullptr, y, kInstMostForward, &v, &g)
-        || !inst_apart(x, y, n * sample_size * sizeof(T)))
+        || !apart(x, y, n * sample_size * sizeof(T)))
         return false;
     g.max_polls = polls;
     g.states = static_cast<unsigned long long*>(state);
@@ -1794,8 +1788,8 @@ bool inst_backward_team(int n, size_t sample_size, const void* y, const void* dy
     InstTeam g;
     int v;
     const size_t bytes = n * sample_size * sizeof(T);
-    if (!state || !inst_team<T>(n, sample_size, y, dy, nullptr, kInstMostBackward, &v, &g) || !inst_apart(y, dx, bytes)
-        || !inst_apart(dy, dx, bytes) || vector_width<T>(sample_size, v, {dx}) != v) // the outputs take no part in the cut
+    if (!state || !inst_team<T>(n, sample_size, y, dy, nullptr, kInstMostBackward, &v, &g) || !apart(y, dx, bytes)
+        || !apart(dy, dx, bytes) || vector_width<T>(sample_size, v, {dx}) != v) // the outputs take no part in the cut
         return false;
     g.max_polls = polls;
     g.states = static_cast<unsigned long long*>(state);

@@ -19,18 +19,14 @@
 // 1,048,576 elements took 29.6 us, of four 22.6.  Up to 64 chunks more CUs are worth more (16 x 86,016
 // in members of four 17.3, N 1, 158,652 15.3 and 13.8).
 //
-// The exchange is that of the batch-norm teams (h2x_bn_team.hpp): half a partial travels
-// with the tag of the call in one 64-bit access, the tag is the sample's counter plus
-// one, read before a member stores anything, and every member adds one to the counter
-// when it has all partials.  After max_polls looks a member works out what it misses from
-// memory, which is why outputs may not overlap inputs.
+// The exchange is that of h2x_device.hpp, with a counter a sample; the two of a forward pass share a tag.
 #pragma once
 
 // State of a sample, zero before its first call: the counter on a line of its own, then two
 // words a member for each of the two exchanges.
 // (256 chunks in members of four, or 64 in members of one.)
-constexpr uint32_t kInstMembers = 64, kInstCounterWords = 16;
-constexpr uint32_t kInstStateWords = kInstCounterWords + 2 * 2 * kInstMembers;
+constexpr uint32_t kInstMembers = 64;
+constexpr uint32_t kInstStateWords = kCounterWords + 2 * 2 * kInstMembers;
 
 struct InstTeam
 {
@@ -50,13 +46,11 @@ __device__ __forceinline__ double inst_exchange(double part, const InstTeam& g, 
 {
     constexpr uint32_t kChunks = TEAM / kBlockSize;
     const uint32_t members = g.members.divisor, t = threadIdx.x;
-    unsigned long long* const low = state + kInstCounterWords + WHICH * 2 * kInstMembers;
-    unsigned long long* const high = low + kInstMembers;
+    unsigned long long* const words = state + kCounterWords + WHICH * 2 * kInstMembers;
     if (t == 0)
     {
-        const unsigned long long bits = __double_as_longlong(part);
-        team_store(low + member, *tag, static_cast<uint32_t>(bits));
-        team_store(high + member, *tag, static_cast<uint32_t>(bits >> 32));
+        const double own[1] = {part};
+        team_put<1>(words, kInstMembers, member, *tag, own);
         shared[kInstMembers] = 0;
         shared[kInstMembers + 1] = *tag;
     }
@@ -66,15 +60,9 @@ __device__ __forceinline__ double inst_exchange(double part, const InstTeam& g, 
     const uint32_t mine = t / kChunks;
     if (t % kChunks == 0 && mine < members)
     {
-        bool there = false;
-        for (uint32_t poll = 0; poll < g.max_polls && !there; ++poll)
-        {
-            if (poll > 0)
-                __builtin_amdgcn_s_sleep(4);
-            const unsigned long long hi = team_load(high + mine), lo = team_load(low + mine);
-            there = hi >> 32 == *tag && lo >> 32 == *tag;
-            s = __longlong_as_double(hi << 32 | (lo & 0xffffffffull));
-        }
+        double theirs[1] = {0.0};
+        const bool there = team_get<1>(words, kInstMembers, mine, *tag, g.max_polls, theirs);
+        s = theirs[0];
         shared[mine] = !there;
         if (!there)
             shared[kInstMembers] = 1; // every writer stores the same
@@ -89,13 +77,6 @@ __device__ __forceinline__ double inst_exchange(double part, const InstTeam& g, 
                     s = r;
             }
     return s;
-}
-
-// One to the counter, by a member that has all partials.
-__device__ __forceinline__ void inst_leave(unsigned long long* state)
-{
-    if (threadIdx.x == 0)
-        __hip_atomic_fetch_add(state, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // f(k, bytes) for the vectors of a thread in its chunk of a member, in the order of the staged reductions; they
@@ -216,7 +197,7 @@ __global__ __launch_bounds__(TEAM, TEAM == kBlockSize ? 2 : 4) void softmax_inst
     const uint32_t n = fastdiv(blockIdx.x, g.members);
     const uint32_t member = blockIdx.x - n * g.members.divisor;
     unsigned long long* const state = g.states + static_cast<size_t>(n) * kInstStateWords;
-    uint32_t tag = threadIdx.x == 0 ? static_cast<uint32_t>(team_load(state)) + 1 : 0;
+    uint32_t tag = threadIdx.x == 0 ? team_tag(state) : 0;
     const T* const xp = x + static_cast<size_t>(n) * g.sample_size;
     P v[V];
     inst_chunk<T, TEAM, VEC, V>(g, member, [&](int k, uint32_t i) { v[k] = P::load(inst_at<VEC>(xp, k, i)); });
@@ -244,7 +225,8 @@ __global__ __launch_bounds__(TEAM, TEAM == kBlockSize ? 2 : 4) void softmax_inst
         });
         return inst_partial<TEAM>(r, lds);
     });
-    inst_leave(state);
+    if (threadIdx.x == 0)
+        team_leave(state);
     const T sum = static_cast<T>(inst_total<TEAM>(s, lds));
     if (member == 0 && threadIdx.x == 0)
     {
@@ -274,7 +256,7 @@ __global__ __launch_bounds__(TEAM, TEAM == kBlockSize ? 2 : 4) void softmax_inst
     const uint32_t n = fastdiv(blockIdx.x, g.members);
     const uint32_t member = blockIdx.x - n * g.members.divisor;
     unsigned long long* const state = g.states + static_cast<size_t>(n) * kInstStateWords;
-    uint32_t tag = threadIdx.x == 0 ? static_cast<uint32_t>(team_load(state)) + 1 : 0;
+    uint32_t tag = threadIdx.x == 0 ? team_tag(state) : 0;
     const T* const yp = y + static_cast<size_t>(n) * g.sample_size;
     const T* const dp = dy + static_cast<size_t>(n) * g.sample_size;
     P v[V], d[V];
@@ -291,7 +273,8 @@ __global__ __launch_bounds__(TEAM, TEAM == kBlockSize ? 2 : 4) void softmax_inst
         });
         return inst_partial<TEAM>(r, lds);
     });
-    inst_leave(state);
+    if (threadIdx.x == 0)
+        team_leave(state);
     const T dot = static_cast<T>(inst_total<TEAM>(s, lds));
     if (member == 0 && threadIdx.x == 0)
         sample_dp[n] = dot;
