@@ -1564,17 +1564,28 @@ size_t inst_chunk_bytes(int num_samples)
     return size_t(kBlockSize) * 16 * (num_samples <= 1 ? 4 : num_samples == 2 ? 8 : 16);
 }
 
+// Samples that are no whole vectors are cut as those of whole vectors are: with chunks a quarter of that, members of four chunks
+// hold 16 KB, and there are four times as many (forward + backward, by teams, N 23, 142,071 floats 59.7 -> 27.5 us, N 12, 241,997
+// 50.7 -> 26.9; separate launches 37 and 35).  Chunks of more than 32 KB pay there only if members of four fill most of one
+// round of the chip (N 5, 3,054,213 floats, 315 members, 143 us, in chunks of 16 KB, and no teams, 122; N 3, 2,097,657, 129
+// members, 59 and 54; with 144 to 256 members the same either way).
 InstChunking inst_chunking(size_t sample_size, int num_samples, int vec, size_t elem_bytes)
 {
-    const int gmax = inst_groups_per_sample_max(num_samples);
-    const size_t tile = static_cast<size_t>(kBlockSize) * vec * kInstUnroll;
-    size_t chunk = std::max((sample_size + gmax - 1) / gmax, std::min((sample_size + kInstCombine - 1) / kInstCombine,
-                                                                      inst_chunk_bytes(num_samples) / elem_bytes));
-    chunk = (chunk + tile - 1) / tile * tile;
-    InstChunking c;
-    c.chunk = chunk;
-    c.groups = static_cast<int>((sample_size + chunk - 1) / chunk);
-    return c;
+    const size_t gmax = inst_groups_per_sample_max(num_samples);
+    const size_t tile = kBlockSize * (16 / elem_bytes) * kInstUnroll;
+    const auto cut = [&](size_t bytes) {
+        const size_t chunk = std::max((sample_size + gmax - 1) / gmax,
+                                      std::min((sample_size + kInstCombine - 1) / kInstCombine, bytes / elem_bytes));
+        InstChunking c;
+        c.chunk = (chunk + tile - 1) / tile * tile;
+        c.groups = static_cast<int>((sample_size + c.chunk - 1) / c.chunk);
+        return c;
+    };
+    const InstChunking c = cut(inst_chunk_bytes(num_samples));
+    if (vec * elem_bytes == 16 || c.chunk * elem_bytes <= (size_t(32) << 10))
+        return c;
+    const size_t members = static_cast<size_t>((c.groups + 3) / 4) * num_samples;
+    return c.groups <= kInstCombine && members > 140 && members <= 256 ? c : cut(size_t(16) << 10);
 }
 
 // How a reduction over samples is cut.  out: takes part in the choice of the vector width.

@@ -121,3 +121,17 @@ def test_size_of_the_state():
     for dtype in (capi.F32, capi.F64):
         for n, size in ((1, 40001), (3, 64 * 4096), (2, 256 * 2048), (40, 51 * 4096)):
             assert need(dtype, n, size) == n * (128 + 2 * 64 * 2 * 8)
+
+
+# samples of single elements around 64 chunks, and of chunks around 32 KB, whose members are one round of the chip or two
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n,size", [(2, 64 * 4096 - 1), (2, 64 * 4096 + 1), (3, 256 * 8192 - 1), (4, 256 * 8192 + 1)])
+def test_samples_of_single_elements(n, size, dtype):
+    test_teams_equal_the_staged_calls(n, size, dtype, -1)
+
+
+@pytest.mark.parametrize("n,size,team", [(5, 3054213, False), (3, 2097657, False), (3, 3145731, True),
+                                         (5, 1596595, True), (5, 3063970, False), (5, 3063972, True)])
+def test_large_chunks_of_single_elements(n, size, team):
+    from dihydrogen_amd import capi
+    assert (capi.load().h2x_softmax_instance_state_needed(capi.F32, n, size) > 0) == team
