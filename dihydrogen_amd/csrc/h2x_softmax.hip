@@ -1664,11 +1664,36 @@ int inst_map(int n, size_t sample_size, const void* y, const void* dy, const voi
 // Vectors of 16 bytes a thread that members of four chunks hold at most: beyond, 1024 threads lack the registers.
 constexpr int kInstMostForward = 16, kInstMostBackward = 8;
 
+// What a forward pass by members of four chunks takes, and one in separate launches, in us: the bytes, and for every round of the
+// chip, which holds one such member a CU, what it needs for its loads, two exchanges and stores.  Fitted to 1160 calls;
+// members of one chunk, and backward passes, which exchange once, are never slower than separate launches.  Forward,
+// separate launches, by teams: N 6, 2,145,024 floats, 198 members of 256 KB, 40 and 52; N 7, 1,280,796, 280 members of 128 KB,
+// a second round that is nearly empty, 29 and 35; N 4, 3,932,160, 240 members of 256 KB, 58 and 47.
+struct InstForwardCost
+{
+    float team, per_round[3], wait; // per_round: of 64, 128, 256 KB; wait: of a round, for 64 members
+    float launches, launches_per_mb, launches_beyond; // beyond: more a MB from 40 MB
+};
+// whole vectors, single elements
+constexpr InstForwardCost kInstForwardCost[2] = {{5.1f, {4.0f, 8.6f, 13.2f}, 2.1f, 8.9f, 0.56f, 0.24f},
+                                                 {2.0f, {8.6f, 13.6f, 21.0f}, 1.1f, 9.7f, 0.82f, 0.04f}};
+constexpr float kInstTeamPerMb = 0.30f;
+
+bool inst_forward_pays(const InstForwardCost& cost, size_t bytes, size_t members, size_t n, int each)
+{
+    const uint32_t cus = compute_units();
+    const float mb = bytes * 1e-6f, rounds = std::ceil(static_cast<float>(members * n) / (cus ? cus : 256));
+    const float round = cost.per_round[each <= 4 ? 0 : each <= 8 ? 1 : 2] + cost.wait * members / 64;
+    return cost.team + kInstTeamPerMb * mb + rounds * round
+           < cost.launches + cost.launches_per_mb * mb + cost.launches_beyond * std::max(mb - 40, 0.0f);
+}
+
 // A team for samples cut as the staged sums are, or false: of up to 64 members of one chunk, or of four (see
 // h2x_softmax_team.hpp).  Members fit a CU once at least, so a team is within a quarter of the chip.
-template <typename T>
-bool inst_team(int n, size_t sample_size, const void* a, const void* b, const void* out, int most, int* v, InstTeam* g)
+template <typename T, bool FORWARD>
+bool inst_team(int n, size_t sample_size, const void* a, const void* b, const void* out, int* v, InstTeam* g)
 {
+    constexpr int most = FORWARD ? kInstMostForward : kInstMostBackward;
     if (sample_size <= kInstSmallSample<T> || n <= 0)
         return false;
     const InstChunking ch = inst_plan<T>(n, sample_size, a, b, out, v);
@@ -1677,6 +1702,9 @@ bool inst_team(int n, size_t sample_size, const void* a, const void* b, const vo
     const int members = (ch.groups + chunks - 1) / chunks;
     static_assert(4 * kInstMembers >= kInstCombine, "members of four hold all chunks");
     if (ch.groups > kInstCombine || each > (chunks == 1 ? 16 : most) || 4 * members > static_cast<int>(compute_units()))
+        return false;
+    if (FORWARD && chunks == 4
+        && !inst_forward_pays(kInstForwardCost[*v != 16 / sizeof(T)], n * sample_size * sizeof(T), members, n, each))
         return false;
     g->members = make_fastdiv(static_cast<uint32_t>(members));
     g->chunks = static_cast<uint32_t>(chunks);
@@ -1778,7 +1806,7 @@ bool inst_forward_team(int n, size_t sample_size, const void* x, void* y, void* 
 {
     InstTeam g;
     int v;
-    if (!state || !inst_team<T>(n, sample_size, x, nullptr, y, kInstMostForward, &v, &g)
+    if (!state || !inst_team<T, true>(n, sample_size, x, nullptr, y, &v, &g)
         || !apart(x, y, n * sample_size * sizeof(T)))
         return false;
     g.max_polls = polls;
@@ -1799,7 +1827,7 @@ bool inst_backward_team(int n, size_t sample_size, const void* y, const void* dy
     InstTeam g;
     int v;
     const size_t bytes = n * sample_size * sizeof(T);
-    if (!state || !inst_team<T>(n, sample_size, y, dy, nullptr, kInstMostBackward, &v, &g) || !apart(y, dx, bytes)
+    if (!state || !inst_team<T, false>(n, sample_size, y, dy, nullptr, &v, &g) || !apart(y, dx, bytes)
         || !apart(dy, dx, bytes) || vector_width<T>(sample_size, v, {dx}) != v) // the outputs take no part in the cut
         return false;
     g.max_polls = polls;
@@ -1983,7 +2011,8 @@ extern "C" size_t h2x_softmax_instance_state_needed(h2x_dtype dtype, int num_sam
     const auto team = [&](auto zero) {
         InstTeam g;
         int v;
-        return inst_team<decltype(zero)>(num_samples, sample_size, nullptr, nullptr, nullptr, kInstMostForward, &v, &g);
+        return inst_team<decltype(zero), true>(num_samples, sample_size, nullptr, nullptr, nullptr, &v, &g)
+               || inst_team<decltype(zero), false>(num_samples, sample_size, nullptr, nullptr, nullptr, &v, &g);
     };
     return (dtype == H2X_F32 ? team(0.0f) : team(0.0)) ? num_samples * kInstStateWords * sizeof(unsigned long long) : 0;
 }

@@ -131,7 +131,23 @@ def test_samples_of_single_elements(n, size, dtype):
 
 
 @pytest.mark.parametrize("n,size,team", [(5, 3054213, False), (3, 2097657, False), (3, 3145731, True),
-                                         (5, 1596595, True), (5, 3063970, False), (5, 3063972, True)])
+                                         (5, 1596595, True), (5, 3063970, False), (4, 3932156, True)])
 def test_large_chunks_of_single_elements(n, size, team):
     from dihydrogen_amd import capi
     assert (capi.load().h2x_softmax_instance_state_needed(capi.F32, n, size) > 0) == team
+
+
+# members of 256 KB on three quarters of the chip, of 128 KB on a little more than all of it; members of 256 KB on 240 CUs
+@pytest.mark.parametrize("n,size,team", [(6, 2145024, False), (7, 1280796, False), (4, 3932160, True), (256, 40001, True)])
+def test_forward_by_teams_where_it_pays(n, size, team):
+    """A member counts its arrival in the state of its sample."""
+    import torch
+    from dihydrogen_amd import capi
+    lib, p = capi.load(), lambda t: t.data_ptr()
+    x = torch.randn(n, size, device="cuda")
+    y, mx, ex = torch.empty_like(x), torch.empty(n, device="cuda"), torch.empty(n, device="cuda")
+    ws = torch.empty(lib.h2x_softmax_instance_workspace_bytes(n), dtype=torch.uint8, device="cuda")
+    state = torch.zeros(lib.h2x_softmax_instance_state_needed(capi.F32, n, size) + 8, dtype=torch.uint8, device="cuda")
+    capi.check(lib.h2x_softmax_instance_forward_once(capi.F32, n, size, p(x), p(y), p(mx), p(ex), p(ws), p(state), -1, None))
+    torch.cuda.synchronize()
+    assert bool(state.any()) == team
