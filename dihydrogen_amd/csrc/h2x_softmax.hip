@@ -559,7 +559,14 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
     using P = Pack<T, VEC>;
     __shared__ T lds[WAVES][kWaveSize * VEC];
     const int lane = threadIdx.x % kWaveSize;
-    const int g = wave_index();
+    // Of more than 256 channels in floats the index stays a lane's own: as a scalar, the addresses
+    // and the tests of all those channels are scalars too, more than there are (16 waves with 24
+    // channels each spill 31 of them into vector registers, with 48 153; up to 256 channels a wave
+    // of 16 spills two).  us, scalar and so: N 4, C 428, 20 x 26 12.4 -> 8.0, N 2, C 494, 34 x 19
+    // 13.3 -> 8.6, N 8, C 395, 46 x 46 31.5 -> 25.2; 245 drawn sizes 0.94 of the time, the worst
+    // 1.08.  Doubles fill the vector registers first (1.01 to 1.06 of the scalar's time), and the
+    // forward pass, of half the addresses, is faster with the scalar.
+    const int g = sizeof(T) == 4 && WAVES * CPW > 256 ? static_cast<int>(threadIdx.x / kWaveSize) : wave_index();
     size_t base;
     const bool active = tile_pixels<VEC>(tiles, num_channels, spatial, flat_samples, &base);
     const T* yp = y + base;
