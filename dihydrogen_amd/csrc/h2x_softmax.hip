@@ -167,6 +167,12 @@ __device__ __forceinline__ bool tile_pixels(const WideTiles& t, int num_channels
 // 256 x 256, 20 MB, 20.8 and 21.3, N 2, C 16, 384 x 384, 19 MB, 24.1 and 26.8.  Rows that are no whole
 // vectors share their lines with the tile next door and are not streamed (N 30, C 179, 43 x 43, 40 MB,
 // 49.3 and 52.2; N 16, C 21, 255 x 257 78.5 both ways).  With y past the caches too the first takes 76.9.
+// That is the call alone.  Between neighbours that write x, make dy of y and read dx (one set of tensors,
+// elementwise kernels, all five launches, normally -> streamed): N 16, C 21, 256 x 256 188.8 -> 167.7, N 8, C 32 134.4 ->
+// 126.2, N 16, C 500, 48 x 48 164.2 -> 156.8, N 6, C 19 63.7 and 63.9, N 4, C 100, 128 x 128 57.5 -> 57.0, but N 2,
+// C 64, 32 MB, 67.8 -> 69.1.  The kernel behind it reads a streamed dx from memory: backward + consumer of 64 MB
+// 49.3 -> 53.4, of 28 MB 24.0 -> 27.0; y and what else is live stay cached instead and give back as much or
+// more.  Called over and over on one set of 63 MB, with nothing in between, 48.7 -> 55.7.
 constexpr size_t kStreamBytes = size_t(24) << 20;
 
 template <typename T>
