@@ -62,7 +62,7 @@ def test_what_runs_in_two_launches(shape, strides):
     for backward in (0, 1):
         b = (ctypes.c_ubyte * 16)()
         status = capi.load().h2x_bn_audit_ordered(shape[-1], ctypes.byref(_geometry(shape, strides)), backward, 1, b, b, b, 16)
-        assert status in (-1, -2)
+        assert status == -2  # unsupported: played into 16 bytes, what is supported gives -1
 
 
 @pytest.mark.parametrize("case,needed", [((8, 32, 33, 33, 33), True), ((8, 64, 1, 56, 56), True), ((1, 200, 1, 40, 40), False),
