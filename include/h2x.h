@@ -424,11 +424,13 @@ int h2x_bn_backward_local_strided(h2x_dtype dtype,
  * The same again for tensors that lie alike, reading every element once where
  * a channel is held in registers between the sums and the output: by one workgroup
  * (up to about 80000 floats a channel forward and 65000 backward) or by a team of
- * workgroups (larger channels, or few, up to about 4 million floats forward and 2
- * million backward, outputs that do not overlap inputs); otherwise what
+ * workgroups (larger channels, or few, up to about 4 million floats, backward beyond 2
+ * million only in tensors below 240 MiB, with a halo 104 MiB; outputs that do not overlap
+ * inputs), where an estimate of the time says so; otherwise what
  * h2x_bn_forward_local_strided and h2x_bn_backward_local_strided do.  The terms of
  * the sums are the same and are added in fp64: of floats in another order, of doubles in
- * the same one (channels of up to half a million doubles, segments beyond 256 elements).
+ * the same one (channels of up to 2 million doubles forward and half a million backward,
+ * segments beyond 256 elements).
  *
  * team_state: h2x_bn_team_state_bytes() of the number of channels, or more, zeroed
  * once before the first call and then left to these calls, one after another, in any
