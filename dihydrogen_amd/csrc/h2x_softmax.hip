@@ -159,8 +159,9 @@ __device__ __forceinline__ bool tile_pixels(const WideTiles& t, int num_channels
 }
 
 // Cache policy.  The backward pass reads the y that the forward pass has written; x and dy are read
-// and dx is written once.  Tensors of which a call's set does not fit the 256 MB memory-side cache
-// are streamed (STREAM): x and dy are loaded and dx is stored past the caches, y alone stays.
+// and dx is written once.  Tensors of 24 MiB and more are streamed (STREAM): x and dy are loaded and dx is stored past
+// the caches, y alone stays.  (x, y, dy and dx of such a layer, 96 MiB, fit the 256 MB memory-side cache by themselves; with
+// those of its neighbours, or of two more layers like it, they do not, and that is what was measured.)
 // Forward + backward, us going round three sets of tensors, before -> streamed: N 16, C 21, 256 x 256, 88 MB,
 // 74.6 -> 69.8; N 8, C 32, 256 x 256, 67 MB, 60.3 -> 53.5; N 16, C 500, 48 x 48, 74 MB, 90.5 -> 82.5; N 6, C 19,
 // 256 x 256, 30 MB, 29.8 -> 28.2; N 4, C 100, 128 x 128, 26 MB, 27.3 -> 25.6; below, the caches hold what is read: N 4, C 19,
