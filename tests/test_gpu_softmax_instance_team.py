@@ -151,3 +151,41 @@ def test_forward_by_teams_where_it_pays(n, size, team):
     capi.check(lib.h2x_softmax_instance_forward_once(capi.F32, n, size, p(x), p(y), p(mx), p(ex), p(ws), p(state), -1, None))
     torch.cuda.synchronize()
     assert bool(state.any()) == team
+
+
+# members of one chunk and of four, whose vectors are whole or single elements by the alignment of what takes part in the cut
+@pytest.mark.parametrize("team", [True, False])
+@pytest.mark.parametrize("skewed", ["x", "y", "dy", "dx"])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n,size", [(3, 32772), (2, 64 * 4096), (2, 64 * 4096 + 4), (3, 256 * 4096)])  # within a backward team
+def test_one_tensor_off_alignment(n, size, dtype, skewed, team):
+    """The staged calls' bits, by teams and by the separate launches.  dx takes no part in the cut: beside aligned y and dy
+    no team serves it."""
+    import torch
+    from dihydrogen_amd import capi
+    lib, p = capi.load(), lambda t: t.data_ptr()
+    tdt, dt = (torch.float32, capi.F32) if dtype == np.float32 else (torch.float64, capi.F64)
+    room = {name: torch.full((n * size + 2,), 7.0, device="cuda", dtype=tdt) for name in ("x", "y", "dy", "dx", "ys", "dxs")}
+    t = {name: r[int(name.rstrip("s") == skewed):][:n * size].view(n, size) for name, r in room.items()}
+    t["x"].normal_(0, 2), t["dy"].normal_(0, 1)
+    ws = torch.empty(lib.h2x_softmax_instance_workspace_bytes(n), dtype=torch.uint8, device="cuda")
+    state = torch.zeros(lib.h2x_softmax_instance_state_needed(dt, n, 40001), dtype=torch.uint8, device="cuda")
+    mx, ex, dp, mxs, exs, dps = (torch.empty(n, device="cuda", dtype=tdt) for _ in range(6))
+    at = p(state) if team else None
+    capi.check(lib.h2x_softmax_instance_forward_once(dt, n, size, p(t["x"]), p(t["y"]), p(mx), p(ex), p(ws), at, -1, None))
+    torch.cuda.synchronize()
+    arrivals = state.view(torch.int64).reshape(n, -1)[:, 0].clone()
+    capi.check(lib.h2x_softmax_instance_backward_once(dt, n, size, p(t["y"]), p(t["dy"]), p(t["dx"]), p(dp), p(ws), at, -1, None))
+    capi.check(lib.h2x_softmax_instance_max(dt, n, size, p(t["x"]), p(mxs), p(ws), None))
+    capi.check(lib.h2x_softmax_instance_exp(dt, n, size, p(t["x"]), p(mxs), p(t["ys"]), p(exs), p(ws), None))
+    capi.check(lib.h2x_softmax_instance_normalize(dt, n, size, p(exs), p(t["ys"]), None))
+    capi.check(lib.h2x_softmax_instance_dot(dt, n, size, p(t["ys"]), p(t["dy"]), p(dps), p(ws), None))
+    capi.check(lib.h2x_softmax_instance_gradient(dt, n, size, p(t["ys"]), p(t["dy"]), p(dps), p(t["dxs"]), None))
+    torch.cuda.synchronize()
+    served = state.view(torch.int64).reshape(n, -1)[:, 0] > arrivals
+    assert bool(served.any()) == (team and skewed != "dx") and bool(served.all()) == bool(served.any())
+    for a, b in ((mx, mxs), (ex, exs), (t["y"], t["ys"]), (dp, dps), (t["dx"], t["dxs"])):
+        assert torch.equal(a, b)
+    for name, r in room.items():  # nothing beside the tensors was written
+        first = int(name.rstrip("s") == skewed)
+        assert bool((r[:first] == 7).all()) and bool((r[first + n * size:] == 7).all())
