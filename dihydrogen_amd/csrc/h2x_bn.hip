@@ -2830,27 +2830,35 @@ constexpr uint32_t kFewestMembers = 16, kFewestLarger = 128;
 // What a pass takes beyond what all ways to run it share, in us: the bytes it moves, at the rate that members of
 // its size reach, and for every round of workgroups that the chip holds at once what a member needs between its first
 // load and its last store, the longer the larger its team.  Members that are mostly padding cost what full ones do;
-// beyond the first round one that is not full costs half of what it lacks.  In two launches x (backward: x and dy)
-// is read twice.  Fitted to some 12000 calls of 4 to 300 MB a tensor, floats and doubles, each timed in all the ways that hold
-// it, going round three sets of tensors: the way these name takes 0.3 % longer than the fastest one on average, with halos
-// 0.7 (backward) and 1.8 %.  Rules on the number of workgroups alone took 0.6 to 3.5 % longer, and more where the last round
-// is nearly empty or members are mostly padding (forward, N 4, C 16, 96 x 63 x 84, 2000 members of 64 KB, 66 us, as now 53;
-// doubles, forward, backward, N 184, C 91, 23 x 26 with a halo of 1 64, 105 and 57, 85; N 160, C 133, 23 x 19 with a halo of 1 67, 112
-// and 58, 81).  Where two ways are close they may miss: forward, N 32, C 256, 56 x 56, 1792 members of 64 KB 42.0, 1024 of 128 KB 40.4.
+// beyond the first round one that is not full costs less, by a part of what it lacks.  In two launches x (backward: x and dy)
+// is read twice.  Haloed outputs of floats that are stored normally (kHaloedNormalStores) push out what members have read
+// from some 30 MiB on.  Fitted to calls of 4 to 300 MB a tensor, each timed in all the ways that hold it, forward with
+// backward, going round three sets of tensors; where only differences between the ways count.  The way these name makes both
+// together 0.2 % longer than the fastest one on average (2053 dense tensors of floats; also in the half not fitted to), with
+// halos 1.2 % (2402; doubles 0.3 and 1.2).  Rules on the number of workgroups alone made it 0.9 % longer, with
+// halos 2.5, and more where the last round is nearly empty or members are mostly padding (forward, N 4, C 16, 96 x 63 x 84,
+// 2000 members of 64 KB, 66 us, as now 53; doubles, forward, backward, N 184, C 91, 23 x 26 with a halo of 1 64, 105 and 57, 85;
+// N 160, C 133, 23 x 19 with a halo of 1 67, 112 and 58, 81).
 struct PassCost
 {
     float wait; // of a round, for a team of 64
     struct
     {
         float per_mb, per_round;
-    } members[3]; // of 512 threads with 4 and 8 vectors; then 512 with 16 (forward), 1024 with 8 (backward)
+    } members[3]; // of 512 threads with 4 and 8 vectors; then 512 with 16 (forward), 1024 with 8 (backward, floats)
     float launches, launches_per_mb;
+    float displaced_per_mb; // of members
+    float saved; // of what the last round of several lacks
 };
-// dense (or whole) tensors, and rows with a halo between them
-constexpr PassCost kForwardCost[2] = {{2.2f, {{0.31f, 2.5f}, {0.30f, 3.9f}, {0.28f, 6.8f}}, 4.2f, 0.57f},
-                                      {2.0f, {{0.31f, 3.1f}, {0.29f, 4.9f}, {0.30f, 6.8f}}, 5.3f, 0.49f}};
-constexpr PassCost kBackwardCost[2] = {{1.7f, {{0.49f, 2.8f}, {0.38f, 5.4f}, {0.41f, 9.2f}}, 9.3f, 0.78f},
-                                       {1.7f, {{0.47f, 2.9f}, {0.38f, 5.5f}, {0.36f, 10.0f}}, 4.7f, 0.76f}};
+// Floats and doubles, each of dense (or whole) tensors, and of rows with a halo between them.
+constexpr PassCost kForwardCost[2][2] = {{{1.71f, {{0.336f, 2.85f}, {0.329f, 3.8f}, {0.24f, 9.21f}}, 4.2f, 0.57f, 0.0f, 0.3f},
+                                          {2.25f, {{0.345f, 2.69f}, {0.358f, 3.66f}, {0.397f, 4.12f}}, 4.73f, 0.438f, 0.48f, 0.5f}},
+                                         {{2.2f, {{0.31f, 2.5f}, {0.30f, 3.9f}, {0.28f, 6.8f}}, 4.2f, 0.57f, 0.0f, 0.5f},
+                                          {3.65f, {{0.246f, 2.53f}, {0.309f, 3.54f}, {0.272f, 8.04f}}, 4.23f, 0.526f, 0.0f, 0.25f}}};
+constexpr PassCost kBackwardCost[2][2] = {{{0.18f, {{0.522f, 4.28f}, {0.524f, 4.45f}, {0.263f, 13.6f}}, 9.3f, 0.78f, 0.0f, 0.3f},
+                                           {0.01f, {{0.553f, 4.15f}, {0.404f, 7.21f}, {0.615f, 6.6f}}, 5.25f, 0.798f, 0.0f, 0.5f}},
+                                          {{1.7f, {{0.49f, 2.8f}, {0.38f, 5.4f}, {}}, 9.3f, 0.78f, 0.0f, 0.5f},
+                                           {4.03f, {{0.415f, 3.9f}, {0.492f, 5.06f}, {}}, 4.84f, 0.891f, 0.0f, 0.25f}}};
 // Workgroups of each size of member that a CU holds (measured: the time of a call steps up where there is one more).
 constexpr uint32_t kForwardOnCu[3] = {3, 3, 2}, kBackwardOnCu[3] = {3, 2, 1}, kBackwardDoublesOnCu[3] = {2, 2, 1};
 
@@ -2859,7 +2867,14 @@ struct PassShape
     size_t bytes;        // of a tensor, and of the lines at the ends of haloed rows
     uint32_t channels;
     bool rows;           // haloed
+    size_t displaced;    // bytes of haloed rows stored normally, beyond the first 30 MiB
 };
+
+size_t displaced_bytes(size_t bytes, bool stream)
+{
+    constexpr size_t kBeside = size_t(30) << 20;
+    return stream || bytes < kBeside ? 0 : bytes - kBeside;
+}
 
 // Rows that do not follow one another bring up to a line of what is between them along.
 size_t moved_bytes(size_t rows, size_t width, size_t pitch, size_t item)
@@ -2871,7 +2886,7 @@ size_t moved_bytes(size_t rows, size_t width, size_t pitch, size_t item)
 template <typename T, bool FORWARD>
 int cheapest_pass(const PassShape& p, const uint32_t (&members)[3], bool forced)
 {
-    const PassCost& cost = (FORWARD ? kForwardCost : kBackwardCost)[p.rows];
+    const PassCost& cost = (FORWARD ? kForwardCost : kBackwardCost)[sizeof(T) == 8][p.rows];
     const auto& on_cu = FORWARD ? kForwardOnCu : sizeof(T) == 4 ? kBackwardOnCu : kBackwardDoublesOnCu;
     const uint32_t cus = compute_units();
     const float mb = p.bytes * 1e-6f;
@@ -2882,8 +2897,9 @@ int cheapest_pass(const PassShape& p, const uint32_t (&members)[3], bool forced)
         if (members[i] == 0)
             continue;
         const float full = static_cast<float>(static_cast<uint64_t>(members[i]) * p.channels) / ((cus ? cus : 256) * on_cu[i]);
-        const float rounds = full <= 1 ? 1 : (full + std::ceil(full)) / 2;
-        const float us = cost.members[i].per_mb * mb + rounds * (cost.members[i].per_round + cost.wait * members[i] / 64);
+        const float rounds = full <= 1 ? 1 : cost.saved * full + (1 - cost.saved) * std::ceil(full);
+        const float us = cost.members[i].per_mb * mb + rounds * (cost.members[i].per_round + cost.wait * members[i] / 64)
+                         + cost.displaced_per_mb * p.displaced * 1e-6f;
         if (us < least)
         {
             least = us;
@@ -2903,29 +2919,32 @@ uint32_t fit_team(size_t members, uint32_t channels, size_t sums, uint32_t most,
                : static_cast<uint32_t>(members);
 }
 
-PassShape pass_shape(const OnceGeometry& g)
+PassShape pass_shape(const OnceGeometry& g, bool stream)
 {
-    const size_t rows = g.vectors / g.spr.divisor;
-    const size_t pitch = g.h.divisor > 1 ? g.sy : g.d.divisor > 1 ? g.sz : g.width;
-    return {moved_bytes(rows * g.num_channels, g.width, std::max<size_t>(pitch, g.width), sizeof(float)), g.num_channels,
-            !dense_rows(g)};
+    const size_t rows = g.vectors / g.spr.divisor * g.num_channels;
+    const size_t pitch = std::max<size_t>(g.h.divisor > 1 ? g.sy : g.d.divisor > 1 ? g.sz : g.width, g.width);
+    return {moved_bytes(rows, g.width, pitch, sizeof(float)), g.num_channels, !dense_rows(g),
+            displaced_bytes(rows * pitch * sizeof(float), stream)};
 }
-PassShape pass_shape(const ClearGeometry& g)
+PassShape pass_shape(const ClearGeometry& g, bool)
 {
-    return {static_cast<size_t>(g.vectors) * g.num_channels * 16, g.num_channels, false};
+    return {static_cast<size_t>(g.vectors) * g.num_channels * 16, g.num_channels, false, 0};
 }
 
 // Backward, teams of 65 to 128 members of 128 KB only in tensors that the memory-side cache nearly holds.  Dense ones below
 // 240 MiB: 7 % less than two launches on average (N 16, C 10, 64^3, 168 MB, 117 us and 131; N 2, C 6, 110 x 120 x 130 55 and
 // 69; N 8, C 13, 73 x 85 x 84, 217 MB, 162 and 170; 17 % more at worst; N 16, C 16, 64^3, 268 MB, 231 and 202).  With a halo below
 // 104 MiB, where x, dy and dx take half of it: 7 % less (N 100, C 8, 200 x 160, 102 MB, 87 and 101), beyond 9 % more (N 158, C
-// 13, 25 x 23 x 21 128 and 112; N 14, C 11, 65 x 66 x 48, halo of 2, 150 and 133); where the halo is cleared never
-// (4 % more; N 50, C 16, 33 x 36 x 45 with a halo of 2 206 and 171).
+// 13, 25 x 23 x 21 128 and 112; N 14, C 11, 65 x 66 x 48, halo of 2, 150 and 133) unless rows are long, which leaves few partial
+// lines: from 80 elements 1 % less, up to 10 (N 4, C 8, 96^3, forward + backward 154 and 171; N 118, C 15, 124 x 152, halo of 2,
+// 183 and 195).  Where the halo is cleared never (4 % more; N 50, C 16, 33 x 36 x 45 with a halo of 2 206 and 171).
 constexpr size_t kHeldTensor = size_t(240) << 20, kHeldRows = size_t(104) << 20;
+constexpr uint32_t kLongRow = 80;
 
 bool for_large_teams(const OnceGeometry& g)
 {
-    return static_cast<size_t>(g.vectors) * g.num_channels * 16 < (dense_rows(g) ? kHeldTensor : kHeldRows);
+    return static_cast<size_t>(g.vectors) * g.num_channels * 16
+           < (dense_rows(g) || g.width >= kLongRow ? kHeldTensor : kHeldRows);
 }
 bool for_large_teams(const ClearGeometry&)
 {
@@ -2942,7 +2961,7 @@ bool team_variant(const G& g, const OnceForward<T>* a, bool stream, bool forced,
         return fit_team(m, g.num_channels, 2 * m, most, forced ? 1 : least);
     };
     const uint32_t members[3] = {fit(512 * 4, kFewestMembers), fit(512 * 8, kFewestLarger), fit(512 * 16, kFewestLarger)};
-    const int best = cheapest_pass<T, true>(pass_shape(g), members, forced);
+    const int best = cheapest_pass<T, true>(pass_shape(g, stream), members, forced);
     if (best < 0 || !a)
         return best >= 0;
     if (best == 0)
@@ -2964,7 +2983,7 @@ bool team_variant(const G& g, const OnceBackward<T>* a, bool stream, bool forced
     };
     const uint32_t members[3] = {fit(512 * 4, kFewestMembers, most / 2), fit(512 * 8, kFewestLarger, most / 2),
                                  fit(1024 * 8, kFewestLarger, for_large_teams(g) ? most : most / 2)};
-    const int best = cheapest_pass<T, false>(pass_shape(g), members, forced);
+    const int best = cheapest_pass<T, false>(pass_shape(g, stream), members, forced);
     if (best < 0 || !a)
         return best >= 0;
     if (best == 0)
@@ -3164,7 +3183,7 @@ bool ordered_by_teams(const OrderedGeometry& g, const A* a, size_t bytes, bool r
                            ordered_members<512, 8, kSums>(g, kForward ? most : most / 2, larger), 0};
     if constexpr (kForward)
         members[2] = ordered_members<512, 16, kSums>(g, most, larger);
-    const int best = cheapest_pass<double, kForward>({bytes, g.num_channels, rows}, members, forced);
+    const int best = cheapest_pass<double, kForward>({bytes, g.num_channels, rows, 0}, members, forced);
     if (best < 0 || !a)
         return best >= 0;
     if (best == 0)
@@ -3230,8 +3249,8 @@ bool ordered_launch(int n, int c, size_t s, std::initializer_list<const HostTens
     if (team_polls)
         g.max_polls = *team_polls;
     g.streams_gradient = output.strided || streams_gradient(n * s / 2, c);
-    return ordered_variant(g, &a, moved_bytes(output, n, c, s), rows, !output.strided || bytes > kHaloedNormalStores,
-                           teams ? most_members() : 0,
+    const bool stream = !output.strided || bytes > kHaloedNormalStores;
+    return ordered_variant(g, &a, moved_bytes(output, n, c, s), rows, stream, teams ? most_members() : 0,
                            team_polls != nullptr, state, st, &team);
 }
 
