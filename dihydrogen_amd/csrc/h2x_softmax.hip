@@ -1679,26 +1679,28 @@ int inst_map(int n, size_t sample_size, const void* y, const void* dy, const voi
 constexpr int kInstMostForward = 16, kInstMostBackward = 8;
 
 // What a forward pass by members of four chunks takes, and one in separate launches, in us: the bytes, and for every round of the
-// chip, which holds one such member a CU, what it needs for its loads, two exchanges and stores.  Fitted to 1160 calls;
-// members of one chunk, and backward passes, which exchange once, are never slower than separate launches.  Forward,
-// separate launches, by teams: N 6, 2,145,024 floats, 198 members of 256 KB, 40 and 52; N 7, 1,280,796, 280 members of 128 KB,
-// a second round that is nearly empty, 29 and 35; N 4, 3,932,160, 240 members of 256 KB, 58 and 47.
+// chip, which holds one such member a CU, what it needs for its loads, two exchanges and stores; only the difference of both
+// counts.  Fitted to 1380 calls, forward with backward; the way it names makes both 0.1 to 0.2 % longer than the faster one
+// on average, always teams 0.7 (single elements), 3.2 and 4.8 %, never 8.1, 2.7 and 2.2 %.  Members of one chunk, and backward
+// passes, which exchange once, are never slower than separate launches.  Forward, separate launches, by teams: N 6,
+// 2,145,024 floats, 264 members, a second round that is nearly empty, 40 and 52; N 7, 1,280,796, 280 members, 29 and 35; N 4,
+// 3,932,160, 240 members of 256 KB, 58 and 47.
 struct InstForwardCost
 {
-    float team, per_round[3], wait; // per_round: of 64, 128, 256 KB; wait: of a round, for 64 members
+    float team, team_per_mb, per_round[3], wait; // per_round: of 64, 128, 256 KB; wait: of a round, for 64 members
     float launches, launches_per_mb, launches_beyond; // beyond: more a MB from 40 MB
 };
-// whole vectors, single elements
-constexpr InstForwardCost kInstForwardCost[2] = {{5.1f, {4.0f, 8.6f, 13.2f}, 2.1f, 8.9f, 0.56f, 0.24f},
-                                                 {2.0f, {8.6f, 13.6f, 21.0f}, 1.1f, 9.7f, 0.82f, 0.04f}};
-constexpr float kInstTeamPerMb = 0.30f;
+// whole vectors of floats and of doubles, single elements
+constexpr InstForwardCost kInstForwardCost[3] = {{9.19f, 0.122f, {4.82f, 10.4f, 14.2f}, 2.6f, 10.96f, 0.638f, 0.119f},
+                                                 {2.16f, 0.314f, {10.8f, 13.6f, 17.0f}, 1.22f, 10.2f, 0.7f, 0.159f},
+                                                 {0.1f, 0.209f, {9.33f, 9.1f, 0.25f}, 2.69f, 9.46f, 0.774f, 0.027f}};
 
 bool inst_forward_pays(const InstForwardCost& cost, size_t bytes, size_t members, size_t n, int each)
 {
     const uint32_t cus = compute_units();
     const float mb = bytes * 1e-6f, rounds = std::ceil(static_cast<float>(members * n) / (cus ? cus : 256));
     const float round = cost.per_round[each <= 4 ? 0 : each <= 8 ? 1 : 2] + cost.wait * members / 64;
-    return cost.team + kInstTeamPerMb * mb + rounds * round
+    return cost.team + cost.team_per_mb * mb + rounds * round
            < cost.launches + cost.launches_per_mb * mb + cost.launches_beyond * std::max(mb - 40, 0.0f);
 }
 
@@ -1718,7 +1720,7 @@ bool inst_team(int n, size_t sample_size, const void* a, const void* b, const vo
     if (ch.groups > kInstCombine || each > (chunks == 1 ? 16 : most) || 4 * members > static_cast<int>(compute_units()))
         return false;
     if (FORWARD && chunks == 4
-        && !inst_forward_pays(kInstForwardCost[*v != 16 / sizeof(T)], n * sample_size * sizeof(T), members, n, each))
+        && !inst_forward_pays(kInstForwardCost[*v != 16 / sizeof(T) ? 2 : sizeof(T) == 8], n * sample_size * sizeof(T), members, n, each))
         return false;
     g->members = make_fastdiv(static_cast<uint32_t>(members));
     g->chunks = static_cast<uint32_t>(chunks);
