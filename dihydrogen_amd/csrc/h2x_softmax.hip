@@ -1580,14 +1580,15 @@ size_t inst_chunk_bytes(int num_samples)
 
 // Samples that are no whole vectors are cut as those of whole vectors are: with chunks a quarter of that, members of four chunks
 // hold 16 KB, and there are four times as many (forward + backward, by teams, N 23, 142,071 floats 59.7 -> 27.5 us, N 12, 241,997
-// 50.7 -> 26.9; separate launches 37 and 35).  Chunks of more than 32 KB pay there only if members of four fill most of one
-// round of the chip (N 5, 3,054,213 floats, 315 members, 143 us, in chunks of 16 KB, and no teams, 122; N 3, 2,097,657, 129
-// members, 59 and 54; with 144 to 256 members the same either way).
+// 50.7 -> 26.9; separate launches 37 and 35).  Few samples leave CUs idle with members of four such chunks, and are cut finer up to
+// three quarters of a round of the chip (N 2, 138,475 doubles, 34 and 68 members, 17.3 and 16.0; N 2, 439,890 floats 19.6 and 18.7).
+// Chunks of more than 32 KB pay there only if members of four fill most of one round of the chip (N 5, 3,054,213 floats, 315
+// members, 143 us, in chunks of 16 KB, and no teams, 122; N 3, 2,097,657, 129 members, 59 and 54; with 144 to 256 members the same
+// either way).
 InstChunking inst_chunking(size_t sample_size, int num_samples, int vec, size_t elem_bytes)
 {
     const size_t gmax = inst_groups_per_sample_max(num_samples);
-    const size_t tile = kBlockSize * (16 / elem_bytes) * kInstUnroll;
-    const auto cut = [&](size_t bytes) {
+    const auto cut = [&](size_t bytes, size_t tile) {
         const size_t chunk = std::max((sample_size + gmax - 1) / gmax,
                                       std::min((sample_size + kInstCombine - 1) / kInstCombine, bytes / elem_bytes));
         InstChunking c;
@@ -1595,11 +1596,17 @@ InstChunking inst_chunking(size_t sample_size, int num_samples, int vec, size_t 
         c.groups = static_cast<int>((sample_size + c.chunk - 1) / c.chunk);
         return c;
     };
-    const InstChunking c = cut(inst_chunk_bytes(num_samples));
-    if (vec * elem_bytes == 16 || c.chunk * elem_bytes <= (size_t(32) << 10))
+    const size_t most = inst_chunk_bytes(num_samples), tile = kBlockSize * (16 / elem_bytes) * kInstUnroll;
+    const InstChunking c = cut(most, tile);
+    if (vec * elem_bytes == 16)
         return c;
-    const size_t members = static_cast<size_t>((c.groups + 3) / 4) * num_samples;
-    return c.groups <= kInstCombine && members > 140 && members <= 256 ? c : cut(size_t(16) << 10);
+    const auto members = [&](const InstChunking& of) { return static_cast<size_t>((of.groups + 3) / 4) * num_samples; };
+    if (c.chunk * elem_bytes <= (size_t(32) << 10))
+    {
+        const InstChunking fine = cut(most, tile / (16 / elem_bytes));
+        return c.groups > kInstCombine / 4 && fine.groups <= kInstCombine && members(fine) <= 192 ? fine : c;
+    }
+    return c.groups <= kInstCombine && members(c) > 140 && members(c) <= 256 ? c : cut(size_t(16) << 10, tile);
 }
 
 // How a reduction over samples is cut.  out: takes part in the choice of the vector width.
@@ -1719,7 +1726,7 @@ bool inst_team(int n, size_t sample_size, const void* a, const void* b, const vo
     static_assert(4 * kInstMembers >= kInstCombine, "members of four hold all chunks");
     if (ch.groups > kInstCombine || each > (chunks == 1 ? 16 : most) || 4 * members > static_cast<int>(compute_units()))
         return false;
-    if (FORWARD && chunks == 4
+    if (FORWARD && chunks == 4 && each >= 4 // (members of finer chunks are few, and pay)
         && !inst_forward_pays(kInstForwardCost[*v != 16 / sizeof(T) ? 2 : sizeof(T) == 8], n * sample_size * sizeof(T), members, n, each))
         return false;
     g->members = make_fastdiv(static_cast<uint32_t>(members));
