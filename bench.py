@@ -576,17 +576,17 @@ def cpu_baseline(repeats: int = 5):
 # TCC_EA0_WRREQ_64B), request counts summed over the L2 channels, per dispatch.
 # label -> (bytes read, bytes written) per launch
 PMC_TRAFFIC = {
-    "bn_forward": (270147456, 268852736),
-    "bn_backward": (541897088, 269621824),
-    "bn_sums": (268455424, 131072),
-    "bn_apply": (268466176, 268474496),
-    "bn_backprop1": (536909824, 131072),
-    "bn_backprop2": (536907264, 268435456),
-    "halo_dim0_pack": (147893888, 8652800),    # 4 faces (2 ranks) a launch, four launches a step
-    "halo_dim0_unpack": (9221184, 43264000),
+    "bn_forward": (270064640, 268873792),
+    "bn_backward": (541834944, 269624704),
+    "bn_sums": (268458496, 131072),
+    "bn_apply": (268466176, 268472192),
+    "bn_backprop1": (536912960, 131072),
+    "bn_backprop2": (536906240, 268435456),
+    "halo_dim0_pack": (147785216, 8652800),    # 4 faces (2 ranks) a launch, four launches a step
+    "halo_dim0_unpack": (9219200, 43264000),
     "halo_dim1_pack": (42624768, 34611200),
-    "halo_dim1_unpack": (34632448, 36216416),
-    "halo_dim2_pack": (34694400, 34611200),
+    "halo_dim1_unpack": (34632448, 36217760),
+    "halo_dim2_pack": (34695424, 34611200),
     "halo_dim2_unpack": (34632448, 34619392),
 }
 # steps of the timed region whose dominant-kernel launches are bracketed by events: every EVENT_EVERY-th
@@ -594,8 +594,8 @@ EVENT_EVERY = 4
 
 # sha256 (first 16 hex digits) of the kernel sources the table was measured with, see
 # kernel_sources_sha(); with other sources the traffic fields are omitted
-PMC_SOURCES_SHA = "8aead0fd548e93b6"
-PMC_COMMIT = "b6c4b54"
+PMC_SOURCES_SHA = "2e7a97b3560f5c84"
+PMC_COMMIT = "2585ae3"
 
 KERNEL_OF = {
     "bn_forward": "bn_team_forward_kernel<float,512,16>",
