@@ -255,14 +255,8 @@ __global__ __launch_bounds__(once_block<TEAM>()) void bn_once_backward_kernel(co
         return;
     const int64_t base = c * g.stride_c;
     T xv[K][VEC], dv[K > IN_LDS ? K - IN_LDS : 1][VEC];
-    uint32_t at[kKept ? K : 1];
+    uint32_t at[K];
     auto live = [&](int u) { return u * TEAM < g.vectors && u * TEAM + t < g.vectors; };
-    uint32_t again = t; // of the present step: where nothing is kept the compiler shall not keep it either
-    auto place = [&](int u) { return kKept ? at[kKept ? u : 0] : once_place<VEC>(g, u * TEAM + again); };
-    auto next_step = [&] {
-        if constexpr (!kKept)
-            asm volatile("" : "+v"(again));
-    };
     auto gradient = [&](int u, T (&d)[VEC]) {
 #pragma unroll
         for (int j = 0; j < VEC; ++j)
@@ -272,23 +266,21 @@ __global__ __launch_bounds__(once_block<TEAM>()) void bn_once_backward_kernel(co
     for (int u = 0; u < K; ++u)
         if (live(u))
         {
-            const uint32_t p = once_place<VEC>(g, u * TEAM + t);
-            if constexpr (kKept)
-                at[u] = p;
-            load_vec<T, VEC, false>(a.x + base + G::offset(p), xv[u]);
+            at[u] = once_place<VEC>(g, u * TEAM + t);
+            load_vec<T, VEC, false>(a.x + base + G::offset(at[u]), xv[u]);
             if (u < IN_LDS)
             {
                 T d[VEC];
-                load_vec<T, VEC, false>(a.dy + base + G::offset(p), d);
-                V w;
+                load_vec<T, VEC, false>(a.dy + base + G::offset(at[u]), d);
+                V p;
 #pragma unroll
                 for (int j = 0; j < VEC; ++j)
-                    w[j] = d[j];
-                parked[(u < IN_LDS ? u : 0) * TEAM + t] = w;
+                    p[j] = d[j];
+                parked[(u < IN_LDS ? u : 0) * TEAM + t] = p;
             }
             else
             {
-                load_vec<T, VEC, false>(a.dy + base + G::offset(p), dv[u < IN_LDS ? 0 : u - IN_LDS]);
+                load_vec<T, VEC, false>(a.dy + base + G::offset(at[u]), dv[u < IN_LDS ? 0 : u - IN_LDS]);
             }
         }
     const T m = a.mean[c];
@@ -296,17 +288,20 @@ __global__ __launch_bounds__(once_block<TEAM>()) void bn_once_backward_kernel(co
     const T inv_stdev = inv_sqrt_t(a.var[c] + a.epsilon);
     const T dvar_factor = inv_stdev * inv_stdev * inv_stdev / T(2);
     double s[4] = {0.0, 0.0, 0.0, 0.0};
-    next_step();
+    [[maybe_unused]] uint32_t again = t; // of the present step: where nothing is kept the compiler shall not keep it either
+    if constexpr (!kKept)
+        asm volatile("" : "+v"(again));
 #pragma unroll
     for (int u = 0; u < K; ++u)
         if (live(u))
         {
-            const uint32_t p = place(u);
+            if constexpr (!kKept)
+                at[u] = once_place<VEC>(g, u * TEAM + again);
             T d[VEC];
             gradient(u, d);
 #pragma unroll
             for (int j = 0; j < VEC; ++j)
-                if (G::counts(p, j))
+                if (G::counts(at[u], j))
                 {
                     const T xm = xv[u][j] - m;
                     const T dxhat = d[j] * sc;
@@ -329,19 +324,21 @@ __global__ __launch_bounds__(once_block<TEAM>()) void bn_once_backward_kernel(co
     }
     const T dmean_term = dmean / a.n;
     const T dvar_term = dvar * T(2) / a.n_minus_1;
-    next_step();
+    if constexpr (!kKept)
+        asm volatile("" : "+v"(again));
 #pragma unroll
     for (int u = 0; u < K; ++u)
         if (live(u))
         {
-            const uint32_t p = place(u);
+            if constexpr (!kKept)
+                at[u] = once_place<VEC>(g, u * TEAM + again);
             T d[VEC];
             gradient(u, d);
 #pragma unroll
             for (int j = 0; j < VEC; ++j)
-                xv[u][j] = G::kClears && !G::counts(p, j)
+                xv[u][j] = G::kClears && !G::counts(at[u], j)
                                ? T(0)
                                : fma_t(xv[u][j] - m, dvar_term, fma_t(d[j] * sc, inv_stdev, dmean_term));
-            store_once<T, VEC, STREAM>(a.dx + base + G::offset(p), xv[u]);
+            store_once<T, VEC, STREAM>(a.dx + base + G::offset(at[u]), xv[u]);
         }
 }
