@@ -576,16 +576,16 @@ def cpu_baseline(repeats: int = 5):
 # TCC_EA0_WRREQ_64B), request counts summed over the L2 channels, per dispatch.
 # label -> (bytes read, bytes written) per launch
 PMC_TRAFFIC = {
-    "bn_forward": (270064640, 268873792),
-    "bn_backward": (541834944, 269624704),
-    "bn_sums": (268458496, 131072),
-    "bn_apply": (268466176, 268472192),
-    "bn_backprop1": (536912960, 131072),
+    "bn_forward": (270054656, 268850048),
+    "bn_backward": (541286528, 269631328),
+    "bn_sums": (268457472, 131072),
+    "bn_apply": (268466176, 268503808),
+    "bn_backprop1": (536912896, 131072),
     "bn_backprop2": (536906240, 268435456),
-    "halo_dim0_pack": (147785216, 8652800),    # 4 faces (2 ranks) a launch, four launches a step
-    "halo_dim0_unpack": (9219200, 43264000),
+    "halo_dim0_pack": (147835520, 8652800),    # 4 faces (2 ranks) a launch, four launches a step
+    "halo_dim0_unpack": (9219904, 43264000),
     "halo_dim1_pack": (42624768, 34611200),
-    "halo_dim1_unpack": (34632448, 36217760),
+    "halo_dim1_unpack": (34632448, 36215328),
     "halo_dim2_pack": (34695424, 34611200),
     "halo_dim2_unpack": (34632448, 34619392),
 }
@@ -594,8 +594,8 @@ EVENT_EVERY = 4
 
 # sha256 (first 16 hex digits) of the kernel sources the table was measured with, see
 # kernel_sources_sha(); with other sources the traffic fields are omitted
-PMC_SOURCES_SHA = "2e7a97b3560f5c84"
-PMC_COMMIT = "2585ae3"
+PMC_SOURCES_SHA = "abc7713f1a78f849"
+PMC_COMMIT = "9ddd2b6"
 
 KERNEL_OF = {
     "bn_forward": "bn_team_forward_kernel<float,512,16>",
