@@ -52,3 +52,14 @@ def test_large_teams_backward(shape, members):
                                            ((2, 2, 40, 20, 20, 0), 0), ((32, 512, 1, 28, 28, 0), 0)])
 def test_forward(shape, members):
     assert _forward_members(once._Problem(*shape)) == members
+
+
+# members of 64 KB of each tensor, one round of the chip, not three of 32 KB a CU; long haloed rows above 104 MiB
+@pytest.mark.parametrize("shape,members", [((120, 48, 8, 10, 12, 1), 8), ((250, 90, 1, 16, 15, 1), 4), ((4, 8, 96, 96, 96, 1), 108)])
+def test_backward_with_a_halo(shape, members):
+    assert _backward_members(once._Problem(*shape)) == members
+
+
+@pytest.mark.parametrize("shape,members", [((76, 6, 18, 21, 20, 0), 36), ((32, 256, 1, 56, 56, 0), 4)])
+def test_forward_in_larger_members(shape, members):
+    assert _forward_members(once._Problem(*shape)) == members

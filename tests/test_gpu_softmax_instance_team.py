@@ -189,3 +189,20 @@ def test_one_tensor_off_alignment(n, size, dtype, skewed, team):
     for name, r in room.items():  # nothing beside the tensors was written
         first = int(name.rstrip("s") == skewed)
         assert bool((r[:first] == 7).all()) and bool((r[first + n * size:] == 7).all())
+
+
+# members of four chunks of 8 KB, of few samples; of one of 16 KB; whole vectors, members of four in two rounds of the chip
+@pytest.mark.parametrize("n,size,members", [(2, 439890, 54), (3, 332793, 41), (12, 241997, 60), (7, 1004304, 62)])
+def test_members_of_a_forward_pass(n, size, members):
+    import torch
+    from dihydrogen_amd import capi
+    lib, p = capi.load(), lambda t: t.data_ptr()
+    x = torch.randn(n, size, device="cuda")
+    y, mx, ex = torch.empty_like(x), torch.empty(n, device="cuda"), torch.empty(n, device="cuda")
+    ws = torch.empty(lib.h2x_softmax_instance_workspace_bytes(n), dtype=torch.uint8, device="cuda")
+    state = torch.zeros(lib.h2x_softmax_instance_state_needed(capi.F32, n, 40001), dtype=torch.uint8, device="cuda")
+    capi.check(lib.h2x_softmax_instance_forward_once(capi.F32, n, size, p(x), p(y), p(mx), p(ex), p(ws), p(state), -1, None))
+    torch.cuda.synchronize()
+    arrivals = state.view(torch.int64).reshape(n, -1)[:, 0]
+    assert arrivals.tolist() == [members] * n
+    assert bool(((y.double() - torch.softmax(x.double(), 1)).abs() <= 16 * torch.finfo(torch.float32).eps * y.double()).all())
