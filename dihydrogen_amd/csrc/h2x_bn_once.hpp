@@ -124,33 +124,32 @@ __device__ __forceinline__ void store_once(T* p, const T (&r)[VEC])
     }
 }
 
-// Sums over the TEAM threads that share a channel: a wave, or a whole workgroup.
+// N sums over the TEAM threads that share a channel, a wave or a whole workgroup: group k of the lanes of each wave
+// returns the k-th (wave_sums).  lds: N doubles a wave.
 template <int TEAM, int N>
-__device__ __forceinline__ void team_sum(double (&v)[N], double* lds)
+__device__ __forceinline__ double lane_sums(const double (&s)[N], double* lds)
 {
-#pragma unroll
-    for (int k = 0; k < N; ++k)
-        v[k] = wave_sum(v[k]);
+    double v = wave_sums<N>(s);
     if constexpr (TEAM > kWaveSize)
     {
         constexpr int kWaves = TEAM / kWaveSize;
-        if ((threadIdx.x & (kWaveSize - 1)) == 0)
-        {
-#pragma unroll
-            for (int k = 0; k < N; ++k)
-                lds[k * kWaves + threadIdx.x / kWaveSize] = v[k];
-        }
+        constexpr uint32_t kGroup = kWaveSize / N;
+        static_assert(kWaves <= 16, "a group of lanes adds what the waves have left");
+        const uint32_t lane = threadIdx.x % kWaveSize, k = lane / kGroup, w = lane % kGroup;
+        if (w == 0)
+            lds[k * kWaves + threadIdx.x / kWaveSize] = v;
         __syncthreads();
-#pragma unroll
-        for (int k = 0; k < N; ++k)
-        {
-            double t = lds[k * kWaves];
-#pragma unroll
-            for (int w = 1; w < kWaves; ++w)
-                t += lds[k * kWaves + w];
-            v[k] = t;
-        }
+        v = lane_group_sum<N>(w < kWaves ? lds[k * kWaves + w] : 0.0);
     }
+    return v;
+}
+template <int TEAM, int N>
+__device__ __forceinline__ void team_sum(double (&v)[N], double* lds)
+{
+    const double t = lane_sums<TEAM, N>(v, lds);
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+        v[k] = read_lane(t, k * (kWaveSize / N));
 }
 
 // TEAM threads with K vectors each serve a channel; teams of one wave share a

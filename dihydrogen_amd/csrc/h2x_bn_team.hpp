@@ -62,55 +62,124 @@ __host__ __device__ __forceinline__ uint32_t team_member(uint32_t i, uint32_t me
     return xcd * (members / kNumXcd) + (xcd < left ? xcd : left) + i / kNumXcd;
 }
 
-// The sums of all members in v[] of every thread, given this member's own in v[] of
-// thread 0 and the tag it made of the counter.  recompute(member, sums) is called by the
-// whole workgroup.
-template <int TEAM, int N, typename G, typename F>
-__device__ __forceinline__ void team_exchange(double (&v)[N], const TeamGeometry<G>& g, uint32_t member,
-                                              unsigned long long* state, uint32_t tag, double* lds,
-                                              uint32_t* missing, const F& recompute)
+// Teams of up to this many members look at all words at once.  Larger ones look at one word of each member until all have
+// come, and then at the others; between looks they sleep 44 x 64 clocks, 1.2 us: what hundreds of waiting workgroups read
+// takes the memory from those that load (N 4, C 64, 64^3, teams of 32 and 64, forward + backward going round three sets of tensors: all
+// words every 0.1 us 266 us, one word every 0.15 us 245, every 0.4 us 242, every 1.2 us 240, every 1.9 us 242, every 2.9 us 246).
+// Teams of 4 lose by it (N 8, C 64, 56 x 56 11.7 us, one word every 1.2 us 13.5), of 8 and 15 too (N 8, C 64, 30^3 with a halo
+// 73.8 and 74.7).
+constexpr uint32_t kSmallTeam = 16;
+
+// What the waves of a member leave one another, and what a member knows of the others.
+template <int TEAM, int N>
+struct TeamShared
 {
-    const uint32_t members = g.members.divisor, t = threadIdx.x;
-    unsigned long long* const sums = state + kCounterWords;
-    if (t == 0)
+    static constexpr uint32_t kGroup = kWaveSize / N; // lanes, and members that a wave looks after
+    double waves[2][N * TEAM / kWaveSize];
+    double theirs[N][kMaxMembers];
+    double parts[kMaxMembers / kGroup][N];        // what the members of a wave make together
+    unsigned long long late[kMaxMembers / kGroup]; // lanes whose sum was not there in time
+};
+
+// The N sums of all members in v[] of every thread, given this member's own as lane_sums leaves them, and the tag it
+// made of the counter.  The lanes of the first wave that hold the sums store them; a wave looks after as many members as a group
+// has lanes, group k after their k-th sums, and leaves what it adds up to all.  recompute(member, sums): the terms of a thread,
+// called by the whole workgroup.  (With the first thread storing all sums, a thread a member looking at all of its
+// words and two more reductions through LDS, N 8, C 64, 56 x 56, forward + backward, took 13.8 us; so 11.75.)
+template <int TEAM, int N, typename G, typename F>
+__device__ __forceinline__ void team_exchange(double own, double (&v)[N], const TeamGeometry<G>& g, uint32_t member,
+                                              unsigned long long* state, uint32_t tag, TeamShared<TEAM, N>& shared,
+                                              const F& recompute)
+{
+    constexpr uint32_t kGroup = kWaveSize / N;
+    static_assert(TEAM / kWaveSize * kGroup >= kMaxMembers, "a wave for a group of members");
+    const uint32_t members = g.members.divisor, lane = threadIdx.x % kWaveSize, wave = threadIdx.x / kWaveSize;
+    const uint32_t k = lane / kGroup, m = wave * kGroup + lane % kGroup;
+    const uint32_t lookers = (members + kGroup - 1) / kGroup; // waves
+    unsigned long long* const words = state + kCounterWords + 2 * k * members;
+    if (threadIdx.x < kWaveSize && lane % kGroup == 0)
     {
-        team_put<N>(sums, members, member, tag, v);
-        missing[kMaxMembers] = 0;
-        missing[kMaxMembers + 1] = tag;
+        const double mine[1] = {own};
+        team_put<1>(words, members, member, tag, mine);
     }
-    __syncthreads();
-    tag = missing[kMaxMembers + 1];
-    double s[N];
-#pragma unroll
-    for (int k = 0; k < N; ++k)
-        s[k] = 0.0;
-    if (t < members)
+    if (wave < lookers) // uniform
     {
-        const bool there = team_get<N>(sums, members, t, tag, g.max_polls, s);
-        missing[t] = !there;
-        if (!there)
-            missing[kMaxMembers] = 1; // every writer stores the same
-    }
-    __syncthreads();
-    if (t == 0)
-        team_leave(state);
-    if (missing[kMaxMembers])
-        for (uint32_t m = 0; m < members; ++m)
-            if (missing[m]) // uniform
+        const unsigned long long* const at = words + m;
+        double s = 0.0;
+        bool there = m >= members, seen = members <= kSmallTeam;
+        for (uint32_t poll = 0; poll < g.max_polls; ++poll) // uniform
+        {
+            if (poll > 0)
+                __builtin_amdgcn_s_sleep(4);
+            if (!seen)
             {
-                double r[N];
-                recompute(m, r);
-                if (t == m)
+                if (__any(!there && k == N - 1 && team_load(at) >> 32 != tag))
                 {
-#pragma unroll
-                    for (int k = 0; k < N; ++k)
-                        s[k] = r[k];
+                    __builtin_amdgcn_s_sleep(40);
+                    continue;
                 }
+                seen = true;
             }
-    team_sum<TEAM>(s, lds);
+            if (!there)
+            {
+                const unsigned long long lo = team_load(at), hi = team_load(at + members);
+                there = lo >> 32 == tag && hi >> 32 == tag;
+                if (there)
+                    s = __longlong_as_double(hi << 32 | (lo & 0xffffffffull));
+            }
+            if (__all(there))
+                break;
+        }
+        shared.theirs[k][m] = s;
+        const unsigned long long late = __ballot(!there);
+        if (lane == 0)
+            shared.late[wave] = late;
+        const double part = lane_group_sum<N>(s);
+        if (lane % kGroup == 0)
+            shared.parts[wave][k] = part;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+        team_leave(state);
+    unsigned long long late = shared.late[0];
+    for (uint32_t w = 1; w < lookers; ++w)
+        late |= shared.late[w];
+    if (late) // uniform
+    {
+        for (uint32_t i = 0; i < members; ++i)
+        {
+            unsigned long long lanes = 0;
 #pragma unroll
-    for (int k = 0; k < N; ++k)
-        v[k] = s[k];
+            for (int n = 0; n < N; ++n)
+                lanes |= shared.late[i / kGroup] >> (n * kGroup + i % kGroup);
+            if (!(lanes & 1)) // uniform
+                continue;
+            double r[N];
+#pragma unroll
+            for (int n = 0; n < N; ++n)
+                r[n] = 0.0;
+            recompute(i, r);
+            const double t = lane_sums<TEAM, N>(r, shared.waves[1]);
+            if (threadIdx.x < kWaveSize && lane % kGroup == 0)
+                shared.theirs[k][i] = t;
+            __syncthreads(); // waves[1] is written again
+        }
+        if (wave < lookers)
+        {
+            const double part = lane_group_sum<N>(shared.theirs[k][m]);
+            if (lane % kGroup == 0)
+                shared.parts[wave][k] = part;
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+    {
+        double t = shared.parts[0][n];
+        for (uint32_t w = 1; w < lookers; ++w)
+            t += shared.parts[w][n];
+        v[n] = t;
+    }
 }
 
 // The terms of the vector at place `at`.
@@ -150,14 +219,12 @@ __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometr
                                                                       unsigned long long* states)
 {
     constexpr int VEC = 16 / sizeof(T);
-    constexpr int kWaves = TEAM / kWaveSize;
-    __shared__ double lds[3][2 * kWaves];
-    __shared__ uint32_t missing[kMaxMembers + 2];
+    __shared__ TeamShared<TEAM, 2> shared;
     const uint32_t c = fastdiv(blockIdx.x, g.members);
     const uint32_t member = team_member(blockIdx.x - c * g.members.divisor, g.members.divisor);
     const T* const x = a.x + c * g.once.stride_c;
     unsigned long long* const state = states + team_state_at(c);
-    const uint32_t tag = threadIdx.x == 0 ? team_tag(state) : 0;
+    uint32_t tag = team_tag(state);
     const uint32_t first = member * g.span;
     const uint32_t end = first + g.span < g.once.vectors ? first + g.span : g.once.vectors;
     T v[K][VEC];
@@ -175,9 +242,9 @@ __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometr
     for (int u = 0; u < K; ++u)
         if (live(u))
             add_forward_terms<G, T, VEC>(s, v[u], at[u]);
-    team_sum<TEAM>(s, lds[0]);
-    team_exchange<TEAM, 2>(s, g, member, state, tag, lds[1], missing, [&](uint32_t other, double (&r)[2]) {
-        r[0] = r[1] = 0.0;
+    asm volatile("" : "+v"(tag)); // every wave has it before any stores: beyond the barrier others may leave
+    const double own = lane_sums<TEAM, 2>(s, shared.waves[0]);
+    team_exchange<TEAM, 2>(own, s, g, member, state, tag, shared, [&](uint32_t other, double (&r)[2]) {
         const uint32_t stop = (other + 1) * g.span < g.once.vectors ? (other + 1) * g.span : g.once.vectors;
         for (uint32_t i = other * g.span + threadIdx.x; i < stop; i += TEAM)
         {
@@ -186,8 +253,6 @@ __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometr
             load_vec<T, VEC, false>(x + G::offset(p), w);
             add_forward_terms<G, T, VEC>(r, w, p);
         }
-        __syncthreads(); // lds[2] may still be read
-        team_sum<TEAM>(r, lds[2]);
     });
     T m, variance;
     sums_to_mean_var(static_cast<T>(s[0]), static_cast<T>(s[1]), a.n, &m, &variance);
@@ -218,14 +283,12 @@ __global__ __launch_bounds__(TEAM) void bn_team_backward_kernel(const TeamGeomet
                                                                        unsigned long long* states)
 {
     constexpr int VEC = 16 / sizeof(T);
-    constexpr int kWaves = TEAM / kWaveSize;
-    __shared__ double lds[3][4 * kWaves];
-    __shared__ uint32_t missing[kMaxMembers + 2];
+    __shared__ TeamShared<TEAM, 4> shared;
     const uint32_t c = fastdiv(blockIdx.x, g.members);
     const uint32_t member = team_member(blockIdx.x - c * g.members.divisor, g.members.divisor);
     const int64_t base = c * g.once.stride_c;
     unsigned long long* const state = states + team_state_at(c);
-    const uint32_t tag = threadIdx.x == 0 ? team_tag(state) : 0;
+    uint32_t tag = team_tag(state);
     const uint32_t first = member * g.span;
     const uint32_t end = first + g.span < g.once.vectors ? first + g.span : g.once.vectors;
     T xv[K][VEC], dv[K][VEC];
@@ -248,9 +311,9 @@ __global__ __launch_bounds__(TEAM) void bn_team_backward_kernel(const TeamGeomet
     for (int u = 0; u < K; ++u)
         if (live(u))
             add_backward_terms<G, T, VEC>(s, xv[u], dv[u], at[u], m, sc, inv_stdev);
-    team_sum<TEAM>(s, lds[0]);
-    team_exchange<TEAM, 4>(s, g, member, state, tag, lds[1], missing, [&](uint32_t other, double (&r)[4]) {
-        r[0] = r[1] = r[2] = r[3] = 0.0;
+    asm volatile("" : "+v"(tag)); // every wave has it before any stores: beyond the barrier others may leave
+    const double own = lane_sums<TEAM, 4>(s, shared.waves[0]);
+    team_exchange<TEAM, 4>(own, s, g, member, state, tag, shared, [&](uint32_t other, double (&r)[4]) {
         const uint32_t stop = (other + 1) * g.span < g.once.vectors ? (other + 1) * g.span : g.once.vectors;
         for (uint32_t i = other * g.span + threadIdx.x; i < stop; i += TEAM)
         {
@@ -260,8 +323,6 @@ __global__ __launch_bounds__(TEAM) void bn_team_backward_kernel(const TeamGeomet
             load_vec<T, VEC, false>(a.dy + base + G::offset(p), d);
             add_backward_terms<G, T, VEC>(r, w, d, p, m, sc, inv_stdev);
         }
-        __syncthreads(); // lds[2] may still be read
-        team_sum<TEAM>(r, lds[2]);
     });
     const T dmean = static_cast<T>(s[2] * -static_cast<double>(inv_stdev));
     const T dvar = static_cast<T>(s[3] * -static_cast<double>(dvar_factor));

@@ -179,6 +179,52 @@ __device__ __forceinline__ T wave_combine(T v, const F& f)
     return f(v, dpp_move<kDppQuadSwap1>(v));
 }
 
+// Several sums over the 64 lanes of a wave at once: the lanes are cut into N groups (two or four), and group k returns the
+// total of v[k], all its lanes the same bits.  In a fixed order.  Four sums take seven additions in a row so, one after another 24.
+template <int N>
+__device__ __forceinline__ double lane_group_sum(double v)
+{
+    static_assert(N == 2 || N == 4, "groups of 32 or of 16 lanes");
+    if constexpr (N == 2)
+        v = combine_apart<16>(v, [](double a, double b) { return a + b; });
+    v += dpp_move<kDppRowRor8>(v);
+    v += dpp_move<kDppRowRor4>(v); // lanes 8 apart hold the same
+    v += dpp_move<kDppQuadSwap2>(v);
+    return v + dpp_move<kDppQuadSwap1>(v);
+}
+// Of each pair of lanes D (16 or 32) apart: the sum of a in the even row (lower half), that of b in the odd one.
+template <int D>
+__device__ __forceinline__ double add_apart(double a, double b)
+{
+    const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+    const uint32_t xl = static_cast<uint32_t>(x), xh = static_cast<uint32_t>(x >> 32), yl = static_cast<uint32_t>(y),
+                   yh = static_cast<uint32_t>(y >> 32);
+    // what a has in the odd rows and b in the even ones change places
+    const auto lo = D == 16 ? __builtin_amdgcn_permlane16_swap(xl, yl, false, false)
+                            : __builtin_amdgcn_permlane32_swap(xl, yl, false, false);
+    const auto hi = D == 16 ? __builtin_amdgcn_permlane16_swap(xh, yh, false, false)
+                            : __builtin_amdgcn_permlane32_swap(xh, yh, false, false);
+    const uint32_t l0 = lo[0], l1 = lo[1], h0 = hi[0], h1 = hi[1];
+    return __longlong_as_double(static_cast<long long>(static_cast<unsigned long long>(h0) << 32 | l0))
+           + __longlong_as_double(static_cast<long long>(static_cast<unsigned long long>(h1) << 32 | l1));
+}
+template <int N>
+__device__ __forceinline__ double wave_sums(const double (&v)[N])
+{
+    if constexpr (N == 2)
+        return lane_group_sum<2>(add_apart<32>(v[0], v[1]));
+    else
+        return lane_group_sum<4>(add_apart<16>(add_apart<32>(v[0], v[2]), add_apart<32>(v[1], v[3])));
+}
+// What lane `lane` holds, in a scalar register.
+__device__ __forceinline__ double read_lane(double v, int lane)
+{
+    const unsigned long long bits = __double_as_longlong(v);
+    const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(bits), lane);
+    const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(bits >> 32), lane);
+    return __longlong_as_double(static_cast<long long>(static_cast<unsigned long long>(hi) << 32 | lo));
+}
+
 // Steps of wave_sum from those that add lanes `first` apart (1, 2 or 4).  Lanes that are no multiple of
 // `first` hold nothing and get nothing.
 __device__ __forceinline__ double wave_sum_from(double v, uint32_t first)
