@@ -14,10 +14,10 @@
 //
 // Bound by memory, and by the wait for the last member of a team.  Two launches each way ->
 // this, forward + backward, us going round three sets of tensors:
-//   N 8, C 32, 33^3              98 -> 87       N 4, C 64, 56 x 56            19 -> 14
-//   N 64, C 512, 20 x 20        137 -> 109      N 8, C 100, 64 x 64           40 -> 29
-//   N 16, C 32, 112 x 112        70 -> 55       N 12, C 9, 113 x 123, halo    27 -> 22
-//   N 4, C 213, 17 x 20 x 23, halo of 1  85 -> 76
+//   N 8, C 32, 33^3              98 -> 75       N 4, C 64, 56 x 56            19 -> 12.5
+//   N 64, C 512, 20 x 20        137 -> 101      N 8, C 100, 64 x 64           40 -> 26
+//   N 16, C 32, 112 x 112        70 -> 49       N 12, C 9, 113 x 123, halo    27 -> 21
+//   N 4, C 213, 17 x 20 x 23, halo of 1  85 -> 72
 // (33^3 is 18 units a segment, the last of them half empty: 144 groups, 36 members.)
 #pragma once
 
@@ -96,14 +96,13 @@ __device__ __forceinline__ void ordered_partials(const OrderedGeometry& g, doubl
             add(b * kOrderedBatch + j, s);
         if (b - p * g.group_batches.divisor + 1 < g.group_batches.divisor)
             continue;
+        const double t = wave_sums_in_order<N>(s);
+        if (threadIdx.x % kWaveSize < N)
+            sums[((p * kQuarters + wave / kWavesPerBlock) * kWavesPerBlock + wave % kWavesPerBlock) * N
+                 + threadIdx.x % kWaveSize] = t;
 #pragma unroll
         for (int k = 0; k < N; ++k)
-        {
-            const double t = wave_sum(s[k]);
-            if (threadIdx.x % kWaveSize == 0)
-                sums[((p * kQuarters + wave / kWavesPerBlock) * kWavesPerBlock + wave % kWavesPerBlock) * N + k] = t;
             s[k] = 0.0;
-        }
     }
 }
 
@@ -121,103 +120,165 @@ __device__ __forceinline__ double ordered_partial(const double* sums, uint32_t l
     return 0.0 + t; // as channel_totals starts
 }
 
-// channel_totals over what the first 256 threads hold: lanes `first` apart.  lds: N times four doubles.
-template <int N>
-__device__ __forceinline__ void ordered_totals(double (&v)[N], uint32_t first, double* lds)
+// What the waves of a workgroup leave one another.
+template <int TEAM, int K, int N, bool TEAMS>
+struct OrderedShared
 {
-    if (threadIdx.x < kBlockSize)
-    {
-#pragma unroll
-        for (int k = 0; k < N; ++k)
-        {
-            const double t = wave_sum_from(v[k], first);
-            if (threadIdx.x % kWaveSize == 0)
-                lds[k * kWavesPerBlock + threadIdx.x / kWaveSize] = t;
-        }
-    }
-    __syncthreads();
+    double sums[TEAM / kBlockSize * (K / kOrderedBatch) * kWavesPerBlock * N];
+    double waves[N][kWavesPerBlock];              // of the waves of a staged finishing workgroup
+    unsigned long long late[TEAMS ? kWavesPerBlock : 1]; // lanes whose sum was not there in time
+};
+
+// The totals of those waves.
+template <int N>
+__device__ __forceinline__ void ordered_totals(double (&v)[N], const double (&waves)[N][kWavesPerBlock])
+{
 #pragma unroll
     for (int k = 0; k < N; ++k)
     {
-        double t = lds[k * kWavesPerBlock];
+        double t = waves[k][0];
 #pragma unroll
         for (int w = 1; w < kWavesPerBlock; ++w)
-            t += lds[k * kWavesPerBlock + w];
+            t += waves[k][w];
         v[k] = t;
     }
 }
 
-// The sums of the channel in v[] of every thread, from the partial sums in `sums`.  Teams: as
-// team_exchange, tags and all; recompute(m) leaves the partial sums of member m in `sums`.
+// The sums of the channel in v[] of every thread, from the partial sums in `shared`.  Teams: a counter, tags and looks as in
+// team_exchange; recompute(m) leaves the partial sums of member m in `shared`.  What a thread of channel_totals starts
+// with, or the thread in steps of two or four where the members exchange sums of as many partials, the same lane of the first four
+// waves looks for; the lanes in between take the other sums, so that the steps of the tree that are left add
+// all of them at once.  (With a lane an item, all its sums one after another, N 8, C 32, 33^3 forward + backward, took 86.2 us,
+// so 75.4; N 24, C 461, 24 x 30 with a halo of 1 98.8 and 86.0; N 16, C 32, 112 x 112 54.7 and 49.0.)
 template <int TEAM, int K, int N, bool TEAMS, typename F>
 __device__ __forceinline__ void ordered_exchange(double (&v)[N], const OrderedGeometry& g, uint32_t member,
-                                                 unsigned long long* state, uint32_t tag, double* sums, double* lds,
-                                                 uint32_t* missing, const F& recompute)
+                                                 unsigned long long* state, uint32_t tag,
+                                                 OrderedShared<TEAM, K, N, TEAMS>& shared, const F& recompute)
 {
     constexpr uint32_t kQuarters = TEAM / kBlockSize;
     const uint32_t t = threadIdx.x, own = g.passes * kQuarters; // groups of a member
+    const uint32_t lane = t % kWaveSize, wave = t / kWaveSize;
+    __syncthreads();
     if constexpr (!TEAMS)
     {
-        __syncthreads();
+        if (t < kBlockSize)
+        {
 #pragma unroll
-        for (int k = 0; k < N; ++k)
-            v[k] = t < own ? ordered_partial<N>(sums, t, t < g.groups, k) : 0.0;
-        ordered_totals<N>(v, 1, lds);
+            for (int k = 0; k < N; ++k)
+                v[k] = t < own ? ordered_partial<N>(shared.sums, t, t < g.groups, k) : 0.0;
+            const double total = wave_sums_in_order<N>(v);
+            if (lane < N)
+                shared.waves[lane][wave] = total;
+        }
+        __syncthreads();
+        ordered_totals<N>(v, shared.waves);
     }
     else
     {
         // an item: what the tree makes of two or four neighbouring partial sums
         const uint32_t width = own % 4 == 0 ? 4 : 2, per_member = own / width;
-        const uint32_t items = (g.groups + width - 1) / width, item = t / width;
+        const uint32_t items = (g.groups + width - 1) / width;
         const auto item_of = [&](uint32_t m, uint32_t i, int k) {
             const auto at = [&](uint32_t j) {
-                return ordered_partial<N>(sums, i * width + j, m * own + i * width + j < g.groups, k);
+                return ordered_partial<N>(shared.sums, i * width + j, m * own + i * width + j < g.groups, k);
             };
             const double low = at(0) + at(1);
             return width == 2 ? low : low + (at(2) + at(3));
         };
         unsigned long long* const words = state + kCounterWords;
-        if (t < kMaxMembers)
-            missing[t] = 0;
-        if (t == 0)
+        if (t < per_member * N && member * per_member + t / N < items)
         {
-            missing[kMaxMembers] = 0;
-            missing[kMaxMembers + 1] = tag;
+            const double mine[1] = {item_of(member, t / N, t % N)};
+            team_put<1>(words + 2 * (t % N) * items, items, member * per_member + t / N, tag, mine);
         }
-        __syncthreads();
-        tag = missing[kMaxMembers + 1];
-        if (t < per_member && member * per_member + t < items)
+        // the sums of its item that a lane looks for: one, or, of four with items on every other lane, two
+        const uint32_t item = t / width, first = t % width;
+        const bool two = N == 4 && width == 2; // uniform
+        const bool reads = t < kBlockSize && item < items && first < N;
+        double s[2] = {0.0, 0.0};
+        const auto leave_waves = [&] {
+            if (t >= kBlockSize)
+                return;
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                if (i == 0 || two)
+                {
+                    const double total = wave_sum_from(s[i], width);
+                    const uint32_t k = first + i * 2;
+                    if (lane < width && k < N)
+                        shared.waves[k][wave] = total;
+                }
+        };
+        if (t < kBlockSize) // whole waves
         {
-            double own_items[N];
-#pragma unroll
-            for (int k = 0; k < N; ++k)
-                own_items[k] = item_of(member, t, k);
-            team_put<N>(words, items, member * per_member + t, tag, own_items);
+            const unsigned long long* const at = words + 2 * first * items + item;
+            bool there = !reads, seen = items <= kSmallTeam;
+            for (uint32_t poll = 0; poll < g.max_polls; ++poll) // uniform
+            {
+                if (poll > 0)
+                    __builtin_amdgcn_s_sleep(4);
+                if (!seen)
+                {
+                    if (__any(!there && first == 0 && team_load(at) >> 32 != tag))
+                    {
+                        if (gridDim.x > kCrowd) // uniform
+                            __builtin_amdgcn_s_sleep(40);
+                        continue;
+                    }
+                    seen = true;
+                }
+                if (!there)
+                {
+                    double one[1];
+                    there = team_get<1>(at, items, 0, tag, 1, one);
+                    s[0] = one[0];
+                    if (two)
+                    {
+                        there = team_get<1>(at + 4 * items, items, 0, tag, 1, one) && there;
+                        s[1] = one[0];
+                    }
+                }
+                if (__all(there))
+                    break;
+            }
+            if (!there || !reads)
+                s[0] = s[1] = 0.0;
+            const unsigned long long late = __ballot(!there);
+            if (lane == 0)
+                shared.late[wave] = late;
+            leave_waves();
         }
-#pragma unroll
-        for (int k = 0; k < N; ++k)
-            v[k] = 0.0;
-        const bool reads = t % width == 0 && t < kBlockSize && item < items;
-        if (reads && !team_get<N>(words, items, item, tag, g.max_polls, v)) // every writer stores the same
-            missing[item / per_member] = missing[kMaxMembers] = 1;
         __syncthreads();
         if (t == 0)
             team_leave(state);
-        if (missing[kMaxMembers])
-            for (uint32_t m = 0; m < g.members.divisor; ++m)
-                if (missing[m]) // uniform
-                {
-                    __syncthreads(); // the sums may still be read
-                    recompute(m);
-                    __syncthreads();
-                    if (reads && item / per_member == m)
-                    {
+        unsigned long long late = 0;
 #pragma unroll
-                        for (int k = 0; k < N; ++k)
-                            v[k] = item_of(m, item - m * per_member, k);
-                    }
+        for (int w = 0; w < kWavesPerBlock; ++w)
+            late |= shared.late[w];
+        if (late) // uniform
+        {
+            for (uint32_t m = 0; m < g.members.divisor; ++m)
+            {
+                bool missing = false;
+                for (uint32_t i = m * per_member; i < (m + 1) * per_member && i < items; ++i)
+                    missing = missing
+                              || (shared.late[i * width / kWaveSize] >> i * width % kWaveSize & ((1u << width) - 1)) != 0;
+                if (!missing) // uniform
+                    continue;
+                __syncthreads(); // the sums may still be read
+                recompute(m);
+                __syncthreads();
+                if (reads && item / per_member == m)
+                {
+                    s[0] = item_of(m, item - m * per_member, first);
+                    if (two)
+                        s[1] = item_of(m, item - m * per_member, first + 2);
                 }
-        ordered_totals<N>(v, width, lds);
+            }
+            leave_waves();
+            __syncthreads();
+        }
+        ordered_totals<N>(v, shared.waves);
     }
 }
 
@@ -240,15 +301,14 @@ __global__ __launch_bounds__(TEAM, TEAMS ? 4 : 1) void bn_ordered_forward_kernel
                                                                   unsigned long long* states)
 {
     typedef double T;
-    constexpr int VEC = 2, kQuarters = TEAM / kBlockSize;
-    __shared__ double sums[kQuarters * (K / kOrderedBatch) * kWavesPerBlock * 2], lds[2 * kWavesPerBlock];
-    __shared__ uint32_t missing[TEAMS ? kMaxMembers + 2 : 1];
+    constexpr int VEC = 2;
+    __shared__ OrderedShared<TEAM, K, 2, TEAMS> shared;
     uint32_t member;
     const uint32_t c = ordered_channel<TEAMS>(g, &member);
     if (c >= g.num_channels)
         return;
     unsigned long long* const state = TEAMS ? states + team_state_at(c) : nullptr;
-    const uint32_t tag = TEAMS && threadIdx.x == 0 ? team_tag(state) : 0;
+    uint32_t tag = TEAMS ? team_tag(state) : 0;
     const uint32_t quarter = __builtin_amdgcn_readfirstlane(threadIdx.x / kBlockSize), t = threadIdx.x % kBlockSize;
     const T* const x = a.x + c * g.map.stride_c;
     const auto place = [&](uint32_t m, int u) {
@@ -275,13 +335,15 @@ __global__ __launch_bounds__(TEAM, TEAMS ? 4 : 1) void bn_ordered_forward_kernel
         if (at[u] != kNowhere)
             load_vec<T, VEC, !ROWS>(x + (at[u] >> 1), v[u]);
     }
-    ordered_partials<TEAM, K, 2>(g, sums, [&](int u, double (&s)[2]) {
+    ordered_partials<TEAM, K, 2>(g, shared.sums, [&](int u, double (&s)[2]) {
         if (at[u] != kNowhere)
             terms(s, v[u], at[u]);
     });
+    if constexpr (TEAMS)
+        asm volatile("" : "+v"(tag)); // every wave has it before any stores
     double s[2];
-    ordered_exchange<TEAM, K, 2, TEAMS>(s, g, member, state, tag, sums, lds, missing, [&](uint32_t other) {
-        ordered_partials<TEAM, K, 2>(g, sums, [&](int u, double (&r)[2]) {
+    ordered_exchange<TEAM, K, 2, TEAMS>(s, g, member, state, tag, shared, [&](uint32_t other) {
+        ordered_partials<TEAM, K, 2>(g, shared.sums, [&](int u, double (&r)[2]) {
             const uint32_t p = place(other, u);
             if (p == kNowhere)
                 return;
@@ -319,15 +381,14 @@ __global__ __launch_bounds__(TEAM, TEAMS ? 4 : 1) void bn_ordered_backward_kerne
                                                                    unsigned long long* states)
 {
     typedef double T;
-    constexpr int VEC = 2, kQuarters = TEAM / kBlockSize;
-    __shared__ double sums[kQuarters * (K / kOrderedBatch) * kWavesPerBlock * 4], lds[4 * kWavesPerBlock];
-    __shared__ uint32_t missing[TEAMS ? kMaxMembers + 2 : 1];
+    constexpr int VEC = 2;
+    __shared__ OrderedShared<TEAM, K, 4, TEAMS> shared;
     uint32_t member;
     const uint32_t c = ordered_channel<TEAMS>(g, &member);
     if (c >= g.num_channels)
         return;
     unsigned long long* const state = TEAMS ? states + team_state_at(c) : nullptr;
-    const uint32_t tag = TEAMS && threadIdx.x == 0 ? team_tag(state) : 0;
+    uint32_t tag = TEAMS ? team_tag(state) : 0;
     const uint32_t quarter = __builtin_amdgcn_readfirstlane(threadIdx.x / kBlockSize), t = threadIdx.x % kBlockSize;
     const int64_t base = c * g.map.stride_c;
     const auto place = [&](uint32_t m, int u) {
@@ -367,13 +428,15 @@ __global__ __launch_bounds__(TEAM, TEAMS ? 4 : 1) void bn_ordered_backward_kerne
                 s[3] = __builtin_fma(dxhat * xm, neg_fac, s[3]);
             }
     };
-    ordered_partials<TEAM, K, 4>(g, sums, [&](int u, double (&s)[4]) {
+    ordered_partials<TEAM, K, 4>(g, shared.sums, [&](int u, double (&s)[4]) {
         if (at[u] != kNowhere)
             terms(s, xv[u], dv[u], at[u]);
     });
+    if constexpr (TEAMS)
+        asm volatile("" : "+v"(tag)); // every wave has it before any stores
     double s[4];
-    ordered_exchange<TEAM, K, 4, TEAMS>(s, g, member, state, tag, sums, lds, missing, [&](uint32_t other) {
-        ordered_partials<TEAM, K, 4>(g, sums, [&](int u, double (&r)[4]) {
+    ordered_exchange<TEAM, K, 4, TEAMS>(s, g, member, state, tag, shared, [&](uint32_t other) {
+        ordered_partials<TEAM, K, 4>(g, shared.sums, [&](int u, double (&r)[4]) {
             const uint32_t p = place(other, u);
             if (p == kNowhere)
                 return;

@@ -62,13 +62,16 @@ __host__ __device__ __forceinline__ uint32_t team_member(uint32_t i, uint32_t me
     return xcd * (members / kNumXcd) + (xcd < left ? xcd : left) + i / kNumXcd;
 }
 
-// Teams of up to this many members look at all words at once.  Larger ones look at one word of each member until all have
-// come, and then at the others; between looks they sleep 44 x 64 clocks, 1.2 us: what hundreds of waiting workgroups read
-// takes the memory from those that load (N 4, C 64, 64^3, teams of 32 and 64, forward + backward going round three sets of tensors: all
-// words every 0.1 us 266 us, one word every 0.15 us 245, every 0.4 us 242, every 1.2 us 240, every 1.9 us 242, every 2.9 us 246).
-// Teams of 4 lose by it (N 8, C 64, 56 x 56 11.7 us, one word every 1.2 us 13.5), of 8 and 15 too (N 8, C 64, 30^3 with a halo
-// 73.8 and 74.7).
-constexpr uint32_t kSmallTeam = 16;
+// Teams of up to kSmallTeam members look at all words at once.  Larger ones look at one word of each member until all have
+// come, and then at the others: what waiting workgroups read takes the memory from those that load.  Between looks they sleep
+// 4 x 64 clocks, 0.1 us, and 44 x 64, 1.2 us, where a launch has more than kCrowd workgroups, about those that the chip holds at
+// once, hundreds of which wait all the time.  N 4, C 64, 64^3, teams of 32 and 64, forward + backward going round three sets
+// of tensors: all words every 0.1 us 266 us, one word every 0.15 us 245, every 0.4 us 242, every 1.2 us 240, every 1.9 us 242, every
+// 2.9 us 246.  Small teams lose by one word every 1.2 us (of 4, N 8, C 64, 56 x 56, 11.7 us and 13.5; of 8 and 15, N 8, C 64, 30^3 with
+// a halo, 73.8 and 74.7), small launches by the long sleep (N 3, C 6, 43 x 50 x 38 15.1 us, with the short one 13.6; N 15, C 4, 22 x
+// 17 x 22, doubles, 15.1 and 13.9; up to 1024 workgroups, N 23, C 21, 144 x 155, 45.0 and 42.0), doubles by all words there (N 81, C 9, 33 x 41 16.9
+// and 19.0).
+constexpr uint32_t kSmallTeam = 16, kCrowd = 1024;
 
 // What the waves of a member leave one another, and what a member knows of the others.
 template <int TEAM, int N>
@@ -115,7 +118,8 @@ __device__ __forceinline__ void team_exchange(double own, double (&v)[N], const 
             {
                 if (__any(!there && k == N - 1 && team_load(at) >> 32 != tag))
                 {
-                    __builtin_amdgcn_s_sleep(40);
+                    if (gridDim.x > kCrowd) // uniform
+                        __builtin_amdgcn_s_sleep(40);
                     continue;
                 }
                 seen = true;

@@ -216,6 +216,30 @@ __device__ __forceinline__ double wave_sums(const double (&v)[N])
     else
         return lane_group_sum<4>(add_apart<16>(add_apart<32>(v[0], v[2]), add_apart<32>(v[1], v[3])));
 }
+// wave_sum of two or four sums at once, bit for bit: lane k (k < N) returns the total of v[k].  The first steps of the
+// tree, lanes 1 apart and, of four sums, 2 apart, leave one sum a lane; the others take an addition each.
+template <int N>
+__device__ __forceinline__ double wave_sums_in_order(const double (&v)[N])
+{
+    static_assert(N == 2 || N == 4, "a sum a lane of a pair or a quad");
+    // even lanes (of quads: the lower pair) keep the first of two and send the second
+    const auto halve = [](bool upper, double a, double b, auto swap) {
+        return (upper ? b : a) + swap(upper ? a : b);
+    };
+    const uint32_t lane = threadIdx.x;
+    const auto next = [](double x) { return dpp_move<kDppQuadSwap1>(x); };
+    const auto pair = [](double x) { return dpp_move<kDppQuadSwap2>(x); };
+    double t = halve(lane & 1, v[0], v[1], next);
+    if constexpr (N == 4)
+        t = halve(lane & 2, t, halve(lane & 1, v[2], v[3], next), pair);
+    else
+        t += pair(t);
+    t += dpp_move<kDppRowRor4>(t);
+    t += dpp_move<kDppRowRor8>(t);
+    const auto add = [](double a, double b) { return a + b; };
+    t = combine_apart<16>(t, add);
+    return combine_apart<32>(t, add);
+}
 // What lane `lane` holds, in a scalar register.
 __device__ __forceinline__ double read_lane(double v, int lane)
 {
