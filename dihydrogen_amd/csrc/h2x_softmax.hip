@@ -1685,30 +1685,29 @@ int inst_map(int n, size_t sample_size, const void* y, const void* dy, const voi
 // Vectors of 16 bytes a thread that members of four chunks hold at most: beyond, 1024 threads lack the registers.
 constexpr int kInstMostForward = 16, kInstMostBackward = 8;
 
-// What a forward pass by members of four chunks takes, and one in separate launches, in us: the bytes, and for every round of the
-// chip, which holds one such member a CU, what it needs for its loads, two exchanges and stores; only the difference of both
-// counts.  Fitted to 1380 calls, forward with backward; the way it names makes both 0.1 to 0.2 % longer than the faster one
-// on average, always teams 0.7 (single elements), 3.2 and 4.8 %, never 8.1, 2.7 and 2.2 %.  Members of one chunk, and backward
-// passes, which exchange once, are never slower than separate launches.  Forward, separate launches, by teams: N 6,
-// 2,145,024 floats, 264 members, a second round that is nearly empty, 40 and 52; N 7, 1,280,796, 280 members, 29 and 35; N 4,
-// 3,932,160, 240 members of 256 KB, 58 and 47.
+// What a forward pass by members of four chunks takes more than one in separate launches, in us: by the bytes, and for every
+// round of the chip, which holds two members of up to four vectors a thread a CU, or one larger one (of eight, whose team may fill
+// a quarter of the chip, the second ones start late), what it needs for its loads, two exchanges and stores.  Fitted to 353 calls,
+// forward with backward; the way it names makes both 0.1 to 0.2 % longer than the faster one on average (also of 170
+// calls not fitted to), 3.9 at most, always teams 0.6, 0.5 and (single elements) 0.1, never 6.8, 6.4 and 15.7 %.  Members of one chunk, and
+// backward passes, which exchange once, are never slower than separate launches.  Forward + backward, separate launches,
+// by teams: N 1, 760,320 floats 16.7 and 17.8; N 2, 1,853,544 27.3 and 28.1; N 7, 1,280,796, more than a round, 62 and 61; N 24,
+// 318,008 45.2 and 38.8; N 7, 264,306 23.2 and 19.2; N 4, 915,840 doubles 43.3 and 38.7.
 struct InstForwardCost
 {
-    float team, team_per_mb, per_round[3], wait; // per_round: of 64, 128, 256 KB; wait: of a round, for 64 members
-    float launches, launches_per_mb, launches_beyond; // beyond: more a MB from 40 MB
+    float base, per_mb, per_mb_beyond, per_round[3], wait; // beyond: 40 MB; per_round: of 64, 128, 256 KB; wait: of a round, for 64 members
 };
 // whole vectors of floats and of doubles, single elements
-constexpr InstForwardCost kInstForwardCost[3] = {{9.19f, 0.122f, {4.82f, 10.4f, 14.2f}, 2.6f, 10.96f, 0.638f, 0.119f},
-                                                 {2.16f, 0.314f, {10.8f, 13.6f, 17.0f}, 1.22f, 10.2f, 0.7f, 0.159f},
-                                                 {0.1f, 0.209f, {9.33f, 9.1f, 0.25f}, 2.69f, 9.46f, 0.774f, 0.027f}};
+constexpr InstForwardCost kInstForwardCost[3] = {{-2.19f, -0.179f, -0.292f, {0.71f, 2.1f, 4.91f}, 4.17f},
+                                                 {-0.52f, -0.182f, -0.155f, {-0.75f, 0.51f, 7.41f}, 3.17f},
+                                                 {-7.29f, -0.419f, 0.04f, {5.79f, 5.13f, 15.2f}, 3.93f}};
 
 bool inst_forward_pays(const InstForwardCost& cost, size_t bytes, size_t members, size_t n, int each)
 {
     const uint32_t cus = compute_units();
-    const float mb = bytes * 1e-6f, rounds = std::ceil(static_cast<float>(members * n) / (cus ? cus : 256));
+    const float mb = bytes * 1e-6f, on_chip = static_cast<float>((cus ? cus : 256) * (each <= 4 ? 2 : 1));
     const float round = cost.per_round[each <= 4 ? 0 : each <= 8 ? 1 : 2] + cost.wait * members / 64;
-    return cost.team + cost.team_per_mb * mb + rounds * round
-           < cost.launches + cost.launches_per_mb * mb + cost.launches_beyond * std::max(mb - 40, 0.0f);
+    return cost.base + cost.per_mb * mb + cost.per_mb_beyond * std::max(mb - 40, 0.0f) + std::ceil(members * n / on_chip) * round < 0;
 }
 
 // A team for samples cut as the staged sums are, or false: of up to 64 members of one chunk, or of four (see

@@ -11,10 +11,10 @@
 // partial t.  Members of four chunks exchange sums of four neighbouring partials, the first
 // steps of that tree.  Separate launches -> by teams, forward + backward, us, going round three
 // sets of tensors:
-//   N 1, 33,759 elements     15.8 -> 11.8      N 8, 800,000             48.0 -> 39.5
-//   N 16, 86,016             19.2 -> 16.6      N 32, 344,064            74.7 -> 61.9
-//   N 2, 58,100              16.0 -> 12.8      N 32, 688,128           134.9 -> 114
-//   N 1, 773,145             23.3 -> 19.6      N 4, 3,932,160           98.2 -> 87.2
+//   N 1, 33,759 elements     15.8 -> 10.9      N 8, 800,000             48.0 -> 39.6
+//   N 16, 86,016             19.2 -> 15.8      N 32, 344,064            74.7 -> 56.9
+//   N 2, 58,100              16.0 -> 9.8       N 32, 688,128           134.9 -> 102
+//   N 1, 773,145             23.3 -> 18.9      N 4, 3,932,160           98.2 -> 86.3
 // A member looks at what all others store: with members of one chunk throughout, 256 of them, N 2,
 // 1,048,576 elements took 29.6 us, of four 22.6.  Up to 64 chunks more CUs are worth more (16 x 86,016
 // in members of four 17.3, N 1, 158,652 15.3 and 13.8).
@@ -37,47 +37,15 @@ struct InstTeam
     unsigned long long* states;
 };
 
-// What member m exchanges in thread TEAM / kBlockSize * m, given this member's own in thread 0.
-// recompute(member) is called by the whole workgroup.  shared: kInstMembers + 2 words.
-template <int TEAM, int WHICH, typename F>
-__device__ __forceinline__ double inst_exchange(double part, const InstTeam& g, uint32_t member,
-                                                unsigned long long* state, uint32_t* tag, uint32_t* shared,
-                                                const F& recompute)
+// What the waves of a member leave one another.  Each array is written once, so nothing waits for it to be read.
+template <int TEAM>
+struct InstShared
 {
-    constexpr uint32_t kChunks = TEAM / kBlockSize;
-    const uint32_t members = g.members.divisor, t = threadIdx.x;
-    unsigned long long* const words = state + kCounterWords + WHICH * 2 * kInstMembers;
-    if (t == 0)
-    {
-        const double own[1] = {part};
-        team_put<1>(words, kInstMembers, member, *tag, own);
-        shared[kInstMembers] = 0;
-        shared[kInstMembers + 1] = *tag;
-    }
-    __syncthreads();
-    *tag = shared[kInstMembers + 1];
-    double s = 0.0;
-    const uint32_t mine = t / kChunks;
-    if (t % kChunks == 0 && mine < members)
-    {
-        double theirs[1] = {0.0};
-        const bool there = team_get<1>(words, kInstMembers, mine, *tag, g.max_polls, theirs);
-        s = theirs[0];
-        shared[mine] = !there;
-        if (!there)
-            shared[kInstMembers] = 1; // every writer stores the same
-    }
-    __syncthreads();
-    if (shared[kInstMembers])
-        for (uint32_t m = 0; m < members; ++m)
-            if (shared[m]) // uniform
-            {
-                const double r = recompute(m);
-                if (t == m * kChunks)
-                    s = r;
-            }
-    return s;
-}
+    double waves[2][TEAM / kWaveSize]; // of each exchange
+    double again[TEAM / kWaveSize];    // of a member whose result is worked out here
+    double totals[2][kWavesPerBlock];
+    unsigned long long late[2][kWavesPerBlock]; // lanes whose result was not there in time
+};
 
 // f(k, bytes) for the vectors of a thread in its chunk of a member, in the order of the staged reductions; they
 // lie where inst_at says (one offset in a vector register for all of them).
@@ -100,62 +68,114 @@ __device__ __forceinline__ T* inst_at(T* sample, int k, uint32_t bytes)
     return reinterpret_cast<T*>(reinterpret_cast<Byte*>(sample + k * kBlockSize * VEC) + bytes);
 }
 
-// The maximum over the workgroup.
-template <int TEAM>
-__device__ __forceinline__ double inst_maximum(double mine, double* lds)
+// What a member exchanges, in every lane: the maximum over the workgroup, or the sum of its chunk, as block_sum adds, or of
+// four.  waves: a double for each wave.
+template <int TEAM, bool SUM>
+__device__ __forceinline__ double inst_partial(double mine, double* waves)
 {
-    mine = wave_max(mine);
-    __syncthreads(); // lds may still be read
+    constexpr int kWaves = TEAM / kWaveSize, kChunks = TEAM / kBlockSize;
+    mine = SUM ? wave_sum(mine) : wave_max(mine);
     if (threadIdx.x % kWaveSize == 0)
-        lds[threadIdx.x / kWaveSize] = mine;
+        waves[threadIdx.x / kWaveSize] = mine;
     __syncthreads();
-    double r = lds[0];
-#pragma unroll
-    for (int w = 1; w < TEAM / kWaveSize; ++w)
-        r = lds[w] > r ? lds[w] : r;
-    return r;
-}
-
-// The sum that a member exchanges: of its chunk, as block_sum adds, or of four.
-template <int TEAM>
-__device__ __forceinline__ double inst_partial(double mine, double* lds)
-{
-    constexpr int kChunks = TEAM / kBlockSize;
-    mine = wave_sum(mine);
-    __syncthreads();
-    if (threadIdx.x % kWaveSize == 0)
-        lds[threadIdx.x / kWaveSize] = mine;
-    __syncthreads();
-    double p[kChunks];
-#pragma unroll
-    for (int q = 0; q < kChunks; ++q)
+    if constexpr (SUM)
     {
-        p[q] = lds[q * kWavesPerBlock];
+        const double* const w = waves + threadIdx.x % kChunks * kWavesPerBlock;
+        double p = w[0];
 #pragma unroll
-        for (int w = 1; w < kWavesPerBlock; ++w)
-            p[q] += lds[q * kWavesPerBlock + w];
-        p[q] = 0.0 + p[q]; // as inst_combine_sum starts
+        for (int i = 1; i < kWavesPerBlock; ++i)
+            p += w[i];
+        p = 0.0 + p; // as inst_combine_sum starts
+        if constexpr (kChunks == 4)
+        {
+            p += dpp_move<kDppQuadSwap1>(p);
+            p += dpp_move<kDppQuadSwap2>(p);
+        }
+        return p;
     }
-    if constexpr (kChunks == 1)
-        return p[0];
     else
-        return (p[0] + p[1]) + (p[2] + p[3]);
+    {
+        const auto larger = [](double a, double b) { return a > b ? a : b; };
+        double r = waves[threadIdx.x % kWaves];
+        r = larger(r, dpp_move<kDppQuadSwap1>(r));
+        r = larger(r, dpp_move<kDppQuadSwap2>(r));
+        if constexpr (kWaves == 16)
+        {
+            r = larger(r, dpp_move<kDppRowRor4>(r));
+            r = larger(r, dpp_move<kDppRowRor8>(r));
+        }
+        return r;
+    }
 }
 
-// The sum of what the members have exchanged.
-template <int TEAM>
-__device__ __forceinline__ double inst_total(double mine, double* lds)
+// The result of all members, given this member's own and the tag that it made of the counter.  Lanes 0, 1, ... of the first wave
+// look after a member each, or, members of four chunks, lanes 0, 4, ... of the first four: where a thread of the
+// staged combination holds the first of the partials that member has added up, so that the steps left of its tree
+// are wave_sum_from's.  recompute(member): what a thread adds to it, called by the whole workgroup.
+// (With the first thread storing, a reduction through LDS before and behind the look and two barriers each, N 13, 44,880
+// elements, forward + backward, took 11.6 us, so 10.2; N 12, 66,912 12.5 and 10.9.)
+template <int TEAM, int WHICH, bool SUM, typename F>
+__device__ __forceinline__ double inst_exchange(double part, const InstTeam& g, uint32_t member,
+                                                unsigned long long* state, uint32_t tag, InstShared<TEAM>& shared,
+                                                const F& recompute)
 {
-    mine = wave_sum_from(mine, TEAM / kBlockSize);
-    __syncthreads();
-    if (threadIdx.x % kWaveSize == 0)
-        lds[threadIdx.x / kWaveSize] = mine;
-    __syncthreads();
-    double r = lds[0];
+    constexpr uint32_t kChunks = TEAM / kBlockSize;
+    const uint32_t members = g.members.divisor, t = threadIdx.x, mine = t / kChunks;
+    const uint32_t lane = t % kWaveSize, wave = t / kWaveSize;
+    const bool reads = t % kChunks == 0 && mine < members;
+    unsigned long long* const words = state + kCounterWords + WHICH * 2 * kInstMembers;
+    const auto leave_wave = [&](double s) {
+        s = SUM ? wave_sum_from(s, kChunks) : wave_max(s);
+        if (lane == 0)
+            shared.totals[WHICH][wave] = s;
+    };
+    const auto total = [&] {
+        double r = shared.totals[WHICH][0];
 #pragma unroll
-    for (int w = 1; w < kWavesPerBlock; ++w)
-        r += lds[w];
-    return r;
+        for (uint32_t w = 1; w < kChunks; ++w)
+        {
+            const double x = shared.totals[WHICH][w];
+            r = SUM ? r + x : x > r ? x : r;
+        }
+        return r;
+    };
+    if (t == 0)
+    {
+        const double own[1] = {part};
+        team_put<1>(words, kInstMembers, member, tag, own);
+    }
+    double s[1] = {0.0}; // less than any maximum
+    if (wave < kChunks) // uniform
+    {
+        const bool there = !reads || team_get<1>(words, kInstMembers, mine, tag, g.max_polls, s);
+        if (!there)
+            s[0] = 0.0;
+        const unsigned long long late = __ballot(!there);
+        if (lane == 0)
+            shared.late[WHICH][wave] = late;
+        leave_wave(s[0]);
+    }
+    __syncthreads();
+    unsigned long long late = shared.late[WHICH][0];
+#pragma unroll
+    for (uint32_t w = 1; w < kChunks; ++w)
+        late |= shared.late[WHICH][w];
+    if (late) // uniform
+    {
+        for (uint32_t m = 0; m < members; ++m)
+        {
+            if (!(shared.late[WHICH][m * kChunks / kWaveSize] >> m * kChunks % kWaveSize & 1)) // uniform
+                continue;
+            const double r = inst_partial<TEAM, SUM>(recompute(m), shared.again);
+            if (t == m * kChunks)
+                s[0] = r;
+            __syncthreads(); // shared.again is written again
+        }
+        if (wave < kChunks)
+            leave_wave(s[0]);
+        __syncthreads();
+    }
+    return total();
 }
 
 template <typename T, int VEC>
@@ -185,49 +205,56 @@ __device__ __forceinline__ void add_products(double& acc, const Pack<T, VEC>& y,
         acc = __builtin_fma(static_cast<double>(y[j]), static_cast<double>(dy[j]), acc);
 }
 
+// Waves of a SIMD: two members of 1024 threads a CU, for which a thread may have 64 registers, where it holds up to 32 (HELD
+// elements; doubles in single elements spill then).  Forward + backward going round three sets of tensors, 67 registers and one
+// member a CU -> this: N 11, 527,040 floats, 47.0 -> 37.5 us, N 16, 1,225,728 109 -> 95, N 23, 632,400 doubles 157 -> 135.
+template <typename T, int TEAM, int HELD, bool SINGLE>
+constexpr int inst_waves()
+{
+    return TEAM == kBlockSize ? 2 : HELD * sizeof(T) <= 4 * 32 && !(sizeof(T) == 8 && SINGLE) ? 8 : 4;
+}
+
 // VEC elements a vector, up to V vectors a thread.
 template <typename T, int TEAM, int VEC, int V>
-__global__ __launch_bounds__(TEAM, TEAM == kBlockSize ? 2 : 4) void softmax_inst_team_forward_kernel(
+__global__ __launch_bounds__(TEAM, (inst_waves<T, TEAM, VEC * V, VEC == 1>())) void softmax_inst_team_forward_kernel(
     const T* __restrict__ x, T* __restrict__ y, T* __restrict__ sample_max, T* __restrict__ sample_exp,
     const InstTeam g, T min_output)
 {
     using P = Pack<T, VEC>;
-    __shared__ double lds[TEAM / kWaveSize];
-    __shared__ uint32_t shared[kInstMembers + 2];
+    __shared__ InstShared<TEAM> shared;
     const uint32_t n = fastdiv(blockIdx.x, g.members);
     const uint32_t member = blockIdx.x - n * g.members.divisor;
     unsigned long long* const state = g.states + static_cast<size_t>(n) * kInstStateWords;
-    uint32_t tag = threadIdx.x == 0 ? team_tag(state) : 0;
+    uint32_t tag = team_tag(state);
     const T* const xp = x + static_cast<size_t>(n) * g.sample_size;
     P v[V];
     inst_chunk<T, TEAM, VEC, V>(g, member, [&](int k, uint32_t i) { v[k] = P::load(inst_at<VEC>(xp, k, i)); });
 
     T mx = Limits<T>::min_normal;
     inst_chunk<T, TEAM, VEC, V>(g, member, [&](int k, uint32_t) { add_max<T, VEC>(mx, v[k]); });
-    double s = inst_exchange<TEAM, 0>(
-        inst_maximum<TEAM>(static_cast<double>(mx), lds), g, member, state, &tag, shared, [&](uint32_t m) {
+    asm volatile("" : "+v"(tag)); // every wave has it before any stores: beyond the barrier others may leave
+    const T shift = static_cast<T>(inst_exchange<TEAM, 0, false>(
+        inst_partial<TEAM, false>(static_cast<double>(mx), shared.waves[0]), g, member, state, tag, shared, [&](uint32_t m) {
             T r = Limits<T>::min_normal;
             inst_chunk<T, TEAM, VEC, V>(g, m, [&](int k, uint32_t i) {
                 add_max<T, VEC>(r, P::load(inst_at<VEC>(xp, k, i)));
             });
-            return inst_maximum<TEAM>(static_cast<double>(r), lds);
-        });
-    const double least = static_cast<double>(Limits<T>::min_normal); // what threads without a partial hold is less
-    const T shift = static_cast<T>(inst_maximum<TEAM>(s > least ? s : least, lds));
+            return static_cast<double>(r);
+        }));
 
     double acc = 0.0;
     inst_chunk<T, TEAM, VEC, V>(g, member, [&](int k, uint32_t) { add_exponentials<T, VEC>(acc, v[k], shift); });
-    s = inst_exchange<TEAM, 1>(inst_partial<TEAM>(acc, lds), g, member, state, &tag, shared, [&](uint32_t m) {
-        double r = 0.0;
-        inst_chunk<T, TEAM, VEC, V>(g, m, [&](int k, uint32_t i) {
-            P w = P::load(inst_at<VEC>(xp, k, i));
-            add_exponentials<T, VEC>(r, w, shift);
-        });
-        return inst_partial<TEAM>(r, lds);
-    });
+    const T sum = static_cast<T>(inst_exchange<TEAM, 1, true>(
+        inst_partial<TEAM, true>(acc, shared.waves[1]), g, member, state, tag, shared, [&](uint32_t m) {
+            double r = 0.0;
+            inst_chunk<T, TEAM, VEC, V>(g, m, [&](int k, uint32_t i) {
+                P w = P::load(inst_at<VEC>(xp, k, i));
+                add_exponentials<T, VEC>(r, w, shift);
+            });
+            return r;
+        }));
     if (threadIdx.x == 0)
         team_leave(state);
-    const T sum = static_cast<T>(inst_total<TEAM>(s, lds));
     if (member == 0 && threadIdx.x == 0)
     {
         sample_max[n] = shift;
@@ -246,17 +273,16 @@ __global__ __launch_bounds__(TEAM, TEAM == kBlockSize ? 2 : 4) void softmax_inst
 }
 
 template <typename T, int TEAM, int VEC, int V>
-__global__ __launch_bounds__(TEAM, TEAM == kBlockSize ? 2 : 4) void softmax_inst_team_backward_kernel(
+__global__ __launch_bounds__(TEAM, (inst_waves<T, TEAM, 2 * VEC * V, VEC == 1>())) void softmax_inst_team_backward_kernel(
     const T* __restrict__ y, const T* __restrict__ dy, T* __restrict__ dx, T* __restrict__ sample_dp,
     const InstTeam g, T min_output)
 {
     using P = Pack<T, VEC>;
-    __shared__ double lds[TEAM / kWaveSize];
-    __shared__ uint32_t shared[kInstMembers + 2];
+    __shared__ InstShared<TEAM> shared;
     const uint32_t n = fastdiv(blockIdx.x, g.members);
     const uint32_t member = blockIdx.x - n * g.members.divisor;
     unsigned long long* const state = g.states + static_cast<size_t>(n) * kInstStateWords;
-    uint32_t tag = threadIdx.x == 0 ? team_tag(state) : 0;
+    uint32_t tag = team_tag(state);
     const T* const yp = y + static_cast<size_t>(n) * g.sample_size;
     const T* const dp = dy + static_cast<size_t>(n) * g.sample_size;
     P v[V], d[V];
@@ -266,16 +292,17 @@ __global__ __launch_bounds__(TEAM, TEAM == kBlockSize ? 2 : 4) void softmax_inst
     });
     double acc = 0.0;
     inst_chunk<T, TEAM, VEC, V>(g, member, [&](int k, uint32_t) { add_products<T, VEC>(acc, v[k], d[k]); });
-    const double s = inst_exchange<TEAM, 0>(inst_partial<TEAM>(acc, lds), g, member, state, &tag, shared, [&](uint32_t m) {
-        double r = 0.0;
-        inst_chunk<T, TEAM, VEC, V>(g, m, [&](int k, uint32_t i) {
-            add_products<T, VEC>(r, P::load(inst_at<VEC>(yp, k, i)), P::load(inst_at<VEC>(dp, k, i)));
-        });
-        return inst_partial<TEAM>(r, lds);
-    });
+    asm volatile("" : "+v"(tag)); // every wave has it before any stores: beyond the barrier others may leave
+    const T dot = static_cast<T>(inst_exchange<TEAM, 0, true>(
+        inst_partial<TEAM, true>(acc, shared.waves[0]), g, member, state, tag, shared, [&](uint32_t m) {
+            double r = 0.0;
+            inst_chunk<T, TEAM, VEC, V>(g, m, [&](int k, uint32_t i) {
+                add_products<T, VEC>(r, P::load(inst_at<VEC>(yp, k, i)), P::load(inst_at<VEC>(dp, k, i)));
+            });
+            return r;
+        }));
     if (threadIdx.x == 0)
         team_leave(state);
-    const T dot = static_cast<T>(inst_total<TEAM>(s, lds));
     if (member == 0 && threadIdx.x == 0)
         sample_dp[n] = dot;
     T* const op = dx + static_cast<size_t>(n) * g.sample_size;
