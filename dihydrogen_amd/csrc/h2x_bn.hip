@@ -2995,13 +2995,31 @@ bool team_variant(const G& g, const OnceBackward<T>* a, bool stream, bool forced
     return true;
 }
 
-// Channels that one workgroup of 1024 threads would hold, but few: the teams first
-// (forward + backward, N 8, C 64, 56 x 56 13.3 us, by workgroups 15.0; N 1, C 32, 32^3 13.1 and 16.8; N 1, C 96,
-// 32^3 15.3 and 17.5; but N 8, C 128, 56 x 56 16.6 and 15.6; half the size, N 4, C 64, 56 x 56, 13.0 and 11.0).
+// Channels that one workgroup of 1024 threads would hold, for teams first: where such workgroups leave much of the chip idle, or
+// a CU holds one of them, which loads, adds and stores with nothing beside it.  Forward + backward in us, by workgroups and by
+// teams, going round three sets of tensors (330 calls):
+//   few channels (N 8, C 64, 56 x 56 14.4 and 11.8; C 16 13.5 and 10.9; with 4096 vectors or fewer equal);
+//   more than 8192 vectors, with 16 or 20 a thread: 15 % less on average, 2 % more at worst, but for channels that fill one round
+//   of the chip (C 128, N 16 27.9 and 23.2; N 6, C 283, 90 x 99 77.7 and 54.9; N 1, C 682, 203 x 188, cleared 118 and 96; N 6, C 174, 5 %
+//   more);
+//   up to 8192, whose backward workgroups a CU holds one of: with a halo, or dense, where channels leave half of a second round
+//   empty, or an eighth of more rounds (N 53, C 1185, 21 x 22 with a halo 173 and 158; C 622, 6800 vectors 4 % less; C 401 and 506,
+//   3 and 9 % more, C 1022 7); cleared, unless they nearly fill the rounds (N 7, C 328, 15 x 15 x 12 49 and 37; C 202 and 993, 6 % more).
+// The state of more than 2048 channels would be as large as many a tensor.
 template <typename G>
 bool teams_first(const G& g)
 {
-    return g.vectors > 4096 && g.num_channels <= kOnceManyChannels;
+    constexpr uint32_t kMostChannels = 2048;
+    if (g.vectors <= 4096 || g.num_channels > kMostChannels)
+        return false;
+    if (g.num_channels <= kOnceManyChannels || g.vectors > 8192)
+        return true;
+    const uint32_t known = compute_units(), cus = known ? known : 256;
+    const uint32_t rounds = (g.num_channels + cus - 1) / cus;
+    const uint32_t filled = g.num_channels * 16 / (rounds * cus); // sixteenths of the rounds
+    if constexpr (G::kClears)
+        return rounds == 1 ? filled <= 10 : filled < 15;
+    return rounds > 1 && filled < (rounds == 2 ? 12 : 14);
 }
 
 // A team keeps within half of the chip.

@@ -12,8 +12,9 @@
 // (one set of tensors over and over: up to 256 MB of it stay in the memory-side cache)
 //
 // A channel is as large as the registers of one CU allow: 512 KB, of which the
-// largest variants hold 320 KB forward, 256 KB and 128 KB of LDS backward.  Larger ones, and few, are for
-// teams of workgroups (h2x_bn_team.hpp).
+// largest variants hold 320 KB forward, 256 KB and 128 KB of LDS backward.  Larger ones, few, and those that would leave
+// CUs idle or alone with one workgroup are for teams of workgroups (h2x_bn_team.hpp), where the caller has a state for them and
+// outputs lie apart from inputs.
 //
 // The elements are those of the other kernels: rows in vectors of 16 bytes that may
 // start on any element, the last vector of a row that is no whole number of vectors
