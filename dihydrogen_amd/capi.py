@@ -327,8 +327,9 @@ _calls = None
 
 def calls():
     """The native module whose functions call the library (csrc/h2x_python.cpp): the entry points
-    the layers call once per step, under their own names, taking torch tensors, addresses or None
-    for pointers and returning the status.  Raises if it is absent."""
+    the layers call once per step, under their own names, taking torch tensors, local tensors (the
+    address of the first interior element), addresses or None for pointers and returning the status.
+    Raises if it is absent."""
     global _calls
     if _calls is None:
         load()
@@ -337,6 +338,8 @@ def calls():
         except ImportError as e:
             raise H2XError("_h2xcall.so is missing: build it with `make -C dihydrogen_amd/csrc` "
                            "(or __graft_entry__.build()); there is no fallback path") from e
+        from .tensor import Tensor
+        _h2xcall.tensor_type(Tensor)  # for a pointer: the address of its first interior element
         _calls = _h2xcall
     return _calls
 

@@ -186,11 +186,11 @@ class BatchNormalization:
         ns = lx.samples if lx.active else 0
         if lx.dense:
             capi.check(self._calls.h2x_bn_channel_sums_and_sqsums(
-                lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, input.get_base_ptr(), mean, var,
+                lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, input, mean, var,
                 self._ws(lx.channels), _stream_handle(self.stream)), "channel_sums_and_sqsums")
         else:  # halo on an inner spatial dimension: the generic path of batchnorm.cu:232-248
             capi.check(self._calls.h2x_bn_channel_sums_and_sqsums_strided(
-                lx.dtype, ns, _tensor_geometry(lx, ns), input.get_base_ptr(), mean, var,
+                lx.dtype, ns, _tensor_geometry(lx, ns), input, mean, var,
                 self._ws(lx.channels), _stream_handle(self.stream)), "channel_sums_and_sqsums (strided)")
         return 0
 
@@ -218,14 +218,14 @@ class BatchNormalization:
                 output.get_buffer(), self.epsilon, _stream_handle(self.stream)), "batch_normalization (clearing)")
         elif lx.dense and ly.dense:
             status = self._calls.h2x_bn_batch_normalization(
-                lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ly.spatial_real, input.get_base_ptr(), mean,
-                var, scale, bias, output.get_base_ptr(), self.epsilon, _stream_handle(self.stream))
+                lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ly.spatial_real, input, mean,
+                var, scale, bias, output, self.epsilon, _stream_handle(self.stream))
             if status:
                 capi.check(status, "batch_normalization")
         else:
             capi.check(self._calls.h2x_bn_batch_normalization_strided(
-                lx.dtype, ns, _tensor_geometry(lx, ns), _tensor_geometry(ly, ns), input.get_base_ptr(), mean, var,
-                scale, bias, output.get_base_ptr(), self.epsilon, _stream_handle(self.stream)),
+                lx.dtype, ns, _tensor_geometry(lx, ns), _tensor_geometry(ly, ns), input, mean, var,
+                scale, bias, output, self.epsilon, _stream_handle(self.stream)),
                 "batch_normalization (strided)")
 
     def forward_stage2(self, input: Tensor, mean, var, running_mean, running_var, scale, bias,
@@ -271,13 +271,13 @@ class BatchNormalization:
             per_sum = self._elements_per_sum(lx)
             if lx.extents != ly.extents and _pair_in_order(lx, ly):
                 capi.check(self._calls.h2x_bn_forward_local(
-                    lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ly.spatial_real, input.get_base_ptr(),
+                    lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ly.spatial_real, input,
                     scale, bias, per_sum, self.decay, self.epsilon, mean, var, running_mean, running_var,
-                    output.get_base_ptr(), self._ws(lx.channels), _stream_handle(self.stream)), "bn forward (local)")
+                    output, self._ws(lx.channels), _stream_handle(self.stream)), "bn forward (local)")
                 return 0
             status = self._calls.h2x_bn_forward_once(
-                lx.dtype, ns, lx.geometry_address, _tensor_geometry(ly, ns), input.get_base_ptr(), scale, bias, per_sum,
-                self.decay, self.epsilon, mean, var, running_mean, running_var, output.get_base_ptr(),
+                lx.dtype, ns, lx.geometry_address, _tensor_geometry(ly, ns), input, scale, bias, per_sum,
+                self.decay, self.epsilon, mean, var, running_mean, running_var, output,
                 self._ws(lx.channels), self._team_state(lx, False), _stream_handle(self.stream))
             if status:
                 capi.check(status, "bn forward (local)")
@@ -297,12 +297,12 @@ class BatchNormalization:
                 self._ws(lx.channels), _stream_handle(self.stream))
         if lx.dense and ld.dense:
             capi.check(self._calls.h2x_bn_backprop1(
-                lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ld.spatial_real, input.get_base_ptr(),
-                d_output.get_base_ptr(), *tail), "backprop1")
+                lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ld.spatial_real, input,
+                d_output, *tail), "backprop1")
         else:
             capi.check(self._calls.h2x_bn_backprop1_strided(
-                lx.dtype, ns, _tensor_geometry(lx, ns), _tensor_geometry(ld, ns), input.get_base_ptr(),
-                d_output.get_base_ptr(), *tail), "backprop1 (strided)")
+                lx.dtype, ns, _tensor_geometry(lx, ns), _tensor_geometry(ld, ns), input,
+                d_output, *tail), "backprop1 (strided)")
         return 0
 
     def backward_allreduce(self, scale_gradient, bias_gradient, mean_gradient, var_gradient,
@@ -319,8 +319,8 @@ class BatchNormalization:
                         var_gradient, d_input: Tensor) -> int:
         lx, ld, li = _dense_layout(input), _dense_layout(d_output), _dense_layout(d_input)
         ns = self.num_current_samples
-        tail = (input.get_base_ptr(), d_output.get_base_ptr(), mean, var, scale, mean_gradient, var_gradient,
-                d_input.get_base_ptr(), self.epsilon, _stream_handle(self.stream))
+        tail = (input, d_output, mean, var, scale, mean_gradient, var_gradient,
+                d_input, self.epsilon, _stream_handle(self.stream))
         if self.clear_output_halo and ns == lx.samples and _share_a_haloed_geometry(lx, ld, li):
             capi.check(self._calls.h2x_bn_backprop2_clearing(
                 lx.dtype, self._num_per_sum(input), li.haloed_geometry_address, input.get_buffer(),
@@ -360,14 +360,14 @@ class BatchNormalization:
             if (lx.extents != ld.extents or lx.extents != li.extents) and _pair_in_order(lx, ld, li):
                 capi.check(self._calls.h2x_bn_backward_local(
                     lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ld.spatial_real, li.spatial_real, per_sum,
-                    input.get_base_ptr(), d_output.get_base_ptr(), mean, var, scale, scale_gradient, bias_gradient,
-                    mean_gradient, var_gradient, d_input.get_base_ptr(), self.epsilon, self._ws(lx.channels),
+                    input, d_output, mean, var, scale, scale_gradient, bias_gradient,
+                    mean_gradient, var_gradient, d_input, self.epsilon, self._ws(lx.channels),
                     _stream_handle(self.stream)), "bn backward (local)")
                 return 0
             status = self._calls.h2x_bn_backward_once(
                 lx.dtype, ns, per_sum, lx.geometry_address, _tensor_geometry(ld, ns), _tensor_geometry(li, ns),
-                input.get_base_ptr(), d_output.get_base_ptr(), mean, var, scale, scale_gradient, bias_gradient,
-                mean_gradient, var_gradient, d_input.get_base_ptr(), self.epsilon, self._ws(lx.channels),
+                input, d_output, mean, var, scale, scale_gradient, bias_gradient,
+                mean_gradient, var_gradient, d_input, self.epsilon, self._ws(lx.channels),
                 self._team_state(lx, False), _stream_handle(self.stream))
             if status:
                 capi.check(status, "bn backward (local)")
@@ -454,9 +454,12 @@ class Softmax:
         self.mode = SoftmaxMode.CHANNEL
         self._lib = capi.load()
         self._calls = capi.calls()
+        # buffers and what they hold: calls to ask a tensor would be a tenth of a small call
         self._ws: Optional[torch.Tensor] = None
         self._scalars: Optional[torch.Tensor] = None
         self._state: Optional[torch.Tensor] = None
+        self._ws_bytes = self._scalars_count = self._state_bytes = 0
+        self._scalars_type: Optional[torch.dtype] = None
 
     def setup(self, input: Tensor, mode: SoftmaxMode) -> None:
         self.mode = mode
@@ -468,25 +471,27 @@ class Softmax:
             raise NotImplementedError("softmax assumes a dense local tensor")  # softmax.cu:562-563
         return l
 
-    def _workspace(self, n: int) -> torch.Tensor:
-        need = self._calls.h2x_softmax_instance_workspace_bytes(n)
-        if self._ws is None or self._ws.numel() < need:
-            self._ws = _buffer_of(self.stream, need, torch.uint8)
+    def _workspace(self, l: Layout) -> torch.Tensor:
+        need = l.instance_workspace_bytes
+        if self._ws_bytes < need:
+            self._ws, self._ws_bytes = _buffer_of(self.stream, need, torch.uint8), need
         return self._ws
 
     def _team_state(self, l: Layout) -> Optional[torch.Tensor]:
         """Where the workgroups that share a sample exchange its partial results; None where no workgroups do."""
         need = l.instance_state_bytes
-        if need and (self._state is None or self._state.numel() < need):
-            self._state = _buffer_of(self.stream, need, torch.uint8, zero=True)
-        return self._state if need else None
+        if need == 0:
+            return None
+        if self._state_bytes < need:
+            self._state, self._state_bytes = _buffer_of(self.stream, need, torch.uint8, zero=True), need
+        return self._state
 
     def _sample_scalars(self, t: Tensor, count: int) -> torch.Tensor:
         """`count` scalars of t's type that nobody reads after the call: kept like the workspace."""
-        b = self._scalars
-        if b is None or b.dtype != t.dtype or b.numel() < count:
-            b = self._scalars = _buffer_of(self.stream, count, t.dtype)
-        return b
+        if self._scalars_count < count or self._scalars_type is not t.dtype:
+            self._scalars = _buffer_of(self.stream, count, t.dtype)
+            self._scalars_count, self._scalars_type = count, t.dtype
+        return self._scalars
 
     def forward(self, x: Tensor, y: Tensor) -> int:
         l = self._geometry(x)
@@ -496,29 +501,29 @@ class Softmax:
         st = _stream_handle(self.stream)
         if self.mode == SoftmaxMode.CHANNEL:
             status = self._calls.h2x_softmax_channel_forward(
-                l.dtype, n, l.channels, l.spatial, x.get_base_ptr(), y.get_base_ptr(), st)
+                l.dtype, n, l.channels, l.spatial, x, y, st)
             if status:
                 capi.check(status, "softmax forward")
             return 0
         # instance mode: softmax.cu:723-746
-        calls, dt, size, ws = self._calls, l.dtype, l.channels * l.spatial, self._workspace(n)
+        calls, dt, size, ws = self._calls, l.dtype, l.channels * l.spatial, self._workspace(l)
         if self.allreduce is None:
             # every sample is whole on this rank: the stages need not be separate calls
             scalars = self._sample_scalars(x, 2 * n).data_ptr()
             status = calls.h2x_softmax_instance_forward_once(
-                dt, n, size, x.get_base_ptr(), y.get_base_ptr(), scalars,
-                scalars + n * self._scalars.element_size(), ws, self._team_state(l), -1, st)
+                dt, n, size, x, y, scalars,
+                scalars + n * x.dtype.itemsize, ws, self._team_state(l), -1, st)
             if status:
                 capi.check(status, "softmax instance forward")
             return 0
         smax, sexp = (_buffer_of(self.stream, n, x.dtype, x.device) for _ in range(2))
-        capi.check(calls.h2x_softmax_instance_max(dt, n, size, x.get_base_ptr(), smax, ws, st),
+        capi.check(calls.h2x_softmax_instance_max(dt, n, size, x, smax, ws, st),
                    "softmax instance max")
         self.allreduce(smax, True)
-        capi.check(calls.h2x_softmax_instance_exp(dt, n, size, x.get_base_ptr(), smax, y.get_base_ptr(), sexp, ws,
+        capi.check(calls.h2x_softmax_instance_exp(dt, n, size, x, smax, y, sexp, ws,
                                                   st), "softmax instance exp")
         self.allreduce(sexp, False)
-        capi.check(calls.h2x_softmax_instance_normalize(dt, n, size, sexp, y.get_base_ptr(), st),
+        capi.check(calls.h2x_softmax_instance_normalize(dt, n, size, sexp, y, st),
                    "softmax instance normalize")
         return 0
 
@@ -530,25 +535,25 @@ class Softmax:
         st = _stream_handle(self.stream)
         if self.mode == SoftmaxMode.CHANNEL:
             status = self._calls.h2x_softmax_channel_backward(
-                dt, n, l.channels, l.spatial, y.get_base_ptr(), dy.get_base_ptr(), dx.get_base_ptr(), st)
+                dt, n, l.channels, l.spatial, y, dy, dx, st)
             if status:
                 capi.check(status, "softmax backward")
             return 0
         # instance mode: softmax.cu:770-783
-        calls, size, ws = self._calls, l.channels * l.spatial, self._workspace(n)
+        calls, size, ws = self._calls, l.channels * l.spatial, self._workspace(l)
         if self.allreduce is None:
             status = calls.h2x_softmax_instance_backward_once(
-                dt, n, size, y.get_base_ptr(), dy.get_base_ptr(), dx.get_base_ptr(), self._sample_scalars(y, n), ws,
+                dt, n, size, y, dy, dx, self._sample_scalars(y, n), ws,
                 self._team_state(l), -1, st)
             if status:
                 capi.check(status, "softmax instance backward")
             return 0
         sdp = _buffer_of(self.stream, n, y.dtype, y.device)
-        capi.check(calls.h2x_softmax_instance_dot(dt, n, size, y.get_base_ptr(), dy.get_base_ptr(), sdp, ws, st),
+        capi.check(calls.h2x_softmax_instance_dot(dt, n, size, y, dy, sdp, ws, st),
                    "softmax instance dot")
         self.allreduce(sdp, False)
-        capi.check(calls.h2x_softmax_instance_gradient(dt, n, size, y.get_base_ptr(), dy.get_base_ptr(), sdp,
-                                                       dx.get_base_ptr(), st), "softmax instance gradient")
+        capi.check(calls.h2x_softmax_instance_gradient(dt, n, size, y, dy, sdp,
+                                                       dx, st), "softmax instance gradient")
         return 0
 
 
@@ -708,10 +713,9 @@ class HaloExchangeVirtual:
         ranks that differ in their halo widths or type, an empty rank, a halo on channels or
         samples, or next to a neighbour fewer than `cells` halo widths of interior (an exchange
         needs one: its boundary strips are no halo; a reverse one two: they do not overlap)."""
-        addresses = self._addresses()
         kept = self._grid_of
-        if kept is None or kept[0] != addresses:
-            kept = self._grid_of = (addresses, *self._make_grid())
+        if kept is None or not self._calls.same_buffers(kept[0], self.tensors):
+            kept = self._grid_of = (self._addresses(), *self._make_grid())
         return kept[1] if kept[2] >= cells else 0
 
     def _make_grid(self):
@@ -1066,9 +1070,9 @@ class TensorShufflerVirtual:
     def _direct_arguments(self):
         """Pointer arrays of the direct launches, or None where a source shares memory with a
         destination.  They depend only on the tensors' addresses: kept until one is reallocated."""
-        addresses = [t.data.data_ptr() for t in self.src] + [t.data.data_ptr() for t in self.dst]
         kept = self._direct
-        if kept is None or kept[0] != addresses:
+        if kept is None or not self._calls.same_buffers(kept[0], self.src, self.dst):
+            addresses = tuple([t.data.data_ptr() for t in self.src] + [t.data.data_ptr() for t in self.dst])
             ends = [a + t.data.numel() * self.elem_size for a, t in zip(addresses, self.src + self.dst)]
             n = self.num_ranks
             shared = any(addresses[i] < ends[j] and addresses[j] < ends[i] for i in range(n) for j in range(n, 2 * n))

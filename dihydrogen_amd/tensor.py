@@ -201,6 +201,10 @@ class Layout:
         return capi.calls().h2x_softmax_instance_state_needed(self.dtype, self.samples, self.channels * self.spatial)
 
     @_once
+    def instance_workspace_bytes(self) -> int:
+        return capi.calls().h2x_softmax_instance_workspace_bytes(self.samples)
+
+    @_once
     def clearing_team_state_bytes(self) -> int:
         """The same for calls that clear their output's halo."""
         return capi.calls().h2x_bn_team_state_needed_clearing(self.dtype, self.haloed_geometry_address)

@@ -1,0 +1,58 @@
+"""What the native calls take for a pointer, and how they compare the buffers of tensors."""
+import pytest
+import torch
+
+from dihydrogen_amd import capi
+from dihydrogen_amd.tensor import Distribution, LocaleVirtual, Tensor
+
+
+class Derived(Tensor):
+    """Its interior begins elsewhere: a call asks it, not its base class."""
+
+    def get_base_ptr(self):
+        return super().get_base_ptr() + 4
+
+
+def _tensor(overlap, kind=Tensor, device="cpu"):
+    dist = Distribution.make_overlapped_distribution([1, 1, 1, 1], overlap)
+    return kind([5, 4, 3, 2], LocaleVirtual(0, 1), dist, device=device).allocate()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", [Tensor, Derived])
+@pytest.mark.parametrize("overlap", [[0, 0, 0, 0], [2, 1, 0, 0]])
+def test_a_local_tensor_is_the_address_of_its_interior(kind, overlap):
+    t = _tensor(overlap, kind, "cuda")
+    t.data.copy_(torch.arange(t.data.numel()))
+    # 24 elements from there on lie in the buffer
+    got, want = torch.zeros(24, device="cuda"), torch.zeros(24, device="cuda")
+    for src, dst in ((t, got), (t.get_base_ptr(), want)):
+        assert capi.calls().h2x_softmax_channel_forward(t.h2x_dtype, 2, 3, 4, src, dst.data_ptr(), None) == 0
+    first = t.base_offset() + (kind is Derived)
+    x = t.data[first:first + 24].cpu().double().view(2, 3, 4)
+    assert torch.equal(got, want)
+    torch.testing.assert_close(got.cpu().double().view(2, 3, 4), torch.softmax(x, 1), rtol=1e-5, atol=1e-7)
+
+
+def test_what_has_no_address_is_refused():
+    t = _tensor([0, 0, 0, 0])
+    t.data = None
+    for p in (t, object(), "0"):
+        with pytest.raises(AttributeError):
+            capi.calls().h2x_softmax_channel_forward(0, 0, 0, 0, p, None, None)
+
+
+def test_buffers_are_compared_in_order_and_number():
+    same, ts = capi.calls().same_buffers, [_tensor([0, 0, 0, 0], kind) for kind in (Tensor, Derived, Tensor)]
+    at = tuple(t.get_buffer() for t in ts)
+    assert same(at, ts) and same(at, ts[:1], ts[1:]) and same((), []) and same(())
+    assert not same(at, ts[:2]) and not same(at[:2], ts) and not same(at, ts[::-1]) and not same(at, ts, ts)
+    ts[1].data = None
+    assert not same(at, ts) and same((at[0], 0, at[2]), ts)
+    ts[1].allocate()
+    assert same((at[0], ts[1].get_buffer(), at[2]), ts)
+    for bad in ((list(at), ts), (at, tuple(ts)), (("a", "b", "c"), ts)):
+        with pytest.raises(TypeError):
+            same(*bad)
+    with pytest.raises(AttributeError):
+        same((1,), [object()])
