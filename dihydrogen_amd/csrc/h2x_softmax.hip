@@ -146,15 +146,15 @@ struct WideTiles
     unsigned int samples;
 };
 
-template <int VEC>
+template <int VEC, int LANES = kWaveSize>
 __device__ __forceinline__ bool tile_pixels(const WideTiles& t, int num_channels, size_t spatial, int flat_samples,
                                             size_t* base)
 {
     const unsigned int tile = xcd_contiguous(blockIdx.x, gridDim.x);
     const unsigned int n = fastdiv(tile, t.per_sample);
     const unsigned int sample = blockIdx.y + n;
-    const size_t first = static_cast<size_t>(tile - n * t.per_sample.divisor) * kWaveSize;
-    return lane_pixels<VEC>(first + threadIdx.x % kWaveSize, num_channels, spatial, flat_samples, base, sample)
+    const size_t first = static_cast<size_t>(tile - n * t.per_sample.divisor) * LANES;
+    return lane_pixels<VEC>(first + threadIdx.x % LANES, num_channels, spatial, flat_samples, base, sample)
            && sample < t.samples;
 }
 
@@ -458,6 +458,17 @@ __device__ __forceinline__ T sum_of_waves(const T (&lds)[WAVES][N], int i)
     return t[0];
 }
 
+// The values of the lanes that serve a pixel, LANES apart, combined.
+template <int LANES, typename T, typename F>
+__device__ __forceinline__ T pixel_combine(T v, const F& f)
+{
+    if constexpr (LANES <= 32)
+        v = combine_apart<32>(v, f);
+    if constexpr (LANES <= 16)
+        v = combine_apart<16>(v, f);
+    return v;
+}
+
 // forward, up to WAVES * CPW channels, register-resident.  A workgroup serves
 // 64 * VEC neighbouring pixels; its WAVES waves share the channels (wave g takes
 // c = g, g + WAVES, ...: CPW of them at most) and keep their values in registers,
@@ -467,17 +478,23 @@ __device__ __forceinline__ T sum_of_waves(const T (&lds)[WAVES][N], int i)
 // (N 16, C 150, 128 x 128: 100 us there, 63 us with the tile in registers).  Bound by
 // memory where there are several tiles a CU, else by a wave's chain of loads,
 // exponentials and sums.
-template <typename T, int VEC, int CPW, int WAVES, bool STREAM>
+// Where there are few tiles, a pixel is for 64 / LANES lanes of a wave instead of one: a workgroup serves LANES
+// pixels, lane l of wave g the channels (g + k * WAVES) * 64 / LANES + l / LANES, the chain is that many times shorter
+// and there are as many more workgroups, for rows of 64 or 128 bytes (see launch_split_for).
+template <typename T, int VEC, int CPW, int WAVES, int LANES, bool STREAM>
 __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
     const T* __restrict__ x, T* __restrict__ y, int num_channels, size_t spatial, int flat_samples,
     const WideTiles tiles)
 {
     using P = Pack<T, VEC>;
-    __shared__ T lds[WAVES][kWaveSize * VEC];
-    const int lane = threadIdx.x % kWaveSize;
+    __shared__ T lds[WAVES][LANES * VEC];
+    constexpr int kApart = kWaveSize / LANES; // channels that a wave takes at once
+    const int lane = threadIdx.x % LANES, q = threadIdx.x % kWaveSize / LANES;
     const int g = wave_index();
     size_t base;
-    const bool active = tile_pixels<VEC>(tiles, num_channels, spatial, flat_samples, &base);
+    const bool active = tile_pixels<VEC, LANES>(tiles, num_channels, spatial, flat_samples, &base);
+    base += q * spatial;
+    const int channels = num_channels - q; // of those that start at this lane's
     const T* xp = x + base;
     T* yp = y + base;
     constexpr T kMin = Limits<T>::min_normal;
@@ -494,18 +511,22 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
     {
 #pragma unroll
         for (int k = 0; k < CPW; ++k)
-            if (g + k * WAVES < num_channels)
-                v[k] = P::template load<STREAM>(xp + static_cast<size_t>(g + k * WAVES) * spatial);
+            if ((g + k * WAVES) * kApart < channels)
+                v[k] = P::template load<STREAM>(xp + static_cast<size_t>((g + k * WAVES) * kApart) * spatial);
 #pragma unroll
         for (int k = 0; k < CPW; ++k)
-            if (g + k * WAVES < num_channels)
+            if ((g + k * WAVES) * kApart < channels)
 #pragma unroll
                 for (int j = 0; j < VEC; ++j)
                     mx[j] = v[k][j] > mx[j] ? v[k][j] : mx[j];
     }
 #pragma unroll
     for (int j = 0; j < VEC; ++j)
-        lds[g][lane * VEC + j] = mx[j];
+    {
+        mx[j] = pixel_combine<LANES>(mx[j], [](T p, T r) { return r > p ? r : p; });
+        if (q == 0)
+            lds[g][lane * VEC + j] = mx[j];
+    }
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < VEC; ++j)
@@ -518,7 +539,7 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
     {
 #pragma unroll
         for (int k = 0; k < CPW; ++k)
-            if (g + k * WAVES < num_channels)
+            if ((g + k * WAVES) * kApart < channels)
 #pragma unroll
                 for (int j = 0; j < VEC; ++j)
                 {
@@ -529,7 +550,11 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
     }
 #pragma unroll
     for (int j = 0; j < VEC; ++j)
-        lds[g][lane * VEC + j] = sum[j];
+    {
+        sum[j] = pixel_combine<LANES>(sum[j], [](T p, T r) { return p + r; });
+        if (q == 0)
+            lds[g][lane * VEC + j] = sum[j];
+    }
     __syncthreads();
     T inv[VEC];
 #pragma unroll
@@ -541,7 +566,7 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
     {
 #pragma unroll
         for (int k = 0; k < CPW; ++k)
-            if (g + k * WAVES < num_channels)
+            if ((g + k * WAVES) * kApart < channels)
             {
 #pragma unroll
                 for (int j = 0; j < VEC; ++j)
@@ -549,7 +574,7 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
                     const T r = v[k][j] * inv[j];
                     v[k][j] = r > kMin ? r : kMin;
                 }
-                P::store(yp + static_cast<size_t>(g + k * WAVES) * spatial, v[k]);
+                P::store(yp + static_cast<size_t>((g + k * WAVES) * kApart) * spatial, v[k]);
             }
     }
 }
@@ -557,15 +582,16 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
 // backward likewise: y and dy of up to WAVES * CPW channels in registers.  All of y is
 // asked for before any of dy: alternating, the wave waited more often (N 4, C 150,
 // 65 x 97 in four waves 15.9 us against 10.2).
-template <typename T, int VEC, int CPW, int WAVES, bool STREAM>
+template <typename T, int VEC, int CPW, int WAVES, int LANES, bool STREAM>
 __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
     const T* __restrict__ y, const T* __restrict__ dy, T* __restrict__ dx, int num_channels,
     size_t spatial, int flat_samples,
     const WideTiles tiles)
 {
     using P = Pack<T, VEC>;
-    __shared__ T lds[WAVES][kWaveSize * VEC];
-    const int lane = threadIdx.x % kWaveSize;
+    __shared__ T lds[WAVES][LANES * VEC];
+    constexpr int kApart = kWaveSize / LANES; // channels that a wave takes at once
+    const int lane = threadIdx.x % LANES, q = threadIdx.x % kWaveSize / LANES;
     // Of more than 256 channels in floats the index stays a lane's own: as a scalar, the addresses
     // and the tests of all those channels are scalars too, more than there are (16 waves with 24
     // channels each spill 31 of them into vector registers, with 48 153; up to 256 channels a wave
@@ -575,7 +601,9 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
     // forward pass, of half the addresses, is faster with the scalar.
     const int g = sizeof(T) == 4 && WAVES * CPW > 256 ? static_cast<int>(threadIdx.x / kWaveSize) : wave_index();
     size_t base;
-    const bool active = tile_pixels<VEC>(tiles, num_channels, spatial, flat_samples, &base);
+    const bool active = tile_pixels<VEC, LANES>(tiles, num_channels, spatial, flat_samples, &base);
+    base += q * spatial;
+    const int channels = num_channels - q; // of those that start at this lane's
     const T* yp = y + base;
     const T* gp = dy + base;
     T* op = dx + base;
@@ -590,22 +618,26 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
     {
 #pragma unroll
         for (int k = 0; k < CPW; ++k)
-            if (g + k * WAVES < num_channels)
-                yv[k] = P::load(yp + static_cast<size_t>(g + k * WAVES) * spatial);
+            if ((g + k * WAVES) * kApart < channels)
+                yv[k] = P::load(yp + static_cast<size_t>((g + k * WAVES) * kApart) * spatial);
 #pragma unroll
         for (int k = 0; k < CPW; ++k)
-            if (g + k * WAVES < num_channels)
-                gv[k] = P::template load<STREAM>(gp + static_cast<size_t>(g + k * WAVES) * spatial);
+            if ((g + k * WAVES) * kApart < channels)
+                gv[k] = P::template load<STREAM>(gp + static_cast<size_t>((g + k * WAVES) * kApart) * spatial);
 #pragma unroll
         for (int k = 0; k < CPW; ++k)
-            if (g + k * WAVES < num_channels)
+            if ((g + k * WAVES) * kApart < channels)
 #pragma unroll
                 for (int j = 0; j < VEC; ++j)
                     dp[j] = fma_t(yv[k][j], gv[k][j], dp[j]);
     }
 #pragma unroll
     for (int j = 0; j < VEC; ++j)
-        lds[g][lane * VEC + j] = dp[j];
+    {
+        dp[j] = pixel_combine<LANES>(dp[j], [](T p, T r) { return p + r; });
+        if (q == 0)
+            lds[g][lane * VEC + j] = dp[j];
+    }
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < VEC; ++j)
@@ -616,12 +648,12 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
     {
 #pragma unroll
         for (int k = 0; k < CPW; ++k)
-            if (g + k * WAVES < num_channels)
+            if ((g + k * WAVES) * kApart < channels)
             {
 #pragma unroll
                 for (int j = 0; j < VEC; ++j)
                     yv[k][j] = yv[k][j] > kMin ? yv[k][j] * (gv[k][j] - dp[j]) : T(0);
-                P::template store<STREAM>(op + static_cast<size_t>(g + k * WAVES) * spatial, yv[k]);
+                P::template store<STREAM>(op + static_cast<size_t>((g + k * WAVES) * kApart) * spatial, yv[k]);
             }
     }
 }
@@ -868,10 +900,10 @@ dim3 pixel_grid_xcd(size_t spatial, int vec, int num_samples, int flat)
 // a sample, 23.3 and 18.0; N 25, C 120, 24 x 24, 9 tiles, 14.9 and 10.9; N 29, C 338, 24 x 37, 14 tiles,
 // 43.6 and 41.4; but N 30, C 179, 43 x 43, 29 tiles, 47.3 and 48.0, N 8, C 40, 128 x 128, 128 tiles,
 // 20.1 and 21.4: samples one after another reach the memory more evenly).
-dim3 wide_grid(size_t spatial, int vec, int num_samples, int flat, WideTiles* t)
+dim3 wide_grid(size_t spatial, int lanes, int vec, int num_samples, int flat, WideTiles* t)
 {
-    const dim3 by_sample = tile_grid(spatial, kWaveSize, vec, num_samples, flat);
-    const size_t per_block = static_cast<size_t>(kWaveSize) * vec;
+    const dim3 by_sample = tile_grid(spatial, lanes, vec, num_samples, flat);
+    const size_t per_block = static_cast<size_t>(lanes) * vec;
     const size_t tiles = (spatial + per_block - 1) / per_block;
     t->samples = flat > 0 ? 1 : num_samples;
     const bool through = flat == 0 && by_sample.x * static_cast<size_t>(8) > tiles * 9;
@@ -912,48 +944,59 @@ constexpr int kManySamples = 2048;
 // (softmax_*_split_kernel) with the smallest register tile that holds them: tiles wider
 // than needed cost time, since every lane walks the whole tile under a predicate.  Eight
 // waves against four, N 4, C 150, 65 x 97: forward 10.2 and 11.7 us; N 1: 5.7 and 8.0; N 16:
-// 29.8 and 34.3.  More channels than the largest tile holds (1024 forward, 768 backward;
-// double: 512 and 384, with five words of scratch a lane; N 18, C 270, 27 x 40 backward, re-reading 40.3 us, in
+// 29.8 and 34.3.  More channels than the largest tile holds (1024 forward, 768 backward, 1024 where
+// tiles are few; double: 512, or 1024; N 18, C 270, 27 x 40 backward, re-reading 40.3 us, in
 // registers 27.9) take the re-reading kernel.
-template <int VEC, int CPW, int WAVES, typename T>
+template <int VEC, int CPW, int WAVES, int LANES = kWaveSize, bool MAY_STREAM = true, typename T>
 int launch_split(const T* x, T* y, int n, int c, size_t s, bool stream, hipStream_t st)
 {
     const int flat = VEC == 1 ? flat_samples(n, s) : 0;
     WideTiles tiles;
-    const dim3 grid = wide_grid(s, VEC, n, flat, &tiles);
-    if (stream)
-        launch(softmax_fwd_split_kernel<T, VEC, CPW, WAVES, true>, grid, WAVES * kWaveSize, st, x, y, c, s, flat,
-               tiles);
+    const dim3 grid = wide_grid(s, LANES, VEC, n, flat, &tiles);
+    if (MAY_STREAM && stream)
+        launch(softmax_fwd_split_kernel<T, VEC, CPW, WAVES, LANES, MAY_STREAM>, grid, WAVES * kWaveSize, st, x, y, c,
+               s, flat, tiles);
     else
-        launch(softmax_fwd_split_kernel<T, VEC, CPW, WAVES, false>, grid, WAVES * kWaveSize, st, x, y, c, s, flat,
-               tiles);
+        launch(softmax_fwd_split_kernel<T, VEC, CPW, WAVES, LANES, false>, grid, WAVES * kWaveSize, st, x, y, c, s,
+               flat, tiles);
     return launch_status();
 }
 
-template <int VEC, int CPW, int WAVES, typename T>
+template <int VEC, int CPW, int WAVES, int LANES = kWaveSize, bool MAY_STREAM = true, typename T>
 int launch_split(const T* y, const T* dy, T* dx, int n, int c, size_t s, bool stream, hipStream_t st)
 {
     const int flat = VEC == 1 ? flat_samples(n, s) : 0;
     WideTiles tiles;
-    const dim3 grid = wide_grid(s, VEC, n, flat, &tiles);
-    if (stream)
-        launch(softmax_bwd_split_kernel<T, VEC, CPW, WAVES, true>, grid, WAVES * kWaveSize, st, y, dy, dx, c, s,
+    const dim3 grid = wide_grid(s, LANES, VEC, n, flat, &tiles);
+    if (MAY_STREAM && stream)
+        launch(softmax_bwd_split_kernel<T, VEC, CPW, WAVES, LANES, MAY_STREAM>, grid, WAVES * kWaveSize, st, y, dy, dx, c, s,
                flat, tiles);
     else
-        launch(softmax_bwd_split_kernel<T, VEC, CPW, WAVES, false>, grid, WAVES * kWaveSize, st, y, dy, dx, c, s,
+        launch(softmax_bwd_split_kernel<T, VEC, CPW, WAVES, LANES, false>, grid, WAVES * kWaveSize, st, y, dy, dx, c, s,
                flat, tiles);
     return launch_status();
 }
 
 constexpr int kNoSplit = -1000; // not the status of a launch
 
-// The split kernel for 33 channels and more, or kNoSplit.  Eight waves with up to 64
-// channels each; sixteen, whose chains of exponentials and sums are half as long, where
-// the tiles of 64 pixels are no more than the CUs (N 4, C 500, 21 x 21: forward 10.6 us, backward
-// 9.1, eight waves 12.4 and 11.3; N 8, C 400, 64 x 64: 32.3 and 36.8, eight waves 30.1 and 35.3),
-// and beyond what eight hold.  Two pixels a lane where that leaves two tiles a CU
-// forward, one backward (N 1, C 60, 384 x 384, 1152 tiles of two pixels a lane: 13.3 and 22.2 us,
-// one pixel 14.3 and 25.4; N 8, C 256, 64 x 64, 256 of them: 17.8 and 21.6, one pixel 16.5 and 23.7).
+// The split kernel for 33 channels and more, or kNoSplit.  Forward + backward, us, by tiles of 64 pixels (16 waves up
+// to 256 tiles, else 8) -> as now:
+// * Up to 256 tiles, no more than the CUs: 16 pixels a tile and 8 waves, four times the workgroups, each with half the
+//   channels a lane.  N 1, C 447, 17 x 13 16.9 -> 8.7; N 7, C 507, 13 x 16 19.9 -> 9.7; N 4, C 341, 50 x 40 17.8 -> 14.3; doubles, whose
+//   exponentials are longer: N 2, C 421, 20 x 19 40.6 -> 12.2, N 5, C 217, 14 x 13 17.3 -> 8.7.  Up to 96
+//   channels (64 of doubles) the launches are all there is (8.1 both ways), and beyond 16 MiB (20) the
+//   parts of lines cost as much: N 28, C 420, 25 x 15 23.3 and 25.6, N 19, C 237, 26 x 26 of doubles 29.5 and 31.2.
+// * 257 to 512 tiles, one or two a CU: 32 pixels, for as many channels a lane as with 16 waves of 64.  N 27, C 133, 23 x 28 16.3 ->
+//   13.8; N 5, C 151, 92 x 67 23.2 -> 19.6; N 4, C 150, 65 x 97 18.4 both ways.  Not where the tensors are streamed (N 1, C 306,
+//   195 x 164 43.2 and 50.2: whole lines count there), nor beyond 384 channels (N 2, C 398, 119 x 107 52 and 57).
+// * Doubles of 257 to 512 channels, of any size: 32 pixels and 8 waves, whose values fit the registers (16 waves of 64
+//   pixels kept five words in scratch, and beyond 384 channels backward read everything twice).  N 17, C 490, 46 x 51 244 -> 185;
+//   N 1, C 267, 197 x 189 112 -> 89.
+// * Sixteen waves of 64 pixels remain for at most 256 tiles of few or of very many channels, and beyond 512 of floats (N 8, C 400,
+//   64 x 64, 512 tiles: 32.3 forward and 36.8 backward, eight waves 30.1 and 35.3).
+// * Two pixels a lane where that leaves two tiles a CU
+//   forward, one backward (N 1, C 60, 384 x 384, 1152 tiles of two pixels a lane: 13.3 and 22.2 us,
+//   one pixel 14.3 and 25.4; N 8, C 256, 64 x 64, 256 of them: 17.8 and 21.6, one pixel 16.5 and 23.7).
 template <typename T, typename... P>
 int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
 {
@@ -963,20 +1006,42 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
     const int flat = flat_samples(n, s);
     const size_t pixels = flat > 0 ? s * n : s, samples = flat > 0 ? 1 : n;
     const size_t tiles = (pixels + kWaveSize - 1) / kWaveSize * samples;
-    if ((tiles <= 256 && c > 64) || c > (kFloat ? 512 : 256))
+    const size_t elements = s * c * n;
+    if (tiles <= 256 && c > (kFloat ? 96 : 64) && c <= 1024 && elements * sizeof(T) <= size_t(kFloat ? 16 : 20) << 20)
     {
-        if (c <= 128) return launch_split<1, 8, 16>(p..., n, c, s, stream, st);
-        if (c <= 192) return launch_split<1, 12, 16>(p..., n, c, s, stream, st);
-        if (c <= 256) return launch_split<1, 16, 16>(p..., n, c, s, stream, st);
-        if (c <= 384) return launch_split<1, 24, 16>(p..., n, c, s, stream, st);
-        if constexpr (kFloat || kForward)
-        {
-            if (c <= 512) return launch_split<1, 32, 16>(p..., n, c, s, stream, st);
-        }
+        if (c <= 128) return launch_split<1, 4, 8, 16, false>(p..., n, c, s, stream, st);
+        if (c <= 192) return launch_split<1, 6, 8, 16, false>(p..., n, c, s, stream, st);
+        if (c <= 256) return launch_split<1, 8, 8, 16, false>(p..., n, c, s, stream, st);
+        if (c <= 384) return launch_split<1, 12, 8, 16, false>(p..., n, c, s, stream, st);
+        if (c <= 512) return launch_split<1, 16, 8, 16, false>(p..., n, c, s, stream, st);
+        if (c <= 768) return launch_split<1, 24, 8, 16, false>(p..., n, c, s, stream, st);
+        return launch_split<1, 32, 8, 16, false>(p..., n, c, s, stream, st);
+    }
+    if (tiles > 256 && tiles <= 512 && c > 64 && c <= (kFloat ? 384 : 256) && !stream)
+    {
+        if (c <= 128) return launch_split<1, 8, 8, 32, false>(p..., n, c, s, stream, st);
+        if (c <= 192) return launch_split<1, 12, 8, 32, false>(p..., n, c, s, stream, st);
+        if (c <= 256) return launch_split<1, 16, 8, 32, false>(p..., n, c, s, stream, st);
+        if constexpr (kFloat)
+            return launch_split<1, 24, 8, 32, false>(p..., n, c, s, stream, st);
+    }
+    if constexpr (!kFloat)
+    {
+        if (c > 512) return kNoSplit;
+        if (c > 384) return launch_split<1, 32, 8, 32>(p..., n, c, s, stream, st);
+        if (c > 256) return launch_split<1, 24, 8, 32>(p..., n, c, s, stream, st);
+    }
+    if ((tiles <= 256 && c > 64) || c > 512)
+    {
         if constexpr (kFloat)
         {
+            if (c <= 96) return launch_split<1, 8, 16>(p..., n, c, s, stream, st);
+            if (c <= 384) return launch_split<1, 24, 16>(p..., n, c, s, stream, st);
+            if (c <= 512) return launch_split<1, 32, 16>(p..., n, c, s, stream, st);
             if (c <= 768) return launch_split<1, 48, 16>(p..., n, c, s, stream, st);
         }
+        else
+            return launch_split<1, 16, 16>(p..., n, c, s, stream, st);
         if constexpr (kFloat && kForward)
         {
             if (c <= 1024) return launch_split<1, 64, 16>(p..., n, c, s, stream, st);
@@ -1125,7 +1190,7 @@ int forward_impl(int n, int c, size_t s, const void* xv, void* yv, hipStream_t s
         return status;
     const int flat = flat_samples(n, s);
     WideTiles tiles;
-    const dim3 grid = wide_grid(s, 1, n, flat, &tiles);
+    const dim3 grid = wide_grid(s, kWaveSize, 1, n, flat, &tiles);
     launch(softmax_fwd_wide_kernel<T>, grid, kBlockSize, st, x, y, c, s, flat, tiles);
     return launch_status();
 }
@@ -1193,7 +1258,7 @@ int backward_impl(int n, int c, size_t s, const void* yv, const void* dyv, void*
         return status;
     const int flat = flat_samples(n, s);
     WideTiles tiles;
-    const dim3 grid = wide_grid(s, 1, n, flat, &tiles);
+    const dim3 grid = wide_grid(s, kWaveSize, 1, n, flat, &tiles);
     launch(softmax_bwd_wide_kernel<T>, grid, kBlockSize, st, y, dy, dx, c, s, flat, tiles);
     return launch_status();
 }
