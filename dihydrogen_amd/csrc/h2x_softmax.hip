@@ -899,14 +899,17 @@ dim3 pixel_grid_xcd(size_t spatial, int vec, int num_samples, int flat)
 // XCDs for every sample (forward + backward, us, filled up and counted through: N 32, C 300, 14 x 14, 4 tiles
 // a sample, 23.3 and 18.0; N 25, C 120, 24 x 24, 9 tiles, 14.9 and 10.9; N 29, C 338, 24 x 37, 14 tiles,
 // 43.6 and 41.4; but N 30, C 179, 43 x 43, 29 tiles, 47.3 and 48.0, N 8, C 40, 128 x 128, 128 tiles,
-// 20.1 and 21.4: samples one after another reach the memory more evenly).
+// 20.1 and 21.4: samples one after another reach the memory more evenly).  Also where only the filling makes them more
+// than two a CU: a third would start when the first two are done, on the XCDs that have it (N 11, C 135, 45 x 61, 473 tiles filled up to 528,
+// 19.3 and 17.4; N 5, C 151, 92 x 67, 485 to 520, 20.7 and 18.8).
 dim3 wide_grid(size_t spatial, int lanes, int vec, int num_samples, int flat, WideTiles* t)
 {
     const dim3 by_sample = tile_grid(spatial, lanes, vec, num_samples, flat);
     const size_t per_block = static_cast<size_t>(lanes) * vec;
     const size_t tiles = (spatial + per_block - 1) / per_block;
     t->samples = flat > 0 ? 1 : num_samples;
-    const bool through = flat == 0 && by_sample.x * static_cast<size_t>(8) > tiles * 9;
+    const size_t launched = by_sample.x * static_cast<size_t>(num_samples), all = tiles * num_samples;
+    const bool through = flat == 0 && (launched * 8 > all * 9 || (lanes == kWaveSize && all <= 512 && launched > 512));
     t->per_sample = make_fastdiv(through ? static_cast<uint32_t>(tiles) : by_sample.x);
     if (!through)
         return by_sample;
@@ -942,7 +945,8 @@ constexpr int kManySamples = 2048;
 // thread keeps all channels of its pixels (softmax_*_reg_kernel: 21 channels of
 // N 16, 256 x 256 in 28 / 40 us).  Beyond, the waves of a workgroup share the channels
 // (softmax_*_split_kernel) with the smallest register tile that holds them: tiles wider
-// than needed cost time, since every lane walks the whole tile under a predicate.  Eight
+// than needed cost time, since every lane walks the whole tile under a predicate (N 1, C 79, 135 x 192 in
+// tiles of 128 channels 12.0, of 96 11.0 us; N 2, C 89, 115 x 115 13.2 and 11.9).  Eight
 // waves against four, N 4, C 150, 65 x 97: forward 10.2 and 11.7 us; N 1: 5.7 and 8.0; N 16:
 // 29.8 and 34.3.  More channels than the largest tile holds (1024 forward, 768 backward, 1024 where
 // tiles are few; double: 512, or 1024; N 18, C 270, 27 x 40 backward, re-reading 40.3 us, in
@@ -986,9 +990,12 @@ constexpr int kNoSplit = -1000; // not the status of a launch
 //   exponentials are longer: N 2, C 421, 20 x 19 40.6 -> 12.2, N 5, C 217, 14 x 13 17.3 -> 8.7.  Up to 96
 //   channels (64 of doubles) the launches are all there is (8.1 both ways), and beyond 16 MiB (20) the
 //   parts of lines cost as much: N 28, C 420, 25 x 15 23.3 and 25.6, N 19, C 237, 26 x 26 of doubles 29.5 and 31.2.
-// * 257 to 512 tiles, one or two a CU: 32 pixels, for as many channels a lane as with 16 waves of 64.  N 27, C 133, 23 x 28 16.3 ->
-//   13.8; N 5, C 151, 92 x 67 23.2 -> 19.6; N 4, C 150, 65 x 97 18.4 both ways.  Not where the tensors are streamed (N 1, C 306,
-//   195 x 164 43.2 and 50.2: whole lines count there), nor beyond 384 channels (N 2, C 398, 119 x 107 52 and 57).
+// * From 257 tiles to about two a CU: forward, floats of 65 to 256 channels, 16 pixels and 4 waves, a lane's chain as short as with 16
+//   waves of 64 (32 pixels and 8 waves: N 4, C 150, 65 x 97 0.6 us more, N 3, C 129, 84 x 65 13.5 for 12.7; but N 20, C 197,
+//   32 x 25 15.4 for 16.1); else 32 pixels and 8 waves, backward to one and a half tiles a CU (beyond, N 4, C 150, 65 x 97 0.2 us
+//   more).  N 27, C 133, 23 x 28 16.3 -> 13.1; N 4, C 150, 65 x 97 18.4 -> 17.0; N 22, C 143, 38 x 33 18.3 -> 17.1.  Not
+//   where the tensors are streamed (N 1, C 306, 195 x 164 43.2 and 50.2: whole lines count there), nor beyond 384
+//   channels (N 2, C 398, 119 x 107 52 and 57).
 // * Doubles of 257 to 512 channels, of any size: 32 pixels and 8 waves, whose values fit the registers (16 waves of 64
 //   pixels kept five words in scratch, and beyond 384 channels backward read everything twice).  N 17, C 490, 46 x 51 244 -> 185;
 //   N 1, C 267, 197 x 189 112 -> 89.
@@ -1017,11 +1024,22 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
         if (c <= 768) return launch_split<1, 24, 8, 16, false>(p..., n, c, s, stream, st);
         return launch_split<1, 32, 8, 16, false>(p..., n, c, s, stream, st);
     }
-    if (tiles > 256 && tiles <= 512 && c > 64 && c <= (kFloat ? 384 : 256) && !stream)
+    if (kForward && kFloat && tiles > 256 && tiles <= 576 && c > 64 && c <= 256 && !stream)
     {
-        if (c <= 128) return launch_split<1, 8, 8, 32, false>(p..., n, c, s, stream, st);
-        if (c <= 192) return launch_split<1, 12, 8, 32, false>(p..., n, c, s, stream, st);
-        if (c <= 256) return launch_split<1, 16, 8, 32, false>(p..., n, c, s, stream, st);
+        if (c <= 96) return launch_split<1, 6, 4, 16, false>(p..., n, c, s, stream, st);
+        if (c <= 128) return launch_split<1, 8, 4, 16, false>(p..., n, c, s, stream, st);
+        if (c <= 160) return launch_split<1, 10, 4, 16, false>(p..., n, c, s, stream, st);
+        if (c <= 192) return launch_split<1, 12, 4, 16, false>(p..., n, c, s, stream, st);
+        return launch_split<1, 16, 4, 16, false>(p..., n, c, s, stream, st);
+    }
+    if (tiles > 256 && tiles <= (kFloat && !kForward ? 384 : 512) && c > 64 && c <= (kFloat ? 384 : 256) && !stream)
+    {
+        if constexpr (!(kFloat && kForward))
+        {
+            if (c <= 128) return launch_split<1, 8, 8, 32, false>(p..., n, c, s, stream, st);
+            if (c <= 192) return launch_split<1, 12, 8, 32, false>(p..., n, c, s, stream, st);
+            if (c <= 256) return launch_split<1, 16, 8, 32, false>(p..., n, c, s, stream, st);
+        }
         if constexpr (kFloat)
             return launch_split<1, 24, 8, 32, false>(p..., n, c, s, stream, st);
     }
@@ -1053,14 +1071,23 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
         if (v >= 2 && c <= 256 && (s + 2 * kWaveSize - 1) / (2 * kWaveSize) * n >= (kForward ? 512 : 256))
         {
             if (c <= 64) return launch_split<2, 8, 8>(p..., n, c, s, stream, st);
+    if (c <= 96) return launch_split<2, 12, 8>(p..., n, c, s, stream, st);
+            if (c <= 96) return launch_split<2, 12, 8>(p..., n, c, s, stream, st);
             if (c <= 128) return launch_split<2, 16, 8>(p..., n, c, s, stream, st);
+    if (c <= 160) return launch_split<2, 20, 8>(p..., n, c, s, stream, st);
+            if (c <= 160) return launch_split<2, 20, 8>(p..., n, c, s, stream, st);
             if (c <= 192) return launch_split<2, 24, 8>(p..., n, c, s, stream, st);
+    if (c <= 224) return launch_split<2, 28, 8>(p..., n, c, s, stream, st);
+            if (c <= 224) return launch_split<2, 28, 8>(p..., n, c, s, stream, st);
             return launch_split<2, 32, 8>(p..., n, c, s, stream, st);
         }
     }
     if (c <= 64) return launch_split<1, 8, 8>(p..., n, c, s, stream, st);
+    if (c <= 96) return launch_split<1, 12, 8>(p..., n, c, s, stream, st);
     if (c <= 128) return launch_split<1, 16, 8>(p..., n, c, s, stream, st);
+    if (c <= 160) return launch_split<1, 20, 8>(p..., n, c, s, stream, st);
     if (c <= 192) return launch_split<1, 24, 8>(p..., n, c, s, stream, st);
+    if (c <= 224) return launch_split<1, 28, 8>(p..., n, c, s, stream, st);
     if (c <= 256) return launch_split<1, 32, 8>(p..., n, c, s, stream, st);
     if constexpr (kFloat)
     {
