@@ -8,11 +8,11 @@
 // 5 to 7 TB/s; here every element is read once.  Bound by memory and by the wait for the
 // last member of a team.  Forward, backward in us, two launches each way -> by teams, going round
 // three sets of tensors:
-//   N 8, C 64, 30^3, halo of 1      38, 54 -> 35, 42     N 32, C 256, 56 x 56     48, 85 -> 40, 63
-//   N 4, C 64, 64^3                116, 189 -> 104, 166  N 64, C 128, 40 x 40     27, 45 -> 19, 31
-//   N 8, C 64, 64^3                257, 411 -> 211, 365  N 2, C 32, 48^3          16, 28 -> 13, 17
-//   N 1, C 64, 96^3                 98, 160 -> 88, 140   N 64, C 64, 57^2, halo   31, 51 -> 32, 40
-//   N 2, C 16, 48^3, halo of 1      12, 17 -> 11, 13     N 8, C 64, 56 x 56      8.6, 10.6 -> 6.1, 8.4
+//   N 8, C 64, 30^3, halo of 1      38, 54 -> 34, 40     N 32, C 256, 56 x 56     48, 85 -> 39, 58
+//   N 4, C 64, 64^3                116, 189 -> 101, 152  N 64, C 128, 40 x 40     27, 45 -> 18, 28
+//   N 8, C 64, 64^3                257, 411 -> 200, 344  N 2, C 32, 48^3          16, 28 -> 12, 15
+//   N 1, C 64, 96^3                 98, 160 -> 87, 131   N 64, C 64, 57^2, halo   31, 51 -> 31, 38
+//   N 2, C 16, 48^3, halo of 1      12, 17 -> 10, 12     N 8, C 64, 56 x 56      8.6, 10.6 -> 5.7, 7.0
 // Looking at a counter of arrivals instead of the sums themselves was slower the
 // larger the team (64 members, N 4, C 64, 64^3: 119 us against 98): one address.
 //
