@@ -576,17 +576,17 @@ def cpu_baseline(repeats: int = 5):
 # TCC_EA0_WRREQ_64B), request counts summed over the L2 channels, per dispatch.
 # label -> (bytes read, bytes written) per launch
 PMC_TRAFFIC = {
-    "bn_forward": (270054656, 268850048),
-    "bn_backward": (541286528, 269631328),
-    "bn_sums": (268457472, 131072),
-    "bn_apply": (268466176, 268503808),
-    "bn_backprop1": (536912896, 131072),
-    "bn_backprop2": (536906240, 268435456),
-    "halo_dim0_pack": (147835520, 8652800),    # 4 faces (2 ranks) a launch, four launches a step
-    "halo_dim0_unpack": (9219904, 43264000),
-    "halo_dim1_pack": (42624768, 34611200),
-    "halo_dim1_unpack": (34632448, 36215328),
-    "halo_dim2_pack": (34695424, 34611200),
+    "bn_forward": (269445632, 268963808),
+    "bn_backward": (539850496, 269649600),
+    "bn_sums": (268459008, 131072),
+    "bn_apply": (268467200, 268490880),
+    "bn_backprop1": (536912384, 131072),
+    "bn_backprop2": (536902144, 268435456),
+    "halo_dim0_pack": (147810816, 8652800),    # 4 faces (2 ranks) a launch, four launches a step
+    "halo_dim0_unpack": (9217920, 43264000),
+    "halo_dim1_pack": (42625920, 34611200),
+    "halo_dim1_unpack": (34632448, 36218400),
+    "halo_dim2_pack": (34694400, 34611200),
     "halo_dim2_unpack": (34632448, 34619392),
 }
 # steps of the timed region whose dominant-kernel launches are bracketed by events: every EVENT_EVERY-th
@@ -594,8 +594,8 @@ EVENT_EVERY = 4
 
 # sha256 (first 16 hex digits) of the kernel sources the table was measured with, see
 # kernel_sources_sha(); with other sources the traffic fields are omitted
-PMC_SOURCES_SHA = "abc7713f1a78f849"
-PMC_COMMIT = "9ddd2b6"
+PMC_SOURCES_SHA = "25e471531c65f6ad"
+PMC_COMMIT = "3421070"
 
 KERNEL_OF = {
     "bn_forward": "bn_team_forward_kernel<float,512,16>",
