@@ -1024,13 +1024,16 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
         if (c <= 768) return launch_split<1, 24, 8, 16, false>(p..., n, c, s, stream, st);
         return launch_split<1, 32, 8, 16, false>(p..., n, c, s, stream, st);
     }
-    if (kForward && kFloat && tiles > 256 && tiles <= 576 && c > 64 && c <= 256 && !stream)
+    if constexpr (kForward && kFloat)
     {
-        if (c <= 96) return launch_split<1, 6, 4, 16, false>(p..., n, c, s, stream, st);
-        if (c <= 128) return launch_split<1, 8, 4, 16, false>(p..., n, c, s, stream, st);
-        if (c <= 160) return launch_split<1, 10, 4, 16, false>(p..., n, c, s, stream, st);
-        if (c <= 192) return launch_split<1, 12, 4, 16, false>(p..., n, c, s, stream, st);
-        return launch_split<1, 16, 4, 16, false>(p..., n, c, s, stream, st);
+        if (tiles > 256 && tiles <= 576 && c > 64 && c <= 256 && !stream)
+        {
+            if (c <= 96) return launch_split<1, 6, 4, 16, false>(p..., n, c, s, stream, st);
+            if (c <= 128) return launch_split<1, 8, 4, 16, false>(p..., n, c, s, stream, st);
+            if (c <= 160) return launch_split<1, 10, 4, 16, false>(p..., n, c, s, stream, st);
+            if (c <= 192) return launch_split<1, 12, 4, 16, false>(p..., n, c, s, stream, st);
+            return launch_split<1, 16, 4, 16, false>(p..., n, c, s, stream, st);
+        }
     }
     if (tiles > 256 && tiles <= (kFloat && !kForward ? 384 : 512) && c > 64 && c <= (kFloat ? 384 : 256) && !stream)
     {
