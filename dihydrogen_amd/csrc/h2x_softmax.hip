@@ -946,7 +946,8 @@ constexpr int kManySamples = 2048;
 // N 16, 256 x 256 in 28 / 40 us).  Beyond, the waves of a workgroup share the channels
 // (softmax_*_split_kernel) with the smallest register tile that holds them: tiles wider
 // than needed cost time, since every lane walks the whole tile under a predicate (N 1, C 79, 135 x 192 in
-// tiles of 128 channels 12.0, of 96 11.0 us; N 2, C 89, 115 x 115 13.2 and 11.9).  Eight
+// tiles of 128 channels 12.0, of 96 11.0 us; N 2, C 89, 115 x 115 13.2 and 11.9; N 2, C 393, 78 x 126 in 512 43.7, in
+// 448 42.0; but of 257 to 320 channels some are 4 % faster in 320 than in 384, and others 2 % slower).  Eight
 // waves against four, N 4, C 150, 65 x 97: forward 10.2 and 11.7 us; N 1: 5.7 and 8.0; N 16:
 // 29.8 and 34.3.  More channels than the largest tile holds (1024 forward, 768 backward, 1024 where
 // tiles are few; double: 512, or 1024; N 18, C 270, 27 x 40 backward, re-reading 40.3 us, in
@@ -1095,6 +1096,7 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
     if constexpr (kFloat)
     {
         if (c <= 384) return launch_split<1, 48, 8>(p..., n, c, s, stream, st);
+        if (c <= 448) return launch_split<1, 56, 8>(p..., n, c, s, stream, st);
         if (c <= 512) return launch_split<1, 64, 8>(p..., n, c, s, stream, st);
     }
     return kNoSplit;

@@ -20,7 +20,7 @@ def test_sixteen_pixels(c, n, spatial, dtype):
     (1, 65, 257 * 64 - 31, "float32"), (1, 384, 257 * 64 - 33, "float32"), (128, 385, 65 * 2, "float32"),
     (1, 96, 300 * 64, "float32"), (1, 97, 300 * 64 - 47, "float32"), (1, 129, 383 * 64 + 1, "float32"), (1, 161, 385 * 64 - 1, "float32"),
     (1, 193, 576 * 64 - 15, "float32"), (1, 256, 577 * 64, "float32"), (1, 225, 600 * 64 - 1, "float32"), (11, 135, 45 * 61, "float32"),
-    (1, 66, 512 * 64 - 1, "float32"), (1, 66, 512 * 64 + 1, "float32"), (300, 70, 107, "float32"), (1, 130, 300 * 64, "float32"),
+    (1, 448, 600 * 64 - 1, "float32"), (1, 449, 600 * 64 - 1, "float32"), (1, 66, 512 * 64 - 1, "float32"), (1, 66, 512 * 64 + 1, "float32"), (300, 70, 107, "float32"), (1, 130, 300 * 64, "float32"),
     (1, 160, 256 * 64, "float64"), (1, 161, 256 * 64, "float64"), (1, 193, 256 * 64, "float64"), (1, 65, 257 * 64 - 31, "float64"),
     (1, 256, 400 * 64 - 33, "float64"), (1, 257, 600 * 64 - 33, "float64"), (2, 386, 300 * 64 + 2, "float64"),
     (1, 512, 513 * 64 + 31, "float64"), (1, 513, 257 * 64 + 1, "float64"), (1, 256, 513 * 64, "float64"),
