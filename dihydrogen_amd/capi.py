@@ -327,8 +327,8 @@ _calls = None
 
 def calls():
     """The native module whose functions call the library (csrc/h2x_python.cpp): the entry points
-    the layers call once per step, under their own names, taking torch tensors, local tensors (the
-    address of the first interior element), addresses or None for pointers and returning the status.
+    the layers call once per step, under their own names, taking torch tensors, local tensors (what
+    their get_base_ptr() returns), addresses or None for pointers and returning the status.
     Raises if it is absent."""
     global _calls
     if _calls is None:
@@ -338,8 +338,9 @@ def calls():
         except ImportError as e:
             raise H2XError("_h2xcall.so is missing: build it with `make -C dihydrogen_amd/csrc` "
                            "(or __graft_entry__.build()); there is no fallback path") from e
-        from .tensor import Tensor
-        _h2xcall.tensor_type(Tensor)  # for a pointer: the address of its first interior element
+        import torch
+        from .tensor import GET_BASE_PTR, Tensor
+        _h2xcall.pointer_types(torch.Tensor, Tensor, GET_BASE_PTR)
         _calls = _h2xcall
     return _calls
 

@@ -5,9 +5,9 @@
 // spent more time on that than the GPU on the work.  Here each entry point is
 // one METH_FASTCALL function whose argument conversions are generated from its
 // C signature: integers and floats as they are, and for a pointer None, an
-// address, any object with a data_ptr() method (a torch tensor), or one with a get_base_ptr()
-// method, a local tensor (where it is of the very type given to tensor_type() its `data` and `base_bytes` are
-// read here: 0.1 us less than a method that is written in Python).  Every
+// address, a torch tensor, any other object with a get_base_ptr() method (a local tensor: the method is asked, also where
+// there is a data_ptr() too, or, where it is the one given to pointer_types(), what it does is
+// done here, 0.1 us less than in Python), or one with a data_ptr() method alone.  Every
 // function returns what the C function returns (a status or a size).  The GIL
 // is released during the call, as ctypes does.
 #define PY_SSIZE_T_CLEAN
@@ -24,19 +24,36 @@ namespace
 {
 
 PyObject *s_data_ptr = nullptr, *s_get_base_ptr = nullptr, *s_data = nullptr, *s_base_bytes = nullptr; // interned names
-PyTypeObject* s_tensor_type = nullptr;
+PyTypeObject *s_torch_tensor = nullptr, *s_local_tensor = nullptr;
+PyObject* s_base_ptr_method = nullptr; // of s_local_tensor
+
+bool as_address(PyObject* address, void** out)
+{
+    *out = PyLong_AsVoidPtr(address);
+    return *out != nullptr || !PyErr_Occurred();
+}
 
 // What o's method returns, an address; false: an exception is set.
 bool address_by(PyObject* method, PyObject* o, void** out)
 {
     PyObject* const address = PyObject_CallMethodNoArgs(o, method);
-    if (!address)
-        return false;
-    *out = PyLong_AsVoidPtr(address);
-    Py_DECREF(address);
-    return *out != nullptr || !PyErr_Occurred();
+    const bool ok = address && as_address(address, out);
+    Py_XDECREF(address);
+    return ok;
 }
 
+// Whether o is a local tensor of the very class whose get_base_ptr() is known, replaced on neither the class nor the
+// object.  (Two look-ups in dictionaries; to make the bound method and compare it took twice as long.)
+bool has_known_base(PyObject* o)
+{
+    if (Py_TYPE(o) != s_local_tensor
+        || PyDict_GetItemWithError(s_local_tensor->tp_dict, s_get_base_ptr) != s_base_ptr_method)
+        return false;
+    PyObject** const own = _PyObject_GetDictPtr(o);
+    return !own || !*own || !PyDict_GetItemWithError(*own, s_get_base_ptr);
+}
+
+// What that get_base_ptr() returns: data.data_ptr() + base_bytes.
 bool base_of(PyObject* o, void** out)
 {
     PyObject* const data = PyObject_GetAttr(o, s_data);
@@ -57,24 +74,25 @@ bool base_of(PyObject* o, void** out)
     return true;
 }
 
-// Any other object's: which method it has is not asked of a torch tensor, where that would be a second look-up.
 bool address_of(PyObject* o, void** out)
 {
-    if (address_by(s_data_ptr, o, out))
-        return true;
-    if (!PyErr_ExceptionMatches(PyExc_AttributeError))
-        return false;
-    PyObject *type, *value, *trace;
-    PyErr_Fetch(&type, &value, &trace);
-    if (PyObject_HasAttr(o, s_data_ptr) || !PyObject_HasAttr(o, s_get_base_ptr))
+    if (has_known_base(o))
+        return base_of(o, out);
+    if (s_torch_tensor && PyObject_TypeCheck(o, s_torch_tensor))
+        return address_by(s_data_ptr, o, out);
+    PyObject* const method = PyObject_GetAttr(o, s_get_base_ptr);
+    if (!method)
     {
-        PyErr_Restore(type, value, trace);
-        return false;
+        if (!PyErr_ExceptionMatches(PyExc_AttributeError))
+            return false;
+        PyErr_Clear();
+        return address_by(s_data_ptr, o, out);
     }
-    Py_XDECREF(type);
-    Py_XDECREF(value);
-    Py_XDECREF(trace);
-    return address_by(s_get_base_ptr, o, out);
+    PyObject* const address = PyObject_CallNoArgs(method);
+    Py_DECREF(method);
+    const bool ok = address && as_address(address, out);
+    Py_XDECREF(address);
+    return ok;
 }
 
 template <typename P>
@@ -94,7 +112,7 @@ bool convert(PyObject* o, P* out)
             return p != nullptr || !PyErr_Occurred();
         }
         void* p;
-        if (!(Py_TYPE(o) == s_tensor_type ? base_of(o, &p) : address_of(o, &p)))
+        if (!address_of(o, &p))
             return false;
         *out = reinterpret_cast<P>(p);
         return true;
@@ -144,14 +162,20 @@ struct Entry<F>
     }
 };
 
-// tensor_type(type): of local tensors.
-PyObject* tensor_type(PyObject*, PyObject* type)
+// pointer_types(torch.Tensor, the class of local tensors, its get_base_ptr)
+PyObject* pointer_types(PyObject*, PyObject* const* args, Py_ssize_t nargs)
 {
-    if (!PyType_Check(type))
-        return PyErr_Format(PyExc_TypeError, "a type");
-    Py_INCREF(type);
-    Py_XDECREF(reinterpret_cast<PyObject*>(s_tensor_type));
-    s_tensor_type = reinterpret_cast<PyTypeObject*>(type);
+    if (nargs != 3 || !PyType_Check(args[0]) || !PyType_Check(args[1]))
+        return PyErr_Format(PyExc_TypeError, "two types and a function");
+    PyObject* const before[] = {reinterpret_cast<PyObject*>(s_torch_tensor), reinterpret_cast<PyObject*>(s_local_tensor),
+                                s_base_ptr_method};
+    for (Py_ssize_t i = 0; i < nargs; ++i)
+        Py_INCREF(args[i]);
+    s_torch_tensor = reinterpret_cast<PyTypeObject*>(args[0]);
+    s_local_tensor = reinterpret_cast<PyTypeObject*>(args[1]);
+    s_base_ptr_method = args[2];
+    for (PyObject* const o : before)
+        Py_XDECREF(o);
     Py_RETURN_NONE;
 }
 
@@ -240,7 +264,8 @@ PyMethodDef s_methods[] = {H2X_ENTRY(h2x_bn_channel_sums_and_sqsums),
                            H2X_ENTRY(h2x_shuffle_direct),
                            H2X_ENTRY(h2x_shuffle_pack_batched),
                            H2X_ENTRY(h2x_shuffle_unpack_batched),
-                           {"tensor_type", tensor_type, METH_O, nullptr},
+                           {"pointer_types",
+                            reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&pointer_types)), METH_FASTCALL, nullptr},
                            {"same_buffers",
                             reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&same_buffers)), METH_FASTCALL, nullptr},
                            {nullptr, nullptr, 0, nullptr}};

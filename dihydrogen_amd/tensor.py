@@ -319,3 +319,7 @@ class Tensor:
         for axis, (o, l) in enumerate(zip(reversed(self.overlap), reversed(self.local_shape))):
             v = v.narrow(axis, o, l)
         return v
+
+
+# what the native module does by itself for a tensor that has no other get_base_ptr() (csrc/h2x_python.cpp)
+GET_BASE_PTR = Tensor.get_base_ptr

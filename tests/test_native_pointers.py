@@ -1,4 +1,6 @@
 """What the native calls take for a pointer, and how they compare the buffers of tensors."""
+import ctypes
+
 import pytest
 import torch
 
@@ -32,6 +34,56 @@ def test_a_local_tensor_is_the_address_of_its_interior(kind, overlap):
     x = t.data[first:first + 24].cpu().double().view(2, 3, 4)
     assert torch.equal(got, want)
     torch.testing.assert_close(got.cpu().double().view(2, 3, 4), torch.softmax(x, 1), rtol=1e-5, atol=1e-7)
+
+
+class WithBuffer(Tensor):
+    """Names its allocation as torch names a tensor's; its interior is elsewhere."""
+
+    def data_ptr(self):
+        return self.get_buffer()
+
+
+class Alike:
+    """No Tensor, with both methods."""
+
+    def __init__(self, t):
+        self.get_base_ptr, self.data_ptr = t.get_base_ptr, t.get_buffer
+
+
+@pytest.mark.parametrize("kind", ["tensor", "derived", "with data_ptr", "alike", "replaced on the object",
+                                  "replaced on the class"])
+def test_the_address_is_what_get_base_ptr_returns(kind, monkeypatch):
+    """Shown on the host: a call that reads a geometry, and geometries in the tensor's buffer."""
+    # of 64 and, where the interior begins, of 128 channels, one element further on of 256
+    dist = Distribution.make_overlapped_distribution([1] * 4, [1, 0, 0, 0])
+    item = ctypes.sizeof(capi.TensorGeometry)
+    cls = {"derived": Derived, "with data_ptr": WithBuffer}.get(kind, Tensor)
+    t = cls([4096, 1, 1, 1], LocaleVirtual(0, 1), dist, torch.uint8, "cpu")
+    monkeypatch.setattr(t, "base_bytes", item)
+    t.allocate()
+    for i, channels in enumerate((64, 128, 256)):
+        g = capi.TensorGeometry()
+        g.num_dims = 4
+        for d, (extent, stride) in enumerate(zip((64, 64, channels, 16), (1, 64, 4096, 4096 * channels))):
+            g.local_shape[d], g.strides[d] = extent, stride
+        at = i * item
+        t.data[at:at + item] = torch.frombuffer(bytearray(bytes(g)), dtype=torch.uint8)
+    needed = capi.calls().h2x_bn_team_state_needed
+    sizes = [needed(capi.F32, 16, t.get_buffer() + i * item) for i in range(3)]
+    assert 0 < sizes[0] < sizes[1] < sizes[2]
+    o, want = t, 1
+    if kind == "derived":
+        monkeypatch.setattr(Derived, "get_base_ptr", lambda self: Tensor.get_base_ptr(self) + item)
+        want = 2
+    elif kind == "alike":
+        o = Alike(t)
+    elif kind == "replaced on the object":
+        monkeypatch.setattr(t, "get_base_ptr", lambda: t.get_buffer() + 2 * item)
+        want = 2
+    elif kind == "replaced on the class":
+        monkeypatch.setattr(Tensor, "get_base_ptr", lambda self: self.get_buffer() + 2 * item)
+        want = 2
+    assert needed(capi.F32, 16, o) == sizes[want]
 
 
 def test_what_has_no_address_is_refused():
