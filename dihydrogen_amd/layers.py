@@ -68,6 +68,25 @@ def _first_stream_handle() -> int:
     return _current_stream(_current_device())
 
 
+class _Kept:
+    """What a layer keeps for its calls on one stream, each buffer behind what it is for: calls on other streams,
+    which may run at the same time, have their own.  (A tuple is replaced as a whole: threads may share a layer.)"""
+    __slots__ = ("workspace", "scalars", "state")
+
+    def __init__(self):
+        self.workspace = self.state = (-1, None)
+        self.scalars = (-1, None, None)
+
+
+def _first_use(kept: dict, handle: int) -> _Kept:
+    """For a stream that a layer has not been used on.  A graph is captured on a stream of its own, and uses what the
+    layer keeps for the newest of its other streams (that of the warm-up): a state made during the capture would be
+    cleared by the graph's replays, at each of them, and by nothing else."""
+    if kept and torch.cuda.is_current_stream_capturing():
+        return next(reversed(list(kept.values())))
+    return kept.setdefault(handle, _Kept())
+
+
 def _dense_layout(t: Tensor) -> Layout:
     """The layout of a tensor with no halo on its channel and sample dimensions."""
     l = t.layout
@@ -116,6 +135,9 @@ class BatchNormalization:
     ``allreduce``, if given, is called as ``allreduce(list_of_per_channel_tensors)``
     where the reference sums over ranks (batchnorm.hpp:185-214,360-400); with the
     default ``None`` the layer is a single rank and the step is the identity.
+
+    Calls on different streams may run at the same time if their outputs are apart.  A captured
+    graph shares the buffers of a stream (_first_use): its replays and the calls there follow one another.
     """
 
     def __init__(self, num_dims: int, decay: float, epsilon: float, global_stats: bool = False,
@@ -139,36 +161,42 @@ class BatchNormalization:
         self.num_current_samples = 0
         self._lib = capi.load()
         self._calls = capi.calls()
-        self._workspace: Optional[torch.Tensor] = None
-        self._workspace_channels = -1
-        self._state: Optional[torch.Tensor] = None
-        self._state_channels = -1
+        self._kept = {}  # by the handle of a stream
 
     # batchnorm.hpp:467-475
     def set_num_samples(self, n: int) -> None:
         self.num_current_samples = int(n)
 
-    def _ws(self, num_channels: int) -> torch.Tensor:
-        if self._workspace is None or self._workspace_channels != num_channels:
-            nbytes = self._lib.h2x_bn_workspace_bytes(num_channels)
-            self._workspace = _buffer_of(self.stream, nbytes, torch.uint8)
-            self._workspace_channels = num_channels
-        return self._workspace
+    def _ws(self, num_channels: int, st: int) -> torch.Tensor:
+        kept = self._kept.get(st) or _first_use(self._kept, st)
+        channels, ws = kept.workspace
+        if channels != num_channels:
+            ws = _buffer_of(self.stream, self._lib.h2x_bn_workspace_bytes(num_channels), torch.uint8)
+            kept.workspace = num_channels, ws
+        return ws
 
-    def _team_state(self, l: Layout, clearing: bool) -> Optional[torch.Tensor]:
+    def _team_state(self, l: Layout, clearing: bool, st: int) -> Optional[torch.Tensor]:
         """Where the workgroups that share a channel exchange its sums; None where no workgroups
         do.  Smaller channels than 16 K floats or 4 K doubles need none."""
         double = l.dtype == capi.F64
         if l.samples * l.spatial_real <= (4096 if double else 16384) or double and clearing:
             return None
-        if self._state is None or self._state_channels < l.channels:
+        kept = self._kept.get(st) or _first_use(self._kept, st)
+        channels, state = kept.state
+        if channels < l.channels:
             nbytes = (l.ordered_state_bytes if double else
                       l.clearing_team_state_bytes if clearing else l.team_state_bytes)
             if nbytes == 0:
                 return None
-            self._state = _buffer_of(self.stream, nbytes, torch.uint8, zero=True)
-            self._state_channels = l.channels
-        return self._state
+            state = _buffer_of(self.stream, nbytes, torch.uint8, zero=True)
+            kept.state = l.channels, state
+        return state
+
+    @property
+    def _state(self) -> Optional[torch.Tensor]:
+        """The state for calls on the stream that a call would go to."""
+        kept = self._kept.get(_stream_handle(self.stream))
+        return kept and kept.state[1]
 
     def _num_per_sum(self, t: Tensor) -> int:
         """Elements per channel of the global (global_stats) or local shape
@@ -183,15 +211,15 @@ class BatchNormalization:
         if not is_training:
             return 0
         _dense_layout(input)
-        ns = lx.samples if lx.active else 0
+        ns, st = lx.samples if lx.active else 0, _stream_handle(self.stream)
         if lx.dense:
             capi.check(self._calls.h2x_bn_channel_sums_and_sqsums(
                 lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, input, mean, var,
-                self._ws(lx.channels), _stream_handle(self.stream)), "channel_sums_and_sqsums")
+                self._ws(lx.channels, st), st), "channel_sums_and_sqsums")
         else:  # halo on an inner spatial dimension: the generic path of batchnorm.cu:232-248
             capi.check(self._calls.h2x_bn_channel_sums_and_sqsums_strided(
                 lx.dtype, ns, _tensor_geometry(lx, ns), input, mean, var,
-                self._ws(lx.channels), _stream_handle(self.stream)), "channel_sums_and_sqsums (strided)")
+                self._ws(lx.channels, st), st), "channel_sums_and_sqsums (strided)")
         return 0
 
     def forward_allreduce(self, mean: torch.Tensor, var: torch.Tensor, is_training: bool = True) -> int:
@@ -257,10 +285,11 @@ class BatchNormalization:
         if local and self.clear_output_halo and (lx.haloed or ly.haloed):
             local = False  # the stages, unless a whole pass clears the halo
             if _share_a_haloed_geometry(lx, ly):
+                st = _stream_handle(self.stream)
                 status = self._calls.h2x_bn_forward_clearing(
                     lx.dtype, lx.haloed_geometry_address, input.get_buffer(), scale, bias, self._elements_per_sum(lx),
                     self.decay, self.epsilon, mean, var, running_mean, running_var, output.get_buffer(),
-                    self._team_state(lx, True), _stream_handle(self.stream))
+                    self._team_state(lx, True, st), st)
                 if status != capi.ERR_UNSUPPORTED:
                     self.num_current_samples = lx.samples
                     capi.check(status, "bn forward (clearing)")
@@ -268,17 +297,17 @@ class BatchNormalization:
         if local:
             _dense_layout(input), _dense_layout(output)
             ns = self.num_current_samples = lx.samples
-            per_sum = self._elements_per_sum(lx)
+            per_sum, st = self._elements_per_sum(lx), _stream_handle(self.stream)
             if lx.extents != ly.extents and _pair_in_order(lx, ly):
                 capi.check(self._calls.h2x_bn_forward_local(
                     lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ly.spatial_real, input,
                     scale, bias, per_sum, self.decay, self.epsilon, mean, var, running_mean, running_var,
-                    output, self._ws(lx.channels), _stream_handle(self.stream)), "bn forward (local)")
+                    output, self._ws(lx.channels, st), st), "bn forward (local)")
                 return 0
             status = self._calls.h2x_bn_forward_once(
                 lx.dtype, ns, lx.geometry_address, _tensor_geometry(ly, ns), input, scale, bias, per_sum,
                 self.decay, self.epsilon, mean, var, running_mean, running_var, output,
-                self._ws(lx.channels), self._team_state(lx, False), _stream_handle(self.stream))
+                self._ws(lx.channels, st), self._team_state(lx, False, st), st)
             if status:
                 capi.check(status, "bn forward (local)")
             return 0
@@ -292,9 +321,9 @@ class BatchNormalization:
                         bias_gradient, mean_gradient, var_gradient) -> int:
         lx, ld = _dense_layout(input), _dense_layout(d_output)
         self.num_current_samples = lx.samples
-        ns = lx.samples if lx.active else 0
+        ns, st = lx.samples if lx.active else 0, _stream_handle(self.stream)
         tail = (mean, var, scale, scale_gradient, bias_gradient, mean_gradient, var_gradient, self.epsilon,
-                self._ws(lx.channels), _stream_handle(self.stream))
+                self._ws(lx.channels, st), st)
         if lx.dense and ld.dense:
             capi.check(self._calls.h2x_bn_backprop1(
                 lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ld.spatial_real, input,
@@ -344,11 +373,11 @@ class BatchNormalization:
         if local and self.clear_output_halo and (lx.haloed or ld.haloed or li.haloed):
             local = False
             if _share_a_haloed_geometry(lx, ld, li):
+                st = _stream_handle(self.stream)
                 status = self._calls.h2x_bn_backward_clearing(
                     lx.dtype, self._elements_per_sum(lx), lx.haloed_geometry_address, input.get_buffer(),
                     d_output.get_buffer(), mean, var, scale, scale_gradient, bias_gradient, mean_gradient,
-                    var_gradient, d_input.get_buffer(), self.epsilon, self._team_state(lx, True),
-                    _stream_handle(self.stream))
+                    var_gradient, d_input.get_buffer(), self.epsilon, self._team_state(lx, True, st), st)
                 if status != capi.ERR_UNSUPPORTED:
                     self.num_current_samples = lx.samples
                     capi.check(status, "bn backward (clearing)")
@@ -356,19 +385,19 @@ class BatchNormalization:
         if local:
             _dense_layout(input), _dense_layout(d_output), _dense_layout(d_input)
             ns = self.num_current_samples = lx.samples
-            per_sum = self._elements_per_sum(lx)
+            per_sum, st = self._elements_per_sum(lx), _stream_handle(self.stream)
             if (lx.extents != ld.extents or lx.extents != li.extents) and _pair_in_order(lx, ld, li):
                 capi.check(self._calls.h2x_bn_backward_local(
                     lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ld.spatial_real, li.spatial_real, per_sum,
                     input, d_output, mean, var, scale, scale_gradient, bias_gradient,
-                    mean_gradient, var_gradient, d_input, self.epsilon, self._ws(lx.channels),
-                    _stream_handle(self.stream)), "bn backward (local)")
+                    mean_gradient, var_gradient, d_input, self.epsilon, self._ws(lx.channels, st), st),
+                    "bn backward (local)")
                 return 0
             status = self._calls.h2x_bn_backward_once(
                 lx.dtype, ns, per_sum, lx.geometry_address, _tensor_geometry(ld, ns), _tensor_geometry(li, ns),
                 input, d_output, mean, var, scale, scale_gradient, bias_gradient,
-                mean_gradient, var_gradient, d_input, self.epsilon, self._ws(lx.channels),
-                self._team_state(lx, False), _stream_handle(self.stream))
+                mean_gradient, var_gradient, d_input, self.epsilon, self._ws(lx.channels, st),
+                self._team_state(lx, False, st), st)
             if status:
                 capi.check(status, "bn backward (local)")
             return 0
@@ -446,6 +475,8 @@ class Softmax:
     ``allreduce(values, is_max)``, if given, is called on the per-sample scalars of
     instance mode where the reference all-reduces them over the ranks that share
     a sample (softmax.hpp:52-62); ``None`` means every sample is whole on this rank.
+
+    Calls on different streams and captured graphs: as BatchNormalization's.
     """
 
     def __init__(self, stream: Optional[torch.cuda.Stream] = None,
@@ -454,12 +485,7 @@ class Softmax:
         self.mode = SoftmaxMode.CHANNEL
         self._lib = capi.load()
         self._calls = capi.calls()
-        # buffers and what they hold: calls to ask a tensor would be a tenth of a small call
-        self._ws: Optional[torch.Tensor] = None
-        self._scalars: Optional[torch.Tensor] = None
-        self._state: Optional[torch.Tensor] = None
-        self._ws_bytes = self._scalars_count = self._state_bytes = 0
-        self._scalars_type: Optional[torch.dtype] = None
+        self._kept = {}  # by the handle of a stream
 
     def setup(self, input: Tensor, mode: SoftmaxMode) -> None:
         self.mode = mode
@@ -471,27 +497,33 @@ class Softmax:
             raise NotImplementedError("softmax assumes a dense local tensor")  # softmax.cu:562-563
         return l
 
-    def _workspace(self, l: Layout) -> torch.Tensor:
+    # (what a buffer holds stands beside it: calls to ask a tensor would be a tenth of a small call)
+    def _workspace(self, l: Layout, kept: _Kept) -> torch.Tensor:
+        held, ws = kept.workspace
         need = l.instance_workspace_bytes
-        if self._ws_bytes < need:
-            self._ws, self._ws_bytes = _buffer_of(self.stream, need, torch.uint8), need
-        return self._ws
+        if held < need:
+            ws = _buffer_of(self.stream, need, torch.uint8)
+            kept.workspace = need, ws
+        return ws
 
-    def _team_state(self, l: Layout) -> Optional[torch.Tensor]:
+    def _team_state(self, l: Layout, kept: _Kept) -> Optional[torch.Tensor]:
         """Where the workgroups that share a sample exchange its partial results; None where no workgroups do."""
         need = l.instance_state_bytes
         if need == 0:
             return None
-        if self._state_bytes < need:
-            self._state, self._state_bytes = _buffer_of(self.stream, need, torch.uint8, zero=True), need
-        return self._state
+        held, state = kept.state
+        if held < need:
+            state = _buffer_of(self.stream, need, torch.uint8, zero=True)
+            kept.state = need, state
+        return state
 
-    def _sample_scalars(self, t: Tensor, count: int) -> torch.Tensor:
+    def _sample_scalars(self, t: Tensor, count: int, kept: _Kept) -> torch.Tensor:
         """`count` scalars of t's type that nobody reads after the call: kept like the workspace."""
-        if self._scalars_count < count or self._scalars_type is not t.dtype:
-            self._scalars = _buffer_of(self.stream, count, t.dtype)
-            self._scalars_count, self._scalars_type = count, t.dtype
-        return self._scalars
+        held, dtype, scalars = kept.scalars
+        if held < count or dtype is not t.dtype:
+            scalars = _buffer_of(self.stream, count, t.dtype)
+            kept.scalars = count, t.dtype, scalars
+        return scalars
 
     def forward(self, x: Tensor, y: Tensor) -> int:
         l = self._geometry(x)
@@ -506,13 +538,14 @@ class Softmax:
                 capi.check(status, "softmax forward")
             return 0
         # instance mode: softmax.cu:723-746
-        calls, dt, size, ws = self._calls, l.dtype, l.channels * l.spatial, self._workspace(l)
+        kept = self._kept.get(st) or _first_use(self._kept, st)
+        calls, dt, size, ws = self._calls, l.dtype, l.channels * l.spatial, self._workspace(l, kept)
         if self.allreduce is None:
             # every sample is whole on this rank: the stages need not be separate calls
-            scalars = self._sample_scalars(x, 2 * n).data_ptr()
+            scalars = self._sample_scalars(x, 2 * n, kept).data_ptr()
             status = calls.h2x_softmax_instance_forward_once(
                 dt, n, size, x, y, scalars,
-                scalars + n * x.dtype.itemsize, ws, self._team_state(l), -1, st)
+                scalars + n * x.dtype.itemsize, ws, self._team_state(l, kept), -1, st)
             if status:
                 capi.check(status, "softmax instance forward")
             return 0
@@ -540,11 +573,12 @@ class Softmax:
                 capi.check(status, "softmax backward")
             return 0
         # instance mode: softmax.cu:770-783
-        calls, size, ws = self._calls, l.channels * l.spatial, self._workspace(l)
+        kept = self._kept.get(st) or _first_use(self._kept, st)
+        calls, size, ws = self._calls, l.channels * l.spatial, self._workspace(l, kept)
         if self.allreduce is None:
             status = calls.h2x_softmax_instance_backward_once(
-                dt, n, size, y, dy, dx, self._sample_scalars(y, n), ws,
-                self._team_state(l), -1, st)
+                dt, n, size, y, dy, dx, self._sample_scalars(y, n, kept), ws,
+                self._team_state(l, kept), -1, st)
             if status:
                 capi.check(status, "softmax instance backward")
             return 0

@@ -45,3 +45,42 @@ def test_layer_on_its_own_stream_while_the_current_one_is_busy(halo):
     for (ya, da, va), (yb, db, vb) in zip(want, got):
         for a, b in zip([ya.data, da.data] + va, [yb.data, db.data] + vb):
             assert torch.equal(a, b)
+
+
+def test_one_layer_on_two_streams_at_once():
+    """Channels that teams share: each stream has its own state, so no call takes the other's sums for its own."""
+    import torch
+    from dihydrogen_amd.layers import BatchNormalization
+    from dihydrogen_amd.tensor import Distribution, LocaleVirtual, Tensor
+    g = torch.Generator(device="cuda").manual_seed(4)
+    dist, c, calls = Distribution.make_localized_distribution(4), 128, 8
+    make = lambda: Tensor([56, 56, c, 16], LocaleVirtual(0, 1), dist).allocate()
+    vec = lambda v: torch.full((c,), v, device="cuda")
+    scale, bias = vec(1.25), vec(-0.5)
+    sides = []
+    for _ in range(2):
+        x, dy = make(), make()
+        for t in (x, dy):
+            t.data.normal_(0.5, 2, generator=g)
+        sides.append((torch.cuda.Stream(), x, dy, [(make(), make(), [vec(0.0) for _ in range(8)]) for _ in range(calls + 1)]))
+
+    def run(layer, x, dy, out):
+        y, dx, v = out
+        layer.forward(x, *v[:4], scale, bias, y, True)
+        layer.backward(x, dy, *v[:2], scale, *v[4:], dx)
+
+    layer = BatchNormalization(4, 0.9, 1e-5)
+    for _, x, dy, outs in sides:
+        run(layer, x, dy, outs[calls])      # one after the other
+    assert layer._state is not None         # this size is for several workgroups a channel
+    torch.cuda.synchronize()
+    for i in range(calls):
+        for stream, x, dy, outs in sides:
+            with torch.cuda.stream(stream):
+                run(layer, x, dy, outs[i])
+    torch.cuda.synchronize()
+    for _, _, _, outs in sides:
+        y, dx, v = outs[calls]
+        for out in outs[:calls]:
+            for a, b in zip([y.data, dx.data] + v, [out[0].data, out[1].data] + out[2]):
+                assert torch.equal(a, b)

@@ -141,3 +141,73 @@ def test_what_is_packed_on_a_stream_of_its_own_is_waited_for(made, monkeypatch):
     assert waited == [stream]
     xch.recv_buffer(1, 0, capi.LHS)     # packed with the first
     assert waited == [stream]
+
+
+def _normalized(layer_stream=None):
+    """A batch-norm whose channels teams share, and a step of it."""
+    x, y = _tensors([56, 56, 128, 16], Distribution.make_localized_distribution(4), 2)
+    bn = BatchNormalization(4, 0.9, 1e-5, stream=layer_stream)
+
+    def step():
+        bn.forward(x, *[x.data] * 6, y)
+        bn.backward(x, y, *[x.data] * 7, y)
+    return bn, step
+
+
+def _classified(layer_stream=None):
+    x, y = _tensors([100, 100, 21, 2], Distribution.make_localized_distribution(4), 2)
+    sm = Softmax(layer_stream)
+    sm.setup(x, SoftmaxMode.INSTANCE)
+
+    def step():
+        sm.forward(x, y)
+        sm.backward(y, y, x)
+    return sm, step
+
+
+@pytest.mark.parametrize("use", [_normalized, _classified])
+def test_streams_share_no_buffer(use, made, monkeypatch):
+    """Calls on two streams may run at the same time: what a launch writes to belongs to its stream.  A graph is captured
+    on a stream of its own and makes nothing there."""
+    current, capturing, passed = [1], [False], []
+    monkeypatch.setattr(layers, "_stream_handle", lambda stream: stream.cuda_stream if stream else current[0])
+    monkeypatch.setattr(layers.torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+
+    class Calls(_Calls):
+        def __getattr__(self, name):
+            if "_needed" in name or "workspace_bytes" in name:
+                return getattr(self.native, name)
+            return lambda *args: passed.append([a.data_ptr() for a in args if a is not None and hasattr(a, "data_ptr")
+                                                and id(a) in buffers] + [a for a in args if a in scalars]) or 0
+
+    buffers, scalars = {}, set()
+    device_buffer = layers._device_buffer
+
+    def recorded(*args, **kwargs):
+        b = device_buffer(*args, **kwargs)
+        buffers[id(b)] = b
+        scalars.add(b.data_ptr())
+        return b
+
+    monkeypatch.setattr(layers, "_device_buffer", recorded)
+    monkeypatch.setattr(capi, "calls", Calls)
+    layer, step = use()
+
+    def on(stream):
+        current[0] = stream
+        passed.clear()
+        step()
+        return [set(p) for p in passed]
+
+    first, count = on(1), len(buffers)
+    second = on(2)
+    assert count and len(buffers) == 2 * count
+    assert all(a and not a & b for a, b in zip(first, second))
+    assert on(1) == first and on(2) == second and len(buffers) == 2 * count
+    capturing[0] = True
+    assert on(3) == second and on(1) == first and len(buffers) == 2 * count
+    capturing[0] = False
+    assert not any(a & b for a, b in zip(on(3), second)) and len(buffers) == 3 * count
+    # of a layer with a stream of its own, whichever is current
+    layer, step = use(_Stream())
+    assert on(1) == on(2)
