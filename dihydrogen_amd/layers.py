@@ -497,33 +497,31 @@ class Softmax:
             raise NotImplementedError("softmax assumes a dense local tensor")  # softmax.cu:562-563
         return l
 
-    # (what a buffer holds stands beside it: calls to ask a tensor would be a tenth of a small call)
-    def _workspace(self, l: Layout, kept: _Kept) -> torch.Tensor:
+    def _buffers(self, l: Layout, t: Tensor, count: int, st: int):
+        """The workspace; `count` scalars of t's type that nobody reads after the call; and where the workgroups that
+        share a sample exchange its partial results (None where no workgroups do).  count = 0: the workspace alone.
+        (In one go, and by what stands beside each buffer: a call for each, and to ask the tensors, would be a tenth of a
+        small softmax.)"""
+        kept = self._kept.get(st) or _first_use(self._kept, st)
         held, ws = kept.workspace
         need = l.instance_workspace_bytes
         if held < need:
             ws = _buffer_of(self.stream, need, torch.uint8)
             kept.workspace = need, ws
-        return ws
-
-    def _team_state(self, l: Layout, kept: _Kept) -> Optional[torch.Tensor]:
-        """Where the workgroups that share a sample exchange its partial results; None where no workgroups do."""
-        need = l.instance_state_bytes
-        if need == 0:
-            return None
-        held, state = kept.state
-        if held < need:
-            state = _buffer_of(self.stream, need, torch.uint8, zero=True)
-            kept.state = need, state
-        return state
-
-    def _sample_scalars(self, t: Tensor, count: int, kept: _Kept) -> torch.Tensor:
-        """`count` scalars of t's type that nobody reads after the call: kept like the workspace."""
+        if count == 0:
+            return ws, None, None
         held, dtype, scalars = kept.scalars
         if held < count or dtype is not t.dtype:
             scalars = _buffer_of(self.stream, count, t.dtype)
             kept.scalars = count, t.dtype, scalars
-        return scalars
+        need = l.instance_state_bytes
+        if need == 0:
+            return ws, scalars, None
+        held, state = kept.state
+        if held < need:
+            state = _buffer_of(self.stream, need, torch.uint8, zero=True)
+            kept.state = need, state
+        return ws, scalars, state
 
     def forward(self, x: Tensor, y: Tensor) -> int:
         l = self._geometry(x)
@@ -538,17 +536,18 @@ class Softmax:
                 capi.check(status, "softmax forward")
             return 0
         # instance mode: softmax.cu:723-746
-        kept = self._kept.get(st) or _first_use(self._kept, st)
-        calls, dt, size, ws = self._calls, l.dtype, l.channels * l.spatial, self._workspace(l, kept)
+        calls, dt, size = self._calls, l.dtype, l.channels * l.spatial
         if self.allreduce is None:
             # every sample is whole on this rank: the stages need not be separate calls
-            scalars = self._sample_scalars(x, 2 * n, kept).data_ptr()
+            ws, scalars, state = self._buffers(l, x, 2 * n, st)
+            scalars = scalars.data_ptr()
             status = calls.h2x_softmax_instance_forward_once(
                 dt, n, size, x, y, scalars,
-                scalars + n * x.dtype.itemsize, ws, self._team_state(l, kept), -1, st)
+                scalars + n * x.dtype.itemsize, ws, state, -1, st)
             if status:
                 capi.check(status, "softmax instance forward")
             return 0
+        ws, _, _ = self._buffers(l, x, 0, st)
         smax, sexp = (_buffer_of(self.stream, n, x.dtype, x.device) for _ in range(2))
         capi.check(calls.h2x_softmax_instance_max(dt, n, size, x, smax, ws, st),
                    "softmax instance max")
@@ -573,15 +572,15 @@ class Softmax:
                 capi.check(status, "softmax backward")
             return 0
         # instance mode: softmax.cu:770-783
-        kept = self._kept.get(st) or _first_use(self._kept, st)
-        calls, size, ws = self._calls, l.channels * l.spatial, self._workspace(l, kept)
+        calls, size = self._calls, l.channels * l.spatial
         if self.allreduce is None:
+            ws, scalars, state = self._buffers(l, y, n, st)
             status = calls.h2x_softmax_instance_backward_once(
-                dt, n, size, y, dy, dx, self._sample_scalars(y, n, kept), ws,
-                self._team_state(l, kept), -1, st)
+                dt, n, size, y, dy, dx, scalars, ws, state, -1, st)
             if status:
                 capi.check(status, "softmax instance backward")
             return 0
+        ws, _, _ = self._buffers(l, y, 0, st)
         sdp = _buffer_of(self.stream, n, y.dtype, y.device)
         capi.check(calls.h2x_softmax_instance_dot(dt, n, size, y, dy, sdp, ws, st),
                    "softmax instance dot")
