@@ -2819,8 +2819,8 @@ void team_launch(const G& once, const A<T>& a, bool stream, uint32_t members, ui
         issue_team<T, TEAM, K, G::kClears>(g, a, states, st);
 }
 
-// Looks of about a microsecond: a team that other streams keep off the chip for longer
-// works its sums out (2 ms against the tens of microseconds of a launch).
+// Looks of about a microsecond, or of two in launches of more than kCrowd workgroups, which sleep longer between them: a team
+// that other streams keep off the chip for 2 ms, or for 5, works its sums out (a launch takes tens to hundreds of us).
 constexpr uint32_t kTeamPolls = 2048;
 // Workgroups from which teams are taken, of the smallest members and of larger ones (forward + backward, N 1, C 1, 64^3, 32
 // workgroups of 32 KB, 17.0 us in two launches, 13.2 by them; backward N 2, C 1, 96^3 11.6 in two launches, 14.6 in 54 of 128 KB;

@@ -212,21 +212,17 @@ __device__ __forceinline__ void ordered_exchange(double (&v)[N], const OrderedGe
         if (t < kBlockSize) // whole waves
         {
             const unsigned long long* const at = words + 2 * first * items + item;
-            bool there = !reads, seen = items <= kSmallTeam;
-            for (uint32_t poll = 0; poll < g.max_polls; ++poll) // uniform
-            {
-                if (poll > 0)
-                    __builtin_amdgcn_s_sleep(4);
-                if (!seen)
+            bool there = !reads;
+            uint32_t looks = g.max_polls; // uniform
+            if (items > kSmallTeam)
+                for (; looks > 1 && __any(!there && first == 0 && team_load(at) >> 32 != tag); --looks)
                 {
-                    if (__any(!there && first == 0 && team_load(at) >> 32 != tag))
-                    {
-                        if (gridDim.x > kCrowd) // uniform
-                            __builtin_amdgcn_s_sleep(40);
-                        continue;
-                    }
-                    seen = true;
+                    __builtin_amdgcn_s_sleep(4);
+                    if (gridDim.x > kCrowd) // uniform
+                        __builtin_amdgcn_s_sleep(40);
                 }
+            for (; looks > 0; --looks)
+            {
                 if (!there)
                 {
                     double one[1];
@@ -240,6 +236,7 @@ __device__ __forceinline__ void ordered_exchange(double (&v)[N], const OrderedGe
                 }
                 if (__all(there))
                     break;
+                __builtin_amdgcn_s_sleep(4);
             }
             if (!there || !reads)
                 s[0] = s[1] = 0.0;

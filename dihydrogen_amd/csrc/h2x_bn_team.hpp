@@ -109,21 +109,17 @@ __device__ __forceinline__ void team_exchange(double own, double (&v)[N], const 
     {
         const unsigned long long* const at = words + m;
         double s = 0.0;
-        bool there = m >= members, seen = members <= kSmallTeam;
-        for (uint32_t poll = 0; poll < g.max_polls; ++poll) // uniform
-        {
-            if (poll > 0)
-                __builtin_amdgcn_s_sleep(4);
-            if (!seen)
+        bool there = m >= members;
+        uint32_t looks = g.max_polls; // uniform
+        if (members > kSmallTeam)     // (the last look is one at all words: it takes what has come, whoever is missing)
+            for (; looks > 1 && __any(!there && k == N - 1 && team_load(at) >> 32 != tag); --looks)
             {
-                if (__any(!there && k == N - 1 && team_load(at) >> 32 != tag))
-                {
-                    if (gridDim.x > kCrowd) // uniform
-                        __builtin_amdgcn_s_sleep(40);
-                    continue;
-                }
-                seen = true;
+                __builtin_amdgcn_s_sleep(4);
+                if (gridDim.x > kCrowd) // uniform
+                    __builtin_amdgcn_s_sleep(40);
             }
+        for (; looks > 0; --looks)
+        {
             if (!there)
             {
                 const unsigned long long lo = team_load(at), hi = team_load(at + members);
@@ -133,6 +129,7 @@ __device__ __forceinline__ void team_exchange(double own, double (&v)[N], const 
             }
             if (__all(there))
                 break;
+            __builtin_amdgcn_s_sleep(4);
         }
         shared.theirs[k][m] = s;
         const unsigned long long late = __ballot(!there);

@@ -115,6 +115,21 @@ def test_channel_in_a_team(shape):
     _close(p.run("once"), by_team)
 
 
+# 33 to 64 members a channel: two waves look after them forward, three and four backward
+@pytest.mark.parametrize("shape", [(1, 1, 1, 800, 820, 0), (1, 2, 62, 90, 94, 1), (1, 1, 1, 900, 1160, 0)])
+def test_members_that_several_waves_look_after(shape):
+    """The same bits when all, some or none of the others' sums are worked out."""
+    import torch
+    p = _Problem(*shape)
+    counter = p.state.view(torch.int64)[:1]
+    by_team = p.run("team", 2048)
+    assert int(counter) > 2 * 32    # members, forward and backward: each has added one
+    _close(by_team, p.run("local_strided"))
+    for polls in (0, 1, 2, 3, 2048):
+        for a, b in zip(by_team, p.run("team", polls)):
+            assert torch.equal(a, b)
+
+
 def test_one_state_for_calls_of_other_sizes():
     """Teams of other sizes, forward and backward, leave sums of earlier calls in the state: none is taken for a new one."""
     import torch

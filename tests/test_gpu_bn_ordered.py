@@ -108,6 +108,18 @@ def test_channel_in_a_team(shape):
     _same(p.run("once"), want)
 
 
+# more than 64 groups a channel: several waves look after their sums, in steps of four and of two
+@pytest.mark.parametrize("shape", [(1, 1, 1, 640, 512, 0), (1, 2, 50, 62, 64, 1), (1, 1, 1, 460, 400, 0)])
+def test_groups_that_several_waves_look_after(shape):
+    """The same bits when all, some or none of the others' sums are worked out."""
+    p = _Problem(*shape)
+    counter = p.state.view(p.torch.int64)[:1]
+    want = p.run("local_strided")
+    for polls in (2048, 0, 1, 2, 3, 2048):
+        _same(p.run("team", polls), want)
+    assert int(counter) > 6 * 2 * 16
+
+
 def test_one_state_for_doubles_and_calls_of_other_sizes():
     problems = [_Problem(*s) for s in [(2, 3, 40, 32, 32), (1, 3, 1, 64, 300), (3, 3, 17, 18, 19, 2)]]
     wants = [p.run("local_strided") for p in problems]
