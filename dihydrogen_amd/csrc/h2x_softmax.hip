@@ -1057,7 +1057,7 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
     {
         if constexpr (kFloat)
         {
-            if (c <= 96) return launch_split<1, 8, 16>(p..., n, c, s, stream, st);
+            if (c <= 96) return launch_split<1, 8, 16, kWaveSize, false>(p..., n, c, s, stream, st);
             if (c <= 384) return launch_split<1, 24, 16>(p..., n, c, s, stream, st);
             if (c <= 512) return launch_split<1, 32, 16>(p..., n, c, s, stream, st);
             if (c <= 768) return launch_split<1, 48, 16>(p..., n, c, s, stream, st);
@@ -1075,22 +1075,21 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
         if (v >= 2 && c <= 256 && (s + 2 * kWaveSize - 1) / (2 * kWaveSize) * n >= (kForward ? 512 : 256))
         {
             if (c <= 64) return launch_split<2, 8, 8>(p..., n, c, s, stream, st);
-    if (c <= 96) return launch_split<2, 12, 8>(p..., n, c, s, stream, st);
             if (c <= 96) return launch_split<2, 12, 8>(p..., n, c, s, stream, st);
             if (c <= 128) return launch_split<2, 16, 8>(p..., n, c, s, stream, st);
-    if (c <= 160) return launch_split<2, 20, 8>(p..., n, c, s, stream, st);
             if (c <= 160) return launch_split<2, 20, 8>(p..., n, c, s, stream, st);
             if (c <= 192) return launch_split<2, 24, 8>(p..., n, c, s, stream, st);
-    if (c <= 224) return launch_split<2, 28, 8>(p..., n, c, s, stream, st);
             if (c <= 224) return launch_split<2, 28, 8>(p..., n, c, s, stream, st);
             return launch_split<2, 32, 8>(p..., n, c, s, stream, st);
         }
     }
-    if (c <= 64) return launch_split<1, 8, 8>(p..., n, c, s, stream, st);
-    if (c <= 96) return launch_split<1, 12, 8>(p..., n, c, s, stream, st);
-    if (c <= 128) return launch_split<1, 16, 8>(p..., n, c, s, stream, st);
-    if (c <= 160) return launch_split<1, 20, 8>(p..., n, c, s, stream, st);
-    if (c <= 192) return launch_split<1, 24, 8>(p..., n, c, s, stream, st);
+    // (floats that are streamed have, with few channels, the pixels for two a lane)
+    constexpr bool kStreams96 = !kFloat, kStreams192 = !kFloat || kForward;
+    if (c <= 64) return launch_split<1, 8, 8, kWaveSize, kStreams96>(p..., n, c, s, stream, st);
+    if (c <= 96) return launch_split<1, 12, 8, kWaveSize, kStreams96>(p..., n, c, s, stream, st);
+    if (c <= 128) return launch_split<1, 16, 8, kWaveSize, kStreams192>(p..., n, c, s, stream, st);
+    if (c <= 160) return launch_split<1, 20, 8, kWaveSize, kStreams192>(p..., n, c, s, stream, st);
+    if (c <= 192) return launch_split<1, 24, 8, kWaveSize, kStreams192>(p..., n, c, s, stream, st);
     if (c <= 224) return launch_split<1, 28, 8>(p..., n, c, s, stream, st);
     if (c <= 256) return launch_split<1, 32, 8>(p..., n, c, s, stream, st);
     if constexpr (kFloat)
