@@ -592,14 +592,20 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
     __shared__ T lds[WAVES][LANES * VEC];
     constexpr int kApart = kWaveSize / LANES; // channels that a wave takes at once
     const int lane = threadIdx.x % LANES, q = threadIdx.x % kWaveSize / LANES;
-    // Of more than 256 channels in floats the index stays a lane's own: as a scalar, the addresses
+    // Of more than 256 channels in floats, a lane a pixel, the index stays a lane's own: as a scalar, the addresses
     // and the tests of all those channels are scalars too, more than there are (16 waves with 24
     // channels each spill 31 of them into vector registers, with 48 153; up to 256 channels a wave
     // of 16 spills two).  us, scalar and so: N 4, C 428, 20 x 26 12.4 -> 8.0, N 2, C 494, 34 x 19
-    // 13.3 -> 8.6, N 8, C 395, 46 x 46 31.5 -> 25.2; 245 drawn sizes 0.94 of the time, the worst
+    // 13.3 -> 8.6 (both in tiles of 16 pixels now), N 8, C 395, 46 x 46 31.5 -> 25.2; 245 drawn sizes 0.94 of the time, the worst
     // 1.08.  Doubles fill the vector registers first (1.01 to 1.06 of the scalar's time), and the
     // forward pass, of half the addresses, is faster with the scalar.
-    const int g = sizeof(T) == 4 && WAVES * CPW > 256 ? static_cast<int>(threadIdx.x / kWaveSize) : wave_index();
+    // With several lanes a pixel the tests are the lanes' own in any case, and the scalar is 4 to 8 % faster, although 24 and 32
+    // channels a lane spill 35 and 77 scalars (scalar and so: N 6, C 270, 20 x 30 4.4 and 4.8 us; N 1, C 512, 90 x 90 10.4 and 11.1;
+    // N 1, C 1000, 50 x 52 8.9 and 9.3, but N 1, C 900, 17 x 13 6.8 and 5.7; in tiles of 32 pixels N 23, C 380, 30 x 33 25.2 and 26.4,
+    // N 1, C 270, 128 x 130 11.9 and 11.7), but for 24 a lane in tiles of 16 (N 8, C 520, 11 x 12 5.1 and 4.6; N 1, C 768,
+    // 70 x 75 12.6 and 12.1).
+    constexpr bool kOwnIndex = sizeof(T) == 4 && (LANES == kWaveSize ? WAVES * CPW > 256 : LANES == 16 && CPW == 24);
+    const int g = kOwnIndex ? static_cast<int>(threadIdx.x / kWaveSize) : wave_index();
     size_t base;
     const bool active = tile_pixels<VEC, LANES>(tiles, num_channels, spatial, flat_samples, &base);
     base += q * spatial;
