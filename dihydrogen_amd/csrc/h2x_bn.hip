@@ -2888,7 +2888,7 @@ int cheapest_pass(const PassShape& p, const uint32_t (&members)[3], bool forced)
 {
     const PassCost& cost = (FORWARD ? kForwardCost : kBackwardCost)[sizeof(T) == 8][p.rows];
     const auto& on_cu = FORWARD ? kForwardOnCu : sizeof(T) == 4 ? kBackwardOnCu : kBackwardDoublesOnCu;
-    const uint32_t cus = compute_units();
+    const uint32_t cus = chip_units();
     const float mb = p.bytes * 1e-6f;
     float least = forced ? std::numeric_limits<float>::max() : cost.launches + cost.launches_per_mb * mb;
     int best = -1;
@@ -2896,7 +2896,7 @@ int cheapest_pass(const PassShape& p, const uint32_t (&members)[3], bool forced)
     {
         if (members[i] == 0)
             continue;
-        const float full = static_cast<float>(static_cast<uint64_t>(members[i]) * p.channels) / ((cus ? cus : 256) * on_cu[i]);
+        const float full = static_cast<float>(static_cast<uint64_t>(members[i]) * p.channels) / (cus * on_cu[i]);
         const float rounds = full <= 1 ? 1 : cost.saved * full + (1 - cost.saved) * std::ceil(full);
         const float us = cost.members[i].per_mb * mb + rounds * (cost.members[i].per_round + cost.wait * members[i] / 64)
                          + cost.displaced_per_mb * p.displaced * 1e-6f;
@@ -3014,7 +3014,7 @@ bool teams_first(const G& g)
         return false;
     if (g.num_channels <= kOnceManyChannels || g.vectors > 8192)
         return true;
-    const uint32_t known = compute_units(), cus = known ? known : 256;
+    const uint32_t cus = chip_units();
     const uint32_t rounds = (g.num_channels + cus - 1) / cus;
     const uint32_t filled = g.num_channels * 16 / (rounds * cus); // sixteenths of the rounds
     if constexpr (G::kClears)

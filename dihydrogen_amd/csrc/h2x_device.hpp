@@ -388,6 +388,13 @@ inline uint32_t compute_units()
     return static_cast<uint32_t>(cus);
 }
 
+// CUs that a launch rule counts with: an MI355X's where no device can be asked.
+inline uint32_t chip_units()
+{
+    const uint32_t cus = compute_units();
+    return cus ? cus : 256;
+}
+
 // ---- workgroup order ---------------------------------------------------------
 // Workgroups go to the eight XCDs round-robin (workgroup i runs on XCD i mod
 // 8) and every XCD has its own L2 with its own address-interleaved channels.

@@ -915,7 +915,8 @@ dim3 wide_grid(size_t spatial, int lanes, int vec, int num_samples, int flat, Wi
     const size_t tiles = (spatial + per_block - 1) / per_block;
     t->samples = flat > 0 ? 1 : num_samples;
     const size_t launched = by_sample.x * static_cast<size_t>(num_samples), all = tiles * num_samples;
-    const bool through = flat == 0 && (launched * 8 > all * 9 || (lanes == kWaveSize && all <= 512 && launched > 512));
+    const size_t two = 2 * chip_units();
+    const bool through = flat == 0 && (launched * 8 > all * 9 || (lanes == kWaveSize && all <= two && launched > two));
     t->per_sample = make_fastdiv(through ? static_cast<uint32_t>(tiles) : by_sample.x);
     if (!through)
         return by_sample;
@@ -990,8 +991,8 @@ int launch_split(const T* y, const T* dy, T* dx, int n, int c, size_t s, bool st
 
 constexpr int kNoSplit = -1000; // not the status of a launch
 
-// The split kernel for 33 channels and more, or kNoSplit.  Forward + backward, us, by tiles of 64 pixels (16 waves up
-// to 256 tiles, else 8) -> as now:
+// The split kernel for 33 channels and more, or kNoSplit.  (Tiles are of 64 pixels; their numbers below are those for 256 CUs.)
+// Forward + backward, us, by such tiles (16 waves up to 256 of them, else 8) -> as now:
 // * Up to 256 tiles, no more than the CUs: 16 pixels a tile and 8 waves, four times the workgroups, each with half the
 //   channels a lane.  N 1, C 447, 17 x 13 16.9 -> 8.7; N 7, C 507, 13 x 16 19.9 -> 9.7; N 4, C 341, 50 x 40 17.8 -> 14.3; doubles, whose
 //   exponentials are longer: N 2, C 421, 20 x 19 40.6 -> 12.2, N 5, C 217, 14 x 13 17.3 -> 8.7.  Up to 96
@@ -1020,8 +1021,8 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
     const int flat = flat_samples(n, s);
     const size_t pixels = flat > 0 ? s * n : s, samples = flat > 0 ? 1 : n;
     const size_t tiles = (pixels + kWaveSize - 1) / kWaveSize * samples;
-    const size_t elements = s * c * n;
-    if (tiles <= 256 && c > (kFloat ? 96 : 64) && c <= 1024 && elements * sizeof(T) <= size_t(kFloat ? 16 : 20) << 20)
+    const size_t elements = s * c * n, cus = chip_units();
+    if (tiles <= cus && c > (kFloat ? 96 : 64) && c <= 1024 && elements * sizeof(T) <= size_t(kFloat ? 16 : 20) << 20)
     {
         if (c <= 128) return launch_split<1, 4, 8, 16, false>(p..., n, c, s, stream, st);
         if (c <= 192) return launch_split<1, 6, 8, 16, false>(p..., n, c, s, stream, st);
@@ -1033,7 +1034,7 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
     }
     if constexpr (kForward && kFloat)
     {
-        if (tiles > 256 && tiles <= 576 && c > 64 && c <= 256 && !stream)
+        if (tiles > cus && tiles <= cus * 9 / 4 && c > 64 && c <= 256 && !stream)
         {
             if (c <= 96) return launch_split<1, 6, 4, 16, false>(p..., n, c, s, stream, st);
             if (c <= 128) return launch_split<1, 8, 4, 16, false>(p..., n, c, s, stream, st);
@@ -1042,7 +1043,7 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
             return launch_split<1, 16, 4, 16, false>(p..., n, c, s, stream, st);
         }
     }
-    if (tiles > 256 && tiles <= (kFloat && !kForward ? 384 : 512) && c > 64 && c <= (kFloat ? 384 : 256) && !stream)
+    if (tiles > cus && tiles <= (kFloat && !kForward ? cus * 3 / 2 : cus * 2) && c > 64 && c <= (kFloat ? 384 : 256) && !stream)
     {
         if constexpr (!(kFloat && kForward))
         {
@@ -1059,7 +1060,7 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
         if (c > 384) return launch_split<1, 32, 8, 32>(p..., n, c, s, stream, st);
         if (c > 256) return launch_split<1, 24, 8, 32>(p..., n, c, s, stream, st);
     }
-    if ((tiles <= 256 && c > 64) || c > 512)
+    if ((tiles <= cus && c > 64) || c > 512)
     {
         if constexpr (kFloat)
         {
@@ -1078,7 +1079,7 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
     }
     if constexpr (kFloat)
     {
-        if (v >= 2 && c <= 256 && (s + 2 * kWaveSize - 1) / (2 * kWaveSize) * n >= (kForward ? 512 : 256))
+        if (v >= 2 && c <= 256 && (s + 2 * kWaveSize - 1) / (2 * kWaveSize) * n >= (kForward ? 2 : 1) * cus)
         {
             if (c <= 64) return launch_split<2, 8, 8>(p..., n, c, s, stream, st);
             if (c <= 96) return launch_split<2, 12, 8>(p..., n, c, s, stream, st);
@@ -1806,8 +1807,7 @@ constexpr InstForwardCost kInstForwardCost[3] = {{-2.19f, -0.179f, -0.292f, {0.7
 
 bool inst_forward_pays(const InstForwardCost& cost, size_t bytes, size_t members, size_t n, int each)
 {
-    const uint32_t cus = compute_units();
-    const float mb = bytes * 1e-6f, on_chip = static_cast<float>((cus ? cus : 256) * (each <= 4 ? 2 : 1));
+    const float mb = bytes * 1e-6f, on_chip = static_cast<float>(chip_units() * (each <= 4 ? 2 : 1));
     const float round = cost.per_round[each <= 4 ? 0 : each <= 8 ? 1 : 2] + cost.wait * members / 64;
     return cost.base + cost.per_mb * mb + cost.per_mb_beyond * std::max(mb - 40, 0.0f) + std::ceil(members * n / on_chip) * round < 0;
 }
