@@ -206,8 +206,11 @@ __device__ __forceinline__ void add_products(double& acc, const Pack<T, VEC>& y,
 }
 
 // Waves of a SIMD: two members of 1024 threads a CU, for which a thread may have 64 registers, where it holds up to 32 (HELD
-// elements; doubles in single elements spill then).  Forward + backward going round three sets of tensors, 67 registers and one
-// member a CU -> this: N 11, 527,040 floats, 47.0 -> 37.5 us, N 16, 1,225,728 109 -> 95, N 23, 632,400 doubles 157 -> 135.
+// elements; doubles in single elements spill then).  Without the bound the compiler gives forward floats of 8 vectors 67 registers,
+// doubles 69, backward floats of 4 vectors 66, and single elements (61 and 59) too many scalars: one member a CU.  us, without ->
+// with, going round three sets of tensors: forward N 16, 1,225,728 floats 59.3 -> 51.5, N 23, 632,400 doubles 82.2 -> 68.0; backward
+// N 11, 527,040 floats 17.3 -> 15.5; single elements N 24, 318,009 24.6 -> 20.8 forward, 21.7 -> 18.9 backward, but, where all members
+// have a CU of their own, N 4, 500,001 12.8 -> 13.0 and 9.1 -> 9.45, N 11, 263,537 12.6 -> 12.8 and 10.1 -> 10.4.
 template <typename T, int TEAM, int HELD, bool SINGLE>
 constexpr int inst_waves()
 {
