@@ -187,10 +187,7 @@ __device__ __forceinline__ void ordered_exchange(double (&v)[N], const OrderedGe
         };
         unsigned long long* const words = state + kCounterWords;
         if (t < per_member * N && member * per_member + t / N < items)
-        {
-            const double mine[1] = {item_of(member, t / N, t % N)};
-            team_put<1>(words + 2 * (t % N) * items, items, member * per_member + t / N, tag, mine);
-        }
+            team_put(words + 2 * (t % N) * items, items, member * per_member + t / N, tag, item_of(member, t / N, t % N));
         // the sums of its item that a lane looks for: one, or, of four with items on every other lane, two
         const uint32_t item = t / width, first = t % width;
         const bool two = N == 4 && width == 2; // uniform
@@ -225,14 +222,9 @@ __device__ __forceinline__ void ordered_exchange(double (&v)[N], const OrderedGe
             {
                 if (!there)
                 {
-                    double one[1];
-                    there = team_get<1>(at, items, 0, tag, 1, one);
-                    s[0] = one[0];
+                    there = team_look(at, items, tag, &s[0]);
                     if (two)
-                    {
-                        there = team_get<1>(at + 4 * items, items, 0, tag, 1, one) && there;
-                        s[1] = one[0];
-                    }
+                        there = team_look(at + 4 * items, items, tag, &s[1]) && there;
                 }
                 if (__all(there))
                     break;

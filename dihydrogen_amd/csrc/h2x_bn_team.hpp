@@ -23,7 +23,8 @@
 // other streams fill it; the launch rule keeps a team within half of it.
 #pragma once
 
-constexpr uint32_t kMaxMembers = 128;  // a thread looks after one, no team has fewer threads
+// (A wave looks after 64 / N members with N lanes each, N sums: 8 waves after 128 of four sums, the most that team_exchange takes.)
+constexpr uint32_t kMaxMembers = 128;
 
 // State of a channel, zero before its first call: the counter on a line of its own, then
 // two words a sum.  A channel has room for 256 sums, members times sums of a member: 128 forward, 64 backward.  Larger teams are
@@ -101,10 +102,7 @@ __device__ __forceinline__ void team_exchange(double own, double (&v)[N], const 
     const uint32_t lookers = (members + kGroup - 1) / kGroup; // waves
     unsigned long long* const words = state + kCounterWords + 2 * k * members;
     if (threadIdx.x < kWaveSize && lane % kGroup == 0)
-    {
-        const double mine[1] = {own};
-        team_put<1>(words, members, member, tag, mine);
-    }
+        team_put(words, members, member, tag, own);
     if (wave < lookers) // uniform
     {
         const unsigned long long* const at = words + m;
@@ -121,12 +119,7 @@ __device__ __forceinline__ void team_exchange(double own, double (&v)[N], const 
         for (; looks > 0; --looks)
         {
             if (!there)
-            {
-                const unsigned long long lo = team_load(at), hi = team_load(at + members);
-                there = lo >> 32 == tag && hi >> 32 == tag;
-                if (there)
-                    s = __longlong_as_double(hi << 32 | (lo & 0xffffffffull));
-            }
+                there = team_look(at, members, tag, &s);
             if (__all(there))
                 break;
             __builtin_amdgcn_s_sleep(4);

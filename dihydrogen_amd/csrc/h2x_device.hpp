@@ -249,8 +249,8 @@ __device__ __forceinline__ double read_lane(double v, int lane)
     return __longlong_as_double(static_cast<long long>(static_cast<unsigned long long>(hi) << 32 | lo));
 }
 
-// Steps of wave_sum from those that add lanes `first` apart (1, 2 or 4).  Lanes that are no multiple of
-// `first` hold nothing and get nothing.
+// Steps of wave_sum from those that add lanes `first` apart (1, 2 or 4): lanes that leave the same remainder when divided by
+// `first` are added, each such set by itself, and all of them return its sum.
 __device__ __forceinline__ double wave_sum_from(double v, uint32_t first)
 {
     if (first < 2)
@@ -325,41 +325,32 @@ __device__ __forceinline__ void team_leave(unsigned long long* state)
 {
     __hip_atomic_fetch_add(state, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// Stores v at place `at` of `places`; the same word of all places lies side by side, so that a look reads few lines.
-template <int N>
-__device__ __forceinline__ void team_put(unsigned long long* words, uint32_t places, uint32_t at, uint32_t tag,
-                                         const double (&v)[N])
+// Stores v at place `at` of `places`; the same half of all places lies side by side, so that a look reads few lines.
+__device__ __forceinline__ void team_put(unsigned long long* words, uint32_t places, uint32_t at, uint32_t tag, double v)
 {
-#pragma unroll
-    for (int k = 0; k < N; ++k)
-    {
-        const unsigned long long bits = __double_as_longlong(v[k]);
-        team_store(words + 2 * k * places + at, tag, static_cast<uint32_t>(bits));
-        team_store(words + (2 * k + 1) * places + at, tag, static_cast<uint32_t>(bits >> 32));
-    }
+    const unsigned long long bits = __double_as_longlong(v);
+    team_store(words + at, tag, static_cast<uint32_t>(bits));
+    team_store(words + places + at, tag, static_cast<uint32_t>(bits >> 32));
 }
-// What place `at` holds, once it holds it; false after max_polls looks.
-template <int N>
-__device__ __forceinline__ bool team_get(const unsigned long long* words, uint32_t places, uint32_t at, uint32_t tag,
-                                         uint32_t max_polls, double (&v)[N])
+// Whether a place, whose first half lies at `at`, holds what this call has stored; then that in *v.
+__device__ __forceinline__ bool team_look(const unsigned long long* at, uint32_t places, uint32_t tag, double* v)
 {
-    const unsigned long long* const mine = words + at;
+    const unsigned long long lo = team_load(at), hi = team_load(at + places);
+    const bool there = lo >> 32 == tag && hi >> 32 == tag;
+    if (there)
+        *v = __longlong_as_double(hi << 32 | (lo & 0xffffffffull));
+    return there;
+}
+// What it holds, once it holds it; false after max_polls looks.
+__device__ __forceinline__ bool team_get(const unsigned long long* at, uint32_t places, uint32_t tag, uint32_t max_polls,
+                                         double* v)
+{
     bool there = false;
     for (uint32_t poll = 0; poll < max_polls && !there; ++poll)
     {
         if (poll > 0)
             __builtin_amdgcn_s_sleep(4);
-        if constexpr (N > 1)
-            if (team_load(mine + (2 * N - 1) * places) >> 32 != tag) // the word stored last
-                continue;
-        there = true;
-#pragma unroll
-        for (int k = 0; k < N; ++k)
-        {
-            const unsigned long long lo = team_load(mine + 2 * k * places), hi = team_load(mine + (2 * k + 1) * places);
-            v[k] = __longlong_as_double(hi << 32 | (lo & 0xffffffffull));
-            there = there && lo >> 32 == tag && hi >> 32 == tag;
-        }
+        there = team_look(at, places, tag, v);
     }
     return there;
 }

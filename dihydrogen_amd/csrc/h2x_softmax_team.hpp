@@ -140,20 +140,17 @@ __device__ __forceinline__ double inst_exchange(double part, const InstTeam& g, 
         return r;
     };
     if (t == 0)
-    {
-        const double own[1] = {part};
-        team_put<1>(words, kInstMembers, member, tag, own);
-    }
-    double s[1] = {0.0}; // less than any maximum
+        team_put(words, kInstMembers, member, tag, part);
+    double s = 0.0; // less than any maximum
     if (wave < kChunks) // uniform
     {
-        const bool there = !reads || team_get<1>(words, kInstMembers, mine, tag, g.max_polls, s);
+        const bool there = !reads || team_get(words + mine, kInstMembers, tag, g.max_polls, &s);
         if (!there)
-            s[0] = 0.0;
+            s = 0.0;
         const unsigned long long late = __ballot(!there);
         if (lane == 0)
             shared.late[WHICH][wave] = late;
-        leave_wave(s[0]);
+        leave_wave(s);
     }
     __syncthreads();
     unsigned long long late = shared.late[WHICH][0];
@@ -168,11 +165,11 @@ __device__ __forceinline__ double inst_exchange(double part, const InstTeam& g, 
                 continue;
             const double r = inst_partial<TEAM, SUM>(recompute(m), shared.again);
             if (t == m * kChunks)
-                s[0] = r;
+                s = r;
             __syncthreads(); // shared.again is written again
         }
         if (wave < kChunks)
-            leave_wave(s[0]);
+            leave_wave(s);
         __syncthreads();
     }
     return total();
