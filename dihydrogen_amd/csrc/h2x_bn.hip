@@ -2838,7 +2838,10 @@ constexpr uint32_t kFewestMembers = 16, kFewestLarger = 128;
 // halos 1.2 % (2402; doubles 0.3 and 1.2).  Rules on the number of workgroups alone made it 0.9 % longer, with
 // halos 2.5, and more where the last round is nearly empty or members are mostly padding (forward, N 4, C 16, 96 x 63 x 84,
 // 2000 members of 64 KB, 66 us, as now 53; doubles, forward, backward, N 184, C 91, 23 x 26 with a halo of 1 64, 105 and 57, 85;
-// N 160, C 133, 23 x 19 with a halo of 1 67, 112 and 58, 81).
+// N 160, C 133, 23 x 19 with a halo of 1 67, 112 and 58, 81).  That was with four barriers between a member's last load and its
+// first store; with the two of now the rounds and waits of teams cost less than these constants say, and two launches are named
+// where teams are level (N 4, C 64, 64^3 with a halo of 1, forward in two launches, as named, 317, by teams 319; going over one
+// set 295 both; N 8, C 64, 30^3, by teams, as named, 74.5, forward in two launches 78.5).
 struct PassCost
 {
     float wait; // of a round, for a team of 64
