@@ -84,3 +84,54 @@ def test_one_layer_on_two_streams_at_once():
         for out in outs[:calls]:
             for a, b in zip([y.data, dx.data] + v, [out[0].data, out[1].data] + out[2]):
                 assert torch.equal(a, b)
+
+
+def test_a_graph_makes_no_buffers_of_its_own(monkeypatch):
+    """Captured on another stream than the warm-up's: the replays and eager calls between them share one state, cleared once."""
+    import torch
+    from dihydrogen_amd import layers
+    from dihydrogen_amd.layers import BatchNormalization, Softmax, SoftmaxMode
+    from dihydrogen_amd.tensor import Distribution, LocaleVirtual, Tensor
+    g = torch.Generator(device="cuda").manual_seed(5)
+    dist, c = Distribution.make_localized_distribution(4), 128
+    x, dy, y, dx = (Tensor([56, 56, c, 16], LocaleVirtual(0, 1), dist).allocate() for _ in range(4))
+    sx, sy, sdx = (Tensor([128, 128, 21, 2], LocaleVirtual(0, 1), dist).allocate() for _ in range(3))
+    v = [torch.zeros(c, device="cuda") for _ in range(8)]
+    scale, bias = torch.full((c,), 1.25, device="cuda"), torch.full((c,), -0.5, device="cuda")
+    bn, sm = BatchNormalization(4, 0.9, 1e-5), Softmax()
+    sm.setup(sx, SoftmaxMode.INSTANCE)
+
+    def step():
+        bn.forward(x, *v[:4], scale, bias, y, True)
+        bn.backward(x, dy, *v[:2], scale, *v[4:], dx)
+        sm.forward(sx, sy)
+        sm.backward(sy, sx, sdx)
+
+    def fresh():
+        for t in (x, dy, sx):
+            t.data.normal_(0.5, 2, generator=g)
+        for t in v:
+            t.zero_()
+
+    fresh()
+    step()
+    torch.cuda.synchronize()
+    assert bn._state is not None and sx.layout.instance_state_bytes > 0
+    made, device_buffer = [], layers._device_buffer
+    monkeypatch.setattr(layers, "_device_buffer", lambda *a, **k: made.append(a) or device_buffer(*a, **k))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        step()
+    assert not made
+    for _ in range(4):
+        fresh()
+        graph.replay()
+        torch.cuda.synchronize()
+        outputs = [t.data for t in (y, dx, sy, sdx)] + v
+        got = [t.clone() for t in outputs]
+        for t in v:
+            t.zero_()
+        step()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, outputs))
+    assert not made
