@@ -339,8 +339,8 @@ def calls():
             raise H2XError("_h2xcall.so is missing: build it with `make -C dihydrogen_amd/csrc` "
                            "(or __graft_entry__.build()); there is no fallback path") from e
         import torch
-        from .tensor import GET_BASE_PTR, Tensor
-        _h2xcall.pointer_types(torch.Tensor, Tensor, GET_BASE_PTR)
+        from .tensor import BASE_PTR_PARTS, Tensor
+        _h2xcall.pointer_types(torch.Tensor, Tensor, *BASE_PTR_PARTS)
         _calls = _h2xcall
     return _calls
 

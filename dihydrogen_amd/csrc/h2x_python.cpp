@@ -25,7 +25,8 @@ namespace
 
 PyObject *s_data_ptr = nullptr, *s_get_base_ptr = nullptr, *s_data = nullptr, *s_base_bytes = nullptr; // interned names
 PyTypeObject *s_torch_tensor = nullptr, *s_local_tensor = nullptr;
-PyObject* s_base_ptr_method = nullptr; // of s_local_tensor
+PyObject *s_base_ptr_method = nullptr, *s_base_bytes_property = nullptr; // of s_local_tensor
+unsigned int s_known_version = 0;
 
 bool as_address(PyObject* address, void** out)
 {
@@ -42,42 +43,52 @@ bool address_by(PyObject* method, PyObject* o, void** out)
     return ok;
 }
 
-// Whether o is a local tensor of the very class whose get_base_ptr() is known, replaced on neither the class nor the
-// object.  (Two look-ups in dictionaries; to make the bound method and compare it took twice as long.)
-bool has_known_base(PyObject* o)
+// Whether the class of local tensors still reads `data` and `base_bytes` as it did and has the get_base_ptr() that is known.
+// A class that nobody has changed since it was looked at has its version tag still.
+bool class_is_known()
 {
-    if (Py_TYPE(o) != s_local_tensor
-        || PyDict_GetItemWithError(s_local_tensor->tp_dict, s_get_base_ptr) != s_base_ptr_method)
+    PyTypeObject* const t = s_local_tensor;
+    const bool valid = PyType_HasFeature(t, Py_TPFLAGS_VALID_VERSION_TAG);
+    if (valid && t->tp_version_tag == s_known_version)
+        return true;
+    if (t->tp_getattro != PyObject_GenericGetAttr
+        || PyDict_GetItemWithError(t->tp_dict, s_get_base_ptr) != s_base_ptr_method
+        || PyDict_GetItemWithError(t->tp_dict, s_base_bytes) != s_base_bytes_property
+        || PyDict_GetItemWithError(t->tp_dict, s_data))
         return false;
-    PyObject** const own = _PyObject_GetDictPtr(o);
-    return !own || !*own || !PyDict_GetItemWithError(*own, s_get_base_ptr);
+    if (valid)
+        s_known_version = t->tp_version_tag;
+    return true;
 }
 
-// What that get_base_ptr() returns: data.data_ptr() + base_bytes.
-bool base_of(PyObject* o, void** out)
+// What the get_base_ptr() of a local tensor of that very class returns: data.data_ptr() + base_bytes, read from the object's
+// dictionary (three look-ups; by way of attributes 40 ns more).  0: not such a tensor, or not yet; -1: an exception is set.
+int base_of(PyObject* o, void** out)
 {
-    PyObject* const data = PyObject_GetAttr(o, s_data);
-    if (!data)
-        return false;
+    if (Py_TYPE(o) != s_local_tensor || !class_is_known())
+        return 0;
+    PyObject** const own = _PyObject_GetDictPtr(o);
+    if (!own || !*own || PyDict_GetItemWithError(*own, s_get_base_ptr)) // (replaced on the object)
+        return 0;
+    PyObject *const data = PyDict_GetItemWithError(*own, s_data), *const bytes = PyDict_GetItemWithError(*own, s_base_bytes);
+    if (!data || !bytes)
+        return 0;
+    const Py_ssize_t offset = PyLong_AsSsize_t(bytes);
+    if (offset == -1 && PyErr_Occurred())
+        return -1;
+    Py_INCREF(data);
     const bool ok = address_by(s_data_ptr, data, out);
     Py_DECREF(data);
     if (!ok)
-        return false;
-    PyObject* const bytes = PyObject_GetAttr(o, s_base_bytes);
-    if (!bytes)
-        return false;
-    const Py_ssize_t offset = PyLong_AsSsize_t(bytes);
-    Py_DECREF(bytes);
-    if (offset == -1 && PyErr_Occurred())
-        return false;
+        return -1;
     *out = reinterpret_cast<void*>(reinterpret_cast<uintptr_t>(*out) + offset);
-    return true;
+    return 1;
 }
 
 bool address_of(PyObject* o, void** out)
 {
-    if (has_known_base(o))
-        return base_of(o, out);
+    if (const int known = base_of(o, out))
+        return known > 0;
     if (s_torch_tensor && PyObject_TypeCheck(o, s_torch_tensor))
         return address_by(s_data_ptr, o, out);
     PyObject* const method = PyObject_GetAttr(o, s_get_base_ptr);
@@ -162,18 +173,20 @@ struct Entry<F>
     }
 };
 
-// pointer_types(torch.Tensor, the class of local tensors, its get_base_ptr)
+// pointer_types(torch.Tensor, the class of local tensors, its get_base_ptr, its base_bytes)
 PyObject* pointer_types(PyObject*, PyObject* const* args, Py_ssize_t nargs)
 {
-    if (nargs != 3 || !PyType_Check(args[0]) || !PyType_Check(args[1]))
-        return PyErr_Format(PyExc_TypeError, "two types and a function");
+    if (nargs != 4 || !PyType_Check(args[0]) || !PyType_Check(args[1]))
+        return PyErr_Format(PyExc_TypeError, "two types, a function and a property");
     PyObject* const before[] = {reinterpret_cast<PyObject*>(s_torch_tensor), reinterpret_cast<PyObject*>(s_local_tensor),
-                                s_base_ptr_method};
+                                s_base_ptr_method, s_base_bytes_property};
     for (Py_ssize_t i = 0; i < nargs; ++i)
         Py_INCREF(args[i]);
     s_torch_tensor = reinterpret_cast<PyTypeObject*>(args[0]);
     s_local_tensor = reinterpret_cast<PyTypeObject*>(args[1]);
     s_base_ptr_method = args[2];
+    s_base_bytes_property = args[3];
+    s_known_version = 0;
     for (PyObject* const o : before)
         Py_XDECREF(o);
     Py_RETURN_NONE;

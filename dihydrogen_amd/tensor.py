@@ -321,5 +321,5 @@ class Tensor:
         return v
 
 
-# what the native module does by itself for a tensor that has no other get_base_ptr() (csrc/h2x_python.cpp)
-GET_BASE_PTR = Tensor.get_base_ptr
+# what the native module does by itself for a tensor that has no others (csrc/h2x_python.cpp)
+BASE_PTR_PARTS = Tensor.get_base_ptr, Tensor.base_bytes

@@ -51,7 +51,7 @@ class Alike:
 
 
 @pytest.mark.parametrize("kind", ["tensor", "derived", "with data_ptr", "alike", "replaced on the object",
-                                  "replaced on the class"])
+                                  "replaced on the class", "offset replaced on the class", "data replaced on the class"])
 def test_the_address_is_what_get_base_ptr_returns(kind, monkeypatch):
     """Shown on the host: a call that reads a geometry, and geometries in the tensor's buffer."""
     # of 64 and, where the interior begins, of 128 channels, one element further on of 256
@@ -72,6 +72,8 @@ def test_the_address_is_what_get_base_ptr_returns(kind, monkeypatch):
     sizes = [needed(capi.F32, 16, t.get_buffer() + i * item) for i in range(3)]
     assert 0 < sizes[0] < sizes[1] < sizes[2]
     o, want = t, 1
+    if kind != "derived":
+        assert [needed(capi.F32, 16, t) for _ in range(2)] == [sizes[1]] * 2  # from here on the class is known as it is
     if kind == "derived":
         monkeypatch.setattr(Derived, "get_base_ptr", lambda self: Tensor.get_base_ptr(self) + item)
         want = 2
@@ -83,7 +85,16 @@ def test_the_address_is_what_get_base_ptr_returns(kind, monkeypatch):
     elif kind == "replaced on the class":
         monkeypatch.setattr(Tensor, "get_base_ptr", lambda self: self.get_buffer() + 2 * item)
         want = 2
+    elif kind == "offset replaced on the class":
+        monkeypatch.setattr(Tensor, "base_bytes", property(lambda self: 2 * item))
+        want = 2
+    elif kind == "data replaced on the class":
+        later = t.data[item:]
+        monkeypatch.setattr(Tensor, "data", property(lambda self: later), raising=False)
+        want = 2
     assert needed(capi.F32, 16, o) == sizes[want]
+    monkeypatch.undo()
+    assert t.data is not None
 
 
 def test_what_has_no_address_is_refused():
