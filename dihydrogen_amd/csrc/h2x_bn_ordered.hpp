@@ -299,6 +299,7 @@ __global__ __launch_bounds__(TEAM, TEAMS ? 4 : 1) void bn_ordered_forward_kernel
     unsigned long long* const state = TEAMS ? states + team_state_at(c) : nullptr;
     uint32_t tag = TEAMS ? team_tag(state) : 0;
     const uint32_t quarter = __builtin_amdgcn_readfirstlane(threadIdx.x / kBlockSize), t = threadIdx.x % kBlockSize;
+    const ChannelParams<T> params(a, c);
     const T* const x = a.x + c * g.map.stride_c;
     const auto place = [&](uint32_t m, int u) {
         const uint32_t p = fastdiv(u / kOrderedBatch, g.group_batches);
@@ -344,14 +345,9 @@ __global__ __launch_bounds__(TEAM, TEAMS ? 4 : 1) void bn_ordered_forward_kernel
     T m, variance;
     sums_to_mean_var(s[0], s[1], a.n, &m, &variance);
     if (member == 0 && threadIdx.x == 0)
-    {
-        a.mean[c] = m;
-        a.var[c] = variance;
-        a.running_mean[c] = fma_t(a.decay, a.running_mean[c], (T(1) - a.decay) * m);
-        a.running_var[c] = fma_t(a.decay, a.running_var[c], (T(1) - a.decay) * variance);
-    }
+        params.store_statistics(a, c, m, variance);
     const T inv_stdev = inv_sqrt_t(variance + a.epsilon);
-    const T sc = a.scale[c], bi = a.bias[c];
+    const T sc = params.scale, bi = params.bias;
     T* const y = a.y + c * g.map.stride_c;
 #pragma unroll
     for (int u = 0; u < K; ++u)

@@ -216,6 +216,7 @@ __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometr
     __shared__ TeamShared<TEAM, 2> shared;
     const uint32_t c = fastdiv(blockIdx.x, g.members);
     const uint32_t member = team_member(blockIdx.x - c * g.members.divisor, g.members.divisor);
+    const ChannelParams<T> params(a, c);
     const T* const x = a.x + c * g.once.stride_c;
     unsigned long long* const state = states + team_state_at(c);
     uint32_t tag = team_tag(state);
@@ -251,14 +252,9 @@ __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometr
     T m, variance;
     sums_to_mean_var(static_cast<T>(s[0]), static_cast<T>(s[1]), a.n, &m, &variance);
     if (member == 0 && threadIdx.x == 0)
-    {
-        a.mean[c] = m;
-        a.var[c] = variance;
-        a.running_mean[c] = fma_t(a.decay, a.running_mean[c], (T(1) - a.decay) * m);
-        a.running_var[c] = fma_t(a.decay, a.running_var[c], (T(1) - a.decay) * variance);
-    }
+        params.store_statistics(a, c, m, variance);
     const T inv_stdev = inv_sqrt_t(variance + a.epsilon);
-    const T sc = a.scale[c], bi = a.bias[c];
+    const T sc = params.scale, bi = params.bias;
     T* const y = a.y + c * g.once.stride_c;
 #pragma unroll
     for (int u = 0; u < K; ++u)
