@@ -1350,6 +1350,8 @@ __global__ __launch_bounds__(kBlockSize) void bn_backprop2_short_kernel(
 
 // ---- whole channels in one workgroup: one launch ------------------------------
 #include "h2x_bn_once.hpp"
+
+#include "h2x_bn_window.hpp"
 // ---- whole channels in several workgroups: one launch ---------------------------
 #include "h2x_bn_team.hpp"
 
@@ -2752,10 +2754,75 @@ bool streamed(const OnceGeometry& g, int n)
     return dense_rows(g) ? g.width * sizeof(float) >= kStreamRow : reach_bytes(g, n) > kHaloedNormalStores;
 }
 
+// ---- windows of neighbouring channels: which calls ---------------------------------
+// Short dense segments (those that are stored normally) of tensors from 21 MiB, whose sets of x, y, dy and dx the memory-side
+// cache does not hold from pass to pass.  Backward a CU holds two workgroups of up to four samples a thread; of seven or
+// eight it holds one, of five and six too, with registers idle.  Where the windows are one round of the chip, or fill the last
+// round, or segments are of up to 40 elements.  Forward + backward in us, by a workgroup a channel and by windows, going round
+// three sets of tensors:
+//   one round: N 128, C 1024, 7 x 7 32.1 and 26.5; N 72, C 1983, 6 x 7 28.4 and 24.8 (four channels); N 104, C 830, 8 x 9 28.5 and 26.3;
+//   N 85, C 593, 11 x 11 28.8 and 26.9; N 256, C 512, 7 x 7, seven samples, 32.4 and 28.0; five samples N 170, C 759, 7 x 8 31.5 and 34.6;
+//   rounds filled: N 128, C 2048, 7 x 7 64.1 and 56.3; N 256, C 1024, 7 x 7 67.1 and 58.0; not: N 80, C 1039, 8 x 10 28.6 and 30.4, N 143,
+//   C 1122, 8 x 7 41.7 and 43.3, seven or eight samples N 135, C 669, 10 x 11 44.3 and 49.8, N 125, C 1204, 11 x 9 66.4 and 71.6;
+//   short: N 151, C 1394, 5 x 7 37.6 and 33.9; N 238, C 1325, 5 x 4 33.7 and 29.6; N 141, C 1629, 5 x 6 34.7 and 34.1;
+//   eight samples of whole 64-byte pieces, which share no line halves: N 238, C 1514, 8 x 8 91.3 and 101.0;
+//   smaller tensors: N 128, C 1024, 6 x 6, 19 MB, 18.7 and 19.5; N 64, C 1024, 7 x 7, 13 MB, 15.6 both; N 41, C 1661, 8 x 10, 21.8 MB,
+//   22.1 and 23.8.  Segments of 128 to 160 elements lose up to a third.
+constexpr int kWindowBlock = 1024;
+constexpr size_t kWindowBytes = size_t(21) << 20;
+
+template <int K>
+void issue_window(const WindowGeometry& g, const OnceForward<float>& a, uint32_t blocks, hipStream_t st)
+{
+    launch(bn_window_forward_kernel<float, kWindowBlock, K>, blocks, kWindowBlock, st, g, a);
+}
+template <int K>
+void issue_window(const WindowGeometry& g, const OnceBackward<float>& a, uint32_t blocks, hipStream_t st)
+{
+    launch(bn_window_backward_kernel<float, kWindowBlock, K>, blocks, kWindowBlock, st, g, a);
+}
+
+// False: the call is not for windows.
+template <typename A>
+bool window_launch(const OnceGeometry& o, const A& a, int n, hipStream_t st)
+{
+    // (channels that lie side by side: a window is one run of memory in each sample)
+    if (!dense_rows(o) || streamed(o, n) || o.stride_c < o.width || o.stride_c > 2 * static_cast<int64_t>(o.width)
+        || static_cast<size_t>(o.width) * n * o.num_channels * sizeof(float) < kWindowBytes)
+        return false;
+    WindowGeometry g;
+    g.width = o.width;
+    g.num_channels = o.num_channels;
+    g.samples = static_cast<uint32_t>(n);
+    g.spr = o.spr;
+    g.stride_n = o.stride_n;
+    g.stride_c = o.stride_c;
+    const uint32_t cus = chip_units();
+    for (const uint32_t channels : {4u, 2u})
+    {
+        const uint32_t windows = (o.num_channels + channels - 1) / channels;
+        g.channels = channels;
+        g.slots = make_fastdiv(channels * o.spr.divisor); // up to 128: a segment that is stored normally has 32 vectors
+        g.rows = kWindowBlock / g.slots.divisor;
+        const uint32_t turns = (g.samples + g.rows - 1) / g.rows, blocks = (windows + kNumXcd - 1) / kNumXcd * kNumXcd;
+        const bool few = turns <= 4;
+        const uint32_t round = few ? 2 * cus : cus, rounds = (windows + round - 1) / round;
+        const bool fills = rounds == 1 ? windows >= cus : windows * 16 >= rounds * round * 15;
+        if (few && (fills || (o.width <= 40 && windows >= cus)))
+            issue_window<4>(g, a, blocks, st);
+        else if (channels == 2 && (turns == 7 || turns == 8) && fills && o.width % 16 != 0)
+            issue_window<8>(g, a, blocks, st);
+        else
+            continue;
+        return true;
+    }
+    return false;
+}
+
 template <typename A>
 bool once_launch(const OnceGeometry& g, const A& a, int n, hipStream_t st)
 {
-    return streamed(g, n) ? once_launch<true>(g, a, st) : once_launch<false>(g, a, st);
+    return window_launch(g, a, n, st) || (streamed(g, n) ? once_launch<true>(g, a, st) : once_launch<false>(g, a, st));
 }
 
 // ---- whole channels in several workgroups: which calls, which team ---------------
