@@ -61,11 +61,25 @@ constexpr int kRanksPerTurn = 2;
 // on 4 x 2, 5,500 rows: 9.4 and 11.1).
 constexpr int64_t kLineRows = 4096;
 
+// One end of a row of a rank, halo cell 0: where its values come from.
+struct RowEnd
+{
+    char* from;     // halo cell 0 of row 0 lies here: at the neighbour's other end, without one at this end of this rank
+    uint32_t pitch; // elements of a row there
+    uint32_t filled; // there is a neighbour
+};
+
 // Whole words throughout: a byte cannot be read through the scalar cache, and a
-// workgroup spends most of its time before its first access on what it reads here.
+// workgroup spends most of its time before its first access on what it reads here.  What can be
+// followed on the host is: the rank that a region's cells come from, and the neighbours along a row.  (A chain of a
+// dozen loads, some of them through the vector memory, to one of five scalar ones, us, exchange or clear and exchange: 4 x 64 x
+// 57 x 57 on 2 x 2 6.95 -> 6.55, 3 x 40 x 127 x 327 on 2 x 4, halos of 2 6.23 -> 5.66, 2 x 97 x 187 x 181 on 2 x 2 5.25 -> 4.80,
+// 3 x 50 x 16 x 36 x 72 on 2 x 4, halos of 3 26.3 -> 24.9.  Asking for all of the arguments' lines at once before the chain gave no more.)
 struct Rank
 {
     char* tensor;                 // start of the real allocation
+    RowEnd end[2];
+    uint32_t source[kMaxSpatial]; // by the digit of dimension 2, eight bits by that of dimension 1: see source_of()
     int32_t local[kMaxSpatial];   // interior extents
     int32_t peer[kMaxSpatial][2]; // rank of the neighbour, or -1
     FastDiv units;                // by vectors (or elements) of an interior row
@@ -76,7 +90,6 @@ struct Rank
 
 struct Args
 {
-    Rank rank[kMaxRanks];
     uint32_t first[kMaxRegions]; // first workgroup of a region (beyond the last one: none)
     uint32_t code[kMaxRegions];  // ends + 4 * digit of dimension 1 + 16 * digit of dimension 2;
                                  // digits: 0 interior, 1 lower, 2 upper halo
@@ -89,36 +102,59 @@ struct Args
     int32_t seam[kMaxRanks];       // the lower rank of each
     int32_t width[kMaxSpatial];
     uint32_t outer; // channels x samples
+    Rank rank[kMaxRanks];
 };
 
-// Cells of a rank in dimension d (1 or 2) of a region: extent, and the start in
-// the destination and - stepping to `src`, where there is a neighbour - in the
-// source.
-template <bool CLEAR>
-__host__ __device__ __forceinline__ void along(const Args& a, const Rank& me, int d, int digit, int* src, bool* moved,
-                                               FastDiv* div, uint32_t* to, uint32_t* from)
+// The rank that the cells of a region come from, four bits, and in which dimensions it is another one.
+constexpr uint32_t kSourceRank = 15, kStepped = 8; // bit 4 for dimension 1, bit 5 for dimension 2
+constexpr uint32_t kSteppedAny = 3 * 2 * kStepped;
+
+// Start of a region's cells in dimension d (1 or 2) of a rank of so many interior cells, and where
+// they start in the neighbour `src` they come from: the lower halo is its last interior
+// cells, the upper one its first.
+__host__ __device__ __forceinline__ uint32_t region_start(int w, int local, uint32_t digit)
 {
-    const int w = a.width[d], local = me.local[d];
-    *div = digit == 0 ? me.extent[d - 1] : a.halo[d];
-    *to = digit == 0 ? w : digit == 1 ? 0 : w + local;
-    *from = *to;
-    if (digit == 0)
-        return;
-    if constexpr (CLEAR)
-    {
-        *moved = *moved || (me.clear >> (2 * d + digit - 1) & 1);
-    }
-    else
-    {
-        const int p = a.rank[*src].peer[d][digit - 1];
-        if (p >= 0)
-        {
-            *src = p;
-            *moved = true;
-            // the lower halo is the neighbour's last interior cells, the upper one its first
-            *from = digit == 1 ? a.rank[p].local[d] : w;
-        }
-    }
+    return digit == 0 ? w : digit == 1 ? 0 : w + local;
+}
+__host__ __device__ __forceinline__ uint32_t source_start(int w, int local, uint32_t digit, bool stepped)
+{
+    return !stepped ? region_start(w, local, digit) : digit == 1 ? local : w;
+}
+
+// The same value, in a scalar register (all lanes hold it): two values that are read by scalar loads
+// stay two, instead of one vector load from either place.
+__host__ __device__ __forceinline__ uint32_t in_scalar(uint32_t v)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_readfirstlane(v);
+#else
+    return v;
+#endif
+}
+__host__ __device__ __forceinline__ uint64_t in_scalar(const char* p)
+{
+    const uint64_t v = reinterpret_cast<uintptr_t>(p);
+    return static_cast<uint64_t>(in_scalar(static_cast<uint32_t>(v >> 32))) << 32 | in_scalar(static_cast<uint32_t>(v));
+}
+template <typename T>
+__host__ __device__ __forceinline__ const T* global_place(uint64_t v)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    return (const T*) reinterpret_cast<const T __attribute__((address_space(1)))*>(v);
+#else
+    return reinterpret_cast<const T*>(v);
+#endif
+}
+
+// The loads of a turn go out one after another: what a thread loads together, twice the lines of memory
+// between their load and their store, is slower where the line is all that bounds (N x C x extents on a grid,
+// us, together and so: 4 x 3 x 314 x 77 x 155 on 4 x 1 x 2, periodic 35.9 and 33.1; 5 x 4 x 99 x 61 x 92 on 2 x 1 x 2, halos
+// of 3 16.9 and 15.8; 15 x 11 x 15 x 25 x 18 on 2^3, halos of 2 12.7 and 12.0) and no faster elsewhere.
+__host__ __device__ __forceinline__ void one_by_one()
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    __builtin_amdgcn_s_waitcnt(0x0f70); // vector memory only
+#endif
 }
 
 template <typename T, bool CLEAR, typename Mem>
@@ -141,12 +177,15 @@ __host__ __device__ __forceinline__ void body(const Args& a, uint32_t block, uin
     const int r = static_cast<int>((block - first - local_block * turns.divisor) * (ends ? a.line : 1));
     const Rank& me = a.rank[r]; // ends: the first one of its line
 
-    int src = r;
-    bool moved = false; // some dimension has a neighbour to copy from (CLEAR: a strip to clear)
-    FastDiv div_y, div_z;
-    uint32_t y_to, z_to, y_from, z_from;
-    along<CLEAR>(a, me, 1, code >> 2 & 3, &src, &moved, &div_y, &y_to, &y_from);
-    along<CLEAR>(a, me, 2, code >> 4, &src, &moved, &div_z, &z_to, &z_from);
+    const uint32_t digit_y = code >> 2 & 3, digit_z = code >> 4;
+    const FastDiv div_y = digit_y == 0 ? me.extent[0] : a.halo[1], div_z = digit_z == 0 ? me.extent[1] : a.halo[2];
+    // what of it lies in a strip that has a neighbour to copy from (CLEAR: that is cleared) along dimension 1 or 2
+    const uint32_t source = CLEAR ? static_cast<uint32_t>(r) : me.source[digit_z] >> (8 * digit_y);
+    const uint32_t src = CLEAR ? r : source & kSourceRank; // ends: the first one of a line
+    const bool moved = CLEAR ? (digit_y && (me.clear >> (1 + digit_y) & 1)) || (digit_z && (me.clear >> (3 + digit_z) & 1))
+                             : (source & kSteppedAny) != 0;
+    const Rank& from_rank = a.rank[src];
+    const uint32_t y_to = region_start(a.width[1], me.local[1], digit_y), z_to = region_start(a.width[2], me.local[2], digit_z);
     const FastDiv div_x = ends ? a.both_ends : me.units;
     const uint32_t at = local_block * kBlock + thread;
     if (at >= div_y.divisor * div_z.divisor * a.outer * div_x.divisor || (!ends && !moved))
@@ -159,13 +198,18 @@ __host__ __device__ __forceinline__ void body(const Args& a, uint32_t block, uin
     const uint32_t z = yz - o * div_z.divisor;
     // rows of the real tensors (whose elements are fewer than 2^31)
     const uint32_t w = a.width[0];
-    auto real = [&](int q, int d) { return static_cast<uint32_t>(a.rank[q].local[d] + 2 * a.width[d]); };
-    const uint32_t row_to = (o * real(r, 2) + z_to + z) * real(r, 1) + y_to + y;
-    const uint32_t row_from = (o * real(src, 2) + z_from + z) * real(src, 1) + y_from + y;
+    const auto real = [&](const Rank& q, int d) { return static_cast<uint32_t>(q.local[d] + 2 * a.width[d]); };
+    const uint32_t row_to = (o * real(me, 2) + z_to + z) * real(me, 1) + y_to + y;
+    uint32_t row_from = row_to;
+    if constexpr (!CLEAR)
+        row_from = (o * real(from_rank, 2)
+                    + source_start(a.width[2], from_rank.local[2], digit_z, source & 4 * kStepped) + z)
+                       * real(from_rank, 1)
+                   + source_start(a.width[1], from_rank.local[1], digit_y, source & 2 * kStepped) + y;
     if (!ends)
     {
-        T* const to = reinterpret_cast<T*>(me.tensor) + row_to * real(r, 0) + w;
-        const T* const from = reinterpret_cast<const T*>(a.rank[src].tensor) + row_from * real(src, 0) + w;
+        T* const to = reinterpret_cast<T*>(me.tensor) + row_to * real(me, 0) + w;
+        const T* const from = reinterpret_cast<const T*>(from_rank.tensor) + row_from * real(from_rank, 0) + w;
         if (me.vectors)
         {
             x *= VEC;
@@ -185,8 +229,7 @@ __host__ __device__ __forceinline__ void body(const Args& a, uint32_t block, uin
         return;
     }
     // The ends of a row in every rank of the line: the lower end's cells, then the upper end's, then
-    // the next row's, so that what neighbouring lanes write at a row seam lies side by side.  `src` is
-    // the first rank of the line that the other dimensions step to.
+    // the next row's, so that what neighbouring lanes write at a row seam lies side by side.
     const bool upper = x >= w;
     const uint32_t j = upper ? x - w : x;
 #pragma unroll 1
@@ -207,17 +250,17 @@ __host__ __device__ __forceinline__ void body(const Args& a, uint32_t block, uin
             }
             else
             {
-                // from the neighbour's other end of the row; without one from the same end, halo to halo
-                const Rank& same = a.rank[src + base + i];
-                const int lo = same.peer[0][0], hi = same.peer[0][1];
-                const Rank& below = a.rank[lo >= 0 ? lo : src + base + i];
-                const Rank& above = a.rank[hi >= 0 ? hi : src + base + i];
-                live[i] = moved || (upper ? hi : lo) >= 0;
-                const uint32_t at_lo = lo >= 0 ? below.local[0] : 0, at_hi = w + (hi >= 0 ? 0 : above.local[0]);
-                const uint32_t from = row_from * ((upper ? above.local[0] : below.local[0]) + 2 * w)
-                                      + (upper ? at_hi : at_lo) + j;
+                const RowEnd& lo = a.rank[src + base + i].end[0];
+                const RowEnd& hi = a.rank[src + base + i].end[1];
+                const uint64_t lo_from = in_scalar(lo.from), hi_from = in_scalar(hi.from);
+                const uint32_t lo_pitch = in_scalar(lo.pitch), hi_pitch = in_scalar(hi.pitch);
+                const uint32_t lo_filled = in_scalar(lo.filled), hi_filled = in_scalar(hi.filled);
+                live[i] = moved || (upper ? hi_filled : lo_filled) != 0;
                 if (live[i])
-                    v[i] = mem.load1(reinterpret_cast<const T*>(upper ? above.tensor : below.tensor) + from);
+                    v[i] = mem.load1(global_place<T>(upper ? hi_from : lo_from)
+                                     + (row_from * (upper ? hi_pitch : lo_pitch) + j));
+                if (i + 1 < kRanksPerTurn)
+                    one_by_one();
             }
         }
 #pragma unroll
@@ -600,6 +643,44 @@ bool order_into_lines(Args* a, int num_ranks)
     return true;
 }
 
+// Follows the neighbours of ranks that lie in lines: where a region's cells and a row's ends come from.
+void resolve_sources(Args* a, int num_ranks, int elem_size)
+{
+    for (int r = 0; r < num_ranks; ++r)
+    {
+        Rank& k = a->rank[r];
+        for (uint32_t dz = 0; dz < 3; ++dz)
+        {
+            k.source[dz] = 0;
+            for (uint32_t dy = 0; dy < 3; ++dy)
+            {
+                uint32_t src = static_cast<uint32_t>(r), stepped = 0;
+                for (int d = 1; d < kMaxSpatial; ++d)
+                {
+                    const uint32_t digit = d == 1 ? dy : dz;
+                    const int p = digit ? a->rank[src].peer[d][digit - 1] : -1;
+                    if (p >= 0)
+                    {
+                        src = static_cast<uint32_t>(p);
+                        stepped |= kStepped << d;
+                    }
+                }
+                k.source[dz] |= (src | stepped) << (8 * dy);
+            }
+        }
+        for (int side = 0; side < 2; ++side)
+        {
+            const int p = k.peer[0][side];
+            const Rank& q = p >= 0 ? a->rank[p] : k;
+            // the neighbour's other end, or this end: of {halo, interior, halo}, cells 0, w, local or w + local
+            const int64_t cell = side == 0 ? (p >= 0 ? q.local[0] : 0) : a->width[0] + (p >= 0 ? 0 : q.local[0]);
+            k.end[side].from = q.tensor + cell * elem_size;
+            k.end[side].pitch = static_cast<uint32_t>(q.local[0] + 2 * a->width[0]);
+            k.end[side].filled = p >= 0;
+        }
+    }
+}
+
 template <bool CLEAR>
 int run(h2x_dtype dtype, const h2x_halo_grid* h, int only_unfilled, h2x_stream_t stream)
 {
@@ -616,6 +697,8 @@ int run(h2x_dtype dtype, const h2x_halo_grid* h, int only_unfilled, h2x_stream_t
         return H2X_ERR_INVALID_ARGUMENT;
     if (!order_into_lines(&a, h->num_ranks))
         return H2X_ERR_UNSUPPORTED;
+    if constexpr (!CLEAR)
+        resolve_sources(&a, h->num_ranks, es);
     // Regions with the same work for every rank: blocks for the largest rank.
     int num_regions = 0;
     uint64_t blocks = 0;
