@@ -79,7 +79,7 @@ struct Rank
 {
     char* tensor;                 // start of the real allocation
     RowEnd end[2];
-    uint32_t source[kMaxSpatial]; // by the digit of dimension 2, eight bits by that of dimension 1: see source_of()
+    uint32_t source[kMaxSpatial]; // by the digit of dimension 2, eight bits by that of dimension 1: see kSourceRank
     int32_t local[kMaxSpatial];   // interior extents
     int32_t peer[kMaxSpatial][2]; // rank of the neighbour, or -1
     FastDiv units;                // by vectors (or elements) of an interior row

@@ -17,6 +17,7 @@
 
 #include <cfloat>
 #include <cmath>
+#include <limits>
 #include <type_traits>
 
 namespace h2x
@@ -108,9 +109,7 @@ struct Pack
 };
 
 // The wave of a thread, as the scalar that it is: which channels a wave takes, and where they
-// lie, is then worked out once a wave and not in every lane (1000 vector instructions a wave of
-// softmax_fwd_split_kernel with 24 channels, 560 with it; forward + backward, us: N 16, C 500, 48 x 48 83.0 -> 73.0, N 2,
-// C 900, 30 x 30 72 -> 64, N 30, C 179, 43 x 43 50.0 -> 47.4, N 4, C 150, 65 x 97 19.4 -> 18.6).
+// lie, is then worked out once a wave and not in every lane.
 __device__ __forceinline__ int wave_index()
 {
     return __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
@@ -156,6 +155,61 @@ __device__ __forceinline__ bool tile_pixels(const WideTiles& t, int num_channels
     const size_t first = static_cast<size_t>(tile - n * t.per_sample.divisor) * LANES;
     return lane_pixels<VEC>(first + threadIdx.x % LANES, num_channels, spatial, flat_samples, base, sample)
            && sample < t.samples;
+}
+
+// What a workgroup of the split kernels serves: the first element of its tile, the same for all its threads,
+// and from there the bytes to the lane's first pixel (of a lane without pixels: 0, which can be read).
+struct TilePlace
+{
+    size_t first;
+    uint32_t offset;
+    bool active; // the lane has pixels
+    bool any;    // the tile has
+};
+
+template <typename T, int VEC, int LANES>
+__device__ __forceinline__ TilePlace tile_place(const WideTiles& t, int num_channels, size_t spatial, int flat_samples)
+{
+    TilePlace p;
+    const unsigned int tile = xcd_contiguous(blockIdx.x, gridDim.x);
+    const unsigned int lane = threadIdx.x % LANES;
+    const size_t sample_size = num_channels * spatial;
+    if (flat_samples > 0)
+    {
+        const unsigned int size = static_cast<unsigned int>(spatial), pixel = tile * LANES + lane;
+        const unsigned int n0 = tile * LANES / size, n = pixel / size;
+        p.first = n0 * sample_size + (tile * LANES - n0 * size);
+        p.any = n0 < static_cast<unsigned int>(flat_samples);
+        p.active = n < static_cast<unsigned int>(flat_samples);
+        const size_t at = n * sample_size + (pixel - n * size);
+        p.offset = p.active ? static_cast<uint32_t>(at - p.first) * sizeof(T) : 0;
+        return p;
+    }
+    const unsigned int n = fastdiv(tile, t.per_sample), sample = blockIdx.y + n;
+    const size_t pixel = static_cast<size_t>(tile - n * t.per_sample.divisor) * (LANES * VEC);
+    p.first = sample * sample_size + pixel;
+    p.any = sample < t.samples && pixel < spatial;
+    p.active = pixel + lane * VEC < spatial;
+    p.offset = p.active ? lane * (VEC * sizeof(T)) : 0;
+    return p;
+}
+
+// The element `offset` bytes behind p, which all lanes share: scalar registers and one vector register address it.
+template <typename T>
+__device__ __forceinline__ T* element(T* p, uint32_t offset)
+{
+    using C = std::conditional_t<std::is_const_v<T>, const char, char>;
+    return reinterpret_cast<T*>(reinterpret_cast<C*>(p) + offset);
+}
+
+// The larger of the two, b where a is no number (b is one).
+__device__ __forceinline__ float larger(float a, float b)
+{
+    return __builtin_amdgcn_fmed3f(a, b, __builtin_inff());
+}
+__device__ __forceinline__ double larger(double a, double b)
+{
+    return a > b ? a : b;
 }
 
 // Cache policy.  The backward pass reads the y that the forward pass has written; x and dy are read
@@ -481,7 +535,15 @@ __device__ __forceinline__ T pixel_combine(T v, const F& f)
 // Where there are few tiles, a pixel is for 64 / LANES lanes of a wave instead of one: a workgroup serves LANES
 // pixels, lane l of wave g the channels (g + k * WAVES) * 64 / LANES + l / LANES, the chain is that many times shorter
 // and there are as many more workgroups, for rows of 64 or 128 bytes (see launch_split_for).
-template <typename T, int VEC, int CPW, int WAVES, int LANES, bool STREAM>
+// The chain of a wave counts: 19 vector and 6 scalar instructions a channel forward, of which the exponential takes 13.  So the first
+// CERTAIN channels of a wave, which the smallest channel count of the variant has, are not asked for; a channel that is not there is
+// -infinity (backward 0), with no further question; lanes without pixels work on the tile's first one and store
+// nothing; and addresses are a running scalar pointer and a lane's offset in bytes.  Asking before each load, term
+// and store, with addresses of 64 bits a lane (23 and 22 instructions, backward 13 and 30 with registers spilled), forward + backward in
+// us -> so: N 4, C 150, 65 x 97 17.5 -> 16.8; N 2, C 209, 15 x 15 6.85 -> 5.75; N 5, C 308, 56 x 52 21.8 -> 20.6; N 2, C 322,
+// 75 x 110 26.7 -> 24.0; N 4, C 431, 99 x 126 111 -> 102; doubles N 4, C 472, 49 x 44 47.3 -> 43.6; of 47 calls the mean
+// is 0.950, and those bound by memory are level (N 1, C 39, 316 x 354 18.4 and 18.5, N 13, C 47, 220 x 134 63.6 and 64.5).
+template <typename T, int VEC, int CPW, int CERTAIN, int WAVES, int LANES, bool STREAM>
 __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
     const T* __restrict__ x, T* __restrict__ y, int num_channels, size_t spatial, int flat_samples,
     const WideTiles tiles)
@@ -491,39 +553,35 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
     constexpr int kApart = kWaveSize / LANES; // channels that a wave takes at once
     const int lane = threadIdx.x % LANES, q = threadIdx.x % kWaveSize / LANES;
     const int g = wave_index();
-    size_t base;
-    const bool active = tile_pixels<VEC, LANES>(tiles, num_channels, spatial, flat_samples, &base);
-    base += q * spatial;
-    const int channels = num_channels - q; // of those that start at this lane's
-    const T* xp = x + base;
-    T* yp = y + base;
+    const TilePlace place = tile_place<T, VEC, LANES>(tiles, num_channels, spatial, flat_samples);
+    if (!place.any) // the whole workgroup
+        return;
+    const uint32_t offset = place.offset + static_cast<uint32_t>(q * spatial * sizeof(T));
+    const size_t first = place.first + g * kApart * spatial, step = WAVES * kApart * spatial;
+    const auto exists = [&](int k) { return k < CERTAIN || (g + k * WAVES) * kApart + q < num_channels; };
     constexpr T kMin = Limits<T>::min_normal;
 
     P v[CPW];
     T mx[VEC], sum[VEC];
+    const T* xp = x + first;
+#pragma unroll
+    for (int k = 0; k < CPW; ++k, xp += step)
+    {
+        if (exists(k))
+            v[k] = P::template load<STREAM>(element(xp, offset));
+        else
+#pragma unroll
+            for (int j = 0; j < VEC; ++j)
+                v[k][j] = -std::numeric_limits<T>::infinity(); // no maximum, and exactly 0 in the sum
+    }
 #pragma unroll
     for (int j = 0; j < VEC; ++j)
     {
         mx[j] = kMin;
-        sum[j] = T(0);
-    }
-    if (active)
-    {
 #pragma unroll
         for (int k = 0; k < CPW; ++k)
-            if ((g + k * WAVES) * kApart < channels)
-                v[k] = P::template load<STREAM>(xp + static_cast<size_t>((g + k * WAVES) * kApart) * spatial);
-#pragma unroll
-        for (int k = 0; k < CPW; ++k)
-            if ((g + k * WAVES) * kApart < channels)
-#pragma unroll
-                for (int j = 0; j < VEC; ++j)
-                    mx[j] = v[k][j] > mx[j] ? v[k][j] : mx[j];
-    }
-#pragma unroll
-    for (int j = 0; j < VEC; ++j)
-    {
-        mx[j] = pixel_combine<LANES>(mx[j], [](T p, T r) { return r > p ? r : p; });
+            mx[j] = larger(v[k][j], mx[j]);
+        mx[j] = pixel_combine<LANES>(mx[j], [](T p, T r) { return larger(p, r); });
         if (q == 0)
             lds[g][lane * VEC + j] = mx[j];
     }
@@ -532,22 +590,21 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
     for (int j = 0; j < VEC; ++j)
 #pragma unroll
         for (int w = 0; w < WAVES; ++w)
-            mx[j] = lds[w][lane * VEC + j] > mx[j] ? lds[w][lane * VEC + j] : mx[j];
+            mx[j] = larger(lds[w][lane * VEC + j], mx[j]);
     __syncthreads();
 
-    if (active)
-    {
 #pragma unroll
-        for (int k = 0; k < CPW; ++k)
-            if ((g + k * WAVES) * kApart < channels)
+    for (int j = 0; j < VEC; ++j)
+        sum[j] = T(0);
 #pragma unroll
-                for (int j = 0; j < VEC; ++j)
-                {
-                    const T e = exp_t(v[k][j] - mx[j]);
-                    v[k][j] = e;
-                    sum[j] += e;
-                }
-    }
+    for (int k = 0; k < CPW; ++k)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j)
+        {
+            const T e = exp_t(v[k][j] - mx[j]);
+            v[k][j] = e;
+            sum[j] += e;
+        }
 #pragma unroll
     for (int j = 0; j < VEC; ++j)
     {
@@ -562,27 +619,24 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
     {
         inv[j] = T(1) / sum_of_waves<T, WAVES>(lds, lane * VEC + j);
     }
-    if (active)
-    {
+    if (!place.active)
+        return;
+    T* yp = y + first;
 #pragma unroll
-        for (int k = 0; k < CPW; ++k)
-            if ((g + k * WAVES) * kApart < channels)
-            {
+    for (int k = 0; k < CPW; ++k, yp += step)
+        if (exists(k))
+        {
 #pragma unroll
-                for (int j = 0; j < VEC; ++j)
-                {
-                    const T r = v[k][j] * inv[j];
-                    v[k][j] = r > kMin ? r : kMin;
-                }
-                P::store(yp + static_cast<size_t>((g + k * WAVES) * kApart) * spatial, v[k]);
-            }
-    }
+            for (int j = 0; j < VEC; ++j)
+                v[k][j] = larger(v[k][j] * inv[j], kMin);
+            P::store(element(yp, offset), v[k]);
+        }
 }
 
 // backward likewise: y and dy of up to WAVES * CPW channels in registers.  All of y is
 // asked for before any of dy: alternating, the wave waited more often (N 4, C 150,
 // 65 x 97 in four waves 15.9 us against 10.2).
-template <typename T, int VEC, int CPW, int WAVES, int LANES, bool STREAM>
+template <typename T, int VEC, int CPW, int CERTAIN, int WAVES, int LANES, bool STREAM>
 __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
     const T* __restrict__ y, const T* __restrict__ dy, T* __restrict__ dx, int num_channels,
     size_t spatial, int flat_samples,
@@ -592,54 +646,38 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
     __shared__ T lds[WAVES][LANES * VEC];
     constexpr int kApart = kWaveSize / LANES; // channels that a wave takes at once
     const int lane = threadIdx.x % LANES, q = threadIdx.x % kWaveSize / LANES;
-    // Of more than 256 channels in floats, a lane a pixel, the index stays a lane's own: as a scalar, the addresses
-    // and the tests of all those channels are scalars too, more than there are (16 waves with 24
-    // channels each spill 31 of them into vector registers, with 48 153; up to 256 channels a wave
-    // of 16 spills two).  us, scalar and so: N 4, C 428, 20 x 26 12.4 -> 8.0, N 2, C 494, 34 x 19
-    // 13.3 -> 8.6 (both in tiles of 16 pixels now), N 8, C 395, 46 x 46 31.5 -> 25.2; 245 drawn sizes 0.94 of the time, the worst
-    // 1.08.  Doubles fill the vector registers first (1.01 to 1.06 of the scalar's time), and the
-    // forward pass, of half the addresses, is faster with the scalar.
-    // With several lanes a pixel the tests are the lanes' own in any case, and the scalar is 4 to 8 % faster, although 24 and 32
-    // channels a lane spill 35 and 77 scalars (scalar and so: N 6, C 270, 20 x 30 4.4 and 4.8 us; N 1, C 512, 90 x 90 10.4 and 11.1;
-    // N 1, C 1000, 50 x 52 8.9 and 9.3, but N 1, C 900, 17 x 13 6.8 and 5.7; in tiles of 32 pixels N 23, C 380, 30 x 33 25.2 and 26.4,
-    // N 1, C 270, 128 x 130 11.9 and 11.7), but for 24 a lane in tiles of 16 (N 8, C 520, 11 x 12 5.1 and 4.6; N 1, C 768,
-    // 70 x 75 12.6 and 12.1).
-    constexpr bool kOwnIndex = sizeof(T) == 4 && (LANES == kWaveSize ? WAVES * CPW > 256 : LANES == 16 && CPW == 24);
-    const int g = kOwnIndex ? static_cast<int>(threadIdx.x / kWaveSize) : wave_index();
-    size_t base;
-    const bool active = tile_pixels<VEC, LANES>(tiles, num_channels, spatial, flat_samples, &base);
-    base += q * spatial;
-    const int channels = num_channels - q; // of those that start at this lane's
-    const T* yp = y + base;
-    const T* gp = dy + base;
-    T* op = dx + base;
+    const int g = wave_index();
+    const TilePlace place = tile_place<T, VEC, LANES>(tiles, num_channels, spatial, flat_samples);
+    if (!place.any) // the whole workgroup
+        return;
+    const uint32_t offset = place.offset + static_cast<uint32_t>(q * spatial * sizeof(T));
+    const size_t first = place.first + g * kApart * spatial, step = WAVES * kApart * spatial;
+    const auto exists = [&](int k) { return k < CERTAIN || (g + k * WAVES) * kApart + q < num_channels; };
     constexpr T kMin = Limits<T>::min_normal;
 
     P yv[CPW], gv[CPW];
+    const auto load = [&](const T* p, P(&v)[CPW], auto stream) {
+#pragma unroll
+        for (int k = 0; k < CPW; ++k, p += step)
+        {
+            if (exists(k))
+                v[k] = P::template load<decltype(stream)::value>(element(p, offset));
+            else
+#pragma unroll
+                for (int j = 0; j < VEC; ++j)
+                    v[k][j] = T(0);
+        }
+    };
+    load(y + first, yv, std::false_type());
+    load(dy + first, gv, std::bool_constant<STREAM>());
     T dp[VEC];
 #pragma unroll
     for (int j = 0; j < VEC; ++j)
+    {
         dp[j] = T(0);
-    if (active)
-    {
 #pragma unroll
         for (int k = 0; k < CPW; ++k)
-            if ((g + k * WAVES) * kApart < channels)
-                yv[k] = P::load(yp + static_cast<size_t>((g + k * WAVES) * kApart) * spatial);
-#pragma unroll
-        for (int k = 0; k < CPW; ++k)
-            if ((g + k * WAVES) * kApart < channels)
-                gv[k] = P::template load<STREAM>(gp + static_cast<size_t>((g + k * WAVES) * kApart) * spatial);
-#pragma unroll
-        for (int k = 0; k < CPW; ++k)
-            if ((g + k * WAVES) * kApart < channels)
-#pragma unroll
-                for (int j = 0; j < VEC; ++j)
-                    dp[j] = fma_t(yv[k][j], gv[k][j], dp[j]);
-    }
-#pragma unroll
-    for (int j = 0; j < VEC; ++j)
-    {
+            dp[j] = fma_t(yv[k][j], gv[k][j], dp[j]);
         dp[j] = pixel_combine<LANES>(dp[j], [](T p, T r) { return p + r; });
         if (q == 0)
             lds[g][lane * VEC + j] = dp[j];
@@ -650,18 +688,18 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
     {
         dp[j] = sum_of_waves<T, WAVES>(lds, lane * VEC + j);
     }
-    if (active)
-    {
+    if (!place.active)
+        return;
+    T* op = dx + first;
 #pragma unroll
-        for (int k = 0; k < CPW; ++k)
-            if ((g + k * WAVES) * kApart < channels)
-            {
+    for (int k = 0; k < CPW; ++k, op += step)
+        if (exists(k))
+        {
 #pragma unroll
-                for (int j = 0; j < VEC; ++j)
-                    yv[k][j] = yv[k][j] > kMin ? yv[k][j] * (gv[k][j] - dp[j]) : T(0);
-                P::template store<STREAM>(op + static_cast<size_t>((g + k * WAVES) * kApart) * spatial, yv[k]);
-            }
-    }
+            for (int j = 0; j < VEC; ++j)
+                yv[k][j] = yv[k][j] > kMin ? yv[k][j] * (gv[k][j] - dp[j]) : T(0);
+            P::template store<STREAM>(element(op, offset), yv[k]);
+        }
 }
 
 // One pixel per sample (the output of a fully connected layer): the channels of
@@ -959,37 +997,41 @@ constexpr int kManySamples = 2048;
 // 29.8 and 34.3.  More channels than the largest tile holds (1024 forward, 768 backward, 1024 where
 // tiles are few; double: 512, or 1024; N 18, C 270, 27 x 40 backward, re-reading 40.3 us, in
 // registers 27.9) take the re-reading kernel.
-template <int VEC, int CPW, int WAVES, int LANES = kWaveSize, bool MAY_STREAM = true, typename T>
+constexpr int kNoSplit = -1000; // not the status of a launch
+
+template <int VEC, int CPW, int CERTAIN, int WAVES, int LANES = kWaveSize, bool MAY_STREAM = true, typename T>
 int launch_split(const T* x, T* y, int n, int c, size_t s, bool stream, hipStream_t st)
 {
+    if (c < CERTAIN * WAVES * (kWaveSize / LANES))
+        return kNoSplit;
     const int flat = VEC == 1 ? flat_samples(n, s) : 0;
     WideTiles tiles;
     const dim3 grid = wide_grid(s, LANES, VEC, n, flat, &tiles);
     if (MAY_STREAM && stream)
-        launch(softmax_fwd_split_kernel<T, VEC, CPW, WAVES, LANES, MAY_STREAM>, grid, WAVES * kWaveSize, st, x, y, c,
+        launch(softmax_fwd_split_kernel<T, VEC, CPW, CERTAIN, WAVES, LANES, MAY_STREAM>, grid, WAVES * kWaveSize, st, x, y, c,
                s, flat, tiles);
     else
-        launch(softmax_fwd_split_kernel<T, VEC, CPW, WAVES, LANES, false>, grid, WAVES * kWaveSize, st, x, y, c, s,
+        launch(softmax_fwd_split_kernel<T, VEC, CPW, CERTAIN, WAVES, LANES, false>, grid, WAVES * kWaveSize, st, x, y, c, s,
                flat, tiles);
     return launch_status();
 }
 
-template <int VEC, int CPW, int WAVES, int LANES = kWaveSize, bool MAY_STREAM = true, typename T>
+template <int VEC, int CPW, int CERTAIN, int WAVES, int LANES = kWaveSize, bool MAY_STREAM = true, typename T>
 int launch_split(const T* y, const T* dy, T* dx, int n, int c, size_t s, bool stream, hipStream_t st)
 {
+    if (c < CERTAIN * WAVES * (kWaveSize / LANES))
+        return kNoSplit;
     const int flat = VEC == 1 ? flat_samples(n, s) : 0;
     WideTiles tiles;
     const dim3 grid = wide_grid(s, LANES, VEC, n, flat, &tiles);
     if (MAY_STREAM && stream)
-        launch(softmax_bwd_split_kernel<T, VEC, CPW, WAVES, LANES, MAY_STREAM>, grid, WAVES * kWaveSize, st, y, dy, dx, c, s,
+        launch(softmax_bwd_split_kernel<T, VEC, CPW, CERTAIN, WAVES, LANES, MAY_STREAM>, grid, WAVES * kWaveSize, st, y, dy, dx, c, s,
                flat, tiles);
     else
-        launch(softmax_bwd_split_kernel<T, VEC, CPW, WAVES, LANES, false>, grid, WAVES * kWaveSize, st, y, dy, dx, c, s,
+        launch(softmax_bwd_split_kernel<T, VEC, CPW, CERTAIN, WAVES, LANES, false>, grid, WAVES * kWaveSize, st, y, dy, dx, c, s,
                flat, tiles);
     return launch_status();
 }
-
-constexpr int kNoSplit = -1000; // not the status of a launch
 
 // The split kernel for 33 channels and more, or kNoSplit.  (Tiles are of 64 pixels; their numbers below are those for 256 CUs.)
 // Forward + backward, us, by such tiles (16 waves up to 256 of them, else 8) -> as now:
@@ -1024,56 +1066,56 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
     const size_t elements = s * c * n, cus = chip_units();
     if (tiles <= cus && c > (kFloat ? 96 : 64) && c <= 1024 && elements * sizeof(T) <= size_t(kFloat ? 16 : 20) << 20)
     {
-        if (c <= 128) return launch_split<1, 4, 8, 16, false>(p..., n, c, s, stream, st);
-        if (c <= 192) return launch_split<1, 6, 8, 16, false>(p..., n, c, s, stream, st);
-        if (c <= 256) return launch_split<1, 8, 8, 16, false>(p..., n, c, s, stream, st);
-        if (c <= 384) return launch_split<1, 12, 8, 16, false>(p..., n, c, s, stream, st);
-        if (c <= 512) return launch_split<1, 16, 8, 16, false>(p..., n, c, s, stream, st);
-        if (c <= 768) return launch_split<1, 24, 8, 16, false>(p..., n, c, s, stream, st);
-        return launch_split<1, 32, 8, 16, false>(p..., n, c, s, stream, st);
+        if (c <= 128) return launch_split<1, 4, 2, 8, 16, false>(p..., n, c, s, stream, st);
+        if (c <= 192) return launch_split<1, 6, 4, 8, 16, false>(p..., n, c, s, stream, st);
+        if (c <= 256) return launch_split<1, 8, 6, 8, 16, false>(p..., n, c, s, stream, st);
+        if (c <= 384) return launch_split<1, 12, 8, 8, 16, false>(p..., n, c, s, stream, st);
+        if (c <= 512) return launch_split<1, 16, 12, 8, 16, false>(p..., n, c, s, stream, st);
+        if (c <= 768) return launch_split<1, 24, 16, 8, 16, false>(p..., n, c, s, stream, st);
+        return launch_split<1, 32, 24, 8, 16, false>(p..., n, c, s, stream, st);
     }
     if constexpr (kForward && kFloat)
     {
         if (tiles > cus && tiles <= cus * 9 / 4 && c > 64 && c <= 256 && !stream)
         {
-            if (c <= 96) return launch_split<1, 6, 4, 16, false>(p..., n, c, s, stream, st);
-            if (c <= 128) return launch_split<1, 8, 4, 16, false>(p..., n, c, s, stream, st);
-            if (c <= 160) return launch_split<1, 10, 4, 16, false>(p..., n, c, s, stream, st);
-            if (c <= 192) return launch_split<1, 12, 4, 16, false>(p..., n, c, s, stream, st);
-            return launch_split<1, 16, 4, 16, false>(p..., n, c, s, stream, st);
+            if (c <= 96) return launch_split<1, 6, 4, 4, 16, false>(p..., n, c, s, stream, st);
+            if (c <= 128) return launch_split<1, 8, 6, 4, 16, false>(p..., n, c, s, stream, st);
+            if (c <= 160) return launch_split<1, 10, 8, 4, 16, false>(p..., n, c, s, stream, st);
+            if (c <= 192) return launch_split<1, 12, 10, 4, 16, false>(p..., n, c, s, stream, st);
+            return launch_split<1, 16, 12, 4, 16, false>(p..., n, c, s, stream, st);
         }
     }
     if (tiles > cus && tiles <= (kFloat && !kForward ? cus * 3 / 2 : cus * 2) && c > 64 && c <= (kFloat ? 384 : 256) && !stream)
     {
         if constexpr (!(kFloat && kForward))
         {
-            if (c <= 128) return launch_split<1, 8, 8, 32, false>(p..., n, c, s, stream, st);
-            if (c <= 192) return launch_split<1, 12, 8, 32, false>(p..., n, c, s, stream, st);
-            if (c <= 256) return launch_split<1, 16, 8, 32, false>(p..., n, c, s, stream, st);
+            if (c <= 128) return launch_split<1, 8, 4, 8, 32, false>(p..., n, c, s, stream, st);
+            if (c <= 192) return launch_split<1, 12, 8, 8, 32, false>(p..., n, c, s, stream, st);
+            if (c <= 256) return launch_split<1, 16, 12, 8, 32, false>(p..., n, c, s, stream, st);
         }
         if constexpr (kFloat)
-            return launch_split<1, 24, 8, 32, false>(p..., n, c, s, stream, st);
+            return launch_split<1, 24, 16, 8, 32, false>(p..., n, c, s, stream, st);
     }
     if constexpr (!kFloat)
     {
         if (c > 512) return kNoSplit;
-        if (c > 384) return launch_split<1, 32, 8, 32>(p..., n, c, s, stream, st);
-        if (c > 256) return launch_split<1, 24, 8, 32>(p..., n, c, s, stream, st);
+        if (c > 384) return launch_split<1, 32, 24, 8, 32>(p..., n, c, s, stream, st);
+        if (c > 256) return launch_split<1, 24, 16, 8, 32>(p..., n, c, s, stream, st);
     }
     if ((tiles <= cus && c > 64) || c > 512)
     {
         if constexpr (kFloat)
         {
-            if (c <= 96) return launch_split<1, 8, 16, kWaveSize, false>(p..., n, c, s, stream, st);
-            if (c <= 384) return launch_split<1, 24, 16>(p..., n, c, s, stream, st);
-            if (c <= 512) return launch_split<1, 32, 16>(p..., n, c, s, stream, st);
-            if (c <= 768) return launch_split<1, 48, 16>(p..., n, c, s, stream, st);
+            if (c <= 96) return launch_split<1, 8, 4, 16, kWaveSize, false>(p..., n, c, s, stream, st);
+            if (c <= 384) return launch_split<1, 24, 6, 16>(p..., n, c, s, stream, st);
+            if (c <= 512) return launch_split<1, 32, 24, 16>(p..., n, c, s, stream, st);
+            if (c <= 768) return launch_split<1, 48, 32, 16>(p..., n, c, s, stream, st);
         }
         else
-            return launch_split<1, 16, 16>(p..., n, c, s, stream, st);
+            return launch_split<1, 16, 4, 16>(p..., n, c, s, stream, st);
         if constexpr (kFloat && kForward)
         {
-            if (c <= 1024) return launch_split<1, 64, 16>(p..., n, c, s, stream, st);
+            if (c <= 1024) return launch_split<1, 64, 48, 16>(p..., n, c, s, stream, st);
         }
         return kNoSplit;
     }
@@ -1081,29 +1123,29 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
     {
         if (v >= 2 && c <= 256 && (s + 2 * kWaveSize - 1) / (2 * kWaveSize) * n >= (kForward ? 2 : 1) * cus)
         {
-            if (c <= 64) return launch_split<2, 8, 8>(p..., n, c, s, stream, st);
-            if (c <= 96) return launch_split<2, 12, 8>(p..., n, c, s, stream, st);
-            if (c <= 128) return launch_split<2, 16, 8>(p..., n, c, s, stream, st);
-            if (c <= 160) return launch_split<2, 20, 8>(p..., n, c, s, stream, st);
-            if (c <= 192) return launch_split<2, 24, 8>(p..., n, c, s, stream, st);
-            if (c <= 224) return launch_split<2, 28, 8>(p..., n, c, s, stream, st);
-            return launch_split<2, 32, 8>(p..., n, c, s, stream, st);
+            if (c <= 64) return launch_split<2, 8, 4, 8>(p..., n, c, s, stream, st);
+            if (c <= 96) return launch_split<2, 12, 8, 8>(p..., n, c, s, stream, st);
+            if (c <= 128) return launch_split<2, 16, 12, 8>(p..., n, c, s, stream, st);
+            if (c <= 160) return launch_split<2, 20, 16, 8>(p..., n, c, s, stream, st);
+            if (c <= 192) return launch_split<2, 24, 20, 8>(p..., n, c, s, stream, st);
+            if (c <= 224) return launch_split<2, 28, 24, 8>(p..., n, c, s, stream, st);
+            return launch_split<2, 32, 28, 8>(p..., n, c, s, stream, st);
         }
     }
     // (floats that are streamed have, with few channels, the pixels for two a lane)
     constexpr bool kStreams96 = !kFloat, kStreams192 = !kFloat || kForward;
-    if (c <= 64) return launch_split<1, 8, 8, kWaveSize, kStreams96>(p..., n, c, s, stream, st);
-    if (c <= 96) return launch_split<1, 12, 8, kWaveSize, kStreams96>(p..., n, c, s, stream, st);
-    if (c <= 128) return launch_split<1, 16, 8, kWaveSize, kStreams192>(p..., n, c, s, stream, st);
-    if (c <= 160) return launch_split<1, 20, 8, kWaveSize, kStreams192>(p..., n, c, s, stream, st);
-    if (c <= 192) return launch_split<1, 24, 8, kWaveSize, kStreams192>(p..., n, c, s, stream, st);
-    if (c <= 224) return launch_split<1, 28, 8>(p..., n, c, s, stream, st);
-    if (c <= 256) return launch_split<1, 32, 8>(p..., n, c, s, stream, st);
+    if (c <= 64) return launch_split<1, 8, 4, 8, kWaveSize, kStreams96>(p..., n, c, s, stream, st);
+    if (c <= 96) return launch_split<1, 12, 8, 8, kWaveSize, kStreams96>(p..., n, c, s, stream, st);
+    if (c <= 128) return launch_split<1, 16, 12, 8, kWaveSize, kStreams192>(p..., n, c, s, stream, st);
+    if (c <= 160) return launch_split<1, 20, 16, 8, kWaveSize, kStreams192>(p..., n, c, s, stream, st);
+    if (c <= 192) return launch_split<1, 24, 20, 8, kWaveSize, kStreams192>(p..., n, c, s, stream, st);
+    if (c <= 224) return launch_split<1, 28, 24, 8>(p..., n, c, s, stream, st);
+    if (c <= 256) return launch_split<1, 32, 28, 8>(p..., n, c, s, stream, st);
     if constexpr (kFloat)
     {
-        if (c <= 384) return launch_split<1, 48, 8>(p..., n, c, s, stream, st);
-        if (c <= 448) return launch_split<1, 56, 8>(p..., n, c, s, stream, st);
-        if (c <= 512) return launch_split<1, 64, 8>(p..., n, c, s, stream, st);
+        if (c <= 384) return launch_split<1, 48, 32, 8>(p..., n, c, s, stream, st);
+        if (c <= 448) return launch_split<1, 56, 48, 8>(p..., n, c, s, stream, st);
+        if (c <= 512) return launch_split<1, 64, 56, 8>(p..., n, c, s, stream, st);
     }
     return kNoSplit;
 }
