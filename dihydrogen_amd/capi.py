@@ -231,6 +231,8 @@ SIGNATURES = {
     "h2x_bn_audit_once": (c_int, [c_int, POINTER(TensorGeometry), c_uint32, c_void_p, c_void_p, c_size_t]),
     "h2x_bn_audit_ordered": (c_int, [c_int, POINTER(TensorGeometry), c_int, c_uint32, c_void_p, c_void_p, c_void_p,
                                      c_size_t]),
+    "h2x_bn_audit_short": (c_int, [c_int, POINTER(TensorGeometry), c_int, c_uint32, c_uint32, c_void_p, c_void_p, c_void_p,
+                                   c_size_t]),
     "h2x_bn_batch_normalization_clearing": (c_int, [c_int, POINTER(HaloedGeometry), c_void_p, c_void_p, c_void_p,
                                                     c_void_p, c_void_p, c_void_p, c_double, c_void_p]),
     "h2x_bn_backprop2_clearing": (c_int, [c_int, c_size_t, POINTER(HaloedGeometry), c_void_p, c_void_p, c_void_p,

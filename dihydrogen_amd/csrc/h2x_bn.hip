@@ -1357,6 +1357,8 @@ __global__ __launch_bounds__(kBlockSize) void bn_backprop2_short_kernel(
 
 #include "h2x_bn_ordered.hpp"
 
+#include "h2x_bn_short.hpp"
+
 // ---- host side ---------------------------------------------------------------
 
 template <typename T>
@@ -3310,6 +3312,123 @@ bool ordered_variant(const OrderedGeometry& g, const A* a, size_t bytes, bool ro
     return by_teams();
 }
 
+// ---- short segments of doubles, in the order of the staged calls -------------------
+// Dense or haloed tensors that lie alike (`ts`: the inputs, x first), cut as the staged reduction cuts them; g->turns is the
+// samples of a lane in a range.
+bool short_once_geometry(int num_samples, int num_channels, size_t spatial, std::initializer_list<const HostTensor*> ts,
+                         const HostTensor& output, ShortOnceGeometry* g)
+{
+    const HostTensor& x = **ts.begin();
+    for (const HostTensor* t : ts)
+        if (!lie_alike({t, &output}))
+            return false;
+    ShortGeometry sg;
+    if (!short_segments<double>(num_samples, num_channels, spatial, {&x}, &sg))
+        return false;
+    const size_t last = (num_samples - 1) * static_cast<size_t>(x.map.stride_n)
+                        + (std::min(num_channels, kBlockSize * 4) - 1) * static_cast<size_t>(x.map.stride_c)
+                        + short_span(x, spatial);
+    if (last >= (1ull << 30))
+        return false;
+    const int unroll = ts.size() == 1 ? kUnroll : kUnroll / 2;
+    const int groups = short_reduction_groups(&sg, max_groups_per_channel(num_channels), unroll, sizeof(double));
+    const ShortTensor t = short_tensor(x, sg);
+    g->row = static_cast<uint32_t>(sg.row);
+    g->slots_per_row = make_fastdiv(static_cast<uint32_t>(sg.slots_per_row));
+    g->slots = make_fastdiv(static_cast<uint32_t>(sg.slots));
+    g->h = make_fastdiv(static_cast<uint32_t>(t.h));
+    g->sy = t.sy;
+    g->sz = t.sz;
+    g->stride_n = static_cast<uint32_t>(t.stride_n);
+    g->stride_c = t.stride_c;
+    g->rows = make_fastdiv(static_cast<uint32_t>(sg.rows));
+    g->turns = make_fastdiv(static_cast<uint32_t>((sg.samples_per_group + sg.rows - 1) / sg.rows));
+    g->per = static_cast<uint32_t>(sg.samples_per_group);
+    g->ranges = static_cast<uint32_t>(groups);
+    g->num_samples = static_cast<uint32_t>(num_samples);
+    g->num_channels = static_cast<uint32_t>(num_channels);
+    return true;
+}
+
+// Fewer windows than this that play ranges one after another (g.passes) leave the chip idle longer than a second launch takes:
+// forward, or backward, N 255, C 34, 4 x 7 x 4 5.8 us more than in two launches, N 231, C 20, 6 x 7 3.9, N 85, C 22, 4 x 7 x 5 level.
+constexpr uint32_t kShortWindows = 64;
+
+template <int VEC, int TEAM, int K>
+void issue_short_once(const ShortOnceGeometry& g, const OnceForward<double>& a, uint32_t blocks, hipStream_t st)
+{
+    launch(bn_short_once_forward_kernel<VEC, TEAM, K>, blocks, TEAM, st, g, a);
+}
+template <int VEC, int TEAM, int K>
+void issue_short_once(const ShortOnceGeometry& g, const OnceBackward<double>& a, uint32_t blocks, hipStream_t st)
+{
+    launch(bn_short_once_backward_kernel<VEC, TEAM, K>, blocks, TEAM, st, g, a);
+}
+
+// Windows of workgroups of `threads` with `vectors` each that play up to most_passes ranges a thread; 0: such a workgroup does
+// not hold a channel.
+uint32_t short_once_windows(ShortOnceGeometry* g, uint32_t threads, uint32_t vectors, uint32_t most_passes)
+{
+    const uint32_t passes = std::min(vectors / g->turns.divisor, most_passes);
+    if (passes == 0)
+        return 0;
+    g->together = (g->ranges + passes - 1) / passes;
+    g->passes = (g->ranges + g->together - 1) / g->together;
+    const uint32_t lanes = g->slots.divisor * g->rows.divisor * g->together; // of a channel
+    if (lanes > threads)
+        return 0;
+    const uint32_t channels = std::min(threads / lanes, g->num_channels);
+    g->channels = make_fastdiv(channels);
+    return (g->num_channels + channels - 1) / channels;
+}
+
+// False: workgroups of TEAM threads with K vectors each do not hold a channel, or are not for this call.
+template <int TEAM, int K, typename A>
+bool short_once(ShortOnceGeometry g, const A& a, hipStream_t st)
+{
+    constexpr bool kForward = std::is_same<A, OnceForward<double>>::value;
+    const uint32_t windows = short_once_windows(&g, TEAM, K, short_once_passes<K, kForward>());
+    if (windows == 0 || (g.passes > 1 && windows < kShortWindows))
+        return false;
+    // The largest workgroups have to have more than ten of sixteen lanes play something (forward in us, by them less in two launches: 1024 threads
+    // N 29, C 911, 12 x 20, nine, +5.0, N 38, C 489, 14 x 11 with a halo, 10.5, -4.6; 512 threads N 71, C 291, 8 x 10, ten, +3.6, N 129, C
+    // 319, 8 x 5 with a halo, 12, -3.3); those of 16 vectors in one pass (N 70, C 135, 12 x 11, three, +1.1), and in more than a round of
+    // the chip nearly all of them (N 83, C 1398, 12 x 8 with a halo, 12, +9, N 46, C 832, 16 x 12, 15, -3.4).
+    const uint32_t playing = g.channels.divisor * g.slots.divisor * g.rows.divisor * g.together;
+    if (TEAM * K >= 1024 * 8 && playing * 16 <= TEAM * 10)
+        return false;
+    if (TEAM * K >= 1024 * 8 && K == 16 && (g.passes > 1 || (windows > 2 * chip_units() && playing * 16 < TEAM * 14)))
+        return false;
+    // (the smallest workgroup of so many vectors, backward: N 71, C 291, 8 x 10 3.4 us more than in two launches, N 109, C 1893, 5 x 6, 947 of
+    // them, 18.2 less)
+    if (TEAM == 256 && K == 16 && windows <= 2 * chip_units())
+        return false;
+    const uint32_t blocks = (windows + kNumXcd - 1) / kNumXcd * kNumXcd;
+    if (g.row == 1)
+        issue_short_once<1, TEAM, K>(g, a, blocks, st);
+    else
+        issue_short_once<2, TEAM, K>(g, a, blocks, st);
+    return true;
+}
+
+// The smallest workgroup that holds a channel; more threads before more vectors a thread.
+template <typename A>
+bool short_once_launch(int n, int c, size_t s, std::initializer_list<const HostTensor*> ts, const HostTensor& output, const A& a,
+                       hipStream_t st)
+{
+    ShortOnceGeometry g;
+    if (!short_once_geometry(n, c, s, ts, output, &g))
+        return false;
+    if (short_once<256, 4>(g, a, st) || short_once<512, 4>(g, a, st))
+        return true;
+    if constexpr (std::is_same<A, OnceForward<double>>::value)
+        return short_once<256, 8>(g, a, st) || short_once<512, 8>(g, a, st) || short_once<1024, 8>(g, a, st)
+               || short_once<512, 16>(g, a, st);
+    else
+        return short_once<1024, 4>(g, a, st) || short_once<256, 8>(g, a, st) || short_once<512, 8>(g, a, st)
+               || short_once<1024, 8>(g, a, st) || short_once<256, 16>(g, a, st);
+}
+
 size_t moved_bytes(const HostTensor& t, int n, int c, size_t s)
 {
     const size_t all = static_cast<size_t>(n) * c * s;
@@ -3327,6 +3446,8 @@ bool ordered_launch(int n, int c, size_t s, std::initializer_list<const HostTens
 {
     OrderedGeometry g;
     bool rows, team;
+    if (!team_polls && short_once_launch(n, c, s, ts, output, a, st))
+        return true;
     if (!ordered_geometry(n, c, s, ts, output, &g, &rows))
         return false;
     const size_t bytes = (static_cast<size_t>(c - 1) * output.map.stride_c + static_cast<size_t>(n - 1) * output.map.stride_n
@@ -4114,5 +4235,50 @@ extern "C" int h2x_bn_audit_ordered(int num_samples, const h2x_tensor_geometry* 
                             group[e + v] = static_cast<unsigned short>(k + 1);
                         }
                     }
+    return H2X_SUCCESS;
+}
+
+// Plays on the host which elements the workgroups that hold short segments of doubles touch.
+extern "C" int h2x_bn_audit_short(int num_samples, const h2x_tensor_geometry* geometry, int backward, unsigned int threads,
+                                  unsigned int vectors, unsigned char* counted, unsigned char* stored, unsigned short* range,
+                                  size_t elements)
+{
+    if (!geometry || !counted || !stored || !range || threads == 0 || threads > 1024)
+        return H2X_ERR_INVALID_ARGUMENT;
+    HostTensor t;
+    ShortOnceGeometry g;
+    int c;
+    size_t s;
+    const int err = strided_tensor<double>(geometry, reinterpret_cast<const void*>(uintptr_t(256)), num_samples, &t, &c, &s);
+    if (err)
+        return err;
+    if (num_samples <= 0 || c <= 0 || s == 0
+        || !(backward ? short_once_geometry(num_samples, c, s, {&t, &t}, t, &g) : short_once_geometry(num_samples, c, s, {&t}, t, &g)))
+        return H2X_ERR_UNSUPPORTED;
+    const uint32_t windows = short_once_windows(&g, threads, vectors, 4), vec = g.row == 1 ? 1 : 2;
+    if (windows == 0)
+        return H2X_ERR_UNSUPPORTED;
+    for (uint32_t w = 0; w < windows; ++w)
+        for (uint32_t thread = 0; thread < threads; ++thread)
+        {
+            const ShortOnceLane l = vec == 1 ? short_once_lane<1>(g, w, thread) : short_once_lane<2>(g, w, thread);
+            for (uint32_t u = 0; l.live && u < g.passes * g.turns.divisor; ++u)
+            {
+                const uint32_t p = u / g.turns.divisor, n = short_once_sample(g, l, p, u - p * g.turns.divisor);
+                if (n >= g.num_samples)
+                    continue;
+                const size_t e = static_cast<size_t>(w * g.channels.divisor * g.stride_c) + (l.at + n * g.stride_n);
+                if (e + vec > elements)
+                    return H2X_ERR_INVALID_ARGUMENT;
+                for (uint32_t v = 0; v < vec; ++v)
+                {
+                    stored[e + v] = 1;
+                    if (v < l.skip)
+                        continue;
+                    ++counted[e + v];
+                    range[e + v] = static_cast<unsigned short>(p * g.together + l.q + 1);
+                }
+            }
+        }
     return H2X_SUCCESS;
 }

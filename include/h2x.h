@@ -429,8 +429,8 @@ int h2x_bn_backward_local_strided(h2x_dtype dtype,
  * inputs), where an estimate of the time says so; otherwise what
  * h2x_bn_forward_local_strided and h2x_bn_backward_local_strided do.  The terms of
  * the sums are the same and are added in fp64: of floats in another order, of doubles in
- * the same one (channels of up to 2 million doubles forward and half a million backward,
- * segments beyond 256 elements).
+ * the same one (channels of up to 2 million doubles forward and half a million backward;
+ * with segments of up to 256 elements what one workgroup holds).
  *
  * team_state: h2x_bn_team_state_bytes() of the number of channels, or more, zeroed
  * once before the first call and then left to these calls, one after another, in any
@@ -551,6 +551,20 @@ int h2x_bn_audit_ordered(int num_samples,
                          unsigned char* stored,
                          unsigned short* group,
                          size_t elements);
+
+/**
+ * The same for double tensors of segments of up to 256 elements, by workgroups of `threads` that hold `vectors`
+ * each; `range`: one more than the range of samples whose sum an element is added to.
+ */
+int h2x_bn_audit_short(int num_samples,
+                       const h2x_tensor_geometry* geometry,
+                       int backward,
+                       unsigned int threads,
+                       unsigned int vectors,
+                       unsigned char* counted,
+                       unsigned char* stored,
+                       unsigned short* range,
+                       size_t elements);
 
 /**
  * The local part of a haloed tensor as it lies in memory: the real (allocated)
