@@ -220,7 +220,7 @@ __device__ __forceinline__ void load_vec(const T* p, T (&r)[VEC])
     }
 }
 
-template <typename T, int VEC, bool ALIGNED = true>
+template <typename T, int VEC, bool ALIGNED = true, bool STREAM = true>
 __device__ __forceinline__ void store_vec(T* p, const T (&r)[VEC])
 {
     // Outputs are written once and not read by the next kernel of the layer;
@@ -228,7 +228,10 @@ __device__ __forceinline__ void store_vec(T* p, const T (&r)[VEC])
     // kernel reads again, from the 256 MB memory-side cache.
     if constexpr (VEC == 1)
     {
-        __builtin_nontemporal_store(r[0], p);
+        if constexpr (STREAM)
+            __builtin_nontemporal_store(r[0], p);
+        else
+            *p = r[0];
     }
     else
     {
@@ -237,7 +240,10 @@ __device__ __forceinline__ void store_vec(T* p, const T (&r)[VEC])
 #pragma unroll
         for (int j = 0; j < VEC; ++j)
             t[j] = r[j];
-        __builtin_nontemporal_store(t, reinterpret_cast<V*>(p));
+        if constexpr (STREAM)
+            __builtin_nontemporal_store(t, reinterpret_cast<V*>(p));
+        else
+            *reinterpret_cast<V*>(p) = t;
     }
 }
 
@@ -282,27 +288,27 @@ __device__ __forceinline__ void load_in(const T* p, const TensorMap& m, size_t i
 // rewrite (rows layout): the elements a vector shares with the one before it
 // may be stored by both (the output shares no memory with the inputs they were
 // made from).
-template <typename T, int VEC, int LAYOUT>
+template <typename T, int VEC, int LAYOUT, bool STREAM = true>
 __device__ __forceinline__ void store_out(T* p, const TensorMap& m, size_t i, const Place& pl,
                                           const T (&r)[VEC], bool rewrite)
 {
     if constexpr (VEC == 1 || LAYOUT == kLayoutDense)
     {
-        store_vec<T, VEC, LAYOUT == kLayoutDense>(p + seg_offset<LAYOUT != kLayoutDense>(m, i), r);
+        store_vec<T, VEC, LAYOUT == kLayoutDense, STREAM>(p + seg_offset<LAYOUT != kLayoutDense>(m, i), r);
     }
     else
     {
         T* q = p + (row_offset(m, pl) + pl.first);
         if (pl.skip == 0 || rewrite)
         {
-            store_vec<T, VEC, false>(q, r);
+            store_vec<T, VEC, false, STREAM>(q, r);
         }
         else
         {
 #pragma unroll
             for (int j = 1; j < VEC; ++j)
                 if (j >= static_cast<int>(pl.skip))
-                    __builtin_nontemporal_store(r[j], q + j);
+                    store_vec<T, 1, true, STREAM>(q + j, {r[j]});
         }
     }
 }
@@ -530,17 +536,27 @@ struct FusedStats
     bool sequential;    // the partials come from a short-segment kernel and are added one after the other
 };
 
+// How a normalising kernel works: with statistics that it reads, past the caches; with those that it makes of partial sums; as the first,
+// with normal stores (see kNormalStores).
+enum ApplyMode : int
+{
+    kPlainApply = 0,
+    kFusedApply = 1,
+    kNormalApply = 2
+};
+
 // ---- forward: normalise ------------------------------------------------------
 // Replaces batch_normalization_opt_kernel, batchnorm.cu:420-455.  FUSED: mean
 // and variance are not read but made from the partial sums of bn_sums_kernel
 // (bn_finish_kernel + bn_statistics_kernel folded in).
-template <typename T, int VEC, int LAYOUT, bool FUSED = false>
+template <typename T, int VEC, int LAYOUT, int MODE>
 __global__ __launch_bounds__(kBlockSize) void bn_apply_kernel(
     const T* __restrict__ x, const T* __restrict__ mean, const T* __restrict__ var,
     const T* __restrict__ scale, const T* __restrict__ bias, T* __restrict__ y, T epsilon,
     int num_channels, size_t spatial, const TensorMap mx, const TensorMap my, size_t chunk,
     int chunks_per_seg, const FusedStats<T> fused = FusedStats<T>())
 {
+    constexpr bool FUSED = MODE == kFusedApply, STREAM = MODE != kNormalApply;
     const size_t seg = blockIdx.x / chunks_per_seg;
     const int k = blockIdx.x - seg * chunks_per_seg;
     const int c = seg % num_channels;
@@ -594,7 +610,7 @@ __global__ __launch_bounds__(kBlockSize) void bn_apply_kernel(
 #pragma unroll
             for (int j = 0; j < VEC; ++j)
                 v[u][j] = fma_t((v[u][j] - m) * inv_stdev, sc, bi);
-            store_out<T, VEC, LAYOUT>(yp, my, tile + u * kStride + threadIdx.x * VEC, pl[u], v[u], true);
+            store_out<T, VEC, LAYOUT, STREAM>(yp, my, tile + u * kStride + threadIdx.x * VEC, pl[u], v[u], true);
         }
     }
     for (size_t i = tile + threadIdx.x * VEC; i + VEC <= end; i += kStride)
@@ -605,7 +621,7 @@ __global__ __launch_bounds__(kBlockSize) void bn_apply_kernel(
 #pragma unroll
         for (int j = 0; j < VEC; ++j)
             v[j] = fma_t((v[j] - m) * inv_stdev, sc, bi);
-        store_out<T, VEC, LAYOUT>(yp, my, i, pl, v, true);
+        store_out<T, VEC, LAYOUT, STREAM>(yp, my, i, pl, v, true);
     }
 }
 
@@ -930,20 +946,20 @@ __device__ __forceinline__ void load_slot(const T* p, const ShortLane& l, T (&r)
 // rewrite: the output does not alias an input, so the elements in which the
 // last vector of a row overlaps its neighbour may be stored by both lanes (each
 // made the same values from the same inputs) and every lane stores a whole vector.
-template <typename T, int VEC, int TAIL>
+template <typename T, int VEC, int TAIL, bool STREAM = true>
 __device__ __forceinline__ void store_slot(T* p, const ShortLane& l, const T (&r)[VEC],
                                            bool rewrite)
 {
     if (TAIL == kTailNone || (TAIL == kTailOverlap && (rewrite || l.skip == 0)))
     {
-        store_vec<T, VEC, false>(p, r);
+        store_vec<T, VEC, false, STREAM>(p, r);
     }
     else
     {
 #pragma unroll
         for (int j = 0; j < VEC; ++j)
             if (slot_owns<VEC, TAIL>(l, j))
-                __builtin_nontemporal_store(r[j], p + j);
+                store_vec<T, 1, true, STREAM>(p + j, {r[j]});
     }
 }
 
@@ -1112,12 +1128,13 @@ __global__ __launch_bounds__(kBlockSize) void bn_sums_short_kernel(
     finish_short<T, 2>(g, l, acc, partials, always_partials, out);
 }
 
-template <typename T, int VEC, int TAIL, bool FUSED>
+template <typename T, int VEC, int TAIL, int MODE>
 __global__ __launch_bounds__(kBlockSize) void bn_apply_short_kernel(
     const T* __restrict__ x, const T* __restrict__ mean, const T* __restrict__ var,
     const T* __restrict__ scale, const T* __restrict__ bias, T* __restrict__ y, T epsilon,
     const ShortTensor tx, const ShortTensor ty, const ShortGeometry g, const FusedStats<T> fused)
 {
+    constexpr bool FUSED = MODE == kFusedApply, STREAM = MODE != kNormalApply;
     const ShortLane l = short_lane<VEC, TAIL>(g, static_cast<int>(threadIdx.x), static_cast<int>(blockIdx.x));
     T m = T(0), variance = T(0);
     if constexpr (FUSED)
@@ -1175,7 +1192,7 @@ __global__ __launch_bounds__(kBlockSize) void bn_apply_short_kernel(
 #pragma unroll
             for (int j = 0; j < VEC; ++j)
                 v[u][j] = fma_t((v[u][j] - m) * inv_stdev, sc, bi);
-            store_slot<T, VEC, TAIL>(yp + (n + u) * y_stride_n, l, v[u], true);
+            store_slot<T, VEC, TAIL, STREAM>(yp + (n + u) * y_stride_n, l, v[u], true);
         }
     }
     for (; n < end; ++n)
@@ -1185,7 +1202,7 @@ __global__ __launch_bounds__(kBlockSize) void bn_apply_short_kernel(
 #pragma unroll
         for (int j = 0; j < VEC; ++j)
             v[j] = fma_t((v[j] - m) * inv_stdev, sc, bi);
-        store_slot<T, VEC, TAIL>(yp + n * y_stride_n, l, v, true);
+        store_slot<T, VEC, TAIL, STREAM>(yp + n * y_stride_n, l, v, true);
     }
 }
 
@@ -1997,6 +2014,23 @@ Chunking elementwise_chunking(size_t spatial, size_t segments, int vw, int unrol
     return c;
 }
 
+// Haloed outputs that lie within this many bytes are stored normally by a pass that reads its statistics, inference or the staged one: the ends of
+// their rows are partial lines, which the caches merge with the neighbours'; larger ones push the inputs out of the memory-side cache.  Inference, past
+// the caches and normally, us going round three sets of tensors: N 106, C 257, 13 x 12, halo of 2, 28 MiB 14.1 and 10.4; N 27, C
+// 57, 14 x 11 x 10, halo of 2, 22 MiB 9.1 and 7.1; doubles N 125, C 346, 7 x 8, 30 MiB 14.9 and 11.3; below 5 MiB level; larger N 5, C 7,
+// 63 x 67 x 61, 38 MiB 14.0 and 13.2, N 152, C 5, 29 x 21 x 21, 47 MiB 19.4 and 20.4, N 25, C 245, 41 x 60, 62 MiB 23.8 and 33.1.  The line
+// lies below where inference alone would have it for the training that runs in stages, and reads x again: forward + backward there 5 % less with 29 to 32 MiB.
+// (With normal stores of dx, and of passes that finish their sums, training in stages loses up to 10 %: N 8, C 60, 129 x 142, 35 MiB 60.7 and 66.1.)
+constexpr size_t kNormalStores = size_t(32) << 20;
+
+bool stored_normally(const HostTensor& output, int num_samples, int num_channels, size_t spatial, size_t elem_bytes)
+{
+    return output.strided
+           && (static_cast<size_t>(num_channels - 1) * output.map.stride_c
+               + static_cast<size_t>(num_samples - 1) * output.map.stride_n + short_span(output, spatial)) * elem_bytes
+                  <= kNormalStores;
+}
+
 template <typename T>
 int apply_impl(int num_samples, int num_channels, size_t spatial, const HostTensor& tx_in,
                const HostTensor& ty_in, const void* x, const void* mean, const void* var,
@@ -2005,6 +2039,7 @@ int apply_impl(int num_samples, int num_channels, size_t spatial, const HostTens
 {
     if (static_cast<size_t>(num_samples) * num_channels == 0 || spatial == 0)
         return H2X_SUCCESS;
+    const bool normally = stored_normally(ty_in, num_samples, num_channels, spatial, sizeof(T));
     ShortGeometry sg;
     const bool is_short = short_segments<T>(num_samples, num_channels, spatial, {&tx_in, &ty_in}, &sg);
     if (fused && fused->sequential != is_short)
@@ -2021,13 +2056,19 @@ int apply_impl(int num_samples, int num_channels, size_t spatial, const HostTens
         if (logged(rec))
             return H2X_SUCCESS;
         if (fused)
-            H2X_DISPATCH_SHORT_FUSED(bn_apply_short_kernel, true, grid, static_cast<const T*>(x),
+            H2X_DISPATCH_SHORT_FUSED(bn_apply_short_kernel, kFusedApply, grid, static_cast<const T*>(x),
                                      nullptr, nullptr, static_cast<const T*>(scale),
                                      static_cast<const T*>(bias), static_cast<T*>(y),
                                      static_cast<T>(epsilon), short_tensor(tx_in, sg),
                                      short_tensor(ty_in, sg), sg, *fused);
+        else if (normally)
+            H2X_DISPATCH_SHORT_FUSED(bn_apply_short_kernel, kNormalApply, grid, static_cast<const T*>(x),
+                                     static_cast<const T*>(mean), static_cast<const T*>(var),
+                                     static_cast<const T*>(scale), static_cast<const T*>(bias),
+                                     static_cast<T*>(y), static_cast<T>(epsilon),
+                                     short_tensor(tx_in, sg), short_tensor(ty_in, sg), sg, FusedStats<T>());
         else
-            H2X_DISPATCH_SHORT_FUSED(bn_apply_short_kernel, false, grid, static_cast<const T*>(x),
+            H2X_DISPATCH_SHORT_FUSED(bn_apply_short_kernel, kPlainApply, grid, static_cast<const T*>(x),
                                      static_cast<const T*>(mean), static_cast<const T*>(var),
                                      static_cast<const T*>(scale), static_cast<const T*>(bias),
                                      static_cast<T*>(y), static_cast<T>(epsilon),
@@ -2059,12 +2100,19 @@ int apply_impl(int num_samples, int num_channels, size_t spatial, const HostTens
     if (logged(rec))
         return H2X_SUCCESS;
     if (fused)
-        H2X_DISPATCH_ELEMENTWISE(bn_apply_kernel, true, grid, static_cast<const T*>(x), nullptr,
+        H2X_DISPATCH_ELEMENTWISE(bn_apply_kernel, kFusedApply, grid, static_cast<const T*>(x), nullptr,
                                  nullptr, static_cast<const T*>(scale), static_cast<const T*>(bias),
                                  static_cast<T*>(y), static_cast<T>(epsilon), num_channels, spatial,
                                  tx.map, ty.map, ch.chunk, ch.chunks_per_seg, *fused);
+    else if (normally && vw > 1) // (such a launch goes row by row)
+        launch(bn_apply_kernel<T, full_vec<T>(), kLayoutRows, kNormalApply>, grid, kBlockSize, stream,
+               static_cast<const T*>(x),
+               static_cast<const T*>(mean), static_cast<const T*>(var),
+               static_cast<const T*>(scale), static_cast<const T*>(bias),
+               static_cast<T*>(y), static_cast<T>(epsilon), num_channels, spatial,
+               tx.map, ty.map, ch.chunk, ch.chunks_per_seg, FusedStats<T>());
     else
-        H2X_DISPATCH_ELEMENTWISE(bn_apply_kernel, false, grid, static_cast<const T*>(x),
+        H2X_DISPATCH_ELEMENTWISE(bn_apply_kernel, kPlainApply, grid, static_cast<const T*>(x),
                                  static_cast<const T*>(mean), static_cast<const T*>(var),
                                  static_cast<const T*>(scale), static_cast<const T*>(bias),
                                  static_cast<T*>(y), static_cast<T>(epsilon), num_channels, spatial,
