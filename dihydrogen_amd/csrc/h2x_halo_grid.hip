@@ -98,8 +98,6 @@ struct Args
     FastDiv ranks;                 // by num_ranks
     FastDiv lines;                 // by the number of lines
     int32_t line;                  // ranks in a line
-    FastDiv seams;                 // by the number of seams in the dimension of a reverse exchange
-    int32_t seam[kMaxRanks];       // the lower rank of each
     int32_t width[kMaxSpatial];
     uint32_t outer; // channels x samples
     Rank rank[kMaxRanks];
@@ -275,10 +273,56 @@ __host__ __device__ __forceinline__ void body(const Args& a, uint32_t block, uin
     }
 }
 
-// One dimension of the reverse exchange: the halo strips of `dim` are folded into
+// A seam of two ranks in the dimension of a reverse exchange.  What a workgroup reads of its arguments stands between its start and its
+// first access, so all that can be followed is followed on the host: two scalar loads, one after the other, instead of five (reverse exchanges, us: 4 x 64 x
+// 57 x 57 on 2 x 2 9.2 -> 7.9; 8 x 6 x 13 x 13 x 12 on 2^3, periodic, halos of 3 14.4 -> 12.5; 2 x 34 x 68 x 105 x 34 of doubles on 2 x 2 x 1 9.9 -> 8.3; 9 x
+// 2 x 63 x 156 x 131 on 1 x 2 x 2, periodic 25.5 -> 21.2; 1 x 32 x 256^3 on 2^3, periodic 304 -> 297).
+struct FoldSeam
+{
+    char *lower, *upper;              // the lower rank's upper boundary cells, whose upper halo follows them; the upper rank's lower halo,
+                                      // whose lower boundary cells follow it: in row 0
+    uint32_t lower_pitch, upper_pitch; // elements from row to row
+    uint32_t run, rows;               // elements of a strip that lie together; how often
+    FastDiv units;                    // by vectors (or elements) of a run
+    uint32_t vectors;                 // a run holds at least one vector
+};
+
+struct FoldArgs
+{
+    FastDiv turns; // by the number of seams, or lines of ranks, that take turns workgroup by workgroup
+    int32_t line;  // seams of a line; of a ring, seam i is the upper one of rank i
+    FastDiv cells; // by the threads that serve a row's ends
+    FoldSeam seam[kMaxRanks];
+};
+
+// How a dimension is folded: strip by strip, or dimension 0 line by line, with both sides of every seam or one end of
+// every rank's row in a thread.
+enum Fold : int
+{
+    kStrips = 0,
+    kOpenLines = 1,
+    kRings = 2
+};
+
+// Where the cells of one side of a seam are and where what is added to them comes from, both from the start of a row.
+template <typename T>
+struct FoldSide
+{
+    T* to;
+    const T* from;
+};
+template <typename T>
+__host__ __device__ __forceinline__ FoldSide<T> fold_side(const FoldSeam& s, uint32_t row, bool of_upper)
+{
+    T* const lower = reinterpret_cast<T*>(s.lower) + row * s.lower_pitch;
+    T* const upper = reinterpret_cast<T*>(s.upper) + row * s.upper_pitch;
+    return of_upper ? FoldSide<T>{upper + s.run, lower + s.run} : FoldSide<T>{lower, upper};
+}
+
+// One dimension of the reverse exchange: the halo strips of the dimension are folded into
 // the boundary cells of the ranks they belong to.  A strip spans the real extents
 // of the other dimensions, so along memory it is runs of `width` times the real
-// extents below `dim`, one per index above it.  A thread serves the same vector of
+// extents below it, one per index above it.  A thread serves the same vector of
 // both strips of a seam, what each rank gives and takes there: four loads in
 // flight, and what a rank gives lies beside what it takes, in a line of memory that
 // they often share (both strips of a rank and, so, both of a seam, us, N x C x extents on
@@ -288,41 +332,24 @@ __host__ __device__ __forceinline__ void body(const Args& a, uint32_t block, uin
 // different dimensions stay launches of their own: a later one reads halo cells that
 // an earlier one has added to.
 template <typename T, typename Op, typename Mem>
-__host__ __device__ __forceinline__ void fold_body(const Args& a, uint32_t block, uint32_t thread, int dim, Op op,
+__host__ __device__ __forceinline__ void fold_body(const FoldArgs& a, uint32_t block, uint32_t thread, Op op,
                                                    const Mem& mem)
 {
     constexpr int VEC = 16 / sizeof(T);
     using W = typename Words<T, VEC>::unaligned_t;
-    const uint32_t local_block = fastdiv(block, a.seams);
-    const int r = a.seam[block - local_block * a.seams.divisor];
-    const Rank& me = a.rank[r];
-    const int hi = me.peer[dim][1];
-    // real extents below, along and above the dimension
-    int64_t below = 1, above = a.outer;
-    for (int d = 0; d < kMaxSpatial; ++d)
-    {
-        const int64_t real = me.local[d] + 2 * a.width[d];
-        below *= d < dim ? real : 1;
-        above *= d > dim ? real : 1;
-    }
-    const int64_t w = a.width[dim];
-    const uint32_t run = static_cast<uint32_t>(w * below);
+    const uint32_t local_block = fastdiv(block, a.turns);
+    const FoldSeam& seam = a.seam[block - local_block * a.turns.divisor];
     const uint32_t at = local_block * kBlock + thread;
-    const uint32_t row = fastdiv(at, me.units);
-    if (row >= above)
+    const uint32_t row = fastdiv(at, seam.units);
+    if (row >= seam.rows)
         return;
-    auto pitch = [&](int q) { return (a.rank[q].local[dim] + 2 * w) * below; };
-    // this rank's upper boundary cells take the upper neighbour's lower halo, and the other way round
-    T* const mine = reinterpret_cast<T*>(me.tensor) + (row * pitch(r) + me.local[dim] * below);
-    T* const theirs = reinterpret_cast<T*>(a.rank[hi].tensor) + row * pitch(hi);
-    T* const to[2] = {mine, theirs + w * below};
-    const T* const from[2] = {theirs, mine + w * below};
-    uint32_t x = at - row * me.units.divisor;
+    const FoldSide<T> side[2] = {fold_side<T>(seam, row, false), fold_side<T>(seam, row, true)};
+    uint32_t x = at - row * seam.units.divisor;
     uint32_t n = 1;
-    if (me.vectors)
+    if (seam.vectors)
     {
         x *= VEC;
-        n = run - x < VEC ? run - x : VEC;
+        n = seam.run - x < VEC ? seam.run - x : VEC;
     }
     if (n == VEC)
     {
@@ -330,8 +357,8 @@ __host__ __device__ __forceinline__ void fold_body(const Args& a, uint32_t block
 #pragma unroll
         for (int i = 0; i < 2; ++i)
         {
-            s[i] = mem.template load<VEC, false>(from[i] + x);
-            t[i] = mem.template load<VEC, false>(to[i] + x);
+            s[i] = mem.template load<VEC, false>(side[i].from + x);
+            t[i] = mem.template load<VEC, false>(side[i].to + x);
         }
 #pragma unroll
         for (int i = 0; i < 2; ++i)
@@ -339,83 +366,81 @@ __host__ __device__ __forceinline__ void fold_body(const Args& a, uint32_t block
 #pragma unroll
             for (int j = 0; j < VEC; ++j)
                 t[i][j] = op(t[i][j], s[i][j]);
-            mem.template store<VEC, false>(to[i] + x, t[i]);
+            mem.template store<VEC, false>(side[i].to + x, t[i]);
         }
         return;
     }
     for (const uint32_t end = x + n; x < end; ++x)
     {
-        const T s0 = mem.load1(from[0] + x), t0 = mem.load1(to[0] + x);
-        const T s1 = mem.load1(from[1] + x), t1 = mem.load1(to[1] + x);
-        mem.store1(to[0] + x, op(t0, s0));
-        mem.store1(to[1] + x, op(t1, s1));
+        const T s0 = mem.load1(side[0].from + x), t0 = mem.load1(side[0].to + x);
+        const T s1 = mem.load1(side[1].from + x), t1 = mem.load1(side[1].to + x);
+        mem.store1(side[0].to + x, op(t0, s0));
+        mem.store1(side[1].to + x, op(t1, s1));
     }
 }
 
 template <typename T, typename Op>
-__global__ __launch_bounds__(kBlock, 8) void halo_fold_kernel(const Args a, int dim, Op op)
+__global__ __launch_bounds__(kBlock, 8) void halo_fold_kernel(const FoldArgs a, Op op)
 {
-    fold_body<T, Op, DeviceMem>(a, blockIdx.x, threadIdx.x, dim, op, DeviceMem());
+    fold_body<T, Op, DeviceMem>(a, blockIdx.x, threadIdx.x, op, DeviceMem());
 }
 
 // Dimension 0 for all ranks of a line in the same thread: the two lines of memory at a
 // seam of two ranks hold what both give and take, and a workgroup per rank reads them
 // twice and writes them back from two XCDs.  RINGS (every rank has both neighbours): a
 // thread serves one end of a row in every rank, so that the upper ends and the next
-// row's lower ends are neighbouring lanes' work; open lines: both sides of every seam,
+// row's lower ends, which share a line of memory, are neighbouring lanes' work; open lines: both sides of every seam,
 // so that no lane is idle.  Reverse exchanges, rank by rank and so (us; N x C x extents
 // on a grid, halo 1 unless noted): 1 x 32 x 128^3 on 2^3, periodic 96.7 -> 87.8 (seam by
 // seam 98.4), 4 x 32 x 64^3 on 1 x 2 x 4 110 -> 97, 8 x 16 x 64^3 of doubles on 2^3,
 // halo 3 173 -> 135, 15 x 8 x 33 x 57 x 45 of doubles on 2^3 43.0 -> 39.5 (end by end
 // 43.3), 8 x 64 x 112^2 on 2 x 2, periodic 15.8 -> 11.7.
-template <typename T, typename Op, bool RINGS, typename Mem>
-__host__ __device__ __forceinline__ void fold_ends_body(const Args& a, uint32_t block, uint32_t thread, Op op,
+template <typename T, typename Op, int BY, typename Mem>
+__host__ __device__ __forceinline__ void fold_ends_body(const FoldArgs& a, uint32_t block, uint32_t thread, Op op,
                                                         const Mem& mem)
 {
-    constexpr int kCells = RINGS ? 1 : 2;
-    const uint32_t local_block = fastdiv(block, a.lines);
-    const int r = static_cast<int>((block - local_block * a.lines.divisor) * a.line);
-    const uint32_t w = a.width[0];
-    const uint32_t rows = static_cast<uint32_t>(a.rank[r].local[1] + 2 * a.width[1])
-                          * static_cast<uint32_t>(a.rank[r].local[2] + 2 * a.width[2]) * a.outer;
+    constexpr int kCells = BY == kOpenLines ? 2 : 1;
+    const uint32_t local_block = fastdiv(block, a.turns);
+    const FoldSeam* const line = a.seam + (block - local_block * a.turns.divisor) * a.line;
+    const uint32_t w = line[0].run;
     const uint32_t at = local_block * kBlock + thread;
-    const uint32_t row = fastdiv(at, RINGS ? a.both_ends : a.halo[0]);
-    if (row >= rows)
+    const uint32_t row = fastdiv(at, a.cells);
+    if (row >= line[0].rows)
         return;
-    const uint32_t x = at - row * (RINGS ? 2 * w : w);
-    const uint32_t j = x < w ? x : x - w;
+    const uint32_t x = at - row * a.cells.divisor;
+    const bool lower_end = x < w; // of a rank's row
+    const uint32_t j = lower_end ? x : x - w;
 #pragma unroll 1
     for (int base = 0; base < a.line; base += kRanksPerTurn)
     {
         T s[kRanksPerTurn][kCells], t[kRanksPerTurn][kCells];
         T* to[kRanksPerTurn][kCells];
-        // a boundary cell of k takes a halo cell of its neighbour: the upper one from the lower halo, and so on
-        auto load = [&](int i, int c, const Rank& k, bool upper, const char* neighbour, uint32_t local) {
-            to[i][c] = reinterpret_cast<T*>(k.tensor) + (row * (k.local[0] + 2 * w) + (upper ? k.local[0] : w) + j);
-            s[i][c] = mem.load1(reinterpret_cast<const T*>(neighbour)
-                                + (row * (local + 2 * w) + (upper ? 0 : local + w) + j));
-            t[i][c] = mem.load1(to[i][c]);
-        };
 #pragma unroll
         for (int i = 0; i < kRanksPerTurn; ++i)
         {
             to[i][0] = nullptr;
             if (base + i >= a.line)
                 continue;
-            const Rank& k = a.rank[r + base + i];
-            if (k.peer[0][1] < 0)
+            const FoldSeam& above = line[base + i];
+            if constexpr (BY == kRings)
+            {
+                const FoldSeam& below = line[base + i > 0 ? base + i - 1 : a.line - 1];
+                // (Taking the lower end of the next rank, at the same seam, is faster by up to a tenth where the ends of the rows stay in
+                // the caches and slower by as much beyond: the upper end of a row and the lower end of the next share a line.)
+                const uint32_t lower_start = row * below.upper_pitch + below.run, upper_start = row * above.lower_pitch;
+                to[i][0] = reinterpret_cast<T*>(lower_end ? below.upper : above.lower) + ((lower_end ? lower_start : upper_start) + j);
+                s[i][0] = mem.load1(reinterpret_cast<const T*>(lower_end ? below.lower : above.upper)
+                                    + (row * (lower_end ? below.lower_pitch : above.upper_pitch) + (lower_end ? w : 0) + j));
+                t[i][0] = mem.load1(to[i][0]);
                 continue;
-            const Rank& above = a.rank[k.peer[0][1]];
-            if constexpr (RINGS)
-            {
-                const Rank& below = a.rank[k.peer[0][0]];
-                const bool upper = x >= w;
-                load(i, 0, k, upper, upper ? above.tensor : below.tensor, upper ? above.local[0] : below.local[0]);
             }
-            else
+#pragma unroll
+            for (int c = 0; c < kCells; ++c)
             {
-                load(i, 0, k, true, above.tensor, above.local[0]);
-                load(i, 1, above, false, k.tensor, k.local[0]);
+                const FoldSide<T> side = fold_side<T>(above, row, c == 1);
+                to[i][c] = side.to + j;
+                s[i][c] = mem.load1(side.from + j);
+                t[i][c] = mem.load1(to[i][c]);
             }
         }
 #pragma unroll
@@ -429,51 +454,55 @@ __host__ __device__ __forceinline__ void fold_ends_body(const Args& a, uint32_t 
     }
 }
 
-template <typename T, typename Op, bool RINGS>
-__global__ __launch_bounds__(kBlock, 8) void halo_fold_ends_kernel(const Args a, Op op)
+template <typename T, typename Op, int BY>
+__global__ __launch_bounds__(kBlock, 8) void halo_fold_ends_kernel(const FoldArgs a, Op op)
 {
-    fold_ends_body<T, Op, RINGS, DeviceMem>(a, blockIdx.x, threadIdx.x, op, DeviceMem());
+    fold_ends_body<T, Op, BY, DeviceMem>(a, blockIdx.x, threadIdx.x, op, DeviceMem());
 }
 
-// In place of the dimension: the ends of the rows, line by line.
-constexpr int kRings = -1, kOpenLines = -2;
-
-template <typename T, typename Op>
-int issue_fold(const Args& a, uint32_t blocks, int dim, hipStream_t stream)
+template <typename T, typename Op, int BY>
+int issue_fold(const FoldArgs& a, uint32_t blocks, hipStream_t stream)
 {
     if (Audit* const audit = current_audit())
     {
         const TraceMem mem{audit};
         for (uint32_t block = 0; block < blocks; ++block)
             for (uint32_t thread = 0; thread < kBlock; ++thread)
-                if (dim == kRings)
-                    fold_ends_body<T, Op, true, TraceMem>(a, block, thread, Op(), mem);
-                else if (dim == kOpenLines)
-                    fold_ends_body<T, Op, false, TraceMem>(a, block, thread, Op(), mem);
+                if constexpr (BY == kStrips)
+                    fold_body<T, Op, TraceMem>(a, block, thread, Op(), mem);
                 else
-                    fold_body<T, Op, TraceMem>(a, block, thread, dim, Op(), mem);
+                    fold_ends_body<T, Op, BY, TraceMem>(a, block, thread, Op(), mem);
         ++audit->launches;
         audit->workgroups += blocks;
         return H2X_SUCCESS;
     }
-    if (dim == kRings)
-        launch(halo_fold_ends_kernel<T, Op, true>, dim3(blocks), kBlock, stream, a, Op());
-    else if (dim == kOpenLines)
-        launch(halo_fold_ends_kernel<T, Op, false>, dim3(blocks), kBlock, stream, a, Op());
+    if constexpr (BY == kStrips)
+        launch(halo_fold_kernel<T, Op>, dim3(blocks), kBlock, stream, a, Op());
     else
-        launch(halo_fold_kernel<T, Op>, dim3(blocks), kBlock, stream, a, dim, Op());
+        launch(halo_fold_ends_kernel<T, Op, BY>, dim3(blocks), kBlock, stream, a, Op());
     return launch_status();
 }
 
+template <typename T, typename Op>
+int issue_fold(const FoldArgs& a, uint32_t blocks, Fold by, hipStream_t stream)
+{
+    switch (by)
+    {
+    case kStrips: return issue_fold<T, Op, kStrips>(a, blocks, stream);
+    case kOpenLines: return issue_fold<T, Op, kOpenLines>(a, blocks, stream);
+    default: return issue_fold<T, Op, kRings>(a, blocks, stream);
+    }
+}
+
 template <typename T>
-int issue_fold(int op, const Args& a, uint32_t blocks, int dim, hipStream_t stream)
+int issue_fold(int op, const FoldArgs& a, uint32_t blocks, Fold by, hipStream_t stream)
 {
     switch (op)
     {
-    case H2X_HALO_ID: return issue_fold<T, copy::OpId>(a, blocks, dim, stream);
-    case H2X_HALO_SUM: return issue_fold<T, copy::OpSum>(a, blocks, dim, stream);
-    case H2X_HALO_MAX: return issue_fold<T, copy::OpMax>(a, blocks, dim, stream);
-    default: return issue_fold<T, copy::OpMin>(a, blocks, dim, stream);
+    case H2X_HALO_ID: return issue_fold<T, copy::OpId>(a, blocks, by, stream);
+    case H2X_HALO_SUM: return issue_fold<T, copy::OpSum>(a, blocks, by, stream);
+    case H2X_HALO_MAX: return issue_fold<T, copy::OpMax>(a, blocks, by, stream);
+    default: return issue_fold<T, copy::OpMin>(a, blocks, by, stream);
     }
 }
 
@@ -760,58 +789,63 @@ int run_fold(h2x_dtype dtype, const h2x_halo_grid* h, int op, h2x_stream_t strea
     bool lines = rows >= kLineRows && a.width[0] > 0 && order_into_lines(&a, h->num_ranks);
     const bool rings = lines && a.rank[0].peer[0][0] >= 0;
     const int64_t vec = 16 / es;
-    uint64_t blocks[kMaxSpatial] = {}, longest = 0; // workgroups of the largest line
-    FastDiv units[kMaxSpatial][kMaxRanks];
-    bool vectors[kMaxSpatial][kMaxRanks];
+    FoldArgs f[kMaxSpatial];
+    uint64_t blocks[kMaxSpatial] = {};
     for (int dim = 0; dim < kMaxSpatial; ++dim)
     {
-        bool any = false;
+        uint32_t seams = 0;
         uint64_t most = 0; // workgroups of the largest rank
+        uint64_t longest = 0; // and of the largest line
         for (int r = 0; r < h->num_ranks; ++r)
         {
             const Rank& k = a.rank[r];
-            any = any || k.peer[dim][0] >= 0 || k.peer[dim][1] >= 0;
-            int64_t run = a.width[dim], above = a.outer;
+            int64_t below = 1, above = a.outer;
             for (int d = 0; d < kMaxSpatial; ++d)
-                (d < dim ? run : above) *= d == dim ? 1 : k.local[d] + 2 * a.width[d];
-            vectors[dim][r] = run >= vec;
+                (d < dim ? below : above) *= d == dim ? 1 : k.local[d] + 2 * a.width[d];
+            const int64_t run = a.width[dim] * below;
             const int64_t n = run >= vec ? (run + vec - 1) / vec : std::max<int64_t>(run, 1);
-            units[dim][r] = make_fastdiv(static_cast<uint32_t>(n));
             most = std::max<uint64_t>(most, (n * above + kBlock - 1) / kBlock);
-            if (dim == 0)
-                longest = std::max<uint64_t>(longest, ((rings ? 2 : 1) * run * above + kBlock - 1) / kBlock);
+            longest = std::max<uint64_t>(longest, ((rings ? 2 : 1) * run * above + kBlock - 1) / kBlock);
+            if (k.peer[dim][1] < 0)
+                continue;
+            const Rank& u = a.rank[k.peer[dim][1]];
+            FoldSeam& seam = f[dim].seam[seams++];
+            seam.lower = k.tensor + k.local[dim] * below * es;
+            seam.upper = u.tensor;
+            seam.lower_pitch = static_cast<uint32_t>((k.local[dim] + 2 * a.width[dim]) * below);
+            seam.upper_pitch = static_cast<uint32_t>((u.local[dim] + 2 * a.width[dim]) * below);
+            seam.run = static_cast<uint32_t>(run);
+            seam.rows = static_cast<uint32_t>(above);
+            seam.units = make_fastdiv(static_cast<uint32_t>(n));
+            seam.vectors = run >= vec;
         }
-        if (!any)
+        if (seams == 0)
             continue;
-        blocks[dim] = most * h->num_ranks;
-        if (most > kMaxRankBlocks || blocks[dim] > kMaxBlocks)
+        if (most > kMaxRankBlocks || most * h->num_ranks > kMaxBlocks)
             return H2X_ERR_TOO_LARGE;
-    }
-    // (what can be launched is a matter of the ranks alone)
-    if (lines && blocks[0] > 0)
-    {
-        lines = longest <= kMaxRankBlocks && longest * a.lines.divisor <= kMaxBlocks;
-        blocks[0] = lines ? longest * a.lines.divisor : blocks[0];
+        f[dim].turns = make_fastdiv(seams);
+        blocks[dim] = most * seams;
+        // (what can be launched is a matter of the ranks alone)
+        // (open lines and rings side by side have no one number of seams)
+        if (dim == 0)
+            lines = lines && longest <= kMaxRankBlocks && longest * a.lines.divisor <= kMaxBlocks
+                    && seams == (rings ? a.line : a.line - 1) * a.lines.divisor;
+        if (dim == 0 && lines)
+        {
+            f[0].turns = a.lines;
+            f[0].line = static_cast<int32_t>(seams / a.lines.divisor);
+            f[0].cells = rings ? a.both_ends : a.halo[0];
+            blocks[0] = longest * a.lines.divisor;
+        }
     }
     for (int dim = 0; dim < kMaxSpatial && err == 0; ++dim)
     {
         if (blocks[dim] == 0)
             continue;
-        uint32_t seams = 0;
-        for (int r = 0; r < h->num_ranks; ++r)
-        {
-            a.rank[r].units = units[dim][r];
-            a.rank[r].vectors = vectors[dim][r];
-            if (a.rank[r].peer[dim][1] >= 0)
-                a.seam[seams++] = r;
-        }
-        a.seams = make_fastdiv(seams);
-        uint32_t n = static_cast<uint32_t>(blocks[dim]);
-        if (dim > 0 || !lines)
-            n = n / h->num_ranks * seams;
-        const int by = dim > 0 || !lines ? dim : rings ? kRings : kOpenLines;
-        err = es == 4 ? issue_fold<float>(op, a, n, by, as_stream(stream))
-                      : issue_fold<double>(op, a, n, by, as_stream(stream));
+        const Fold by = dim > 0 || !lines ? kStrips : rings ? kRings : kOpenLines;
+        const uint32_t n = static_cast<uint32_t>(blocks[dim]);
+        err = es == 4 ? issue_fold<float>(op, f[dim], n, by, as_stream(stream))
+                      : issue_fold<double>(op, f[dim], n, by, as_stream(stream));
     }
     return err;
 }
