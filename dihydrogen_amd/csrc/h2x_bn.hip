@@ -3238,23 +3238,23 @@ bool ordered_geometry(int num_samples, int num_channels, size_t spatial, std::in
     return true;
 }
 
-template <int TEAM, int K, bool TEAMS, bool ROWS, bool STREAM>
-void issue_ordered(const OrderedGeometry& g, const OnceForward<double>& a, unsigned long long* states, uint32_t blocks,
+template <int TEAM, int K, bool TEAMS, bool ROWS, bool STREAM, typename G>
+void issue_ordered(const G& g, const OnceForward<double>& a, unsigned long long* states, uint32_t blocks,
                    hipStream_t st)
 {
-    launch(bn_ordered_forward_kernel<TEAM, K, TEAMS, ROWS, STREAM>, blocks, TEAM, st, g, a, states);
+    launch(bn_ordered_forward_kernel<TEAM, K, TEAMS, ROWS, STREAM, G>, blocks, TEAM, st, g, a, states);
 }
-template <int TEAM, int K, bool TEAMS, bool ROWS, bool STREAM>
-void issue_ordered(const OrderedGeometry& g, const OnceBackward<double>& a, unsigned long long* states, uint32_t blocks,
+template <int TEAM, int K, bool TEAMS, bool ROWS, bool STREAM, typename G>
+void issue_ordered(const G& g, const OnceBackward<double>& a, unsigned long long* states, uint32_t blocks,
                    hipStream_t st)
 {
     if constexpr (K >= 8)
         if (g.streams_gradient)
         {
-            launch(bn_ordered_backward_kernel<TEAM, K, TEAMS, ROWS, STREAM, true>, blocks, TEAM, st, g, a, states);
+            launch(bn_ordered_backward_kernel<TEAM, K, TEAMS, ROWS, STREAM, true, G>, blocks, TEAM, st, g, a, states);
             return;
         }
-    launch(bn_ordered_backward_kernel<TEAM, K, TEAMS, ROWS, STREAM, false>, blocks, TEAM, st, g, a, states);
+    launch(bn_ordered_backward_kernel<TEAM, K, TEAMS, ROWS, STREAM, false, G>, blocks, TEAM, st, g, a, states);
 }
 
 // Groups that a workgroup of TEAM threads with K vectors each holds.
@@ -3264,12 +3264,14 @@ uint32_t ordered_holds(const OrderedGeometry& g)
     return TEAM / kBlockSize * (K / kOrderedBatch / g.group_batches.divisor);
 }
 
-template <int TEAM, int K, bool TEAMS, typename A>
-void ordered_issue(const OrderedGeometry& g, const A& a, bool rows, bool stream, void* state, hipStream_t st)
+template <int TEAM, int K, bool TEAMS, typename G, typename A>
+void ordered_issue(const G& g, const A& a, bool rows, bool stream, void* state, hipStream_t st)
 {
     unsigned long long* const states = static_cast<unsigned long long*>(state);
     const uint32_t blocks = TEAMS ? g.num_channels * g.members.divisor : (g.num_channels + kNumXcd - 1) / kNumXcd * kNumXcd;
-    if (!rows)
+    if constexpr (std::is_same<G, OrderedClearing>::value) // (rows, for the others are not haloed)
+        return issue_ordered<TEAM, K, TEAMS, true, false>(g, a, states, blocks, st);
+    else if (!rows)
         issue_ordered<TEAM, K, TEAMS, false, true>(g, a, states, blocks, st);
     else if (stream)
         issue_ordered<TEAM, K, TEAMS, true, true>(g, a, states, blocks, st);
@@ -3278,8 +3280,8 @@ void ordered_issue(const OrderedGeometry& g, const A& a, bool rows, bool stream,
 }
 
 // One workgroup a channel.  Without a: whether.
-template <int TEAM, int K, typename A>
-bool ordered_once(OrderedGeometry g, const A* a, bool rows, bool stream, hipStream_t st)
+template <int TEAM, int K, typename G, typename A>
+bool ordered_once(G g, const A* a, bool rows, bool stream, hipStream_t st)
 {
     if (g.groups > ordered_holds<TEAM, K>(g))
         return false;
@@ -3301,8 +3303,8 @@ uint32_t ordered_members(const OrderedGeometry& g, uint32_t most, uint32_t least
     return fit_team((g.groups + own - 1) / own, g.num_channels, (g.groups + width - 1) / width * SUMS, most, least);
 }
 
-template <int TEAM, int K, typename A>
-void ordered_team(OrderedGeometry g, const A& a, bool rows, bool stream, uint32_t members, void* state, hipStream_t st)
+template <int TEAM, int K, typename G, typename A>
+void ordered_team(G g, const A& a, bool rows, bool stream, uint32_t members, void* state, hipStream_t st)
 {
     g.passes = K / kOrderedBatch / g.group_batches.divisor;
     g.members = make_fastdiv(members);
@@ -3310,8 +3312,8 @@ void ordered_team(OrderedGeometry g, const A& a, bool rows, bool stream, uint32_
 }
 
 // By teams, as for floats (team_variant).
-template <typename A>
-bool ordered_by_teams(const OrderedGeometry& g, const A* a, size_t bytes, bool rows, bool stream, uint32_t most, bool forced,
+template <typename G, typename A>
+bool ordered_by_teams(const G& g, const A* a, size_t bytes, bool rows, bool stream, uint32_t most, bool forced,
                       void* state, hipStream_t st)
 {
     constexpr bool kForward = std::is_same<A, OnceForward<double>>::value;
@@ -3335,8 +3337,8 @@ bool ordered_by_teams(const OrderedGeometry& g, const A* a, size_t bytes, bool r
 
 // Which of them, as for floats (once_launch, team_variant).  most_members 0: no teams, where the outputs
 // overlap the inputs or there is no state.  bytes: see PassShape.  *team: whether it is one.
-template <typename A>
-bool ordered_variant(const OrderedGeometry& g, const A* a, size_t bytes, bool rows, bool stream, uint32_t most, bool forced,
+template <typename G, typename A>
+bool ordered_variant(const G& g, const A* a, size_t bytes, bool rows, bool stream, uint32_t most, bool forced,
                      void* state, hipStream_t st, bool* team)
 {
     constexpr bool kForward = std::is_same<A, OnceForward<double>>::value;
@@ -3402,15 +3404,15 @@ bool short_once_geometry(int num_samples, int num_channels, size_t spatial, std:
 // forward, or backward, N 255, C 34, 4 x 7 x 4 5.8 us more than in two launches, N 231, C 20, 6 x 7 3.9, N 85, C 22, 4 x 7 x 5 level.
 constexpr uint32_t kShortWindows = 64;
 
-template <int VEC, int TEAM, int K>
-void issue_short_once(const ShortOnceGeometry& g, const OnceForward<double>& a, uint32_t blocks, hipStream_t st)
+template <int VEC, int TEAM, int K, typename G>
+void issue_short_once(const G& g, const OnceForward<double>& a, uint32_t blocks, hipStream_t st)
 {
-    launch(bn_short_once_forward_kernel<VEC, TEAM, K>, blocks, TEAM, st, g, a);
+    launch(bn_short_once_forward_kernel<VEC, TEAM, K, G>, blocks, TEAM, st, g, a);
 }
-template <int VEC, int TEAM, int K>
-void issue_short_once(const ShortOnceGeometry& g, const OnceBackward<double>& a, uint32_t blocks, hipStream_t st)
+template <int VEC, int TEAM, int K, typename G>
+void issue_short_once(const G& g, const OnceBackward<double>& a, uint32_t blocks, hipStream_t st)
 {
-    launch(bn_short_once_backward_kernel<VEC, TEAM, K>, blocks, TEAM, st, g, a);
+    launch(bn_short_once_backward_kernel<VEC, TEAM, K, G>, blocks, TEAM, st, g, a);
 }
 
 // Windows of workgroups of `threads` with `vectors` each that play up to most_passes ranges a thread; 0: such a workgroup does
@@ -3431,8 +3433,8 @@ uint32_t short_once_windows(ShortOnceGeometry* g, uint32_t threads, uint32_t vec
 }
 
 // False: workgroups of TEAM threads with K vectors each do not hold a channel, or are not for this call.
-template <int TEAM, int K, typename A>
-bool short_once(ShortOnceGeometry g, const A& a, hipStream_t st)
+template <int TEAM, int K, typename G, typename A>
+bool short_once(G g, const A& a, hipStream_t st)
 {
     constexpr bool kForward = std::is_same<A, OnceForward<double>>::value;
     const uint32_t windows = short_once_windows(&g, TEAM, K, short_once_passes<K, kForward>());
@@ -3460,13 +3462,9 @@ bool short_once(ShortOnceGeometry g, const A& a, hipStream_t st)
 }
 
 // The smallest workgroup that holds a channel; more threads before more vectors a thread.
-template <typename A>
-bool short_once_launch(int n, int c, size_t s, std::initializer_list<const HostTensor*> ts, const HostTensor& output, const A& a,
-                       hipStream_t st)
+template <typename G, typename A>
+bool short_once_launch(const G& g, const A& a, hipStream_t st)
 {
-    ShortOnceGeometry g;
-    if (!short_once_geometry(n, c, s, ts, output, &g))
-        return false;
     if (short_once<256, 4>(g, a, st) || short_once<512, 4>(g, a, st))
         return true;
     if constexpr (std::is_same<A, OnceForward<double>>::value)
@@ -3486,17 +3484,38 @@ size_t moved_bytes(const HostTensor& t, int n, int c, size_t s)
     return moved_bytes(all / w, w, std::max(pitch, w), sizeof(double));
 }
 
-// False: the staged kernels, in two launches.
+// Outputs whose halo is cleared, larger than this, are left to the staged calls, which store whole lines past the caches, unless a few long
+// segments, or one workgroup a channel with little halo, leave few parts of lines to store.  Forward + backward in us, staged and by
+// these: N 8, C 64, 30^3, 128 MiB 168 and 199; N 63, C 65, 29 x 39, 40 MiB 67.0 and 72.1; N 48, C 242, 9 x 8 x 7, 88 MiB 120 and 136;
+// rows of 80 elements and more: N 1, C 744, 149 x 140, 122 MiB 168 and 140; N 12, C 61, 85 x 84, 42 MiB 69 and 56; one workgroup: N 4, C 1963, 63 x 52,
+// halo of 2, 225 MiB 298 and 258; N 3, C 1290, 35 x 48, halo of 2, 60 MiB 88 and 69; smaller: N 12, C 77, 11 x 15 x 15, halo of 2, 38 MiB 58 and 42; N 5,
+// C 16, 38 x 65 30.4 and 13.7; short segments of any size: N 193, C 941, 4 x 5, 58 MiB 301 and 100.
+constexpr size_t kClearedByOrder = size_t(39) << 20;
+
+// False: the staged kernels.  halo: the output's is cleared.
 template <typename A>
 bool ordered_launch(int n, int c, size_t s, std::initializer_list<const HostTensor*> ts, const HostTensor& output,
                     std::initializer_list<const void*> inputs, const void* out, const A& a, void* state,
-                    const uint32_t* team_polls, hipStream_t st)
+                    const uint32_t* team_polls, hipStream_t st, const HaloCells* halo = nullptr)
 {
-    OrderedGeometry g;
+    ShortOnceClearing sg;
+    if (!team_polls && short_once_geometry(n, c, s, ts, output, &sg))
+    {
+        if (!halo)
+        {
+            if (short_once_launch<ShortOnceGeometry>(sg, a, st))
+                return true;
+        }
+        else
+        {
+            sg.halo = *halo;
+            if (short_once_launch(sg, a, st))
+                return true;
+        }
+    }
+    OrderedClearing g;
     bool rows, team;
-    if (!team_polls && short_once_launch(n, c, s, ts, output, a, st))
-        return true;
-    if (!ordered_geometry(n, c, s, ts, output, &g, &rows))
+    if (!ordered_geometry(n, c, s, ts, output, &g, &rows) || (halo && !rows))
         return false;
     const size_t bytes = (static_cast<size_t>(c - 1) * output.map.stride_c + static_cast<size_t>(n - 1) * output.map.stride_n
                           + short_span(output, s)) * sizeof(double);
@@ -3507,8 +3526,23 @@ bool ordered_launch(int n, int c, size_t s, std::initializer_list<const HostTens
         g.max_polls = *team_polls;
     g.streams_gradient = output.strided || streams_gradient(n * s / 2, c);
     const bool stream = !output.strided || bytes > kHaloedNormalStores;
-    return ordered_variant(g, &a, moved_bytes(output, n, c, s), rows, stream, teams ? most_members() : 0,
-                           team_polls != nullptr, state, st, &team);
+    const size_t moved = moved_bytes(output, n, c, s);
+    uint32_t most = teams ? most_members() : 0;
+    const size_t allocated = static_cast<size_t>(n) * output.map.stride_n * sizeof(double), inside = size_t(n) * c * s * sizeof(double);
+    // (units that segments fill a quarter of, in more than a round of workgroups: N 11, C 333, 8 x 6 x 7 40.0 and 42.6 us, C 165 32.9 and 24.1)
+    if (halo && c > static_cast<int>(chip_units())
+        && static_cast<size_t>(g.groups) * g.group_batches.divisor * kOrderedBatch * kBlockSize > 2 * size_t(n) * s)
+        return false;
+    if (halo && allocated > kClearedByOrder && output.row < kLongRow)
+    {
+        if (allocated * 10 > inside * 13)
+            return false;
+        most = 0; // no teams
+    }
+    if (!halo)
+        return ordered_variant<OrderedGeometry>(g, &a, moved, rows, stream, most, team_polls != nullptr, state, st, &team);
+    g.halo = *halo;
+    return ordered_variant(g, &a, moved, rows, stream, most, false, state, st, &team);
 }
 
 // team_polls: by teams or not at all, however few workgroups that is, with this many looks.
@@ -3637,6 +3671,97 @@ int clear_geometry(const h2x_haloed_geometry* h, ClearGeometry* g, size_t* bytes
     g->num_channels = static_cast<uint32_t>(c);
     *bytes = n * c * real * sizeof(float);
     return H2X_SUCCESS;
+}
+
+// Double tensors of one haloed geometry, as the calls that leave the halo alone see them, and the halo cells of a channel.
+int haloed_tensor(const h2x_haloed_geometry* h, const void* buffer, HostTensor* t, const void** interior, int* channels,
+                  size_t* spatial, HaloCells* halo)
+{
+    RealBox box;
+    size_t real;
+    int err = real_box(h, &box, &real);
+    if (err)
+        return err;
+    const int nd = h->num_dims, ns = nd - 2;
+    const size_t n = h->local_shape[nd - 1], c = h->local_shape[nd - 2];
+    if (n == 0 || c == 0 || c > 0x7fffffffull || n > 0x7fffffffull || n * c * real >= (1ull << 30))
+        return H2X_ERR_UNSUPPORTED;
+    h2x_tensor_geometry g = {};
+    g.num_dims = nd;
+    int64_t stride = 1, origin = 0;
+    for (int d = 0; d < nd; ++d)
+    {
+        if (h->local_shape[d] == 0)
+            return H2X_ERR_UNSUPPORTED;
+        g.local_shape[d] = h->local_shape[d];
+        g.strides[d] = stride;
+        origin += h->lower_halo[d] * stride;
+        stride *= h->real_shape[d];
+    }
+    *interior = static_cast<const double*>(buffer) + origin;
+    err = strided_tensor<double>(&g, *interior, static_cast<int>(n), t, channels, spatial);
+    if (err)
+        return err;
+    uint32_t local[3] = {1, 1, 1}, extent[3] = {1, 1, 1}, lo[3] = {0, 0, 0};
+    for (int d = 0; d < ns; ++d)
+    {
+        local[d] = static_cast<uint32_t>(h->local_shape[d]);
+        extent[d] = static_cast<uint32_t>(h->real_shape[d]);
+        lo[d] = static_cast<uint32_t>(h->lower_halo[d]);
+    }
+    const uint32_t samples = static_cast<uint32_t>(n);
+    halo->before = lo[0];
+    halo->after = extent[0] - lo[0] - local[0];
+    halo->width = local[0];
+    halo->h = make_fastdiv(local[1]);
+    halo->d = make_fastdiv(local[2]);
+    halo->pitch = extent[0];
+    halo->units = make_fastdiv((extent[0] + 1) / 2);
+    halo->real_h = make_fastdiv(extent[1]);
+    const uint32_t beside = extent[1] - local[1];
+    halo->beside = make_fastdiv(std::max(beside, 1u));
+    halo->outer = (extent[2] - local[2]) * extent[1];
+    const uint32_t rows = halo->outer + local[2] * beside;
+    halo->rows = make_fastdiv(std::max(rows, 1u));
+    halo->lo_y = lo[1];
+    halo->lo_z = lo[2];
+    halo->real_plane = extent[0] * extent[1];
+    halo->ends = extent[0] > local[0] ? samples * local[1] * local[2] : 0;
+    halo->whole = samples * rows * halo->units.divisor;
+    halo->stride_n = static_cast<uint32_t>(g.strides[nd - 1]);
+    halo->origin = origin;
+    return H2X_SUCCESS;
+}
+
+// A whole pass over double tensors that clears the halo, with the bits of the staged calls; H2X_ERR_UNSUPPORTED: in these.
+// `inputs`, `output`: pointers of `a`, of buffers first and then of their interiors.
+template <typename A>
+int clearing_ordered(const h2x_haloed_geometry* h, A* a, std::initializer_list<const double**> inputs, double** output,
+                     void* team_state, hipStream_t st)
+{
+    HostTensor in[2], out;
+    HaloCells halo;
+    int c;
+    size_t s, k = 0;
+    const void* interior;
+    for (const double** p : inputs)
+    {
+        const int err = *p ? haloed_tensor(h, *p, &in[k++], &interior, &c, &s, &halo) : H2X_ERR_UNSUPPORTED;
+        if (err)
+            return err;
+        *p = static_cast<const double*>(interior);
+    }
+    const int err = *output ? haloed_tensor(h, *output, &out, &interior, &c, &s, &halo) : H2X_ERR_UNSUPPORTED;
+    if (err)
+        return err;
+    *output = static_cast<double*>(const_cast<void*>(interior));
+    const int n = static_cast<int>(h->local_shape[h->num_dims - 1]);
+    bool launched;
+    if constexpr (std::is_same<A, OnceForward<double>>::value)
+        launched = ordered_launch(n, c, s, {&in[0]}, out, {a->x}, a->y, *a, team_state, nullptr, st, &halo);
+    else
+        launched = ordered_launch(n, c, s, {&in[0], &in[1]}, out, {a->x, a->dy}, a->dx, *a, team_state, nullptr, st, &halo);
+    return launched ? launch_status() : H2X_ERR_UNSUPPORTED;
 }
 
 // The same for such tensors, by one workgroup or a team a channel; H2X_ERR_UNSUPPORTED: in the
@@ -4174,8 +4299,17 @@ extern "C" int h2x_bn_forward_clearing(h2x_dtype dtype, const h2x_haloed_geometr
 {
     if (!geometry || !scale || !bias || !mean || !var || !running_mean || !running_var)
         return H2X_ERR_INVALID_ARGUMENT;
-    if (dtype != H2X_F32 || num_per_sum == 0)
+    if ((dtype != H2X_F32 && dtype != H2X_F64) || num_per_sum == 0)
         return H2X_ERR_UNSUPPORTED;
+    if (dtype == H2X_F64)
+    {
+        typedef double T;
+        OnceForward<T> a{static_cast<const T*>(x_buffer), static_cast<const T*>(scale), static_cast<const T*>(bias),
+                         static_cast<T*>(mean), static_cast<T*>(var), static_cast<T*>(running_mean),
+                         static_cast<T*>(running_var), static_cast<T*>(y_buffer), static_cast<T>(num_per_sum),
+                         static_cast<T>(decay), static_cast<T>(epsilon)};
+        return clearing_ordered(geometry, &a, {&a.x}, &a.y, team_state, as_stream(stream));
+    }
     typedef float T;
     const OnceForward<T> a{static_cast<const T*>(x_buffer), static_cast<const T*>(scale), static_cast<const T*>(bias),
                            static_cast<T*>(mean), static_cast<T*>(var), static_cast<T*>(running_mean),
@@ -4192,6 +4326,16 @@ extern "C" int h2x_bn_backward_clearing(h2x_dtype dtype, size_t num_per_sum, con
 {
     if (!geometry || !mean || !var || !scale || !dscale || !dbias || !dmean || !dvar)
         return H2X_ERR_INVALID_ARGUMENT;
+    if (dtype == H2X_F64)
+    {
+        typedef double T;
+        OnceBackward<T> a{static_cast<const T*>(x_buffer), static_cast<const T*>(dy_buffer),
+                          static_cast<const T*>(mean), static_cast<const T*>(var), static_cast<const T*>(scale),
+                          static_cast<T*>(dscale), static_cast<T*>(dbias), static_cast<T*>(dmean),
+                          static_cast<T*>(dvar), static_cast<T*>(dx_buffer), static_cast<T>(num_per_sum),
+                          static_cast<T>(num_per_sum - 1), static_cast<T>(epsilon)};
+        return clearing_ordered(geometry, &a, {&a.x, &a.dy}, &a.dx, team_state, as_stream(stream));
+    }
     if (dtype != H2X_F32)
         return H2X_ERR_UNSUPPORTED;
     typedef float T;

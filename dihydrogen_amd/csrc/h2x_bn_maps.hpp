@@ -208,5 +208,58 @@ __host__ __device__ __forceinline__ void interior_mask(const RealBox& b, uint32_
     }
 }
 
+// The halo cells of a channel, all samples: those at the ends of the interior rows, and the rows that lie in the halo whole.
+struct HaloCells
+{
+    uint32_t before, after;  // cells of a real row on either side of its interior ones
+    uint32_t width;          // and those between
+    FastDiv h, d;            // interior rows of a plane, planes of a segment
+    uint32_t pitch;          // cells of a real row
+    FastDiv units;           // pairs of cells that it is padded to: the last one starts early (one cell: a pitch of 1)
+    FastDiv real_h;          // real rows of a plane
+    FastDiv beside, rows;    // halo rows of an interior plane (at least 1: there may be none), of a segment
+    uint32_t outer;          // of these in planes of the halo: they come first
+    uint32_t lo_y, lo_z;     // rows before the interior ones, planes likewise
+    uint32_t real_plane;     // cells
+    uint32_t ends, whole;    // interior rows with ends, units of halo rows: of all samples
+    uint32_t stride_n;
+    int64_t origin;          // of the first interior element, from the start of the segment
+};
+
+// Element offset, from the start of the channel's first segment, of the first cell of interior row i; the cells before and after the
+// row's interior ones are to be cleared.
+__host__ __device__ __forceinline__ uint32_t halo_row_start(const HaloCells& g, uint32_t i)
+{
+    const uint32_t q = fastdiv(i, g.h), y = i - q * g.h.divisor;
+    const uint32_t n = fastdiv(q, g.d), z = q - n * g.d.divisor;
+    return n * g.stride_n + (z + g.lo_z) * g.real_plane + (y + g.lo_y) * g.pitch;
+}
+
+// The same of unit i of the rows that lie in the halo whole.
+__host__ __device__ __forceinline__ uint32_t halo_whole_unit(const HaloCells& g, uint32_t i)
+{
+    const uint32_t r = fastdiv(i, g.units), pair = 2 * (i - r * g.units.divisor);
+    const uint32_t x = pair + 2 <= g.pitch || g.pitch == 1 ? pair : g.pitch - 2;
+    const uint32_t n = fastdiv(r, g.rows);
+    uint32_t k = r - n * g.rows.divisor, y, z;
+    if (k < g.outer)
+    {
+        z = fastdiv(k, g.real_h);
+        y = k - z * g.real_h.divisor;
+        if (z >= g.lo_z)
+            z += g.d.divisor;
+    }
+    else
+    {
+        k -= g.outer;
+        z = fastdiv(k, g.beside);
+        y = k - z * g.beside.divisor;
+        z += g.lo_z;
+        if (y >= g.lo_y)
+            y += g.h.divisor;
+    }
+    return n * g.stride_n + z * g.real_plane + y * g.pitch + x;
+}
+
 } // namespace bn
 } // namespace h2x

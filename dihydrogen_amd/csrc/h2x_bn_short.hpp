@@ -33,6 +33,12 @@ struct ShortOnceGeometry
     uint32_t num_samples, num_channels;
 };
 
+// Haloed tensors of one geometry whose output's halo is cleared.
+struct ShortOnceClearing : ShortOnceGeometry
+{
+    HaloCells halo;
+};
+
 // What a lane plays.
 struct ShortOnceLane
 {
@@ -164,8 +170,8 @@ __device__ __forceinline__ void short_once_each(const ShortOnceGeometry& g, cons
     }
 }
 
-template <int VEC, int TEAM, int K>
-__global__ __launch_bounds__(TEAM) void bn_short_once_forward_kernel(const ShortOnceGeometry g, const OnceForward<double> a)
+template <int VEC, int TEAM, int K, typename G>
+__global__ __launch_bounds__(TEAM) void bn_short_once_forward_kernel(const G g, const OnceForward<double> a)
 {
     typedef double T;
     constexpr int kPasses = short_once_passes<K, true>();
@@ -204,6 +210,9 @@ __global__ __launch_bounds__(TEAM) void bn_short_once_forward_kernel(const Short
                 }
             });
     short_once_totals<TEAM, kPasses, 2>(g, l, s, sums);
+    if constexpr (std::is_same<G, ShortOnceClearing>::value)
+        for (uint32_t i = 0; i < g.channels.divisor && first + i < g.num_channels; ++i)
+            clear_halo_cells(g.halo, a.y + (first + i) * g.stride_c, threadIdx.x, TEAM);
     if (!l.live)
         return;
     T m, variance;
@@ -224,8 +233,8 @@ __global__ __launch_bounds__(TEAM) void bn_short_once_forward_kernel(const Short
         none);
 }
 
-template <int VEC, int TEAM, int K>
-__global__ __launch_bounds__(TEAM) void bn_short_once_backward_kernel(const ShortOnceGeometry g, const OnceBackward<double> a)
+template <int VEC, int TEAM, int K, typename G>
+__global__ __launch_bounds__(TEAM) void bn_short_once_backward_kernel(const G g, const OnceBackward<double> a)
 {
     typedef double T;
     constexpr int kPasses = short_once_passes<K, false>();
@@ -279,6 +288,9 @@ __global__ __launch_bounds__(TEAM) void bn_short_once_backward_kernel(const Shor
                 }
             });
     short_once_totals<TEAM, kPasses, 4>(g, l, s, sums);
+    if constexpr (std::is_same<G, ShortOnceClearing>::value)
+        for (uint32_t i = 0; i < g.channels.divisor && first + i < g.num_channels; ++i)
+            clear_halo_cells(g.halo, a.dx + (first + i) * g.stride_c, threadIdx.x, TEAM);
     if (!l.live)
         return;
     if (threadIdx.x == l.channel * g.slots.divisor)

@@ -179,7 +179,7 @@ class BatchNormalization:
         """Where the workgroups that share a channel exchange its sums; None where no workgroups
         do.  Smaller channels than 16 K floats or 4 K doubles need none."""
         double = l.dtype == capi.F64
-        if l.samples * l.spatial_real <= (4096 if double else 16384) or double and clearing:
+        if l.samples * l.spatial_real <= (4096 if double else 16384):
             return None
         kept = self._kept.get(st) or _first_use(self._kept, st)
         channels, state = kept.state
