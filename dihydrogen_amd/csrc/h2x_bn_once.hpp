@@ -167,6 +167,8 @@ struct OnceForward
     const T *x, *scale, *bias;
     T *mean, *var, *running_mean, *running_var, *y;
     T n, decay, epsilon;
+    // a program that keeps no running statistics may give the buffers of mean and variance for them, or one for both
+    bool shared = running_mean == mean || running_mean == var || running_var == mean || running_var == var || running_var == running_mean;
 };
 
 // What the threads of channel c need once its sums are there, loaded before the elements: behind the sums nothing else hides the
@@ -180,9 +182,17 @@ struct ChannelParams
         : scale(a.scale[c]), bias(a.bias[c]), running_mean(a.running_mean[c]), running_var(a.running_var[c])
     {
     }
-    // by one thread a channel
+    // By one thread a channel.  Shared buffers are read where they are due, as in the staged calls.
     __device__ __forceinline__ void store_statistics(const OnceForward<T>& a, uint32_t c, T m, T variance) const
     {
+        if (a.shared) // uniform
+        {
+            a.mean[c] = m;
+            a.var[c] = variance;
+            a.running_mean[c] = fma_t(a.decay, a.running_mean[c], (T(1) - a.decay) * m);
+            a.running_var[c] = fma_t(a.decay, a.running_var[c], (T(1) - a.decay) * variance);
+            return;
+        }
         a.mean[c] = m;
         a.var[c] = variance;
         a.running_mean[c] = fma_t(a.decay, running_mean, (T(1) - a.decay) * m);
