@@ -171,9 +171,19 @@ struct OnceForward
     bool shared = running_mean == mean || running_mean == var || running_var == mean || running_var == var || running_var == running_mean;
 };
 
+// By one thread a channel; the running statistics are read where they are due.
+template <typename T>
+__device__ __forceinline__ void update_statistics(const OnceForward<T>& a, uint32_t c, T m, T variance)
+{
+    a.mean[c] = m;
+    a.var[c] = variance;
+    a.running_mean[c] = fma_t(a.decay, a.running_mean[c], (T(1) - a.decay) * m);
+    a.running_var[c] = fma_t(a.decay, a.running_var[c], (T(1) - a.decay) * variance);
+}
+
 // What the threads of channel c need once its sums are there, loaded before the elements: behind the sums nothing else hides the
-// wait (forward in us, loaded behind the sums and so: N 24, C 224, 5 x 4 3.58 and 3.16; N 3, C 17, 31 x 22 x 18, by teams, 5.53 and
-// 5.14; N 16, C 256, 28 x 28 6.59 and 6.42; N 64, C 512, 14 x 14 11.16 and 10.97; from 20 us on equal).
+// wait (forward in us, loaded behind the sums and so: N 24, C 224, 5 x 4 3.40 and 3.08; N 16, C 256, 28 x 28 6.59 and 6.42; N 64, C 512,
+// 14 x 14 12.2 and 12.0; from 20 us on equal).
 template <typename T>
 struct ChannelParams
 {
@@ -182,17 +192,11 @@ struct ChannelParams
         : scale(a.scale[c]), bias(a.bias[c]), running_mean(a.running_mean[c]), running_var(a.running_var[c])
     {
     }
-    // By one thread a channel.  Shared buffers are read where they are due, as in the staged calls.
+    // by one thread a channel
     __device__ __forceinline__ void store_statistics(const OnceForward<T>& a, uint32_t c, T m, T variance) const
     {
         if (a.shared) // uniform
-        {
-            a.mean[c] = m;
-            a.var[c] = variance;
-            a.running_mean[c] = fma_t(a.decay, a.running_mean[c], (T(1) - a.decay) * m);
-            a.running_var[c] = fma_t(a.decay, a.running_var[c], (T(1) - a.decay) * variance);
-            return;
-        }
+            return update_statistics(a, c, m, variance);
         a.mean[c] = m;
         a.var[c] = variance;
         a.running_mean[c] = fma_t(a.decay, running_mean, (T(1) - a.decay) * m);

@@ -208,15 +208,23 @@ __device__ __forceinline__ void add_backward_terms(double (&s)[4], const T (&x)[
         }
 }
 
+// Scale and bias are loaded behind the elements: they are scalars, and a wave that asks for them first waits for them before its first
+// element.  The exchange hides them (forward in us, loaded behind the exchange, before the elements and so: N 3, C 17, 31 x 22 x 18 5.4, 5.1 and 5.1;
+// N 32, C 256, 56 x 56 41.0, 40.2 and 39.6, over one set of tensors 33.0, 34.7 and 33.5; N 4, C 64, 64^3 102.8, 102.7 and 101.8, over one set 83.7, 86.3 and
+// 84.8, where what is loaded late spreads the stores).
+// kOneByOne: a wave of a large member whose output's halo is cleared waits for each of its stores (forward in us, at once and so: N 29, C 24, 19 x 32 x 29 31.3
+// and 29.5; N 9, C 128, 124 x 107 30.8 and 28.4; N 3, C 373, 27 x 29 x 38, halo of 2 83.6 and 78.2; N 188, C 301, 8 x 7 x 8 89.6 and 84.9).  Members of 8
+// vectors a thread lose by it (N 3, C 655, 121 x 88 31.1 and 33.2; N 166, C 201, 14 x 20, halo of 2 22.4 and 23.4), dense tensors too where they go round
+// several sets (N 1, C 64, 128 x 128 x 64 95.8 and 100).
 template <typename T, int TEAM, int K, bool STREAM, typename G>
 __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometry<G> g, const OnceForward<T> a,
                                                                       unsigned long long* states)
 {
     constexpr int VEC = 16 / sizeof(T);
+    constexpr bool kOneByOne = G::kClears && K == 16;
     __shared__ TeamShared<TEAM, 2> shared;
     const uint32_t c = fastdiv(blockIdx.x, g.members);
     const uint32_t member = team_member(blockIdx.x - c * g.members.divisor, g.members.divisor);
-    const ChannelParams<T> params(a, c);
     const T* const x = a.x + c * g.once.stride_c;
     unsigned long long* const state = states + team_state_at(c);
     uint32_t tag = team_tag(state);
@@ -232,6 +240,7 @@ __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometr
             at[u] = once_place<VEC>(g.once, first + u * TEAM + threadIdx.x);
             load_vec<T, VEC, false>(x + G::offset(at[u]), v[u]);
         }
+    const T sc = a.scale[c], bi = a.bias[c];
     double s[2] = {0.0, 0.0};
 #pragma unroll
     for (int u = 0; u < K; ++u)
@@ -252,9 +261,8 @@ __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometr
     T m, variance;
     sums_to_mean_var(static_cast<T>(s[0]), static_cast<T>(s[1]), a.n, &m, &variance);
     if (member == 0 && threadIdx.x == 0)
-        params.store_statistics(a, c, m, variance);
+        update_statistics(a, c, m, variance);
     const T inv_stdev = inv_sqrt_t(variance + a.epsilon);
-    const T sc = params.scale, bi = params.bias;
     T* const y = a.y + c * g.once.stride_c;
 #pragma unroll
     for (int u = 0; u < K; ++u)
@@ -263,6 +271,8 @@ __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometr
 #pragma unroll
             for (int j = 0; j < VEC; ++j)
                 v[u][j] = G::kClears && !G::counts(at[u], j) ? T(0) : fma_t((v[u][j] - m) * inv_stdev, sc, bi);
+            if constexpr (kOneByOne)
+                __builtin_amdgcn_s_waitcnt(0x0f70); // vector memory only
             store_once<T, VEC, STREAM>(y + G::offset(at[u]), v[u]);
         }
 }
