@@ -537,12 +537,15 @@ __device__ __forceinline__ T pixel_combine(T v, const F& f)
 // and there are as many more workgroups, for rows of 64 or 128 bytes (see launch_split_for).
 // The chain of a wave counts: 19 vector and 6 scalar instructions a channel forward, of which the exponential takes 13.  So the first
 // CERTAIN channels of a wave, which the smallest channel count of the variant has, are not asked for; a channel that is not there is
-// -infinity (backward 0), with no further question; lanes without pixels work on the tile's first one and store
-// nothing; and addresses are a running scalar pointer and a lane's offset in bytes.  Asking before each load, term
+// -infinity (backward 0), with no further question but, where a wave lacks it as a whole, one ahead of its exponential; lanes without pixels
+// work on the tile's first one and store nothing; and addresses are a running scalar pointer and a lane's offset in bytes.  Asking before each load, term
 // and store, with addresses of 64 bits a lane (23 and 22 instructions, backward 13 and 30 with registers spilled), forward + backward in
 // us -> so: N 4, C 150, 65 x 97 17.5 -> 16.8; N 2, C 209, 15 x 15 6.85 -> 5.75; N 5, C 308, 56 x 52 21.8 -> 20.6; N 2, C 322,
 // 75 x 110 26.7 -> 24.0; N 4, C 431, 99 x 126 111 -> 102; doubles N 4, C 472, 49 x 44 47.3 -> 43.6; of 47 calls the mean
-// is 0.950, and those bound by memory are level (N 1, C 39, 316 x 354 18.4 and 18.5, N 13, C 47, 220 x 134 63.6 and 64.5).
+// is 0.950.  The question ahead of the exponential is for tiles that are half empty, without it and with it: N 1, C 39, 316 x 354 (asking each time 17.9)
+// 18.0 and 17.1; N 13, C 42, 220 x 134 (56.2) 57.4 and 56.2; doubles N 4, C 33, 128 x 128 (18.0) 18.4 and 17.4.  One round of workgroups of full tiles
+// whose tensors are streamed does lose, a wave's loads now being together: N 1, C 60, 316 x 354 28.7 -> 29.5, N 8, C 60, 112 x 125 28.2 -> 29.0 (two rounds,
+// N 2, C 60, 316 x 354 52.5 -> 49.8).
 template <typename T, int VEC, int CPW, int CERTAIN, int WAVES, int LANES, bool STREAM>
 __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
     const T* __restrict__ x, T* __restrict__ y, int num_channels, size_t spatial, int flat_samples,
@@ -598,6 +601,9 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
         sum[j] = T(0);
 #pragma unroll
     for (int k = 0; k < CPW; ++k)
+    {
+        if (LANES == kWaveSize && !exists(k)) // uniform, and so are all that follow
+            break;
 #pragma unroll
         for (int j = 0; j < VEC; ++j)
         {
@@ -605,6 +611,7 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
             v[k][j] = e;
             sum[j] += e;
         }
+    }
 #pragma unroll
     for (int j = 0; j < VEC; ++j)
     {
