@@ -123,6 +123,11 @@ class BnAuditReport(ctypes.Structure):
                 ("launch", BnAuditLaunch * BN_AUDIT_MAX_LAUNCHES)]
 
 
+class BnPlannedLaunch(ctypes.Structure):
+    """struct h2x_bn_planned_launch"""
+    _fields_ = [("kernel", c_int32), ("workgroups", c_uint32), ("threads", c_uint32), ("vectors", c_uint32)]
+
+
 class ShuffleGeometry(ctypes.Structure):
     """struct h2x_shuffle_geometry"""
     _fields_ = [
@@ -248,6 +253,8 @@ SIGNATURES = {
     "h2x_copy_audit_begin": (c_int, []),
     "h2x_copy_audit_add_region": (c_int, [POINTER(CopyAuditRegion)]),
     "h2x_copy_audit_end": (c_int, [POINTER(CopyAuditReport)]),
+    "h2x_bn_planned": (c_int, [c_int, c_int, c_int, POINTER(TensorGeometry), POINTER(HaloedGeometry), c_int,
+                               POINTER(BnPlannedLaunch), POINTER(c_int)]),
     "h2x_bn_audit_clearing": (c_int, [c_int, c_int, POINTER(HaloedGeometry), POINTER(c_uint64),
                                       POINTER(BnAuditReport)]),
     "h2x_tensor_transform": (c_int, [c_int, c_int, c_int, POINTER(POINTER(TensorGeometry)), POINTER(c_void_p),

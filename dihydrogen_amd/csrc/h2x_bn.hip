@@ -83,6 +83,20 @@ int issued()
     return t_launch_log ? static_cast<int>(H2X_SUCCESS) : launch_status();
 }
 
+// A launch of a kernel whose threads hold `vectors` vectors of their channel each.
+template <typename... P, typename... A>
+void launch_whole(Kernel kernel, int vectors, void (*f)(P...), uint32_t blocks, int threads, hipStream_t st, A&&... args)
+{
+    if (!t_launch_log)
+        return launch(f, blocks, threads, st, std::forward<A>(args)...);
+    LaunchRecord r;
+    r.kernel = kernel;
+    r.grid_x = blocks;
+    r.threads = threads;
+    r.vectors = vectors;
+    logged(r);
+}
+
 // Installs a log for the lifetime of the object and puts the previous one back.
 struct ScopedLaunchLog
 {
@@ -2735,7 +2749,7 @@ constexpr unsigned int kOnceManyChannels = 96;
 template <int TEAM, int K, bool STREAM, typename G>
 void issue_once(const G& g, const OnceForward<float>& a, hipStream_t st)
 {
-    launch(bn_once_forward_kernel<float, TEAM, K, STREAM, G>, once_grid<TEAM>(g), once_block<TEAM>(), st, g, a);
+    launch_whole(kKernelOnce, K, bn_once_forward_kernel<float, TEAM, K, STREAM, G>, once_grid<TEAM>(g), once_block<TEAM>(), st, g, a);
 }
 template <int TEAM, int K, bool STREAM, typename G>
 void issue_once(const G& g, const OnceBackward<float>& a, hipStream_t st)
@@ -2747,8 +2761,8 @@ void issue_once(const G& g, const OnceBackward<float>& a, hipStream_t st)
     // spilled (9 words of scratch a lane), and the kernel remains faster than two launches: N 4, C 256, 112 x 112 47.5 ->
     // 38.7, N 2, C 512, 30^3 97 -> 90, N 16, C 1024, 54 x 54 154 -> 142 (going round three sets of tensors).
     constexpr int kInLds = TEAM * K > 8192 ? 9 : 0;
-    launch(bn_once_backward_kernel<float, TEAM, K, STREAM, kInLds, G>, once_grid<TEAM>(g), once_block<TEAM>(), st,
-           g, a);
+    launch_whole(kKernelOnce, K, bn_once_backward_kernel<float, TEAM, K, STREAM, kInLds, G>, once_grid<TEAM>(g), once_block<TEAM>(),
+                 st, g, a);
 }
 
 // A channel fits the registers of one workgroup, in a variant that pays.
@@ -2824,12 +2838,12 @@ constexpr size_t kWindowBytes = size_t(21) << 20;
 template <int K>
 void issue_window(const WindowGeometry& g, const OnceForward<float>& a, uint32_t blocks, hipStream_t st)
 {
-    launch(bn_window_forward_kernel<float, kWindowBlock, K>, blocks, kWindowBlock, st, g, a);
+    launch_whole(kKernelWindow, K, bn_window_forward_kernel<float, kWindowBlock, K>, blocks, kWindowBlock, st, g, a);
 }
 template <int K>
 void issue_window(const WindowGeometry& g, const OnceBackward<float>& a, uint32_t blocks, hipStream_t st)
 {
-    launch(bn_window_backward_kernel<float, kWindowBlock, K>, blocks, kWindowBlock, st, g, a);
+    launch_whole(kKernelWindow, K, bn_window_backward_kernel<float, kWindowBlock, K>, blocks, kWindowBlock, st, g, a);
 }
 
 // False: the call is not for windows.
@@ -2904,8 +2918,8 @@ bool streams_gradient(const G& g)
 template <typename T, int TEAM, int K, bool STREAM, typename G>
 void issue_team(const TeamGeometry<G>& g, const OnceForward<T>& a, unsigned long long* states, hipStream_t st)
 {
-    launch(bn_team_forward_kernel<T, TEAM, K, STREAM, G>, g.once.num_channels * g.members.divisor, TEAM, st, g, a,
-           states);
+    launch_whole(kKernelTeam, K, bn_team_forward_kernel<T, TEAM, K, STREAM, G>, g.once.num_channels * g.members.divisor, TEAM, st,
+                 g, a, states);
 }
 template <typename T, int TEAM, int K, bool STREAM, typename G>
 void issue_team(const TeamGeometry<G>& g, const OnceBackward<T>& a, unsigned long long* states, hipStream_t st)
@@ -2914,10 +2928,10 @@ void issue_team(const TeamGeometry<G>& g, const OnceBackward<T>& a, unsigned lon
     if constexpr (K >= 8) // the smallest members are those of small tensors
         if (streams_gradient(g.once))
         {
-            launch(bn_team_backward_kernel<T, TEAM, K, STREAM, true, G>, blocks, TEAM, st, g, a, states);
+            launch_whole(kKernelTeam, K, bn_team_backward_kernel<T, TEAM, K, STREAM, true, G>, blocks, TEAM, st, g, a, states);
             return;
         }
-    launch(bn_team_backward_kernel<T, TEAM, K, STREAM, false, G>, blocks, TEAM, st, g, a, states);
+    launch_whole(kKernelTeam, K, bn_team_backward_kernel<T, TEAM, K, STREAM, false, G>, blocks, TEAM, st, g, a, states);
 }
 
 template <int TEAM, int K, typename G, template <typename> class A, typename T>
@@ -3242,19 +3256,21 @@ template <int TEAM, int K, bool TEAMS, bool ROWS, bool STREAM, typename G>
 void issue_ordered(const G& g, const OnceForward<double>& a, unsigned long long* states, uint32_t blocks,
                    hipStream_t st)
 {
-    launch(bn_ordered_forward_kernel<TEAM, K, TEAMS, ROWS, STREAM, G>, blocks, TEAM, st, g, a, states);
+    constexpr Kernel kOrdered = TEAMS ? kKernelOrderedTeam : kKernelOrdered;
+    launch_whole(kOrdered, K, bn_ordered_forward_kernel<TEAM, K, TEAMS, ROWS, STREAM, G>, blocks, TEAM, st, g, a, states);
 }
 template <int TEAM, int K, bool TEAMS, bool ROWS, bool STREAM, typename G>
 void issue_ordered(const G& g, const OnceBackward<double>& a, unsigned long long* states, uint32_t blocks,
                    hipStream_t st)
 {
+    constexpr Kernel kOrdered = TEAMS ? kKernelOrderedTeam : kKernelOrdered;
     if constexpr (K >= 8)
         if (g.streams_gradient)
         {
-            launch(bn_ordered_backward_kernel<TEAM, K, TEAMS, ROWS, STREAM, true, G>, blocks, TEAM, st, g, a, states);
+            launch_whole(kOrdered, K, bn_ordered_backward_kernel<TEAM, K, TEAMS, ROWS, STREAM, true, G>, blocks, TEAM, st, g, a, states);
             return;
         }
-    launch(bn_ordered_backward_kernel<TEAM, K, TEAMS, ROWS, STREAM, false, G>, blocks, TEAM, st, g, a, states);
+    launch_whole(kOrdered, K, bn_ordered_backward_kernel<TEAM, K, TEAMS, ROWS, STREAM, false, G>, blocks, TEAM, st, g, a, states);
 }
 
 // Groups that a workgroup of TEAM threads with K vectors each holds.
@@ -3407,12 +3423,12 @@ constexpr uint32_t kShortWindows = 64;
 template <int VEC, int TEAM, int K, typename G>
 void issue_short_once(const G& g, const OnceForward<double>& a, uint32_t blocks, hipStream_t st)
 {
-    launch(bn_short_once_forward_kernel<VEC, TEAM, K, G>, blocks, TEAM, st, g, a);
+    launch_whole(kKernelShortOnce, K, bn_short_once_forward_kernel<VEC, TEAM, K, G>, blocks, TEAM, st, g, a);
 }
 template <int VEC, int TEAM, int K, typename G>
 void issue_short_once(const G& g, const OnceBackward<double>& a, uint32_t blocks, hipStream_t st)
 {
-    launch(bn_short_once_backward_kernel<VEC, TEAM, K, G>, blocks, TEAM, st, g, a);
+    launch_whole(kKernelShortOnce, K, bn_short_once_backward_kernel<VEC, TEAM, K, G>, blocks, TEAM, st, g, a);
 }
 
 // Windows of workgroups of `threads` with `vectors` each that play up to most_passes ranges a thread; 0: such a workgroup does
@@ -3568,12 +3584,12 @@ int forward_once(int n, const h2x_tensor_geometry* gx, const h2x_tensor_geometry
                                    static_cast<T*>(running_var), static_cast<T*>(y), static_cast<T>(num_per_sum),
                                    static_cast<T>(decay), static_cast<T>(eps)};
             if (team_polls)
-                return launch_by_teams(g, a, n, {x}, y, true, *team_polls, team_state, st) ? launch_status()
-                                                                            : H2X_ERR_UNSUPPORTED;
+                return launch_by_teams(g, a, n, {x}, y, true, *team_polls, team_state, st) ? issued()
+                                                                                           : H2X_ERR_UNSUPPORTED;
             const auto by_teams = [&] { return launch_by_teams(g, a, n, {x}, y, false, kTeamPolls, team_state, st); };
             const bool teams = teams_first(g);
             if ((teams && by_teams()) || once_launch(g, a, n, st) || (!teams && by_teams()))
-                return launch_status();
+                return issued();
         }
     }
     else if (x && y && n > 0 && c > 0 && s > 0 && num_per_sum > 0)
@@ -3583,7 +3599,7 @@ int forward_once(int n, const h2x_tensor_geometry* gx, const h2x_tensor_geometry
                                static_cast<T*>(running_var), static_cast<T*>(y), static_cast<T>(num_per_sum),
                                static_cast<T>(decay), static_cast<T>(eps)};
         if (ordered_launch(n, c, s, {&tx}, ty, {x}, y, a, team_state, team_polls, st))
-            return launch_status();
+            return issued();
     }
     if (team_polls)
         return H2X_ERR_UNSUPPORTED;
@@ -3615,12 +3631,12 @@ int backward_once(int n, size_t num_per_sum, const h2x_tensor_geometry* gx, cons
                                     static_cast<T*>(dx), static_cast<T>(num_per_sum),
                                     static_cast<T>(num_per_sum - 1), static_cast<T>(eps)};
             if (team_polls)
-                return launch_by_teams(g, a, n, {x, dy}, dx, true, *team_polls, team_state, st) ? launch_status()
-                                                                            : H2X_ERR_UNSUPPORTED;
+                return launch_by_teams(g, a, n, {x, dy}, dx, true, *team_polls, team_state, st) ? issued()
+                                                                                                : H2X_ERR_UNSUPPORTED;
             const auto by_teams = [&] { return launch_by_teams(g, a, n, {x, dy}, dx, false, kTeamPolls, team_state, st); };
             const bool teams = teams_first(g);
             if ((teams && by_teams()) || once_launch(g, a, n, st) || (!teams && by_teams()))
-                return launch_status();
+                return issued();
         }
     }
     else if (x && dy && dx && n > 0 && c > 0 && s > 0)
@@ -3631,7 +3647,7 @@ int backward_once(int n, size_t num_per_sum, const h2x_tensor_geometry* gx, cons
                                 static_cast<T*>(dx), static_cast<T>(num_per_sum),
                                 static_cast<T>(num_per_sum - 1), static_cast<T>(eps)};
         if (ordered_launch(n, c, s, {&tx, &td}, to, {x, dy}, dx, a, team_state, team_polls, st))
-            return launch_status();
+            return issued();
     }
     if (team_polls)
         return H2X_ERR_UNSUPPORTED;
@@ -3761,7 +3777,7 @@ int clearing_ordered(const h2x_haloed_geometry* h, A* a, std::initializer_list<c
         launched = ordered_launch(n, c, s, {&in[0]}, out, {a->x}, a->y, *a, team_state, nullptr, st, &halo);
     else
         launched = ordered_launch(n, c, s, {&in[0], &in[1]}, out, {a->x, a->dy}, a->dx, *a, team_state, nullptr, st, &halo);
-    return launched ? launch_status() : H2X_ERR_UNSUPPORTED;
+    return launched ? issued() : H2X_ERR_UNSUPPORTED;
 }
 
 // The same for such tensors, by one workgroup or a team a channel; H2X_ERR_UNSUPPORTED: in the
@@ -3785,7 +3801,7 @@ int clearing_once(const h2x_haloed_geometry* h, const A& a, std::initializer_lis
     };
     const bool teams = teams_first(g);
     if ((teams && by_teams()) || once_launch<true>(g, a, st) || (!teams && by_teams()))
-        return launch_status();
+        return issued();
     return H2X_ERR_UNSUPPORTED;
 }
 
@@ -4472,5 +4488,45 @@ extern "C" int h2x_bn_audit_short(int num_samples, const h2x_tensor_geometry* ge
                 }
             }
         }
+    return H2X_SUCCESS;
+}
+
+// What a whole pass over tensors of one geometry launches, by the entry points' own choice.
+extern "C" int h2x_bn_planned(int backward, h2x_dtype dtype, int num_samples, const h2x_tensor_geometry* geometry,
+                              const h2x_haloed_geometry* cleared, int with_state, h2x_bn_planned_launch* launches,
+                              int* num_launches)
+{
+    if (!geometry == !cleared || !launches || !num_launches)
+        return H2X_ERR_INVALID_ARGUMENT;
+    // addresses that nobody follows, apart from one another
+    const auto at = [](int i) { return reinterpret_cast<void*>(static_cast<uintptr_t>(i) << 40); };
+    void *const x = at(1), *const dy = at(2), *const out = at(3), *const ws = at(4), *const state = with_state ? at(5) : nullptr;
+    void *const mean = at(6), *const var = at(7), *const scale = at(8), *const s0 = at(9), *const s1 = at(10), *const s2 = at(11),
+               *const s3 = at(12);
+    constexpr size_t kPerSum = 2;
+    constexpr double kDecay = 0.9, kEpsilon = 1e-5;
+    LaunchLog log;
+    ScopedLaunchLog scope(&log);
+    int err;
+    if (cleared)
+        err = backward ? h2x_bn_backward_clearing(dtype, kPerSum, cleared, x, dy, mean, var, scale, s0, s1, s2, s3, out, kEpsilon,
+                                                  state, nullptr)
+                       : h2x_bn_forward_clearing(dtype, cleared, x, scale, s0, kPerSum, kDecay, kEpsilon, mean, var, s1, s2, out,
+                                                 state, nullptr);
+    else
+        err = backward ? h2x_bn_backward_once(dtype, num_samples, kPerSum, geometry, geometry, geometry, x, dy, mean, var, scale,
+                                              s0, s1, s2, s3, out, kEpsilon, ws, state, nullptr)
+                       : h2x_bn_forward_once(dtype, num_samples, geometry, geometry, x, scale, s0, kPerSum, kDecay, kEpsilon,
+                                             mean, var, s1, s2, out, ws, state, nullptr);
+    if (err)
+        return err;
+    if (log.records.size() > H2X_BN_AUDIT_MAX_LAUNCHES)
+        return H2X_ERR_TOO_LARGE;
+    *num_launches = static_cast<int>(log.records.size());
+    for (size_t i = 0; i < log.records.size(); ++i)
+    {
+        const LaunchRecord& r = log.records[i];
+        launches[i] = {r.kernel, r.grid_x * r.grid_y, static_cast<uint32_t>(r.threads), static_cast<uint32_t>(r.vectors)};
+    }
     return H2X_SUCCESS;
 }

@@ -24,7 +24,14 @@ enum Kernel : int
     kKernelFinish = 4,      // adds the partial sums of a reduction
     kKernelStatistics = 5,  // sums -> mean / variance / running statistics
     kKernelFill = 6,        // zeroes per-channel outputs (empty tensors)
-    kKernelClearing = 7     // normalise / input gradient over the real tensor, halo of the output zeroed
+    kKernelClearing = 7,    // normalise / input gradient over the real tensor, halo of the output zeroed
+    // kernels that hold whole channels
+    kKernelOnce = 8,         // a workgroup, or a wave, a channel
+    kKernelWindow = 9,       // a workgroup for neighbouring channels
+    kKernelTeam = 10,        // a team of workgroups a channel
+    kKernelOrdered = 11,     // doubles, in the staged order: a workgroup a channel
+    kKernelOrderedTeam = 12, // by teams
+    kKernelShortOnce = 13    // doubles, short segments: a workgroup for neighbouring channels
 };
 
 enum Family : int
@@ -62,6 +69,7 @@ struct LaunchRecord
     ShortGeometry geometry;                // short family
     RealBox box;                           // halo-clearing kernel: real extents and interior
     size_t real = 0;                       // halo-clearing kernel: cells of a real segment
+    int threads = 0, vectors = 0;          // kernels that hold whole channels: of a workgroup, of a thread
 };
 
 struct LaunchLog

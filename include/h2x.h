@@ -757,6 +757,29 @@ int h2x_bn_audit_clearing(int backward,
                           h2x_bn_audit_report* report);
 
 /**
+ * What h2x_bn_forward_once (`backward` 0) or h2x_bn_backward_once would launch for tensors of `geometry` that are apart and
+ * aligned as an allocator aligns them, or - with `cleared` in its place - h2x_bn_forward_clearing or
+ * h2x_bn_backward_clearing; with_state 0: without a team_state.  Nothing is launched.  `launches` has room for
+ * H2X_BN_AUDIT_MAX_LAUNCHES.  Returns what the entry point returns.
+ */
+typedef struct h2x_bn_planned_launch
+{
+    int32_t kernel; /* as in h2x_bn_audit_launch; 8 a workgroup a channel, 9 for neighbouring channels, 10 a team a channel; doubles:
+                       11 a workgroup a channel, 12 a team, 13 short segments */
+    uint32_t workgroups;
+    uint32_t threads, vectors; /* from kernel 8: of a workgroup; 16-byte vectors that a thread holds */
+} h2x_bn_planned_launch;
+
+int h2x_bn_planned(int backward,
+                   h2x_dtype dtype,
+                   int num_samples,
+                   const h2x_tensor_geometry* geometry,
+                   const h2x_haloed_geometry* cleared,
+                   int with_state,
+                   h2x_bn_planned_launch* launches,
+                   int* num_launches);
+
+/**
  * Launch audit of the copy entry points (halo pack / unpack / clear / fused
  * exchange, shuffle plans, pack and unpack), on the host: no GPU call is made
  * and no pointer is followed.  No counterpart in the reference.  Between

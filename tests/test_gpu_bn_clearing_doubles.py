@@ -13,7 +13,10 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(3, 5, (4, 6), (1, 1)), (24, 142, (6, 6), (1, 1)), (16, 47, (7, 6), (2, 2)), (9, 7, (3, 4, 5), (1, 2, 1)), (5, 3, (9, 1), (1, 1)),
           (26, 40, (22, 18), (1, 1)), (2, 5, (28, 23, 32), (1, 1, 1)), (20, 25, (11, 10, 7), (1, 1, 1)), (4, 30, (19, 30), (2, 0)),
           (4, 30, (19, 30), (0, 1)), (1, 29, (35, 30, 36), (1, 1, 1)), (2, 6, (20, 40, 33), (0, 1, 2)), (3, 2, (300, 40), (3, 3)),
-          (2, 300, (17, 31), (1, 1)), (70, 130, (18, 16), (1, 1))]
+          (2, 300, (17, 31), (1, 1)), (70, 130, (18, 16), (1, 1)), (4, 30, (64, 64), (0, 1))]
+# of these the ones that stay in the staged calls, one by the estimate of the time and one whose halo on the outermost dimension alone leaves
+# dense segments
+STAGED = SHAPES[-2:]
 
 
 @pytest.mark.parametrize("in_place", [False, True])

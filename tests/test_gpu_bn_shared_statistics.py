@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(torch.float32, 8, 5, (32, 32), 0), (torch.float32, 128, 1023, (7, 7), 0), (torch.float32, 2, 3, (40, 32, 32), 0),
           (torch.float32, 3, 7, (2, 1), 0), (torch.float32, 2, 96, (61, 32), 2), (torch.float64, 30, 70, (10, 11), 0),
           (torch.float64, 3, 3, (45, 47), 0), (torch.float64, 2, 2, (32, 32, 40), 0), (torch.float64, 60, 20, (6, 4), 1)]
+KERNELS = [[8], [9], [10], [0, 1], [8], [13], [11], [12], [13]]  # forward, of each: see h2x_bn_planned
 
 
 @pytest.mark.parametrize("one_buffer", [False, True])
