@@ -3448,13 +3448,54 @@ uint32_t short_once_windows(ShortOnceGeometry* g, uint32_t threads, uint32_t vec
     return (g->num_channels + channels - 1) / channels;
 }
 
+// Outputs whose halo is cleared, larger than this, are left to the staged calls, which store whole lines past the caches, unless a few long
+// segments, or one workgroup a channel with little halo, leave few parts of lines to store.  Forward + backward in us, staged and by
+// these: N 8, C 64, 30^3, 128 MiB 168 and 199; N 63, C 65, 29 x 39, 40 MiB 67.0 and 72.1; N 48, C 242, 9 x 8 x 7, 88 MiB 120 and 136;
+// rows of 80 elements and more: N 1, C 744, 149 x 140, 122 MiB 168 and 140; N 12, C 61, 85 x 84, 42 MiB 69 and 56; one workgroup: N 4, C 1963, 63 x 52,
+// halo of 2, 225 MiB 298 and 258; N 3, C 1290, 35 x 48, halo of 2, 60 MiB 88 and 69; smaller: N 12, C 77, 11 x 15 x 15, halo of 2, 38 MiB 58 and 42; N 5,
+// C 16, 38 x 65 30.4 and 13.7.
+constexpr size_t kClearedByOrder = size_t(39) << 20;
+
+// Whether short segments whose output's halo is cleared are for `windows` workgroups that hold so many vectors.  The staged calls take a
+// time for each segment, and those of up to 200 cells, allocated, are always for one launch (N 193, C 941, 4 x 5 301 and 100 us, N 176, C 910, 3 x 2
+// 255 and 38); beyond they run at memory's rate, and a workgroup with all of a channel's cells to itself needs neighbours that
+// keep memory busy.  Forward + backward in us, staged and in one launch each way, of 220 calls:
+//   few workgroups of much: N 106, C 26, 4^3, halo of 3 36 and 62; N 119, C 88, 4 x 5 x 6, halo of 2 65 and 89; N 92, C 71, 4^3, halo of 2 38 and 41; more
+//   of them N 43, C 107, 5 x 5 x 4, halo of 3 62 and 52; of little N 29, C 72, 7 x 6 x 6, halo of 2 41 and 34;
+//   the largest, one a CU, in more than one round: N 57, C 454, 18 x 9, halo of 3 95 and 115; N 36, C 359, 16 x 13, halo of 3 65 and 75; in one
+//   N 83, C 183, 9 x 13, halo of 3 61 and 49; N 53, C 120, 11 x 16, halo of 2 37 and 31;
+//   large outputs in a little more than one round: N 53, C 284, 4 x 4 x 5, halo of 2 73 and 95 (C 350 106 and 100);
+//   and with less halo than three times the interior, segments of more than 350 cells: N 22, C 1078, 20 x 12, halo of 3 115 and 123; N 18, C 896, 18 x 12,
+//   halo of 2 67 and 72; up to 350 N 41, C 556, 9 x 16, halo of 2 80 and 70; with more N 9, C 412, 7 x 5 x 4, halo of 3 55 and 40.
+bool clearing_pays(const ShortOnceClearing& g, uint32_t windows, uint32_t vectors)
+{
+    constexpr size_t kMuch = 260000;
+    const size_t segment = g.stride_c, allocated = segment * g.num_channels * g.num_samples * sizeof(double);
+    const size_t inside = static_cast<size_t>(g.halo.width) * g.halo.h.divisor * g.halo.d.divisor;
+    if (segment <= 200)
+        return true;
+    const uint32_t cus = chip_units();
+    const bool much = allocated > kMuch * windows;
+    if (much && windows * 8 < cus * 3)
+        return false;
+    if (vectors >= 1024 * 8 && windows > cus)
+        return false;
+    if (allocated <= kClearedByOrder)
+        return true;
+    return !(g.num_channels > cus && g.num_channels * 20 < cus * 23) && (segment <= 350 || segment >= 4 * inside);
+}
+bool clearing_pays(const ShortOnceGeometry&, uint32_t, uint32_t)
+{
+    return true; // nothing is cleared
+}
+
 // False: workgroups of TEAM threads with K vectors each do not hold a channel, or are not for this call.
 template <int TEAM, int K, typename G, typename A>
 bool short_once(G g, const A& a, hipStream_t st)
 {
     constexpr bool kForward = std::is_same<A, OnceForward<double>>::value;
     const uint32_t windows = short_once_windows(&g, TEAM, K, short_once_passes<K, kForward>());
-    if (windows == 0 || (g.passes > 1 && windows < kShortWindows))
+    if (windows == 0 || (g.passes > 1 && windows < kShortWindows) || !clearing_pays(g, windows, TEAM * K))
         return false;
     // The largest workgroups have to have more than ten of sixteen lanes play something (forward in us, by them less in two launches: 1024 threads
     // N 29, C 911, 12 x 20, nine, +5.0, N 38, C 489, 14 x 11 with a halo, 10.5, -4.6; 512 threads N 71, C 291, 8 x 10, ten, +3.6, N 129, C
@@ -3499,14 +3540,6 @@ size_t moved_bytes(const HostTensor& t, int n, int c, size_t s)
     const size_t w = t.row, h = t.map.h.divisor, pitch = h > 1 ? t.map.sy : s > w * h ? t.map.sz : w;
     return moved_bytes(all / w, w, std::max(pitch, w), sizeof(double));
 }
-
-// Outputs whose halo is cleared, larger than this, are left to the staged calls, which store whole lines past the caches, unless a few long
-// segments, or one workgroup a channel with little halo, leave few parts of lines to store.  Forward + backward in us, staged and by
-// these: N 8, C 64, 30^3, 128 MiB 168 and 199; N 63, C 65, 29 x 39, 40 MiB 67.0 and 72.1; N 48, C 242, 9 x 8 x 7, 88 MiB 120 and 136;
-// rows of 80 elements and more: N 1, C 744, 149 x 140, 122 MiB 168 and 140; N 12, C 61, 85 x 84, 42 MiB 69 and 56; one workgroup: N 4, C 1963, 63 x 52,
-// halo of 2, 225 MiB 298 and 258; N 3, C 1290, 35 x 48, halo of 2, 60 MiB 88 and 69; smaller: N 12, C 77, 11 x 15 x 15, halo of 2, 38 MiB 58 and 42; N 5,
-// C 16, 38 x 65 30.4 and 13.7; short segments of any size: N 193, C 941, 4 x 5, 58 MiB 301 and 100.
-constexpr size_t kClearedByOrder = size_t(39) << 20;
 
 // False: the staged kernels.  halo: the output's is cleared.
 template <typename A>

@@ -89,6 +89,19 @@ def test_doubles_whose_halo_is_cleared(n, c, spatial, halo):
         assert kernels == [[CLEARING[n, c, spatial]]] * 2
 
 
+# N, C, spatial extents, halo; forward and backward: the two sides of each line of clearing_pays
+@pytest.mark.parametrize("n,c,spatial,halo,kernels", [
+    (176, 910, (2, 3), 1, "11"), (110, 1655, (6, 5), 3, "11"),                         # up to 200 cells of a segment
+    (106, 26, (4, 4, 4), 3, "00"), (119, 88, (6, 5, 4), 2, "00"), (43, 107, (4, 5, 5), 3, "11"), (29, 72, (6, 6, 7), 2, "11"),  # few workgroups
+    (57, 454, (9, 18), 3, "00"), (83, 183, (13, 9), 3, "11"), (30, 290, (20, 12), 3, "01"),  # the largest ones, in rounds
+    (53, 284, (5, 4, 4), 2, "00"), (51, 350, (6, 4, 5), 2, "11"),                      # a little more than a round
+    (22, 1078, (12, 20), 3, "00"), (41, 556, (16, 9), 2, "11"), (9, 412, (4, 5, 7), 3, "11"), (17, 482, (14, 16), 2, "11")])  # large outputs
+def test_short_segments_whose_halo_is_cleared(n, c, spatial, halo, kernels):
+    for backward in (0, 1):
+        planned = _kernels(backward, capi.F64, n, cleared=_haloed(spatial + (c, n), (halo,) * len(spatial)))
+        assert planned == ([SHORT] if kernels[backward] == "1" else None)
+
+
 @pytest.mark.parametrize("dtype,n,c,spatial,halo", shared.SHAPES)
 def test_shared_statistics_come_by_every_way(dtype, n, c, spatial, halo):
     real = tuple(e + 2 * halo for e in spatial)
