@@ -2037,12 +2037,24 @@ Chunking elementwise_chunking(size_t spatial, size_t segments, int vw, int unrol
 // (With normal stores of dx, and of passes that finish their sums, training in stages loses up to 10 %: N 8, C 60, 129 x 142, 35 MiB 60.7 and 66.1.)
 constexpr size_t kNormalStores = size_t(32) << 20;
 
-bool stored_normally(const HostTensor& output, int num_samples, int num_channels, size_t spatial, size_t elem_bytes)
+// Of tensors with one plane a channel and segments beyond the short ones, whose partial lines are few or many to a workgroup, these lose (inference, us,
+// past the caches and normally, of 190 calls): from 5 to 10 MiB, where three sets of inputs stay in the L2 if nothing else goes there, N 15, C 16, 65 x 99, halo
+// of 2 4.78 and 5.13, doubles N 3, C 11, 183 x 151, halo of 2 4.53 and 5.00 (below 5 MiB 0.98 of the time on average); and segments of up to 700 floats or 470
+// doubles, N 68, C 61, 17 x 27, halo of 2, 10 MiB 6.86 and 7.58, N 36, C 310, 19 x 23, 22 MiB 12.5 and 13.4, doubles N 13, C 195, 20 x 23, halo of 2 6.23 and
+// 6.68.  The others from 10 MiB N 29, C 15, 94 x 75 7.15 and 6.77, N 62, C 35, 38 x 37, halo of 3 8.50 and 7.50, doubles N 58, C 88, 23 x 30 13.4 and 12.2; several planes of any size 0.78 to 1.04 of the time, 0.92 on average.
+constexpr size_t kPlaneInL2 = size_t(5) << 20, kPlaneBeyondL2 = size_t(10) << 20, kPlaneFloats = 700, kPlaneDoubles = 470;
+
+bool stored_normally(const HostTensor& output, int num_samples, int num_channels, size_t spatial, size_t elem_bytes, bool is_short)
 {
-    return output.strided
-           && (static_cast<size_t>(num_channels - 1) * output.map.stride_c
-               + static_cast<size_t>(num_samples - 1) * output.map.stride_n + short_span(output, spatial)) * elem_bytes
-                  <= kNormalStores;
+    if (!output.strided)
+        return false;
+    const size_t bytes = (static_cast<size_t>(num_channels - 1) * output.map.stride_c
+                          + static_cast<size_t>(num_samples - 1) * output.map.stride_n + short_span(output, spatial)) * elem_bytes;
+    if (bytes > kNormalStores)
+        return false;
+    const bool one_plane = spatial == static_cast<size_t>(output.map.w.divisor) * output.map.h.divisor;
+    return is_short || !one_plane || bytes < kPlaneInL2
+           || (bytes >= kPlaneBeyondL2 && spatial > (elem_bytes == sizeof(float) ? kPlaneFloats : kPlaneDoubles));
 }
 
 template <typename T>
@@ -2053,9 +2065,9 @@ int apply_impl(int num_samples, int num_channels, size_t spatial, const HostTens
 {
     if (static_cast<size_t>(num_samples) * num_channels == 0 || spatial == 0)
         return H2X_SUCCESS;
-    const bool normally = stored_normally(ty_in, num_samples, num_channels, spatial, sizeof(T));
     ShortGeometry sg;
     const bool is_short = short_segments<T>(num_samples, num_channels, spatial, {&tx_in, &ty_in}, &sg);
+    const bool normally = stored_normally(ty_in, num_samples, num_channels, spatial, sizeof(T), is_short);
     if (fused && fused->sequential != is_short)
         return H2X_ERR_UNSUPPORTED; // the partials are laid out for the other family of kernels
     if (is_short)

@@ -1,4 +1,5 @@
-"""Normalising haloed tensors with statistics that are given: outputs up to 32 MiB are stored normally, larger ones past the caches.
+"""Normalising haloed tensors with statistics that are given: outputs up to 32 MiB are stored normally but for some of one plane, larger
+ones past the caches.
 The samples of a larger tensor, all at once and in two halves: the same bits, and the halo as it was."""
 import pytest
 import torch
