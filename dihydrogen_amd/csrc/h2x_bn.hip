@@ -3430,7 +3430,9 @@ bool short_once_geometry(int num_samples, int num_channels, size_t spatial, std:
 
 // Fewer windows than this that play ranges one after another (g.passes) leave the chip idle longer than a second launch takes:
 // forward, or backward, N 255, C 34, 4 x 7 x 4 5.8 us more than in two launches, N 231, C 20, 6 x 7 3.9, N 85, C 22, 4 x 7 x 5 level.
-constexpr uint32_t kShortWindows = 64;
+// So do the largest workgroups with many samples, whose rows one thread adds up: forward in us, in two launches and so, N 112, C 10, 5 x 4 x 6 8.3 and 10.2, N 145,
+// C 13, 7 x 8 8.2 and 9.5, N 83, C 27, 10 x 11 with a halo 8.9 and 10.0; N 56, C 21, 5 x 6 x 5 with a halo 9.0 and 8.5, N 34, C 12, 17 x 15 with a halo 8.4 and 8.2.
+constexpr uint32_t kShortWindows = 64, kShortManySamples = 64;
 
 template <int VEC, int TEAM, int K, typename G>
 void issue_short_once(const G& g, const OnceForward<double>& a, uint32_t blocks, hipStream_t st)
@@ -3507,7 +3509,8 @@ bool short_once(G g, const A& a, hipStream_t st)
 {
     constexpr bool kForward = std::is_same<A, OnceForward<double>>::value;
     const uint32_t windows = short_once_windows(&g, TEAM, K, short_once_passes<K, kForward>());
-    if (windows == 0 || (g.passes > 1 && windows < kShortWindows) || !clearing_pays(g, windows, TEAM * K))
+    const bool idles = g.passes > 1 || (TEAM * K >= 1024 * 8 && g.num_samples > kShortManySamples);
+    if (windows == 0 || (idles && windows < kShortWindows) || !clearing_pays(g, windows, TEAM * K))
         return false;
     // The largest workgroups have to have more than ten of sixteen lanes play something (forward in us, by them less in two launches: 1024 threads
     // N 29, C 911, 12 x 20, nine, +5.0, N 38, C 489, 14 x 11 with a halo, 10.5, -4.6; 512 threads N 71, C 291, 8 x 10, ten, +3.6, N 129, C

@@ -77,6 +77,12 @@ def test_short_segments_of_doubles(shape):
     assert backward == (TWO_LAUNCHES[1] if shape in TWO_BOTH_WAYS + TWO_BACKWARD else [SHORT])
 
 
+@pytest.mark.parametrize("n,c,d,h,w,halo,forward", [(112, 10, 5, 4, 6, 0, TWO_LAUNCHES[0]), (83, 27, 1, 10, 11, 1, TWO_LAUNCHES[0]),
+                                                    (56, 21, 5, 6, 5, 1, [SHORT]), (139, 70, 1, 9, 7, 0, [SHORT])])
+def test_few_workgroups_with_many_samples(n, c, d, h, w, halo, forward):
+    assert _once(capi.F64, n, c, d, h, w, halo)[0] == forward
+
+
 CLEARING = dict(zip([s[:3] for s in clearing.SHAPES], [SHORT] * 5 + [ORDERED_TEAM] * 3 + [ORDERED] * 2 + [ORDERED_TEAM] * 3 + [ORDERED]))
 
 
