@@ -253,6 +253,7 @@ SIGNATURES = {
     "h2x_copy_audit_begin": (c_int, []),
     "h2x_copy_audit_add_region": (c_int, [POINTER(CopyAuditRegion)]),
     "h2x_copy_audit_end": (c_int, [POINTER(CopyAuditReport)]),
+    "h2x_bn_audit_cleared": (c_int, [POINTER(HaloedGeometry), c_uint32, c_void_p, c_size_t]),
     "h2x_bn_planned": (c_int, [c_int, c_int, c_int, POINTER(TensorGeometry), POINTER(HaloedGeometry), c_int,
                                POINTER(BnPlannedLaunch), POINTER(c_int)]),
     "h2x_bn_audit_clearing": (c_int, [c_int, c_int, POINTER(HaloedGeometry), POINTER(c_uint64),

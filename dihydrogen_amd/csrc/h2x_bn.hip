@@ -3508,7 +3508,7 @@ template <int TEAM, int K, typename G, typename A>
 bool short_once(G g, const A& a, hipStream_t st)
 {
     constexpr bool kForward = std::is_same<A, OnceForward<double>>::value;
-    const uint32_t windows = short_once_windows(&g, TEAM, K, short_once_passes<K, kForward>());
+    const uint32_t windows = short_once_windows(&g, TEAM, K, short_once_passes(K, kForward));
     const bool idles = g.passes > 1 || (TEAM * K >= 1024 * 8 && g.num_samples > kShortManySamples);
     if (windows == 0 || (idles && windows < kShortWindows) || !clearing_pays(g, windows, TEAM * K))
         return false;
@@ -3533,18 +3533,31 @@ bool short_once(G g, const A& a, hipStream_t st)
     return true;
 }
 
-// The smallest workgroup that holds a channel; more threads before more vectors a thread.
+template <int THREADS, int VECTORS>
+struct ShortWorkgroup
+{
+    static constexpr int threads = THREADS, vectors = VECTORS;
+};
+
+// f of the workgroups that there are, until one is true: the smallest first, more threads before more vectors a thread.
+template <bool FORWARD, typename F>
+bool any_short_workgroup(const F& f)
+{
+    if (f(ShortWorkgroup<256, 4>()) || f(ShortWorkgroup<512, 4>()))
+        return true;
+    if constexpr (FORWARD)
+        return f(ShortWorkgroup<256, 8>()) || f(ShortWorkgroup<512, 8>()) || f(ShortWorkgroup<1024, 8>()) || f(ShortWorkgroup<512, 16>());
+    else
+        return f(ShortWorkgroup<1024, 4>()) || f(ShortWorkgroup<256, 8>()) || f(ShortWorkgroup<512, 8>())
+               || f(ShortWorkgroup<1024, 8>()) || f(ShortWorkgroup<256, 16>());
+}
+
+// The smallest workgroup that holds a channel.
 template <typename G, typename A>
 bool short_once_launch(const G& g, const A& a, hipStream_t st)
 {
-    if (short_once<256, 4>(g, a, st) || short_once<512, 4>(g, a, st))
-        return true;
-    if constexpr (std::is_same<A, OnceForward<double>>::value)
-        return short_once<256, 8>(g, a, st) || short_once<512, 8>(g, a, st) || short_once<1024, 8>(g, a, st)
-               || short_once<512, 16>(g, a, st);
-    else
-        return short_once<1024, 4>(g, a, st) || short_once<256, 8>(g, a, st) || short_once<512, 8>(g, a, st)
-               || short_once<1024, 8>(g, a, st) || short_once<256, 16>(g, a, st);
+    return any_short_workgroup<std::is_same<A, OnceForward<double>>::value>(
+        [&](auto w) { return short_once<decltype(w)::threads, decltype(w)::vectors>(g, a, st); });
 }
 
 size_t moved_bytes(const HostTensor& t, int n, int c, size_t s)
@@ -4499,7 +4512,7 @@ extern "C" int h2x_bn_audit_short(int num_samples, const h2x_tensor_geometry* ge
                                   unsigned int vectors, unsigned char* counted, unsigned char* stored, unsigned short* range,
                                   size_t elements)
 {
-    if (!geometry || !counted || !stored || !range || threads == 0 || threads > 1024)
+    if (!geometry || !counted || !stored || !range)
         return H2X_ERR_INVALID_ARGUMENT;
     HostTensor t;
     ShortOnceGeometry g;
@@ -4511,7 +4524,10 @@ extern "C" int h2x_bn_audit_short(int num_samples, const h2x_tensor_geometry* ge
     if (num_samples <= 0 || c <= 0 || s == 0
         || !(backward ? short_once_geometry(num_samples, c, s, {&t, &t}, t, &g) : short_once_geometry(num_samples, c, s, {&t}, t, &g)))
         return H2X_ERR_UNSUPPORTED;
-    const uint32_t windows = short_once_windows(&g, threads, vectors, 4), vec = g.row == 1 ? 1 : 2;
+    const auto same = [&](auto w) { return decltype(w)::threads == threads && decltype(w)::vectors == vectors; };
+    if (!(backward ? any_short_workgroup<false>(same) : any_short_workgroup<true>(same)))
+        return H2X_ERR_INVALID_ARGUMENT;
+    const uint32_t windows = short_once_windows(&g, threads, vectors, short_once_passes(vectors, !backward)), vec = g.row == 1 ? 1 : 2;
     if (windows == 0)
         return H2X_ERR_UNSUPPORTED;
     for (uint32_t w = 0; w < windows; ++w)
@@ -4537,6 +4553,40 @@ extern "C" int h2x_bn_audit_short(int num_samples, const h2x_tensor_geometry* ge
             }
         }
     return H2X_SUCCESS;
+}
+
+// Plays on the host which cells the passes over double tensors clear, by so many threads a channel.
+extern "C" int h2x_bn_audit_cleared(const h2x_haloed_geometry* geometry, unsigned int threads, unsigned char* cleared, size_t cells)
+{
+    if (!geometry || !cleared || threads == 0)
+        return H2X_ERR_INVALID_ARGUMENT;
+    HostTensor t;
+    HaloCells halo;
+    int c;
+    size_t s;
+    const void* interior;
+    const int err = haloed_tensor(geometry, reinterpret_cast<const void*>(uintptr_t(256)), &t, &interior, &c, &s, &halo);
+    if (err)
+        return err;
+    size_t outside = 0;
+    for (int channel = 0; channel < c; ++channel)
+    {
+        // (the kernels start from the interior's first element of the channel)
+        const int64_t first = static_cast<const double*>(interior) - reinterpret_cast<const double*>(uintptr_t(256))
+                              + channel * t.map.stride_c - halo.origin;
+        const auto one = [&](uint32_t i) {
+            if (static_cast<size_t>(first + i) < cells)
+                cleared[first + i] = 1;
+            else
+                ++outside;
+        };
+        for (uint32_t at = 0; at < threads; ++at)
+            each_halo_cell(halo, at, threads, one, [&](uint32_t i) {
+                one(i);
+                one(i + 1);
+            });
+    }
+    return outside ? H2X_ERR_INVALID_ARGUMENT : H2X_SUCCESS;
 }
 
 // What a whole pass over tensors of one geometry launches, by the entry points' own choice.

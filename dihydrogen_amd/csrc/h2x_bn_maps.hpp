@@ -261,5 +261,28 @@ __host__ __device__ __forceinline__ uint32_t halo_whole_unit(const HaloCells& g,
     return n * g.stride_n + z * g.real_plane + y * g.pitch + x;
 }
 
+// The halo cells of a channel that thread `at` of `threads` clears, as offsets from the start of the channel's first segment:
+// one(i), or pair(i) for i and i + 1 (some pairs share a cell).
+template <typename One, typename Pair>
+__host__ __device__ __forceinline__ void each_halo_cell(const HaloCells& g, uint32_t at, uint32_t threads, const One& one,
+                                                        const Pair& pair)
+{
+    for (uint32_t i = at; i < g.ends; i += threads)
+    {
+        const uint32_t row = halo_row_start(g, i);
+        for (uint32_t j = 0; j < g.before; ++j)
+            one(row + j);
+        for (uint32_t j = 0; j < g.after; ++j)
+            one(row + g.before + g.width + j);
+    }
+    for (uint32_t i = at; i < g.whole; i += threads)
+    {
+        if (g.pitch > 1) // uniform
+            pair(halo_whole_unit(g, i));
+        else
+            one(halo_whole_unit(g, i));
+    }
+}
+
 } // namespace bn
 } // namespace h2x

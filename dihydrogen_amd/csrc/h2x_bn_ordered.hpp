@@ -46,33 +46,18 @@ struct OrderedClearing : OrderedGeometry
 
 // Zeros in the halo cells of a channel, by threads `at`, at + threads, ...  (Whole passes of doubles, forward + backward in us, in the staged calls,
 // up to seven launches, and so: N 1, C 115, 49 x 58, halo of 2 30.9 -> 10.7; N 24, C 542, 6 x 6 36.7 -> 17.8; N 12, C 61, 85 x 84 69 -> 56; 80
-// drawn calls 0.76 of their time.)  Behind the stores of the interior, whose lines they
-// complete while these are in the cache; stored normally, as those are.
+// drawn calls 0.76 of their time.)  Stored normally, as the interior is, whose lines they complete in the cache: behind it, or, by the kernels
+// of short segments, before it.
 template <typename T>
 __device__ __forceinline__ void clear_halo_cells(const HaloCells& g, T* interior, uint32_t at, uint32_t threads)
 {
     T* const y = interior - g.origin;
-    for (uint32_t i = at; i < g.ends; i += threads)
-    {
-        T* const row = y + halo_row_start(g, i);
-        for (uint32_t j = 0; j < g.before; ++j)
-            row[j] = T(0);
-        for (uint32_t j = 0; j < g.after; ++j)
-            row[g.before + g.width + j] = T(0);
-    }
-    for (uint32_t i = at; i < g.whole; i += threads)
-    {
-        T* const p = y + halo_whole_unit(g, i);
-        if (g.pitch > 1) // uniform
-        {
+    each_halo_cell(
+        g, at, threads, [&](uint32_t i) { y[i] = T(0); },
+        [&](uint32_t i) {
             const T zeros[2] = {T(0), T(0)};
-            store_once<T, 2, false>(p, zeros);
-        }
-        else
-        {
-            *p = T(0);
-        }
-    }
+            store_once<T, 2, false>(y + i, zeros);
+        });
 }
 
 constexpr int kOrderedBatch = 4; // vectors a thread: kUnroll of the staged kernels

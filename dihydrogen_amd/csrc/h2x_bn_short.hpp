@@ -146,10 +146,9 @@ __device__ __forceinline__ void short_once_totals(const ShortOnceGeometry& g, co
 // Ranges that one thread plays, at most: a workgroup keeps the sums of each of its threads for each.  Backward no more than leave
 // the CU as many workgroups as its registers do (four ranges, or two by 1024 threads, 1.012 times as long on average, N 10, C 52, 13 x 15 11.7 and
 // 15.0 us).
-template <int K, bool FORWARD>
-constexpr int short_once_passes()
+constexpr int short_once_passes(int vectors, bool forward)
 {
-    return FORWARD ? 4 : K / 4;
+    return forward ? 4 : vectors / 4;
 }
 
 // The vectors of a lane: f(u, n) for vector u of sample n, between them done(p) where those of a pass end.
@@ -174,7 +173,7 @@ template <int VEC, int TEAM, int K, typename G>
 __global__ __launch_bounds__(TEAM) void bn_short_once_forward_kernel(const G g, const OnceForward<double> a)
 {
     typedef double T;
-    constexpr int kPasses = short_once_passes<K, true>();
+    constexpr int kPasses = short_once_passes(K, true);
     __shared__ double sums[2][kPasses][TEAM];
     const uint32_t window = xcd_contiguous(blockIdx.x, gridDim.x);
     if (window * g.channels.divisor >= g.num_channels)
@@ -237,7 +236,7 @@ template <int VEC, int TEAM, int K, typename G>
 __global__ __launch_bounds__(TEAM) void bn_short_once_backward_kernel(const G g, const OnceBackward<double> a)
 {
     typedef double T;
-    constexpr int kPasses = short_once_passes<K, false>();
+    constexpr int kPasses = short_once_passes(K, false);
     __shared__ double sums[4][kPasses][TEAM];
     const uint32_t window = xcd_contiguous(blockIdx.x, gridDim.x);
     if (window * g.channels.divisor >= g.num_channels)

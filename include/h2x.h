@@ -554,7 +554,8 @@ int h2x_bn_audit_ordered(int num_samples,
 
 /**
  * The same for double tensors of segments of up to 256 elements, by workgroups of `threads` that hold `vectors`
- * each; `range`: one more than the range of samples whose sum an element is added to.
+ * each (others than the calls launch are an invalid argument); `range`: one more than the range of samples whose sum an element
+ * is added to.
  */
 int h2x_bn_audit_short(int num_samples,
                        const h2x_tensor_geometry* geometry,
@@ -755,6 +756,15 @@ int h2x_bn_audit_clearing(int backward,
                           const h2x_haloed_geometry* geometry,
                           const uint64_t* address,
                           h2x_bn_audit_report* report);
+
+/**
+ * Sets cleared[i] for every cell i of a double tensor (all of its allocation, `cells` of them) that h2x_bn_forward_clearing and
+ * _backward_clearing clear, played with `threads` threads a channel.
+ */
+int h2x_bn_audit_cleared(const h2x_haloed_geometry* geometry,
+                         unsigned int threads,
+                         unsigned char* cleared,
+                         size_t cells);
 
 /**
  * What h2x_bn_forward_once (`backward` 0) or h2x_bn_backward_once would launch for tensors of `geometry` that are apart and

@@ -21,7 +21,14 @@ CASES = [
     ((15, 17, 2, 64), (1, 15, 255 * 64, 255)),             # samples inside channels
     ((3, 3, 600, 8), (1, 3, 9, 5400)),
     ((255, 1, 1, 120), (1, 255, 255, 255)),
+    ((255, 1, 1, 50), (1, 255, 255, 255)),
 ]
+NOT_HELD = [[((255, 1, 1, 120), (1, 255, 255, 255))]] * 2  # by any workgroup, forward and backward
+
+
+# threads and vectors of the workgroups that there are, forward and backward
+LAUNCHED = [{(256, 4), (512, 4), (256, 8), (512, 8), (1024, 8), (512, 16)},
+            {(256, 4), (512, 4), (1024, 4), (256, 8), (512, 8), (1024, 8), (256, 16)}]
 
 
 def _play(shape, strides, backward, threads, vectors):
@@ -40,6 +47,9 @@ def test_every_element_counts_once_in_the_staged_order(shape, strides, backward)
     for threads in (256, 512, 1024):
         for vectors in (4, 8, 16):
             status, counted, stored, rng = _play(shape, strides, backward, threads, vectors)
+            if (threads, vectors) not in LAUNCHED[backward]:
+                assert status == -1
+                continue
             if status == -2:  # does not hold a channel
                 continue
             assert status == 0
@@ -55,8 +65,30 @@ def test_every_element_counts_once_in_the_staged_order(shape, strides, backward)
                 whole = np.broadcast_to(of_sample.reshape([-1] + [1] * (len(shape) - 1)), at.shape)
                 assert np.array_equal(rng[at], whole)
             assert np.array_equal(rng, ranges)
-    assert ranges is not None
+    assert (ranges is None) == ((shape, strides) in NOT_HELD[backward])
 
 
 def test_long_segments_are_not_for_these():
     assert _play((16, 17, 2, 4), (1, 16, 272, 544), 0, 1024, 16)[0] == -2
+
+
+@pytest.mark.parametrize("dims", [2, 3])
+def test_every_halo_cell_is_cleared_and_no_other(dims):
+    """Boxes with uneven and one-sided halos."""
+    rnd = np.random.RandomState(dims)
+    lib = capi.load()
+    for _ in range(400):
+        local, lower, upper = (rnd.randint(lo, hi, dims) for lo, hi in ((1, 8), (0, 4), (0, 4)))
+        n, c = rnd.randint(1, 4, 2)
+        g = capi.HaloedGeometry()
+        g.num_dims = dims + 2
+        for d in range(dims):
+            g.local_shape[d], g.real_shape[d], g.lower_halo[d] = local[d], local[d] + lower[d] + upper[d], lower[d]
+        for d, e in ((dims, c), (dims + 1, n)):
+            g.local_shape[d] = g.real_shape[d] = e
+        want = np.ones([n, c] + [l + lo + up for l, lo, up in zip(local, lower, upper)][::-1], np.uint8)
+        want[(Ellipsis,) + tuple(slice(lo, lo + l) for l, lo in zip(local, lower))[::-1]] = 0
+        cleared = np.zeros(want.size, np.uint8)
+        threads = int(rnd.choice([1, 7, 256, 1024]))
+        assert lib.h2x_bn_audit_cleared(ctypes.byref(g), threads, cleared.ctypes.data, cleared.size) == 0
+        assert np.array_equal(cleared, want.ravel()), (local, lower, upper, n, c)
