@@ -3297,7 +3297,7 @@ void ordered_issue(const G& g, const A& a, bool rows, bool stream, void* state, 
 {
     unsigned long long* const states = static_cast<unsigned long long*>(state);
     const uint32_t blocks = TEAMS ? g.num_channels * g.members.divisor : (g.num_channels + kNumXcd - 1) / kNumXcd * kNumXcd;
-    if constexpr (std::is_same<G, OrderedClearing>::value) // (rows, for the others are not haloed)
+    if constexpr (std::is_same<G, OrderedClearing>::value) // (rows: see ordered_launch)
         return issue_ordered<TEAM, K, TEAMS, true, false>(g, a, states, blocks, st);
     else if (!rows)
         issue_ordered<TEAM, K, TEAMS, false, true>(g, a, states, blocks, st);
@@ -3592,6 +3592,7 @@ bool ordered_launch(int n, int c, size_t s, std::initializer_list<const HostTens
     }
     OrderedClearing g;
     bool rows, team;
+    // (a halo on the outermost spatial dimension alone leaves dense segments, which the kernels that clear are not built for: staged)
     if (!ordered_geometry(n, c, s, ts, output, &g, &rows) || (halo && !rows))
         return false;
     const size_t bytes = (static_cast<size_t>(c - 1) * output.map.stride_c + static_cast<size_t>(n - 1) * output.map.stride_n

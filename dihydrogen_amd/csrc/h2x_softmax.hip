@@ -145,15 +145,15 @@ struct WideTiles
     unsigned int samples;
 };
 
-template <int VEC, int LANES = kWaveSize>
+// One pixel a lane.
 __device__ __forceinline__ bool tile_pixels(const WideTiles& t, int num_channels, size_t spatial, int flat_samples,
                                             size_t* base)
 {
     const unsigned int tile = xcd_contiguous(blockIdx.x, gridDim.x);
     const unsigned int n = fastdiv(tile, t.per_sample);
     const unsigned int sample = blockIdx.y + n;
-    const size_t first = static_cast<size_t>(tile - n * t.per_sample.divisor) * LANES;
-    return lane_pixels<VEC>(first + threadIdx.x % LANES, num_channels, spatial, flat_samples, base, sample)
+    const size_t first = static_cast<size_t>(tile - n * t.per_sample.divisor) * kWaveSize;
+    return lane_pixels<1>(first + threadIdx.x % kWaveSize, num_channels, spatial, flat_samples, base, sample)
            && sample < t.samples;
 }
 
@@ -316,7 +316,7 @@ __global__ __launch_bounds__(kBlockSize) void softmax_fwd_wide_kernel(
     const int lane = threadIdx.x % kWaveSize;
     const int g = wave_index();
     size_t base;
-    const bool active = tile_pixels<1>(tiles, num_channels, spatial, flat_samples, &base);
+    const bool active = tile_pixels(tiles, num_channels, spatial, flat_samples, &base);
     const T* xp = x + base;
     T* yp = y + base;
     constexpr T kMin = Limits<T>::min_normal;
@@ -445,7 +445,7 @@ __global__ __launch_bounds__(kBlockSize) void softmax_bwd_wide_kernel(
     const int lane = threadIdx.x % kWaveSize;
     const int g = wave_index();
     size_t base;
-    const bool active = tile_pixels<1>(tiles, num_channels, spatial, flat_samples, &base);
+    const bool active = tile_pixels(tiles, num_channels, spatial, flat_samples, &base);
     const T* yp = y + base;
     const T* gp = dy + base;
     T* op = dx + base;

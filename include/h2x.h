@@ -630,7 +630,8 @@ int h2x_bn_backprop2_clearing(h2x_dtype dtype,
  * A whole forward or backward pass of a rank that shares its statistics with no one,
  * the output's halo left cleared as by the two calls above: for tensors whose
  * channels one workgroup, or a team of them, holds in registers, of doubles with the bits of
- * those calls and where that is faster than they are.
+ * those calls, where that is faster than they are and, beyond segments of 256 elements, a spatial dimension other than the
+ * outermost has a halo.
  * H2X_ERR_UNSUPPORTED, with nothing launched, for others.  team_state as above;
  * h2x_bn_team_state_needed_clearing() is its size for these calls on floats, or 0, and
  * h2x_bn_ordered_state_needed() for those on doubles.
