@@ -175,6 +175,8 @@ __host__ __device__ __forceinline__ void box_offsets(const Box& box, uint32_t g,
 // its alignment.)
 struct DeviceMem
 {
+    // of cells that lie in so many strips
+    __device__ __forceinline__ const DeviceMem& of_strips(int) const { return *this; }
     template <int VEC, bool ALIGNED, typename T>
     __device__ __forceinline__ typename Words<T, VEC>::unaligned_t load(const T* p) const
     {
@@ -681,10 +683,17 @@ Audit* current_audit();
 struct TraceMem
 {
     Audit* audit;
+    int strips = 1; // a cell counts once for each strip that it is touched for
+    TraceMem of_strips(int n) const { return TraceMem{audit, n}; }
+    void touch(const void* p, size_t bytes, size_t alignment, bool is_store) const
+    {
+        for (int i = 0; i < strips; ++i)
+            audit->touch(p, bytes, alignment, is_store);
+    }
     template <int VEC, bool ALIGNED, typename T>
     typename Words<T, VEC>::unaligned_t load(const T* p) const
     {
-        audit->touch(p, sizeof(T) * VEC, ALIGNED ? sizeof(T) * VEC : sizeof(T), false);
+        touch(p, sizeof(T) * VEC, ALIGNED ? sizeof(T) * VEC : sizeof(T), false);
         typename Words<T, VEC>::unaligned_t v;
         for (int j = 0; j < VEC; ++j)
             v[j] = T(0);
@@ -698,12 +707,12 @@ struct TraceMem
     template <int VEC, bool ALIGNED, typename T>
     void store(T* p, typename Words<T, VEC>::unaligned_t) const
     {
-        audit->touch(p, sizeof(T) * VEC, ALIGNED ? sizeof(T) * VEC : sizeof(T), true);
+        touch(p, sizeof(T) * VEC, ALIGNED ? sizeof(T) * VEC : sizeof(T), true);
     }
     template <typename T>
     T load1(const T* p) const
     {
-        audit->touch(p, sizeof(T), sizeof(T), false);
+        touch(p, sizeof(T), sizeof(T), false);
         return T(0);
     }
     template <typename T>
@@ -714,7 +723,7 @@ struct TraceMem
     template <typename T>
     void store1(T* p, T) const
     {
-        audit->touch(p, sizeof(T), sizeof(T), true);
+        touch(p, sizeof(T), sizeof(T), true);
     }
 };
 

@@ -60,6 +60,12 @@ constexpr int kRanksPerTurn = 2;
 // (5 x 2 x 14 x 6 x 47 of doubles on 2 x 1 x 4, 660 rows: line by line 8.4 us, rank by rank 7.9; 9 x 8 x 287 x 109
 // on 4 x 2, 5,500 rows: 9.4 and 11.1).
 constexpr int64_t kLineRows = 4096;
+// Halo strips in bytes, of all ranks, up to which a reverse exchange of two or three dimensions is one launch.  It saves one launch or two,
+// of 1.5 to 2.5 us each; its regions, a few times as many as strips, keep more workgroups waiting for few cells, and beyond these sizes
+// it takes longer (three launches or two and one, us: 2 x 3 x 15 x 21 x 17 on 2^3 9.4 and 5.5; 1 x 11 x 46 x 67 x 50 on 2^3, 0.76 MB
+// 10.2 and 6.8; 9 x 11 x 28 x 34 x 28 on 2^3, periodic, 4.3 MB 17.0 and 14.2; 6 x 50 x 27^2 x 25 on 2^3, halos of 2, 18 MB 35.9 and 43; two dimensions: 1 x 32
+// x 57 x 57 on 2 x 2 6.4 and 5.3; 2 x 44 x 264 x 116 on 4 x 2, 0.70 MB 6.9 and 6.5; 2 x 15 x 15 x 30 x 79 on 2 x 4, 0.98 MB 8.6 and 10.8).
+constexpr uint64_t kFoldBytes2 = 640 << 10, kFoldBytes3 = 4608 << 10;
 
 // One end of a row of a rank, halo cell 0: where its values come from.
 struct RowEnd
@@ -84,7 +90,7 @@ struct Rank
     int32_t peer[kMaxSpatial][2]; // rank of the neighbour, or -1
     FastDiv units;                // by vectors (or elements) of an interior row
     FastDiv extent[2];            // by local[1], local[2]
-    uint32_t clear;               // bit 2 * d + side: this strip is cleared
+    uint32_t clear;               // bit 2 * d + side: this strip is cleared (reverse: there is no neighbour); see kRestEmpty
     uint32_t vectors;             // the interior row holds at least one vector
 };
 
@@ -106,6 +112,8 @@ struct Args
 // The rank that the cells of a region come from, four bits, and in which dimensions it is another one.
 constexpr uint32_t kSourceRank = 15, kStepped = 8; // bit 4 for dimension 1, bit 5 for dimension 2
 constexpr uint32_t kSteppedAny = 3 * 2 * kStepped;
+// Of Rank::clear, from here on: the strips of dimension d leave nothing of the rank's real extent.
+constexpr uint32_t kRestEmpty = 2 * kMaxSpatial;
 
 // Start of a region's cells in dimension d (1 or 2) of a rank of so many interior cells, and where
 // they start in the neighbour `src` they come from: the lower halo is its last interior
@@ -329,8 +337,8 @@ __host__ __device__ __forceinline__ FoldSide<T> fold_side(const FoldSeam& s, uin
 // a grid: 13 x 47 x 27 x 42 x 15 on 1 x 2 x 1, periodic, halo of 1 10.9 and 9.3; 2 x 12 x 116 x
 // 316 x 84 on 2 x 4 x 1, periodic 15.0 and 13.8; 4 x 85 x 27 x 38 x 14 on 2 x 2 x 1, halos of 3
 // 12.6 and 11.8; counting ranks without a seam too, whose XCDs then idle, 14.8).  Phases of
-// different dimensions stay launches of their own: a later one reads halo cells that
-// an earlier one has added to.
+// different dimensions are launches of their own: a later one reads halo cells that
+// an earlier one has added to (small ones go in one launch, fold_grid_body).
 template <typename T, typename Op, typename Mem>
 __host__ __device__ __forceinline__ void fold_body(const FoldArgs& a, uint32_t block, uint32_t thread, Op op,
                                                    const Mem& mem)
@@ -503,6 +511,213 @@ int issue_fold(int op, const FoldArgs& a, uint32_t blocks, Fold by, hipStream_t 
     case H2X_HALO_SUM: return issue_fold<T, copy::OpSum>(a, blocks, by, stream);
     case H2X_HALO_MAX: return issue_fold<T, copy::OpMax>(a, blocks, by, stream);
     default: return issue_fold<T, copy::OpMin>(a, blocks, by, stream);
+    }
+}
+
+// The reverse exchange of several dimensions in one launch.  Phase after phase, every cell of a boundary strip takes in the halo cell
+// of its neighbour along the phase's dimension, which has taken in others before.  Cells whose values meet are a group: per
+// dimension in which they lie at a seam, the boundary cell of one rank and the halo cell of its neighbour that stands for it.
+// A halo cell is of one group alone (a rank has at least two halo widths of interior along such a dimension), so groups have no order: a thread loads the two, four or
+// eight cells of one, plays the phases on them, with their roundings, and stores those that lie in a boundary strip.
+//
+// The groups of a rank are those whose cells in all boundary strips are its own: regions per {elsewhere, lower, upper
+// boundary} of the outer two dimensions, as vectors along what of the rows is no end ("elsewhere" of dimension 0), and the ends.
+template <typename F>
+__host__ __device__ __forceinline__ void fold_outer(uint32_t dims, F combine)
+{
+#pragma unroll
+    for (int i = 0; i < 4; i += 2)
+        if ((dims & 1) && (i & ~dims) == 0)
+            combine(i, i + 1);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        if ((dims & 2) && (i & ~dims) == 0)
+            combine(i, i + 2);
+}
+
+// Start of what a rank's seams along dimension d leave of its real extent.
+__host__ __device__ __forceinline__ uint32_t rest_start(const Rank& k, int d, int w)
+{
+    return k.clear >> (2 * d) & 1 ? 0 : 2 * w;
+}
+
+template <typename T, typename Op, typename Mem>
+__host__ __device__ __forceinline__ void fold_grid_body(const Args& a, uint32_t block, uint32_t thread, Op op, const Mem& mem)
+{
+    constexpr int VEC = 16 / sizeof(T);
+    using W = typename Words<T, VEC>::unaligned_t;
+    uint32_t first = 0, code = a.code[0];
+#pragma unroll
+    for (int i = 1; i < kMaxRegions; ++i)
+        if (block >= a.first[i])
+        {
+            first = a.first[i];
+            code = a.code[i];
+        }
+    const bool ends = code & 1;
+    const FastDiv& turns = ends ? a.lines : a.ranks;
+    const uint32_t local_block = fastdiv(block - first, turns);
+    const uint32_t r = (block - first - local_block * turns.divisor) * (ends ? a.line : 1);
+    const Rank& me = a.rank[r]; // ends: the first one of its line
+    const uint32_t digit_y = code >> 2 & 3, digit_z = code >> 4;
+    // bit 0: a seam along dimension 1, bit 1: along dimension 2; cell i of a group lies in the halo along those of its bits
+    const uint32_t dims = (digit_y != 0) | (digit_z != 0) << 1;
+    const uint32_t both = me.source[digit_z] >> (8 * digit_y);
+    const uint32_t empty = (ends ? 0 : 1) | (digit_y ? 0 : 2) | (digit_z ? 0 : 4);
+    if ((both & kSteppedAny) != dims * 2 * kStepped || (me.clear >> kRestEmpty & empty))
+        return;
+    const uint32_t ranks[4] = {r, me.source[0] >> (8 * digit_y) & kSourceRank, me.source[digit_z] & kSourceRank, both & kSourceRank};
+    const FastDiv div_y = digit_y == 0 ? me.extent[0] : a.halo[1], div_z = digit_z == 0 ? me.extent[1] : a.halo[2];
+    const FastDiv div_x = ends ? a.both_ends : me.units;
+    const uint32_t at = local_block * kBlock + thread;
+    if (at >= div_y.divisor * div_z.divisor * a.outer * div_x.divisor)
+        return;
+    const uint32_t row_at = fastdiv(at, div_x);
+    uint32_t x = at - row_at * div_x.divisor;
+    const uint32_t yz = fastdiv(row_at, div_y), o = fastdiv(yz, div_z);
+    const int wy = a.width[1], wz = a.width[2];
+    const uint32_t y = row_at - yz * div_y.divisor
+                       + (digit_y == 0 ? rest_start(me, 1, wy) : static_cast<uint32_t>(digit_y == 1 ? wy : me.local[1]));
+    const uint32_t z = yz - o * div_z.divisor
+                       + (digit_z == 0 ? rest_start(me, 2, wz) : static_cast<uint32_t>(digit_z == 1 ? wz : me.local[2]));
+    // the halo cell that stands for a lower boundary cell lies behind the lower neighbour's interior, ...
+    const uint32_t y_halo = y + (digit_y == 1 ? a.rank[ranks[1]].local[1] : -me.local[1]);
+    const uint32_t z_halo = z + (digit_z == 1 ? a.rank[ranks[2]].local[2] : -me.local[2]);
+    uint32_t row[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+    {
+        const Rank& q = a.rank[ranks[i]];
+        row[i] = (o * (q.local[2] + 2 * wz) + (i & 2 ? z_halo : z)) * (q.local[1] + 2 * wy) + (i & 1 ? y_halo : y);
+    }
+    const uint32_t w = a.width[0], pitch = me.local[0] + 2 * w; // (neighbours along dimensions 1 and 2 have rows as long)
+    const auto mine = [&](int i) { return (i & ~dims) == 0; };
+    // how many of the strips of a phase cell i lies in, as boundary and in all: what an audit counts
+    const auto boundary = [&](int i, int end) { return (dims & ~i & 1) + (dims >> 1 & ~i >> 1 & 1) + end; };
+    const int seams = boundary(0, ends);
+    if (!ends)
+    {
+        const uint32_t start = rest_start(me, 0, w);
+        uint32_t n = 1;
+        if (me.vectors)
+        {
+            const uint32_t count = (me.clear >> 1 & 1 ? pitch : me.local[0]) - start;
+            x *= VEC;
+            n = count - x < VEC ? count - x : VEC;
+        }
+        T* at_cell[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            at_cell[i] = reinterpret_cast<T*>(a.rank[ranks[i]].tensor) + (row[i] * pitch + start + x);
+        if (n == VEC)
+        {
+            W v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (mine(i))
+                    v[i] = mem.of_strips(seams).template load<VEC, false>(at_cell[i]);
+            fold_outer(dims, [&](int to, int from) {
+#pragma unroll
+                for (int j = 0; j < VEC; ++j)
+                    v[to][j] = op(v[to][j], v[from][j]);
+            });
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (mine(i) && boundary(i, 0))
+                    mem.of_strips(boundary(i, 0)).template store<VEC, false>(at_cell[i], v[i]);
+            return;
+        }
+        for (uint32_t j = 0; j < n; ++j)
+        {
+            T v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (mine(i))
+                    v[i] = mem.of_strips(seams).load1(at_cell[i] + j);
+            fold_outer(dims, [&](int to, int from) { v[to] = op(v[to], v[from]); });
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (mine(i) && boundary(i, 0))
+                    mem.of_strips(boundary(i, 0)).store1(at_cell[i] + j, v[i]);
+        }
+        return;
+    }
+    // the ends of a row in every rank of the line, side by side with the next row's
+    const bool upper = x >= w;
+    const uint32_t j = upper ? x - w : x;
+    const auto end_of = [&](int k, int i, T** inner_at, T** halo_at) {
+        const Rank& q = a.rank[ranks[i] + k];
+        const uint64_t lo_from = in_scalar(q.end[0].from), hi_from = in_scalar(q.end[1].from);
+        const uint32_t lo_pitch = in_scalar(q.end[0].pitch), hi_pitch = in_scalar(q.end[1].pitch);
+        *inner_at = reinterpret_cast<T*>(q.tensor) + (row[i] * (q.local[0] + 2 * w) + (upper ? q.local[0] : w) + j);
+        *halo_at = const_cast<T*>(global_place<T>(upper ? hi_from : lo_from)) + (row[i] * (upper ? hi_pitch : lo_pitch) + j);
+    };
+#pragma unroll 1
+    for (int k = 0; k < a.line; ++k)
+    {
+        if (a.rank[r + k].clear >> (upper ? 1 : 0) & 1)
+            continue;
+        T inner[4], halo[4];
+        T *inner_at[4], *halo_at[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (mine(i))
+            {
+                end_of(k, i, &inner_at[i], &halo_at[i]);
+                inner[i] = mem.of_strips(seams).load1(inner_at[i]);
+                halo[i] = mem.of_strips(seams).load1(halo_at[i]);
+            }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (mine(i))
+                inner[i] = op(inner[i], halo[i]);
+        fold_outer(dims, [&](int to, int from) {
+            inner[to] = op(inner[to], inner[from]);
+            halo[to] = op(halo[to], halo[from]);
+        });
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (mine(i))
+            {
+                mem.of_strips(boundary(i, 1)).store1(inner_at[i], inner[i]);
+                if (boundary(i, 0))
+                    mem.of_strips(boundary(i, 0)).store1(halo_at[i], halo[i]);
+            }
+    }
+}
+
+template <typename T, typename Op>
+__global__ __launch_bounds__(kBlock, 8) void halo_fold_grid_kernel(const Args a, Op op)
+{
+    fold_grid_body<T, Op, DeviceMem>(a, blockIdx.x, threadIdx.x, op, DeviceMem());
+}
+
+template <typename T, typename Op>
+int issue_fold_grid(const Args& a, uint32_t blocks, hipStream_t stream)
+{
+    if (Audit* const audit = current_audit())
+    {
+        const TraceMem mem{audit};
+        for (uint32_t block = 0; block < blocks; ++block)
+            for (uint32_t thread = 0; thread < kBlock; ++thread)
+                fold_grid_body<T, Op, TraceMem>(a, block, thread, Op(), mem);
+        ++audit->launches;
+        audit->workgroups += blocks;
+        return H2X_SUCCESS;
+    }
+    launch(halo_fold_grid_kernel<T, Op>, dim3(blocks), kBlock, stream, a, Op());
+    return launch_status();
+}
+
+template <typename T>
+int issue_fold_grid(int op, const Args& a, uint32_t blocks, hipStream_t stream)
+{
+    switch (op)
+    {
+    case H2X_HALO_ID: return issue_fold_grid<T, copy::OpId>(a, blocks, stream);
+    case H2X_HALO_SUM: return issue_fold_grid<T, copy::OpSum>(a, blocks, stream);
+    case H2X_HALO_MAX: return issue_fold_grid<T, copy::OpMax>(a, blocks, stream);
+    default: return issue_fold_grid<T, copy::OpMin>(a, blocks, stream);
     }
 }
 
@@ -773,6 +988,89 @@ int run(h2x_dtype dtype, const h2x_halo_grid* h, int only_unfilled, h2x_stream_t
                    : issue<uint64_t, CLEAR>(a, static_cast<uint32_t>(blocks), as_stream(stream));
 }
 
+// Whether a reverse exchange goes in one launch.
+bool folds_in_one_launch(const Args& a, int num_ranks, int es)
+{
+    int dims = 0;
+    uint64_t cells = 0;
+    for (int d = 0; d < kMaxSpatial; ++d)
+    {
+        uint64_t strips = 0;
+        for (int r = 0; r < num_ranks; ++r)
+        {
+            const Rank& k = a.rank[r];
+            uint64_t strip = static_cast<uint64_t>(a.outer) * a.width[d];
+            for (int e = 0; e < kMaxSpatial; ++e)
+                strip *= e == d ? 1 : k.local[e] + 2 * a.width[e];
+            strips += strip * ((k.peer[d][0] >= 0) + (k.peer[d][1] >= 0));
+        }
+        dims += strips != 0;
+        cells += strips;
+    }
+    return dims > 1 && cells * es <= (dims == 2 ? kFoldBytes2 : kFoldBytes3) && is_grid(a, num_ranks);
+}
+
+int run_fold_grid(Args& a, int num_ranks, int es, int op, hipStream_t stream)
+{
+    // (4 x 2 grids of 2D samples, 114 x 259: rank by rank 5.7 us, line by line 7.2; 160^3 on 2^3: 8.6 and 6.4)
+    const int64_t rows = static_cast<int64_t>(a.rank[0].local[1]) * a.rank[0].local[2] * a.outer;
+    if (rows < kLineRows || !order_into_lines(&a, num_ranks))
+    {
+        a.line = 1;
+        a.lines = a.ranks;
+    }
+    resolve_sources(&a, num_ranks, es);
+    const uint32_t vec = 16 / es;
+    uint32_t rest[kMaxRanks][kMaxSpatial];
+    for (int r = 0; r < num_ranks; ++r)
+    {
+        Rank& k = a.rank[r];
+        for (int d = 0; d < kMaxSpatial; ++d)
+        {
+            const int seams = (k.peer[d][0] >= 0) + (k.peer[d][1] >= 0);
+            rest[r][d] = static_cast<uint32_t>(k.local[d] + 2 * a.width[d] - 2 * seams * a.width[d]);
+            k.clear |= static_cast<uint32_t>(rest[r][d] == 0) << (kRestEmpty + d);
+        }
+        k.vectors = rest[r][0] >= vec;
+        k.units = make_fastdiv(std::max(k.vectors ? (rest[r][0] + vec - 1) / vec : rest[r][0], 1u));
+        for (int d = 1; d < kMaxSpatial; ++d)
+            k.extent[d - 1] = make_fastdiv(std::max(rest[r][d], 1u));
+        for (int side = 0; side < 2; ++side)
+            if (k.peer[0][side] >= 0)
+            {
+                const Rank& q = a.rank[k.peer[0][side]]; // its upper halo follows its interior, its lower one comes first
+                k.end[side].from = q.tensor + (side == 0 ? static_cast<int64_t>(a.width[0] + q.local[0]) * es : 0);
+            }
+    }
+    int num_regions = 0;
+    uint64_t blocks = 0;
+    std::fill(a.first, a.first + kMaxRegions, ~0u);
+    for (int ends = 1; ends >= 0; --ends)
+        for (int dz = 0; dz < 3; ++dz)
+            for (int dy = 0; dy < 3; ++dy)
+            {
+                uint64_t most = 0;
+                for (int r = 0; r < num_ranks; ++r)
+                {
+                    const Rank& k = a.rank[r];
+                    if ((!ends && !dy && !dz) || (dy && k.peer[1][dy - 1] < 0) || (dz && k.peer[2][dz - 1] < 0)
+                        || (ends && k.peer[0][0] < 0 && k.peer[0][1] < 0))
+                        continue;
+                    const uint64_t threads = static_cast<uint64_t>(dy ? a.width[1] : rest[r][1]) * (dz ? a.width[2] : rest[r][2])
+                                             * a.outer * (ends ? 2 * a.width[0] : rest[r][0] ? k.units.divisor : 0);
+                    most = std::max(most, (threads + kBlock - 1) / kBlock);
+                }
+                if (most == 0)
+                    continue;
+                const int g = num_regions++;
+                a.first[g] = static_cast<uint32_t>(blocks);
+                a.code[g] = static_cast<uint32_t>(ends + 4 * dy + 16 * dz);
+                blocks += most * (ends ? a.lines.divisor : a.ranks.divisor);
+            }
+    return es == 4 ? issue_fold_grid<float>(op, a, static_cast<uint32_t>(blocks), stream)
+                   : issue_fold_grid<double>(op, a, static_cast<uint32_t>(blocks), stream);
+}
+
 int run_fold(h2x_dtype dtype, const h2x_halo_grid* h, int op, h2x_stream_t stream)
 {
     const int es = dtype == H2X_F32 ? 4 : dtype == H2X_F64 ? 8 : 0;
@@ -781,9 +1079,11 @@ int run_fold(h2x_dtype dtype, const h2x_halo_grid* h, int op, h2x_stream_t strea
     if (!h || op < H2X_HALO_ID || op > H2X_HALO_MIN)
         return H2X_ERR_INVALID_ARGUMENT;
     Args a;
-    int err = make_args(*h, 2, 0, es, &a);
+    int err = make_args(*h, 2, 1, es, &a);
     if (err != 0)
         return err;
+    if (folds_in_one_launch(a, h->num_ranks, es))
+        return run_fold_grid(a, h->num_ranks, es, op, as_stream(stream));
     const int64_t rows = static_cast<int64_t>(a.rank[0].local[1] + 2 * a.width[1])
                          * (a.rank[0].local[2] + 2 * a.width[2]) * a.outer;
     bool lines = rows >= kLineRows && a.width[0] > 0 && order_into_lines(&a, h->num_ranks);

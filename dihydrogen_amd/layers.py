@@ -612,7 +612,7 @@ class HaloExchangeVirtual:
     side for the opposite side, so the transfer is free.  A packed exchange is
     two launches a dimension (pack all ranks and sides, unpack all ranks and
     sides).  A full-width exchange of tensors that share a GPU goes straight
-    from tensor to tensor, in one launch (reverse: one a dimension), unless
+    from tensor to tensor, in one launch (large reverse ones: one a dimension), unless
     a receive buffer was asked for, ``launch_hook`` is set or ``_grid`` names
     another reason.  ``periodic`` wraps neighbours at the grid edge; the reference
     never does (MPI_PROC_NULL, halo_exchange_cuda.hpp:343-345).

@@ -1178,7 +1178,7 @@ typedef struct h2x_halo_grid
 int h2x_halo_grid_exchange(h2x_dtype dtype, const h2x_halo_grid* grid, h2x_stream_t stream);
 
 /**
- * The reverse exchange of full-width halos of all ranks, one launch a dimension:
+ * The reverse exchange of full-width halos of all ranks, one launch a dimension (small ones in one):
  * halo strips are combined with `op` (h2x_halo_op) into the boundary cells they
  * belong to, innermost dimension first, as packing and unpacking them does.  A rank
  * with a neighbour needs at least twice the halo's width of interior cells along
