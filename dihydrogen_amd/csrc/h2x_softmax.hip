@@ -709,6 +709,105 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
         }
 }
 
+// Up to 32 channels of few pixels: a workgroup of 256 threads serves LANES pixels, thread group g their channels g, g + 256 / LANES, ...
+// A lane's chain of loads, exponentials and stores is that many times shorter, and there are as many more workgroups.  The exponentials
+// (backward the values) go through LDS, where each thread adds those of its pixel in channel order: the same bits as by one thread a pixel.
+template <typename T, int CMAX, int LANES>
+__global__ __launch_bounds__(kBlockSize) void softmax_fwd_shared_kernel(
+    const T* __restrict__ x, T* __restrict__ y, int num_channels, size_t spatial, int flat_samples, const WideTiles tiles)
+{
+    constexpr int kGroups = kBlockSize / LANES, kEach = (CMAX + kGroups - 1) / kGroups;
+    __shared__ T largest[kGroups][LANES];
+    __shared__ T terms[CMAX][LANES];
+    const int lane = threadIdx.x % LANES, g = threadIdx.x / LANES;
+    const TilePlace place = tile_place<T, 1, LANES>(tiles, num_channels, spatial, flat_samples);
+    if (!place.any) // the whole workgroup
+        return;
+    constexpr T kMin = Limits<T>::min_normal;
+    const auto exists = [&](int k) { return g + k * kGroups < num_channels; };
+    const T* const xp = element(x + place.first, place.offset) + g * spatial;
+    T v[kEach], mx = kMin;
+#pragma unroll
+    for (int k = 0; k < kEach; ++k)
+        if (exists(k))
+            v[k] = xp[k * kGroups * spatial];
+#pragma unroll
+    for (int k = 0; k < kEach; ++k)
+        if (exists(k))
+            mx = v[k] > mx ? v[k] : mx;
+    largest[g][lane] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kGroups; ++i)
+        mx = largest[i][lane] > mx ? largest[i][lane] : mx;
+#pragma unroll
+    for (int k = 0; k < kEach; ++k)
+        if (exists(k))
+            terms[g + k * kGroups][lane] = v[k] = exp_t(v[k] - mx);
+    __syncthreads();
+    T sum = T(0);
+#pragma unroll
+    for (int c = 0; c < CMAX; ++c)
+        if (c < num_channels)
+            sum += terms[c][lane];
+    sum = T(1) / sum;
+    if (!place.active)
+        return;
+    T* const yp = element(y + place.first, place.offset) + g * spatial;
+#pragma unroll
+    for (int k = 0; k < kEach; ++k)
+        if (exists(k))
+        {
+            const T r = v[k] * sum;
+            yp[k * kGroups * spatial] = r > kMin ? r : kMin;
+        }
+}
+
+template <typename T, int CMAX, int LANES>
+__global__ __launch_bounds__(kBlockSize) void softmax_bwd_shared_kernel(
+    const T* __restrict__ y, const T* __restrict__ dy, T* __restrict__ dx, int num_channels, size_t spatial, int flat_samples,
+    const WideTiles tiles)
+{
+    constexpr int kGroups = kBlockSize / LANES, kEach = (CMAX + kGroups - 1) / kGroups;
+    __shared__ T terms[2][CMAX][LANES];
+    const int lane = threadIdx.x % LANES, g = threadIdx.x / LANES;
+    const TilePlace place = tile_place<T, 1, LANES>(tiles, num_channels, spatial, flat_samples);
+    if (!place.any) // the whole workgroup
+        return;
+    constexpr T kMin = Limits<T>::min_normal;
+    const auto exists = [&](int k) { return g + k * kGroups < num_channels; };
+    const T* const yp = element(y + place.first, place.offset) + g * spatial;
+    const T* const gp = element(dy + place.first, place.offset) + g * spatial;
+    T yv[kEach], gv[kEach];
+#pragma unroll
+    for (int k = 0; k < kEach; ++k)
+        if (exists(k))
+        {
+            yv[k] = yp[k * kGroups * spatial];
+            gv[k] = gp[k * kGroups * spatial];
+        }
+#pragma unroll
+    for (int k = 0; k < kEach; ++k)
+        if (exists(k))
+        {
+            terms[0][g + k * kGroups][lane] = yv[k];
+            terms[1][g + k * kGroups][lane] = gv[k];
+        }
+    __syncthreads();
+    T dp = T(0);
+#pragma unroll
+    for (int c = 0; c < CMAX; ++c)
+        if (c < num_channels)
+            dp = fma_t(terms[0][c][lane], terms[1][c][lane], dp);
+    if (!place.active)
+        return;
+    T* const op = element(dx + place.first, place.offset) + g * spatial;
+#pragma unroll
+    for (int k = 0; k < kEach; ++k)
+        if (exists(k))
+            op[k * kGroups * spatial] = yv[k] > kMin ? yv[k] * (gv[k] - dp) : T(0);
+}
+
 // One pixel per sample (the output of a fully connected layer): the channels of
 // a sample are contiguous, so a wave takes a sample, lane l the channels l,
 // l + 64, ... (CPL of them at most), and maxima, sums and dot products are
@@ -1157,6 +1256,49 @@ int launch_split_for(int v, int n, int c, size_t s, hipStream_t st, P... p)
     return kNoSplit;
 }
 
+template <int CMAX, int LANES, typename T>
+int launch_shared(const T* x, T* y, int n, int c, size_t s, hipStream_t st)
+{
+    WideTiles tiles;
+    const int flat = flat_samples(n, s);
+    const dim3 grid = wide_grid(s, LANES, 1, n, flat, &tiles);
+    launch(softmax_fwd_shared_kernel<T, CMAX, LANES>, grid, kBlockSize, st, x, y, c, s, flat, tiles);
+    return launch_status();
+}
+
+template <int CMAX, int LANES, typename T>
+int launch_shared(const T* y, const T* dy, T* dx, int n, int c, size_t s, hipStream_t st)
+{
+    WideTiles tiles;
+    const int flat = flat_samples(n, s);
+    const dim3 grid = wide_grid(s, LANES, 1, n, flat, &tiles);
+    launch(softmax_bwd_shared_kernel<T, CMAX, LANES>, grid, kBlockSize, st, y, dy, dx, c, s, flat, tiles);
+    return launch_status();
+}
+
+// Up to 32 channels: the threads of a workgroup share them, or kNoSplit.  Where one thread a pixel leaves CUs waiting for its chain; with more
+// pixels the sums that every thread forms cost more than the chain.  Us in a graph, a thread a pixel and so (32 pixels forward, 16 backward; 64
+// pixels are slower throughout, and at 2^17 pixels all of them are):
+//   floats, C 32, 4608 pixels 4.9 / 4.1 and 3.6 / 3.3, 2^14 5.1 / 4.3 and 4.0 / 3.9, 2^15 5.3 / 4.5 and 4.4 / 4.8, 2^16 6.0 / 6.4 and 6.0 / 8.6;
+//   C 12, 2^14 3.1 / 2.7 and 2.9 / 2.7; C 8, 2^15 2.8 / 2.4 and 2.8 / 2.8;
+//   doubles, whose exponentials are longer, C 32, 4608 pixels 8.6 / 5.2 and 4.1 / 3.8, 2^16 12.3 / 10.0 and 9.8 / 12.3, 3 x 2^16 23.3 and 24.1
+//   forward; C 12, 2^14 4.6 / 3.2 and 3.4 / 2.9, 2^16 5.2 and 5.1 forward; C 6, 2^15 3.3 / 2.6 and 3.0 / 3.0.
+template <typename T, typename... P>
+int launch_shared_for(int n, int c, size_t s, hipStream_t st, P... p)
+{
+    constexpr bool kForward = sizeof...(P) == 2, kFloat = sizeof(T) == 4;
+    const size_t pixels = s * n, cus = chip_units();
+    if (c > 32 || pixels > cus * (!kForward ? 64 : kFloat ? 128 : 256) || c <= (kForward && !kFloat ? 4 : 8))
+        return kNoSplit;
+    constexpr int kLanes = kForward ? 32 : 16;
+    if constexpr (kForward && !kFloat)
+    {
+        if (c <= 8) return launch_shared<8, kLanes>(p..., n, c, s, st);
+    }
+    if (c <= 16) return launch_shared<16, kLanes>(p..., n, c, s, st);
+    return launch_shared<32, kLanes>(p..., n, c, s, st);
+}
+
 // Calls f(elements a lane, lanes) with constants for samples of `size` contiguous elements that
 // lanes hold in registers: a wave while samples are short, or many (it needs no barrier), else
 // a workgroup, of 1024 threads with up to MAX_LARGE elements each where 256 would have more than 16.
@@ -1205,8 +1347,7 @@ unsigned int lanes_grid(int n)
 // us, 4, 2 and 1 a lane, going round three sets of tensors: N 1, C 16, 128 x 128 11.5, 7.9, 6.9; N 2, C 12,
 // 256 x 256 12.9, 10.3, 9.3; N 4, C 16, 256 x 256 21.2, 17.7, 17.7; N 8, C 16, 256 x 256 32.8, 29.7, 33.1; N 16, C 16,
 // 256 x 256 52.8 and 55.0; N 32, C 16, 256 x 256 108 and 104; N 1, C 32, 256 x 256, by 2 and 1, 15.7 and 12.4.
-// (Shared by the waves of a workgroup, as more channels are, C 32 of 128 x 128 pixels take 6.8 us instead of 8.9, but
-// their sums would not be added in channel order.)
+// (Still fewer pixels go to launch_shared_for.)
 int pixels_a_lane(int widest, size_t pixels, size_t bytes)
 {
     constexpr size_t kOnePixel = size_t(1) << 18, kTwoPixels = size_t(1) << 20, kFromMemory = size_t(68) << 20;
@@ -1233,6 +1374,8 @@ int forward_impl(int n, int c, size_t s, const void* xv, void* yv, hipStream_t s
     const int widest = s < kFlatBelow ? 1 : vector_width<T>(s, 4 / kWords, {xv, yv});
     const bool stream = streamed<T>(widest, n, c, s);
     const int v4 = pixels_a_lane(widest, n * s, n * s * c * sizeof(T));
+    if (const int shared = launch_shared_for<T>(n, c, s, st, x, y); shared != kNoSplit)
+        return shared;
 #define H2X_FWD(V, CM)                                                                             \
     do                                                                                             \
     {                                                                                              \
@@ -1305,6 +1448,8 @@ int backward_impl(int n, int c, size_t s, const void* yv, const void* dyv, void*
     const int widest = s < kFlatBelow ? 1 : vector_width<T>(s, 4 / kWords, {yv, dyv, dxv});
     const bool stream = streamed<T>(widest, n, c, s);
     const int v4 = pixels_a_lane(widest, n * s, n * s * c * sizeof(T));
+    if (const int shared = launch_shared_for<T>(n, c, s, st, y, dy, dx); shared != kNoSplit)
+        return shared;
 #define H2X_BWD(V, CM)                                                                             \
     do                                                                                             \
     {                                                                                              \
