@@ -76,6 +76,30 @@ __host__ __device__ __forceinline__ uint32_t short_once_sample(const ShortOnceGe
     return of_range < g.per && range < g.ranges ? range * g.per + of_range : ~0u;
 }
 
+// Terms 0 to n - 1, one after the other; n is uniform and at least 1.  An addition that waits for the read before it takes 100 clocks: they
+// are read ahead of the additions, eight at a time.  (The sums of a range and those of the ranges by a thread each, reads ahead, against one
+// thread a channel, read by read, forward + backward in us: N 254, C 149, 3 x 3 16.5 -> 13.1, N 243, C 1065, 1 x 1 13.2 -> 10.7; N 18, C 776, 15 x 15
+// 43.5 -> 35.8; N 148, C 334, 5 x 5 23.7 -> 22.5; 55 drawn calls 0.97.  In finish_short, whose workgroups have two to eight rows, the reads beyond the
+// last row cost more than they save: N 67, C 55, 9 x 11 21.1 and 22.4.)
+template <typename F>
+__device__ __forceinline__ double sum_in_order(uint32_t n, const F& term)
+{
+    constexpr uint32_t kBatch = 8;
+    double t = term(0);
+    for (uint32_t i = 1; i < n; i += kBatch)
+    {
+        double w[kBatch];
+#pragma unroll
+        for (uint32_t j = 0; j < kBatch; ++j)
+            w[j] = term(i + j < n ? i + j : n - 1);
+#pragma unroll
+        for (uint32_t j = 0; j < kBatch; ++j)
+            if (i + j < n)
+                t += w[j];
+    }
+    return t;
+}
+
 // The N sums of a lane's channel from what the lanes have left in sums[k][pass][thread], in the order of finish_short and
 // sequential_totals.
 template <int TEAM, int PASSES, int N>
@@ -122,20 +146,33 @@ __device__ __forceinline__ void short_once_totals(const ShortOnceGeometry& g, co
         }
         __syncthreads();
     }
-    for (uint32_t i = threadIdx.x; i < channels * N; i += TEAM)
-    {
-        const uint32_t k = i / channels, c = i - k * channels;
-        double total = 0.0;
-        for (uint32_t range = 0; range < g.ranges; ++range)
+    // the rows of each range, then the ranges, each of them by a thread
+    const auto top = [&](uint32_t k, uint32_t range, uint32_t c) {
+        uint32_t p = 0;
+#pragma unroll
+        for (int i = 1; i < PASSES; ++i)
+            p += range >= i * g.together;
+        return &sums[k][p][((range - p * g.together) * rows * channels + c) * slots];
+    };
+    if (rows > 1) // uniform
+        for (uint32_t i = threadIdx.x; i < channels * N * g.ranges; i += TEAM)
         {
-            const uint32_t p = range / g.together, q = range - p * g.together;
-            const double* const tops = &sums[k][p][(q * rows * channels + c) * slots];
-            double t = tops[0];
-            for (uint32_t r = 1; r < rows; ++r)
-                t += tops[r * channels * slots];
-            total = range == 0 ? t : total + t;
+            const uint32_t of_sum = fastdiv(i, g.channels);
+            uint32_t k = 0;
+#pragma unroll
+            for (int n = 1; n < N; ++n)
+                k += of_sum >= n * g.ranges;
+            double* const first = top(k, of_sum - k * g.ranges, i - of_sum * channels);
+            *first = sum_in_order(rows, [&](uint32_t r) { return first[r * channels * slots]; }); // read by this thread alone
         }
-        sums[k][0][c * slots] = total; // read by this thread alone, above
+    if (g.ranges > 1)
+    {
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < channels * N; i += TEAM)
+        {
+            const uint32_t k = fastdiv(i, g.channels), c = i - k * channels;
+            sums[k][0][c * slots] = sum_in_order(g.ranges, [&](uint32_t range) { return *top(k, range, c); });
+        }
     }
     __syncthreads();
 #pragma unroll
