@@ -102,8 +102,8 @@ __device__ __forceinline__ double sum_in_order(uint32_t n, const F& term)
 
 // The N sums of a lane's channel from what the lanes have left in sums[k][pass][thread], in the order of finish_short and
 // sequential_totals.
-template <int TEAM, int PASSES, int N>
-__device__ __forceinline__ void short_once_totals(const ShortOnceGeometry& g, const ShortOnceLane& l, double (&v)[N],
+template <int TEAM, int PASSES, int N, typename G>
+__device__ __forceinline__ void short_once_totals(const G& g, const ShortOnceLane& l, double (&v)[N],
                                                   double (&sums)[N][PASSES][TEAM])
 {
     const uint32_t slots = g.slots.divisor, channels = g.channels.divisor, rows = g.rows.divisor;
@@ -115,7 +115,42 @@ __device__ __forceinline__ void short_once_totals(const ShortOnceGeometry& g, co
         const uint32_t width = 2u << (31 - __builtin_clz(slots - 1)), lanes = width < kWaveSize ? width : kWaveSize;
         const uint32_t at_once = kWaveSize / lanes, slot = lane & (lanes - 1);
         const uint32_t runs = g.together * rows * channels, trees = runs * g.passes * N;
-        for (uint32_t first = wave * at_once; first < trees; first += TEAM / kWaveSize * at_once) // uniform
+        uint32_t first = wave * at_once; // uniform
+        // Backward, which has twice the trees: two of them at once wait for their exchanges together (forward + backward in us, one by one and so: N 18,
+        // C 386, 8 x 9 15.5 and 14.9; N 15, C 136, 7 x 10 with a halo 11.8 and 11.2; N 42, C 271, 4 x 6 12.4 and 11.9; forward, four at
+        // once, or trees wider than a wave 2 to 10 % longer; where a large output's halo is cleared, and what waits longer spreads the stores, N 158, C
+        // 610, 7 x 4 68.5 and 70.4).
+        if constexpr (N == 4 && !std::is_same<G, ShortOnceClearing>::value)
+            if (width <= kWaveSize)
+                for (constexpr uint32_t kStep = TEAM / kWaveSize; first + kStep * at_once < trees; first += 2 * kStep * at_once)
+                {
+                    double* leaves[2];
+                    double t[2];
+                    bool mine[2];
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                    {
+                        const uint32_t tree = first + i * kStep * at_once + lane / lanes;
+                        const uint32_t kind = tree / runs, run = tree - kind * runs;
+                        leaves[i] = &sums[0][0][0] + (kind % N * PASSES + kind / N) * TEAM + run * slots;
+                        mine[i] = tree < trees;
+                        t[i] = mine[i] && slot < slots ? leaves[i][slot] : 0.0;
+                    }
+                    for (uint32_t step = lanes / 2; step >= 1; step /= 2)
+                    {
+                        const double o[2] = {__shfl_down(t[0], step), __shfl_down(t[1], step)};
+                        if (slot < step && slot + step < slots)
+                        {
+                            t[0] += o[0];
+                            t[1] += o[1];
+                        }
+                    }
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                        if (mine[i] && slot == 0)
+                            leaves[i][0] = t[i]; // read by this wave alone, above
+                }
+        for (; first < trees; first += TEAM / kWaveSize * at_once)
         {
             const uint32_t tree = first + lane / lanes;
             const uint32_t kind = tree / runs, run = tree - kind * runs;
