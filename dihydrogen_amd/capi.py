@@ -343,12 +343,12 @@ def calls():
     global _calls
     if _calls is None:
         load()
+        import torch  # before the module, which is linked with its libraries
         try:
             from . import _h2xcall
         except ImportError as e:
             raise H2XError("_h2xcall.so is missing: build it with `make -C dihydrogen_amd/csrc` "
                            "(or __graft_entry__.build()); there is no fallback path") from e
-        import torch
         from .tensor import BASE_PTR_PARTS, Tensor
         _h2xcall.pointer_types(torch.Tensor, Tensor, *BASE_PTR_PARTS)
         _calls = _h2xcall

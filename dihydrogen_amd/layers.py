@@ -115,10 +115,15 @@ class _Struct:
         return ctypes.addressof(self._value)
 
 
-def _share_a_haloed_geometry(*layouts: Layout) -> bool:
+def _share_a_haloed_geometry(l0: Layout, *layouts: Layout) -> bool:
     """Tensors with a halo on a spatial dimension whose local parts lie in memory alike."""
-    l0 = layouts[0]
-    return l0.haloed and not l0.channel_halo and all(l.alike == l0.alike for l in layouts)
+    if not l0.haloed or l0.channel_halo:
+        return False
+    alike = l0.alike
+    for l in layouts:
+        if l.alike != alike:
+            return False
+    return True
 
 
 def _pair_in_order(l0: Layout, *layouts: Layout) -> bool:
@@ -176,21 +181,32 @@ class BatchNormalization:
         return ws
 
     def _team_state(self, l: Layout, clearing: bool, st: int) -> Optional[torch.Tensor]:
-        """Where the workgroups that share a channel exchange its sums; None where no workgroups
-        do.  Smaller channels than 16 K floats or 4 K doubles need none."""
-        double = l.dtype == capi.F64
-        if l.samples * l.spatial_real <= (4096 if double else 16384):
+        """Where the workgroups that share a channel exchange its sums; None where no workgroups do."""
+        if l.small_channels:
             return None
         kept = self._kept.get(st) or _first_use(self._kept, st)
         channels, state = kept.state
         if channels < l.channels:
-            nbytes = (l.ordered_state_bytes if double else
+            nbytes = (l.ordered_state_bytes if l.dtype == capi.F64 else
                       l.clearing_team_state_bytes if clearing else l.team_state_bytes)
             if nbytes == 0:
                 return None
             state = _buffer_of(self.stream, nbytes, torch.uint8, zero=True)
             kept.state = l.channels, state
         return state
+
+    def _buffers(self, l: Layout, st: int):
+        """The workspace and the state of a call, from one look at what is kept for its stream: a small call spends as long on
+        looking things up as on anything but the launch."""
+        kept = self._kept.get(st) or _first_use(self._kept, st)
+        num_channels = l.channels
+        channels, ws = kept.workspace
+        if channels != num_channels:
+            ws = self._ws(num_channels, st)
+        if l.small_channels:
+            return ws, None
+        channels, state = kept.state
+        return ws, state if channels >= num_channels else self._team_state(l, False, st)
 
     @property
     def _state(self) -> Optional[torch.Tensor]:
@@ -266,22 +282,19 @@ class BatchNormalization:
             self.batch_normalization(input, running_mean, running_var, scale, bias, output)  # :243-247
         return 0
 
-    def _runs_local(self, l0: Layout) -> bool:
-        """No all-reduce between the stages, a rank that owns elements."""
-        return self.fuse_local and l0.active and (self.allreduce is None or not self.global_stats)
-
     def _elements_per_sum(self, l: Layout) -> int:
         return l.per_channel_global if self.global_stats else l.per_channel_local
 
     def forward(self, input, mean, var, running_mean, running_var, scale, bias, output,
                 is_training: bool = True) -> int:
         lx, ly = input.layout, output.layout
+        # (local: no all-reduce between the stages, a rank that owns elements)
         if not is_training:
             # the stages would do nothing but this: no sums, no all-reduce
             self.num_current_samples = lx.samples
             self.batch_normalization(input, running_mean, running_var, scale, bias, output)
             return 0
-        local = self._runs_local(lx)
+        local = self.fuse_local and lx.active and (self.allreduce is None or not self.global_stats)
         if local and self.clear_output_halo and (lx.haloed or ly.haloed):
             local = False  # the stages, unless a whole pass clears the halo
             if _share_a_haloed_geometry(lx, ly):
@@ -295,19 +308,21 @@ class BatchNormalization:
                     capi.check(status, "bn forward (clearing)")
                     return 0
         if local:
-            _dense_layout(input), _dense_layout(output)
+            if lx.channel_halo or ly.channel_halo:
+                _dense_layout(input), _dense_layout(output)  # raises
             ns = self.num_current_samples = lx.samples
-            per_sum, st = self._elements_per_sum(lx), _stream_handle(self.stream)
+            per_sum, st = lx.per_channel_global if self.global_stats else lx.per_channel_local, _stream_handle(self.stream)
             if lx.extents != ly.extents and _pair_in_order(lx, ly):
                 capi.check(self._calls.h2x_bn_forward_local(
                     lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ly.spatial_real, input,
                     scale, bias, per_sum, self.decay, self.epsilon, mean, var, running_mean, running_var,
                     output, self._ws(lx.channels, st), st), "bn forward (local)")
                 return 0
+            ws, state = self._buffers(lx, st)
             status = self._calls.h2x_bn_forward_once(
-                lx.dtype, ns, lx.geometry_address, _tensor_geometry(ly, ns), input, scale, bias, per_sum,
-                self.decay, self.epsilon, mean, var, running_mean, running_var, output,
-                self._ws(lx.channels, st), self._team_state(lx, False, st), st)
+                lx.dtype, ns, lx.geometry_address, ly.geometry_address if ly.samples == ns else _tensor_geometry(ly, ns),
+                input, scale, bias, per_sum, self.decay, self.epsilon, mean, var, running_mean, running_var, output,
+                ws, state, st)
             if status:
                 capi.check(status, "bn forward (local)")
             return 0
@@ -369,7 +384,7 @@ class BatchNormalization:
     def backward(self, input, d_output, mean, var, scale, scale_gradient, bias_gradient,
                  mean_gradient, var_gradient, d_input) -> int:
         lx, ld, li = input.layout, d_output.layout, d_input.layout
-        local = self._runs_local(lx)
+        local = self.fuse_local and lx.active and (self.allreduce is None or not self.global_stats)
         if local and self.clear_output_halo and (lx.haloed or ld.haloed or li.haloed):
             local = False
             if _share_a_haloed_geometry(lx, ld, li):
@@ -383,9 +398,10 @@ class BatchNormalization:
                     capi.check(status, "bn backward (clearing)")
                     return 0
         if local:
-            _dense_layout(input), _dense_layout(d_output), _dense_layout(d_input)
+            if lx.channel_halo or ld.channel_halo or li.channel_halo:
+                _dense_layout(input), _dense_layout(d_output), _dense_layout(d_input)  # raises
             ns = self.num_current_samples = lx.samples
-            per_sum, st = self._elements_per_sum(lx), _stream_handle(self.stream)
+            per_sum, st = lx.per_channel_global if self.global_stats else lx.per_channel_local, _stream_handle(self.stream)
             if (lx.extents != ld.extents or lx.extents != li.extents) and _pair_in_order(lx, ld, li):
                 capi.check(self._calls.h2x_bn_backward_local(
                     lx.dtype, ns, lx.channels, lx.spatial, lx.spatial_real, ld.spatial_real, li.spatial_real, per_sum,
@@ -393,11 +409,12 @@ class BatchNormalization:
                     mean_gradient, var_gradient, d_input, self.epsilon, self._ws(lx.channels, st), st),
                     "bn backward (local)")
                 return 0
+            ws, state = self._buffers(lx, st)
             status = self._calls.h2x_bn_backward_once(
-                lx.dtype, ns, per_sum, lx.geometry_address, _tensor_geometry(ld, ns), _tensor_geometry(li, ns),
+                lx.dtype, ns, per_sum, lx.geometry_address, ld.geometry_address if ld.samples == ns else _tensor_geometry(ld, ns),
+                li.geometry_address if li.samples == ns else _tensor_geometry(li, ns),
                 input, d_output, mean, var, scale, scale_gradient, bias_gradient,
-                mean_gradient, var_gradient, d_input, self.epsilon, self._ws(lx.channels, st),
-                self._team_state(lx, False, st), st)
+                mean_gradient, var_gradient, d_input, self.epsilon, ws, state, st)
             if status:
                 capi.check(status, "bn backward (local)")
             return 0

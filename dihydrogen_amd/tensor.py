@@ -162,6 +162,8 @@ class Layout:
         # elements per channel of the local and of the global shape
         self.per_channel_local = spatial * samples if channels else 0
         self.per_channel_global = math.prod(shape) // shape[ns] if shape[ns] else 0
+        # channels that no workgroups share: up to 16 K floats or 4 K doubles
+        self.small_channels = samples * spatial_real <= (4096 if self.dtype == capi.F64 else 16384)
 
     @_once
     def alike(self):

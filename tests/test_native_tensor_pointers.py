@@ -1,0 +1,61 @@
+"""The address that a native call takes of a torch tensor: what its data_ptr() returns, or raises.  Shown on the host, by a call that
+reads a geometry out of the tensor's memory."""
+import ctypes
+
+import pytest
+import torch
+
+from dihydrogen_amd import capi
+
+ITEM = ctypes.sizeof(capi.TensorGeometry)
+
+
+class Shifted(torch.Tensor):
+    """One item further on."""
+
+    def data_ptr(self):
+        return super().data_ptr() + ITEM
+
+
+def _geometries():
+    """The bytes of a geometry that teams have a state for, and of one with twice the channels; the states."""
+    raw, needed = bytearray(), []
+    for c in (64, 128):
+        g = capi.TensorGeometry()
+        g.num_dims = 4
+        g.local_shape[:4] = 64, 64, c, 16
+        g.strides[:4] = 1, 64, 4096, 4096 * c
+        raw += bytes(g)
+        needed.append(capi.calls().h2x_bn_team_state_needed(capi.F32, 16, ctypes.addressof(g)))
+    assert len(raw) == 2 * ITEM and 0 < needed[0] < needed[1]
+    return torch.frombuffer(raw, dtype=torch.uint8), needed
+
+
+def _needed(pointer):
+    return capi.calls().h2x_bn_team_state_needed(capi.F32, 16, pointer)
+
+
+def test_tensors_views_and_parameters():
+    t, (first, second) = _geometries()
+    assert _needed(t) == _needed(t.data_ptr()) == first
+    assert _needed(t[ITEM:]) == second
+    assert _needed(torch.nn.Parameter(t[ITEM:], requires_grad=False)) == second
+
+
+def test_a_class_with_a_data_ptr_of_its_own_is_asked():
+    t, (first, second) = _geometries()
+    assert _needed(t.as_subclass(Shifted)) == second
+
+
+def test_a_tensor_without_memory_raises_what_data_ptr_raises():
+    messages = []
+
+    def asked(x):
+        for ask in (lambda: x.data_ptr(), lambda: _needed(x)):
+            with pytest.raises(RuntimeError) as e:
+                ask()
+            messages.append(str(e.value))
+        return x
+
+    torch.func.vmap(asked)(torch.zeros(2, 3))
+    assert messages[0] == messages[1]
