@@ -1836,6 +1836,31 @@ constexpr int kInstLargeLanes = 128 / sizeof(T);
 template <typename T>
 constexpr size_t kInstSmallSample = kInstLargeLanes<T> * size_t(1024);
 
+// Elements of a chunk of samples that a workgroup holds (inst_chunking cuts them so).
+template <typename T>
+constexpr size_t kInstSmallChunk = size_t(kBlockSize) * (16 / sizeof(T)) * kInstUnroll;
+
+// Whether a workgroup holds a sample whose sums are added in the order of chunks, as those of larger samples are, so that a team can run a whole pass
+// (softmax_inst_team_*_kernel), and a workgroup, in whole vectors, any (softmax_inst_rounds_kernel).  vec: elements of a vector.
+// Single elements: only what teams may take, of the upper half; forward + backward, one workgroup's lanes -> in rounds in us, N 2, 12001 floats 10.4 and 10.2, but
+// N 256, 17101 22.5 and 23.2, dot products and gradients alone 32 and 34.  Lane by lane -> by teams: N 4, 17101 floats 13.7 -> 10.8, N 64
+// 15.4 -> 13.7, N 2, 28225 16.7 -> 10.9; N 4, 9001 doubles 13.4 -> 10.0; in place, in rounds, 14.0 -> 12.2, 15.4 -> 13.6, 16.9 -> 14.9, 13.6 -> 12.4.
+template <typename T>
+bool inst_by_chunks(int n, size_t sample_size, int vec)
+{
+    if (n <= 0 || sample_size > kInstSmallSample<T> || sample_size <= kInstSmallChunk<T>)
+        return false;
+    const size_t chunks = (sample_size + kInstSmallChunk<T> - 1) / kInstSmallChunk<T>;
+    return vec == 16 / sizeof(T) || (chunks > 4 && chunks * n <= 2 * chip_units());
+}
+
+// Whether the lanes of a wave or a workgroup hold a sample, each adding up its own elements.
+template <typename T>
+bool inst_by_lanes(int n, size_t sample_size, int vec)
+{
+    return n > 0 && sample_size <= kInstSmallSample<T> && !inst_by_chunks<T>(n, sample_size, vec);
+}
+
 template <typename T, int MODE>
 int inst_small(int n, size_t sample_size, const void* a, const void* b, void* out,
                const void* param, void* result, void* result2, T min_output, hipStream_t st)
@@ -1849,6 +1874,8 @@ int inst_small(int n, size_t sample_size, const void* a, const void* b, void* ou
         return launch_status();
     });
 }
+
+#include "h2x_softmax_team.hpp"
 
 template <typename T>
 T inst_min_output()
@@ -1915,6 +1942,36 @@ InstChunking inst_plan(int n, size_t sample_size, const void* a, const void* b, 
     return inst_chunking(sample_size, n, *v, sizeof(T));
 }
 
+// One reduction, or a whole pass, of few samples that a workgroup holds, added in the order of chunks.
+template <typename T, int MODE>
+int inst_rounds(int n, size_t sample_size, const void* a, const void* b, void* out, const void* param, void* result, void* result2,
+                T min_output, hipStream_t st)
+{
+    constexpr int kFull = 16 / sizeof(T);
+    int v;
+    // (dx of a whole pass is as aligned as its inputs)
+    const InstChunking ch = inst_plan<T>(n, sample_size, a, b, MODE == kSmallBackward ? nullptr : out, &v);
+    if (ch.chunk != kInstSmallChunk<T> || ch.groups > 8)
+        return H2X_ERR_INVALID_ARGUMENT; // (never: see inst_chunking)
+    const auto run = [&](auto vec, auto rounds) {
+        constexpr int VEC = decltype(vec)::value, ROUNDS = decltype(rounds)::value;
+        launch(softmax_inst_rounds_kernel<T, VEC, kInstSmallChunk<T> / kBlockSize / VEC, ROUNDS, MODE>, n, 4 * kBlockSize, st,
+               static_cast<const T*>(a), static_cast<const T*>(b), static_cast<T*>(out), static_cast<const T*>(param),
+               static_cast<T*>(result), static_cast<T*>(result2), static_cast<uint32_t>(sample_size), min_output);
+    };
+    const auto wide = [&](auto vec) {
+        if (ch.groups <= 4)
+            run(vec, std::integral_constant<int, 1>());
+        else
+            run(vec, std::integral_constant<int, 2>());
+    };
+    if (v == kFull)
+        wide(std::integral_constant<int, kFull>());
+    else // (teams have more than four chunks)
+        run(std::integral_constant<int, 1>(), std::integral_constant<int, 2>());
+    return launch_status();
+}
+
 // The partial sums of a reduction at `partials` (groups_max of them a sample); no finishing launch.
 template <typename T, int MODE, bool COMBINE = false>
 void inst_partials(int n, size_t sample_size, const void* a, const void* b, void* out, const void* param,
@@ -1940,7 +1997,9 @@ template <typename T, int MODE>
 int inst_reduce(int n, size_t sample_size, const void* a, const void* b, void* out,
                 const void* param, void* result, void* workspace, hipStream_t st)
 {
-    if (sample_size <= kInstSmallSample<T> && n > 0)
+    int v;
+    inst_plan<T>(n, sample_size, a, b, out, &v);
+    if (inst_by_lanes<T>(n, sample_size, v) || (MODE == kInstMax && n > 0 && sample_size <= kInstSmallSample<T>)) // (a maximum in any order)
     {
         constexpr int kSmallMode = MODE == kInstMax      ? kSmallMax
                                    : MODE == kInstExpSum ? kSmallExpSum
@@ -1948,7 +2007,9 @@ int inst_reduce(int n, size_t sample_size, const void* a, const void* b, void* o
                                                          : kSmallDot;
         return inst_small<T, kSmallMode>(n, sample_size, a, b, out, param, result, nullptr, T(0), st);
     }
-    int v;
+    if constexpr (MODE == kInstExpSum || MODE == kInstDot) // (kInstSumExp is of whole passes of larger samples)
+        if (inst_by_chunks<T>(n, sample_size, v))
+            return inst_rounds<T, MODE == kInstDot ? kSmallDot : kSmallExpSum>(n, sample_size, a, b, out, param, result, nullptr, T(0), st);
     double* partials = static_cast<double*>(workspace);
     inst_partials<T, MODE>(n, sample_size, a, b, out, param, partials, st);
     launch(softmax_inst_finish_kernel<T, MODE == kInstMax>, n, kBlockSize, st, partials,
@@ -1976,8 +2037,6 @@ int inst_map(int n, size_t sample_size, const void* y, const void* dy, const voi
                static_cast<const T*>(shift), static_cast<T*>(out), sample_size, min_output, sum_partials, gmax);
     return launch_status();
 }
-
-#include "h2x_softmax_team.hpp"
 
 // Vectors of 16 bytes a thread that members of four chunks hold at most: beyond, 1024 threads lack the registers.
 constexpr int kInstMostForward = 16, kInstMostBackward = 8;
@@ -2012,12 +2071,23 @@ template <typename T, bool FORWARD>
 bool inst_team(int n, size_t sample_size, const void* a, const void* b, const void* out, int* v, InstTeam* g)
 {
     constexpr int most = FORWARD ? kInstMostForward : kInstMostBackward;
-    if (sample_size <= kInstSmallSample<T> || n <= 0)
+    if (n <= 0 || sample_size <= kInstSmallChunk<T>)
         return false;
     const InstChunking ch = inst_plan<T>(n, sample_size, a, b, out, v);
+    if (inst_by_lanes<T>(n, sample_size, *v))
+        return false;
     const int each = static_cast<int>(ch.chunk / kBlockSize / (16 / sizeof(T))); // vectors of 16 bytes
     const int chunks = ch.groups <= static_cast<int>(kInstMembers) ? 1 : 4;
     const int members = (ch.groups + chunks - 1) / chunks;
+    // Of what a workgroup holds, samples of more than four chunks, of which there are few.  One workgroup each and by teams, us: N 64, 5 chunks of floats
+    // 11.6 and 12.2, of doubles 11.3 and 11.9, N 32 11.0 and 9.9; N 128, 5 chunks 15.2 and 15.9, doubles 14.1 and 15.6; N 96, 7 chunks
+    // 19.7 and 17.4, N 128 22.0 and 20.8; N 128, 8 chunks 23.8 and 22.6, N 256 39.4 and 38.1 before a workgroup's first round went without comparisons (37.5 so).
+    if (inst_by_chunks<T>(n, sample_size, *v))
+    {
+        const int cus = static_cast<int>(compute_units());
+        if (ch.groups <= 4 || !(2 * members * n <= 3 * cus || (ch.groups >= 6 && 2 * n <= cus)))
+            return false;
+    }
     static_assert(4 * kInstMembers >= kInstCombine, "members of four hold all chunks");
     if (ch.groups > kInstCombine || each > (chunks == 1 ? 16 : most) || 4 * members > static_cast<int>(compute_units()))
         return false;
@@ -2071,14 +2141,17 @@ template <typename T>
 int inst_forward_local(int n, size_t sample_size, const void* x, void* y, void* sample_max,
                        void* sample_exp, void* workspace, hipStream_t st)
 {
-    if (sample_size <= kInstSmallSample<T> && n > 0)
+    int v;
+    const int sums = inst_plan<T>(n, sample_size, x, nullptr, y, &v).groups;
+    if (inst_by_lanes<T>(n, sample_size, v))
         return inst_small<T, kSmallForward>(n, sample_size, x, nullptr, y, nullptr, sample_max,
                                             sample_exp, inst_min_output<T>(), st);
+    if (inst_by_chunks<T>(n, sample_size, v))
+        return inst_rounds<T, kSmallForward>(n, sample_size, x, nullptr, y, nullptr, sample_max, sample_exp, inst_min_output<T>(), st);
     // `y` takes part in the choice of the vector width only, as in the staged call,
     // so that the sum is cut up and added in the same order
-    int v;
-    const int maxima = inst_plan<T>(n, sample_size, x, nullptr, nullptr, &v).groups;
-    const int sums = inst_plan<T>(n, sample_size, x, nullptr, y, &v).groups;
+    int v_x;
+    const int maxima = inst_plan<T>(n, sample_size, x, nullptr, nullptr, &v_x).groups;
     // the partials of both reductions lie side by side in the workspace
     if (n > 0 && maxima <= kInstCombine && sums <= kInstCombine && maxima + sums <= inst_groups_per_sample_max(n))
     {
@@ -2101,12 +2174,15 @@ template <typename T>
 int inst_backward_local(int n, size_t sample_size, const void* y, const void* dy, void* dx, void* sample_dp,
                         void* workspace, hipStream_t st)
 {
-    if (sample_size <= kInstSmallSample<T> && n > 0)
-        return inst_small<T, kSmallBackward>(n, sample_size, y, dy, dx, nullptr, sample_dp, nullptr,
-                                             inst_min_output<T>(), st);
     int v;
     const int sums = inst_plan<T>(n, sample_size, y, dy, nullptr, &v).groups;
-    if (n > 0 && sums <= kInstCombine)
+    if (inst_by_lanes<T>(n, sample_size, v))
+        return inst_small<T, kSmallBackward>(n, sample_size, y, dy, dx, nullptr, sample_dp, nullptr,
+                                             inst_min_output<T>(), st);
+    const bool by_chunks = inst_by_chunks<T>(n, sample_size, v);
+    if (by_chunks && vector_width<T>(sample_size, v, {dx}) == v) // dx takes no part in the cut
+        return inst_rounds<T, kSmallBackward>(n, sample_size, y, dy, dx, nullptr, sample_dp, nullptr, inst_min_output<T>(), st);
+    if (n > 0 && sums <= kInstCombine && !by_chunks)
     {
         double* const partials = static_cast<double*>(workspace);
         inst_partials<T, kInstDot>(n, sample_size, y, dy, nullptr, nullptr, partials, st);

@@ -313,3 +313,99 @@ __global__ __launch_bounds__(TEAM, (inst_waves<T, TEAM, 2 * VEC * V, VEC == 1>()
         P::store(inst_at<VEC>(op, k, i), v[k]);
     });
 }
+
+// Samples of several chunks that one workgroup holds, where a team is not for the call (many samples, smaller ones, in place, a single reduction, no
+// state): the workgroup plays the chunks, four a round, and adds their sums as the combination of stored ones does: a round's are
+// what a member of four chunks exchanges, and one addition, the last that is not of zeros, is left.  All rounds but the last are of
+// whole chunks.  Bound by the work of a CU and by waits in a row.  The kernel that adds lane by lane, which loads single
+// elements and compares for each, -> this, forward + backward in us, going round three sets of tensors:
+//   floats  N 16, 4100    8.4 -> 7.3      N 16, 12000   10.5 -> 8.7     N 128, 16400  17.0 -> 14.3    N 256, 32768  41.1 -> 37.5
+//   doubles N 16, 4200    9.1 -> 7.7      N 128, 8200   15.4 -> 13.7    N 500, 12000  58.7 -> 52.1    N 500, 16384  78.0 -> 66.7
+//   in place, floats  N 2, 32768  18.2 -> 14.5    N 64, 20000  16.1 -> 12.8    N 256, 28224  29.5 -> 27.5
+// (With comparisons in all rounds N 2, 32768 in place 16.4.)
+template <typename T, int VEC, int V, int ROUNDS, int MODE>
+__global__ __launch_bounds__(4 * kBlockSize) void softmax_inst_rounds_kernel(const T* a, const T* b, T* out, const T* sample_param,
+                                                                             T* __restrict__ result, T* __restrict__ result2,
+                                                                             uint32_t sample_size, T min_output)
+{
+    using P = Pack<T, VEC>;
+    constexpr int TEAM = 4 * kBlockSize;
+    constexpr bool kDot = MODE == kSmallDot || MODE == kSmallBackward;
+    __shared__ double waves[ROUNDS + 1][TEAM / kWaveSize];
+    const uint32_t n = blockIdx.x;
+    InstTeam g = {};
+    g.sample_size = sample_size;
+    g.chunk = kBlockSize * VEC * V;
+    const size_t base = static_cast<size_t>(n) * sample_size;
+    // f(k, bytes) for the vectors of a thread in a round
+    const auto of_round = [&](int r, const auto& f) {
+        if (r + 1 == ROUNDS)
+        {
+            inst_chunk<T, TEAM, VEC, V>(g, r, f);
+            return;
+        }
+        const uint32_t first = (r * 4 + threadIdx.x / kBlockSize) * g.chunk + threadIdx.x % kBlockSize * VEC;
+#pragma unroll
+        for (int k = 0; k < V; ++k)
+            f(k, first * static_cast<uint32_t>(sizeof(T)));
+    };
+    P va[ROUNDS][V], vb[kDot ? ROUNDS : 1][V];
+#pragma unroll
+    for (int r = 0; r < ROUNDS; ++r)
+        of_round(r, [&](int k, uint32_t i) {
+            va[r][k] = P::load(inst_at<VEC>(a + base, k, i));
+            if constexpr (kDot)
+                vb[r][k] = P::load(inst_at<VEC>(b + base, k, i));
+        });
+    T shift = T(0);
+    if constexpr (MODE == kSmallForward)
+    {
+        T mx = Limits<T>::min_normal;
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r)
+            of_round(r, [&](int k, uint32_t) { add_max<T, VEC>(mx, va[r][k]); });
+        shift = static_cast<T>(inst_partial<TEAM, false>(static_cast<double>(mx), waves[ROUNDS]));
+        if (threadIdx.x == 0)
+            result[n] = shift;
+    }
+    else if constexpr (!kDot)
+    {
+        shift = sample_param[n];
+    }
+    double total = 0.0;
+#pragma unroll
+    for (int r = 0; r < ROUNDS; ++r)
+    {
+        double acc = 0.0;
+        of_round(r, [&](int k, uint32_t) {
+            if constexpr (kDot)
+                add_products<T, VEC>(acc, va[r][k], vb[r][k]);
+            else
+                add_exponentials<T, VEC>(acc, va[r][k], shift);
+        });
+        total += inst_partial<TEAM, true>(acc, waves[r]);
+    }
+    const T sum = static_cast<T>(total);
+    if (threadIdx.x == 0)
+        (MODE == kSmallForward ? result2 : result)[n] = sum;
+    if constexpr (MODE != kSmallDot)
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r)
+            of_round(r, [&](int k, uint32_t i) {
+                if constexpr (MODE != kSmallExpSum)
+                {
+#pragma unroll
+                    for (int j = 0; j < VEC; ++j)
+                        if constexpr (MODE == kSmallForward)
+                        {
+                            const T q = va[r][k][j] / sum;
+                            va[r][k][j] = q > min_output ? q : min_output;
+                        }
+                        else
+                        {
+                            va[r][k][j] = va[r][k][j] > min_output ? va[r][k][j] * (vb[r][k][j] - sum) : T(0);
+                        }
+                }
+                P::store(inst_at<VEC>(out + base, k, i), va[r][k]);
+            });
+}
