@@ -978,7 +978,7 @@ __device__ __forceinline__ void store_slot(T* p, const ShortLane& l, const T (&r
 }
 
 // The K sums of channel c from its `groups` partials, one after the other.  The
-// finishing kernel and the consumers that finish a reduction themselves both
+// finishing kernel and the consumers (window_totals) that finish a reduction themselves both
 // add in this order and so arrive at the same bits.  The short-segment kernels
 // keep their partials group by group, partials[(group * C + c) * K + k]:
 // neighbouring lanes, which serve neighbouring channels, then read neighbouring
@@ -1009,6 +1009,47 @@ __device__ __forceinline__ void sequential_totals(const double* __restrict__ par
                 if (g0 + u < groups)
                     t[k] += p[u][k];
     }
+}
+
+// The K sums of the channels of a workgroup's window, added as sequential_totals does, a sum by a thread: totals[k][q] of channel q, and the
+// outputs where the workgroup is the window's first.  Ends with a barrier.  The passes that finish a reduction so are bound by what they wait
+// for before their first store: their first batch of elements is loaded ahead of the sums.  One lane a channel adding all K sums, elements loaded behind them -> this, doubles,
+// forward, backward in us of the two launches, going round three sets of tensors: N 135, C 455, 5 x 7 14.9, 26.3 -> 13.4, 21.4; N 228, C 69, 10 x 9
+// 12.6, 20.7 -> 12.1, 17.5; N 173, C 143, 13 x 10 19.2, 35.4 -> 18.1, 28.2; N 200, C 600, 7 x 7 27.4, 53.6 -> 26.4, 41.9; N 40, C 2000,
+// 14 x 14 with a halo 97, 136 -> 94, 134.  (The elements alone ahead: backward 26.3, 20.1, 35.9, 55.3.  Batches of four samples backward 21.2,
+// 17.1, 29.3, 42.3, and 59 against 58 for N 243, C 306, 4 x 6 x 5; of all four sums in a lane 98 registers instead of 80.)
+template <typename T, int K>
+__device__ __forceinline__ void window_totals(const FusedStats<T>& f, const ShortGeometry& g, T (&totals)[K][kBlockSize], bool store)
+{
+    const size_t pitch = static_cast<size_t>(g.num_channels) * K;
+    for (int i = threadIdx.x; i < g.channels_per_group * K; i += kBlockSize)
+    {
+        const int q = i / K, k = i % K, c = static_cast<int>(blockIdx.x) * g.channels_per_group + q;
+        if (c >= g.num_channels)
+            break;
+        const uint32_t at = static_cast<uint32_t>(c * K + k) * 8u; // in bytes; with a row's start in scalars
+        const auto of_group = [&](int group) {
+            return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(f.partials + group * pitch) + at);
+        };
+        double t = of_group(0);
+        constexpr int kBatch = 7; // with the first as many as kShortMaxGroups
+        for (int g0 = 1; g0 < f.groups; g0 += kBatch)
+        {
+            double p[kBatch];
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u)
+                if (g0 + u < f.groups)
+                    p[u] = of_group(g0 + u);
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u)
+                if (g0 + u < f.groups)
+                    t += p[u];
+        }
+        totals[k][q] = static_cast<T>(t);
+        if (store)
+            f.out[k][c] = totals[k][q];
+    }
+    __syncthreads();
 }
 
 // Adds what the lanes of each channel hold and stores the
@@ -1150,32 +1191,38 @@ __global__ __launch_bounds__(kBlockSize) void bn_apply_short_kernel(
 {
     constexpr bool FUSED = MODE == kFusedApply, STREAM = MODE != kNormalApply;
     const ShortLane l = short_lane<VEC, TAIL>(g, static_cast<int>(threadIdx.x), static_cast<int>(blockIdx.x));
+    const T* const xp = x + l.c * tx.stride_c + slot_offset(l, tx);
+    const int64_t x_stride_n = tx.stride_n, y_stride_n = ty.stride_n;
+    int n = blockIdx.y * g.samples_per_group;
+    const int end =
+        n + g.samples_per_group < g.num_samples ? n + g.samples_per_group : g.num_samples;
+    T v[kUnroll][VEC];
+    const auto load = [&] {
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u)
+            if (n + u < end)
+                load_slot<T, VEC, TAIL>(xp + (n + u) * x_stride_n, l, v[u]);
+    };
+    T sc = T(0), bi = T(0);
+    if (l.valid > 0)
+    {
+        load();
+        sc = scale[l.c];
+        bi = bias[l.c];
+    }
     T m = T(0), variance = T(0);
     if constexpr (FUSED)
     {
-        __shared__ T stats[2][kBlockSize];
-        if (l.leads)
-        {
-            double t[2];
-            sequential_totals<2>(fused.partials, fused.groups, g.num_channels, l.c, t);
-            sums_to_mean_var(static_cast<T>(t[0]), static_cast<T>(t[1]),
-                             static_cast<T>(fused.num_per_sum), &m, &variance);
-            stats[0][l.q] = m;
-            stats[1][l.q] = variance;
-            if (blockIdx.y == 0)
-            {
-                fused.out[0][l.c] = m;
-                fused.out[1][l.c] = variance;
-                fused.out[2][l.c] = fma_t(fused.decay, fused.out[2][l.c], (T(1) - fused.decay) * m);
-                fused.out[3][l.c] =
-                    fma_t(fused.decay, fused.out[3][l.c], (T(1) - fused.decay) * variance);
-            }
-        }
-        __syncthreads();
+        __shared__ T totals[2][kBlockSize];
+        window_totals<T, 2>(fused, g, totals, false);
         if (l.valid > 0)
+            sums_to_mean_var(totals[0][l.q], totals[1][l.q], static_cast<T>(fused.num_per_sum), &m, &variance);
+        if (l.leads && blockIdx.y == 0)
         {
-            m = stats[0][l.q];
-            variance = stats[1][l.q];
+            fused.out[0][l.c] = m;
+            fused.out[1][l.c] = variance;
+            fused.out[2][l.c] = fma_t(fused.decay, fused.out[2][l.c], (T(1) - fused.decay) * m);
+            fused.out[3][l.c] = fma_t(fused.decay, fused.out[3][l.c], (T(1) - fused.decay) * variance);
         }
     }
     else if (l.valid > 0)
@@ -1186,37 +1233,22 @@ __global__ __launch_bounds__(kBlockSize) void bn_apply_short_kernel(
     if (l.valid == 0)
         return;
     const T inv_stdev = inv_sqrt_t(variance + epsilon);
-    const T sc = scale[l.c];
-    const T bi = bias[l.c];
-    const T* xp = x + l.c * tx.stride_c + slot_offset(l, tx);
-    T* yp = y + l.c * ty.stride_c + slot_offset(l, ty);
-    const int64_t x_stride_n = tx.stride_n, y_stride_n = ty.stride_n;
-    int n = blockIdx.y * g.samples_per_group;
-    const int end =
-        n + g.samples_per_group < g.num_samples ? n + g.samples_per_group : g.num_samples;
-    for (; n + kUnroll <= end; n += kUnroll)
+    T* const yp = y + l.c * ty.stride_c + slot_offset(l, ty);
+    for (;;)
     {
-        T v[kUnroll][VEC];
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u)
-            load_slot<T, VEC, TAIL>(xp + (n + u) * x_stride_n, l, v[u]);
+            if (n + u < end)
+            {
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u)
-        {
-#pragma unroll
-            for (int j = 0; j < VEC; ++j)
-                v[u][j] = fma_t((v[u][j] - m) * inv_stdev, sc, bi);
-            store_slot<T, VEC, TAIL, STREAM>(yp + (n + u) * y_stride_n, l, v[u], true);
-        }
-    }
-    for (; n < end; ++n)
-    {
-        T v[VEC];
-        load_slot<T, VEC, TAIL>(xp + n * x_stride_n, l, v);
-#pragma unroll
-        for (int j = 0; j < VEC; ++j)
-            v[j] = fma_t((v[j] - m) * inv_stdev, sc, bi);
-        store_slot<T, VEC, TAIL, STREAM>(yp + n * y_stride_n, l, v, true);
+                for (int j = 0; j < VEC; ++j)
+                    v[u][j] = fma_t((v[u][j] - m) * inv_stdev, sc, bi);
+                store_slot<T, VEC, TAIL, STREAM>(yp + (n + u) * y_stride_n, l, v[u], true);
+            }
+        n += kUnroll;
+        if (n >= end) // uniform
+            break;
+        load();
     }
 }
 
@@ -1299,28 +1331,40 @@ __global__ __launch_bounds__(kBlockSize) void bn_backprop2_short_kernel(
     const ShortTensor to, const ShortGeometry g, bool disjoint, const FusedStats<T> fused)
 {
     const ShortLane l = short_lane<VEC, TAIL>(g, static_cast<int>(threadIdx.x), static_cast<int>(blockIdx.x));
+    constexpr int kBatch = kUnroll / 2; // two streams: same bytes in flight
+    const T* const xp = x + l.c * tx.stride_c + slot_offset(l, tx);
+    const T* const dp = dy + l.c * td.stride_c + slot_offset(l, td);
+    const int64_t x_stride_n = tx.stride_n, d_stride_n = td.stride_n, o_stride_n = to.stride_n;
+    int n = blockIdx.y * g.samples_per_group;
+    const int end =
+        n + g.samples_per_group < g.num_samples ? n + g.samples_per_group : g.num_samples;
+    T xv[kBatch][VEC], dv[kBatch][VEC];
+    const auto load = [&] {
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u)
+            if (n + u < end)
+            {
+                load_slot<T, VEC, TAIL>(xp + (n + u) * x_stride_n, l, xv[u]);
+                load_slot<T, VEC, TAIL, true>(dp + (n + u) * d_stride_n, l, dv[u]);
+            }
+    };
+    T m = T(0), sc = T(0), variance = T(0);
+    if (l.valid > 0)
+    {
+        load();
+        m = mean[l.c];
+        sc = scale[l.c];
+        variance = var[l.c];
+    }
     T dmean_c = T(0), dvar_c = T(0);
     if constexpr (FUSED)
     {
-        __shared__ T totals[2][kBlockSize];
-        if (l.leads)
-        {
-            double t[4];
-            sequential_totals<4>(fused.partials, fused.groups, g.num_channels, l.c, t);
-            totals[0][l.q] = static_cast<T>(t[2]);
-            totals[1][l.q] = static_cast<T>(t[3]);
-            if (blockIdx.y == 0)
-            {
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    fused.out[k][l.c] = static_cast<T>(t[k]);
-            }
-        }
-        __syncthreads();
+        __shared__ T totals[4][kBlockSize];
+        window_totals<T, 4>(fused, g, totals, blockIdx.y == 0);
         if (l.valid > 0)
         {
-            dmean_c = totals[0][l.q];
-            dvar_c = totals[1][l.q];
+            dmean_c = totals[2][l.q];
+            dvar_c = totals[3][l.q];
         }
     }
     else if (l.valid > 0)
@@ -1330,52 +1374,28 @@ __global__ __launch_bounds__(kBlockSize) void bn_backprop2_short_kernel(
     }
     if (l.valid == 0)
         return;
-    const T m = mean[l.c];
-    const T sc = scale[l.c];
-    const T inv_stdev = inv_sqrt_t(var[l.c] + epsilon);
+    const T inv_stdev = inv_sqrt_t(variance + epsilon);
     const T dmean_term = dmean_c / static_cast<T>(num_per_sum);
     const T dvar_term = dvar_c * T(2) / static_cast<T>(num_per_sum - 1);
-    constexpr int kUnroll2 = kUnroll / 2;
-    const T* xp = x + l.c * tx.stride_c + slot_offset(l, tx);
-    const T* dp = dy + l.c * td.stride_c + slot_offset(l, td);
-    T* op = dx + l.c * to.stride_c + slot_offset(l, to);
-    const int64_t x_stride_n = tx.stride_n, d_stride_n = td.stride_n, o_stride_n = to.stride_n;
-    int n = blockIdx.y * g.samples_per_group;
-    const int end =
-        n + g.samples_per_group < g.num_samples ? n + g.samples_per_group : g.num_samples;
-    for (; n + kUnroll2 <= end; n += kUnroll2)
+    T* const op = dx + l.c * to.stride_c + slot_offset(l, to);
+    for (;;)
     {
-        T xv[kUnroll2][VEC], dv[kUnroll2][VEC];
 #pragma unroll
-        for (int u = 0; u < kUnroll2; ++u)
-        {
-            load_slot<T, VEC, TAIL>(xp + (n + u) * x_stride_n, l, xv[u]);
-            load_slot<T, VEC, TAIL, true>(dp + (n + u) * d_stride_n, l, dv[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < kUnroll2; ++u)
-        {
-#pragma unroll
-            for (int j = 0; j < VEC; ++j)
+        for (int u = 0; u < kBatch; ++u)
+            if (n + u < end)
             {
-                const T r = fma_t(dv[u][j] * sc, inv_stdev, dmean_term);
-                xv[u][j] = fma_t(xv[u][j] - m, dvar_term, r);
-            }
-            store_slot<T, VEC, TAIL>(op + (n + u) * o_stride_n, l, xv[u], disjoint);
-        }
-    }
-    for (; n < end; ++n)
-    {
-        T xv[VEC], dv[VEC];
-        load_slot<T, VEC, TAIL>(xp + n * x_stride_n, l, xv);
-        load_slot<T, VEC, TAIL, true>(dp + n * d_stride_n, l, dv);
 #pragma unroll
-        for (int j = 0; j < VEC; ++j)
-        {
-            const T r = fma_t(dv[j] * sc, inv_stdev, dmean_term);
-            xv[j] = fma_t(xv[j] - m, dvar_term, r);
-        }
-        store_slot<T, VEC, TAIL>(op + n * o_stride_n, l, xv, disjoint);
+                for (int j = 0; j < VEC; ++j)
+                {
+                    const T r = fma_t(dv[u][j] * sc, inv_stdev, dmean_term);
+                    xv[u][j] = fma_t(xv[u][j] - m, dvar_term, r);
+                }
+                store_slot<T, VEC, TAIL>(op + (n + u) * o_stride_n, l, xv[u], disjoint);
+            }
+        n += kBatch;
+        if (n >= end) // uniform
+            break;
+        load();
     }
 }
 
