@@ -885,11 +885,10 @@ __global__ __launch_bounds__(kBlockSize) void bn_clearing_kernel(
         for (int u = 0; u < kInFlight; ++u)
         {
             const size_t i = tile + u * kStride + threadIdx.x * VEC;
-            bool inside[VEC];
-            interior_mask<VEC>(box, static_cast<uint32_t>(i), inside);
+            const uint32_t inside = interior_bits<VEC>(box, static_cast<uint32_t>(i));
 #pragma unroll
             for (int j = 0; j < VEC; ++j)
-                xv[u][j] = inside[j] ? result(xv[u][j], BACKWARD ? dv[u][j] : T(0)) : T(0);
+                xv[u][j] = inside >> j & 1 ? result(xv[u][j], BACKWARD ? dv[u][j] : T(0)) : T(0);
             store_vec<T, VEC, true>(op + i, xv[u]);
         }
     }
@@ -899,11 +898,10 @@ __global__ __launch_bounds__(kBlockSize) void bn_clearing_kernel(
         load_vec<T, VEC, true>(xp + i, xv);
         if constexpr (BACKWARD)
             load_vec<T, VEC, true, true>(dp + i, dv);
-        bool inside[VEC];
-        interior_mask<VEC>(box, static_cast<uint32_t>(i), inside);
+        const uint32_t inside = interior_bits<VEC>(box, static_cast<uint32_t>(i));
 #pragma unroll
         for (int j = 0; j < VEC; ++j)
-            xv[j] = inside[j] ? result(xv[j], BACKWARD ? dv[j] : T(0)) : T(0);
+            xv[j] = inside >> j & 1 ? result(xv[j], BACKWARD ? dv[j] : T(0)) : T(0);
         store_vec<T, VEC, true>(op + i, xv);
     }
 }

@@ -17,7 +17,7 @@
 //   short family: lane = short_lane(thread, window); reductions walk samples
 //     first + row, + rows, ...; elementwise kernels every sample of the range.
 //   halo-clearing kernel (bn_clearing_kernel): workgroup b = (segment, chunk)
-//     over the real tensor, vectors as above, interior_mask per vector.
+//     over the real tensor, vectors as above, interior_bits per vector.
 #include "h2x_bn_plan.hpp"
 
 #include <algorithm>
@@ -437,8 +437,7 @@ extern "C" int h2x_bn_audit_clearing(int backward, h2x_dtype dtype, const h2x_ha
                 const size_t end = std::min(begin + r.chunk, r.real);
                 for (size_t i = begin; i + VEC <= end; i += VEC)
                 {
-                    bool inside[VEC];
-                    interior_mask<VEC>(r.box, static_cast<uint32_t>(i), inside);
+                    const uint32_t inside = interior_bits<VEC>(r.box, static_cast<uint32_t>(i));
                     for (int j = 0; j < VEC; ++j)
                     {
                         const size_t at = seg * r.real + i + j;
@@ -454,7 +453,7 @@ extern "C" int h2x_bn_audit_clearing(int backward, h2x_dtype dtype, const h2x_ha
                             ++t[last].outside;
                             continue;
                         }
-                        t[last].outside += inside[j] != (interior[i + j] != 0);
+                        t[last].outside += (inside >> j & 1) != (interior[i + j] != 0);
                         if (stored[at] < 255)
                             ++stored[at];
                     }

@@ -94,13 +94,7 @@ __host__ __device__ __forceinline__ uint32_t once_place(const ClearGeometry& g, 
     // (a last vector that starts early shares only halo cells with the one before it, which stores the same zeros)
     const uint32_t first = (i - n * g.per_segment.divisor) * VEC;
     const uint32_t e = first < g.last ? first : g.last;
-    bool inside[VEC];
-    interior_mask<VEC>(g.box, e, inside);
-    uint32_t mask = 0;
-#pragma unroll
-    for (int j = 0; j < VEC; ++j)
-        mask |= static_cast<uint32_t>(inside[j]) << j;
-    return (e + n * g.stride_n) * 16 + mask;
+    return (e + n * g.stride_n) * 16 + interior_bits<VEC>(g.box, e);
 }
 
 // STREAM: past the caches.  Rows of a few hundred bytes are stored normally: their
