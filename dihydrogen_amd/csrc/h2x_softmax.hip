@@ -1089,8 +1089,8 @@ void launch_bwd(const T* y, const T* dy, T* dx, int n, int c, size_t s, bool str
         launch(softmax_bwd_reg_kernel<T, VEC, CMAX, false>, grid, kBlockSize, st, y, dy, dx, c, s, flat);
 }
 
-// More samples than this fill the chip with a wave each.
-constexpr int kManySamples = 2048;
+// More samples than this fill the chip with a wave each; and more than this leave its waves little to wait for where samples are short.
+constexpr int kManySamples = 2048, kSomeSamples = 512;
 
 // Which kernel serves which channel count (measured on MI355X).  Up to 32 channels a
 // thread keeps all channels of its pixels (softmax_*_reg_kernel: 21 channels of
@@ -1302,9 +1302,12 @@ int launch_shared_for(int n, int c, size_t s, hipStream_t st, P... p)
 // Calls f(elements a lane, lanes) with constants for samples of `size` contiguous elements that
 // lanes hold in registers: a wave while samples are short, or many (it needs no barrier), else
 // a workgroup, of 1024 threads with up to MAX_LARGE elements each where 256 would have more than 16.
-// SPREAD: a workgroup from 257 elements (the sums are fp64; sums of the data's type keep the order that
-// a wave gives them: N 64, 600 channels 4.5 us, in a workgroup 4.1).
-template <bool SPREAD, int MAX_LARGE = 0, typename F>
+// A workgroup from 257 elements on, and from 513 also of more than kSomeSamples: a wave's chain of up to 32 loads, exponentials and stores is what
+// else is waited for (sums of the data's type have fewer terms in a row so).  GPU time, a wave a sample -> a workgroup, forward / backward in us: channels, floats
+// N 16, 1000 3.1 / 2.4 -> 2.2 / 1.8, N 466, 1983 5.1 / 4.2 -> 3.3 / 2.9, N 1418, 1480 6.7 / 6.0 -> 5.6 / 5.4; doubles N 59, 1480 6.6 / 3.8 -> 3.3 / 2.3, N 700, 1000 5.7 /
+// 4.5 -> 4.3 / 3.8, N 1418, 704 6.4 / 5.6 -> 5.7 / 5.2; instances of doubles N 128, 1983 8.6 / 4.6 -> 4.0 / 2.7.  With more samples, floats N 466,
+// 300 2.2 / 1.9 both ways, N 1000, 300 2.4 / 1.9 and 2.8 / 1.9, 500 2.6 / 2.2 and 2.9 / 2.0; N 2600 the same either way.
+template <int MAX_LARGE = 0, typename F>
 int with_lanes(int n, size_t size, const F& f)
 {
 #define H2X_LANES(CPL, LANES)                                                                      \
@@ -1312,7 +1315,7 @@ int with_lanes(int n, size_t size, const F& f)
     if (size <= 1 * kWaveSize) H2X_LANES(1, kWaveSize);
     if (size <= 2 * kWaveSize) H2X_LANES(2, kWaveSize);
     if (size <= 4 * kWaveSize) H2X_LANES(4, kWaveSize);
-    if (!SPREAD || n > kManySamples)
+    if (n > (size <= 2 * kBlockSize ? kSomeSamples : kManySamples))
     {
         if (size <= 8 * kWaveSize) H2X_LANES(8, kWaveSize);
         if (size <= 16 * kWaveSize) H2X_LANES(16, kWaveSize);
@@ -1361,7 +1364,7 @@ int forward_impl(int n, int c, size_t s, const void* xv, void* yv, hipStream_t s
     T* y = static_cast<T*>(yv);
     constexpr int kWords = sizeof(T) / 4;
     if (s == 1 && c <= 32 * kBlockSize)
-        return with_lanes<false>(n, c, [&](auto cpl, auto lanes) {
+        return with_lanes(n, c, [&](auto cpl, auto lanes) {
             constexpr int CPL = decltype(cpl)::value, LANES = decltype(lanes)::value;
             launch(softmax_fwd_row_kernel<T, CPL, LANES>, lanes_grid<LANES>(n), lanes_block<LANES>(), st, x, y, c, n);
             return launch_status();
@@ -1434,7 +1437,7 @@ int backward_impl(int n, int c, size_t s, const void* yv, const void* dyv, void*
     T* dx = static_cast<T*>(dxv);
     constexpr int kWords = sizeof(T) / 4;
     if (s == 1 && c <= 32 * kBlockSize)
-        return with_lanes<false>(n, c, [&](auto cpl, auto lanes) {
+        return with_lanes(n, c, [&](auto cpl, auto lanes) {
             constexpr int CPL = decltype(cpl)::value, LANES = decltype(lanes)::value;
             launch(softmax_bwd_row_kernel<T, CPL, LANES>, lanes_grid<LANES>(n), lanes_block<LANES>(), st, y, dy,
                    dx, c, n);
@@ -1865,7 +1868,7 @@ template <typename T, int MODE>
 int inst_small(int n, size_t sample_size, const void* a, const void* b, void* out,
                const void* param, void* result, void* result2, T min_output, hipStream_t st)
 {
-    return with_lanes<sizeof(T) == 4, kInstLargeLanes<T>>(n, sample_size, [&](auto cpl, auto lanes) {
+    return with_lanes<kInstLargeLanes<T>>(n, sample_size, [&](auto cpl, auto lanes) {
         constexpr int CPL = decltype(cpl)::value, LANES = decltype(lanes)::value;
         launch(softmax_inst_small_kernel<T, CPL, MODE, LANES>, lanes_grid<LANES>(n), lanes_block<LANES>(), st,
                static_cast<const T*>(a), static_cast<const T*>(b), static_cast<T*>(out),
