@@ -580,26 +580,26 @@ def cpu_baseline(repeats: int = 5):
 # TCC_EA0_WRREQ_64B), request counts summed over the L2 channels, per dispatch.
 # label -> (bytes read, bytes written) per launch
 PMC_TRAFFIC = {
-    "bn_forward": (269481984, 269003136),
-    "bn_backward": (539887872, 269647744),
-    "bn_sums": (268460032, 131072),
-    "bn_apply": (268467200, 268480896),
-    "bn_backprop1": (536912384, 131072),
+    "bn_forward": (269489216, 269033824),
+    "bn_backward": (539861952, 269719744),
+    "bn_sums": (268459072, 131072),
+    "bn_apply": (268467200, 268477696),
+    "bn_backprop1": (536909824, 131072),
     "bn_backprop2": (536906240, 268435456),
-    "halo_dim0_pack": (147795200, 8652800),    # 4 faces (2 ranks) a launch, four launches a step
-    "halo_dim0_unpack": (9218368, 43264000),
-    "halo_dim1_pack": (42624832, 34611200),
-    "halo_dim1_unpack": (34633408, 36217728),
-    "halo_dim2_pack": (34694400, 34611200),
-    "halo_dim2_unpack": (34632448, 34619424),
+    "halo_dim0_pack": (147776096, 8652800),    # 4 faces (2 ranks) a launch, four launches a step
+    "halo_dim0_unpack": (9218128, 43264000),
+    "halo_dim1_pack": (42624768, 34611200),
+    "halo_dim1_unpack": (34632448, 36216544),
+    "halo_dim2_pack": (34695424, 34611200),
+    "halo_dim2_unpack": (34632448, 34619648),
 }
 # steps of the timed region whose dominant-kernel launches are bracketed by events: every EVENT_EVERY-th
 EVENT_EVERY = 4
 
 # sha256 (first 16 hex digits) of the kernel sources the table was measured with, see
 # kernel_sources_sha(); with other sources the traffic fields are omitted
-PMC_SOURCES_SHA = "2926489903eb3ca6"
-PMC_COMMIT = "30570f4"
+PMC_SOURCES_SHA = "858fb799a2fbe617"
+PMC_COMMIT = "4d12b66"
 
 KERNEL_OF = {
     "bn_forward": "bn_team_forward_kernel<float,512,16>",
