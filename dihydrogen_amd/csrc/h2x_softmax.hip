@@ -1090,7 +1090,7 @@ void launch_bwd(const T* y, const T* dy, T* dx, int n, int c, size_t s, bool str
 }
 
 // More samples than this fill the chip with a wave each; and more than this leave its waves little to wait for where samples are short.
-constexpr int kManySamples = 2048, kSomeSamples = 512;
+constexpr int kManySamples = 2048, kSomeSamples = 768;
 
 // Which kernel serves which channel count (measured on MI355X).  Up to 32 channels a
 // thread keeps all channels of its pixels (softmax_*_reg_kernel: 21 channels of
@@ -1305,8 +1305,9 @@ int launch_shared_for(int n, int c, size_t s, hipStream_t st, P... p)
 // A workgroup from 257 elements on, and from 513 also of more than kSomeSamples: a wave's chain of up to 32 loads, exponentials and stores is what
 // else is waited for (sums of the data's type have fewer terms in a row so).  GPU time, a wave a sample -> a workgroup, forward / backward in us: channels, floats
 // N 16, 1000 3.1 / 2.4 -> 2.2 / 1.8, N 466, 1983 5.1 / 4.2 -> 3.3 / 2.9, N 1418, 1480 6.7 / 6.0 -> 5.6 / 5.4; doubles N 59, 1480 6.6 / 3.8 -> 3.3 / 2.3, N 700, 1000 5.7 /
-// 4.5 -> 4.3 / 3.8, N 1418, 704 6.4 / 5.6 -> 5.7 / 5.2; instances of doubles N 128, 1983 8.6 / 4.6 -> 4.0 / 2.7.  With more samples, floats N 466,
-// 300 2.2 / 1.9 both ways, N 1000, 300 2.4 / 1.9 and 2.8 / 1.9, 500 2.6 / 2.2 and 2.9 / 2.0; N 2600 the same either way.
+// 4.5 -> 4.3 / 3.8, N 1418, 704 6.4 / 5.6 -> 5.7 / 5.2; instances of doubles N 128, 1983 8.6 / 4.6 -> 4.0 / 2.7.  With more samples, floats, a wave
+// and a workgroup: channels N 700, 300 2.3 / 1.9 and 2.5 / 2.0, N 1000, 300 2.4 / 1.9 and 2.8 / 1.9, 500 2.6 / 2.2 and 2.9 / 2.0; instances N 700, 400 3.0 / 2.2 and 2.7 /
+// 2.1, N 850 3.1 / 2.2 and 3.0 / 2.2, N 1418 3.1 / 2.3 and 3.4 / 2.6; N 2600 the same either way.
 template <int MAX_LARGE = 0, typename F>
 int with_lanes(int n, size_t size, const F& f)
 {
