@@ -1019,15 +1019,18 @@ __device__ __forceinline__ void sequential_totals(const double* __restrict__ par
 template <typename T, int K>
 __device__ __forceinline__ void window_totals(const FusedStats<T>& f, const ShortGeometry& g, T (&totals)[K][kBlockSize], bool store)
 {
+    const int first = static_cast<int>(blockIdx.x) * g.channels_per_group;
     const size_t pitch = static_cast<size_t>(g.num_channels) * K;
+    const double* const window = f.partials + static_cast<size_t>(first) * K;
     for (int i = threadIdx.x; i < g.channels_per_group * K; i += kBlockSize)
     {
-        const int q = i / K, k = i % K, c = static_cast<int>(blockIdx.x) * g.channels_per_group + q;
+        const int q = i / K, k = i % K, c = first + q;
         if (c >= g.num_channels)
             break;
-        const uint32_t at = static_cast<uint32_t>(c * K + k) * 8u; // in bytes; with a row's start in scalars
+        const uint32_t at = static_cast<uint32_t>(i) * 8u; // in bytes, behind the window's first sum, which is in scalars: of many
+                                                           // channels the place among all of a range's needs more bits
         const auto of_group = [&](int group) {
-            return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(f.partials + group * pitch) + at);
+            return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(window + group * pitch) + at);
         };
         double t = of_group(0);
         constexpr int kBatch = 7; // with the first as many as kShortMaxGroups

@@ -46,3 +46,28 @@ def test_the_bits_of_the_staged_calls(channels, segment, in_place, dtype):
             # a mean below 1 and a variance of 0.5 to 2 (q / n - mean^2, q / n up to 3): five roundings relative to 1 or twice that, then six
             eps = torch.finfo(tdt).eps
             assert bool(((results[0][0].double() - want).abs() <= 32 * eps * (1 + want.abs())).all()), n
+
+
+def test_sums_beyond_four_gigabytes_of_partials():
+    """So many channels that a sum's place among a range's partials takes more than 32 bits in bytes (four sums of 8 bytes each from 2^27 channels on)."""
+    import torch
+    from dihydrogen_amd import capi
+    calls, n, c = capi.calls(), 2, (1 << 27) + 300
+    workspace = capi.load().h2x_bn_workspace_bytes(c)
+    if torch.cuda.mem_get_info()[0] < workspace + (20 << 30):
+        pytest.skip("not enough free device memory")
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    ws = torch.empty(workspace, dtype=torch.uint8, device="cuda")
+    x, dy = (torch.randn((n, c), device="cuda", generator=gen) for _ in range(2))
+    mean, var, scale = (torch.rand(c, device="cuda", generator=gen) for _ in range(3))
+    nan = lambda: torch.full((c,), float("nan"), device="cuda")
+    dx, grads, staged = torch.full_like(x, 7), [nan() for _ in range(4)], [nan() for _ in range(4)]
+    assert not calls.h2x_bn_backward_local(capi.F32, n, c, 1, 1, 1, 1, n, x, dy, mean, var, scale, *grads, dx, 1e-5, ws, 0)
+    assert not calls.h2x_bn_backprop1(capi.F32, n, c, 1, 1, 1, x, dy, mean, var, scale, *staged, 1e-5, ws, 0)
+    for a, b in zip(grads, staged):
+        assert torch.equal(a, b)
+    whole, dx = dx, torch.full_like(dx, 7)
+    assert not calls.h2x_bn_backprop2(capi.F32, n, c, 1, 1, 1, 1, n, x, dy, mean, var, scale, staged[2], staged[3], dx, 1e-5, 0)
+    assert torch.equal(whole, dx)
+    del ws, x, dy, dx, whole, grads, staged, mean, var, scale, a, b
+    torch.cuda.empty_cache()
