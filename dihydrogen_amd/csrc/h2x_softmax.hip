@@ -1858,11 +1858,20 @@ bool inst_by_chunks(int n, size_t sample_size, int vec)
     return vec == 16 / sizeof(T) || (chunks > 4 && chunks * n <= 2 * chip_units());
 }
 
-// Whether the lanes of a wave or a workgroup hold a sample, each adding up its own elements.
+// Elements of a vector that the tensors of a call allow.
 template <typename T>
-bool inst_by_lanes(int n, size_t sample_size, int vec)
+int inst_vector(size_t sample_size, const void* a, const void* b, const void* out)
 {
-    return n > 0 && sample_size <= kInstSmallSample<T> && !inst_by_chunks<T>(n, sample_size, vec);
+    return vector_width<T>(sample_size, 16 / sizeof(T), {a, b ? b : a, out ? out : a});
+}
+
+// Whether the lanes of a wave or a workgroup hold a sample, each adding up its own elements.  (Asked before anything is cut: the host's part of a small
+// call is what it is bound by, and samples of one chunk go by lanes whatever the vectors are.)
+template <typename T>
+bool inst_by_lanes(int n, size_t sample_size, const void* a, const void* b, const void* out)
+{
+    return n > 0 && sample_size <= kInstSmallSample<T>
+           && (sample_size <= kInstSmallChunk<T> || !inst_by_chunks<T>(n, sample_size, inst_vector<T>(sample_size, a, b, out)));
 }
 
 template <typename T, int MODE>
@@ -1941,8 +1950,7 @@ InstChunking inst_chunking(size_t sample_size, int num_samples, int vec, size_t 
 template <typename T>
 InstChunking inst_plan(int n, size_t sample_size, const void* a, const void* b, const void* out, int* v)
 {
-    constexpr int kFull = 16 / sizeof(T);
-    *v = vector_width<T>(sample_size, kFull, {a, b ? b : a, out ? out : a});
+    *v = inst_vector<T>(sample_size, a, b, out);
     return inst_chunking(sample_size, n, *v, sizeof(T));
 }
 
@@ -2001,9 +2009,8 @@ template <typename T, int MODE>
 int inst_reduce(int n, size_t sample_size, const void* a, const void* b, void* out,
                 const void* param, void* result, void* workspace, hipStream_t st)
 {
-    int v;
-    inst_plan<T>(n, sample_size, a, b, out, &v);
-    if (inst_by_lanes<T>(n, sample_size, v) || (MODE == kInstMax && n > 0 && sample_size <= kInstSmallSample<T>)) // (a maximum in any order)
+    if ((MODE == kInstMax && n > 0 && sample_size <= kInstSmallSample<T>) // (a maximum in any order)
+        || inst_by_lanes<T>(n, sample_size, a, b, out))
     {
         constexpr int kSmallMode = MODE == kInstMax      ? kSmallMax
                                    : MODE == kInstExpSum ? kSmallExpSum
@@ -2011,14 +2018,15 @@ int inst_reduce(int n, size_t sample_size, const void* a, const void* b, void* o
                                                          : kSmallDot;
         return inst_small<T, kSmallMode>(n, sample_size, a, b, out, param, result, nullptr, T(0), st);
     }
+    int v;
+    const int groups = inst_plan<T>(n, sample_size, a, b, out, &v).groups;
     if constexpr (MODE == kInstExpSum || MODE == kInstDot) // (kInstSumExp is of whole passes of larger samples)
         if (inst_by_chunks<T>(n, sample_size, v))
             return inst_rounds<T, MODE == kInstDot ? kSmallDot : kSmallExpSum>(n, sample_size, a, b, out, param, result, nullptr, T(0), st);
     double* partials = static_cast<double*>(workspace);
     inst_partials<T, MODE>(n, sample_size, a, b, out, param, partials, st);
     launch(softmax_inst_finish_kernel<T, MODE == kInstMax>, n, kBlockSize, st, partials,
-           inst_plan<T>(n, sample_size, a, b, out, &v).groups, inst_groups_per_sample_max(n),
-           static_cast<T*>(result));
+           groups, inst_groups_per_sample_max(n), static_cast<T*>(result));
     return launch_status();
 }
 
@@ -2077,9 +2085,9 @@ bool inst_team(int n, size_t sample_size, const void* a, const void* b, const vo
     constexpr int most = FORWARD ? kInstMostForward : kInstMostBackward;
     if (n <= 0 || sample_size <= kInstSmallChunk<T>)
         return false;
-    const InstChunking ch = inst_plan<T>(n, sample_size, a, b, out, v);
-    if (inst_by_lanes<T>(n, sample_size, *v))
+    if (inst_by_lanes<T>(n, sample_size, a, b, out))
         return false;
+    const InstChunking ch = inst_plan<T>(n, sample_size, a, b, out, v);
     const int each = static_cast<int>(ch.chunk / kBlockSize / (16 / sizeof(T))); // vectors of 16 bytes
     const int chunks = ch.groups <= static_cast<int>(kInstMembers) ? 1 : 4;
     const int members = (ch.groups + chunks - 1) / chunks;
@@ -2145,11 +2153,11 @@ template <typename T>
 int inst_forward_local(int n, size_t sample_size, const void* x, void* y, void* sample_max,
                        void* sample_exp, void* workspace, hipStream_t st)
 {
-    int v;
-    const int sums = inst_plan<T>(n, sample_size, x, nullptr, y, &v).groups;
-    if (inst_by_lanes<T>(n, sample_size, v))
+    if (inst_by_lanes<T>(n, sample_size, x, nullptr, y))
         return inst_small<T, kSmallForward>(n, sample_size, x, nullptr, y, nullptr, sample_max,
                                             sample_exp, inst_min_output<T>(), st);
+    int v;
+    const int sums = inst_plan<T>(n, sample_size, x, nullptr, y, &v).groups;
     if (inst_by_chunks<T>(n, sample_size, v))
         return inst_rounds<T, kSmallForward>(n, sample_size, x, nullptr, y, nullptr, sample_max, sample_exp, inst_min_output<T>(), st);
     // `y` takes part in the choice of the vector width only, as in the staged call,
@@ -2178,11 +2186,11 @@ template <typename T>
 int inst_backward_local(int n, size_t sample_size, const void* y, const void* dy, void* dx, void* sample_dp,
                         void* workspace, hipStream_t st)
 {
-    int v;
-    const int sums = inst_plan<T>(n, sample_size, y, dy, nullptr, &v).groups;
-    if (inst_by_lanes<T>(n, sample_size, v))
+    if (inst_by_lanes<T>(n, sample_size, y, dy, nullptr))
         return inst_small<T, kSmallBackward>(n, sample_size, y, dy, dx, nullptr, sample_dp, nullptr,
                                              inst_min_output<T>(), st);
+    int v;
+    const int sums = inst_plan<T>(n, sample_size, y, dy, nullptr, &v).groups;
     const bool by_chunks = inst_by_chunks<T>(n, sample_size, v);
     if (by_chunks && vector_width<T>(sample_size, v, {dx}) == v) // dx takes no part in the cut
         return inst_rounds<T, kSmallBackward>(n, sample_size, y, dy, dx, nullptr, sample_dp, nullptr, inst_min_output<T>(), st);

@@ -75,7 +75,7 @@ class _Kept:
 
     def __init__(self):
         self.workspace = self.state = (-1, None)
-        self.scalars = (-1, None, None)
+        self.scalars = (-1, None, None, 0, 0)
 
 
 def _first_use(kept: dict, handle: int) -> _Kept:
@@ -515,10 +515,10 @@ class Softmax:
         return l
 
     def _buffers(self, l: Layout, t: Tensor, count: int, st: int):
-        """The workspace; `count` scalars of t's type that nobody reads after the call; and where the workgroups that
-        share a sample exchange its partial results (None where no workgroups do).  count = 0: the workspace alone.
-        (In one go, and by what stands beside each buffer: a call for each, and to ask the tensors, would be a tenth of a
-        small softmax.)"""
+        """The workspace; kept.scalars, whose last two are the addresses of `count` scalars of t's type that nobody reads after
+        the call (hold it until then); and where the workgroups that share a sample exchange its partial results (None where
+        no workgroups do).  count = 0: the workspace alone.  (In one go, and by what stands beside each buffer: a call for
+        each, and to ask the tensors, would be a tenth of a small softmax.)"""
         kept = self._kept.get(st) or _first_use(self._kept, st)
         held, ws = kept.workspace
         need = l.instance_workspace_bytes
@@ -527,10 +527,11 @@ class Softmax:
             kept.workspace = need, ws
         if count == 0:
             return ws, None, None
-        held, dtype, scalars = kept.scalars
-        if held < count or dtype is not t.dtype:
-            scalars = _buffer_of(self.stream, count, t.dtype)
-            kept.scalars = count, t.dtype, scalars
+        scalars = kept.scalars
+        if scalars[0] < count or scalars[1] is not t.dtype:
+            buffer = _buffer_of(self.stream, 2 * count, t.dtype)
+            address = buffer.data_ptr()
+            scalars = kept.scalars = count, t.dtype, buffer, address, address + count * t.dtype.itemsize
         need = l.instance_state_bytes
         if need == 0:
             return ws, scalars, None
@@ -556,11 +557,9 @@ class Softmax:
         calls, dt, size = self._calls, l.dtype, l.channels * l.spatial
         if self.allreduce is None:
             # every sample is whole on this rank: the stages need not be separate calls
-            ws, scalars, state = self._buffers(l, x, 2 * n, st)
-            scalars = scalars.data_ptr()
+            ws, scalars, state = self._buffers(l, x, n, st)
             status = calls.h2x_softmax_instance_forward_once(
-                dt, n, size, x, y, scalars,
-                scalars + n * x.dtype.itemsize, ws, state, -1, st)
+                dt, n, size, x, y, scalars[3], scalars[4], ws, state, -1, st)
             if status:
                 capi.check(status, "softmax instance forward")
             return 0
@@ -593,7 +592,7 @@ class Softmax:
         if self.allreduce is None:
             ws, scalars, state = self._buffers(l, y, n, st)
             status = calls.h2x_softmax_instance_backward_once(
-                dt, n, size, y, dy, dx, scalars, ws, state, -1, st)
+                dt, n, size, y, dy, dx, scalars[3], ws, state, -1, st)
             if status:
                 capi.check(status, "softmax instance backward")
             return 0

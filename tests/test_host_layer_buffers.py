@@ -211,3 +211,41 @@ def test_streams_share_no_buffer(use, made, monkeypatch):
     # of a layer with a stream of its own, whichever is current
     layer, step = use(_Stream())
     assert on(1) == on(2)
+
+
+def test_scalars_of_instance_softmax(made, monkeypatch):
+    """Where a layer tells the native calls to put a sample's maximum and sum: within its buffer and apart, also in a call with fewer samples; the
+    buffer is asked for its address when it is made."""
+    import torch
+    given, buffers, asked = [], [], []
+
+    class Buffer(torch.Tensor):
+        def data_ptr(self):
+            asked.append(self)
+            return super().data_ptr()
+
+    class Recording(_Calls):
+        def __getattr__(self, name):
+            return (lambda *args: given.append(args) or 0) if name.endswith("_once") else super().__getattr__(name)
+
+    def device_buffer(count, dtype, device="cuda", zero=False):
+        buffers.append(torch.zeros(count, dtype=dtype).as_subclass(Buffer))
+        return buffers[-1]
+
+    monkeypatch.setattr(layers, "_device_buffer", device_buffer)
+    monkeypatch.setattr(capi, "calls", Recording)
+    sm = Softmax()
+    dist = Distribution.make_localized_distribution(4)
+    for dtype, n in ((torch.float32, 4), (torch.float32, 4), (torch.float32, 3), (torch.float32, 7), (torch.float64, 7), (torch.float64, 2)):
+        x, y = (Tensor([1, 1, 10, n], LocaleVirtual(0, 1), dist, dtype, device="cpu").allocate() for _ in range(2))
+        sm.setup(x, SoftmaxMode.INSTANCE)
+        for backward in (False, True):
+            given.clear()
+            sm.backward(y, y, x) if backward else sm.forward(x, y)
+            (args,), scalars = given, buffers[-1]
+            first = torch.Tensor.data_ptr(scalars)
+            places = [a - first for a in args if type(a) is int and 0 <= a - first < scalars.nbytes]
+            assert scalars.dtype is dtype and len(places) == 2 - backward
+            assert all(0 <= at <= scalars.nbytes - n * dtype.itemsize for at in places)
+            assert backward or abs(places[1] - places[0]) >= n * dtype.itemsize
+    assert len(asked) == 3 == len([b for b in buffers if b.dtype is not torch.uint8])
