@@ -1089,8 +1089,9 @@ void launch_bwd(const T* y, const T* dy, T* dx, int n, int c, size_t s, bool str
         launch(softmax_bwd_reg_kernel<T, VEC, CMAX, false>, grid, kBlockSize, st, y, dy, dx, c, s, flat);
 }
 
-// More samples than this fill the chip with a wave each; and more than this leave its waves little to wait for where samples are short.
-constexpr int kManySamples = 2048, kSomeSamples = 768;
+// More samples than this fill the chip with a wave each; and more than kSomeSamples (channel softmax of floats, forward: kSomeRows) leave its waves
+// little to wait for where samples are short.
+constexpr int kManySamples = 2048, kSomeSamples = 768, kSomeRows = 512;
 
 // Which kernel serves which channel count (measured on MI355X).  Up to 32 channels a
 // thread keeps all channels of its pixels (softmax_*_reg_kernel: 21 channels of
@@ -1302,21 +1303,22 @@ int launch_shared_for(int n, int c, size_t s, hipStream_t st, P... p)
 // Calls f(elements a lane, lanes) with constants for samples of `size` contiguous elements that
 // lanes hold in registers: a wave while samples are short, or many (it needs no barrier), else
 // a workgroup, of 1024 threads with up to MAX_LARGE elements each where 256 would have more than 16.
-// A workgroup from 257 elements on, and from 513 also of more than kSomeSamples: a wave's chain of up to 32 loads, exponentials and stores is what
+// A workgroup from 257 elements on, and from 513 also of more than `some` samples: a wave's chain of up to 32 loads, exponentials and stores is what
 // else is waited for (sums of the data's type have fewer terms in a row so).  GPU time, a wave a sample -> a workgroup, forward / backward in us: channels, floats
 // N 16, 1000 3.1 / 2.4 -> 2.2 / 1.8, N 466, 1983 5.1 / 4.2 -> 3.3 / 2.9, N 1418, 1480 6.7 / 6.0 -> 5.6 / 5.4; doubles N 59, 1480 6.6 / 3.8 -> 3.3 / 2.3, N 700, 1000 5.7 /
-// 4.5 -> 4.3 / 3.8, N 1418, 704 6.4 / 5.6 -> 5.7 / 5.2; instances of doubles N 128, 1983 8.6 / 4.6 -> 4.0 / 2.7.  With more samples, floats, a wave
-// and a workgroup: channels N 700, 300 2.3 / 1.9 and 2.5 / 2.0, N 1000, 300 2.4 / 1.9 and 2.8 / 1.9, 500 2.6 / 2.2 and 2.9 / 2.0; instances N 700, 400 3.0 / 2.2 and 2.7 /
-// 2.1, N 850 3.1 / 2.2 and 3.0 / 2.2, N 1418 3.1 / 2.3 and 3.4 / 2.6; N 2600 the same either way.
+// 4.5 -> 4.3 / 3.8, N 1418, 704 6.4 / 5.6 -> 5.7 / 5.2; instances of doubles N 128, 1983 8.6 / 4.6 -> 4.0 / 2.7 (at the line, channels, floats N 2048, 600 4.0 / 3.3 -> 4.2 / 3.3, 1000 5.2 / 5.2 both ways).  Up to 512 elements, a wave
+// and a workgroup: channels, floats, 300 and 400 elements, N 466 2.3 / 1.9 and 2.3 / 1.8, N 512 2.3 / 2.0 and 2.3 / 1.9, N 600 2.4 / 2.0 and 2.4 / 1.9, N 700 2.3 / 1.9 and 2.4 /
+// 1.8, N 768 2.4 / 2.0 and 2.6 / 1.9, N 1000 2.4 / 1.9 and 2.8 / 1.9; doubles, 400, N 512 3.4 / 2.4 and 2.7 / 2.1, N 768 3.5 / 2.4 and 3.0 / 2.3; instances, floats, 400, N 700 3.0 / 2.2 and
+// 2.7 / 2.1, N 850 3.1 / 2.2 and 3.0 / 2.2, N 1418 3.1 / 2.3 and 3.4 / 2.6; N 2600 the same either way.
 template <int MAX_LARGE = 0, typename F>
-int with_lanes(int n, size_t size, const F& f)
+int with_lanes(int n, size_t size, int some, const F& f)
 {
 #define H2X_LANES(CPL, LANES)                                                                      \
     return f(std::integral_constant<int, CPL>(), std::integral_constant<int, LANES>())
     if (size <= 1 * kWaveSize) H2X_LANES(1, kWaveSize);
     if (size <= 2 * kWaveSize) H2X_LANES(2, kWaveSize);
     if (size <= 4 * kWaveSize) H2X_LANES(4, kWaveSize);
-    if (n > (size <= 2 * kBlockSize ? kSomeSamples : kManySamples))
+    if (n > (size <= 2 * kBlockSize ? some : kManySamples))
     {
         if (size <= 8 * kWaveSize) H2X_LANES(8, kWaveSize);
         if (size <= 16 * kWaveSize) H2X_LANES(16, kWaveSize);
@@ -1365,7 +1367,7 @@ int forward_impl(int n, int c, size_t s, const void* xv, void* yv, hipStream_t s
     T* y = static_cast<T*>(yv);
     constexpr int kWords = sizeof(T) / 4;
     if (s == 1 && c <= 32 * kBlockSize)
-        return with_lanes(n, c, [&](auto cpl, auto lanes) {
+        return with_lanes(n, c, kWords == 1 ? kSomeRows : kSomeSamples, [&](auto cpl, auto lanes) {
             constexpr int CPL = decltype(cpl)::value, LANES = decltype(lanes)::value;
             launch(softmax_fwd_row_kernel<T, CPL, LANES>, lanes_grid<LANES>(n), lanes_block<LANES>(), st, x, y, c, n);
             return launch_status();
@@ -1438,7 +1440,7 @@ int backward_impl(int n, int c, size_t s, const void* yv, const void* dyv, void*
     T* dx = static_cast<T*>(dxv);
     constexpr int kWords = sizeof(T) / 4;
     if (s == 1 && c <= 32 * kBlockSize)
-        return with_lanes(n, c, [&](auto cpl, auto lanes) {
+        return with_lanes(n, c, kSomeSamples, [&](auto cpl, auto lanes) {
             constexpr int CPL = decltype(cpl)::value, LANES = decltype(lanes)::value;
             launch(softmax_bwd_row_kernel<T, CPL, LANES>, lanes_grid<LANES>(n), lanes_block<LANES>(), st, y, dy,
                    dx, c, n);
@@ -1878,7 +1880,7 @@ template <typename T, int MODE>
 int inst_small(int n, size_t sample_size, const void* a, const void* b, void* out,
                const void* param, void* result, void* result2, T min_output, hipStream_t st)
 {
-    return with_lanes<kInstLargeLanes<T>>(n, sample_size, [&](auto cpl, auto lanes) {
+    return with_lanes<kInstLargeLanes<T>>(n, sample_size, kSomeSamples, [&](auto cpl, auto lanes) {
         constexpr int CPL = decltype(cpl)::value, LANES = decltype(lanes)::value;
         launch(softmax_inst_small_kernel<T, CPL, MODE, LANES>, lanes_grid<LANES>(n), lanes_block<LANES>(), st,
                static_cast<const T*>(a), static_cast<const T*>(b), static_cast<T*>(out),
