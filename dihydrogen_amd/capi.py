@@ -350,7 +350,7 @@ def calls():
             raise H2XError("_h2xcall.so is missing: build it with `make -C dihydrogen_amd/csrc` "
                            "(or __graft_entry__.build()); there is no fallback path") from e
         from .tensor import BASE_PTR_PARTS, Tensor
-        _h2xcall.pointer_types(torch.Tensor, Tensor, *BASE_PTR_PARTS)
+        _h2xcall.pointer_types(torch.Tensor, Tensor, *BASE_PTR_PARTS, torch.__version__, torch.empty(1, device="cpu"))
         _calls = _h2xcall
     return _calls
 

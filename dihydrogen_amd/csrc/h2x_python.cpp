@@ -29,6 +29,7 @@ namespace
 PyObject *s_data_ptr = nullptr, *s_get_base_ptr = nullptr, *s_data = nullptr, *s_base_bytes = nullptr; // interned names
 PyTypeObject *s_torch_tensor = nullptr, *s_local_tensor = nullptr;
 PyObject *s_base_ptr_method = nullptr, *s_base_bytes_property = nullptr; // of s_local_tensor
+bool s_torch_is_known = false; // torch tensors lie in memory as this file was compiled for
 unsigned int s_known_version = 0;
 
 bool as_address(PyObject* address, void** out)
@@ -51,7 +52,7 @@ bool address_by(PyObject* method, PyObject* o, void** out)
 // (One that has no memory to point to raises what the method raises.)
 bool data_ptr_of(PyObject* o, void** out)
 {
-    if (Py_TYPE(o) == s_torch_tensor)
+    if (s_torch_is_known && Py_TYPE(o) == s_torch_tensor)
     {
         try
         {
@@ -195,11 +196,29 @@ struct Entry<F>
     }
 };
 
-// pointer_types(torch.Tensor, the class of local tensors, its get_base_ptr, its base_bytes)
+// Whether torch is the one whose headers this file was compiled with, and has a torch tensor's address where they say.  (Another one's
+// tensors are asked by their method.)
+bool is_known_torch(PyObject* type, PyObject* version, PyObject* tensor)
+{
+    if (PyUnicode_CompareWithASCIIString(version, H2X_TORCH_VERSION) != 0 || reinterpret_cast<PyObject*>(Py_TYPE(tensor)) != type)
+        return false;
+    void* by_method;
+    if (!address_by(s_data_ptr, tensor, &by_method))
+    {
+        PyErr_Clear();
+        return false;
+    }
+    return THPVariable_Unpack(tensor).data_ptr() == by_method;
+}
+
+// pointer_types(torch.Tensor, the class of local tensors, its get_base_ptr, its base_bytes, torch.__version__, a torch tensor with
+// memory): whether torch tensors are asked for their addresses as C++ objects.
 PyObject* pointer_types(PyObject*, PyObject* const* args, Py_ssize_t nargs)
 {
-    if (nargs != 4 || !PyType_Check(args[0]) || !PyType_Check(args[1]))
-        return PyErr_Format(PyExc_TypeError, "two types, a function and a property");
+    if (nargs != 6 || !PyType_Check(args[0]) || !PyType_Check(args[1]) || !PyUnicode_Check(args[4]))
+        return PyErr_Format(PyExc_TypeError, "two types, a function, a property, a version and a tensor");
+    const bool known = is_known_torch(args[0], args[4], args[5]);
+    nargs = 4; // what is kept
     PyObject* const before[] = {reinterpret_cast<PyObject*>(s_torch_tensor), reinterpret_cast<PyObject*>(s_local_tensor),
                                 s_base_ptr_method, s_base_bytes_property};
     for (Py_ssize_t i = 0; i < nargs; ++i)
@@ -209,9 +228,10 @@ PyObject* pointer_types(PyObject*, PyObject* const* args, Py_ssize_t nargs)
     s_base_ptr_method = args[2];
     s_base_bytes_property = args[3];
     s_known_version = 0;
+    s_torch_is_known = known;
     for (PyObject* const o : before)
         Py_XDECREF(o);
-    Py_RETURN_NONE;
+    return PyBool_FromLong(known);
 }
 
 // same_buffers(addresses, *lists): whether the buffers of the lists of local tensors, one list after the other, lie at

@@ -59,3 +59,18 @@ def test_a_tensor_without_memory_raises_what_data_ptr_raises():
 
     torch.func.vmap(asked)(torch.zeros(2, 3))
     assert messages[0] == messages[1]
+
+
+def test_only_the_torch_that_the_module_was_compiled_for_is_read_directly():
+    """Another torch may have its tensors' addresses elsewhere: they are asked by their method."""
+    from dihydrogen_amd.tensor import BASE_PTR_PARTS, Tensor
+    t, (first, second) = _geometries()
+    told = lambda version, sample=t: capi.calls().pointer_types(torch.Tensor, Tensor, *BASE_PTR_PARTS, version, sample)
+    try:
+        for version in ("2.0.0", torch.__version__ + ".1", torch.__version__[:-1], ""):
+            assert told(version) is False
+            assert (_needed(t), _needed(t[ITEM:])) == (first, second)
+        assert told(torch.__version__, t.as_subclass(Shifted)) is False
+    finally:
+        assert told(torch.__version__) is True
+    assert (_needed(t), _needed(t[ITEM:])) == (first, second)
