@@ -5,7 +5,8 @@
 // spent more time on that than the GPU on the work.  Here each entry point is
 // one METH_FASTCALL function whose argument conversions are generated from its
 // C signature: integers and floats as they are, and for a pointer None, an
-// address, a torch tensor (what its data_ptr() returns, or raises), any other object with a get_base_ptr() method (a local tensor: the method is asked, also where
+// address, a torch tensor (what its data_ptr() returns, or raises; where that is torch's own method and no mode listens, it is not
+// called, see data_ptr_of), any other object with a get_base_ptr() method (a local tensor: the method is asked, also where
 // there is a data_ptr() too, or, where it is the one given to pointer_types(), what it does is
 // done here, 0.1 us less than in Python), or one with a data_ptr() method alone.  Every
 // function returns what the C function returns (a status or a size).  The GIL
@@ -13,6 +14,7 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstdint>
@@ -30,6 +32,7 @@ PyObject *s_data_ptr = nullptr, *s_get_base_ptr = nullptr, *s_data = nullptr, *s
 PyTypeObject *s_torch_tensor = nullptr, *s_local_tensor = nullptr;
 PyObject *s_base_ptr_method = nullptr, *s_base_bytes_property = nullptr; // of s_local_tensor
 bool s_torch_is_known = false; // torch tensors lie in memory as this file was compiled for
+unsigned int s_known_torch_version = 0; // tag of the class of torch tensors, when its data_ptr() was looked at
 unsigned int s_known_version = 0;
 
 bool as_address(PyObject* address, void** out)
@@ -47,12 +50,48 @@ bool address_by(PyObject* method, PyObject* o, void** out)
     return ok;
 }
 
-// What o.data_ptr() returns.  A torch tensor of that very class is asked as a C++ object: through its Python method, with an object made of
+// What holds for all pointers of a call, until Python code runs.
+struct Look
+{
+    bool is_new = true, plain = false;
+};
+
+// Whether the data_ptr() of torch tensors is the method that torch has in C++ (a class that nobody has changed since has its version tag
+// still), and no mode for torch's functions is on, which would be told of the call.
+bool calls_are_plain()
+{
+    PyTypeObject* const t = s_torch_tensor;
+    const bool valid = PyType_HasFeature(t, Py_TPFLAGS_VALID_VERSION_TAG);
+    if (!valid || t->tp_version_tag != s_known_torch_version)
+    {
+        PyObject* const method = _PyType_Lookup(t, s_data_ptr);
+        if (t->tp_getattro != PyObject_GenericGetAttr || !method || Py_TYPE(method) != &PyMethodDescr_Type)
+            return false;
+        if (PyType_HasFeature(t, Py_TPFLAGS_VALID_VERSION_TAG)) // (the look-up may have given it one)
+            s_known_torch_version = t->tp_version_tag;
+    }
+    return !at::impl::torch_function_mode_enabled();
+}
+
+// Whether what o.data_ptr() does is known: o is a torch tensor of that very class, and has no data_ptr() of its own.
+bool has_plain_data_ptr(PyObject* o, Look* look)
+{
+    if (!s_torch_is_known || Py_TYPE(o) != s_torch_tensor)
+        return false;
+    if (look->is_new)
+        *look = {false, calls_are_plain()};
+    if (!look->plain)
+        return false;
+    PyObject** const own = _PyObject_GetDictPtr(o);
+    return !own || !*own || !PyDict_GetItemWithError(*own, s_data_ptr);
+}
+
+// What o.data_ptr() returns.  A torch tensor is asked as a C++ object where it can be: through its Python method, with an object made of
 // the address and taken apart again, a pointer took 40 ns, of which a batch-norm backward pass has 14 and a shuffle between 16 ranks 32.
 // (One that has no memory to point to raises what the method raises.)
-bool data_ptr_of(PyObject* o, void** out)
+bool data_ptr_of(PyObject* o, void** out, Look* look)
 {
-    if (s_torch_is_known && Py_TYPE(o) == s_torch_tensor)
+    if (has_plain_data_ptr(o, look))
     {
         try
         {
@@ -63,6 +102,7 @@ bool data_ptr_of(PyObject* o, void** out)
         {
         }
     }
+    look->is_new = true;
     return address_by(s_data_ptr, o, out);
 }
 
@@ -86,7 +126,7 @@ bool class_is_known()
 
 // What the get_base_ptr() of a local tensor of that very class returns: data.data_ptr() + base_bytes, read from the object's
 // dictionary (three look-ups; by way of attributes 40 ns more).  0: not such a tensor, or not yet; -1: an exception is set.
-int base_of(PyObject* o, void** out)
+int base_of(PyObject* o, void** out, Look* look)
 {
     if (Py_TYPE(o) != s_local_tensor || !class_is_known())
         return 0;
@@ -100,7 +140,7 @@ int base_of(PyObject* o, void** out)
     if (offset == -1 && PyErr_Occurred())
         return -1;
     Py_INCREF(data);
-    const bool ok = data_ptr_of(data, out);
+    const bool ok = data_ptr_of(data, out, look);
     Py_DECREF(data);
     if (!ok)
         return -1;
@@ -108,12 +148,13 @@ int base_of(PyObject* o, void** out)
     return 1;
 }
 
-bool address_of(PyObject* o, void** out)
+bool address_of(PyObject* o, void** out, Look* look)
 {
-    if (const int known = base_of(o, out))
+    if (const int known = base_of(o, out, look))
         return known > 0;
     if (s_torch_tensor && PyObject_TypeCheck(o, s_torch_tensor))
-        return data_ptr_of(o, out);
+        return data_ptr_of(o, out, look);
+    look->is_new = true;
     PyObject* const method = PyObject_GetAttr(o, s_get_base_ptr);
     if (!method)
     {
@@ -130,7 +171,7 @@ bool address_of(PyObject* o, void** out)
 }
 
 template <typename P>
-bool convert(PyObject* o, P* out)
+bool convert(PyObject* o, P* out, Look* look)
 {
     if constexpr (std::is_pointer<P>::value)
     {
@@ -146,7 +187,7 @@ bool convert(PyObject* o, P* out)
             return p != nullptr || !PyErr_Occurred();
         }
         void* p;
-        if (!address_of(o, &p))
+        if (!address_of(o, &p, look))
             return false;
         *out = reinterpret_cast<P>(p);
         return true;
@@ -175,7 +216,8 @@ struct Entry<F>
     static PyObject* call(PyObject* const* args, std::index_sequence<I...>)
     {
         std::tuple<P...> v;
-        if (!(convert(args[I], &std::get<I>(v)) && ...))
+        Look look;
+        if (!(convert(args[I], &std::get<I>(v), &look) && ...))
             return nullptr;
         R result;
         Py_BEGIN_ALLOW_THREADS
@@ -227,7 +269,7 @@ PyObject* pointer_types(PyObject*, PyObject* const* args, Py_ssize_t nargs)
     s_local_tensor = reinterpret_cast<PyTypeObject*>(args[1]);
     s_base_ptr_method = args[2];
     s_base_bytes_property = args[3];
-    s_known_version = 0;
+    s_known_version = s_known_torch_version = 0;
     s_torch_is_known = known;
     for (PyObject* const o : before)
         Py_XDECREF(o);
@@ -242,6 +284,7 @@ PyObject* same_buffers(PyObject*, PyObject* const* args, Py_ssize_t nargs)
         return PyErr_Format(PyExc_TypeError, "a tuple of addresses");
     const Py_ssize_t n = PyTuple_GET_SIZE(args[0]);
     Py_ssize_t k = 0;
+    Look look;
     for (Py_ssize_t a = 1; a < nargs; ++a)
     {
         if (!PyList_Check(args[a]))
@@ -253,9 +296,10 @@ PyObject* same_buffers(PyObject*, PyObject* const* args, Py_ssize_t nargs)
             PyObject* const tensor = PyList_GET_ITEM(args[a], i);
             Py_INCREF(tensor); // code that runs for `data` may drop it from the list
             PyObject* const data = PyObject_GetAttr(tensor, s_data);
+            look.is_new |= Py_TYPE(tensor) != s_local_tensor || !class_is_known(); // of that class `data` runs no code
             Py_DECREF(tensor);
             void* p = nullptr;
-            const bool ok = data && (data == Py_None || data_ptr_of(data, &p));
+            const bool ok = data && (data == Py_None || data_ptr_of(data, &p, &look));
             Py_XDECREF(data);
             if (!ok)
                 return nullptr;

@@ -74,3 +74,50 @@ def test_only_the_torch_that_the_module_was_compiled_for_is_read_directly():
     finally:
         assert told(torch.__version__) is True
     assert (_needed(t), _needed(t[ITEM:])) == (first, second)
+
+
+def test_a_mode_is_told_of_the_call():
+    from torch.overrides import TorchFunctionMode
+    t, (first, second) = _geometries()
+
+    class Further(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {})) + (ITEM if func is torch.Tensor.data_ptr else 0)
+
+    with Further():
+        assert _needed(t) == second
+        with torch._C.DisableTorchFunction():
+            assert _needed(t) == first
+    assert _needed(t) == first
+
+
+def test_a_replaced_data_ptr_is_asked(monkeypatch):
+    t, (first, second) = _geometries()
+    own = torch.Tensor.data_ptr
+    for _ in range(2):
+        with monkeypatch.context() as m:
+            m.setattr(torch.Tensor, "data_ptr", lambda self: own(self) + ITEM)
+            assert _needed(t) == second
+        assert _needed(t) == first
+        with monkeypatch.context() as m:
+            m.setattr(torch.Tensor, "unrelated", 1, raising=False)
+            assert _needed(t) == first
+    t.unrelated = 1
+    assert _needed(t) == first
+    t.data_ptr = lambda: own(t) + ITEM
+    assert _needed(t) == second
+    del t.data_ptr
+    assert _needed(t) == first
+
+
+def test_a_replaced_data_ptr_of_local_tensors_data_is_asked(monkeypatch):
+    """Through a local tensor, whose get_base_ptr() the native module plays, and in the comparison of buffers."""
+    from dihydrogen_amd.tensor import Distribution, LocaleVirtual, Tensor
+    t, (first, second) = _geometries()
+    local = Tensor([t.numel()], LocaleVirtual(0, 1), Distribution.make_localized_distribution(1), torch.uint8, device="cpu")
+    local.data = t
+    local.base_bytes
+    own = torch.Tensor.data_ptr
+    assert _needed(local) == first and capi.calls().same_buffers((own(t),), [local])
+    monkeypatch.setattr(torch.Tensor, "data_ptr", lambda self: own(self) + ITEM)
+    assert _needed(local) == second and capi.calls().same_buffers((own(t) + ITEM,), [local])
