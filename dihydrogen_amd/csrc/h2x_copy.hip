@@ -81,6 +81,36 @@ Audit* current_audit()
     return t_audit;
 }
 
+void Audit::touch(const void* p, size_t bytes, size_t align, bool store, int times)
+{
+    const uint64_t at = reinterpret_cast<uintptr_t>(p);
+    if (at % align != 0)
+        misaligned += times;
+    if (thread != 0)
+        for (uint64_t w = at / 4; w < (at + bytes) / 4; ++w)
+        {
+            TouchedBy& by = words[w];
+            uint32_t &mine = store ? by.store : by.load, other = store ? by.load : by.store;
+            shared += mine != 0 || (other != 0 && other != thread);
+            mine = thread;
+        }
+    for (const AuditRegion& r : regions)
+    {
+        if (at >= r.base && at + bytes <= r.base + r.bytes)
+        {
+            uint8_t* const count = store ? r.stores : r.loads;
+            if (count)
+                for (size_t i = 0; i < bytes; ++i)
+                {
+                    uint8_t& c = count[at - r.base + i];
+                    c = static_cast<uint8_t>(std::min(c + times, 255));
+                }
+            return;
+        }
+    }
+    (store ? outside_stores : outside_loads) += bytes * times;
+}
+
 int launch_identity(const LaunchShape& s, const BoxBatch& batch)
 {
     switch (s.elem_size * 16 + s.vec)

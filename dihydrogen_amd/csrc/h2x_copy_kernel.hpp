@@ -19,6 +19,7 @@
 #include "h2x_device.hpp"
 
 #include <type_traits>
+#include <unordered_map>
 #include <vector>
 
 namespace h2x
@@ -175,8 +176,6 @@ __host__ __device__ __forceinline__ void box_offsets(const Box& box, uint32_t g,
 // its alignment.)
 struct DeviceMem
 {
-    // of cells that lie in so many strips
-    __device__ __forceinline__ const DeviceMem& of_strips(int) const { return *this; }
     template <int VEC, bool ALIGNED, typename T>
     __device__ __forceinline__ typename Words<T, VEC>::unaligned_t load(const T* p) const
     {
@@ -652,29 +651,28 @@ struct Audit
     uint64_t launches = 0, workgroups = 0;
     uint64_t outside_loads = 0, outside_stores = 0; // bytes outside every region
     uint64_t misaligned = 0;                        // accesses not aligned as their instruction needs
-
-    void touch(const void* p, size_t bytes, size_t align, bool store)
+    // Of a launch whose threads are followed (0: not): the one that is played, from 1, and the words that are loaded or stored more than once,
+    // or stored by one thread and touched by another.
+    uint32_t thread = 0;
+    uint64_t shared = 0;
+    struct TouchedBy
     {
-        const uint64_t at = reinterpret_cast<uintptr_t>(p);
-        if (at % align != 0)
-            ++misaligned;
-        for (const AuditRegion& r : regions)
-        {
-            if (at >= r.base && at + bytes <= r.base + r.bytes)
-            {
-                uint8_t* const count = store ? r.stores : r.loads;
-                if (count)
-                    for (size_t i = 0; i < bytes; ++i)
-                    {
-                        uint8_t& c = count[at - r.base + i];
-                        if (c < 255)
-                            ++c;
-                    }
-                return;
-            }
-        }
-        (store ? outside_stores : outside_loads) += bytes;
+        uint32_t load = 0, store = 0;
+    };
+    std::unordered_map<uint64_t, TouchedBy> words; // of four bytes
+
+    // Whether no word of the launch whose threads have been followed is shared; ends it.
+    bool followed()
+    {
+        const bool alone = shared == 0;
+        thread = 0;
+        shared = 0;
+        words.clear();
+        return alone;
     }
+
+    // times: what the access counts as.  (h2x_copy.hip: every kernel that is played has it.)
+    void touch(const void* p, size_t bytes, size_t align, bool store, int times = 1);
 };
 
 // The audit open on the calling thread, or null (h2x_copy.hip).
@@ -683,12 +681,10 @@ Audit* current_audit();
 struct TraceMem
 {
     Audit* audit;
-    int strips = 1; // a cell counts once for each strip that it is touched for
-    TraceMem of_strips(int n) const { return TraceMem{audit, n}; }
+    int times = 1; // what an access counts as
     void touch(const void* p, size_t bytes, size_t alignment, bool is_store) const
     {
-        for (int i = 0; i < strips; ++i)
-            audit->touch(p, bytes, alignment, is_store);
+        audit->touch(p, bytes, alignment, is_store, times);
     }
     template <int VEC, bool ALIGNED, typename T>
     typename Words<T, VEC>::unaligned_t load(const T* p) const

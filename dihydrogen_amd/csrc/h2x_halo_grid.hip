@@ -47,6 +47,17 @@ using copy::DeviceMem;
 using copy::TraceMem;
 using copy::Words;
 
+// A cell that a launch touches once for several strips: an audit, which expects a touch for each, counts so many (that it is one touch, and of
+// one thread, the audit sees by the threads, see issue_fold_grid).
+__device__ __forceinline__ const DeviceMem& of_strips(const DeviceMem& mem, int)
+{
+    return mem;
+}
+TraceMem of_strips(const TraceMem& mem, int strips)
+{
+    return TraceMem{mem.audit, strips};
+}
+
 constexpr int kMaxRanks = 16;
 constexpr int kMaxSpatial = 3;
 constexpr int kMaxRegions = 9 + 8;
@@ -468,21 +479,34 @@ __global__ __launch_bounds__(kBlock, 8) void halo_fold_ends_kernel(const FoldArg
     fold_ends_body<T, Op, BY, DeviceMem>(a, blockIdx.x, threadIdx.x, op, DeviceMem());
 }
 
+// A launch of a reverse exchange, played for an audit.  Its threads have no order: each cell is loaded once at most and stored once at most, and who
+// stores it is the only one to touch it, or the call fails.
+template <typename F>
+int play_fold(Audit* audit, uint32_t blocks, const F& body)
+{
+    const TraceMem mem{audit};
+    for (uint32_t block = 0; block < blocks; ++block)
+        for (uint32_t thread = 0; thread < kBlock; ++thread)
+        {
+            audit->thread = block * kBlock + thread + 1;
+            body(block, thread, mem);
+        }
+    ++audit->launches;
+    audit->workgroups += blocks;
+    return audit->followed() ? H2X_SUCCESS : H2X_ERR_INVALID_ARGUMENT;
+}
+
 template <typename T, typename Op, int BY>
 int issue_fold(const FoldArgs& a, uint32_t blocks, hipStream_t stream)
 {
     if (Audit* const audit = current_audit())
     {
-        const TraceMem mem{audit};
-        for (uint32_t block = 0; block < blocks; ++block)
-            for (uint32_t thread = 0; thread < kBlock; ++thread)
-                if constexpr (BY == kStrips)
-                    fold_body<T, Op, TraceMem>(a, block, thread, Op(), mem);
-                else
-                    fold_ends_body<T, Op, BY, TraceMem>(a, block, thread, Op(), mem);
-        ++audit->launches;
-        audit->workgroups += blocks;
-        return H2X_SUCCESS;
+        return play_fold(audit, blocks, [&](uint32_t block, uint32_t thread, const TraceMem& mem) {
+            if constexpr (BY == kStrips)
+                fold_body<T, Op, TraceMem>(a, block, thread, Op(), mem);
+            else
+                fold_ends_body<T, Op, BY, TraceMem>(a, block, thread, Op(), mem);
+        });
     }
     if constexpr (BY == kStrips)
         launch(halo_fold_kernel<T, Op>, dim3(blocks), kBlock, stream, a, Op());
@@ -615,7 +639,7 @@ __host__ __device__ __forceinline__ void fold_grid_body(const Args& a, uint32_t 
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 if (mine(i))
-                    v[i] = mem.of_strips(seams).template load<VEC, false>(at_cell[i]);
+                    v[i] = of_strips(mem, seams).template load<VEC, false>(at_cell[i]);
             fold_outer(dims, [&](int to, int from) {
 #pragma unroll
                 for (int j = 0; j < VEC; ++j)
@@ -624,7 +648,7 @@ __host__ __device__ __forceinline__ void fold_grid_body(const Args& a, uint32_t 
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 if (mine(i) && boundary(i, 0))
-                    mem.of_strips(boundary(i, 0)).template store<VEC, false>(at_cell[i], v[i]);
+                    of_strips(mem, boundary(i, 0)).template store<VEC, false>(at_cell[i], v[i]);
             return;
         }
         for (uint32_t j = 0; j < n; ++j)
@@ -633,12 +657,12 @@ __host__ __device__ __forceinline__ void fold_grid_body(const Args& a, uint32_t 
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 if (mine(i))
-                    v[i] = mem.of_strips(seams).load1(at_cell[i] + j);
+                    v[i] = of_strips(mem, seams).load1(at_cell[i] + j);
             fold_outer(dims, [&](int to, int from) { v[to] = op(v[to], v[from]); });
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 if (mine(i) && boundary(i, 0))
-                    mem.of_strips(boundary(i, 0)).store1(at_cell[i] + j, v[i]);
+                    of_strips(mem, boundary(i, 0)).store1(at_cell[i] + j, v[i]);
         }
         return;
     }
@@ -664,8 +688,8 @@ __host__ __device__ __forceinline__ void fold_grid_body(const Args& a, uint32_t 
             if (mine(i))
             {
                 end_of(k, i, &inner_at[i], &halo_at[i]);
-                inner[i] = mem.of_strips(seams).load1(inner_at[i]);
-                halo[i] = mem.of_strips(seams).load1(halo_at[i]);
+                inner[i] = of_strips(mem, seams).load1(inner_at[i]);
+                halo[i] = of_strips(mem, seams).load1(halo_at[i]);
             }
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -679,9 +703,9 @@ __host__ __device__ __forceinline__ void fold_grid_body(const Args& a, uint32_t 
         for (int i = 0; i < 4; ++i)
             if (mine(i))
             {
-                mem.of_strips(boundary(i, 1)).store1(inner_at[i], inner[i]);
+                of_strips(mem, boundary(i, 1)).store1(inner_at[i], inner[i]);
                 if (boundary(i, 0))
-                    mem.of_strips(boundary(i, 0)).store1(halo_at[i], halo[i]);
+                    of_strips(mem, boundary(i, 0)).store1(halo_at[i], halo[i]);
             }
     }
 }
@@ -697,13 +721,9 @@ int issue_fold_grid(const Args& a, uint32_t blocks, hipStream_t stream)
 {
     if (Audit* const audit = current_audit())
     {
-        const TraceMem mem{audit};
-        for (uint32_t block = 0; block < blocks; ++block)
-            for (uint32_t thread = 0; thread < kBlock; ++thread)
-                fold_grid_body<T, Op, TraceMem>(a, block, thread, Op(), mem);
-        ++audit->launches;
-        audit->workgroups += blocks;
-        return H2X_SUCCESS;
+        return play_fold(audit, blocks, [&](uint32_t block, uint32_t thread, const TraceMem& mem) {
+            fold_grid_body<T, Op, TraceMem>(a, block, thread, Op(), mem);
+        });
     }
     launch(halo_fold_grid_kernel<T, Op>, dim3(blocks), kBlock, stream, a, Op());
     return launch_status();

@@ -804,7 +804,10 @@ int h2x_bn_planned(int backward,
  * often byte base + i would be loaded / stored (saturating at 255; either may
  * be null).  What falls outside every range is counted in the report
  * (`outside_loads`, `outside_stores`, in bytes: must be 0), as are accesses not
- * aligned as their instruction needs (`misaligned`: must be 0).  A shuffle plan
+ * aligned as their instruction needs (`misaligned`: must be 0).  A reverse
+ * exchange of a whole grid counts a cell for each strip that it lies in, as the
+ * phases touch it, and returns H2X_ERR_INVALID_ARGUMENT if a played launch loads or
+ * stores a cell twice, or touches in one thread what another stores.  A shuffle plan
  * made while an audit is open serves audited launches only; destroy it as any
  * other.  Cost: proportional to the elements moved; meant for tests on machines
  * without a GPU.  The stream argument of the audited calls is ignored.

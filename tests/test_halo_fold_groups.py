@@ -1,5 +1,6 @@
-"""Reverse exchanges of several dimensions in one launch: what is read and written (on the CPU, through the launch audit),
-and the tensors against the packed exchange, dimension by dimension, bit for bit."""
+"""Reverse exchanges of several dimensions in one launch: what is read and written (on the CPU, through the launch audit, which counts a
+cell for each of its strips and fails a call in which two threads meet at a cell that one of them stores), and the tensors against the packed
+exchange, dimension by dimension, bit for bit."""
 import pytest
 
 import test_gpu_direct as direct
