@@ -550,8 +550,8 @@ struct FusedStats
     bool sequential;    // the partials come from a short-segment kernel and are added one after the other
 };
 
-// How a normalising kernel works: with statistics that it reads, past the caches; with those that it makes of partial sums; as the first,
-// with normal stores (see kNormalStores).
+// How a normalising kernel works: with statistics that it reads, past the caches; with those that it makes of partial
+// sums; as the first, with normal stores (see kNormalStores).
 enum ApplyMode : int
 {
     kPlainApply = 0,
@@ -1009,13 +1009,15 @@ __device__ __forceinline__ void sequential_totals(const double* __restrict__ par
     }
 }
 
-// The K sums of the channels of a workgroup's window, added as sequential_totals does, a sum by a thread: totals[k][q] of channel q, and the
-// outputs where the workgroup is the window's first.  Ends with a barrier.  The passes that finish a reduction so are bound by what they wait
-// for before their first store: their first batch of elements is loaded ahead of the sums.  One lane a channel adding all K sums, elements loaded behind them -> this, doubles,
-// forward, backward in us of the two launches, going round three sets of tensors: N 135, C 455, 5 x 7 14.9, 26.3 -> 13.4, 21.4; N 228, C 69, 10 x 9
-// 12.6, 20.7 -> 12.1, 17.5; N 173, C 143, 13 x 10 19.2, 35.4 -> 18.1, 28.2; N 200, C 600, 7 x 7 27.4, 53.6 -> 26.4, 41.9; N 40, C 2000,
-// 14 x 14 with a halo 97, 136 -> 94, 134.  (The elements alone ahead: backward 26.3, 20.1, 35.9, 55.3.  Batches of four samples backward 21.2,
-// 17.1, 29.3, 42.3, and 59 against 58 for N 243, C 306, 4 x 6 x 5; of all four sums in a lane 98 registers instead of 80.)
+// The K sums of the channels of a workgroup's window, added as sequential_totals does, a sum by a thread: totals[k][q]
+// of channel q, and the outputs where the workgroup is the window's first. Ends with a barrier. The passes that finish
+// a reduction so are bound by what they wait for before their first store: their first batch of elements is loaded
+// ahead of the sums. One lane a channel adding all K sums, elements loaded behind them -> this, doubles, forward,
+// backward in us of the two launches, going round three sets of tensors: N 135, C 455, 5 x 7 14.9, 26.3 -> 13.4, 21.4;
+// N 228, C 69, 10 x 9 12.6, 20.7 -> 12.1, 17.5; N 173, C 143, 13 x 10 19.2, 35.4 -> 18.1, 28.2; N 200, C 600, 7 x 7
+// 27.4, 53.6 -> 26.4, 41.9; N 40, C 2000, 14 x 14 with a halo 97, 136 -> 94, 134. (The elements alone ahead: backward
+// 26.3, 20.1, 35.9, 55.3. Batches of four samples backward 21.2, 17.1, 29.3, 42.3, and 59 against 58 for N 243, C 306,
+// 4 x 6 x 5; of all four sums in a lane 98 registers instead of 80.)
 template <typename T, int K>
 __device__ __forceinline__ void window_totals(const FusedStats<T>& f, const ShortGeometry& g, T (&totals)[K][kBlockSize], bool store)
 {
@@ -2049,20 +2051,26 @@ Chunking elementwise_chunking(size_t spatial, size_t segments, int vw, int unrol
     return c;
 }
 
-// Haloed outputs that lie within this many bytes are stored normally by a pass that reads its statistics, inference or the staged one: the ends of
-// their rows are partial lines, which the caches merge with the neighbours'; larger ones push the inputs out of the memory-side cache.  Inference, past
-// the caches and normally, us going round three sets of tensors: N 106, C 257, 13 x 12, halo of 2, 28 MiB 14.1 and 10.4; N 27, C
-// 57, 14 x 11 x 10, halo of 2, 22 MiB 9.1 and 7.1; doubles N 125, C 346, 7 x 8, 30 MiB 14.9 and 11.3; below 5 MiB level; larger N 5, C 7,
-// 63 x 67 x 61, 38 MiB 14.0 and 13.2, N 152, C 5, 29 x 21 x 21, 47 MiB 19.4 and 20.4, N 25, C 245, 41 x 60, 62 MiB 23.8 and 33.1.  The line
-// lies below where inference alone would have it for the training that runs in stages, and reads x again: forward + backward there 5 % less with 29 to 32 MiB.
-// (With normal stores of dx, and of passes that finish their sums, training in stages loses up to 10 %: N 8, C 60, 129 x 142, 35 MiB 60.7 and 66.1.)
+// Haloed outputs that lie within this many bytes are stored normally by a pass that reads its statistics, inference or
+// the staged one: the ends of their rows are partial lines, which the caches merge with the neighbours'; larger ones
+// push the inputs out of the memory-side cache. Inference, past the caches and normally, us going round three sets of
+// tensors: N 106, C 257, 13 x 12, halo of 2, 28 MiB 14.1 and 10.4; N 27, C 57, 14 x 11 x 10, halo of 2, 22 MiB 9.1 and
+// 7.1; doubles N 125, C 346, 7 x 8, 30 MiB 14.9 and 11.3; below 5 MiB level; larger N 5, C 7, 63 x 67 x 61, 38 MiB 14.0
+// and 13.2, N 152, C 5, 29 x 21 x 21, 47 MiB 19.4 and 20.4, N 25, C 245, 41 x 60, 62 MiB 23.8 and 33.1. The line lies
+// below where inference alone would have it for the training that runs in stages, and reads x again: forward + backward
+// there 5 % less with 29 to 32 MiB.
+// (With normal stores of dx, and of passes that finish their sums, training in stages loses up to 10 %: N 8, C 60, 129
+// x 142, 35 MiB 60.7 and 66.1.)
 constexpr size_t kNormalStores = size_t(32) << 20;
 
-// Of tensors with one plane a channel and segments beyond the short ones, whose partial lines are few or many to a workgroup, these lose (inference, us,
-// past the caches and normally, of 190 calls): from 5 to 10 MiB, where three sets of inputs stay in the L2 if nothing else goes there, N 15, C 16, 65 x 99, halo
-// of 2 4.78 and 5.13, doubles N 3, C 11, 183 x 151, halo of 2 4.53 and 5.00 (below 5 MiB 0.98 of the time on average); and segments of up to 700 floats or 470
-// doubles, N 68, C 61, 17 x 27, halo of 2, 10 MiB 6.86 and 7.58, N 36, C 310, 19 x 23, 22 MiB 12.5 and 13.4, doubles N 13, C 195, 20 x 23, halo of 2 6.23 and
-// 6.68.  The others from 10 MiB N 29, C 15, 94 x 75 7.15 and 6.77, N 62, C 35, 38 x 37, halo of 3 8.50 and 7.50, doubles N 58, C 88, 23 x 30 13.4 and 12.2; several planes of any size 0.78 to 1.04 of the time, 0.92 on average.
+// Of tensors with one plane a channel and segments beyond the short ones, whose partial lines are few or many to a
+// workgroup, these lose (inference, us, past the caches and normally, of 190 calls): from 5 to 10 MiB, where three sets
+// of inputs stay in the L2 if nothing else goes there, N 15, C 16, 65 x 99, halo of 2 4.78 and 5.13, doubles N 3, C 11,
+// 183 x 151, halo of 2 4.53 and 5.00 (below 5 MiB 0.98 of the time on average); and segments of up to 700 floats or 470
+// doubles, N 68, C 61, 17 x 27, halo of 2, 10 MiB 6.86 and 7.58, N 36, C 310, 19 x 23, 22 MiB 12.5 and 13.4, doubles N
+// 13, C 195, 20 x 23, halo of 2 6.23 and 6.68. The others from 10 MiB N 29, C 15, 94 x 75 7.15 and 6.77, N 62, C 35, 38
+// x 37, halo of 3 8.50 and 7.50, doubles N 58, C 88, 23 x 30 13.4 and 12.2; several planes of any size 0.78 to 1.04 of
+// the time, 0.92 on average.
 constexpr size_t kPlaneInL2 = size_t(5) << 20, kPlaneBeyondL2 = size_t(10) << 20, kPlaneFloats = 700, kPlaneDoubles = 470;
 
 bool stored_normally(const HostTensor& output, int num_samples, int num_channels, size_t spatial, size_t elem_bytes, bool is_short)
@@ -2790,9 +2798,10 @@ void issue_once(const G& g, const OnceBackward<float>& a, hipStream_t st)
     // 144 of the 160 KB.  With 16 vectors a thread and nine of dy parked there the kernel has registers for the rest only if
     // it works the places of the vectors out again in each step (kept, 16 registers and a 16-byte spill that waits for the first
     // load: backward, N 40, C 128, 38 x 38 22.3 -> 20.9 us, N 1, C 361, 35 x 46 x 38 69 -> 61, N 2, C 512, 30^3 with a halo 100
-    // -> 90).  Where the halo is cleared a place is long to work out (N 32, C 116, 13 x 9 x 9 25.2 -> 31.6): it is kept, 16 registers are
-    // spilled (9 words of scratch a lane), and the kernel remains faster than two launches: N 4, C 256, 112 x 112 47.5 ->
-    // 38.7, N 2, C 512, 30^3 97 -> 90, N 16, C 1024, 54 x 54 154 -> 142 (going round three sets of tensors).
+    // -> 90). Where the halo is cleared a place is long to work out (N 32, C 116, 13 x 9 x 9 25.2 -> 31.6): it is kept,
+    // 16 registers are spilled (9 words of scratch a lane), and the kernel remains faster than two launches: N 4, C
+    // 256, 112 x 112 47.5 -> 38.7, N 2, C 512, 30^3 97 -> 90, N 16, C 1024, 54 x 54 154 -> 142 (going round three sets
+    // of tensors).
     constexpr int kInLds = TEAM * K > 8192 ? 9 : 0;
     launch_whole(kKernelOnce, K, bn_once_backward_kernel<float, TEAM, K, STREAM, kInLds, G>, once_grid<TEAM>(g), once_block<TEAM>(),
                  st, g, a);
@@ -2925,13 +2934,13 @@ bool once_launch(const OnceGeometry& g, const A& a, int n, hipStream_t st)
 // ---- whole channels in several workgroups: which calls, which team ---------------
 // Whether a backward pass reads dy, for the last time, past the caches, so that x, which the forward pass has left in
 // the memory-side cache, stays there.  In dense tensors, and whole allocations where the halo is cleared, of `vectors` of 16
-// bytes a channel: from 48 MiB.  Smaller ones the cache holds all together.  Backward in us, dy by the caches, past them (going round three sets of tensors): N 4,
-// C 40, 40^3, 41 MB, 26.0, 27.5; N 96, C 60, 38 x 38, 33 MB, 23.6, 27.2; N 134, C 60, 38 x 38, 46 MB, 29.6, 29.7; N 64, C 64,
-// 56 x 56, 51 MB, 34.0, 32.9; N 32, C 256, 56 x 56, 103 MB, 68, 63; doubles, N 4, C 32, 33^3, 37 MB, 28.9, 31.5; N 32, C 64,
-// 56 x 56, 51 MB, 32.8, 31.7; N 8, C 32, 33^3, 74 MB, 58, 53.  Forward + backward N 4, C 64, 64^3 269, 257, with x past
-// the caches too 10 more.  Cleared: of 28 to 44 MB 4 % more past the caches, of 60 to 95 MB 6 % less (235 calls).  Rows with a
-// halo between them at all sizes: below 28 MB equal, beyond 2 to 8 % less (664 calls; N 4, C 64, 30^3, halo of 1, forward +
-// backward 45, 39).
+// bytes a channel: from 48 MiB. Smaller ones the cache holds all together. Backward in us, dy by the caches, past them
+// (going round three sets of tensors): N 4, C 40, 40^3, 41 MB, 26.0, 27.5; N 96, C 60, 38 x 38, 33 MB, 23.6, 27.2; N
+// 134, C 60, 38 x 38, 46 MB, 29.6, 29.7; N 64, C 64, 56 x 56, 51 MB, 34.0, 32.9; N 32, C 256, 56 x 56, 103 MB, 68, 63;
+// doubles, N 4, C 32, 33^3, 37 MB, 28.9, 31.5; N 32, C 64, 56 x 56, 51 MB, 32.8, 31.7; N 8, C 32, 33^3, 74 MB, 58, 53.
+// Forward + backward N 4, C 64, 64^3 269, 257, with x past the caches too 10 more. Cleared: of 28 to 44 MB 4 % more
+// past the caches, of 60 to 95 MB 6 % less (235 calls). Rows with a halo between them at all sizes: below 28 MB equal,
+// beyond 2 to 8 % less (664 calls; N 4, C 64, 30^3, halo of 1, forward + backward 45, 39).
 constexpr size_t kStreamedGradient = size_t(48) << 20;
 
 bool streams_gradient(size_t vectors, uint32_t num_channels)
@@ -3100,11 +3109,12 @@ PassShape pass_shape(const ClearGeometry& g, bool)
 
 // Backward, teams of 65 to 128 members of 128 KB only in tensors that the memory-side cache nearly holds.  Dense ones below
 // 240 MiB: 7 % less than two launches on average (N 16, C 10, 64^3, 168 MB, 117 us and 131; N 2, C 6, 110 x 120 x 130 55 and
-// 69; N 8, C 13, 73 x 85 x 84, 217 MB, 162 and 170; 17 % more at worst; N 16, C 16, 64^3, 268 MB, 231 and 202).  With a halo below
-// 104 MiB, where x, dy and dx take half of it: 7 % less (N 100, C 8, 200 x 160, 102 MB, 87 and 101), beyond 9 % more (N 158, C
-// 13, 25 x 23 x 21 128 and 112; N 14, C 11, 65 x 66 x 48, halo of 2, 150 and 133) unless rows are long, which leaves few partial
-// lines: from 80 elements 1 % less, up to 10 (N 4, C 8, 96^3, forward + backward 154 and 171; N 118, C 15, 124 x 152, halo of 2,
-// 183 and 195).  Where the halo is cleared never (4 % more; N 50, C 16, 33 x 36 x 45 with a halo of 2 206 and 171).
+// 69; N 8, C 13, 73 x 85 x 84, 217 MB, 162 and 170; 17 % more at worst; N 16, C 16, 64^3, 268 MB, 231 and 202). With a
+// halo below 104 MiB, where x, dy and dx take half of it: 7 % less (N 100, C 8, 200 x 160, 102 MB, 87 and 101), beyond
+// 9 % more (N 158, C 13, 25 x 23 x 21 128 and 112; N 14, C 11, 65 x 66 x 48, halo of 2, 150 and 133) unless rows are
+// long, which leaves few partial lines: from 80 elements 1 % less, up to 10 (N 4, C 8, 96^3, forward + backward 154 and
+// 171; N 118, C 15, 124 x 152, halo of 2, 183 and 195). Where the halo is cleared never (4 % more; N 50, C 16, 33 x 36
+// x 45 with a halo of 2 206 and 171).
 constexpr size_t kHeldTensor = size_t(240) << 20, kHeldRows = size_t(104) << 20;
 constexpr uint32_t kLongRow = 80;
 
@@ -3450,9 +3460,10 @@ bool short_once_geometry(int num_samples, int num_channels, size_t spatial, std:
 }
 
 // Fewer windows than this that play ranges one after another (g.passes) leave the chip idle longer than a second launch takes:
-// forward, or backward, N 255, C 34, 4 x 7 x 4 5.8 us more than in two launches, N 231, C 20, 6 x 7 3.9, N 85, C 22, 4 x 7 x 5 level.
-// So do the largest workgroups with many samples, whose rows one thread adds up: forward in us, in two launches and so, N 112, C 10, 5 x 4 x 6 8.3 and 10.2, N 145,
-// C 13, 7 x 8 8.2 and 9.5, N 83, C 27, 10 x 11 with a halo 8.9 and 10.0; N 56, C 21, 5 x 6 x 5 with a halo 9.0 and 8.5, N 34, C 12, 17 x 15 with a halo 8.4 and 8.2.
+// forward, or backward, N 255, C 34, 4 x 7 x 4 5.8 us more than in two launches, N 231, C 20, 6 x 7 3.9, N 85, C 22, 4
+// x 7 x 5 level. So do the largest workgroups with many samples, whose rows one thread adds up: forward in us, in two
+// launches and so, N 112, C 10, 5 x 4 x 6 8.3 and 10.2, N 145, C 13, 7 x 8 8.2 and 9.5, N 83, C 27, 10 x 11 with a halo
+// 8.9 and 10.0; N 56, C 21, 5 x 6 x 5 with a halo 9.0 and 8.5, N 34, C 12, 17 x 15 with a halo 8.4 and 8.2.
 constexpr uint32_t kShortWindows = 64, kShortManySamples = 64;
 
 template <int VEC, int TEAM, int K, typename G>
@@ -3483,18 +3494,20 @@ uint32_t short_once_windows(ShortOnceGeometry* g, uint32_t threads, uint32_t vec
     return (g->num_channels + channels - 1) / channels;
 }
 
-// Outputs whose halo is cleared, larger than this, are left to the staged calls, which store whole lines past the caches, unless a few long
-// segments, or one workgroup a channel with little halo, leave few parts of lines to store.  Forward + backward in us, staged and by
-// these: N 8, C 64, 30^3, 128 MiB 168 and 199; N 63, C 65, 29 x 39, 40 MiB 67.0 and 72.1; N 48, C 242, 9 x 8 x 7, 88 MiB 120 and 136;
-// rows of 80 elements and more: N 1, C 744, 149 x 140, 122 MiB 168 and 140; N 12, C 61, 85 x 84, 42 MiB 69 and 56; one workgroup: N 4, C 1963, 63 x 52,
-// halo of 2, 225 MiB 298 and 258; N 3, C 1290, 35 x 48, halo of 2, 60 MiB 88 and 69; smaller: N 12, C 77, 11 x 15 x 15, halo of 2, 38 MiB 58 and 42; N 5,
-// C 16, 38 x 65 30.4 and 13.7.
+// Outputs whose halo is cleared, larger than this, are left to the staged calls, which store whole lines past the
+// caches, unless a few long segments, or one workgroup a channel with little halo, leave few parts of lines to store.
+// Forward + backward in us, staged and by these: N 8, C 64, 30^3, 128 MiB 168 and 199; N 63, C 65, 29 x 39, 40 MiB 67.0
+// and 72.1; N 48, C 242, 9 x 8 x 7, 88 MiB 120 and 136; rows of 80 elements and more: N 1, C 744, 149 x 140, 122 MiB
+// 168 and 140; N 12, C 61, 85 x 84, 42 MiB 69 and 56; one workgroup: N 4, C 1963, 63 x 52, halo of 2, 225 MiB 298 and
+// 258; N 3, C 1290, 35 x 48, halo of 2, 60 MiB 88 and 69; smaller: N 12, C 77, 11 x 15 x 15, halo of 2, 38 MiB 58 and
+// 42; N 5, C 16, 38 x 65 30.4 and 13.7.
 constexpr size_t kClearedByOrder = size_t(39) << 20;
 
-// Whether short segments whose output's halo is cleared are for `windows` workgroups that hold so many vectors.  The staged calls take a
-// time for each segment, and those of up to 200 cells, allocated, are always for one launch (N 193, C 941, 4 x 5 301 and 100 us, N 176, C 910, 3 x 2
-// 255 and 38); beyond they run at memory's rate, and a workgroup with all of a channel's cells to itself needs neighbours that
-// keep memory busy.  Forward + backward in us, staged and in one launch each way, of 220 calls:
+// Whether short segments whose output's halo is cleared are for `windows` workgroups that hold so many vectors. The
+// staged calls take a time for each segment, and those of up to 200 cells, allocated, are always for one launch (N 193,
+// C 941, 4 x 5 301 and 100 us, N 176, C 910, 3 x 2 255 and 38); beyond they run at memory's rate, and a workgroup with
+// all of a channel's cells to itself needs neighbours that keep memory busy. Forward + backward in us, staged and in
+// one launch each way, of 220 calls:
 //   few workgroups of much: N 106, C 26, 4^3, halo of 3 36 and 62; N 119, C 88, 4 x 5 x 6, halo of 2 65 and 89; N 92, C 71, 4^3, halo of 2 38 and 41; more
 //   of them N 43, C 107, 5 x 5 x 4, halo of 3 62 and 52; of little N 29, C 72, 7 x 6 x 6, halo of 2 41 and 34;
 //   the largest, one a CU, in more than one round: N 57, C 454, 18 x 9, halo of 3 95 and 115; N 36, C 359, 16 x 13, halo of 3 65 and 75; in one
@@ -3533,17 +3546,18 @@ bool short_once(G g, const A& a, hipStream_t st)
     const bool idles = g.passes > 1 || (TEAM * K >= 1024 * 8 && g.num_samples > kShortManySamples);
     if (windows == 0 || (idles && windows < kShortWindows) || !clearing_pays(g, windows, TEAM * K))
         return false;
-    // The largest workgroups have to have more than ten of sixteen lanes play something (forward in us, by them less in two launches: 1024 threads
-    // N 29, C 911, 12 x 20, nine, +5.0, N 38, C 489, 14 x 11 with a halo, 10.5, -4.6; 512 threads N 71, C 291, 8 x 10, ten, +3.6, N 129, C
-    // 319, 8 x 5 with a halo, 12, -3.3); those of 16 vectors in one pass (N 70, C 135, 12 x 11, three, +1.1), and in more than a round of
-    // the chip nearly all of them (N 83, C 1398, 12 x 8 with a halo, 12, +9, N 46, C 832, 16 x 12, 15, -3.4).
+    // The largest workgroups have to have more than ten of sixteen lanes play something (forward in us, by them less in
+    // two launches: 1024 threads N 29, C 911, 12 x 20, nine, +5.0, N 38, C 489, 14 x 11 with a halo, 10.5, -4.6; 512
+    // threads N 71, C 291, 8 x 10, ten, +3.6, N 129, C 319, 8 x 5 with a halo, 12, -3.3); those of 16 vectors in one
+    // pass (N 70, C 135, 12 x 11, three, +1.1), and in more than a round of the chip nearly all of them (N 83, C 1398,
+    // 12 x 8 with a halo, 12, +9, N 46, C 832, 16 x 12, 15, -3.4).
     const uint32_t playing = g.channels.divisor * g.slots.divisor * g.rows.divisor * g.together;
     if (TEAM * K >= 1024 * 8 && playing * 16 <= TEAM * 10)
         return false;
     if (TEAM * K >= 1024 * 8 && K == 16 && (g.passes > 1 || (windows > 2 * chip_units() && playing * 16 < TEAM * 14)))
         return false;
-    // (the smallest workgroup of so many vectors, backward: N 71, C 291, 8 x 10 3.4 us more than in two launches, N 109, C 1893, 5 x 6, 947 of
-    // them, 18.2 less)
+    // (the smallest workgroup of so many vectors, backward: N 71, C 291, 8 x 10 3.4 us more than in two launches, N
+    // 109, C 1893, 5 x 6, 947 of them, 18.2 less)
     if (TEAM == 256 && K == 16 && windows <= 2 * chip_units())
         return false;
     const uint32_t blocks = (windows + kNumXcd - 1) / kNumXcd * kNumXcd;
@@ -3613,7 +3627,8 @@ bool ordered_launch(int n, int c, size_t s, std::initializer_list<const HostTens
     }
     OrderedClearing g;
     bool rows, team;
-    // (a halo on the outermost spatial dimension alone leaves dense segments, which the kernels that clear are not built for: staged)
+    // (a halo on the outermost spatial dimension alone leaves dense segments, which the kernels that clear are not
+    // built for: staged)
     if (!ordered_geometry(n, c, s, ts, output, &g, &rows) || (halo && !rows))
         return false;
     const size_t bytes = (static_cast<size_t>(c - 1) * output.map.stride_c + static_cast<size_t>(n - 1) * output.map.stride_n
@@ -3628,7 +3643,8 @@ bool ordered_launch(int n, int c, size_t s, std::initializer_list<const HostTens
     const size_t moved = moved_bytes(output, n, c, s);
     uint32_t most = teams ? most_members() : 0;
     const size_t allocated = static_cast<size_t>(n) * output.map.stride_n * sizeof(double), inside = size_t(n) * c * s * sizeof(double);
-    // (units that segments fill a quarter of, in more than a round of workgroups: N 11, C 333, 8 x 6 x 7 40.0 and 42.6 us, C 165 32.9 and 24.1)
+    // (units that segments fill a quarter of, in more than a round of workgroups: N 11, C 333, 8 x 6 x 7 40.0 and 42.6
+    // us, C 165 32.9 and 24.1)
     if (halo && c > static_cast<int>(chip_units())
         && static_cast<size_t>(g.groups) * g.group_batches.divisor * kOrderedBatch * kBlockSize > 2 * size_t(n) * s)
         return false;

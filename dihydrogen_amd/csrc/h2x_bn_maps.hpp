@@ -184,11 +184,13 @@ struct RealBox
     uint32_t lo[3], hi[3]; // interior: lo <= index < hi, per spatial dimension (real coordinates)
 };
 
-// A bit for each of the elements i ... i + VEC - 1 of a real segment: whether it is an interior one.  In rows of a vector or more these are of two rows at most,
-// and the interior ones of a row one run of bits: half the instructions of asking every element.  A workgroup that holds a channel, or most of one, is bound by
-// them where it is alone on its CU.  Batch-norm forward + backward, every element asked -> so, us, going round three sets of tensors: N 4, C 21, 66 x 57, halo
-// of 1 15.5 -> 13.8; N 54, C 42, 12 x 16 14.4 -> 12.9; N 3, C 263, 11 x 15 x 13 18.6 -> 15.8; N 8, C 6, 35 x 33 x 32 18.8 -> 17.0; N 9, C 240, 16 x 15 x
-// 14 42.1 -> 39.7; N 8, C 64, 30^3 61.1 -> 59.0; N 165, C 521, 25 x 19 211.5 -> 211.1.
+// A bit for each of the elements i ... i + VEC - 1 of a real segment: whether it is an interior one. In rows of a
+// vector or more these are of two rows at most, and the interior ones of a row one run of bits: half the instructions
+// of asking every element. A workgroup that holds a channel, or most of one, is bound by them where it is alone on its
+// CU. Batch-norm forward + backward, every element asked -> so, us, going round three sets of tensors: N 4, C 21, 66 x
+// 57, halo of 1 15.5 -> 13.8; N 54, C 42, 12 x 16 14.4 -> 12.9; N 3, C 263, 11 x 15 x 13 18.6 -> 15.8; N 8, C 6, 35 x
+// 33 x 32 18.8 -> 17.0; N 9, C 240, 16 x 15 x 14 42.1 -> 39.7; N 8, C 64, 30^3 61.1 -> 59.0; N 165, C 521, 25 x 19
+// 211.5 -> 211.1.
 template <int VEC>
 __host__ __device__ __forceinline__ uint32_t interior_bits(const RealBox& b, uint32_t i)
 {
@@ -249,8 +251,8 @@ struct HaloCells
     int64_t origin;          // of the first interior element, from the start of the segment
 };
 
-// Element offset, from the start of the channel's first segment, of the first cell of interior row i; the cells before and after the
-// row's interior ones are to be cleared.
+// Element offset, from the start of the channel's first segment, of the first cell of interior row i; the cells before
+// and after the row's interior ones are to be cleared.
 __host__ __device__ __forceinline__ uint32_t halo_row_start(const HaloCells& g, uint32_t i)
 {
     const uint32_t q = fastdiv(i, g.h), y = i - q * g.h.divisor;

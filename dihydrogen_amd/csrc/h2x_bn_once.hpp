@@ -176,8 +176,8 @@ __device__ __forceinline__ void update_statistics(const OnceForward<T>& a, uint3
 }
 
 // What the threads of channel c need once its sums are there, loaded before the elements: behind the sums nothing else hides the
-// wait (forward in us, loaded behind the sums and so: N 24, C 224, 5 x 4 3.40 and 3.08; N 16, C 256, 28 x 28 6.59 and 6.42; N 64, C 512,
-// 14 x 14 12.2 and 12.0; from 20 us on equal).
+// wait (forward in us, loaded behind the sums and so: N 24, C 224, 5 x 4 3.40 and 3.08; N 16, C 256, 28 x 28 6.59 and
+// 6.42; N 64, C 512, 14 x 14 12.2 and 12.0; from 20 us on equal).
 template <typename T>
 struct ChannelParams
 {

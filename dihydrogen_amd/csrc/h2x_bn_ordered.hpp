@@ -44,10 +44,10 @@ struct OrderedClearing : OrderedGeometry
     HaloCells halo;
 };
 
-// Zeros in the halo cells of a channel, by threads `at`, at + threads, ...  (Whole passes of doubles, forward + backward in us, in the staged calls,
-// up to seven launches, and so: N 1, C 115, 49 x 58, halo of 2 30.9 -> 10.7; N 24, C 542, 6 x 6 36.7 -> 17.8; N 12, C 61, 85 x 84 69 -> 56; 80
-// drawn calls 0.76 of their time.)  Stored normally, as the interior is, whose lines they complete in the cache: behind it, or, by the kernels
-// of short segments, before it.
+// Zeros in the halo cells of a channel, by threads `at`, at + threads, ... (Whole passes of doubles, forward + backward
+// in us, in the staged calls, up to seven launches, and so: N 1, C 115, 49 x 58, halo of 2 30.9 -> 10.7; N 24, C 542, 6
+// x 6 36.7 -> 17.8; N 12, C 61, 85 x 84 69 -> 56; 80 drawn calls 0.76 of their time.) Stored normally, as the interior
+// is, whose lines they complete in the cache: behind it, or, by the kernels of short segments, before it.
 template <typename T>
 __device__ __forceinline__ void clear_halo_cells(const HaloCells& g, T* interior, uint32_t at, uint32_t threads)
 {
@@ -168,10 +168,10 @@ __device__ __forceinline__ void ordered_totals(double (&v)[N], const double (&wa
 
 // The sums of the channel in v[] of every thread, from the partial sums in `shared`.  Teams: a counter, tags and looks as in
 // team_exchange; recompute(m) leaves the partial sums of member m in `shared`.  What a thread of channel_totals starts
-// with, or the thread in steps of two or four where the members exchange sums of as many partials, the same lane of the first four
-// waves looks for; the lanes in between take the other sums, so that the steps of the tree that are left add
-// all of them at once.  (With a lane an item, all its sums one after another, N 8, C 32, 33^3 forward + backward, took 86.2 us,
-// so 75.4; N 24, C 461, 24 x 30 with a halo of 1 98.8 and 86.0; N 16, C 32, 112 x 112 54.7 and 49.0.)
+// with, or the thread in steps of two or four where the members exchange sums of as many partials, the same lane of the
+// first four waves looks for; the lanes in between take the other sums, so that the steps of the tree that are left add
+// all of them at once. (With a lane an item, all its sums one after another, N 8, C 32, 33^3 forward + backward, took
+// 86.2 us, so 75.4; N 24, C 461, 24 x 30 with a halo of 1 98.8 and 86.0; N 16, C 32, 112 x 112 54.7 and 49.0.)
 template <int TEAM, int K, int N, bool TEAMS, typename F>
 __device__ __forceinline__ void ordered_exchange(double (&v)[N], const OrderedGeometry& g, uint32_t member,
                                                  unsigned long long* state, uint32_t tag,

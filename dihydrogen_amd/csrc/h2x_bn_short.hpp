@@ -4,8 +4,8 @@
 // The staged short-segment reduction gives each slot (vector) of a channel's segment a lane a row, which adds the
 // samples row, row + rows, ... of a range; the slots of a row are added as a tree, then the rows and the ranges one
 // after the other.  Which channels share a workgroup does not matter to that order.  Here a workgroup holds all samples of a
-// few neighbouring channels in its registers: a lane plays a slot and a row of some ranges, the sums of its ranges go to LDS, waves
-// add the trees there, and y (dx) is written from the registers.
+// few neighbouring channels in its registers: a lane plays a slot and a row of some ranges, the sums of its ranges go
+// to LDS, waves add the trees there, and y (dx) is written from the registers.
 //
 // Bound by launches and waits where tensors are small, else by memory and by registers that a range which is no whole number
 // of a lane's vectors leaves idle.  Two launches each way -> this, forward + backward, us going round three sets of tensors:
@@ -76,11 +76,12 @@ __host__ __device__ __forceinline__ uint32_t short_once_sample(const ShortOnceGe
     return of_range < g.per && range < g.ranges ? range * g.per + of_range : ~0u;
 }
 
-// Terms 0 to n - 1, one after the other; n is uniform and at least 1.  An addition that waits for the read before it takes 100 clocks: they
-// are read ahead of the additions, eight at a time.  (The sums of a range and those of the ranges by a thread each, reads ahead, against one
-// thread a channel, read by read, forward + backward in us: N 254, C 149, 3 x 3 16.5 -> 13.1, N 243, C 1065, 1 x 1 13.2 -> 10.7; N 18, C 776, 15 x 15
-// 43.5 -> 35.8; N 148, C 334, 5 x 5 23.7 -> 22.5; 55 drawn calls 0.97.  In finish_short, whose workgroups have two to eight rows, the reads beyond the
-// last row cost more than they save: N 67, C 55, 9 x 11 21.1 and 22.4.)
+// Terms 0 to n - 1, one after the other; n is uniform and at least 1. An addition that waits for the read before it
+// takes 100 clocks: they are read ahead of the additions, eight at a time. (The sums of a range and those of the ranges
+// by a thread each, reads ahead, against one thread a channel, read by read, forward + backward in us: N 254, C 149, 3
+// x 3 16.5 -> 13.1, N 243, C 1065, 1 x 1 13.2 -> 10.7; N 18, C 776, 15 x 15 43.5 -> 35.8; N 148, C 334, 5 x 5 23.7 ->
+// 22.5; 55 drawn calls 0.97. In finish_short, whose workgroups have two to eight rows, the reads beyond the last row
+// cost more than they save: N 67, C 55, 9 x 11 21.1 and 22.4.)
 template <typename F>
 __device__ __forceinline__ double sum_in_order(uint32_t n, const F& term)
 {
@@ -116,10 +117,11 @@ __device__ __forceinline__ void short_once_totals(const G& g, const ShortOnceLan
         const uint32_t at_once = kWaveSize / lanes, slot = lane & (lanes - 1);
         const uint32_t runs = g.together * rows * channels, trees = runs * g.passes * N;
         uint32_t first = wave * at_once; // uniform
-        // Backward, which has twice the trees: two of them at once wait for their exchanges together (forward + backward in us, one by one and so: N 18,
-        // C 386, 8 x 9 15.5 and 14.9; N 15, C 136, 7 x 10 with a halo 11.8 and 11.2; N 42, C 271, 4 x 6 12.4 and 11.9; forward, four at
-        // once, or trees wider than a wave 2 to 10 % longer; where a large output's halo is cleared, and what waits longer spreads the stores, N 158, C
-        // 610, 7 x 4 68.5 and 70.4).
+        // Backward, which has twice the trees: two of them at once wait for their exchanges together (forward +
+        // backward in us, one by one and so: N 18, C 386, 8 x 9 15.5 and 14.9; N 15, C 136, 7 x 10 with a halo 11.8 and
+        // 11.2; N 42, C 271, 4 x 6 12.4 and 11.9; forward, four at once, or trees wider than a wave 2 to 10 % longer;
+        // where a large output's halo is cleared, and what waits longer spreads the stores, N 158, C 610, 7 x 4 68.5
+        // and 70.4).
         if constexpr (N == 4 && !std::is_same<G, ShortOnceClearing>::value)
             if (width <= kWaveSize)
                 for (constexpr uint32_t kStep = TEAM / kWaveSize; first + kStep * at_once < trees; first += 2 * kStep * at_once)
@@ -216,8 +218,8 @@ __device__ __forceinline__ void short_once_totals(const G& g, const ShortOnceLan
 }
 
 // Ranges that one thread plays, at most: a workgroup keeps the sums of each of its threads for each.  Backward no more than leave
-// the CU as many workgroups as its registers do (four ranges, or two by 1024 threads, 1.012 times as long on average, N 10, C 52, 13 x 15 11.7 and
-// 15.0 us).
+// the CU as many workgroups as its registers do (four ranges, or two by 1024 threads, 1.012 times as long on average, N
+// 10, C 52, 13 x 15 11.7 and 15.0 us).
 constexpr int short_once_passes(int vectors, bool forward)
 {
     return forward ? 4 : vectors / 4;

@@ -23,7 +23,8 @@
 // other streams fill it; the launch rule keeps a team within half of it.
 #pragma once
 
-// (A wave looks after 64 / N members with N lanes each, N sums: 8 waves after 128 of four sums, the most that team_exchange takes.)
+// (A wave looks after 64 / N members with N lanes each, N sums: 8 waves after 128 of four sums, the most that
+// team_exchange takes.)
 constexpr uint32_t kMaxMembers = 128;
 
 // State of a channel, zero before its first call: the counter on a line of its own, then
@@ -67,11 +68,11 @@ __host__ __device__ __forceinline__ uint32_t team_member(uint32_t i, uint32_t me
 // come, and then at the others: what waiting workgroups read takes the memory from those that load.  Between looks they sleep
 // 4 x 64 clocks, 0.1 us, and 44 x 64, 1.2 us, where a launch has more than kCrowd workgroups, about those that the chip holds at
 // once, hundreds of which wait all the time.  N 4, C 64, 64^3, teams of 32 and 64, forward + backward going round three sets
-// of tensors: all words every 0.1 us 266 us, one word every 0.15 us 245, every 0.4 us 242, every 1.2 us 240, every 1.9 us 242, every
-// 2.9 us 246.  Small teams lose by one word every 1.2 us (of 4, N 8, C 64, 56 x 56, 11.7 us and 13.5; of 8 and 15, N 8, C 64, 30^3 with
-// a halo, 73.8 and 74.7), small launches by the long sleep (N 3, C 6, 43 x 50 x 38 15.1 us, with the short one 13.6; N 15, C 4, 22 x
-// 17 x 22, doubles, 15.1 and 13.9; up to 1024 workgroups, N 23, C 21, 144 x 155, 45.0 and 42.0), doubles by all words there (N 81, C 9, 33 x 41 16.9
-// and 19.0).
+// of tensors: all words every 0.1 us 266 us, one word every 0.15 us 245, every 0.4 us 242, every 1.2 us 240, every 1.9
+// us 242, every 2.9 us 246. Small teams lose by one word every 1.2 us (of 4, N 8, C 64, 56 x 56, 11.7 us and 13.5; of 8
+// and 15, N 8, C 64, 30^3 with a halo, 73.8 and 74.7), small launches by the long sleep (N 3, C 6, 43 x 50 x 38 15.1
+// us, with the short one 13.6; N 15, C 4, 22 x 17 x 22, doubles, 15.1 and 13.9; up to 1024 workgroups, N 23, C 21, 144
+// x 155, 45.0 and 42.0), doubles by all words there (N 81, C 9, 33 x 41 16.9 and 19.0).
 constexpr uint32_t kSmallTeam = 16, kCrowd = 1024;
 
 // What the waves of a member leave one another, and what a member knows of the others.
@@ -208,14 +209,15 @@ __device__ __forceinline__ void add_backward_terms(double (&s)[4], const T (&x)[
         }
 }
 
-// Scale and bias are loaded behind the elements: they are scalars, and a wave that asks for them first waits for them before its first
-// element.  The exchange hides them (forward in us, loaded behind the exchange, before the elements and so: N 3, C 17, 31 x 22 x 18 5.4, 5.1 and 5.1;
-// N 32, C 256, 56 x 56 41.0, 40.2 and 39.6, over one set of tensors 33.0, 34.7 and 33.5; N 4, C 64, 64^3 102.8, 102.7 and 101.8, over one set 83.7, 86.3 and
-// 84.8, where what is loaded late spreads the stores).
-// kOneByOne: a wave of a large member whose output's halo is cleared waits for each of its stores (forward in us, at once and so: N 29, C 24, 19 x 32 x 29 31.3
-// and 29.5; N 9, C 128, 124 x 107 30.8 and 28.4; N 3, C 373, 27 x 29 x 38, halo of 2 83.6 and 78.2; N 188, C 301, 8 x 7 x 8 89.6 and 84.9).  Members of 8
-// vectors a thread lose by it (N 3, C 655, 121 x 88 31.1 and 33.2; N 166, C 201, 14 x 20, halo of 2 22.4 and 23.4), dense tensors too where they go round
-// several sets (N 1, C 64, 128 x 128 x 64 95.8 and 100).
+// Scale and bias are loaded behind the elements: they are scalars, and a wave that asks for them first waits for them
+// before its first element. The exchange hides them (forward in us, loaded behind the exchange, before the elements and
+// so: N 3, C 17, 31 x 22 x 18 5.4, 5.1 and 5.1; N 32, C 256, 56 x 56 41.0, 40.2 and 39.6, over one set of tensors 33.0,
+// 34.7 and 33.5; N 4, C 64, 64^3 102.8, 102.7 and 101.8, over one set 83.7, 86.3 and 84.8, where what is loaded late
+// spreads the stores). kOneByOne: a wave of a large member whose output's halo is cleared waits for each of its stores
+// (forward in us, at once and so: N 29, C 24, 19 x 32 x 29 31.3 and 29.5; N 9, C 128, 124 x 107 30.8 and 28.4; N 3, C
+// 373, 27 x 29 x 38, halo of 2 83.6 and 78.2; N 188, C 301, 8 x 7 x 8 89.6 and 84.9). Members of 8 vectors a thread
+// lose by it (N 3, C 655, 121 x 88 31.1 and 33.2; N 166, C 201, 14 x 20, halo of 2 22.4 and 23.4), dense tensors too
+// where they go round several sets (N 1, C 64, 128 x 128 x 64 95.8 and 100).
 template <typename T, int TEAM, int K, bool STREAM, typename G>
 __global__ __launch_bounds__(TEAM) void bn_team_forward_kernel(const TeamGeometry<G> g, const OnceForward<T> a,
                                                                       unsigned long long* states)

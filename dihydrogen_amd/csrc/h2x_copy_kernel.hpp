@@ -651,8 +651,8 @@ struct Audit
     uint64_t launches = 0, workgroups = 0;
     uint64_t outside_loads = 0, outside_stores = 0; // bytes outside every region
     uint64_t misaligned = 0;                        // accesses not aligned as their instruction needs
-    // Of a launch whose threads are followed (0: not): the one that is played, from 1, and the words that are loaded or stored more than once,
-    // or stored by one thread and touched by another.
+    // Of a launch whose threads are followed (0: not): the one that is played, from 1, and the words that are loaded or
+    // stored more than once, or stored by one thread and touched by another.
     uint32_t thread = 0;
     uint64_t shared = 0;
     struct TouchedBy

@@ -180,7 +180,8 @@ __device__ __forceinline__ T wave_combine(T v, const F& f)
 }
 
 // Several sums over the 64 lanes of a wave at once: the lanes are cut into N groups (two or four), and group k returns the
-// total of v[k], all its lanes the same bits.  In a fixed order.  Four sums take seven additions in a row so, one after another 24.
+// total of v[k], all its lanes the same bits. In a fixed order. Four sums take seven additions in a row so, one after
+// another 24.
 template <int N>
 __device__ __forceinline__ double lane_group_sum(double v)
 {

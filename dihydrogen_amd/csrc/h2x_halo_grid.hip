@@ -47,8 +47,8 @@ using copy::DeviceMem;
 using copy::TraceMem;
 using copy::Words;
 
-// A cell that a launch touches once for several strips: an audit, which expects a touch for each, counts so many (that it is one touch, and of
-// one thread, the audit sees by the threads, see issue_fold_grid).
+// A cell that a launch touches once for several strips: an audit, which expects a touch for each, counts so many (that
+// it is one touch, and of one thread, the audit sees by the threads, see issue_fold_grid).
 __device__ __forceinline__ const DeviceMem& of_strips(const DeviceMem& mem, int)
 {
     return mem;
@@ -71,11 +71,15 @@ constexpr int kRanksPerTurn = 2;
 // (5 x 2 x 14 x 6 x 47 of doubles on 2 x 1 x 4, 660 rows: line by line 8.4 us, rank by rank 7.9; 9 x 8 x 287 x 109
 // on 4 x 2, 5,500 rows: 9.4 and 11.1).
 constexpr int64_t kLineRows = 4096;
-// Halo strips in bytes, of all ranks, up to which a reverse exchange of two or three dimensions is one launch.  It saves one launch or two,
-// of 1.5 to 2.5 us each; its regions, a few times as many as strips, keep more workgroups waiting for few cells, and beyond these sizes
-// it takes longer (three launches or two and one, us: 2 x 3 x 15 x 21 x 17 on 2^3 9.4 and 5.5; 1 x 11 x 46 x 67 x 50 on 2^3, 0.76 MB
-// 10.2 and 6.8; 9 x 11 x 28 x 34 x 28 on 2^3, periodic, 4.3 MB 17.0 and 14.2; 6 x 50 x 27^2 x 25 on 2^3, halos of 2, 18 MB 35.9 and 43; two dimensions: 1 x 32
-// x 57 x 57 on 2 x 2 6.4 and 5.3; 2 x 44 x 264 x 116 on 4 x 2, 0.70 MB 6.9 and 6.5; 2 x 15 x 15 x 30 x 79 on 2 x 4, 0.98 MB 8.6 and 10.8).
+// Halo strips in bytes, of all ranks, up to which a reverse exchange of two or three dimensions is one launch.  It saves
+// one launch or two, of 1.5 to 2.5 us each; its regions, a few times as many as strips, keep more workgroups waiting for
+// few cells, which costs more with size.  Three launches or two and one, us:
+//   three dimensions: 2 x 3 x 15 x 21 x 17 on 2^3 9.4 and 5.5; 1 x 11 x 46 x 67 x 50 on 2^3, 0.76 MB 10.2 and 6.8;
+//   9 x 11 x 28 x 34 x 28 on 2^3, periodic, 4.3 MB 17.0 and 14.2; 6 x 50 x 27^2 x 25 on 2^3, halos of 2, 18 MB 35.9, 43;
+//   two: 1 x 32 x 57 x 57 on 2 x 2 6.4 and 5.3; 2 x 44 x 264 x 116 on 4 x 2, 0.70 MB 6.9 and 6.5; 2 x 15 x 15 x 30 x 79
+//   on 2 x 4, 0.98 MB 8.6 and 10.8.
+// The line for two dimensions lies below the last two, on the safe side: just above it one launch gains a twentieth where
+// it gains, and at 0.98 MB loses a quarter.
 constexpr uint64_t kFoldBytes2 = 640 << 10, kFoldBytes3 = 4608 << 10;
 
 // One end of a row of a rank, halo cell 0: where its values come from.
@@ -91,7 +95,8 @@ struct RowEnd
 // followed on the host is: the rank that a region's cells come from, and the neighbours along a row.  (A chain of a
 // dozen loads, some of them through the vector memory, to one of five scalar ones, us, exchange or clear and exchange: 4 x 64 x
 // 57 x 57 on 2 x 2 6.95 -> 6.55, 3 x 40 x 127 x 327 on 2 x 4, halos of 2 6.23 -> 5.66, 2 x 97 x 187 x 181 on 2 x 2 5.25 -> 4.80,
-// 3 x 50 x 16 x 36 x 72 on 2 x 4, halos of 3 26.3 -> 24.9.  Asking for all of the arguments' lines at once before the chain gave no more.)
+// 3 x 50 x 16 x 36 x 72 on 2 x 4, halos of 3 26.3 -> 24.9. Asking for all of the arguments' lines at once before the
+// chain gave no more.)
 struct Rank
 {
     char* tensor;                 // start of the real allocation
@@ -292,10 +297,11 @@ __host__ __device__ __forceinline__ void body(const Args& a, uint32_t block, uin
     }
 }
 
-// A seam of two ranks in the dimension of a reverse exchange.  What a workgroup reads of its arguments stands between its start and its
-// first access, so all that can be followed is followed on the host: two scalar loads, one after the other, instead of five (reverse exchanges, us: 4 x 64 x
-// 57 x 57 on 2 x 2 9.2 -> 7.9; 8 x 6 x 13 x 13 x 12 on 2^3, periodic, halos of 3 14.4 -> 12.5; 2 x 34 x 68 x 105 x 34 of doubles on 2 x 2 x 1 9.9 -> 8.3; 9 x
-// 2 x 63 x 156 x 131 on 1 x 2 x 2, periodic 25.5 -> 21.2; 1 x 32 x 256^3 on 2^3, periodic 304 -> 297).
+// A seam of two ranks in the dimension of a reverse exchange. What a workgroup reads of its arguments stands between
+// its start and its first access, so all that can be followed is followed on the host: two scalar loads, one after the
+// other, instead of five (reverse exchanges, us: 4 x 64 x 57 x 57 on 2 x 2 9.2 -> 7.9; 8 x 6 x 13 x 13 x 12 on 2^3,
+// periodic, halos of 3 14.4 -> 12.5; 2 x 34 x 68 x 105 x 34 of doubles on 2 x 2 x 1 9.9 -> 8.3; 9 x 2 x 63 x 156 x 131
+// on 1 x 2 x 2, periodic 25.5 -> 21.2; 1 x 32 x 256^3 on 2^3, periodic 304 -> 297).
 struct FoldSeam
 {
     char *lower, *upper;              // the lower rank's upper boundary cells, whose upper halo follows them; the upper rank's lower halo,
@@ -444,8 +450,9 @@ __host__ __device__ __forceinline__ void fold_ends_body(const FoldArgs& a, uint3
             if constexpr (BY == kRings)
             {
                 const FoldSeam& below = line[base + i > 0 ? base + i - 1 : a.line - 1];
-                // (Taking the lower end of the next rank, at the same seam, is faster by up to a tenth where the ends of the rows stay in
-                // the caches and slower by as much beyond: the upper end of a row and the lower end of the next share a line.)
+                // (Taking the lower end of the next rank, at the same seam, is faster by up to a tenth where the ends
+                // of the rows stay in the caches and slower by as much beyond: the upper end of a row and the lower end
+                // of the next share a line.)
                 const uint32_t lower_start = row * below.upper_pitch + below.run, upper_start = row * above.lower_pitch;
                 to[i][0] = reinterpret_cast<T*>(lower_end ? below.upper : above.lower) + ((lower_end ? lower_start : upper_start) + j);
                 s[i][0] = mem.load1(reinterpret_cast<const T*>(lower_end ? below.lower : above.upper)
@@ -479,8 +486,8 @@ __global__ __launch_bounds__(kBlock, 8) void halo_fold_ends_kernel(const FoldArg
     fold_ends_body<T, Op, BY, DeviceMem>(a, blockIdx.x, threadIdx.x, op, DeviceMem());
 }
 
-// A launch of a reverse exchange, played for an audit.  Its threads have no order: each cell is loaded once at most and stored once at most, and who
-// stores it is the only one to touch it, or the call fails.
+// A launch of a reverse exchange, played for an audit. Its threads have no order: each cell is loaded once at most and
+// stored once at most, and who stores it is the only one to touch it, or the call fails.
 template <typename F>
 int play_fold(Audit* audit, uint32_t blocks, const F& body)
 {
@@ -538,11 +545,12 @@ int issue_fold(int op, const FoldArgs& a, uint32_t blocks, Fold by, hipStream_t 
     }
 }
 
-// The reverse exchange of several dimensions in one launch.  Phase after phase, every cell of a boundary strip takes in the halo cell
-// of its neighbour along the phase's dimension, which has taken in others before.  Cells whose values meet are a group: per
-// dimension in which they lie at a seam, the boundary cell of one rank and the halo cell of its neighbour that stands for it.
-// A halo cell is of one group alone (a rank has at least two halo widths of interior along such a dimension), so groups have no order: a thread loads the two, four or
-// eight cells of one, plays the phases on them, with their roundings, and stores those that lie in a boundary strip.
+// The reverse exchange of several dimensions in one launch. Phase after phase, every cell of a boundary strip takes in
+// the halo cell of its neighbour along the phase's dimension, which has taken in others before. Cells whose values meet
+// are a group: per dimension in which they lie at a seam, the boundary cell of one rank and the halo cell of its
+// neighbour that stands for it. A halo cell is of one group alone (a rank has at least two halo widths of interior
+// along such a dimension), so groups have no order: a thread loads the two, four or eight cells of one, plays the
+// phases on them, with their roundings, and stores those that lie in a boundary strip.
 //
 // The groups of a rank are those whose cells in all boundary strips are its own: regions per {elsewhere, lower, upper
 // boundary} of the outer two dimensions, as vectors along what of the rows is no end ("elsewhere" of dimension 0), and the ends.

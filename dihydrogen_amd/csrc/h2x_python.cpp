@@ -5,12 +5,11 @@
 // spent more time on that than the GPU on the work.  Here each entry point is
 // one METH_FASTCALL function whose argument conversions are generated from its
 // C signature: integers and floats as they are, and for a pointer None, an
-// address, a torch tensor (what its data_ptr() returns, or raises; where that is torch's own method and no mode listens, it is not
-// called, see data_ptr_of), any other object with a get_base_ptr() method (a local tensor: the method is asked, also where
-// there is a data_ptr() too, or, where it is the one given to pointer_types(), what it does is
-// done here, 0.1 us less than in Python), or one with a data_ptr() method alone.  Every
-// function returns what the C function returns (a status or a size).  The GIL
-// is released during the call, as ctypes does.
+// address, a torch tensor (what its data_ptr() returns, or raises; where that is torch's own method and no mode
+// listens, it is not called, see data_ptr_of), any other object with a get_base_ptr() method (a local tensor: the
+// method is asked, also where there is a data_ptr() too, or, where it is the one given to pointer_types(), what it does
+// is done here, 0.1 us less than in Python), or one with a data_ptr() method alone. Every function returns what the C
+// function returns (a status or a size). The GIL is released during the call, as ctypes does.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -56,8 +55,8 @@ struct Look
     bool is_new = true, plain = false;
 };
 
-// Whether the data_ptr() of torch tensors is the method that torch has in C++ (a class that nobody has changed since has its version tag
-// still), and no mode for torch's functions is on, which would be told of the call.
+// Whether the data_ptr() of torch tensors is the method that torch has in C++ (a class that nobody has changed since
+// has its version tag still), and no mode for torch's functions is on, which would be told of the call.
 bool calls_are_plain()
 {
     PyTypeObject* const t = s_torch_tensor;
@@ -86,8 +85,9 @@ bool has_plain_data_ptr(PyObject* o, Look* look)
     return !own || !*own || !PyDict_GetItemWithError(*own, s_data_ptr);
 }
 
-// What o.data_ptr() returns.  A torch tensor is asked as a C++ object where it can be: through its Python method, with an object made of
-// the address and taken apart again, a pointer took 40 ns, of which a batch-norm backward pass has 14 and a shuffle between 16 ranks 32.
+// What o.data_ptr() returns. A torch tensor is asked as a C++ object where it can be: through its Python method, with
+// an object made of the address and taken apart again, a pointer took 40 ns, of which a batch-norm backward pass has 14
+// and a shuffle between 16 ranks 32.
 // (One that has no memory to point to raises what the method raises.)
 bool data_ptr_of(PyObject* o, void** out, Look* look)
 {
@@ -238,8 +238,8 @@ struct Entry<F>
     }
 };
 
-// Whether torch is the one whose headers this file was compiled with, and has a torch tensor's address where they say.  (Another one's
-// tensors are asked by their method.)
+// Whether torch is the one whose headers this file was compiled with, and has a torch tensor's address where they say.
+// (Another one's tensors are asked by their method.)
 bool is_known_torch(PyObject* type, PyObject* version, PyObject* tensor)
 {
     if (PyUnicode_CompareWithASCIIString(version, H2X_TORCH_VERSION) != 0 || reinterpret_cast<PyObject*>(Py_TYPE(tensor)) != type)
@@ -253,8 +253,8 @@ bool is_known_torch(PyObject* type, PyObject* version, PyObject* tensor)
     return THPVariable_Unpack(tensor).data_ptr() == by_method;
 }
 
-// pointer_types(torch.Tensor, the class of local tensors, its get_base_ptr, its base_bytes, torch.__version__, a torch tensor with
-// memory): whether torch tensors are asked for their addresses as C++ objects.
+// pointer_types(torch.Tensor, the class of local tensors, its get_base_ptr, its base_bytes, torch.__version__, a torch
+// tensor with memory): whether torch tensors are asked for their addresses as C++ objects.
 PyObject* pointer_types(PyObject*, PyObject* const* args, Py_ssize_t nargs)
 {
     if (nargs != 6 || !PyType_Check(args[0]) || !PyType_Check(args[1]) || !PyUnicode_Check(args[4]))

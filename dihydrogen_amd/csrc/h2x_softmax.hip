@@ -535,17 +535,19 @@ __device__ __forceinline__ T pixel_combine(T v, const F& f)
 // Where there are few tiles, a pixel is for 64 / LANES lanes of a wave instead of one: a workgroup serves LANES
 // pixels, lane l of wave g the channels (g + k * WAVES) * 64 / LANES + l / LANES, the chain is that many times shorter
 // and there are as many more workgroups, for rows of 64 or 128 bytes (see launch_split_for).
-// The chain of a wave counts: 19 vector and 6 scalar instructions a channel forward, of which the exponential takes 13.  So the first
-// CERTAIN channels of a wave, which the smallest channel count of the variant has, are not asked for; a channel that is not there is
-// -infinity (backward 0), with no further question but, where a wave lacks it as a whole, one ahead of its exponential; lanes without pixels
-// work on the tile's first one and store nothing; and addresses are a running scalar pointer and a lane's offset in bytes.  Asking before each load, term
-// and store, with addresses of 64 bits a lane (23 and 22 instructions, backward 13 and 30 with registers spilled), forward + backward in
-// us -> so: N 4, C 150, 65 x 97 17.5 -> 16.8; N 2, C 209, 15 x 15 6.85 -> 5.75; N 5, C 308, 56 x 52 21.8 -> 20.6; N 2, C 322,
-// 75 x 110 26.7 -> 24.0; N 4, C 431, 99 x 126 111 -> 102; doubles N 4, C 472, 49 x 44 47.3 -> 43.6; of 47 calls the mean
-// is 0.950.  The question ahead of the exponential is for tiles that are half empty, without it and with it: N 1, C 39, 316 x 354 (asking each time 17.9)
-// 18.0 and 17.1; N 13, C 42, 220 x 134 (56.2) 57.4 and 56.2; doubles N 4, C 33, 128 x 128 (18.0) 18.4 and 17.4.  One round of workgroups of full tiles
-// whose tensors are streamed does lose, a wave's loads now being together: N 1, C 60, 316 x 354 28.7 -> 29.5, N 8, C 60, 112 x 125 28.2 -> 29.0 (two rounds,
-// N 2, C 60, 316 x 354 52.5 -> 49.8).
+// The chain of a wave counts: 19 vector and 6 scalar instructions a channel forward, of which the exponential takes 13.
+// So the first CERTAIN channels of a wave, which the smallest channel count of the variant has, are not asked for; a
+// channel that is not there is -infinity (backward 0), with no further question but, where a wave lacks it as a whole,
+// one ahead of its exponential; lanes without pixels work on the tile's first one and store nothing; and addresses are
+// a running scalar pointer and a lane's offset in bytes. Asking before each load, term and store, with addresses of 64
+// bits a lane (23 and 22 instructions, backward 13 and 30 with registers spilled), forward + backward in us -> so: N 4,
+// C 150, 65 x 97 17.5 -> 16.8; N 2, C 209, 15 x 15 6.85 -> 5.75; N 5, C 308, 56 x 52 21.8 -> 20.6; N 2, C 322, 75 x 110
+// 26.7 -> 24.0; N 4, C 431, 99 x 126 111 -> 102; doubles N 4, C 472, 49 x 44 47.3 -> 43.6; of 47 calls the mean is
+// 0.950. The question ahead of the exponential is for tiles that are half empty, without it and with it: N 1, C 39, 316
+// x 354 (asking each time 17.9) 18.0 and 17.1; N 13, C 42, 220 x 134 (56.2) 57.4 and 56.2; doubles N 4, C 33, 128 x 128
+// (18.0) 18.4 and 17.4. One round of workgroups of full tiles whose tensors are streamed does lose, a wave's loads now
+// being together: N 1, C 60, 316 x 354 28.7 -> 29.5, N 8, C 60, 112 x 125 28.2 -> 29.0 (two rounds, N 2, C 60, 316 x
+// 354 52.5 -> 49.8).
 template <typename T, int VEC, int CPW, int CERTAIN, int WAVES, int LANES, bool STREAM>
 __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_fwd_split_kernel(
     const T* __restrict__ x, T* __restrict__ y, int num_channels, size_t spatial, int flat_samples,
@@ -709,9 +711,10 @@ __global__ __launch_bounds__(WAVES * kWaveSize) void softmax_bwd_split_kernel(
         }
 }
 
-// Up to 32 channels of few pixels: a workgroup of 256 threads serves LANES pixels, thread group g their channels g, g + 256 / LANES, ...
-// A lane's chain of loads, exponentials and stores is that many times shorter, and there are as many more workgroups.  The exponentials
-// (backward the values) go through LDS, where each thread adds those of its pixel in channel order: the same bits as by one thread a pixel.
+// Up to 32 channels of few pixels: a workgroup of 256 threads serves LANES pixels, thread group g their channels g, g +
+// 256 / LANES, ... A lane's chain of loads, exponentials and stores is that many times shorter, and there are as many
+// more workgroups. The exponentials (backward the values) go through LDS, where each thread adds those of its pixel in
+// channel order: the same bits as by one thread a pixel.
 template <typename T, int CMAX, int LANES>
 __global__ __launch_bounds__(kBlockSize) void softmax_fwd_shared_kernel(
     const T* __restrict__ x, T* __restrict__ y, int num_channels, size_t spatial, int flat_samples, const WideTiles tiles)
@@ -1050,8 +1053,8 @@ dim3 pixel_grid_xcd(size_t spatial, int vec, int num_samples, int flat)
 // a sample, 23.3 and 18.0; N 25, C 120, 24 x 24, 9 tiles, 14.9 and 10.9; N 29, C 338, 24 x 37, 14 tiles,
 // 43.6 and 41.4; but N 30, C 179, 43 x 43, 29 tiles, 47.3 and 48.0, N 8, C 40, 128 x 128, 128 tiles,
 // 20.1 and 21.4: samples one after another reach the memory more evenly).  Also where only the filling makes them more
-// than two a CU: a third would start when the first two are done, on the XCDs that have it (N 11, C 135, 45 x 61, 473 tiles filled up to 528,
-// 19.3 and 17.4; N 5, C 151, 92 x 67, 485 to 520, 20.7 and 18.8).
+// than two a CU: a third would start when the first two are done, on the XCDs that have it (N 11, C 135, 45 x 61, 473
+// tiles filled up to 528, 19.3 and 17.4; N 5, C 151, 92 x 67, 485 to 520, 20.7 and 18.8).
 dim3 wide_grid(size_t spatial, int lanes, int vec, int num_samples, int flat, WideTiles* t)
 {
     const dim3 by_sample = tile_grid(spatial, lanes, vec, num_samples, flat);
@@ -1089,8 +1092,8 @@ void launch_bwd(const T* y, const T* dy, T* dx, int n, int c, size_t s, bool str
         launch(softmax_bwd_reg_kernel<T, VEC, CMAX, false>, grid, kBlockSize, st, y, dy, dx, c, s, flat);
 }
 
-// More samples than this fill the chip with a wave each; and more than kSomeSamples (channel softmax of floats, forward: kSomeRows) leave its waves
-// little to wait for where samples are short.
+// More samples than this fill the chip with a wave each; and more than kSomeSamples (channel softmax of floats,
+// forward: kSomeRows) leave its waves little to wait for where samples are short.
 constexpr int kManySamples = 2048, kSomeSamples = 768, kSomeRows = 512;
 
 // Which kernel serves which channel count (measured on MI355X).  Up to 32 channels a
@@ -1277,9 +1280,9 @@ int launch_shared(const T* y, const T* dy, T* dx, int n, int c, size_t s, hipStr
     return launch_status();
 }
 
-// Up to 32 channels: the threads of a workgroup share them, or kNoSplit.  Where one thread a pixel leaves CUs waiting for its chain; with more
-// pixels the sums that every thread forms cost more than the chain.  Us in a graph, a thread a pixel and so (32 pixels forward, 16 backward; 64
-// pixels are slower throughout, and at 2^17 pixels all of them are):
+// Up to 32 channels: the threads of a workgroup share them, or kNoSplit. Where one thread a pixel leaves CUs waiting
+// for its chain; with more pixels the sums that every thread forms cost more than the chain. Us in a graph, a thread a
+// pixel and so (32 pixels forward, 16 backward; 64 pixels are slower throughout, and at 2^17 pixels all of them are):
 //   floats, C 32, 4608 pixels 4.9 / 4.1 and 3.6 / 3.3, 2^14 5.1 / 4.3 and 4.0 / 3.9, 2^15 5.3 / 4.5 and 4.4 / 4.8, 2^16 6.0 / 6.4 and 6.0 / 8.6;
 //   C 12, 2^14 3.1 / 2.7 and 2.9 / 2.7; C 8, 2^15 2.8 / 2.4 and 2.8 / 2.8;
 //   doubles, whose exponentials are longer, C 32, 4608 pixels 8.6 / 5.2 and 4.1 / 3.8, 2^16 12.3 / 10.0 and 9.8 / 12.3, 3 x 2^16 23.3 and 24.1
@@ -1303,13 +1306,17 @@ int launch_shared_for(int n, int c, size_t s, hipStream_t st, P... p)
 // Calls f(elements a lane, lanes) with constants for samples of `size` contiguous elements that
 // lanes hold in registers: a wave while samples are short, or many (it needs no barrier), else
 // a workgroup, of 1024 threads with up to MAX_LARGE elements each where 256 would have more than 16.
-// A workgroup from 257 elements on, and from 513 also of more than `some` samples: a wave's chain of up to 32 loads, exponentials and stores is what
-// else is waited for (sums of the data's type have fewer terms in a row so).  GPU time, a wave a sample -> a workgroup, forward / backward in us: channels, floats
-// N 16, 1000 3.1 / 2.4 -> 2.2 / 1.8, N 466, 1983 5.1 / 4.2 -> 3.3 / 2.9, N 1418, 1480 6.7 / 6.0 -> 5.6 / 5.4; doubles N 59, 1480 6.6 / 3.8 -> 3.3 / 2.3, N 700, 1000 5.7 /
-// 4.5 -> 4.3 / 3.8, N 1418, 704 6.4 / 5.6 -> 5.7 / 5.2; instances of doubles N 128, 1983 8.6 / 4.6 -> 4.0 / 2.7 (at the line, channels, floats N 2048, 600 4.0 / 3.3 -> 4.2 / 3.3, 1000 5.2 / 5.2 both ways).  Up to 512 elements, a wave
-// and a workgroup: channels, floats, 300 and 400 elements, N 466 2.3 / 1.9 and 2.3 / 1.8, N 512 2.3 / 2.0 and 2.3 / 1.9, N 600 2.4 / 2.0 and 2.4 / 1.9, N 700 2.3 / 1.9 and 2.4 /
-// 1.8, N 768 2.4 / 2.0 and 2.6 / 1.9, N 1000 2.4 / 1.9 and 2.8 / 1.9; doubles, 400, N 512 3.4 / 2.4 and 2.7 / 2.1, N 768 3.5 / 2.4 and 3.0 / 2.3; instances, floats, 400, N 700 3.0 / 2.2 and
-// 2.7 / 2.1, N 850 3.1 / 2.2 and 3.0 / 2.2, N 1418 3.1 / 2.3 and 3.4 / 2.6; N 2600 the same either way.
+// A workgroup from 257 elements on, and from 513 also of more than `some` samples: a wave's chain of up to 32 loads,
+// exponentials and stores is what else is waited for (sums of the data's type have fewer terms in a row so; the last
+// bits of a sample of channels differ between the two, and so go with the number of samples). GPU time, a wave a sample
+// -> a workgroup, forward / backward in us: channels, floats N 16, 1000 3.1 / 2.4 -> 2.2 / 1.8, N 466, 1983 5.1 / 4.2
+// -> 3.3 / 2.9, N 1418, 1480 6.7 / 6.0 -> 5.6 / 5.4; doubles N 59, 1480 6.6 / 3.8 -> 3.3 / 2.3, N 700, 1000 5.7 / 4.5
+// -> 4.3 / 3.8, N 1418, 704 6.4 / 5.6 -> 5.7 / 5.2; instances of doubles N 128, 1983 8.6 / 4.6 -> 4.0 / 2.7 (at the
+// line, channels, floats N 2048, 600 4.0 / 3.3 -> 4.2 / 3.3, 1000 5.2 / 5.2 both ways). Up to 512 elements, a wave and
+// a workgroup: channels, floats, 300 and 400 elements, N 466 2.3 / 1.9 and 2.3 / 1.8, N 512 2.3 / 2.0 and 2.3 / 1.9, N
+// 600 2.4 / 2.0 and 2.4 / 1.9, N 700 2.3 / 1.9 and 2.4 / 1.8, N 768 2.4 / 2.0 and 2.6 / 1.9, N 1000 2.4 / 1.9 and 2.8 /
+// 1.9; doubles, 400, N 512 3.4 / 2.4 and 2.7 / 2.1, N 768 3.5 / 2.4 and 3.0 / 2.3; instances, floats, 400, N 700 3.0 /
+// 2.2 and 2.7 / 2.1, N 850 3.1 / 2.2 and 3.0 / 2.2, N 1418 3.1 / 2.3 and 3.4 / 2.6; N 2600 the same either way.
 template <int MAX_LARGE = 0, typename F>
 int with_lanes(int n, size_t size, int some, const F& f)
 {
@@ -1846,11 +1853,13 @@ constexpr size_t kInstSmallSample = kInstLargeLanes<T> * size_t(1024);
 template <typename T>
 constexpr size_t kInstSmallChunk = size_t(kBlockSize) * (16 / sizeof(T)) * kInstUnroll;
 
-// Whether a workgroup holds a sample whose sums are added in the order of chunks, as those of larger samples are, so that a team can run a whole pass
-// (softmax_inst_team_*_kernel), and a workgroup, in whole vectors, any (softmax_inst_rounds_kernel).  vec: elements of a vector.
-// Single elements: only what teams may take, of the upper half; forward + backward, one workgroup's lanes -> in rounds in us, N 2, 12001 floats 10.4 and 10.2, but
-// N 256, 17101 22.5 and 23.2, dot products and gradients alone 32 and 34.  Lane by lane -> by teams: N 4, 17101 floats 13.7 -> 10.8, N 64
-// 15.4 -> 13.7, N 2, 28225 16.7 -> 10.9; N 4, 9001 doubles 13.4 -> 10.0; in place, in rounds, 14.0 -> 12.2, 15.4 -> 13.6, 16.9 -> 14.9, 13.6 -> 12.4.
+// Whether a workgroup holds a sample whose sums are added in the order of chunks, as those of larger samples are, so
+// that a team can run a whole pass (softmax_inst_team_*_kernel), and a workgroup, in whole vectors, any
+// (softmax_inst_rounds_kernel). vec: elements of a vector. Single elements: only what teams may take, of the upper
+// half; forward + backward, one workgroup's lanes -> in rounds in us, N 2, 12001 floats 10.4 and 10.2, but N 256, 17101
+// 22.5 and 23.2, dot products and gradients alone 32 and 34. Lane by lane -> by teams: N 4, 17101 floats 13.7 -> 10.8,
+// N 64 15.4 -> 13.7, N 2, 28225 16.7 -> 10.9; N 4, 9001 doubles 13.4 -> 10.0; in place, in rounds, 14.0 -> 12.2, 15.4
+// -> 13.6, 16.9 -> 14.9, 13.6 -> 12.4.
 template <typename T>
 bool inst_by_chunks(int n, size_t sample_size, int vec)
 {
@@ -1867,8 +1876,9 @@ int inst_vector(size_t sample_size, const void* a, const void* b, const void* ou
     return vector_width<T>(sample_size, 16 / sizeof(T), {a, b ? b : a, out ? out : a});
 }
 
-// Whether the lanes of a wave or a workgroup hold a sample, each adding up its own elements.  (Asked before anything is cut: the host's part of a small
-// call is what it is bound by, and samples of one chunk go by lanes whatever the vectors are.)
+// Whether the lanes of a wave or a workgroup hold a sample, each adding up its own elements. (Asked before anything is
+// cut: the host's part of a small call is what it is bound by, and samples of one chunk go by lanes whatever the
+// vectors are.)
 template <typename T>
 bool inst_by_lanes(int n, size_t sample_size, const void* a, const void* b, const void* out)
 {
@@ -1919,11 +1929,11 @@ size_t inst_chunk_bytes(int num_samples)
 
 // Samples that are no whole vectors are cut as those of whole vectors are: with chunks a quarter of that, members of four chunks
 // hold 16 KB, and there are four times as many (forward + backward, by teams, N 23, 142,071 floats 59.7 -> 27.5 us, N 12, 241,997
-// 50.7 -> 26.9; separate launches 37 and 35).  Few samples leave CUs idle with members of four such chunks, and are cut finer up to
-// three quarters of a round of the chip (N 2, 138,475 doubles, 34 and 68 members, 17.3 and 16.0; N 2, 439,890 floats 19.6 and 18.7).
-// Chunks of more than 32 KB pay there only if members of four fill most of one round of the chip (N 5, 3,054,213 floats, 315
-// members, 143 us, in chunks of 16 KB, and no teams, 122; N 3, 2,097,657, 129 members, 59 and 54; with 144 to 256 members the same
-// either way).
+// 50.7 -> 26.9; separate launches 37 and 35). Few samples leave CUs idle with members of four such chunks, and are cut
+// finer up to three quarters of a round of the chip (N 2, 138,475 doubles, 34 and 68 members, 17.3 and 16.0; N 2,
+// 439,890 floats 19.6 and 18.7). Chunks of more than 32 KB pay there only if members of four fill most of one round of
+// the chip (N 5, 3,054,213 floats, 315 members, 143 us, in chunks of 16 KB, and no teams, 122; N 3, 2,097,657, 129
+// members, 59 and 54; with 144 to 256 members the same either way).
 InstChunking inst_chunking(size_t sample_size, int num_samples, int vec, size_t elem_bytes)
 {
     const size_t gmax = inst_groups_per_sample_max(num_samples);
@@ -2056,13 +2066,14 @@ int inst_map(int n, size_t sample_size, const void* y, const void* dy, const voi
 constexpr int kInstMostForward = 16, kInstMostBackward = 8;
 
 // What a forward pass by members of four chunks takes more than one in separate launches, in us: by the bytes, and for every
-// round of the chip, which holds two members of up to four vectors a thread a CU, or one larger one (of eight, whose team may fill
-// a quarter of the chip, the second ones start late), what it needs for its loads, two exchanges and stores.  Fitted to 353 calls,
-// forward with backward; the way it names makes both 0.1 to 0.2 % longer than the faster one on average (also of 170
-// calls not fitted to), 3.9 at most, always teams 0.6, 0.5 and (single elements) 0.1, never 6.8, 6.4 and 15.7 %.  Members of one chunk, and
-// backward passes, which exchange once, are never slower than separate launches.  Forward + backward, separate launches,
-// by teams: N 1, 760,320 floats 16.7 and 17.8; N 2, 1,853,544 27.3 and 28.1; N 7, 1,280,796, more than a round, 62 and 61; N 24,
-// 318,008 45.2 and 38.8; N 7, 264,306 23.2 and 19.2; N 4, 915,840 doubles 43.3 and 38.7.
+// round of the chip, which holds two members of up to four vectors a thread a CU, or one larger one (of eight, whose
+// team may fill a quarter of the chip, the second ones start late), what it needs for its loads, two exchanges and
+// stores. Fitted to 353 calls, forward with backward; the way it names makes both 0.1 to 0.2 % longer than the faster
+// one on average (also of 170 calls not fitted to), 3.9 at most, always teams 0.6, 0.5 and (single elements) 0.1, never
+// 6.8, 6.4 and 15.7 %. Members of one chunk, and backward passes, which exchange once, are never slower than separate
+// launches. Forward + backward, separate launches, by teams: N 1, 760,320 floats 16.7 and 17.8; N 2, 1,853,544 27.3 and
+// 28.1; N 7, 1,280,796, more than a round, 62 and 61; N 24, 318,008 45.2 and 38.8; N 7, 264,306 23.2 and 19.2; N 4,
+// 915,840 doubles 43.3 and 38.7.
 struct InstForwardCost
 {
     float base, per_mb, per_mb_beyond, per_round[3], wait; // beyond: 40 MB; per_round: of 64, 128, 256 KB; wait: of a round, for 64 members
@@ -2093,9 +2104,10 @@ bool inst_team(int n, size_t sample_size, const void* a, const void* b, const vo
     const int each = static_cast<int>(ch.chunk / kBlockSize / (16 / sizeof(T))); // vectors of 16 bytes
     const int chunks = ch.groups <= static_cast<int>(kInstMembers) ? 1 : 4;
     const int members = (ch.groups + chunks - 1) / chunks;
-    // Of what a workgroup holds, samples of more than four chunks, of which there are few.  One workgroup each and by teams, us: N 64, 5 chunks of floats
-    // 11.6 and 12.2, of doubles 11.3 and 11.9, N 32 11.0 and 9.9; N 128, 5 chunks 15.2 and 15.9, doubles 14.1 and 15.6; N 96, 7 chunks
-    // 19.7 and 17.4, N 128 22.0 and 20.8; N 128, 8 chunks 23.8 and 22.6, N 256 39.4 and 38.1 before a workgroup's first round went without comparisons (37.5 so).
+    // Of what a workgroup holds, samples of more than four chunks, of which there are few. One workgroup each and by
+    // teams, us: N 64, 5 chunks of floats 11.6 and 12.2, of doubles 11.3 and 11.9, N 32 11.0 and 9.9; N 128, 5 chunks
+    // 15.2 and 15.9, doubles 14.1 and 15.6; N 96, 7 chunks 19.7 and 17.4, N 128 22.0 and 20.8; N 128, 8 chunks 23.8 and
+    // 22.6, N 256 39.4 and 38.1 before a workgroup's first round went without comparisons (37.5 so).
     if (inst_by_chunks<T>(n, sample_size, *v))
     {
         const int cus = static_cast<int>(compute_units());

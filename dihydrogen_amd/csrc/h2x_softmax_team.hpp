@@ -1,7 +1,8 @@
-// Instance softmax of samples beyond one workgroup, in one launch each way: the
-// workgroups of a team hold a sample in their registers, one or four chunks of the staged
-// reductions each, and exchange their partial results through memory.  Included by
-// h2x_softmax.hip.
+// Instance softmax of samples of several chunks, in one launch each way.  Teams (samples beyond one
+// workgroup, and few of more than four chunks): the workgroups of a team hold a sample in their registers,
+// one or four chunks of the staged reductions each, and exchange their partial results through memory.
+// One workgroup that plays the chunks of a sample, four a round (softmax_inst_rounds_kernel, below): the
+// other samples of several chunks that it holds.  Included by h2x_softmax.hip.
 //
 // The launches for the maximum, the sum and the map read the sample three times and are
 // bound by their starts; here every element is read once, and what is bound is the wait
@@ -203,11 +204,12 @@ __device__ __forceinline__ void add_products(double& acc, const Pack<T, VEC>& y,
 }
 
 // Waves of a SIMD: two members of 1024 threads a CU, for which a thread may have 64 registers, where it holds up to 32 (HELD
-// elements; doubles in single elements spill then).  Without the bound the compiler gives forward floats of 8 vectors 67 registers,
-// doubles 69, backward floats of 4 vectors 66, and single elements (61 and 59) too many scalars: one member a CU.  us, without ->
-// with, going round three sets of tensors: forward N 16, 1,225,728 floats 59.3 -> 51.5, N 23, 632,400 doubles 82.2 -> 68.0; backward
-// N 11, 527,040 floats 17.3 -> 15.5; single elements N 24, 318,009 24.6 -> 20.8 forward, 21.7 -> 18.9 backward, but, where all members
-// have a CU of their own, N 4, 500,001 12.8 -> 13.0 and 9.1 -> 9.45, N 11, 263,537 12.6 -> 12.8 and 10.1 -> 10.4.
+// elements; doubles in single elements spill then). Without the bound the compiler gives forward floats of 8 vectors 67
+// registers, doubles 69, backward floats of 4 vectors 66, and single elements (61 and 59) too many scalars: one member
+// a CU. us, without -> with, going round three sets of tensors: forward N 16, 1,225,728 floats 59.3 -> 51.5, N 23,
+// 632,400 doubles 82.2 -> 68.0; backward N 11, 527,040 floats 17.3 -> 15.5; single elements N 24, 318,009 24.6 -> 20.8
+// forward, 21.7 -> 18.9 backward, but, where all members have a CU of their own, N 4, 500,001 12.8 -> 13.0 and 9.1 ->
+// 9.45, N 11, 263,537 12.6 -> 12.8 and 10.1 -> 10.4.
 template <typename T, int TEAM, int HELD, bool SINGLE>
 constexpr int inst_waves()
 {
@@ -314,11 +316,12 @@ __global__ __launch_bounds__(TEAM, (inst_waves<T, TEAM, 2 * VEC * V, VEC == 1>()
     });
 }
 
-// Samples of several chunks that one workgroup holds, where a team is not for the call (many samples, smaller ones, in place, a single reduction, no
-// state): the workgroup plays the chunks, four a round, and adds their sums as the combination of stored ones does: a round's are
-// what a member of four chunks exchanges, and one addition, the last that is not of zeros, is left.  All rounds but the last are of
-// whole chunks.  Bound by the work of a CU and by waits in a row.  The kernel that adds lane by lane, which loads single
-// elements and compares for each, -> this, forward + backward in us, going round three sets of tensors:
+// Samples of several chunks that one workgroup holds, where a team is not for the call (many samples, smaller ones, in
+// place, a single reduction, no state): the workgroup plays the chunks, four a round, and adds their sums as the
+// combination of stored ones does: a round's are what a member of four chunks exchanges, and one addition, the last
+// that is not of zeros, is left. All rounds but the last are of whole chunks. Bound by the work of a CU and by waits in
+// a row. The kernel that adds lane by lane, which loads single elements and compares for each, -> this, forward +
+// backward in us, going round three sets of tensors:
 //   floats  N 16, 4100    8.4 -> 7.3      N 16, 12000   10.5 -> 8.7     N 128, 16400  17.0 -> 14.3    N 256, 32768  41.1 -> 37.5
 //   doubles N 16, 4200    9.1 -> 7.7      N 128, 8200   15.4 -> 13.7    N 500, 12000  58.7 -> 52.1    N 500, 16384  78.0 -> 66.7
 //   in place, floats  N 2, 32768  18.2 -> 14.5    N 64, 20000  16.1 -> 12.8    N 256, 28224  29.5 -> 27.5

@@ -902,6 +902,10 @@ int h2x_tensor_reduce_sum(h2x_dtype dtype,
 /* ------------------------------------------------------------------------ */
 /* Channel softmax: dense [num_samples][num_channels][spatial_size] tensors,  */
 /* softmax taken over the channel dimension.                                  */
+/* Sums are in the data's type; the order of a pixel's additions, and with it   */
+/* the last bits, goes with num_channels, spatial_size, the alignment of the    */
+/* tensors, num_samples (a batch cut into parts need not give the bits of the   */
+/* whole) and the device's CUs, and is the same at every call with these alike. */
 /* ------------------------------------------------------------------------ */
 
 /**
@@ -937,7 +941,10 @@ int h2x_softmax_channel_backward(h2x_dtype dtype,
 /* scalars between them when a sample is spread over ranks                     */
 /* (legacy/src/dnn_backend/softmax.cu:705-784,                                */
 /*  legacy/include/distconv/dnn_backend/softmax.hpp:52-62); the stages are    */
-/* the entry points.  Per-sample vectors hold num_samples elements.           */
+/* the entry points.  Per-sample vectors hold num_samples elements.  Sums are  */
+/* in fp64; their order goes with sample_size, num_samples, the alignment of   */
+/* the tensors and the device's CUs, and is that of the stages in the calls    */
+/* that run several of them.                                                   */
 
 /** Workspace (fp64 partials) of the three reducing stages; no initialisation needed. */
 size_t h2x_softmax_instance_workspace_bytes(int num_samples);
