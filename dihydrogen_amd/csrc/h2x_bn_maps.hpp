@@ -191,6 +191,8 @@ struct RealBox
 // 57, halo of 1 15.5 -> 13.8; N 54, C 42, 12 x 16 14.4 -> 12.9; N 3, C 263, 11 x 15 x 13 18.6 -> 15.8; N 8, C 6, 35 x
 // 33 x 32 18.8 -> 17.0; N 9, C 240, 16 x 15 x 14 42.1 -> 39.7; N 8, C 64, 30^3 61.1 -> 59.0; N 165, C 521, 25 x 19
 // 211.5 -> 211.1.
+// Segments that are no whole vectors go by single elements, for which a run is more work than the question (inference, run
+// and question: N 64, C 100, 13 x 17, halo of 1 7.7 and 7.1; N 32, C 21, 51 x 42 x 33, halo of 2 106 and 102.6).
 template <int VEC>
 __host__ __device__ __forceinline__ uint32_t interior_bits(const RealBox& b, uint32_t i)
 {
@@ -198,6 +200,8 @@ __host__ __device__ __forceinline__ uint32_t interior_bits(const RealBox& b, uin
     uint32_t x = i - t * b.wr.divisor;
     uint32_t z = fastdiv(t, b.hr);
     uint32_t y = t - z * b.hr.divisor;
+    if constexpr (VEC == 1) // one question
+        return x >= b.lo[0] && x < b.hi[0] && y >= b.lo[1] && y < b.hi[1] && z >= b.lo[2] && z < b.hi[2];
     const auto row_counts = [&] { return y - b.lo[1] < b.hi[1] - b.lo[1] && z - b.lo[2] < b.hi[2] - b.lo[2]; };
     const auto next_row = [&] {
         if (++y == b.hr.divisor)
