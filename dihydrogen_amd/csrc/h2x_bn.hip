@@ -2866,14 +2866,15 @@ bool streamed(const OnceGeometry& g, int n)
 // eight it holds one, of five and six too, with registers idle.  Where the windows are one round of the chip, or fill the last
 // round, or segments are of up to 40 elements.  Forward + backward in us, by a workgroup a channel and by windows, going round
 // three sets of tensors:
-//   one round: N 128, C 1024, 7 x 7 32.1 and 26.5; N 72, C 1983, 6 x 7 28.4 and 24.8 (four channels); N 104, C 830, 8 x 9 28.5 and 26.3;
-//   N 85, C 593, 11 x 11 28.8 and 26.9; N 256, C 512, 7 x 7, seven samples, 32.4 and 28.0; five samples N 170, C 759, 7 x 8 31.5 and 34.6;
-//   rounds filled: N 128, C 2048, 7 x 7 64.1 and 56.3; N 256, C 1024, 7 x 7 67.1 and 58.0; not: N 80, C 1039, 8 x 10 28.6 and 30.4, N 143,
-//   C 1122, 8 x 7 41.7 and 43.3, seven or eight samples N 135, C 669, 10 x 11 44.3 and 49.8, N 125, C 1204, 11 x 9 66.4 and 71.6;
+//   one round: N 128, C 1024, 7 x 7 32.1 and 26.5; N 72, C 1983, 6 x 7 28.4 and 24.8 (four channels); N 104, C 830, 8 x
+//   9 28.5 and 26.3; N 85, C 593, 11 x 11 28.8 and 26.9; N 256, C 512, 7 x 7, seven samples, 32.4 and 28.0; five
+//   samples N 170, C 759, 7 x 8 31.5 and 34.6; rounds filled: N 128, C 2048, 7 x 7 64.1 and 56.3; N 256, C 1024, 7 x 7
+//   67.1 and 58.0; not: N 80, C 1039, 8 x 10 28.6 and 30.4, N 143, C 1122, 8 x 7 41.7 and 43.3, seven or eight samples
+//   N 135, C 669, 10 x 11 44.3 and 49.8, N 125, C 1204, 11 x 9 66.4 and 71.6;
 //   short: N 151, C 1394, 5 x 7 37.6 and 33.9; N 238, C 1325, 5 x 4 33.7 and 29.6; N 141, C 1629, 5 x 6 34.7 and 34.1;
 //   eight samples of whole 64-byte pieces, which share no line halves: N 238, C 1514, 8 x 8 91.3 and 101.0;
-//   smaller tensors: N 128, C 1024, 6 x 6, 19 MB, 18.7 and 19.5; N 64, C 1024, 7 x 7, 13 MB, 15.6 both; N 41, C 1661, 8 x 10, 21.8 MB,
-//   22.1 and 23.8.  Segments of 128 to 160 elements lose up to a third.
+//   smaller tensors: N 128, C 1024, 6 x 6, 19 MB, 18.7 and 19.5; N 64, C 1024, 7 x 7, 13 MB, 15.6 both; N 41, C 1661, 8
+//   x 10, 21.8 MB, 22.1 and 23.8.  Segments of 128 to 160 elements lose up to a third.
 constexpr int kWindowBlock = 1024;
 constexpr size_t kWindowBytes = size_t(21) << 20;
 
@@ -3177,11 +3178,12 @@ bool team_variant(const G& g, const OnceBackward<T>* a, bool stream, bool forced
 // teams, going round three sets of tensors (330 calls):
 //   few channels (N 8, C 64, 56 x 56 14.4 and 11.8; C 16 13.5 and 10.9; with 4096 vectors or fewer equal);
 //   more than 8192 vectors, with 16 or 20 a thread: 15 % less on average, 2 % more at worst, but for channels that fill one round
-//   of the chip (C 128, N 16 27.9 and 23.2; N 6, C 283, 90 x 99 77.7 and 54.9; N 1, C 682, 203 x 188, cleared 118 and 96; N 6, C 174, 5 %
-//   more);
+//   of the chip (C 128, N 16 27.9 and 23.2; N 6, C 283, 90 x 99 77.7 and 54.9; N 1, C 682, 203 x 188, cleared 118 and
+//   96; N 6, C 174, 5 % more);
 //   up to 8192, whose backward workgroups a CU holds one of: with a halo, or dense, where channels leave half of a second round
-//   empty, or an eighth of more rounds (N 53, C 1185, 21 x 22 with a halo 173 and 158; C 622, 6800 vectors 4 % less; C 401 and 506,
-//   3 and 9 % more, C 1022 7); cleared, unless they nearly fill the rounds (N 7, C 328, 15 x 15 x 12 49 and 37; C 202 and 993, 6 % more).
+//   empty, or an eighth of more rounds (N 53, C 1185, 21 x 22 with a halo 173 and 158; C 622, 6800 vectors 4 % less; C
+//   401 and 506, 3 and 9 % more, C 1022 7); cleared, unless they nearly fill the rounds (N 7, C 328, 15 x 15 x 12 49
+//   and 37; C 202 and 993, 6 % more).
 // The state of more than 2048 channels would be as large as many a tensor.
 template <typename G>
 bool teams_first(const G& g)
@@ -3508,13 +3510,15 @@ constexpr size_t kClearedByOrder = size_t(39) << 20;
 // C 941, 4 x 5 301 and 100 us, N 176, C 910, 3 x 2 255 and 38); beyond they run at memory's rate, and a workgroup with
 // all of a channel's cells to itself needs neighbours that keep memory busy. Forward + backward in us, staged and in
 // one launch each way, of 220 calls:
-//   few workgroups of much: N 106, C 26, 4^3, halo of 3 36 and 62; N 119, C 88, 4 x 5 x 6, halo of 2 65 and 89; N 92, C 71, 4^3, halo of 2 38 and 41; more
-//   of them N 43, C 107, 5 x 5 x 4, halo of 3 62 and 52; of little N 29, C 72, 7 x 6 x 6, halo of 2 41 and 34;
-//   the largest, one a CU, in more than one round: N 57, C 454, 18 x 9, halo of 3 95 and 115; N 36, C 359, 16 x 13, halo of 3 65 and 75; in one
-//   N 83, C 183, 9 x 13, halo of 3 61 and 49; N 53, C 120, 11 x 16, halo of 2 37 and 31;
+//   few workgroups of much: N 106, C 26, 4^3, halo of 3 36 and 62; N 119, C 88, 4 x 5 x 6, halo of 2 65 and 89; N 92, C
+//   71, 4^3, halo of 2 38 and 41; more of them N 43, C 107, 5 x 5 x 4, halo of 3 62 and 52; of little N 29, C 72, 7 x 6
+//   x 6, halo of 2 41 and 34;
+//   the largest, one a CU, in more than one round: N 57, C 454, 18 x 9, halo of 3 95 and 115; N 36, C 359, 16 x 13,
+//   halo of 3 65 and 75; in one N 83, C 183, 9 x 13, halo of 3 61 and 49; N 53, C 120, 11 x 16, halo of 2 37 and 31;
 //   large outputs in a little more than one round: N 53, C 284, 4 x 4 x 5, halo of 2 73 and 95 (C 350 106 and 100);
-//   and with less halo than three times the interior, segments of more than 350 cells: N 22, C 1078, 20 x 12, halo of 3 115 and 123; N 18, C 896, 18 x 12,
-//   halo of 2 67 and 72; up to 350 N 41, C 556, 9 x 16, halo of 2 80 and 70; with more N 9, C 412, 7 x 5 x 4, halo of 3 55 and 40.
+//   and with less halo than three times the interior, segments of more than 350 cells: N 22, C 1078, 20 x 12, halo of 3
+//   115 and 123; N 18, C 896, 18 x 12, halo of 2 67 and 72; up to 350 N 41, C 556, 9 x 16, halo of 2 80 and 70; with
+//   more N 9, C 412, 7 x 5 x 4, halo of 3 55 and 40.
 bool clearing_pays(const ShortOnceClearing& g, uint32_t windows, uint32_t vectors)
 {
     constexpr size_t kMuch = 260000;

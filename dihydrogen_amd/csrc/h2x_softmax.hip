@@ -1146,21 +1146,21 @@ int launch_split(const T* y, const T* dy, T* dx, int n, int c, size_t s, bool st
 // The split kernel for 33 channels and more, or kNoSplit.  (Tiles are of 64 pixels; their numbers below are those for 256 CUs.)
 // Forward + backward, us, by such tiles (16 waves up to 256 of them, else 8) -> as now:
 // * Up to 256 tiles, no more than the CUs: 16 pixels a tile and 8 waves, four times the workgroups, each with half the
-//   channels a lane.  N 1, C 447, 17 x 13 16.9 -> 8.7; N 7, C 507, 13 x 16 19.9 -> 9.7; N 4, C 341, 50 x 40 17.8 -> 14.3; doubles, whose
-//   exponentials are longer: N 2, C 421, 20 x 19 40.6 -> 12.2, N 5, C 217, 14 x 13 17.3 -> 8.7.  Up to 96
-//   channels (64 of doubles) the launches are all there is (8.1 both ways), and beyond 16 MiB (20) the
-//   parts of lines cost as much: N 28, C 420, 25 x 15 23.3 and 25.6, N 19, C 237, 26 x 26 of doubles 29.5 and 31.2.
-// * From 257 tiles to about two a CU: forward, floats of 65 to 256 channels, 16 pixels and 4 waves, a lane's chain as short as with 16
-//   waves of 64 (32 pixels and 8 waves: N 4, C 150, 65 x 97 0.6 us more, N 3, C 129, 84 x 65 13.5 for 12.7; but N 20, C 197,
-//   32 x 25 15.4 for 16.1); else 32 pixels and 8 waves, backward to one and a half tiles a CU (beyond, N 4, C 150, 65 x 97 0.2 us
-//   more).  N 27, C 133, 23 x 28 16.3 -> 13.1; N 4, C 150, 65 x 97 18.4 -> 17.0; N 22, C 143, 38 x 33 18.3 -> 17.1.  Not
-//   where the tensors are streamed (N 1, C 306, 195 x 164 43.2 and 50.2: whole lines count there), nor beyond 384
-//   channels (N 2, C 398, 119 x 107 52 and 57).
+//   channels a lane.  N 1, C 447, 17 x 13 16.9 -> 8.7; N 7, C 507, 13 x 16 19.9 -> 9.7; N 4, C 341, 50 x 40 17.8 ->
+//   14.3; doubles, whose exponentials are longer: N 2, C 421, 20 x 19 40.6 -> 12.2, N 5, C 217, 14 x 13 17.3 -> 8.7.
+//   Up to 96 channels (64 of doubles) the launches are all there is (8.1 both ways), and beyond 16 MiB (20) the parts
+//   of lines cost as much: N 28, C 420, 25 x 15 23.3 and 25.6, N 19, C 237, 26 x 26 of doubles 29.5 and 31.2.
+// * From 257 tiles to about two a CU: forward, floats of 65 to 256 channels, 16 pixels and 4 waves, a lane's chain as
+//   short as with 16 waves of 64 (32 pixels and 8 waves: N 4, C 150, 65 x 97 0.6 us more, N 3, C 129, 84 x 65 13.5 for
+//   12.7; but N 20, C 197, 32 x 25 15.4 for 16.1); else 32 pixels and 8 waves, backward to one and a half tiles a CU
+//   (beyond, N 4, C 150, 65 x 97 0.2 us more).  N 27, C 133, 23 x 28 16.3 -> 13.1; N 4, C 150, 65 x 97 18.4 -> 17.0; N
+//   22, C 143, 38 x 33 18.3 -> 17.1.  Not where the tensors are streamed (N 1, C 306, 195 x 164 43.2 and 50.2: whole
+//   lines count there), nor beyond 384 channels (N 2, C 398, 119 x 107 52 and 57).
 // * Doubles of 257 to 512 channels, of any size: 32 pixels and 8 waves, whose values fit the registers (16 waves of 64
 //   pixels kept five words in scratch, and beyond 384 channels backward read everything twice).  N 17, C 490, 46 x 51 244 -> 185;
 //   N 1, C 267, 197 x 189 112 -> 89.
-// * Sixteen waves of 64 pixels remain for at most 256 tiles of few or of very many channels, and beyond 512 of floats (N 8, C 400,
-//   64 x 64, 512 tiles: 32.3 forward and 36.8 backward, eight waves 30.1 and 35.3).
+// * Sixteen waves of 64 pixels remain for at most 256 tiles of few or of very many channels, and beyond 512 of floats
+//   (N 8, C 400, 64 x 64, 512 tiles: 32.3 forward and 36.8 backward, eight waves 30.1 and 35.3).
 // * Two pixels a lane where that leaves two tiles a CU
 //   forward, one backward (N 1, C 60, 384 x 384, 1152 tiles of two pixels a lane: 13.3 and 22.2 us,
 //   one pixel 14.3 and 25.4; N 8, C 256, 64 x 64, 256 of them: 17.8 and 21.6, one pixel 16.5 and 23.7).
@@ -1283,10 +1283,11 @@ int launch_shared(const T* y, const T* dy, T* dx, int n, int c, size_t s, hipStr
 // Up to 32 channels: the threads of a workgroup share them, or kNoSplit. Where one thread a pixel leaves CUs waiting
 // for its chain; with more pixels the sums that every thread forms cost more than the chain. Us in a graph, a thread a
 // pixel and so (32 pixels forward, 16 backward; 64 pixels are slower throughout, and at 2^17 pixels all of them are):
-//   floats, C 32, 4608 pixels 4.9 / 4.1 and 3.6 / 3.3, 2^14 5.1 / 4.3 and 4.0 / 3.9, 2^15 5.3 / 4.5 and 4.4 / 4.8, 2^16 6.0 / 6.4 and 6.0 / 8.6;
-//   C 12, 2^14 3.1 / 2.7 and 2.9 / 2.7; C 8, 2^15 2.8 / 2.4 and 2.8 / 2.8;
-//   doubles, whose exponentials are longer, C 32, 4608 pixels 8.6 / 5.2 and 4.1 / 3.8, 2^16 12.3 / 10.0 and 9.8 / 12.3, 3 x 2^16 23.3 and 24.1
-//   forward; C 12, 2^14 4.6 / 3.2 and 3.4 / 2.9, 2^16 5.2 and 5.1 forward; C 6, 2^15 3.3 / 2.6 and 3.0 / 3.0.
+//   floats, C 32, 4608 pixels 4.9 / 4.1 and 3.6 / 3.3, 2^14 5.1 / 4.3 and 4.0 / 3.9, 2^15 5.3 / 4.5 and 4.4 / 4.8, 2^16
+//   6.0 / 6.4 and 6.0 / 8.6; C 12, 2^14 3.1 / 2.7 and 2.9 / 2.7; C 8, 2^15 2.8 / 2.4 and 2.8 / 2.8;
+//   doubles, whose exponentials are longer, C 32, 4608 pixels 8.6 / 5.2 and 4.1 / 3.8, 2^16 12.3 / 10.0 and 9.8 / 12.3,
+//   3 x 2^16 23.3 and 24.1 forward; C 12, 2^14 4.6 / 3.2 and 3.4 / 2.9, 2^16 5.2 and 5.1 forward; C 6, 2^15 3.3 / 2.6
+//   and 3.0 / 3.0.
 template <typename T, typename... P>
 int launch_shared_for(int n, int c, size_t s, hipStream_t st, P... p)
 {

@@ -688,9 +688,9 @@ int h2x_bn_backward_clearing(h2x_dtype dtype,
  * share are loaded, and where allowed stored, by both but owned by one.
  * The two-launch stages go through h2x_bn_forward_local / _backward_local for
  * geometries of three dimensions {spatial, channels, samples} with strides
- * {1, real, real * channels}, through their _strided twins otherwise.  Returns what the entry point returns; H2X_ERR_TOO_LARGE if it
- * plans more than H2X_BN_AUDIT_MAX_LAUNCHES launches.  Cost: proportional to
- * the elements of the tensors; meant for tests.
+ * {1, real, real * channels}, through their _strided twins otherwise.  Returns what the entry point returns;
+ * H2X_ERR_TOO_LARGE if it plans more than H2X_BN_AUDIT_MAX_LAUNCHES launches.  Cost: proportional to the elements of
+ * the tensors; meant for tests.
  */
 typedef enum h2x_bn_stage
 {
