@@ -580,16 +580,16 @@ def cpu_baseline(repeats: int = 5):
 # TCC_EA0_WRREQ_64B), request counts summed over the L2 channels, per dispatch.
 # label -> (bytes read, bytes written) per launch
 PMC_TRAFFIC = {
-    "bn_forward": (269481792, 269031136),
-    "bn_backward": (539881216, 269672512),
+    "bn_forward": (269508864, 268990304),
+    "bn_backward": (539907392, 269672704),
     "bn_sums": (268459008, 131072),
-    "bn_apply": (268466176, 268460160),
-    "bn_backprop1": (536907776, 131104),
-    "bn_backprop2": (536906240, 268435456),
-    "halo_dim0_pack": (147865968, 8652800),    # 4 faces (2 ranks) a launch, four launches a step
-    "halo_dim0_unpack": (9218352, 43264000),
-    "halo_dim1_pack": (42625792, 34611200),
-    "halo_dim1_unpack": (34632448, 36217952),
+    "bn_apply": (268466176, 268481792),
+    "bn_backprop1": (536907904, 131104),
+    "bn_backprop2": (536907264, 268435456),
+    "halo_dim0_pack": (147837344, 8652800),    # 4 faces (2 ranks) a launch, four launches a step
+    "halo_dim0_unpack": (9217536, 43264000),
+    "halo_dim1_pack": (42625920, 34611200),
+    "halo_dim1_unpack": (34632512, 36216768),
     "halo_dim2_pack": (34694400, 34611200),
     "halo_dim2_unpack": (34632448, 34619392),
 }
@@ -598,8 +598,8 @@ EVENT_EVERY = 4
 
 # sha256 (first 16 hex digits) of the kernel sources the table was measured with, see
 # kernel_sources_sha(); with other sources the traffic fields are omitted
-PMC_SOURCES_SHA = "24c7ab14e2a95a64"
-PMC_COMMIT = "bcbac81"
+PMC_SOURCES_SHA = "399fe1b989ece6b9"
+PMC_COMMIT = "59dd164"
 
 KERNEL_OF = {
     "bn_forward": "bn_team_forward_kernel<float,512,16>",
